@@ -56,14 +56,25 @@ def _attn_out(q):
     return torch.empty(q.shape, dtype=q.dtype, device=q.device)
 
 
+def _aligned(t):
+    """t, or a copy whose rows begin at multiples of 16 bytes."""
+    if t.data_ptr() % 16 == 0 and t.stride(0) * t.element_size() % 16 == 0:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
 def attention_prefill_batch(q, k_cache, v_cache, batch, scale, out=None):
     if out is None:
         out = _attn_out(q)
     if _PREFILL_IMPL == "mfma":
+        if q.shape[2] != 128:
+            raise RuntimeError("prefill kernel requires head_dim 128")
+        q = _aligned(q)
         meta = batch.prefill_meta(tile_q=128)
-        _C.prefill_attn_mfma(
+        _C.grouped_attn(
             out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens, meta.ctx_lens,
-            meta.row_starts, meta.tile_seq, meta.tile_q0, scale,
+            meta.row_starts, meta.tile_seq, meta.tile_q0, *(None,) * 6,
+            scale, 0.0, _NO_WINDOW, _NO_WINDOW, 0, False, _PREFILL, 1, 1,
         )
     else:
         meta = batch.prefill_meta(tile_q=64)

@@ -39,9 +39,6 @@ void launch_sample_fullvocab(int64_t*, const void*, bool, const float*, const in
                              int, int, hipStream_t);
 void launch_sample(int64_t*, const float*, const float*, const int64_t*, const float*,
                    const float*, const uint8_t*, int, int, hipStream_t);
-void launch_prefill_attn_mfma(void*, const void*, const void*, const void*, const int*,
-                              const int*, const int*, const int*, const int*, const int*,
-                              float, int, int, int, int, int, int, int64_t, hipStream_t);
 void launch_residual_norm(bool, float*, const void*, const void*, const void*, void*, float,
                           int, int, int64_t, const NormForm*, hipStream_t);
 void launch_embed_positions(bool, float*, float*, const int64_t*, const int64_t*, const void*,
@@ -174,11 +171,11 @@ static void decode_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cach
                      max_blocks, kv_block, q_stride, cur_stream());
 }
 
-static void prefill_attn_impl(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
-                              torch::Tensor v_cache, torch::Tensor block_tables,
-                              torch::Tensor seq_lens, torch::Tensor ctx_lens,
-                              torch::Tensor row_starts, torch::Tensor tile_seq,
-                              torch::Tensor tile_q0, double scale, bool mfma) {
+static void prefill_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
+                         torch::Tensor v_cache, torch::Tensor block_tables,
+                         torch::Tensor seq_lens, torch::Tensor ctx_lens,
+                         torch::Tensor row_starts, torch::Tensor tile_seq,
+                         torch::Tensor tile_q0, double scale) {
   CHECK_CUDA(q); CHECK_BF16(q); CHECK_CONT(out);
   const int64_t q_stride = q_token_stride(q);
   TORCH_CHECK(block_tables.scalar_type() == at::kInt);
@@ -188,31 +185,12 @@ static void prefill_attn_impl(torch::Tensor out, torch::Tensor q, torch::Tensor 
   const int max_blocks = block_tables.size(1);
   const int num_tiles = tile_seq.size(0);
   TORCH_CHECK(D == 128, "prefill kernel requires head_dim 128");
-  auto fn = mfma ? launch_prefill_attn_mfma : launch_prefill_attn;
-  fn(out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
-     v_cache.data_ptr(), block_tables.data_ptr<int>(),
-     seq_lens.data_ptr<int>(), ctx_lens.data_ptr<int>(),
-     row_starts.data_ptr<int>(), tile_seq.data_ptr<int>(),
-     tile_q0.data_ptr<int>(), (float)scale, num_tiles, Hq, Hkv, D,
-     max_blocks, kv_block, q_stride, cur_stream());
-}
-
-static void prefill_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
-                         torch::Tensor v_cache, torch::Tensor block_tables,
-                         torch::Tensor seq_lens, torch::Tensor ctx_lens,
-                         torch::Tensor row_starts, torch::Tensor tile_seq,
-                         torch::Tensor tile_q0, double scale) {
-  prefill_attn_impl(out, q, k_cache, v_cache, block_tables, seq_lens, ctx_lens,
-                    row_starts, tile_seq, tile_q0, scale, /*mfma=*/false);
-}
-
-static void prefill_attn_mfma(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
-                              torch::Tensor v_cache, torch::Tensor block_tables,
-                              torch::Tensor seq_lens, torch::Tensor ctx_lens,
-                              torch::Tensor row_starts, torch::Tensor tile_seq,
-                              torch::Tensor tile_q0, double scale) {
-  prefill_attn_impl(out, q, k_cache, v_cache, block_tables, seq_lens, ctx_lens,
-                    row_starts, tile_seq, tile_q0, scale, /*mfma=*/true);
+  launch_prefill_attn(out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
+                      v_cache.data_ptr(), block_tables.data_ptr<int>(),
+                      seq_lens.data_ptr<int>(), ctx_lens.data_ptr<int>(),
+                      row_starts.data_ptr<int>(), tile_seq.data_ptr<int>(),
+                      tile_q0.data_ptr<int>(), (float)scale, num_tiles, Hq, Hkv, D,
+                      max_blocks, kv_block, q_stride, cur_stream());
 }
 
 // C[M,N] = A[M,K] @ B[N,K]^T — the hand-written 256²-tile 8-phase MFMA
@@ -1117,7 +1095,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_cache", &rope_cache);
   m.def("decode_attn", &decode_attn);
   m.def("prefill_attn", &prefill_attn);
-  m.def("prefill_attn_mfma", &prefill_attn_mfma);
   m.def("mfma_probe", &mfma_probe);
   m.def("gemm_bf16", &gemm_bf16);
   m.attr("DEPTH_AHEAD") = DEPTH_AHEAD;

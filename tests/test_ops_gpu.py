@@ -193,6 +193,38 @@ def test_prefill_attn_multi_seq(impl, monkeypatch):
 
 
 @requires_gpu
+@pytest.mark.parametrize("block", [8, 16, 24, 64])
+@pytest.mark.parametrize("H,G,scale", [(8, 8, 0.09), (6, 2, -0.09), (4, 1, 0.0)])
+def test_prompt_tiles_over_pages(block, H, G, scale):
+    """Chunks that end in, at and past tiles of 64 keys and 128 rows, on pages of every
+    kind; what no token has written is NaN."""
+    from op_helpers import make_batch
+
+    chunks = [(0, 1), (0, 63), (5, 59), (0, 129), (300, 5), (127, 130)]
+    batch, _, tables, pages = make_batch(chunks, block, "cuda")
+    kc = torch.full((pages, block, G, 128), float("nan"), device="cuda").bfloat16()
+    vc = kc.clone()
+    for m in batch.prefills:
+        slots = [m.block_table[p // block] * block + p % block for p in range(m.seq_len)]
+        for c in (kc, vc):
+            c.view(-1, G, 128)[slots] = torch.randn(m.seq_len, G, 128, device="cuda").bfloat16()
+    rows = batch.num_prefill_tokens
+    q = torch.randn(rows, (H + 3) * 128, device="cuda").bfloat16()
+    q = q.as_strided((rows, H, 128), (q.stride(0), 128, 1), 8)
+    out = hip().attention_prefill_batch(q, kc, vc, batch, scale)
+    row = 0
+    for m in batch.prefills:
+        mine = slice(row, row + m.query_len)
+        want = ref.attention_prefill(
+            q[mine].cpu().float(), kc.cpu().float(), vc.cpu().float(), m.block_table,
+            m.seq_len, m.ctx_len, scale,
+        )
+        # weights and results are rounded to 8 bits: 2 * 2^-9 of values up to 5
+        assert maxerr(out[mine].cpu(), want) < 0.02, m
+        row += m.query_len
+
+
+@requires_gpu
 def test_sample_greedy_and_filters():
     torch.manual_seed(3)
     B, V = 64, 261
