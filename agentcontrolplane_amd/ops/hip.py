@@ -86,20 +86,27 @@ def attention_prefill_batch(q, k_cache, v_cache, batch, scale, out=None):
 
 
 def attention_decode_batch(q, k_cache, v_cache, batch, scale, out=None):
-    if out is None:
-        out = _attn_out(q)
-    _C.decode_attn(
-        out, q, k_cache, v_cache, batch.decode_tables_i32(), batch.decode_lens_i32(),
-        scale,
+    return _attention_decode(
+        q, k_cache, v_cache, batch.decode_tables_i32(), batch.decode_lens_i32(), scale, out
     )
-    return out
 
 
 def attention_decode_raw(q, k_cache, v_cache, block_tables, seq_lens, scale):
-    out = _attn_out(q)
-    _C.decode_attn(
-        out, q, k_cache, v_cache, block_tables.int().contiguous(),
-        seq_lens.int().contiguous(), scale,
+    return _attention_decode(
+        q, k_cache, v_cache, block_tables.int().contiguous(), seq_lens.int().contiguous(), scale
+    )
+
+
+def _attention_decode(q, k_cache, v_cache, tables, seq_lens, scale, out=None):
+    if out is None:
+        out = _attn_out(q)
+    if q.shape[2] != 128:
+        raise RuntimeError("decode kernel requires head_dim 128")
+    if q.shape[1] > 8 * k_cache.shape[2]:
+        raise RuntimeError("GQA group must be <= 8")
+    _grouped_decode(
+        out, _aligned(q), k_cache, v_cache, tables, seq_lens, None, None, None, scale, 0.0,
+        _NO_WINDOW, _NO_WINDOW, 0, False,
     )
     return out
 
@@ -355,6 +362,33 @@ def attention_inputs(proj, heads, dim, vdim, k_cache, v_cache, batch, eps, conv,
     return q
 
 
+def _grouped_decode(out, q, k_cache, v_cache, tables, seq_lens, sink, bias, gate, scale, cap,
+                    window, chunk, keep_first, sigmoid):
+    """One token per sequence, head sizes of the matrix-core kernels.  Grid and workspace
+    depend on sizes alone, not on the lengths, so that a step can be captured."""
+    (B, H, d), v, G = q.shape, out.shape[2], k_cache.shape[2]
+    gm = next((n for n in (1, 4) if n >= H // G), 8)  # query heads a workgroup holds
+    # pieces of the step's keys: workgroups that fill the chip
+    keys = min(tables.shape[1] * k_cache.shape[1], window + keep_first, chunk)
+    groups = G * -(-(H // G) // gm)
+    pieces, part, ml = 0, None, None
+    if B * groups < _WHOLE_GROUPS and keys > 128:
+        pieces = max(1, _DECODE_GROUPS // groups)
+        part = torch.empty((pieces + B) * H * v, dtype=torch.float32, device=q.device)
+        ml = torch.empty(2 * (pieces + B) * H, dtype=torch.float32, device=q.device)
+    _C.grouped_attn(
+        out, q, k_cache, v_cache, tables, seq_lens, None, None, None, None, sink, bias, gate,
+        None, part, ml, scale, cap, window, chunk, keep_first, sigmoid, _DECODE, gm, pieces,
+    )
+
+
+#: workgroups that a decode step's keys are cut for: 2 rounds of the 2 a CU that fit
+_DECODE_GROUPS = 1024
+#: from so many sequences and key heads on a sequence is one piece (190 x 8, 700 to 1300 keys:
+#: 159 us, cut as fewer ones 169; 250 x 8, 200 to 2000 keys: 235 and 250 us)
+_WHOLE_GROUPS = 1024
+
+
 def grouped_attention(q, k_cache, v_cache, batch, scale: float, cap, window, keep_first: int,
                       sink, out, bias=None, sigmoid=False, gate=None, chunk=None, talk=None):
     from . import LATENT_HEADS
@@ -389,24 +423,23 @@ def grouped_attention(q, k_cache, v_cache, batch, scale: float, cap, window, kee
     if not batch.num_decode:
         return
     tables, rows = batch.decode_tables_i32(), batch.num_decode * H
-    gm, n_split, part, ml = 1, 1, None, None
-    # keys a row may see
-    keys = min(tables.shape[1] * k_cache.shape[1], rest[2] + keep_first, rest[3])
+    if kinds[0] == _DECODE:
+        _grouped_decode(
+            out[P:], q[P:], k_cache, v_cache, tables, batch.decode_lens_i32(), sink, bias,
+            gates(slice(P, None)), *rest,
+        )
+        return
+    n_split, part, ml = 1, None, None
     if kinds[0] == _TALK_DECODE:  # a workgroup has all heads, and 4 waves with 32 keys each
+        keys = min(tables.shape[1] * k_cache.shape[1], rest[2], rest[3])  # a row may see
         n_split = max(1, min(_MAX_SPLIT, 1024 // batch.num_decode, -(-keys // 128)))
-    elif kinds[0] == _DECODE:
-        most = 8 if d + v <= 256 else 4  # query heads a workgroup holds
-        gm = next((n for n in (1, 2, 4) if n >= min(H // G, most)), most)
-        # workgroups that fill the chip; every split has work for its 16 lane groups
-        groups = batch.num_decode * G * -(-(H // G) // gm)
-        n_split = max(1, min(_MAX_SPLIT, 1024 // groups, -(-keys // 128)))
     if n_split > 1:
         part = torch.empty(n_split * rows * v, dtype=torch.float32, device=q.device)
         ml = torch.empty(2 * n_split * rows, dtype=torch.float32, device=q.device)
     _C.grouped_attn(
         out[P:], q[P:], k_cache, v_cache, tables, batch.decode_lens_i32(), None, None, None,
         None, sink, bias, gates(slice(P, None)), talk, part, ml, *rest,
-        kinds[0], gm, n_split,
+        kinds[0], 1, n_split,
     )
 
 

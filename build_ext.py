@@ -26,7 +26,6 @@ def build(verbose: bool = False) -> str:
         os.path.join(CSRC, "block_manager.cpp"),
         os.path.join(CSRC, "elementwise.hip"),
         os.path.join(CSRC, "rope_cache.hip"),
-        os.path.join(CSRC, "decode_attn.hip"),
         os.path.join(CSRC, "prefill_attn.hip"),
         os.path.join(CSRC, "mfma_probe.hip"),
         os.path.join(CSRC, "gemm_bf16.hip"),

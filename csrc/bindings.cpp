@@ -28,9 +28,6 @@ void launch_swiglu(void*, const void*, int64_t, int, hipStream_t);
 void launch_rope_cache(void*, void*, const void*, void*, void*, const int64_t*,
                        const int64_t*, const float*, int, int, int, int, int64_t,
                        int64_t, int64_t, hipStream_t);
-void launch_decode_attn(void*, const void*, const void*, const void*, const int*,
-                        const int*, float, int, int, int, int, int, int, int64_t,
-                        hipStream_t);
 void launch_prefill_attn(void*, const void*, const void*, const void*, const int*,
                          const int*, const int*, const int*, const int*, const int*,
                          float, int, int, int, int, int, int, int64_t, hipStream_t);
@@ -51,7 +48,7 @@ void launch_experts_small(bool, const ExpertsArgs*, int, hipStream_t);
 void launch_experts_f32(bool, const ExpertsArgs*, hipStream_t);
 void launch_experts_gemm(bool, const ExpertsArgs*, hipStream_t);
 void launch_softcap(bool, float*, const void*, float, int64_t, hipStream_t);
-bool launch_grouped_decode(const GroupedArgs*, int, int, int, int, hipStream_t);
+bool launch_grouped_decode(const GroupedArgs*, int, int, int, hipStream_t);
 bool launch_grouped_plain(bool, const GroupedArgs*, int, int, int, hipStream_t);
 bool launch_grouped_prefill(const GroupedArgs*, int, int, hipStream_t);
 int talk_prefill_tokens(int, int, int, int, int);
@@ -149,26 +146,6 @@ static void rope_cache(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                     v_cache.data_ptr(), positions.data_ptr<int64_t>(),
                     slot_mapping.data_ptr<int64_t>(), cos_sin.data_ptr<float>(), N,
                     Hq, Hkv, D, P, q_stride, kv_stride, cur_stream());
-}
-
-static void decode_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
-                        torch::Tensor v_cache, torch::Tensor block_tables,
-                        torch::Tensor seq_lens, double scale) {
-  CHECK_CUDA(q); CHECK_BF16(q); CHECK_CONT(out);
-  CHECK_CONT(k_cache); CHECK_CONT(v_cache);
-  const int64_t q_stride = q_token_stride(q);
-  TORCH_CHECK(block_tables.scalar_type() == at::kInt && seq_lens.scalar_type() == at::kInt);
-  CHECK_CONT(block_tables); CHECK_CONT(seq_lens);
-  const int B = q.size(0), Hq = q.size(1), D = q.size(2);
-  const int Hkv = k_cache.size(2);
-  const int kv_block = k_cache.size(1);
-  const int max_blocks = block_tables.size(1);
-  TORCH_CHECK(D == 128, "decode kernel requires head_dim 128");
-  TORCH_CHECK(Hq % Hkv == 0 && Hq / Hkv <= 8, "GQA group must be <= 8");
-  launch_decode_attn(out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
-                     v_cache.data_ptr(), block_tables.data_ptr<int>(),
-                     seq_lens.data_ptr<int>(), (float)scale, B, Hq, Hkv, D,
-                     max_blocks, kv_block, q_stride, cur_stream());
 }
 
 static void prefill_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
@@ -735,7 +712,9 @@ static void grouped_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
   CHECK_CUDA(tables); CHECK_CONT(tables);
   TORCH_CHECK(tables.scalar_type() == at::kInt && tables.dim() == 2);
   const int seqs = tables.size(0);
-  TORCH_CHECK(window > 0 && keep >= 0 && cap >= 0 && n_split >= 1 && n_split <= 64);
+  // kind 1: n_split is the pieces that a step's keys are cut into, 0: one a sequence
+  TORCH_CHECK(window > 0 && keep >= 0 && cap >= 0 && n_split >= (kind != 1) &&
+              n_split <= (kind == 1 ? 1 << 16 : 64));
   TORCH_CHECK(chunk > 0 && chunk <= (1 << 30) && (keep == 0 || chunk == (1 << 30)),
               "chunks keep no first tokens");
   TORCH_CHECK(kind == 0 || bf16, "the matrix-core kernels take bf16");
@@ -745,11 +724,12 @@ static void grouped_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
   if (tokens == 0 || seqs == 0) return;
   GroupedArgs a{};
   a.out = out.data_ptr();
-  if (n_split > 1) {
+  if (kind == 1 ? n_split > 0 : n_split > 1) {
+    const int64_t rows = kind == 1 ? (n_split + seqs) * H : n_split * tokens * H;
     TORCH_CHECK(part && part_ml && part->is_contiguous() && part_ml->is_contiguous());
     TORCH_CHECK(part->scalar_type() == at::kFloat && part_ml->scalar_type() == at::kFloat);
-    TORCH_CHECK(part->numel() >= n_split * tokens * H * v &&
-                part_ml->numel() >= 2 * n_split * tokens * H, "split workspace");
+    CHECK_CUDA((*part)); CHECK_CUDA((*part_ml));
+    TORCH_CHECK(part->numel() >= rows * v && part_ml->numel() >= 2 * rows, "split workspace");
     a.part = part->data_ptr<float>();
     a.part_ml = (float2*)part_ml->data_ptr<float>();
   }
@@ -797,7 +777,8 @@ static void grouped_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
   a.kv_block = k_cache.size(1);
   a.window = (int)window;
   a.keep = (int)keep;
-  a.n_split = (int)n_split;
+  a.n_split = a.pieces = (int)n_split;
+  a.seqs = seqs;
   a.rows = tokens * H;
   a.scale = (float)scale;
   a.cap = (float)cap;
@@ -805,7 +786,7 @@ static void grouped_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
   const bool ok = kind == 4   ? launch_talk_prefill(&a, d, v, cur_stream())
                   : kind == 3 ? launch_talk_decode(&a, d, v, seqs, cur_stream())
                   : kind == 2   ? launch_grouped_prefill(&a, d, v, cur_stream())
-                  : kind == 1 ? launch_grouped_decode(&a, d, v, seqs, (int)gm, cur_stream())
+                  : kind == 1 ? launch_grouped_decode(&a, d, v, (int)gm, cur_stream())
                               : launch_grouped_plain(bf16, &a, d, v, tokens, cur_stream());
   TORCH_CHECK(ok, "grouped attention: unsupported sizes d ", d, " v ", v);
 }
@@ -1093,7 +1074,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("swiglu", &swiglu);
   m.def("rope_cache", &rope_cache);
-  m.def("decode_attn", &decode_attn);
   m.def("prefill_attn", &prefill_attn);
   m.def("mfma_probe", &mfma_probe);
   m.def("gemm_bf16", &gemm_bf16);

@@ -8,13 +8,21 @@
 // value), so that neither the merge of partial sums nor the output knows about it.
 // Sigmoid weights need no such state: their partial results are plain sums.
 //
-// Decode: a workgroup owns one (sequence, key/value head) and up to GM of its query
-// heads; its 16 lane groups of 16 take every 16th visible key, a few of them in
-// flight, a lane KE dims of the key and VE of the value.  Kept and window keys form one list
-// without gaps, so nothing is masked.  Few workgroups split the list (grid.y).
+// Decode: the keys stream once, from memory to registers.  A wave takes 32 of them at a time,
+// the next 32 in flight meanwhile: keys as the matrix cores want them (16 keys by 8 dims a lane),
+// the heads that share them are the columns of one product; values as 8 dims a lane, weighted in
+// fp32 by the VALU.  Between the two the weights pass through a few LDS rows of the wave.
+// The blocks of 32 that a sequence's query sees are cut into pieces of one size, so that the
+// pieces of a step, whatever its lengths, fill the chip evenly; a workgroup finds its piece from
+// the lengths by itself, and a second launch merges sequences of several pieces.
+// Bound by memory: 5.2 to 5.3 TB/s of keys and values at 64 x 4096 and 256 x 1024 tokens, 32
+// heads over 8.  Before, with products and sums over dims on the VALU, 4.1 TB/s there and 2.0 to
+// 3.0 where lengths differ: 61 x 310 to 4000 tokens 268 -> 122 us, 190 x 700 to 1300 265 -> 159,
+// 1 x 4002 203 -> 15 (two launches and their first loads, not memory).  Without the next block in
+// flight the same kernel takes 350 us at 190 x 700 to 1300; at 3 waves a SIMD the registers for
+// it are not there.
 #include "common_t.h"
 #include "grouped_attn.h"
-#include "latent_attn.h"
 
 #define NEG -1e30f
 #define LOG2E 1.44269504088896f
@@ -32,149 +40,319 @@ static DEV KeyList visible_keys(const GroupedArgs& a, int pos) {
   return k;
 }
 
-template <int KE, int VE, int GM, bool SIG>
-__global__ __launch_bounds__(256, GM * (KE + VE) <= 32 ? 4 : GM * (KE + VE) <= 64 ? 3 : 2) void grouped_decode_kernel(
-    const GroupedArgs a) {
-  constexpr int D = 16 * KE, V = 16 * VE;
-  constexpr int KEYS = GM * (KE + VE) <= 32 ? 4 : 2;  // in flight per lane group
+typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
+typedef float f32x4_v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(4))) const int const_int;
+
+#define KB 32  // keys of a block: one wave's step
+
+// The blocks that a query at position pos sees: those with kept tokens, then those its window
+// or chunk reaches.
+struct Blocks {
+  int kept, first, n;
+  DEV int key(int i) const { return (i < kept ? i : first + i - kept) * KB; }
+};
+
+static DEV Blocks visible_blocks(const GroupedArgs& a, int pos) {
+  Blocks b;
+  b.kept = (min(a.keep, pos + 1) + KB - 1) / KB;
+  b.first = max(b.kept, first_key(a, pos) / KB);
+  b.n = b.kept + max(0, (pos + KB) / KB - b.first);
+  return b;
+}
+
+// A sequence's pieces: ``n`` blocks, ``size`` of them a piece, numbered from ``first`` on.
+struct Pieces {
+  int seq, n, size, pieces, first;
+};
+
+// sum of the lanes up to this one (row shifts and broadcasts of rows' last lanes)
+static DEV int wave_scan(int v) {
+#define SCAN(ctrl, rows) v += __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false)
+  SCAN(0x111, 0xf); SCAN(0x112, 0xf); SCAN(0x114, 0xf); SCAN(0x118, 0xf);
+  SCAN(0x142, 0xa); SCAN(0x143, 0xc);
+#undef SCAN
+  return v;
+}
+
+// a value and the one of lane ^ 16 or lane ^ 32
+template <int LANES>
+static DEV float2 with_lane(float v) {
+  const int i = __float_as_int(v);
+  const auto r = LANES == 32 ? __builtin_amdgcn_permlane32_swap(i, i, false, false)
+                             : __builtin_amdgcn_permlane16_swap(i, i, false, false);
+  return float2{__int_as_float(r[0]), __int_as_float(r[1])};
+}
+template <int LANES>
+static DEV float sum_with(float v) {
+  if constexpr (LANES < 16) return v + __shfl_xor(v, LANES, 64);
+  const float2 r = with_lane<LANES < 16 ? 16 : LANES>(v);
+  return r.x + r.y;
+}
+template <int LANES>
+static DEV float max_with(float v) {
+  const float2 r = with_lane<LANES>(v);
+  return fmaxf(r.x, r.y);
+}
+
+// Pieces have about equally many blocks, a multiple of 4, so many that they are at most
+// a.pieces and one for every sequence.  Half as many pieces, one round of workgroups, are better while they
+// are short (20 x 300 to 1024 keys: 24 us, else 29) or are whole sequences (64 x 1024: 60, else
+// 69); long parts are too uneven (61 x 310 to 4000: 141, else 122).  a.pieces == 0: every
+// sequence is one piece.  Finds those of sequence ``want``, or those with piece ``item``
+// (pieces == 0: there is none).  A wave's lanes read the lengths, 64 at a time.
+static DEV Pieces find_pieces(const GroupedArgs& a, int want, int item) {
+  const int lane = threadIdx.x & 63;
+  auto blocks_of = [&](int seq) {
+    return seq < a.seqs ? visible_blocks(a, a.seq_lens[seq] - 1).n : 0;
+  };
+  Pieces p = {0, 0, 0, 0, 0};
+  if (a.pieces == 0) {
+    p.seq = p.first = item;
+    p.n = p.size = blocks_of(item);
+    p.pieces = 1;
+    return p;
+  }
+  const int mine0 = blocks_of(lane);
+  int total = mine0, longest = mine0;
+  for (int s = 64; s < a.seqs; s += 64) {
+    const int n = blocks_of(s + lane);
+    total += n;
+    longest = max(longest, n);
+  }
+  total = __builtin_amdgcn_readlane(wave_scan(total), 63);
+  const int half = max(1, (total + 2 * a.pieces - 1) / (2 * a.pieces));
+  const int all = max(min(half, 4), (total + 4 * a.pieces - 1) / (4 * a.pieces));
+  const int size = 4 * (__any(longest > 4 * half) ? all : half);
+  int before = 0;
+  for (int s = 0; s < a.seqs; s += 64) {
+    const int n = s ? blocks_of(s + lane) : mine0;
+    // a last piece of under a quarter is shared by the others
+    const int about = max(1, (n + size - (size < 12 ? 0 : size / 4) - 1) / size);
+    const int each = about * size >= n ? size : 4 * ((n + 4 * about - 1) / (4 * about));
+    const int k = s + lane < a.seqs ? max(1, (n + each - 1) / each) : 0;
+    const int upto = before + wave_scan(k);  // pieces up to this lane's
+    const bool mine = want >= 0 ? s + lane == want : item >= upto - k && item < upto;
+    const uint64_t hit = __ballot(mine);
+    if (hit) {
+      const int at = __builtin_ctzll(hit);
+      p.seq = s + at;
+      p.n = __builtin_amdgcn_readlane(n, at);
+      p.size = __builtin_amdgcn_readlane(each, at);
+      p.pieces = __builtin_amdgcn_readlane(k, at);
+      p.first = __builtin_amdgcn_readlane(upto - k, at);
+      break;
+    }
+    before = __builtin_amdgcn_readlane(upto, 63);
+  }
+  return p;
+}
+
+// PAGED: pages of 16 2^n keys, so that a group of 16 keys has one, scalar, place
+template <int DN, int VN, int GM, bool SIG, bool PAGED>
+__global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kernel(const GroupedArgs a) {
+  constexpr int D = 64 * DN, V = 64 * VN, STEPS = D / 32;
+  constexpr int LPK = V / 8, KPL = 64 / LPK, NV = KB / KPL;  // lanes a key, keys a load, loads
+  constexpr bool AHEAD = D + V <= 256;  // the next block's loads fit beside this one's
+  __shared__ float weight[4][KB][GM], rescale[4][GM];
   __shared__ float lds_acc[4][GM][V];
   __shared__ float2 lds_ml[4][GM];
+  __shared__ int slots[PAGED ? 1 : 4][KB];
   const int group = a.H / a.G, per = (group + GM - 1) / GM;  // workgroups per kv head
   const int part = blockIdx.x % per;
-  const int kvh = blockIdx.x / per % a.G, seq = blockIdx.x / (per * a.G);
+  const int kvh = blockIdx.x / per % a.G, item = blockIdx.x / (per * a.G);
   const int h0 = kvh * group + part * GM, heads = min(GM, group - part * GM);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int j = lane & 15, gid = wid * 4 + (lane >> 4);
-  const int64_t row0 = (int64_t)seq * a.H + h0;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, j = lane >> 4;           // product: column (head), rows 4 j ..
+  const int kl = lane / LPK, el = lane % LPK;       // values: key of a load, 8 dims
 
-  const int pos = a.seq_lens[seq] - 1;
-  const KeyList keys = visible_keys(a, pos);
-  const int per_split = (keys.n + a.n_split - 1) / a.n_split;
-  const int x0 = min(keys.n, (int)blockIdx.y * per_split), x1 = min(keys.n, x0 + per_split);
-  if (x0 >= x1) {  // an empty split; those are a row's last ones
-    if ((int)threadIdx.x < heads)
-      a.part_ml[(int64_t)blockIdx.y * a.rows + row0 + threadIdx.x] = float2{NEG, -1.f};
-    return;
+  const Pieces p = find_pieces(a, -1, item);
+  if (p.pieces == 0) return;  // more workgroups than pieces
+  const int seq = p.seq, pos = a.seq_lens[seq] - 1, nth = item - p.first;
+  const Blocks blocks = visible_blocks(a, pos);
+  const int end = min(p.n, (nth + 1) * p.size);
+  const int lo = first_key(a, pos);
+
+  const uint32_t k_row = (uint32_t)a.G * D * 2, v_row = (uint32_t)a.G * V * 2;  // bytes
+  const char* kp = (const char*)a.k_cache + (int64_t)kvh * D * 2;
+  const char* vp = (const char*)a.v_cache + (int64_t)kvh * V * 2;
+  const int* table = a.tables + (int64_t)seq * a.max_blocks;
+  const const_int* pages = (const const_int*)table;
+  const int shift = __builtin_ctz(a.kv_block);
+  struct Place { int slot[2]; };  // of a block's two groups of 16 keys
+  auto find = [&](int i) {
+    Place at;
+    const int key0 = blocks.key(i);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int k = min(key0 + 16 * g, pos & ~15);
+      at.slot[g] = PAGED ? (pages[k >> shift] << shift) + (k & (a.kv_block - 1)) : 0;
+    }
+    return at;
+  };
+  struct Rows {
+    bf16x8_v k[2][STEPS], v[NV];
+  };
+  const uint32_t k_off = c * k_row + j * 16, v_off = kl * v_row + el * 16;
+  auto load = [&](int i, const Place& at, Rows& r) {
+    if constexpr (PAGED) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+          r.k[g][s] = *(const bf16x8_v*)(kp + (uint64_t)(uint32_t)at.slot[g] * k_row + k_off + s * 64);
+#pragma unroll
+      for (int n = 0; n < NV; ++n)
+        r.v[n] = *(const bf16x8_v*)(vp + (uint64_t)(uint32_t)at.slot[n * KPL / 16] * v_row +
+                                  n * KPL % 16 * v_row + v_off);
+    } else {
+      const int k = min(blocks.key(i) + (lane & (KB - 1)), pos);
+      const int page = k / a.kv_block;
+      if (lane < KB) slots[wid][lane] = table[page] * a.kv_block + k - page * a.kv_block;
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const char* kr = kp + (uint64_t)(uint32_t)slots[wid][g * 16 + c] * k_row + j * 16;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) r.k[g][s] = *(const bf16x8_v*)(kr + s * 64);
+      }
+#pragma unroll
+      for (int n = 0; n < NV; ++n)
+        r.v[n] = *(const bf16x8_v*)(vp + (uint64_t)(uint32_t)slots[wid][n * KPL + kl] * v_row + el * 16);
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  Rows r0, r1;
+  int i = nth * p.size + wid;
+  Place at{};
+  if (i < end) {
+    load(i, find(i), r0);
+    if (AHEAD && PAGED) at = find(min(i + 4, p.n - 1));
   }
 
+  // the heads' queries as columns, 8 dims a lane and step
+  const int head = h0 + min(c, heads - 1);
+  bf16x8_v q[STEPS];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s)
+    q[s] = *(const bf16x8_v*)((const bf16_t*)a.q + seq * a.q_stride + (int64_t)head * D + s * 32 + j * 8);
   // scores in the exp2 domain: a factor, or c1 - 2 c1 / (exp2(c3 s) + 1)
   const float c1 = a.cap * LOG2E;
   const float mul = a.cap > 0.f ? 2.f * LOG2E * a.scale / a.cap : a.scale * LOG2E;
-  float q[GM][KE], m[GM], l[GM], acc[GM][VE];
-#pragma unroll
-  for (int g = 0; g < GM; ++g) {
-    const int h = h0 + min(g, heads - 1);
-    const bf16_t* qr = (const bf16_t*)a.q + seq * a.q_stride + (int64_t)h * D + j * KE;
-#pragma unroll
-    for (int e = 0; e < KE; e += (KE < 8 ? KE : 8)) load_f<(KE < 8 ? KE : 8)>(q[g] + e, qr + e);
-    const bool sink = a.sink && blockIdx.y == 0 && gid == 0;
-    m[g] = sink ? a.sink[h] * LOG2E : NEG;
-    l[g] = sink ? 1.f : 0.f;
-#pragma unroll
-    for (int e = 0; e < VE; ++e) acc[g][e] = 0.f;
-  }
-
-  const int* table = a.tables + (int64_t)seq * a.max_blocks;
-  const bf16_t* kc = (const bf16_t*)a.k_cache + kvh * D + j * KE;
-  const bf16_t* vc = (const bf16_t*)a.v_cache + kvh * V + j * VE;
-  int64_t slot[KEYS];
-  auto find = [&](int x) {
-#pragma unroll
-    for (int u = 0; u < KEYS; ++u) {
-      const int k = keys.at(min(x + 16 * u, x1 - 1));
-      slot[u] = (int64_t)table[k / a.kv_block] * a.kv_block + k % a.kv_block;
-    }
-  };
+  const bool sink = a.sink && nth == 0 && wid == 0;
+  float m = sink ? a.sink[head] * LOG2E : NEG, l = sink && j == 0 ? 1.f : 0.f;
   // biases: distances of n_bias - 1 and more share one
   const int far = a.n_bias - 1;
-  float b_far[GM];
+  const float* bias = a.bias ? a.bias + (int64_t)head * a.n_bias : nullptr;
+  const float b_far = bias ? bias[far] * LOG2E : 0.f;
+  float acc[GM][8] = {};
+
+  auto work = [&](int i, Rows& r) {
+    const int key0 = blocks.key(i);
+    auto hidden = [&](int key) { return (key > pos) | ((key < lo) & (key >= a.keep)); };
+    f32x4_v s[2] = {};
 #pragma unroll
-  for (int g = 0; g < GM; ++g)
-    b_far[g] = a.bias ? a.bias[(h0 + min(g, heads - 1)) * a.n_bias + far] * LOG2E : 0.f;
-  find(x0 + gid);
-  for (int x = x0 + gid; x < x1; x += 16 * KEYS) {
-    Pack<bf16_t, KE> k[KEYS];
-    Pack<bf16_t, VE> v[KEYS];
+    for (int st = 0; st < STEPS; ++st)
 #pragma unroll
-    for (int u = 0; u < KEYS; ++u) {
-      k[u] = *(const Pack<bf16_t, KE>*)(kc + slot[u] * a.G * D);
-      v[u] = *(const Pack<bf16_t, VE>*)(vc + slot[u] * a.G * V);
+      for (int g = 0; g < 2; ++g)
+        s[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.k[g][st], q[st], s[g], 0, 0, 0);
+    float w[8], mt = NEG;
+    const bool edge = key0 + KB - 1 > pos || (key0 < lo && key0 + KB > a.keep);
+    const bool near = bias && pos - (key0 + KB - 1) < far;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int key = key0 + (e >> 2) * 16 + 4 * j + (e & 3);
+      float x = s[e >> 2][e & 3] * mul;
+      if (a.cap > 0.f) x = c1 - 2.f * c1 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x) + 1.f);
+      x += near ? bias[min(max(pos - key, 0), far)] * LOG2E : b_far;
+      if (edge && hidden(key)) x = -INFINITY;
+      w[e] = x;
+      mt = fmaxf(mt, x);
     }
-    int dist[KEYS];
-    bool near = false;
+    if (edge) {  // what no token has written may be anything
 #pragma unroll
-    for (int u = 0; u < KEYS; ++u) {
-      dist[u] = pos - keys.at(min(x + 16 * u, x1 - 1));
-      near |= dist[u] < far;
+      for (int n = 0; n < NV; ++n)
+        if (hidden(key0 + n * KPL + kl)) r.v[n] = bf16x8_v{};
     }
-    near &= a.bias != nullptr;
-    find(x + 16 * KEYS);
+    if constexpr (SIG) {
 #pragma unroll
-    for (int g = 0; g < GM; ++g) {
-      float s[KEYS], b[KEYS], mt = m[g];
+      for (int e = 0; e < 8; ++e) w[e] = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-w[e]));
+    } else {
+      mt = max_with<32>(max_with<16>(mt));
+      if (__any(mt > m)) {
+        const float up = fmaxf(m, mt), alpha = __builtin_amdgcn_exp2f(m - up);
+        m = up;
+        l *= alpha;
+        if (lane < GM) rescale[wid][lane] = alpha;
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int u = 0; u < KEYS; ++u) b[u] = b_far[g];
-      if (near) {
-        const float* br = a.bias + (int64_t)(h0 + min(g, heads - 1)) * a.n_bias;
+        for (int g = 0; g < GM; ++g) {
+          const float f = rescale[wid][g];
 #pragma unroll
-        for (int u = 0; u < KEYS; ++u) b[u] = br[min(dist[u], far)] * LOG2E;
-      }
-#pragma unroll
-      for (int u = 0; u < KEYS; ++u) {
-        float dot = 0.f;
-#pragma unroll
-        for (int e = 0; e < KE; ++e) dot += q[g][e] * to_f(k[u].v[e]);
-        dot = row16_sum(dot) * mul;
-        if (a.cap > 0.f)
-          dot = c1 - 2.f * c1 * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(dot) + 1.f);
-        s[u] = x + 16 * u < x1 ? dot + b[u] : -INFINITY;
-        mt = fmaxf(mt, s[u]);
-      }
-      if constexpr (SIG) {
-#pragma unroll
-        for (int u = 0; u < KEYS; ++u) {
-          const float p = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-s[u]));
-#pragma unroll
-          for (int e = 0; e < VE; ++e) acc[g][e] += p * to_f(v[u].v[e]);
+          for (int e = 0; e < 8; ++e) acc[g][e] *= f;
         }
-        continue;
       }
-      const float alpha = __builtin_amdgcn_exp2f(m[g] - mt);
-      m[g] = mt;
-      l[g] *= alpha;
 #pragma unroll
-      for (int e = 0; e < VE; ++e) acc[g][e] *= alpha;
-#pragma unroll
-      for (int u = 0; u < KEYS; ++u) {
-        const float p = __builtin_amdgcn_exp2f(s[u] - mt);
-        l[g] += p;
-#pragma unroll
-        for (int e = 0; e < VE; ++e) acc[g][e] += p * to_f(v[u].v[e]);
+      for (int e = 0; e < 8; ++e) {
+        w[e] = __builtin_amdgcn_exp2f(w[e] - m);
+        l += w[e];
       }
+    }
+    if (c < GM)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) weight[wid][(e >> 2) * 16 + 4 * j + (e & 3)][c] = w[e];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      float f[GM];
+#pragma unroll
+      for (int g = 0; g < GM; ++g) f[g] = weight[wid][n * KPL + kl][g];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = (float)r.v[n][e];
+#pragma unroll
+        for (int g = 0; g < GM; ++g) acc[g][e] += f[g] * v;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  if constexpr (AHEAD) {
+    for (; i < end; i += 8) {
+      if (i + 4 < end) {
+        load(i + 4, at, r1);
+        if (PAGED) at = find(min(i + 8, p.n - 1));
+      }
+      work(i, r0);
+      if (i + 4 >= end) break;
+      if (i + 8 < end) {
+        load(i + 8, at, r0);
+        if (PAGED) at = find(min(i + 12, p.n - 1));
+      }
+      work(i + 4, r1);
+    }
+  } else {
+    for (; i < end; i += 4) {
+      work(i, r0);
+      if (i + 4 < end) load(i + 4, find(i + 4), r0);
     }
   }
 
-  // merge the wave's lane groups by shuffles, the waves through LDS
+  // the lanes with the same dims, then the waves
+  l = sum_with<32>(sum_with<16>(l));
+  if (lane < GM) lds_ml[wid][lane] = float2{m, l};
 #pragma unroll
-  for (int g = 0; g < GM; ++g) {
-    float mx = fmaxf(m[g], __shfl_xor(m[g], 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float w = SIG ? 1.f : __builtin_amdgcn_exp2f(m[g] - mx);
-    float lg = l[g] * w;
-    lg += __shfl_xor(lg, 16, 64);
-    lg += __shfl_xor(lg, 32, 64);
+  for (int g = 0; g < GM; ++g)
 #pragma unroll
-    for (int e = 0; e < VE; ++e) {
-      float o = acc[g][e] * w;
-      o += __shfl_xor(o, 16, 64);
-      o += __shfl_xor(o, 32, 64);
-      if (lane < 16) lds_acc[wid][g][j * VE + e] = o;
+    for (int e = 0; e < 8; ++e) {
+      float o = acc[g][e];
+      if (LPK <= 8) o = sum_with<8>(o);
+      if (LPK <= 16) o = sum_with<16>(o);
+      o = sum_with<32>(o);
+      if (lane < LPK) lds_acc[wid][g][el * 8 + e] = o;
     }
-    if (lane == 0) lds_ml[wid][g] = float2{mx, lg};
-  }
   __syncthreads();
-  for (int i = threadIdx.x; i < heads * V; i += 256) {
-    const int g = i / V, e = i % V;
+  for (int n = threadIdx.x; n < heads * V; n += 256) {
+    const int g = n / V, e = n % V;
     float mx = NEG, sum = 0.f, o = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) mx = fmaxf(mx, lds_ml[w][g].x);
@@ -184,16 +362,46 @@ __global__ __launch_bounds__(256, GM * (KE + VE) <= 32 ? 4 : GM * (KE + VE) <= 6
       sum += f * lds_ml[w][g].y;
       o += f * lds_acc[w][g][e];
     }
-    if (a.n_split == 1) {
-      if (!SIG) o /= sum;
+    if (p.pieces == 1) {
+      if (!SIG) o = sum > 0.f ? o / sum : 0.f;
       if (a.gate) o *= sigmoid_f(bf2f(((const bf16_t*)a.gate)[seq * a.gate_stride + h0 + g]));
       ((bf16_t*)a.out)[seq * a.out_stride + (int64_t)(h0 + g) * V + e] = from_f<bf16_t>(o);
     } else {
-      const int64_t at = (int64_t)blockIdx.y * a.rows + row0 + g;
-      a.part[at * V + e] = o;
-      if (e == 0) a.part_ml[at] = SIG ? float2{0.f, 1.f} : float2{mx, sum};
+      const int64_t row = (int64_t)item * a.H + h0 + g;
+      a.part[row * V + e] = o;
+      if (e == 0) a.part_ml[row] = float2{mx, sum};
     }
   }
+}
+
+// Merge the pieces of one row: a workgroup of V threads per (head, sequence).
+template <bool SIG>
+__global__ __launch_bounds__(256) void merge_pieces_kernel(const GroupedArgs a, const int v) {
+  const int h = blockIdx.x, seq = blockIdx.y, e = threadIdx.x;
+  const Pieces p = find_pieces(a, seq, -1);
+  if (p.pieces == 1) return;  // written by the piece's workgroup
+  float m = NEG, l = 0.f, o = 0.f;
+  if (!SIG) {
+    // maxima and sums, a lane each
+    float sum = 0.f;
+    const int lane = threadIdx.x & 63;
+    for (int i = lane; i < p.pieces; i += 64) m = fmaxf(m, a.part_ml[(int64_t)(p.first + i) * a.H + h].x);
+    m = wave_max(m);
+    for (int i = lane; i < p.pieces; i += 64) {
+      const float2 ml = a.part_ml[(int64_t)(p.first + i) * a.H + h];
+      sum += ml.y * __builtin_amdgcn_exp2f(ml.x - m);
+    }
+    l = wave_sum(sum);
+  }
+#pragma unroll 8
+  for (int i = 0; i < p.pieces; ++i) {
+    const int64_t at = (int64_t)(p.first + i) * a.H + h;
+    const float w = SIG ? 1.f : __builtin_amdgcn_exp2f(a.part_ml[at].x - m);
+    o += w * a.part[at * v + e];
+  }
+  if (!SIG) o = l > 0.f ? o / l : 0.f;
+  if (a.gate) o *= sigmoid_f(bf2f(((const bf16_t*)a.gate)[seq * a.gate_stride + h]));
+  ((bf16_t*)a.out)[seq * a.out_stride + (int64_t)h * v + e] = from_f<bf16_t>(o);
 }
 
 // Any dtype and size: a workgroup per (token, head), its 4 waves stride over the keys,
@@ -303,34 +511,38 @@ __global__ __launch_bounds__(256) void cache_keys_values_kernel(
     v_cache[slots[n] * v_units + u - k_units] = v[n * stride + u - k_units];
 }
 
-template <int KE, int VE, bool SIG>
-static void launch_decode(const GroupedArgs& a, int seqs, int gm, hipStream_t stream) {
-  if (KE + VE > 16 && gm > 4) gm = 4;
+template <int DN, int VN, int GM, bool SIG>
+static void launch_decode(const GroupedArgs& a, hipStream_t stream) {
   const int group = a.H / a.G;
-  const dim3 grid(seqs * a.G * ((group + gm - 1) / gm), a.n_split);
-  if (gm == 1)
-    grouped_decode_kernel<KE, VE, 1, SIG><<<grid, 256, 0, stream>>>(a);
-  else if (gm == 2)
-    grouped_decode_kernel<KE, VE, 2, SIG><<<grid, 256, 0, stream>>>(a);
-  else if (gm == 4)
-    grouped_decode_kernel<KE, VE, 4, SIG><<<grid, 256, 0, stream>>>(a);
-  else if constexpr (KE + VE <= 16)
-    grouped_decode_kernel<KE, VE, 8, SIG><<<grid, 256, 0, stream>>>(a);
+  const int grid = (a.pieces + a.seqs) * a.G * ((group + GM - 1) / GM);
+  const bool paged = a.kv_block >= 16 && (a.kv_block & (a.kv_block - 1)) == 0;
+  auto kernel = paged ? grouped_decode_kernel<DN, VN, GM, SIG, true>
+                      : grouped_decode_kernel<DN, VN, GM, SIG, false>;
+  kernel<<<grid, 256, 0, stream>>>(a);
 }
 
-template <int KE, int VE>
-static bool launch_decode(const GroupedArgs& a, int seqs, int gm, hipStream_t stream) {
-  (a.sigmoid ? launch_decode<KE, VE, true> : launch_decode<KE, VE, false>)(a, seqs, gm, stream);
+template <int DN, int VN>
+static bool launch_decode(const GroupedArgs& a, int gm, hipStream_t stream) {
+  if (gm == 1)
+    (a.sigmoid ? launch_decode<DN, VN, 1, true> : launch_decode<DN, VN, 1, false>)(a, stream);
+  else if (gm == 4)
+    (a.sigmoid ? launch_decode<DN, VN, 4, true> : launch_decode<DN, VN, 4, false>)(a, stream);
+  else if (gm == 8)
+    (a.sigmoid ? launch_decode<DN, VN, 8, true> : launch_decode<DN, VN, 8, false>)(a, stream);
+  else
+    return false;
+  if (a.pieces == 0) return true;
+  auto merge = a.sigmoid ? merge_pieces_kernel<true> : merge_pieces_kernel<false>;
+  merge<<<dim3(a.H, a.seqs), 64 * VN, 0, stream>>>(a, 64 * VN);
   return true;
 }
 
-template <int KE>
-static bool launch_decode_v(const GroupedArgs& a, int v, int seqs, int gm,
-                            hipStream_t stream) {
+template <int DN>
+static bool launch_decode_v(const GroupedArgs& a, int v, int gm, hipStream_t stream) {
   switch (v) {
-    case 64: return launch_decode<KE, 4>(a, seqs, gm, stream);
-    case 128: return launch_decode<KE, 8>(a, seqs, gm, stream);
-    case 256: return launch_decode<KE, 16>(a, seqs, gm, stream);
+    case 64: return launch_decode<DN, 1>(a, gm, stream);
+    case 128: return launch_decode<DN, 2>(a, gm, stream);
+    case 256: return launch_decode<DN, 4>(a, gm, stream);
     default: return false;
   }
 }
@@ -352,20 +564,14 @@ static bool launch_plain(const GroupedArgs& a, int d, int v, int tokens, hipStre
 
 extern "C" {
 
-// gm: query heads of one key/value head per workgroup, 1, 2, 4 or 8 (8 if d + v <= 256)
-bool launch_grouped_decode(const GroupedArgs* a, int d, int v, int seqs, int gm,
-                           hipStream_t stream) {
-  bool ok = false;
+// gm: query heads of one key/value head per workgroup, 1, 4 or 8
+bool launch_grouped_decode(const GroupedArgs* a, int d, int v, int gm, hipStream_t stream) {
   switch (d) {
-    case 64: ok = launch_decode_v<4>(*a, v, seqs, gm, stream); break;
-    case 128: ok = launch_decode_v<8>(*a, v, seqs, gm, stream); break;
-    case 256: ok = launch_decode_v<16>(*a, v, seqs, gm, stream); break;
+    case 64: return launch_decode_v<1>(*a, v, gm, stream);
+    case 128: return launch_decode_v<2>(*a, v, gm, stream);
+    case 256: return launch_decode_v<4>(*a, v, gm, stream);
+    default: return false;
   }
-  if (ok && a->n_split > 1) {
-    const SplitOut out = {a->out, a->gate, a->out_stride, a->gate_stride, a->H, a->sigmoid};
-    launch_split_combine(&out, a->part, a->part_ml, a->rows, v, a->n_split, stream);
-  }
-  return ok;
 }
 
 bool launch_grouped_plain(bool bf16, const GroupedArgs* a, int d, int v, int tokens,

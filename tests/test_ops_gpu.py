@@ -125,6 +125,41 @@ def test_decode_attn(G):
 
 
 @requires_gpu
+@pytest.mark.parametrize("block", [8, 16, 24, 64])
+@pytest.mark.parametrize("H,G", [(8, 8), (7, 1), (6, 2), (16, 2)])
+@pytest.mark.parametrize("lens", [
+    [1], [32, 0, 33], [31, 64, 65, 700, 128, 129, 1, 3000], [40, 7] * 70, [100] * 3 + [5] * 1100,
+], ids=["one", "none", "ragged", "over_64", "whole"])
+def test_decode_pieces(block, H, G, lens):
+    """Steps cut into pieces and merged, or with whole sequences; what no token has written
+    is NaN."""
+    torch.manual_seed(len(lens))
+    need = [-(-n // block) for n in lens]
+    order = torch.randperm(sum(need) + 1)
+    tables = torch.zeros(len(lens), max(need) + 2, dtype=torch.int32)
+    kc = torch.full((len(order), block, G, 128), float("nan"), device="cuda").bfloat16()
+    vc, at, rows = kc.clone(), 0, []
+    for b, (n, k) in enumerate(zip(lens, need)):
+        tables[b, :k] = order[at : at + k]
+        p = torch.arange(n)
+        rows.append(order[at : at + k][p // block] * block + p % block)
+        at += k
+    slots = torch.cat(rows).cuda()
+    for c in (kc, vc):
+        c.view(-1, G, 128)[slots] = torch.randn(len(slots), G, 128, device="cuda").bfloat16()
+    q = torch.randn(len(lens), H, 128, device="cuda").bfloat16()
+    out = hip().attention_decode_raw(
+        q, kc, vc, tables.cuda(), torch.tensor(lens).cuda(), 0.09
+    ).float()
+    keys, values = (c.view(-1, G, 128).float() for c in (kc, vc))
+    for b in {*range(min(10, len(lens))), len(lens) - 1}:
+        k, v = (c[rows[b].cuda()].repeat_interleave(H // G, 1) for c in (keys, values))
+        w = torch.softmax((k * q[b].float()).sum(-1) * 0.09, 0)
+        # fp32 but for the result: 2^-9 of values up to 5
+        assert maxerr(out[b], (w.unsqueeze(-1) * v).sum(0)) < 0.012, (b, lens[b])
+
+
+@requires_gpu
 def test_mfma_fragment_layout_probe():
     """The assumed A/B/D lane maps for v_mfma_f32_32x32x16_bf16 must
     reproduce a plain matmul (asymmetric operands per guide G9/rule 16)."""
