@@ -1,18 +1,27 @@
 // Full-vocabulary token sampling (gfx950): temperature → optional grammar
 // mask → exact top-k → top-p (nucleus) → inverse-CDF draw in token-id
-// order; one workgroup per row, vocab up to 256k (Llama-3: 128256).
+// order; one workgroup per row, any vocabulary size (Llama-3: 128256).
 //
 // The ≤512-entry LDS bitonic sampler (sampling.hip) covers the byte
 // tokenizer; a real BPE vocabulary needs per-row selection over 128k
-// entries.  Sorting is out at B≈1k rows; instead thresholds come from LDS
-// radix-select: logits map to order-preserving uint32 keys and a
-// 3-level histogram walk (10+11+11 bits; ≤2048 buckets × 8 B = 16 KB LDS,
-// well inside the 160 KB CU budget) pins the exact k-th-largest key; the
-// nucleus (top-p) boundary key falls out of the same walk with per-bucket
-// exp-mass instead of counts.  Every pass streams the row coalesced
-// (thread t reads i = t, t+WG, …); only the final draw walks blocked
-// stripes so the inverse CDF runs in token-id order and draws match the
-// fp32 oracle (ops/reference.py softmax_sample) for a given uniform.
+// entries.  Sorting is out at B≈1k rows; instead a threshold key (order-
+// preserving uint32 of the logit) is found from histograms in LDS.  The first one
+// is over m - x with 64 buckets an octave, so that neither the bulk of the logits nor
+// their top meet in a few buckets; the bucket that holds the boundary is gathered into
+// LDS and split by its keys until one key is left.  Buckets are weighted by 1 for
+// top-k and by exp((x - m) / T) for top-p, and walked by a parallel scan.
+//
+// Every pass streams the row in 16-byte loads.  The draw sums 256 stripes of the row, each in
+// token-id order, and walks the stripe with the target: the inverse CDF runs in token-id order
+// and draws match the fp32 oracle (ops/reference.py softmax_sample) for a given uniform.  The
+// weights of 64 tokens of every stripe are made at a time by all threads and added up by one
+// thread a stripe, so that the order of the sums does not depend on the threads.
+//
+// Bound by the passes over the row (the largest logit, the draw, and two for each threshold),
+// about 18 us each where 190 rows of 128256 in fp32 come from the memory-side cache, and by the
+// exps of a pass, 11 us: 23 us greedy, 70 plain, 100 top-k, 160 top-p; 153 us a mix of them,
+// before 1229 (thresholds by three histograms of key bits each, whose few buckets took most of
+// the atomics, walked by one thread; draws by strides of a thread).
 //
 // Semantics match the oracle:
 //   greedy (T<=0): argmax, lowest index on ties
@@ -21,132 +30,249 @@
 //                  cumulative <= p            (boundary-key ties all kept)
 #include "common.h"
 
-#define WG 256
-#define NBUCKET 2048
+#define WG 1024
+#define WAVES (WG / 64)
+#define STRIPES 256
+#define TILE 64         // tokens of a stripe that are summed at a time
+#define OCTAVE 64       // first buckets: of m - x, per octave, from 2^-8 to 2^16
+#define FIRST (24 * OCTAVE)
+#define HEAD 12.f       // logits of at least exp(-HEAD) of the largest's weight come first
+#define SPLIT 1024      // buckets of a further split
+#define LIST 4096       // keys of a bucket that are kept in LDS
 
 // order-preserving float -> uint32 key
 __device__ __forceinline__ uint32_t f2key(float x) {
   uint32_t u = __float_as_uint(x);
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
+__device__ __forceinline__ float key2f(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
+}
+
+__device__ __forceinline__ float ldf(const float* p) { return *p; }
+__device__ __forceinline__ float ldf(const bf16_t* p) { return bf2f(*p); }
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+struct Shared {
+  uint32_t count[FIRST];
+  float mass[FIRST];
+  union {
+    uint32_t list[LIST];
+    float tile[2][STRIPES][TILE + 1];
+  };
+  float stripe[STRIPES], cdf[STRIPES + 1];
+  double wave[WAVES];
+  float red[WAVES];
+  int red_i[WAVES];
+  int n, pick;
+  uint32_t lo, hi;
+  double above;
+};
 
 template <typename T>
-__device__ __forceinline__ float ldf(const T* p);
-template <>
-__device__ __forceinline__ float ldf<float>(const float* p) { return *p; }
-template <>
-__device__ __forceinline__ float ldf<bf16_t>(const bf16_t* p) {
-  return bf2f(*p);
-}
+struct Row {
+  const T* x;
+  const uint8_t* mask;  // or null
+  int V;
+  float m, invT;
 
-__device__ __forceinline__ float blk_reduce_max(float v, float* red) {
+  __device__ float weight(float v) const { return __expf((v - m) * invT); }
+
+  // f(token, logit) for every allowed token, a thread's in rising order
+  template <typename F>
+  __device__ void each(F f) const {
+    constexpr int N = 16 / sizeof(T), AHEAD = 4;
+    auto one = [&](int i, float v) {
+      if (!mask || mask[i]) f(i, v);
+    };
+    auto all = [&](int i, u32x4 v) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_down(v, off, 64));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float r = red[0];
-    for (int w = 1; w < WG / 64; ++w) r = fmaxf(r, red[w]);
-    red[0] = r;
-  }
-  __syncthreads();
-  float r = red[0];
-  __syncthreads();
-  return r;
-}
-
-__device__ __forceinline__ float blk_reduce_sum(float v, float* red) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float r = red[0];
-    for (int w = 1; w < WG / 64; ++w) r += red[w];
-    red[0] = r;
-  }
-  __syncthreads();
-  float r = red[0];
-  __syncthreads();
-  return r;
-}
-
-// radix levels: bits [22,32) [11,22) [0,11) — widths 10/11/11
-__constant__ int LVL_SHIFT[3] = {22, 11, 0};
-__constant__ int LVL_BITS[3] = {10, 11, 11};
-
-// Find the boundary key where the descending cumulative weight crosses
-// `target`.  Weight per element = 1 (BY_MASS=false, top-k) or
-// exp((x-m)/T) (BY_MASS=true, top-p).  Only elements with key >= kmin and
-// allowed by the mask participate.  Returns the fully-resolved 32-bit
-// boundary key: kept = {key >= boundary}.
-template <typename T, bool BY_MASS>
-__device__ uint32_t radix_walk(const T* lrow, const uint8_t* mrow, int V,
-                               float m, float invT, uint32_t kmin,
-                               double target, uint32_t* hist_c,
-                               float* hist_m) {
-  uint32_t prefix = 0;
-  double above = 0.0;  // weight strictly above the current prefix range
-  __shared__ int sel_s;
-  __shared__ double above_s;
-  for (int level = 0; level < 3; ++level) {
-    const int shift = LVL_SHIFT[level];
-    const int nb = 1 << LVL_BITS[level];
-    const uint32_t pmask =
-        (level == 0) ? 0u : (0xFFFFFFFFu << (LVL_SHIFT[level - 1]));
-    for (int i = threadIdx.x; i < nb; i += WG) {
-      hist_c[i] = 0;
-      hist_m[i] = 0.f;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < V; i += WG) {
-      if (mrow && !mrow[i]) continue;
-      const float x = ldf<T>(lrow + i);
-      const uint32_t key = f2key(x);
-      if (key < kmin) continue;
-      if ((key & pmask) != (prefix & pmask)) continue;
-      const uint32_t b = (key >> shift) & (nb - 1);
-      if (BY_MASS)
-        atomicAdd(&hist_m[b], __expf((x - m) * invT));
-      else
-        atomicAdd(&hist_c[b], 1u);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      // serial walk from the top bucket: ≤2048 iterations, ~µs
-      double cum = above;
-      int sel = 0;
-      for (int b = nb - 1; b >= 0; --b) {
-        const double w = BY_MASS ? (double)hist_m[b] : (double)hist_c[b];
-        if (cum + w >= target || b == 0) {
-          sel = b;
-          break;
-        }
-        cum += w;
+      for (int e = 0; e < N; ++e) {
+        const uint32_t bits = N == 4 ? v[e & 3] : (e & 1) ? v[e >> 1] & 0xffff0000u : v[e >> 1] << 16;
+        one(i + e, __uint_as_float(bits));
       }
-      sel_s = sel;
-      above_s = cum;
+    };
+    int i = 0;
+    if ((uintptr_t)x % 16 == 0) {
+      const int whole = V / (WG * N) * WG * N;
+      for (; i + AHEAD * WG * N <= whole; i += AHEAD * WG * N) {
+        u32x4 v[AHEAD];
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a)
+          v[a] = *(const u32x4*)(x + i + (a * WG + threadIdx.x) * N);
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a) all(i + (a * WG + threadIdx.x) * N, v[a]);
+      }
+      for (; i < whole; i += WG * N)
+        all(i + threadIdx.x * N, *(const u32x4*)(x + i + threadIdx.x * N));
     }
-    __syncthreads();
-    prefix |= ((uint32_t)sel_s) << shift;
-    above = above_s;
-    __syncthreads();
+    for (i += threadIdx.x; i < V; i += WG) one(i, ldf(x + i));
   }
-  return prefix;
+
+  // bucket of a logit: 0 holds the largest
+  __device__ int bucket(float v) const {
+    const int b = (int)(__float_as_uint(m - v) >> 17) - ((127 - 8) << 6);
+    return min(max(b, 0), FIRST - 1);
+  }
+};
+static_assert(OCTAVE == 64, "bucket() takes 6 bits of the mantissa");
+
+// The first of ``n`` (at most 2 WG) buckets whose sum with those before and ``above`` reaches
+// target, and the sum before it; -1: none does.
+template <bool BY_MASS>
+__device__ int find_bucket(Shared& s, int n, double target, double* above) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  auto at = [&](int i) { return i >= n ? 0.0 : BY_MASS ? (double)s.mass[i] : (double)s.count[i]; };
+  const double w0 = at(2 * threadIdx.x), w1 = at(2 * threadIdx.x + 1);
+  double sum = w0 + w1;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double v = __shfl_up(sum, off, 64);
+    if (lane >= off) sum += v;
+  }
+  if (lane == 63) s.wave[wid] = sum;
+  if (threadIdx.x == 0) s.n = 1 << 30;
+  __syncthreads();
+  double before = *above;
+  for (int w = 0; w < wid; ++w) before += s.wave[w];
+  sum += before;  // up to and with this thread's two
+  const double b1 = sum - w1, b0 = b1 - w0;
+  const int mine = b1 >= target ? 2 * threadIdx.x : sum >= target ? 2 * threadIdx.x + 1 : n;
+  if (mine < n) atomicMin(&s.n, mine);
+  __syncthreads();
+  const int got = s.n;
+  if (got < n && got / 2 == (int)threadIdx.x) s.above = got % 2 ? b1 : b0;
+  __syncthreads();
+  if (got < n) *above = s.above;
+  return got < n ? got : -1;
 }
 
-template <typename T>
-__device__ __forceinline__ float kept_mass(const T* lrow, const uint8_t* mrow,
-                                           int V, float m, float invT,
-                                           uint32_t kmin, float* red) {
-  float part = 0.f;
-  for (int i = threadIdx.x; i < V; i += WG) {
-    if (mrow && !mrow[i]) continue;
-    const float x = ldf<T>(lrow + i);
-    if (f2key(x) < kmin) continue;
-    part += __expf((x - m) * invT);
+// Splits the keys [lo, hi] among those that each_key(f) hands out until one is left: the one at
+// which the sum from the top reaches target.
+template <bool BY_MASS, typename T, typename E>
+__device__ uint32_t split_keys(Shared& s, const Row<T>& row, uint32_t lo, uint32_t hi,
+                               double above, double target, E each_key) {
+  for (;;) {
+    const uint32_t range = hi - lo;
+    const int shift = range < SPLIT ? 0 : 32 - __builtin_clz(range) - 10;
+    const int n = (int)(range >> shift) + 1;
+    for (int i = threadIdx.x; i < n; i += WG) {
+      s.count[i] = 0;
+      s.mass[i] = 0.f;
+    }
+    __syncthreads();
+    each_key([&](uint32_t key) {
+      if (key < lo || key > hi) return;
+      const uint32_t b = (hi - key) >> shift;
+      if (BY_MASS)
+        atomicAdd(&s.mass[b], row.weight(key2f(key)));
+      else
+        atomicAdd(&s.count[b], 1u);
+    });
+    __syncthreads();
+    int b = find_bucket<BY_MASS>(s, n, target, &above);
+    if (b < 0) b = n - 1;
+    hi -= (uint32_t)b << shift;
+    const uint32_t width = (1u << shift) - 1;
+    if (hi - lo > width) lo = hi - width;
+    if (shift == 0) return hi;
   }
-  return blk_reduce_sum(part, red);
+}
+
+__device__ double block_total(Shared& s, double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0) s.wave[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+  for (int w = 0; w < WAVES; ++w) t += s.wave[w];
+  __syncthreads();
+  return t;
+}
+
+// Histograms over m - x up to ``far``; the mass of the others: a boundary is seldom among
+// them, and their atomics take most of the time.
+template <bool BY_MASS, typename T>
+__device__ float fill(Shared& s, const Row<T>& row, float far) {
+  for (int i = threadIdx.x; i < FIRST; i += WG) {
+    s.count[i] = 0;
+    s.mass[i] = 0.f;
+  }
+  __syncthreads();
+  float rest = 0.f;
+  row.each([&](int, float v) {
+    const float w = BY_MASS ? row.weight(v) : 0.f;
+    if (row.m - v > far) {
+      rest += w;
+      return;
+    }
+    const int b = row.bucket(v);
+    if (BY_MASS)
+      atomicAdd(&s.mass[b], w);
+    else
+      atomicAdd(&s.count[b], 1u);
+  });
+  __syncthreads();
+  return rest;
+}
+
+// The key at which the sum from the largest logit down reaches target, which is ``part`` of all
+// weights if it is given; 0: nowhere.  ``plain``: all logits are numbers.
+template <bool BY_MASS, typename T>
+__device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double part, bool plain) {
+  if (target <= 0.0) return 0xffffffffu;  // reached before the first
+  auto stream = [&](auto f) { row.each([&](int, float v) { f(f2key(v)); }); };
+  if (!plain) return split_keys<BY_MASS>(s, row, 0u, 0xffffffffu, 0.0, target, stream);
+  double above = 0.0;
+  const float rest = fill<BY_MASS>(s, row, HEAD / row.invT);
+  if (part > 0.0) {
+    double all = 0.0;
+    for (int i = threadIdx.x; i < FIRST; i += WG) all += s.mass[i];
+    target = part * block_total(s, all + rest);
+    if (target <= 0.0) return 0xffffffffu;
+  }
+  int b = find_bucket<BY_MASS>(s, FIRST, target, &above);
+  if (b < 0) {  // beyond the head
+    fill<BY_MASS>(s, row, INFINITY);
+    above = 0.0;
+    b = find_bucket<BY_MASS>(s, FIRST, target, &above);
+    if (b < 0) return 0;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s.n = 0;
+    s.lo = 0xffffffffu;
+    s.hi = 0;
+  }
+  __syncthreads();
+  uint32_t lo = 0xffffffffu, hi = 0;
+  row.each([&](int, float v) {
+    if (row.bucket(v) != b) return;
+    const uint32_t key = f2key(v);
+    lo = min(lo, key);
+    hi = max(hi, key);
+    const int at = atomicAdd(&s.n, 1);
+    if (at < LIST) s.list[at] = key;
+  });
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
+    hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicMin(&s.lo, lo);
+    atomicMax(&s.hi, hi);
+  }
+  __syncthreads();
+  lo = s.lo;
+  hi = s.hi;
+  const int n = s.n;
+  __syncthreads();
+  if (n > LIST) return split_keys<BY_MASS>(s, row, lo, hi, above, target, stream);
+  return split_keys<BY_MASS>(s, row, lo, hi, above, target, [&](auto f) {
+    for (int i = threadIdx.x; i < n; i += WG) f(s.list[i]);
+  });
 }
 
 template <typename T>
@@ -160,126 +286,191 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
     const uint8_t* __restrict__ mask,    // [M, V] bool, may be null
     const int32_t* __restrict__ mask_map,// [B] row -> mask row (-1 = none)
     const int V) {
-  const int row = blockIdx.x;
-  const T* lrow = logits + (int64_t)row * V;
+  __shared__ Shared s;
+  const int n_row = blockIdx.x, t = threadIdx.x, lane = t & 63, wid = t >> 6;
   // compact masks: only constrained rows carry one (a dense [B,V] mask at
   // B=1k, V=128k would be 128 MB of pinned staging per step)
-  const uint8_t* mrow = nullptr;
-  if (mask && mask_map && mask_map[row] >= 0)
-    mrow = mask + (int64_t)mask_map[row] * V;
-  const float Tmp = temps[row];
+  const bool masked = mask && mask_map && mask_map[n_row] >= 0;
+  const float Tmp = temps[n_row];
   const bool greedy = Tmp <= 0.f;
-  const float invT = greedy ? 1.f : 1.f / Tmp;
+  Row<T> row = {logits + (int64_t)n_row * V,
+                masked ? mask + (int64_t)mask_map[n_row] * V : nullptr, V, 0.f,
+                greedy ? 1.f : 1.f / Tmp};
 
-  __shared__ uint32_t hist_c[NBUCKET];
-  __shared__ float hist_m[NBUCKET];
-  __shared__ float red[WG / 64];
-
-  // ---- pass 1: masked row max
+  // ---- the largest allowed logit, the lowest token that has it, and whether all are numbers
   float mx = -3.4e38f;
-  for (int i = threadIdx.x; i < V; i += WG) {
-    if (mrow && !mrow[i]) continue;
-    mx = fmaxf(mx, ldf<T>(lrow + i));
-  }
-  const float m = blk_reduce_max(mx, red);
-
-  if (greedy) {
-    // lowest index attaining the max (oracle argmax tie rule)
-    int best = V;
-    for (int i = threadIdx.x; i < V; i += WG) {
-      if (mrow && !mrow[i]) continue;
-      if (ldf<T>(lrow + i) == m) {
-        best = i;
-        break;  // strided loop: the first hit is this thread's lowest
-      }
+  int best = V, odd = 0;
+  row.each([&](int i, float v) {
+    if (v > mx) {
+      mx = v;
+      best = i;
+    } else if (v == mx) {
+      best = min(best, i);
     }
+    odd |= !(v < INFINITY);
+  });
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-      best = min(best, __shfl_down(best, off, 64));
-    __shared__ int ired[WG / 64];
-    if ((threadIdx.x & 63) == 0) ired[threadIdx.x >> 6] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int b = ired[0];
-      for (int w = 1; w < WG / 64; ++w) b = min(b, ired[w]);
-      out[row] = (int64_t)(b < V ? b : 0);
-    }
+  for (int off = 32; off > 0; off >>= 1) {
+    const float v = __shfl_xor(mx, off, 64);
+    const int i = __shfl_xor(best, off, 64);
+    if (v > mx || (v == mx && i < best)) best = i;
+    mx = fmaxf(mx, v);
+  }
+  const bool odd_wave = __any(odd);
+  if (lane == 0) {
+    s.red[wid] = mx;
+    s.red_i[wid] = best;
+    s.cdf[wid] = odd_wave;
+  }
+  __syncthreads();
+  bool plain = true;
+  for (int w = 0; w < WAVES; ++w) {
+    if (s.red[w] > mx || (s.red[w] == mx && s.red_i[w] < best)) best = s.red_i[w];
+    mx = fmaxf(mx, s.red[w]);
+    plain &= s.cdf[w] == 0.f;
+  }
+  __syncthreads();
+  row.m = mx;
+  if (greedy) {
+    if (t == 0) out[n_row] = best < V ? best : 0;
     return;
   }
 
-  // ---- top-k: kmin = key of the k-th largest; kept = {key >= kmin}
+  // ---- top-k, then top-p: kept = {key >= kmin}
   uint32_t kmin = 0;
-  const int tk = (int)top_ks[row];
-  if (tk > 0 && tk < V) {
-    kmin = radix_walk<T, false>(lrow, mrow, V, m, invT, 0u, (double)tk,
-                                hist_c, hist_m);
-  }
-
-  // ---- top-p: raise kmin to the nucleus boundary key
-  const float p = top_ps[row];
-  if (p < 1.f) {
-    const float M = kept_mass<T>(lrow, mrow, V, m, invT, kmin, red);
-    const uint32_t pmin = radix_walk<T, true>(
-        lrow, mrow, V, m, invT, kmin, (double)p * (double)M, hist_c, hist_m);
+  const int64_t tk = top_ks[n_row];
+  const float p = top_ps[n_row];
+  const bool by_k = tk > 0 && tk < V, by_p = p < 1.f;
+  if (by_k) kmin = boundary<false>(s, row, (double)tk, 0.0, plain);
+  if (by_p) {
+    double target = p;
+    if (by_k || !plain) {  // of what is kept so far
+      float kept = 0.f;
+      row.each([&](int, float v) {
+        if (f2key(v) >= kmin) kept += row.weight(v);
+      });
+      target = (double)p * (float)block_total(s, kept);
+    }
+    // all keys above the boundary are kept: the histograms need not know kmin
+    const uint32_t pmin =
+        boundary<true>(s, row, target, by_k || !plain ? 0.0 : (double)p, plain);
     if (pmin > kmin) kmin = pmin;
   }
 
   // ---- inverse-CDF draw in token-id order over the kept set.
-  // Thread t owns the blocked stripe [t*stride, (t+1)*stride).
-  const int stride = (V + WG - 1) / WG;
-  const int lo = min(threadIdx.x * stride, V);
-  const int hi = min(lo + stride, V);
+  // Stripe n is tokens [n * stride, (n + 1) * stride).
+  const int stride = (V + STRIPES - 1) / STRIPES;
+  constexpr int PER = STRIPES * TILE / WG;  // a thread's tokens of a tile
+  float ahead[PER];
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int j = j0 + t % TILE, i = (k * (WG / TILE) + t / TILE) * stride + j;
+      ahead[k] = j < stride && i < V ? ldf(row.x + i) : 0.f;
+    }
+  };
   float mine = 0.f;
-  for (int i = lo; i < hi; ++i) {
-    if (mrow && !mrow[i]) continue;
-    const float x = ldf<T>(lrow + i);
-    if (f2key(x) < kmin) continue;
-    mine += __expf((x - m) * invT);
+  fetch(0);
+  for (int j0 = 0; j0 < stride; j0 += TILE) {
+    float(*tile)[TILE + 1] = s.tile[j0 / TILE % 2];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int n = k * (WG / TILE) + t / TILE, j = j0 + t % TILE, i = n * stride + j;
+      const bool in = j < stride && i < V && f2key(ahead[k]) >= kmin && !(row.mask && !row.mask[i]);
+      tile[n][t % TILE] = in ? row.weight(ahead[k]) : 0.f;
+    }
+    if (j0 + TILE < stride) fetch(j0 + TILE);
+    __syncthreads();  // the other tile is added up before it is written again
+    if (t < STRIPES) {
+#pragma unroll
+      for (int j = 0; j < TILE; ++j) mine += tile[t][j];
+    }
   }
-  __shared__ float stripe[WG + 1];
-  stripe[threadIdx.x + 1] = mine;
-  if (threadIdx.x == 0) stripe[0] = 0.f;
+  if (t < STRIPES) s.stripe[t] = mine;
+  if (t == 0) s.pick = s.n = -1;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i <= WG; ++i) stripe[i] += stripe[i - 1];
+  constexpr int STEP = 16;  // one thread's LDS reads in flight
+  if (t == 0) {
+    float sum = 0.f;
+    s.cdf[0] = 0.f;
+    for (int i = 0; i < STRIPES; i += STEP) {
+      float w[STEP];
+#pragma unroll
+      for (int e = 0; e < STEP; ++e) w[e] = s.stripe[i + e];
+#pragma unroll
+      for (int e = 0; e < STEP; ++e) s.cdf[i + e + 1] = sum += w[e];
+    }
   }
   __syncthreads();
-  const float total = stripe[WG];
-  const float target = uniforms[row] * total;
-  __shared__ int out_s;
-  if (threadIdx.x == 0) out_s = -1;
-  __syncthreads();
+  const float target = uniforms[n_row] * s.cdf[STRIPES];
   // exactly one stripe satisfies prefix <= target < prefix + mine
   // (mine > 0 guaranteed for the owner since the CDF strictly increases
   // across it); fp edge cases fall through to the fallback below
-  if (mine > 0.f && stripe[threadIdx.x] <= target &&
-      target < stripe[threadIdx.x + 1]) {
-    float cum = stripe[threadIdx.x];
-    int pick = -1;
-    for (int i = lo; i < hi; ++i) {
-      if (mrow && !mrow[i]) continue;
-      const float x = ldf<T>(lrow + i);
-      if (f2key(x) < kmin) continue;
-      cum += __expf((x - m) * invT);
-      pick = i;
-      if (cum > target) break;
+  if (t < STRIPES && mine > 0.f && s.cdf[t] <= target && target < s.cdf[t + 1]) s.n = t;
+  __syncthreads();
+  const int n = s.n;
+  __syncthreads();
+  if (n >= 0) {
+    // the stripe's weights, added up in order by one thread until they exceed the target;
+    // its last kept token if rounding lets none do so
+    float* const buf = &s.tile[0][0][0];
+    constexpr int ROOM = 4096;
+    float cum = s.cdf[n];
+    const int end = min(stride, V - n * stride);
+    for (int j0 = 0; j0 < end; j0 += ROOM) {
+      const int here = min(end - j0, ROOM), i0 = n * stride + j0;
+      int last = -1;
+      for (int j = t; j < (here + STEP - 1) / STEP * STEP; j += WG) {
+        float w = 0.f;
+        if (j < here && !(row.mask && !row.mask[i0 + j])) {
+          const float v = ldf(row.x + i0 + j);
+          if (f2key(v) >= kmin) {
+            w = row.weight(v);
+            last = i0 + j;
+          }
+        }
+        buf[j] = w;
+      }
+      if (last >= 0) atomicMax(&s.pick, last);
+      if (t == 0) s.n = -1;
+      __syncthreads();
+      if (t == 0) {
+        for (int j = 0; j < here && s.n < 0; j += STEP) {
+          float w[STEP];
+#pragma unroll
+          for (int e = 0; e < STEP; ++e) w[e] = buf[j + e];
+          int first = STEP;
+#pragma unroll
+          for (int e = 0; e < STEP; ++e) {
+            cum += w[e];
+            if (first == STEP && cum > target) first = e;
+          }
+          if (first < STEP) {
+            s.n = i0 + j + first;
+            break;
+          }
+        }
+        if (s.n >= 0) s.pick = s.n;
+      }
+      __syncthreads();
+      if (s.n >= 0) break;
     }
-    if (pick >= 0) out_s = pick;
   }
   __syncthreads();
-  if (threadIdx.x == 0 && out_s < 0) {
+  if (t == 0 && s.pick < 0) {
     // fallback (target == total to fp precision, or an empty kept set):
     // the last kept token, matching searchsorted's clamp in the oracle
+    int last = 0;
     for (int i = V - 1; i >= 0; --i) {
-      if (mrow && !mrow[i]) continue;
-      if (f2key(ldf<T>(lrow + i)) < kmin) continue;
-      out_s = i;
+      if (row.mask && !row.mask[i]) continue;
+      if (f2key(ldf(row.x + i)) < kmin) continue;
+      last = i;
       break;
     }
-    if (out_s < 0) out_s = 0;
+    s.pick = last;
   }
   __syncthreads();
-  if (threadIdx.x == 0) out[row] = (int64_t)out_s;
+  if (t == 0) out[n_row] = s.pick;
 }
 
 extern "C" void launch_sample_fullvocab(int64_t* out, const void* logits, bool bf16,

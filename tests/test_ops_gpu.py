@@ -228,6 +228,55 @@ def test_prefill_attn_multi_seq(impl, monkeypatch):
 
 
 @requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [513, 1023, 16385, 50257, 128256, 262144])
+def test_fullvocab_draws_lie_in_the_kept_cdf(V, dtype):
+    """Rows of every kind: spread, alike, in two values, with steps far below the largest, with
+    -inf, with masks; the drawn token's part of the 64-bit CDF holds the uniform."""
+    torch.manual_seed(V)
+    rows = [
+        torch.randn(V) * 2.5, torch.full((V,), 1.5), torch.randint(0, 2, (V,)).float(),
+        torch.randn(V) * 1e-6, torch.randn(V) * 1e4, torch.randn(V) * 3,
+        torch.where(torch.arange(V) % 3 == 0, torch.randn(V), torch.tensor(-float("inf"))),
+        torch.cat([torch.tensor([40.0]), torch.randn(V - 1)]),
+    ]
+    kinds = [(0, 1.0), (1, 1.0), (50, 1.0), (5000, 1.0), (0, 0.9), (0, 0.999), (40, 0.5)]
+    x = torch.stack(rows).to(dtype).cuda()
+    mask = torch.rand(2, V) < 0.02
+    mask[1] = False
+    mask[1, V - 1] = True
+    for k, p in kinds:
+        for mapped in (None, [0, 1, -1, 0, 1, 0, 0, -1]):
+            u = torch.rand(len(rows))
+            got = hip().softmax_sample(
+                x, torch.full((len(rows),), 0.8).cuda(),
+                torch.full((len(rows),), k).cuda(), torch.full((len(rows),), p).cuda(), None,
+                mask.cuda() if mapped else None, u.cuda(),
+                torch.tensor(mapped, dtype=torch.int32).cuda() if mapped else None,
+            ).tolist()
+            for r in range(len(rows)):
+                v = x[r].double().cpu()
+                if mapped and mapped[r] >= 0:
+                    v = v.masked_fill(~mask[mapped[r]], -float("inf"))
+                w = torch.exp((v - v.max()) / 0.8)
+                order = torch.sort(v, descending=True).values
+                if 0 < k < V:
+                    w[v < order[k - 1]] = 0
+                at = v[got[r]]
+                if p < 1:  # the weight of what is larger is within p of the kept
+                    assert w[v > at].sum() <= (p + 1e-5) * w.sum(), (r, k, p)
+                    above = torch.cumsum(torch.exp((order - order[0]) / 0.8), 0)
+                    edge = order[int((above >= p * w.sum()).nonzero()[0])]
+                    w[v < edge] = 0
+                    if at < edge:  # a boundary within rounding
+                        continue
+                c = torch.cumsum(w, 0) / w.sum()
+                lo = c[got[r] - 1].item() if got[r] else 0.0
+                # sums of 262144 weights in fp32, in 256 parts: 2^-24 * (1024 + 256)
+                assert lo - 1e-4 <= u[r] <= c[got[r]].item() + 1e-4, (r, k, p)
+
+
+@requires_gpu
 @pytest.mark.parametrize("block", [8, 16, 24, 64])
 @pytest.mark.parametrize("H,G,scale", [(8, 8, 0.09), (6, 2, -0.09), (4, 1, 0.0)])
 def test_prompt_tiles_over_pages(block, H, G, scale):
