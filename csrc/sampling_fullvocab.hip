@@ -17,11 +17,13 @@
 // weights of 64 tokens of every stripe are made at a time by all threads and added up by one
 // thread a stripe, so that the order of the sums does not depend on the threads.
 //
-// Bound by the passes over the row (the largest logit, the draw, and two for each threshold),
-// about 18 us each where 190 rows of 128256 in fp32 come from the memory-side cache, and by the
-// exps of a pass, 11 us: 23 us greedy, 70 plain, 100 top-k, 160 top-p; 153 us a mix of them,
-// before 1229 (thresholds by three histograms of key bits each, whose few buckets took most of
-// the atomics, walked by one thread; draws by strides of a thread).
+// Bound by the passes over the row: 20 us for the largest logit, 15 for the histogram of a top-k
+// and 62 for that of a top-p (30 of it weights, 32 atomics), 16 to gather the bucket, 15 for the
+// draw's sums, where 190 rows of 128256 in fp32 come from the memory-side cache.  Whole calls:
+// 23 us greedy, 60 plain, 93 top-k, 146 top-p or a mix; before 305, 421, 1129, 1302 and 1229
+// (thresholds by three histograms of key bits, whose few buckets met nearly all atomics, walked by
+// one thread; draws by strides of a thread).  Floating masses instead of whole ones in the
+// histogram took as long, a shared list of the bucket 25 us more.
 //
 // Semantics match the oracle:
 //   greedy (T<=0): argmax, lowest index on ties
@@ -38,7 +40,7 @@
 #define FIRST (24 * OCTAVE)
 #define HEAD 12.f       // logits of at least exp(-HEAD) of the largest's weight come first
 #define SPLIT 1024      // buckets of a further split
-#define LIST 4096       // keys of a bucket that are kept in LDS
+#define LIST 32         // keys of a bucket that a thread keeps in LDS
 
 // order-preserving float -> uint32 key
 __device__ __forceinline__ uint32_t f2key(float x) {
@@ -56,10 +58,10 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct Shared {
   uint32_t count[FIRST];
-  float mass[FIRST];
+  unsigned long long mass[FIRST];  // in units of 2^-44: integer atomics are the fast ones
   union {
-    uint32_t list[LIST];
-    float tile[2][STRIPES][TILE + 1];
+    uint32_t list[LIST][WG];
+    float tile[2][STRIPES][TILE + 4];
   };
   float stripe[STRIPES], cdf[STRIPES + 1];
   double wave[WAVES];
@@ -69,6 +71,14 @@ struct Shared {
   uint32_t lo, hi;
   double above;
 };
+
+#define UNIT 0x1p-44
+// a weight, at most 1, in units; what is no number weighs nothing
+__device__ __forceinline__ unsigned long long units(float w) {
+  const float hi = floorf(w * 0x1p24f);  // exact, and so is the rest
+  const float lo = (w - hi * 0x1p-24f) * 0x1p44f;
+  return ((unsigned long long)(uint32_t)hi << 20) + (uint32_t)lo;
+}
 
 template <typename T>
 struct Row {
@@ -116,6 +126,7 @@ struct Row {
     return min(max(b, 0), FIRST - 1);
   }
 };
+static_assert(TILE == 64, "a wave takes 64 tokens of a stripe");
 static_assert(OCTAVE == 64, "bucket() takes 6 bits of the mantissa");
 
 // The first of ``n`` (at most 2 WG) buckets whose sum with those before and ``above`` reaches
@@ -123,7 +134,7 @@ static_assert(OCTAVE == 64, "bucket() takes 6 bits of the mantissa");
 template <bool BY_MASS>
 __device__ int find_bucket(Shared& s, int n, double target, double* above) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  auto at = [&](int i) { return i >= n ? 0.0 : BY_MASS ? (double)s.mass[i] : (double)s.count[i]; };
+  auto at = [&](int i) { return i >= n ? 0.0 : BY_MASS ? s.mass[i] * UNIT : (double)s.count[i]; };
   const double w0 = at(2 * threadIdx.x), w1 = at(2 * threadIdx.x + 1);
   double sum = w0 + w1;
 #pragma unroll
@@ -159,14 +170,14 @@ __device__ uint32_t split_keys(Shared& s, const Row<T>& row, uint32_t lo, uint32
     const int n = (int)(range >> shift) + 1;
     for (int i = threadIdx.x; i < n; i += WG) {
       s.count[i] = 0;
-      s.mass[i] = 0.f;
+      s.mass[i] = 0;
     }
     __syncthreads();
     each_key([&](uint32_t key) {
       if (key < lo || key > hi) return;
       const uint32_t b = (hi - key) >> shift;
       if (BY_MASS)
-        atomicAdd(&s.mass[b], row.weight(key2f(key)));
+        atomicAdd(&s.mass[b], units(row.weight(key2f(key))));
       else
         atomicAdd(&s.count[b], 1u);
     });
@@ -197,7 +208,7 @@ template <bool BY_MASS, typename T>
 __device__ float fill(Shared& s, const Row<T>& row, float far) {
   for (int i = threadIdx.x; i < FIRST; i += WG) {
     s.count[i] = 0;
-    s.mass[i] = 0.f;
+    s.mass[i] = 0;
   }
   __syncthreads();
   float rest = 0.f;
@@ -209,7 +220,7 @@ __device__ float fill(Shared& s, const Row<T>& row, float far) {
     }
     const int b = row.bucket(v);
     if (BY_MASS)
-      atomicAdd(&s.mass[b], w);
+      atomicAdd(&s.mass[b], units(w));
     else
       atomicAdd(&s.count[b], 1u);
   });
@@ -228,7 +239,7 @@ __device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double
   const float rest = fill<BY_MASS>(s, row, HEAD / row.invT);
   if (part > 0.0) {
     double all = 0.0;
-    for (int i = threadIdx.x; i < FIRST; i += WG) all += s.mass[i];
+    for (int i = threadIdx.x; i < FIRST; i += WG) all += s.mass[i] * UNIT;
     target = part * block_total(s, all + rest);
     if (target <= 0.0) return 0xffffffffu;
   }
@@ -247,31 +258,28 @@ __device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double
   }
   __syncthreads();
   uint32_t lo = 0xffffffffu, hi = 0;
+  int n = 0;  // this thread's, in a column of the list
   row.each([&](int, float v) {
     if (row.bucket(v) != b) return;
     const uint32_t key = f2key(v);
     lo = min(lo, key);
     hi = max(hi, key);
-    const int at = atomicAdd(&s.n, 1);
-    if (at < LIST) s.list[at] = key;
+    if (n < LIST) s.list[n][threadIdx.x] = key;
+    ++n;
   });
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
-    hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
-  }
-  if ((threadIdx.x & 63) == 0) {
+  if (n) {
     atomicMin(&s.lo, lo);
     atomicMax(&s.hi, hi);
+    if (n > LIST) s.n = 1;
   }
   __syncthreads();
   lo = s.lo;
   hi = s.hi;
-  const int n = s.n;
+  const bool fits = s.n == 0;
   __syncthreads();
-  if (n > LIST) return split_keys<BY_MASS>(s, row, lo, hi, above, target, stream);
+  if (!fits) return split_keys<BY_MASS>(s, row, lo, hi, above, target, stream);
   return split_keys<BY_MASS>(s, row, lo, hi, above, target, [&](auto f) {
-    for (int i = threadIdx.x; i < n; i += WG) f(s.list[i]);
+    for (int i = 0; i < n; ++i) f(s.list[i][threadIdx.x]);
   });
 }
 
@@ -360,36 +368,51 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
   // ---- inverse-CDF draw in token-id order over the kept set.
   // Stripe n is tokens [n * stride, (n + 1) * stride).
   const int stride = (V + STRIPES - 1) / STRIPES;
-  constexpr int PER = STRIPES * TILE / WG;  // a thread's tokens of a tile
+  constexpr int PER = STRIPES * TILE / WG, ROWS = WG / TILE;  // a thread's tokens of a tile
+  // token of the thread's k-th of a tile: k * ROWS stripes on
+  const int i_first = wid * stride + lane;
   float ahead[PER];
   auto fetch = [&](int j0) {
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int j = j0 + t % TILE, i = (k * (WG / TILE) + t / TILE) * stride + j;
-      ahead[k] = j < stride && i < V ? ldf(row.x + i) : 0.f;
-    }
+    for (int k = 0; k < PER; ++k)
+      ahead[k] = ldf(row.x + min(k * ROWS * stride + j0 + i_first, V - 1));
   };
+  // comparing logits is comparing keys, but for zeros and what is no number
+  const float least = key2f(kmin);
+  const bool by_value = kmin == 0 || (least == least && least != 0.f);
+  const float from = kmin == 0 ? -INFINITY : least;
+  const bool even = V == STRIPES * stride;  // no stripe is shorter
   float mine = 0.f;
   fetch(0);
   for (int j0 = 0; j0 < stride; j0 += TILE) {
-    float(*tile)[TILE + 1] = s.tile[j0 / TILE % 2];
+    float(*tile)[TILE + 4] = s.tile[j0 / TILE % 2];
+    if (even && by_value && plain && !row.mask && j0 + TILE <= stride) {
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int n = k * (WG / TILE) + t / TILE, j = j0 + t % TILE, i = n * stride + j;
-      const bool in = j < stride && i < V && f2key(ahead[k]) >= kmin && !(row.mask && !row.mask[i]);
-      tile[n][t % TILE] = in ? row.weight(ahead[k]) : 0.f;
+      for (int k = 0; k < PER; ++k)
+        tile[k * ROWS + wid][lane] = ahead[k] >= from ? row.weight(ahead[k]) : 0.f;
+    } else {
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int i = k * ROWS * stride + j0 + i_first;
+        const bool in = j0 + lane < stride && i < V && f2key(ahead[k]) >= kmin &&
+                        !(row.mask && !row.mask[i]);
+        tile[k * ROWS + wid][lane] = in ? row.weight(ahead[k]) : 0.f;
+      }
     }
     if (j0 + TILE < stride) fetch(j0 + TILE);
     __syncthreads();  // the other tile is added up before it is written again
     if (t < STRIPES) {
+      float4 w[TILE / 4];
 #pragma unroll
-      for (int j = 0; j < TILE; ++j) mine += tile[t][j];
+      for (int j = 0; j < TILE / 4; ++j) w[j] = *(const float4*)&tile[t][4 * j];
+#pragma unroll
+      for (int j = 0; j < TILE / 4; ++j) mine = mine + w[j].x + w[j].y + w[j].z + w[j].w;
     }
   }
   if (t < STRIPES) s.stripe[t] = mine;
   if (t == 0) s.pick = s.n = -1;
   __syncthreads();
-  constexpr int STEP = 16;  // one thread's LDS reads in flight
+  constexpr int STEP = 32;  // one thread's LDS reads in flight
   if (t == 0) {
     float sum = 0.f;
     s.cdf[0] = 0.f;
@@ -438,7 +461,7 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
         for (int j = 0; j < here && s.n < 0; j += STEP) {
           float w[STEP];
 #pragma unroll
-          for (int e = 0; e < STEP; ++e) w[e] = buf[j + e];
+          for (int e = 0; e < STEP; e += 4) *(float4*)(w + e) = *(const float4*)(buf + j + e);
           int first = STEP;
 #pragma unroll
           for (int e = 0; e < STEP; ++e) {
