@@ -117,7 +117,7 @@ class FetolixLayer:
     def sublayers(self, h: torch.Tensor, batch: FlatBatch, cache: torch.Tensor) -> torch.Tensor:
         """attention(h) + glu(h), [N, width]."""
         m = self.mixer
-        proj = ops.linear(h, self.w_in)
+        proj = ops.step_linear(h, self.w_in)
         mixed = torch.empty(
             h.shape[0], m.out_dim + self.ff_pad, dtype=h.dtype, device=h.device
         )
@@ -277,7 +277,7 @@ class FetolixForCausalLM:
         for r, (i, enters) in enumerate(runs):
             layer = self.layers[i]
             if enters:
-                x = ops.linear(entry, self.loop_in).float()
+                x = ops.step_linear(entry, self.loop_in).float()
                 h = ops.layernorm(x, layer.norm, eps, self.dtype)
             y = layer.sublayers(h, batch, self.caches[r])
             if self.all_reduce is not None:
@@ -295,7 +295,7 @@ class FetolixForCausalLM:
                     x, y, layer.side_gate, batch.token_ids, self.side_embed, i * d
                 )
                 ops.residual_norm(
-                    x, ops.linear(s, layer.side_proj), eps, layer.side_norm, norm, out
+                    x, ops.step_linear(s, layer.side_proj), eps, layer.side_norm, norm, out
                 )
             else:
                 ops.residual_norm(x, y, eps, None, norm, out)
@@ -303,4 +303,4 @@ class FetolixForCausalLM:
             if trace is not None:
                 trace.append(x.clone())
         sel = ops.layernorm(x[batch.logit_rows], self.final_norm, eps, self.dtype)
-        return ops.linear(sel, self.embed).float()
+        return ops.step_linear(sel, self.embed).float()

@@ -153,12 +153,12 @@ class GatedDelta:
     def mix(self, h: torch.Tensor, batch: FlatBatch, state: Tuple[torch.Tensor, torch.Tensor]):
         """h [N, width] -> the heads ahead of W_o [N, heads * vdim] and, if there is one,
         the product beside the mixer's."""
-        proj = ops.linear(h, self.w_in, self.bias)
+        proj = ops.step_linear(h, self.w_in, self.bias)
 
         def section(name, second=None):
             at, rows = self.sections[name]
             x = proj[:, at : at + rows]
-            return x if second is None else ops.linear(x, second)
+            return x if second is None else ops.step_linear(x, second)
 
         out = ops.gated_delta(
             section("qkv"), self.conv, section("b"), section("a", self.w_a2), self.A_log,
@@ -170,4 +170,4 @@ class GatedDelta:
     def forward(self, h: torch.Tensor, batch: FlatBatch,
                 state: Tuple[torch.Tensor, torch.Tensor]) -> torch.Tensor:
         """h [N, width] -> this rank's part of [N, width]."""
-        return ops.linear(self.mix(h, batch, state)[0], self.w_out)
+        return ops.step_linear(self.mix(h, batch, state)[0], self.w_out)

@@ -278,7 +278,7 @@ class GroupedAttention:
         """h [N, width] -> out [N, heads * v] (row-strided): the heads ahead of W_o.
         Returns the product beside the mixer's, if there is one."""
         s, N = self.spec, h.shape[0]
-        proj = ops.linear(h, self.w_in, self.bias)
+        proj = ops.step_linear(h, self.w_in, self.bias)
         row, at = proj.stride(0), self.heads * self.d
         q = proj.as_strided((N, self.heads, self.d), (row, self.d, 1))
         if self.shaped:
@@ -313,4 +313,4 @@ class GroupedAttention:
     def forward(self, h: torch.Tensor, batch: FlatBatch,
                 cache: Tuple[torch.Tensor, torch.Tensor]) -> torch.Tensor:
         """h [N, width] -> this rank's part of [N, width]."""
-        return ops.linear(self.mix(h, batch, cache)[0], self.w_out, self.out_bias)
+        return ops.step_linear(self.mix(h, batch, cache)[0], self.w_out, self.out_bias)

@@ -189,7 +189,7 @@ class LatentAttention:
             batch.positions, batch.slot_mapping, self.cos_sin, cache, *low_rank,
         )
         if s.q_rank:
-            q = ops.linear(cq, self.uq)
+            q = ops.step_linear(cq, self.uq)
         q = q.as_strided((N, H, self.d + self.rot), (q.stride(0), self.d + self.rot, 1))
         out = out.as_strided((N, H, self.v), (out.stride(0), self.v, 1))
         expanded, row0 = batch.memo(

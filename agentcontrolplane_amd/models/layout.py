@@ -79,7 +79,7 @@ def summed_linear(x: torch.Tensor, blocks: List[torch.Tensor],
                   bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [N, sum of k] times the blocks of fuse_columns()."""
     at = blocks[0].shape[1]
-    y = ops.linear(x[:, :at], blocks[0], bias)
+    y = ops.step_linear(x[:, :at], blocks[0], bias)
     for b in blocks[1:]:
         ops.linear_add_(y, x[:, at : at + b.shape[1]], b)
         at += b.shape[1]

@@ -136,12 +136,12 @@ class LobuvikLayer:
         if self.glu:
             g = self.glu
             ops.clamped_glu(
-                ops.linear(h2[:, : self.width], self.gate_up), g.limit, g.alpha, g.offset,
+                ops.step_linear(h2[:, : self.width], self.gate_up), g.limit, g.alpha, g.offset,
                 mixed[:, m.out_dim :], g.cubic,
             )
         heads, bias = mixed[:, : m.out_dim], None
         if self.latent:
-            proj = ops.linear(h1, self.w_in)
+            proj = ops.step_linear(h1, self.w_in)
             q, kv, gate = (
                 proj[:, at : at + rows] if rows else None
                 for at, rows in (self.sections.get(n, (0, 0)) for n in ("q", "kv", "gate"))
@@ -320,4 +320,4 @@ class LobuvikForCausalLM:
             if trace is not None:
                 trace.append(x.clone())
         h = ops.layernorm(x[batch.logit_rows], self.final_norm, eps, self.dtype)
-        return ops.linear(h, self.head).float()
+        return ops.step_linear(h, self.head).float()

@@ -140,7 +140,7 @@ class MixtralForCausalLM(LlamaForCausalLM):
                 normed = ops.rmsnorm(x, lw.input_norm, cfg.rms_eps)
             else:
                 normed, residual = ops.fused_add_rmsnorm(x, residual, lw.input_norm, cfg.rms_eps)
-            qkv = ops.linear(normed, lw.qkv)
+            qkv = ops.step_linear(normed, lw.qkv)
             row = qkv.stride(0)
             q = qkv.as_strided((N, self.n_heads, self.head_dim), (row, self.head_dim, 1))
             k = qkv.as_strided(
@@ -154,7 +154,7 @@ class MixtralForCausalLM(LlamaForCausalLM):
                 self.k_caches[li], self.v_caches[li], self.cos_sin,
             )
             attn = self._attention(li, q, batch)
-            o = ops.linear(attn.reshape(N, qd), lw.o)
+            o = ops.step_linear(attn.reshape(N, qd), lw.o)
             if self.all_reduce is not None:
                 o = self.all_reduce(o)
             normed2, residual = ops.fused_add_rmsnorm(o, residual, lw.post_norm, cfg.rms_eps)
@@ -165,4 +165,4 @@ class MixtralForCausalLM(LlamaForCausalLM):
                 x = self.all_reduce(x)
         normed, _ = ops.fused_add_rmsnorm(x, residual, self.final_norm, cfg.rms_eps)
         sel = normed[batch.logit_rows]
-        return ops.linear(sel, self.lm_head).float()
+        return ops.step_linear(sel, self.lm_head).float()

@@ -136,12 +136,12 @@ class NoganexLayer:
     def mix(self, h: torch.Tensor, batch: FlatBatch, store):
         """(this rank's part of the mixer's result, its gate before the sigmoid)"""
         heads, gate = self.mixer.mix(h, batch, store)
-        return ops.linear(heads, self.mixer.w_out), gate
+        return ops.step_linear(heads, self.mixer.w_out), gate
 
     def feed_forward(self, h: torch.Tensor):
         """h [N, experts' padded width] -> (this rank's part of the result without the
         routed experts, its gate, those: rows and weights per (token, choice), or None)."""
-        proj = ops.linear(h[:, : self.width], self.w_in, self.in_bias)
+        proj = ops.step_linear(h[:, : self.width], self.w_in, self.in_bias)
         at, n = self.sections["rg"]
         routed = self.experts.forward(h) if self.experts else None
         if self.glu:
@@ -150,7 +150,7 @@ class NoganexLayer:
             ops.clamped_glu(
                 proj[:, : 2 * self.ff_pad], g.limit, g.alpha, g.offset, act, g.cubic
             )
-            y = ops.linear(act, self.down, self.down_bias)
+            y = ops.step_linear(act, self.down, self.down_bias)
         else:
             y = torch.zeros(h.shape[0], self.width, dtype=h.dtype, device=h.device)
         return y, proj[:, at : at + n], routed
@@ -327,4 +327,4 @@ class NoganexForCausalLM:
         x = x[batch.logit_rows]
         h = torch.empty(x.shape, dtype=self.dtype, device=self.device)
         ops.residual_norm(x, None, eps, None, self.final_norm, h, center=False)
-        return ops.linear(h, self.head).float().mul_(self.cfg.logit_scale)
+        return ops.step_linear(h, self.head).float().mul_(self.cfg.logit_scale)

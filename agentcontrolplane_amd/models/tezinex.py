@@ -100,10 +100,10 @@ class TezinexLayer:
         return out
 
     def feed_forward(self, h: torch.Tensor) -> torch.Tensor:
-        gate_up = ops.linear(h, self.gate_up)
+        gate_up = ops.step_linear(h, self.gate_up)
         act = torch.empty(h.shape[0], self.ff_pad, dtype=h.dtype, device=h.device)
         ops.clamped_glu(gate_up, self.mlp.limit, self.mlp.alpha, self.mlp.offset, act)
-        return ops.linear(act, self.down)
+        return ops.step_linear(act, self.down)
 
 
 class TezinexForCausalLM:
@@ -272,4 +272,4 @@ class TezinexForCausalLM:
         x = x[batch.logit_rows]
         h = torch.empty(x.shape, dtype=self.dtype, device=self.device)
         ops.residual_norm(x, None, eps, None, self.final_norm, h, **kw)
-        return ops.softcap(ops.linear(h, self.embed), cfg.logit_softcap)
+        return ops.softcap(ops.step_linear(h, self.embed), cfg.logit_softcap)

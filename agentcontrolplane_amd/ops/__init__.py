@@ -71,6 +71,54 @@ def linear(x, w, bias=None):
     return torch.nn.functional.linear(x, w, bias)
 
 
+def _few_rows(x, w, bias=None) -> bool:
+    """Whether csrc/step_linear.hip takes x w^T: at most four rows, and sizes at which it is
+    the faster one.  Four rows, us, against the GEMM library: 4096 x 4096 9 (14), 4096 x 6144 16
+    (23), 65536 x 4096 112 (123); beyond the limits 4096 x 8192 17 (16), 4096 x 14336 28 (25),
+    128256 x 4096 209 (178); eight rows: 28672 x 4096 54 (53), 6144 x 4096 18 (16)."""
+
+    def rows(t):  # of 16-byte units
+        return (
+            t.dim() == 2
+            and t.is_cuda
+            and t.dtype == torch.bfloat16
+            and t.stride(1) == 1
+            and (t.shape[0] == 1 or t.stride(0) % 8 == 0)
+            and t.data_ptr() % 16 == 0
+        )
+
+    return (
+        0 < x.shape[0] <= 4
+        and rows(x)
+        and rows(w)
+        and x.device == w.device
+        and x.shape[1] == w.shape[1]
+        and 0 < w.shape[0] <= 65536
+        and 0 < w.shape[1] < 8192
+        and w.shape[1] % 32 == 0
+        and (
+            bias is None
+            or bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
+            and bias.shape == w.shape[:1]
+        )
+    )
+
+
+def step_linear(x, w, bias=None):
+    """linear() of a step's activations in a model's forward pass, without autograd: the few
+    rows of a small decode step go to a kernel of their own."""
+    if _few_rows(x, w, bias):
+        return _hip().step_linear(x, w, bias)
+    return linear(x, w, bias)
+
+
+def step_linear_swiglu(x, w):
+    """swiglu(step_linear(x, w)), in one pass for a few rows."""
+    if _few_rows(x, w) and w.shape[0] % 16 == 0:
+        return _hip().step_linear(x, w, None, True)
+    return swiglu(linear(x, w))
+
+
 def linear_add_(y, x, w):
     """y += x @ w^T in one GEMM."""
     return y.addmm_(x, w.t())

@@ -117,6 +117,12 @@ def gemm_bf16(x, w):
     return out
 
 
+def step_linear(x, w, bias=None, glu=False):
+    out = torch.empty((x.shape[0], w.shape[0] >> glu), dtype=x.dtype, device=x.device)
+    _C.step_linear(out, x, w, bias, glu)
+    return out
+
+
 def swiglu(gate_up):
     inter = gate_up.shape[-1] // 2
     out = torch.empty(

@@ -15,6 +15,7 @@
 #include "grouped_attn.h"
 #include "latent_attn.h"
 #include "residual_norm.h"
+#include "step_linear.h"
 
 namespace py = pybind11;
 
@@ -123,6 +124,33 @@ static void swiglu(torch::Tensor out, torch::Tensor gate_up) {
   const int64_t n = gate_up.numel() / (2 * inter);
   TORCH_CHECK(inter % 8 == 0, "intermediate size must be a multiple of 8");
   launch_swiglu(out.data_ptr(), gate_up.data_ptr(), n, inter, cur_stream());
+}
+
+static void step_linear(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                        const c10::optional<torch::Tensor>& bias, bool glu) {
+  CHECK_CUDA(x); CHECK_CUDA(w); CHECK_CUDA(out); CHECK_CONT(out);
+  CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(out);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && M <= STEP_LINEAR_ROWS && w.size(1) == K && K > 0 && K % 32 == 0 &&
+              K < (1 << 30) && N > 0 && N < (1 << 30) && (!glu || N % 2 == 0));
+  TORCH_CHECK(out.size(0) == M && out.size(1) == (glu ? N / 2 : N));
+  TORCH_CHECK(x.stride(1) == 1 && w.stride(1) == 1);
+  StepLinearArgs a = {};
+  a.x_stride = M > 1 ? x.stride(0) : K;
+  a.w_stride = N > 1 ? w.stride(0) : K;
+  TORCH_CHECK(a.x_stride % 8 == 0 && a.w_stride % 8 == 0 &&
+              (uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0);
+  if (bias) {
+    CHECK_CUDA((*bias)); CHECK_BF16((*bias)); CHECK_CONT((*bias));
+    TORCH_CHECK(bias->numel() == N);
+    a.bias = bias->data_ptr();
+  }
+  a.out = out.data_ptr();
+  a.x = x.data_ptr();
+  a.w = w.data_ptr();
+  a.M = (int)M; a.N = (int)N; a.K = (int)K;
+  launch_step_linear(&a, glu, cur_stream());
 }
 
 static void rope_cache(torch::Tensor q, torch::Tensor k, torch::Tensor v,
@@ -1073,6 +1101,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("swiglu", &swiglu);
+  m.def("step_linear", &step_linear);
   m.def("rope_cache", &rope_cache);
   m.def("prefill_attn", &prefill_attn);
   m.def("mfma_probe", &mfma_probe);

@@ -10,6 +10,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
+from agentcontrolplane_amd import ops
 from agentcontrolplane_amd.ops import reference as ref
 
 requires_gpu = pytest.mark.skipif(not torch.cuda.is_available(), reason="needs MI355X")
@@ -558,3 +559,54 @@ def test_attention_bias_serving_on_gpu():
         assert res.completion_tokens <= 8
     finally:
         eng.stop()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 2, 4])
+@pytest.mark.parametrize("n,k,kind", [
+    (1, 32, "plain"), (17, 96, "bias"), (16, 288, "strided"), (250, 1120, "bias"),
+    (4096, 4096, "plain"), (33, 8160, "strided"), (16, 64, "glu"), (80, 2976, "glu"),
+    (1504, 4096, "glu"),
+])
+def test_step_linear(m, n, k, kind):
+    """A few rows' products, against double precision: one rounding of the sum to 16 bits, and
+    sums of k terms in 32 bits."""
+    gen = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k + 8, generator=gen).bfloat16().cuda()
+    w = torch.randn(n, k + 16, generator=gen).bfloat16().cuda()
+    x, w = (x[:, 8:], w[:, :k]) if kind == "strided" else (x[:, :k].clone(), w[:, :k].clone())
+    bias = torch.randn(n, generator=gen).bfloat16().cuda() if kind == "bias" else None
+    assert ops._few_rows(x, w, bias)
+    exact = x.double() @ w.double().T + (0 if bias is None else bias.double())
+    # sums: k terms of at most |x||w|, 2^-24 each
+    slack = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    if kind != "glu":
+        got = ops.step_linear(x, w, bias).double()
+        assert ((got - exact).abs() <= 2.0 ** -8 * exact.abs() + slack + 1e-30).all()
+        return
+    got = ops.step_linear_swiglu(x, w).double()
+    g, u = exact.chunk(2, 1)
+    # both halves are off by a rounding and the sums' slack; silu's slope is at most 1.1
+    dg, du = (2.0 ** -8 * t.abs() + s for t, s in zip((g, u), slack.chunk(2, 1)))
+    silu = torch.nn.functional.silu(g)
+    bound = 1.1 * dg * (u.abs() + du) + silu.abs() * du
+    want = silu * u
+    assert ((got - want).abs() <= bound + 2.0 ** -7 * want.abs() + 1e-30).all()
+
+
+@pytest.mark.gpu
+def test_step_linear_leaves_other_forms():
+    """What its kernel does not take goes the way of linear(), with the same result or error."""
+    x = torch.randn(4, 4104, device="cuda").bfloat16()
+    w = torch.randn(64, 4096, device="cuda").bfloat16()
+    lin = torch.nn.functional.linear
+    for a, b in [
+        (torch.randn(5, 4096, device="cuda").bfloat16(), w),
+        (x[:, 1:4097], w), (x[:, :4104:2][:, :2048], w[:, :2048]),
+        (x[:, :4096].float(), w.float()), (x[:0, :4096], w),
+        (x[:, :40], w[:, :40]), (x[:, :4096], w.T.contiguous().T), (x[:, None, :4096], w),
+    ]:
+        assert not ops._few_rows(a, b)
+        assert torch.equal(ops.step_linear(a, b), lin(a, b))
+    with pytest.raises(RuntimeError):
+        ops.step_linear(x[:, :4096], w[:, :2048])
