@@ -392,6 +392,32 @@ def test_delta_single_tokens(device, dtype):
         close(torch.cat(got[s]), case.want(s), dtype)
 
 
+@pytest.mark.parametrize("lens", [
+    [3, 70, 3, 20, 41, 1], [33, 33], [2 + 7 * i % 40 for i in range(64)],
+    [2 + 11 * i % 37 for i in range(67)],
+], ids=["uneven", "equal", "64", "67"])
+@pytest.mark.parametrize("D,V", [(16, 128), (128, 32)])
+def test_delta_uneven_prompts(device, dtype, lens, D, V):
+    """Prompts of many lengths at once, whichever of them the kernels begin with, with both
+    column counts: every sequence has its own rows and state."""
+    case = DeltaCase(2, 2, D, V, 4, lens, dtype, device)
+    for s, rows in enumerate(case.step([(s, n) for s, n in enumerate(lens)])):
+        close(rows, case.want(s), dtype)
+
+
+@pytest.mark.parametrize("lens,columns", [
+    ([1], 1), ([500] * 6, 1), ([500] * 7, 2), ([2600] + [300] * 40, 1),
+    ([2600] + [300] * 44, 2),
+])
+def test_delta_columns_a_lane(lens, columns):
+    """Two once the other sequences have more than 5 times the longest one's tokens (of 2048
+    columns)."""
+    from agentcontrolplane_amd.ops.hip import _scan_columns
+
+    metas = [SeqMeta(i, n, n, 0, [0], True, i) for i, n in enumerate(lens)]
+    assert _scan_columns(metas, 2048) == columns
+
+
 def test_delta_slot_is_used_again(device):
     """A slot's next sequence starts from zero, whatever the last one left, and the
     slots of waiting sequences keep theirs."""
