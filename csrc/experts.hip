@@ -187,7 +187,7 @@ __global__ __launch_bounds__(1024) void group_kernel(
     int row = 0, tile = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + lane;
-      const int c = e < E ? total[e] : 0, t = (c + EXPERT_TILE - 1) / EXPERT_TILE;
+      const int c = e < E ? total[e] : 0, high = expert_tile(c), t = (c + high - 1) / high;
       int cs = c, ts = t;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(1024) void group_kernel(
         offsets[e] = first;
         for (int j = 0; j < t && tile_expert; ++j) {
           tile_expert[tile + ts - t + j] = e;
-          tile_row[tile + ts - t + j] = first + j * EXPERT_TILE;
+          tile_row[tile + ts - t + j] = first + j * high;
         }
       }
       row += __shfl(cs, 63, 64);

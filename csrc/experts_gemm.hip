@@ -1,5 +1,5 @@
 // The routed experts' products for many rows per expert (gfx950): a grouped GEMM over
-// tiles of 256 rows of one expert.
+// tiles of 256 rows of one expert, or up to 320.
 //
 // Rows come grouped by expert.  The first product gathers its token rows and applies the
 // gated unit to its accumulators: a wave's two 32-column fragments are gate and up of
@@ -14,6 +14,15 @@
 //     multiply, the first ones of the next half (raising the priority of multiplying waves
 //     made this slower)
 //   waves whose last 64 or all 128 rows are beyond the expert's last one skip them
+//   tiles of more than 256 rows: each row of waves has 32 more, against the same fragments of
+//     the weights
+//
+// 32 experts of 4096 x 2560, both products: 512 rows each 1212 us; 520 rows 1568 with a third tile
+// for 8 of them, which reads 2 GB of weights once more at 5.5 TB/s, 1295 in two tall tiles; 640
+// rows 1578, now 1352; 4093 tokens to 4 of 32 experts at random 1485, now 1290.  Tiles of up to
+// 128 rows with 3 or 4 chunks in flight gained nothing.
+#include <type_traits>
+
 #include "experts.h"
 #include "gated_act.h"
 
@@ -23,7 +32,8 @@ typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(1))) const char glob_char;
 
 #define PANEL 32768  // one operand's chunk: 256 rows of 128 bytes
-#define SLOTS 4
+#define EXTRA 8192  // chunk of the rows past 256
+#define LDS_BYTES (4 * PANEL + 2 * EXTRA)
 #define WAIT_VM(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
 
 template <bool GLU>
@@ -44,7 +54,11 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
     tn = rest / high;
   }
   const int e = a.tile_expert[tm], row0 = a.tile_row[tm];
-  const int rows = min(EXPERT_TILE, a.offsets[e + 1] - row0);
+  // up to the expert's next tile or end
+  const int tm1 = min(tm + 1, used - 1), e1 = a.tile_expert[tm1], row1 = a.tile_row[tm1];
+  const int end = a.offsets[e + 1];
+  const int rows = (tm1 > tm && e1 == e ? row1 : end) - row0;
+  const bool tall = rows > EXPERT_TILE;
   const int o0 = tn * (GLU ? 128 : 256);  // first output
 
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -52,14 +66,19 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
   const int c = lane & 31, half = lane >> 5;
 
   // this thread's rows of every panel: 8 threads a row
-  const bf16_t *ap[4], *bp[4];
+  const bf16_t *ap[5], *bp[4];
   const bf16_t* w = (const bf16_t*)a.w + (int64_t)e * (GLU ? 2 : 1) * a.O * a.K;
+  auto row_of_x = [&](int row) {
+    const int r = row0 + min(row, rows - 1);
+    return (const bf16_t*)a.x + (int64_t)(GLU ? a.perm[r] / a.top : r) * a.x_stride +
+           ((lane & 7) ^ (lane >> 3)) * 8;
+  };
+  ap[4] = tall ? row_of_x(EXPERT_TILE + wid * 8 + (lane >> 3)) : nullptr;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = wid * 32 + i * 8 + (lane >> 3);
     const int col = ((lane & 7) ^ (lane >> 3)) * 8;
-    const int r = row0 + min(row, rows - 1);
-    ap[i] = (const bf16_t*)a.x + (int64_t)(GLU ? a.perm[r] / a.top : r) * a.x_stride + col;
+    ap[i] = row_of_x(row);
     // 64 weight rows a wave column: 32 gates and the ups beside them, or 64 outputs
     int o = o0 + (GLU ? (row >> 6) * 32 + (row & 31) : row);
     o = min(o, a.O - 1);
@@ -68,7 +87,8 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
   }
   const int chunks = a.K >> 6;
   const int halves = (rows - wm * 128 + 63) >> 6;  // 64-row parts of this wave with rows
-  auto stage = [&](int chunk, int buffer) {  // past the end the last one again: not used
+  // tall_tile: has rows past 256.  Past the end the last chunk again: not used
+  auto stage = [&](auto tall_tile, int chunk, int buffer) {
     chunk = min(chunk, chunks - 1);
     char* dst = lds + 2 * buffer * PANEL + wid * 4096;
 #pragma unroll
@@ -78,6 +98,10 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
       __builtin_amdgcn_global_load_lds((glob_char*)(bp[i] + chunk * 64),
                                        (lds_char*)(dst + PANEL + i * 1024), 16, 0, 0);
     }
+    if (decltype(tall_tile)::value)
+      __builtin_amdgcn_global_load_lds(
+          (glob_char*)(ap[4] + chunk * 64),
+          (lds_char*)(lds + 4 * PANEL + buffer * EXTRA + wid * 1024), 16, 0, 0);
   };
   // fragments of steps 2q, 2q + 1 (16 of K each), rows 0 and 32 of a panel's part
   const char* la = lds + (wm * 128 + c) * 128;
@@ -101,23 +125,28 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
                                                                     acc[2 * h + f][g], 0, 0, 0);
   };
   // chunk c is read by every wave, chunk c + 1 has landed for every wave
-  auto hand_over = [&](int c) {
+  auto hand_over = [&](auto tall_tile, int c) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    stage(c + 2, c & 1);
+    stage(tall_tile, c + 2, c & 1);
   };
 
-  stage(0, 0);
-  stage(1, 1);
-  WAIT_VM(8);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+  auto start = [&](auto tall_tile) {
+    stage(tall_tile, 0, 0);
+    stage(tall_tile, 1, 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(tall_tile)::value ? 9 : 8) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
 
-  // both loops pass the same barriers and stage the same chunks
-  if (halves >= 2) {
-    bf16x8_v a0[2][2], a1[2][2], b[2][2][2];
+  // all loops pass the same barriers and stage the same chunks
+  f32x16_v more[2] = {};  // rows past 256
+  const char* lx = lds + 4 * PANEL + (wm * 32 + c) * 128;
+  auto whole = [&](auto tall_tile, auto has_more) {
+    constexpr bool MORE = decltype(has_more)::value;
+    bf16x8_v a0[2][2], a1[2][2], b[2][2][2], x[2];
     read(b[0], lb, 0);
     read(a0, la, 0);
     for (int c0 = 0; c0 < chunks; c0 += 2) {  // K is a multiple of 128
@@ -127,18 +156,42 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
         multiply(0, 0, a0, b[j & 1]);
         __builtin_amdgcn_sched_barrier(0);
         read(a1, la + here + 8192, j & 1);
+        if (MORE) {
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+            x[s] = *(const bf16x8_v*)(lx + (j >> 1) * EXTRA + at[2 * (j & 1) + s]);
+        }
         __builtin_amdgcn_sched_barrier(0);
         multiply(0, 1, a0, b[j & 1]);
         __builtin_amdgcn_sched_barrier(0);
-        if (j & 1) hand_over(c0 + (j >> 1));
+        if (j & 1) hand_over(tall_tile, c0 + (j >> 1));
         read(b[~j & 1], lb + next, ~j & 1);
         read(a0, la + next, ~j & 1);
         multiply(1, 0, a1, b[j & 1]);
         multiply(1, 1, a1, b[j & 1]);
+        if (MORE) {
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+              more[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[s], b[j & 1][g][s], more[g],
+                                                                0, 0, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+  };
+  const bool extra = rows > EXPERT_TILE + wm * 32;
+  const std::true_type yes;
+  const std::false_type no;
+  if (tall) {
+    start(yes);
+    extra ? whole(yes, yes) : whole(yes, no);
+  } else if (halves >= 2) {
+    start(no);
+    whole(no, no);
   } else {
+    start(no);
     for (int c = 0; c < chunks; ++c) {
       if (halves == 1)
 #pragma unroll
@@ -150,25 +203,24 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
           multiply(0, 0, a0, b);
           multiply(0, 1, a0, b);
         }
-      hand_over(c);
+      hand_over(no, c);
     }
   }
   WAIT_VM(0);  // the loads past the end
 
   // register r of a fragment: row (r & 3) + 8 (r >> 2) + 4 half, column c
   bf16_t* out = (bf16_t*)a.out;
-#pragma unroll
-  for (int f = 0; f < 4; ++f)
+  auto put = [&](int base, const f32x16_v (&sums)[2]) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int row = wm * 128 + f * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
+      const int row = base + (r & 3) + 8 * (r >> 2) + 4 * half;
       if (row >= rows) continue;
       if (GLU) {
         const int o = o0 + wn * 32 + c;
         if (o >= a.O) continue;
         // through the model's precision, as a GEMM stores it
-        const float gate = to_f(from_f<bf16_t>(acc[f][0][r]));
-        const float up = to_f(from_f<bf16_t>(acc[f][1][r]));
+        const float gate = to_f(from_f<bf16_t>(sums[0][r]));
+        const float up = to_f(from_f<bf16_t>(sums[1][r]));
         out[(int64_t)(row0 + row) * a.O + o] =
             from_f<bf16_t>(clamped_glu_f(gate, up, a.limit, a.alpha, a.offset, a.cubic));
       } else {
@@ -176,10 +228,14 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
           const int o = o0 + wn * 64 + g * 32 + c;
-          if (o < a.O) dst[o] = from_f<bf16_t>(acc[f][g][r]);
+          if (o < a.O) dst[o] = from_f<bf16_t>(sums[g][r]);
         }
       }
     }
+  };
+#pragma unroll
+  for (int f = 0; f < 4; ++f) put(wm * 128 + f * 32, acc[f]);
+  if (extra) put(EXPERT_TILE + wm * 32, more);
 }
 
 template <bool GLU>
@@ -187,12 +243,12 @@ static void launch(const ExpertsArgs& a, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) {
     (void)hipFuncSetAttribute((const void*)experts_gemm_kernel<GLU>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, SLOTS * PANEL);
+                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
     attr_set = true;
   }
   const int per = GLU ? 128 : 256;
   const int tiles_n = (a.O + per - 1) / per;
-  experts_gemm_kernel<GLU><<<a.tiles * tiles_n, 512, SLOTS * PANEL, stream>>>(a, tiles_n);
+  experts_gemm_kernel<GLU><<<a.tiles * tiles_n, 512, LDS_BYTES, stream>>>(a, tiles_n);
 }
 
 extern "C" void launch_experts_gemm(bool glu, const ExpertsArgs* a, hipStream_t stream) {

@@ -512,6 +512,25 @@ EXPERTS = [
 ]
 
 
+@pytest.mark.gpu
+def test_experts_tile_heights():
+    """Every height of an expert's tiles: few rows, 256, the even ones up to 320, several."""
+    rows = [0, 1, 64, 65, 255, 256, 257, 288, 289, 320, 321, 512, 513, 577, 640, 641, 961]
+    E, K, I, W = len(rows), 128, 256, 264
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).int()
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(1))].view(-1, 1)
+    h = rand(len(ids), K, dtype=torch.bfloat16, device="cuda")
+    gate_up = rand(E, 2 * I, K, dtype=torch.bfloat16, device="cuda", seed=1, scale=2 * K ** -0.5)
+    down = rand(E, W, I, dtype=torch.bfloat16, device="cuda", seed=2, scale=I ** -0.5)
+    got = ops.moe_experts(h, gate_up, down, ids.cuda(), ClampedGluSpec(I, 1.25)).cpu()
+    for e in range(E):
+        x = {"gate": gate_up[e, :I].double().cpu(), "up": gate_up[e, I:].double().cpu(),
+             "down": down[e].double().cpu()}
+        t = (ids[:, 0] == e).nonzero()[:, 0]
+        if len(t):
+            close(got[t, 0], oracle.clamped_glu(h.double().cpu()[t], x, "", 1.25), torch.bfloat16)
+
+
 @pytest.mark.parametrize("skew", [False, True])
 @pytest.mark.parametrize("n,E,top,K,I,W", EXPERTS)
 def test_experts(device, dtype, n, E, top, K, I, W, skew):
