@@ -44,7 +44,7 @@ void launch_embed_positions(bool, float*, float*, const int64_t*, const int64_t*
 void launch_attn_inputs(bool, const AttnInputsArgs*, hipStream_t);
 void launch_moe_route(bool, int*, float*, const void*, const void*, const float*, int, int, int,
                       int, int64_t, bool, float, hipStream_t);
-void launch_moe_group(int*, int*, int*, int*, const int*, int, int, hipStream_t);
+void launch_moe_group(int*, int*, int*, int*, const int*, int, int, int, hipStream_t);
 void launch_experts_small(bool, const ExpertsArgs*, int, hipStream_t);
 void launch_experts_f32(bool, const ExpertsArgs*, hipStream_t);
 void launch_experts_gemm(bool, const ExpertsArgs*, hipStream_t);
@@ -922,18 +922,19 @@ static void moe_route(torch::Tensor ids, torch::Tensor weights, torch::Tensor h,
                    h.stride(0), sigmoid, (float)scale, cur_stream());
 }
 
-// perm [n], offsets [E + 2]; tiles of EXPERT_TILE rows: at most ceil(n / tile) + E
+// perm [n], offsets [E + 2]; tiles of at least EXPERT_TILE rows: at most ceil(n / tile) + E, each
+// multiplied in this many columns of workgroups
 static void moe_group(torch::Tensor perm, torch::Tensor offsets, OptTensor tile_expert,
-                      OptTensor tile_row, torch::Tensor ids, int64_t E) {
+                      OptTensor tile_row, torch::Tensor ids, int64_t E, int64_t columns) {
   const int64_t n = ids.numel();
   CHECK_CUDA(ids); CHECK_CONT(ids);
   TORCH_CHECK(ids.scalar_type() == at::kInt && E > 0 && E <= 512 && n < (1 << 30));
   const int64_t tiles = tile_expert ? n / EXPERT_TILE + E : 0;
   int* te = (int*)opt_int(tile_expert, tiles);
   int* tr = (int*)opt_int(tile_row, tiles);
-  TORCH_CHECK(!te == !tr, "tiles");
+  TORCH_CHECK(!te == !tr && columns > 0 && columns * (n / EXPERT_TILE + E) < (1 << 30), "tiles");
   launch_moe_group((int*)opt_int(perm, n), (int*)opt_int(offsets, E + 2), te, tr,
-                   ids.data_ptr<int>(), (int)n, (int)E, cur_stream());
+                   ids.data_ptr<int>(), (int)n, (int)E, (int)columns, cur_stream());
 }
 
 // One product of the routed experts (experts.h).  kind: 0 fp32, 1 few rows, 2 tiles

@@ -24,7 +24,7 @@ struct ExpertsArgs {
 
 // Rows of an expert's tiles: even ones of 257 to 320 rows if they cover the expert in fewer tiles,
 // as a small last tile takes all of the expert's weights once more.
-static __host__ __device__ inline int expert_tile(int rows) {
+__device__ static inline int tall_tile(int rows) {
   const int tiles = (rows + TALL_TILE - 1) / TALL_TILE;
   const int even = tiles > 0 ? (rows + tiles - 1) / tiles : 0;
   return even > EXPERT_TILE ? even : EXPERT_TILE;

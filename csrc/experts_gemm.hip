@@ -18,9 +18,9 @@
 //     the weights
 //
 // 32 experts of 4096 x 2560, both products: 512 rows each 1212 us; 520 rows 1568 with a third tile
-// for 8 of them, which reads 2 GB of weights once more at 5.5 TB/s, 1295 in two tall tiles; 640
-// rows 1578, now 1352; 4093 tokens to 4 of 32 experts at random 1485, now 1290.  Tiles of up to
-// 128 rows with 3 or 4 chunks in flight gained nothing.
+// for 8 of them, which reads 2 GB of weights once more at 5.5 TB/s, 1295 in two tall tiles. At
+// random to 4 of 32, 2048 tokens 887, now 652; 4093 1364, now 1094; 8192 2260, now 2119. Tiles of
+// up to 128 rows with 3 or 4 chunks in flight gained nothing.
 #include <type_traits>
 
 #include "experts.h"
@@ -176,6 +176,13 @@ __global__ __launch_bounds__(512, 1) void experts_gemm_kernel(const ExpertsArgs 
             for (int g = 0; g < 2; ++g)
               more[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[s], b[j & 1][g][s], more[g],
                                                                 0, 0, 0);
+        }
+        if (!MORE) {  // reads between the products: 2% (with more rows they spill)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
       }

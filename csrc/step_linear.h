@@ -10,7 +10,7 @@ struct StepLinearArgs {
   const void* w;     // [N, K] rows w_stride apart; GLU: gates, then ups
   const void* bias;  // [N] or null
   int64_t x_stride, w_stride;
-  int M, N, K;       // M at most STEP_LINEAR_ROWS, K a multiple of 32; rows of x and w 16-byte aligned
+  int M, N, K;       // M at most STEP_LINEAR_ROWS, K a multiple of 32; rows 16-byte aligned
 };
 
 extern "C" void launch_step_linear(const StepLinearArgs* a, bool glu, hipStream_t stream);

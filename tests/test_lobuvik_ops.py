@@ -513,10 +513,12 @@ EXPERTS = [
 
 
 @pytest.mark.gpu
-def test_experts_tile_heights():
-    """Every height of an expert's tiles: few rows, 256, the even ones up to 320, several."""
+@pytest.mark.parametrize("I", [256, 3072], ids=["one round", "several"])
+def test_experts_tile_heights(I):
+    """Every height of an expert's tiles: few rows, 256, the even ones up to 320, several; the
+    tall ones where they save a round of workgroups."""
     rows = [0, 1, 64, 65, 255, 256, 257, 288, 289, 320, 321, 512, 513, 577, 640, 641, 961]
-    E, K, I, W = len(rows), 128, 256, 264
+    E, K, W = len(rows), 128, 264
     ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).int()
     ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(1))].view(-1, 1)
     h = rand(len(ids), K, dtype=torch.bfloat16, device="cuda")
