@@ -310,6 +310,44 @@ def test_prompt_tiles_over_pages(block, H, G, scale):
 
 
 @requires_gpu
+@pytest.mark.parametrize("spread", [1.0, 4.0])
+def test_prompt_error_against_64_bits(spread):
+    """Weights rounded to 16 bits make most of the error, and all of it above the result's own
+    rounding: it is no larger than that of a softmax over tiles of 32 keys whose denominator has
+    the weights before rounding."""
+    from op_helpers import make_batch
+
+    n, H, scale = 900, 16, 128 ** -0.5
+    gen = torch.Generator().manual_seed(1)
+    batch, _, _, pages = make_batch([(0, n)], 16, "cuda")
+    table = torch.tensor(batch.prefills[0].block_table)
+    slots = table[torch.arange(n) // 16] * 16 + torch.arange(n) % 16
+    q, k, v = (torch.randn(n, H, 128, generator=gen).mul(x).bfloat16() for x in (spread, 1, 1))
+    kc, vc = torch.zeros(2, pages * 16, H, 128, dtype=torch.bfloat16)
+    kc[slots], vc[slots] = k, v
+    got = hip().attention_prefill_batch(
+        q.cuda(), *(c.view(pages, 16, H, 128).cuda() for c in (kc, vc)), batch, scale
+    ).cpu().double()
+    hidden = torch.ones(n, n).triu(1).bool()
+    err = tiles = 0.0
+    for h in range(H):
+        s = (q[:, h].float() @ k[:, h].float().T * scale).masked_fill(hidden, -math.inf)
+        values = v[:, h].double()
+        want = torch.softmax(s.double(), -1) @ values
+        top, o, total = torch.full((n, 1), -1e30), 0.0, 0.0
+        for t in range(0, n, 32):
+            up = torch.maximum(top, s[:, t : t + 32].amax(1, keepdim=True))
+            w = torch.exp(s[:, t : t + 32] - up)
+            down = torch.exp(top - up).double()
+            o = o * down + w.bfloat16().double() @ values[t : t + 32]
+            total = total * down + w.double().sum(1, keepdim=True)
+            top = up
+        tiles += ((o / total).bfloat16().double() - want).pow(2).sum().item()
+        err += (got[:, h] - want).pow(2).sum().item()
+    assert err <= tiles, (err / tiles) ** 0.5
+
+
+@requires_gpu
 def test_sample_greedy_and_filters():
     torch.manual_seed(3)
     B, V = 64, 261
