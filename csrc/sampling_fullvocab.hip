@@ -232,7 +232,7 @@ __device__ float fill(Shared& s, const Row<T>& row, float far) {
 // weights if it is given; 0: nowhere.  ``plain``: all logits are numbers.
 template <bool BY_MASS, typename T>
 __device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double part, bool plain) {
-  if (target <= 0.0) return 0xffffffffu;  // reached before the first
+  if (target <= 0.0) return f2key(row.m);  // reached before the first, which is kept all the same
   auto stream = [&](auto f) { row.each([&](int, float v) { f(f2key(v)); }); };
   if (!plain) return split_keys<BY_MASS>(s, row, 0u, 0xffffffffu, 0.0, target, stream);
   double above = 0.0;
@@ -241,7 +241,7 @@ __device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double
     double all = 0.0;
     for (int i = threadIdx.x; i < FIRST; i += WG) all += s.mass[i] * UNIT;
     target = part * block_total(s, all + rest);
-    if (target <= 0.0) return 0xffffffffu;
+    if (target <= 0.0) return f2key(row.m);
   }
   int b = find_bucket<BY_MASS>(s, FIRST, target, &above);
   if (b < 0) {  // beyond the head
@@ -482,15 +482,16 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
   __syncthreads();
   if (t == 0 && s.pick < 0) {
     // fallback (target == total to fp precision, or an empty kept set):
-    // the last kept token, matching searchsorted's clamp in the oracle
-    int last = 0;
+    // the last kept token, matching searchsorted's clamp in the oracle; else the last allowed one
+    int last = -1;
     for (int i = V - 1; i >= 0; --i) {
       if (row.mask && !row.mask[i]) continue;
+      if (last < 0) last = i;
       if (f2key(ldf(row.x + i)) < kmin) continue;
       last = i;
       break;
     }
-    s.pick = last;
+    s.pick = max(last, 0);
   }
   __syncthreads();
   if (t == 0) out[n_row] = s.pick;

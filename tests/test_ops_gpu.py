@@ -278,6 +278,34 @@ def test_fullvocab_draws_lie_in_the_kept_cdf(V, dtype):
 
 
 @requires_gpu
+@pytest.mark.parametrize("k", [0, 3])
+@pytest.mark.parametrize("p", [0.0, -1.0])
+@pytest.mark.parametrize("V", [600, 128256])
+def test_fullvocab_top_p_of_zero_keeps_the_largest(V, p, k):
+    """The nucleus always has the largest allowed logits, as many as are equal, as in the oracle; a
+    negative p is taken for zero."""
+    torch.manual_seed(V)
+    x = torch.randn(6, V)
+    x[1, [7, V // 2, V - 3]] = 9.0
+    x[2, 0] = 50.0
+    x[3] = -2.0
+    x[4, : V // 2] = -math.inf
+    mask = torch.rand(2, V) < 0.05
+    mask[:, 0] = False
+    rows = [-1, -1, 0, -1, 1, 1]
+    u = torch.tensor([0.5, 0.5, 0.1, 0.999, 0.3, 0.0])
+    got = hip().softmax_sample(
+        x.cuda(), torch.full((6,), 0.7).cuda(), torch.full((6,), k).cuda(),
+        torch.full((6,), p).cuda(), None, mask.cuda(), u.cuda(),
+        torch.tensor(rows, dtype=torch.int32).cuda(),
+    ).tolist()
+    for r, m in enumerate(rows):
+        v = x[r] if m < 0 else x[r].masked_fill(~mask[m], -math.inf)
+        largest = (v == v.max()).nonzero()[:, 0].tolist()
+        assert got[r] == largest[int(u[r].double().item() * len(largest))], r
+
+
+@requires_gpu
 @pytest.mark.parametrize("block", [8, 16, 24, 64])
 @pytest.mark.parametrize("H,G,scale", [(8, 8, 0.09), (6, 2, -0.09), (4, 1, 0.0)])
 def test_prompt_tiles_over_pages(block, H, G, scale):
