@@ -71,11 +71,34 @@ def linear(x, w, bias=None):
     return torch.nn.functional.linear(x, w, bias)
 
 
-def _few_rows(x, w, bias=None) -> bool:
-    """Whether csrc/step_linear.hip takes x w^T: at most four rows, and sizes at which it is
-    the faster one.  Four rows, us, against the GEMM library: 4096 x 4096 9 (14), 4096 x 6144 16
-    (23), 65536 x 4096 112 (123); beyond the limits 4096 x 8192 17 (16), 4096 x 14336 28 (25),
-    128256 x 4096 209 (178); eight rows: 28672 x 4096 54 (53), 6144 x 4096 18 (16)."""
+def _few_rows_pay(m: int, outs: int, k: int, glu: bool) -> bool:
+    """Whether csrc/step_linear.hip is the faster one for m rows, outs outputs (of a GLU: pairs)
+    and k inner elements; the GEMM library (with a pass of its own for the GLU) is in brackets,
+    us.  Four rows: 4096 x 4096 9 (16), 20048 x 2048 21 (50), 3584 x 3584 9 (12), pairs of 14336 x
+    4096 56 (57) and of 11008 x 4096 43 (53).  Beyond the limits: up to 2048, 65536 x 1024 33
+    (28); up to 4096, 4608 x 3584 14 (12), pairs of 18944 x 3584 67 (59), 16384 x 3072 27 (23); 4096
+    itself, where the library reads at 4 TB/s and less, 128256 outputs 209 (178), and between one
+    and two workgroups a CU 6144 15.2 (14.6), at two rows 14.4 (14.6); above it, 1024 x 4608 10
+    (17), but 5120 x 5120 21 (14), 32000 x 5120 82 (64), 16 x 5120 9 (6) and 4096 x 7168 17 (15); near
+    8192 64 x 8160 13 (13), 1024 x 8064 15 (17), 256 x 8064 14 (13).  Eight rows: 28672 x 4096
+    54 (53)."""
+    if m > 4:
+        return False
+    if k < 2048:
+        return outs <= 28672
+    if k == 2048:
+        return outs <= 51200
+    if k < 4096:
+        return outs <= 4096
+    if k == 4096:
+        return outs <= 65536 and (m <= 2 or glu or not 4096 < outs <= 8192)
+    if k <= 5120:
+        return 64 <= outs <= 2048
+    return 7680 < k < 8192 and (outs <= 64 or 512 <= outs <= 4096)
+
+
+def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
+    """Whether csrc/step_linear.hip takes x w^T: what it can, at the sizes at which it pays."""
 
     def rows(t):  # of 16-byte units
         return (
@@ -93,9 +116,10 @@ def _few_rows(x, w, bias=None) -> bool:
         and rows(w)
         and x.device == w.device
         and x.shape[1] == w.shape[1]
-        and 0 < w.shape[0] <= 65536
-        and 0 < w.shape[1] < 8192
+        and w.shape[0] > 0
+        and w.shape[1] > 0
         and w.shape[1] % 32 == 0
+        and _few_rows_pay(x.shape[0], w.shape[0] >> glu, w.shape[1], glu)
         and (
             bias is None
             or bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
@@ -114,7 +138,7 @@ def step_linear(x, w, bias=None):
 
 def step_linear_swiglu(x, w):
     """swiglu(step_linear(x, w)), in one pass for a few rows."""
-    if _few_rows(x, w) and w.shape[0] % 16 == 0:
+    if w.shape[0] % 16 == 0 and _few_rows(x, w, None, True):
         return _hip().step_linear(x, w, None, True)
     return swiglu(linear(x, w))
 

@@ -8,9 +8,10 @@
 // from L2 in the same form (B; lanes past the last row read it again).  The waves' sums meet in
 // LDS, in a fixed order, in fp32.
 //
-// One row, against the GEMM library (and the GLU's own pass) before, us:
-//   28672 x 4096 GLU 49 (60), 22016 x 4096 GLU 41 (54), 6144 x 4096 15 (16), 4096 x 4096 8.5
-//   (13.3), 20000 x 2048 20 (50), 2048 x 2048 5.6 (8.3).
+// One row, against the GEMM library (and the GLU's own pass) before, us, every weight from
+// memory: 28672 x 4096 GLU 54 (64), 22016 x 4096 GLU 41 (54), 6144 x 4096 14.0 (14.7), 4096 x 4096
+// 8.5 (15.6), 20048 x 2048 22 (50), 2048 x 2048 5.2 (11.0).  384 workgroups (6144 outputs) leave
+// half of the CUs with one and half with two.
 // Half and twice the loads in flight, 4 and 16 waves, the next group's loads during a group's
 // products, 32 outputs a workgroup: all slower by 2 to 40% at most of these sizes.
 #include <type_traits>
