@@ -5,6 +5,8 @@ hipcc cross-compiles gfx950 without a GPU, so this runs in CPU-only CI too.
 The .so lands inside the package (NOT a JIT cache dir) so the gpurun
 snapshot carries it to the GPU box.
 """
+import glob
+import hashlib
 import os
 import shutil
 import sys
@@ -15,6 +17,17 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(ROOT, "csrc")
 PKG = os.path.join(ROOT, "agentcontrolplane_amd")
 BUILD = os.path.join(ROOT, "build", "ext")
+
+
+def headers_digest(folder: str = CSRC) -> str:
+    """Of the headers' contents.  As a part of the device compiler's command it has every kernel
+    built again after a header changed: ninja is told of no header that they include, and a
+    kernel of another layout of its arguments than its launcher's reads anywhere."""
+    digest = hashlib.sha256()
+    for path in sorted(glob.glob(os.path.join(folder, "*.h"))):
+        with open(path, "rb") as f:
+            digest.update(os.path.basename(path).encode() + b"\0" + f.read() + b"\0")
+    return digest.hexdigest()[:16]
 
 
 def build(verbose: bool = False) -> str:
@@ -52,7 +65,7 @@ def build(verbose: bool = False) -> str:
         build_directory=BUILD,
         extra_cflags=["-O3"],
         extra_cuda_cflags=[
-            "-O3", "--offload-arch=gfx950", "-std=c++17",
+            "-O3", "--offload-arch=gfx950", "-std=c++17", f"-DHEADERS_{headers_digest()}",
             # no packed fp32 VALU forms: some give wrong results on gfx950
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         ],
