@@ -98,7 +98,11 @@ def _few_rows_pay(m: int, outs: int, k: int, glu: bool) -> bool:
 
 
 def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
-    """Whether csrc/step_linear.hip takes x w^T: what it can, at the sizes at which it pays."""
+    """Whether csrc/step_linear.hip takes x w^T: what it can, at the sizes at which it pays.
+    It has no derivative: what autograd records is left to the library."""
+
+    def recorded(t):
+        return t is not None and t.requires_grad
 
     def rows(t):  # of 16-byte units
         return (
@@ -125,12 +129,13 @@ def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
             or bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
             and bias.shape == w.shape[:1]
         )
+        and not (torch.is_grad_enabled() and (recorded(x) or recorded(w) or recorded(bias)))
     )
 
 
 def step_linear(x, w, bias=None):
-    """linear() of a step's activations in a model's forward pass, without autograd: the few
-    rows of a small decode step go to a kernel of their own."""
+    """linear() of a step's activations in a model's forward pass: the few rows of a small decode
+    step go to a kernel of their own, unless autograd records them."""
     if _few_rows(x, w, bias):
         return _hip().step_linear(x, w, bias)
     return linear(x, w, bias)

@@ -676,3 +676,20 @@ def test_step_linear_leaves_other_forms():
         assert torch.equal(ops.step_linear(a, b), lin(a, b))
     with pytest.raises(RuntimeError):
         ops.step_linear(x[:, :4096], w[:, :2048])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("needs", ["x", "w", "bias"])
+def test_step_linear_keeps_gradients(needs):
+    """A few rows that autograd records get the derivatives that linear() gives."""
+    gen = torch.Generator().manual_seed(3)
+    shape = {"x": (4, 256), "w": (64, 256), "bias": (64,)}
+    t = {n: torch.randn(*s, generator=gen).bfloat16().cuda() for n, s in shape.items()}
+    t[needs].requires_grad_()
+    got, = torch.autograd.grad(ops.step_linear(t["x"], t["w"], t["bias"]).float().sum(), t[needs])
+    want, = torch.autograd.grad(
+        torch.nn.functional.linear(t["x"], t["w"], t["bias"]).float().sum(), t[needs]
+    )
+    assert torch.equal(got, want)
+    with torch.no_grad():
+        assert ops._few_rows(t["x"], t["w"], t["bias"])
