@@ -373,12 +373,12 @@ def _grouped_decode(out, q, k_cache, v_cache, tables, seq_lens, sink, bias, gate
     """One token per sequence, head sizes of the matrix-core kernels.  Grid and workspace
     depend on sizes alone, not on the lengths, so that a step can be captured."""
     (B, H, d), v, G = q.shape, out.shape[2], k_cache.shape[2]
-    gm = next((n for n in (1, 4) if n >= H // G), 8)  # query heads a workgroup holds
+    gm = next((n for n in (1, 2, 4) if n >= H // G), 8)  # query heads a workgroup holds
     # pieces of the step's keys: workgroups that fill the chip
     keys = min(tables.shape[1] * k_cache.shape[1], window + keep_first, chunk)
     groups = G * -(-(H // G) // gm)
     pieces, part, ml = 0, None, None
-    if B * groups < _WHOLE_GROUPS and keys > 128:
+    if B * groups < _WHOLE_GROUPS and keys > 128 and B * keys <= _C.DECODE_KEYS:
         pieces = max(1, _DECODE_GROUPS // groups)
         part = torch.empty((pieces + B) * H * v, dtype=torch.float32, device=q.device)
         ml = torch.empty(2 * (pieces + B) * H, dtype=torch.float32, device=q.device)

@@ -20,16 +20,20 @@ struct GroupedArgs {
   const int* tile_seq;    // [tiles]; null: decode, one token per sequence
   const int* tile_q0;     // [tiles] first token of the tile within the chunk
   int64_t q_stride, out_stride, gate_stride;
-  int H, G, n_tiles, max_blocks, kv_block, window, keep, n_split, rows, n_bias;
+  int H, G, group, n_tiles, max_blocks, kv_block, window, keep, n_split, rows, n_bias;
   int seqs, pieces;       // decode: about how many pieces the step's keys are cut into
   int chunk;              // only keys of the query's own chunk; 2^30: all
   float scale, cap;       // cap 0: none
   bool sigmoid;           // weights sigmoid(score), not a softmax
 };
 
+// keys of a step that is cut into pieces: the kernel counts their blocks of 32 in 22 bits
+#define DECODE_KEYS (1ll << 26)
+
 #ifdef __HIPCC__
 // first key that position pos sees beyond the kept ones
 static inline __device__ int first_key(const GroupedArgs& a, int pos) {
-  return max(max(0, pos - a.window + 1), pos - pos % a.chunk);
+  const int first = max(0, pos - a.window + 1);
+  return a.chunk < (1 << 30) ? max(first, pos - pos % a.chunk) : first;
 }
 #endif

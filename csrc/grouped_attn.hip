@@ -18,7 +18,7 @@
 // Bound by memory: 5.2 to 5.3 TB/s of keys and values at 64 x 4096 and 256 x 1024 tokens, 32
 // heads over 8.  Before, with products and sums over dims on the VALU, 4.1 TB/s there and 2.0 to
 // 3.0 where lengths differ: 61 x 310 to 4000 tokens 268 -> 122 us, 190 x 700 to 1300 265 -> 159,
-// 1 x 4002 203 -> 15 (two launches and their first loads, not memory).  Without the next block in
+// 1 x 4002 203 -> 14 (two launches and their first loads, not memory).  Without the next block in
 // flight the same kernel takes 350 us at 190 x 700 to 1300; at 3 waves a SIMD the registers for
 // it are not there.
 #include "common_t.h"
@@ -63,7 +63,7 @@ static DEV Blocks visible_blocks(const GroupedArgs& a, int pos) {
 
 // A sequence's pieces: ``n`` blocks, ``size`` of them a piece, numbered from ``first`` on.
 struct Pieces {
-  int seq, n, size, pieces, first;
+  int seq, len, n, size, pieces, first;
 };
 
 // sum of the lanes up to this one (row shifts and broadcasts of rows' last lanes)
@@ -73,6 +73,14 @@ static DEV int wave_scan(int v) {
   SCAN(0x142, 0xa); SCAN(0x143, 0xc);
 #undef SCAN
   return v;
+}
+
+// n / d of whole numbers, 0 <= n < 2^22 (DECODE_KEYS); the general division is three times as long
+static DEV int quotient(int n, int d) {
+  int q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));
+  const int rest = n - q * d;
+  q += rest >= d;
+  return q - (rest < 0);
 }
 
 // a value and the one of lane ^ 16 or lane ^ 32
@@ -96,47 +104,56 @@ static DEV float max_with(float v) {
 }
 
 // Pieces have about equally many blocks, a multiple of 4, so many that they are at most
-// a.pieces and one for every sequence.  Half as many pieces, one round of workgroups, are better while they
-// are short (20 x 300 to 1024 keys: 24 us, else 29) or are whole sequences (64 x 1024: 60, else
-// 69); long parts are too uneven (61 x 310 to 4000: 141, else 122).  a.pieces == 0: every
-// sequence is one piece.  Finds those of sequence ``want``, or those with piece ``item``
-// (pieces == 0: there is none).  A wave's lanes read the lengths, 64 at a time.
+// a.pieces and one for every sequence.  Half as many pieces, one round of workgroups, are better
+// while they have up to 12 blocks (20 x 300 to 1024 keys: 24 us, else 29; with up to 16, 50 x 400 to
+// 1500 in windows of 1024: 49.9, else 46.3) or are whole sequences (64 x 1024: 60, else 69); long
+// parts are too uneven (61 x 310 to 4000: 141, else 122).  a.pieces == 0: every sequence is one
+// piece.  Finds those of sequence ``want``, or those with piece ``item`` (pieces == 0: there is
+// none).  A wave's lanes read the lengths, 64 at a time.
+// Every workgroup begins with this and then waits for its first keys, so that its length counts: with
+// general divisions and a length read twice 64 x 128 keys took 16.6 us, now 15.5, 16 x 1024 with two
+// heads a key head 22.1 and 21.2.  Fewer workgroups with several pieces each: 1 us more.
 static DEV Pieces find_pieces(const GroupedArgs& a, int want, int item) {
   const int lane = threadIdx.x & 63;
-  auto blocks_of = [&](int seq) {
-    return seq < a.seqs ? visible_blocks(a, a.seq_lens[seq] - 1).n : 0;
-  };
-  Pieces p = {0, 0, 0, 0, 0};
+  auto len_of = [&](int seq) { return seq < a.seqs ? a.seq_lens[seq] : 0; };
+  auto blocks_of = [&](int len) { return visible_blocks(a, len - 1).n; };
+  Pieces p = {0, 0, 0, 0, 0, 0};
   if (a.pieces == 0) {
     p.seq = p.first = item;
-    p.n = p.size = blocks_of(item);
+    p.len = a.seq_lens[item];
+    p.n = p.size = blocks_of(p.len);
     p.pieces = 1;
     return p;
   }
-  const int mine0 = blocks_of(lane);
+  const int len0 = len_of(lane), mine0 = blocks_of(len0);
   int total = mine0, longest = mine0;
   for (int s = 64; s < a.seqs; s += 64) {
-    const int n = blocks_of(s + lane);
+    const int n = blocks_of(len_of(s + lane));
     total += n;
     longest = max(longest, n);
   }
   total = __builtin_amdgcn_readlane(wave_scan(total), 63);
-  const int half = max(1, (total + 2 * a.pieces - 1) / (2 * a.pieces));
-  const int all = max(min(half, 4), (total + 4 * a.pieces - 1) / (4 * a.pieces));
+  const int half = max(1, quotient(total + 2 * a.pieces - 1, 2 * a.pieces));
+  const int all = max(min(half, 3), (half + 1) / 2);
   const int size = 4 * (__any(longest > 4 * half) ? all : half);
+  const int spare = size - (size < 12 ? 0 : size / 4) - 1;
   int before = 0;
   for (int s = 0; s < a.seqs; s += 64) {
-    const int n = s ? blocks_of(s + lane) : mine0;
+    const int len = s ? len_of(s + lane) : len0, n = s ? blocks_of(len) : mine0;
     // a last piece of under a quarter is shared by the others
-    const int about = max(1, (n + size - (size < 12 ? 0 : size / 4) - 1) / size);
-    const int each = about * size >= n ? size : 4 * ((n + 4 * about - 1) / (4 * about));
-    const int k = s + lane < a.seqs ? max(1, (n + each - 1) / each) : 0;
+    int k = max(1, quotient(n + spare, size)), each = size;
+    if (k * size < n) {
+      each = 4 * quotient(n + 4 * k - 1, 4 * k);
+      k = quotient(n + each - 1, each);
+    }
+    if (s + lane >= a.seqs) k = 0;
     const int upto = before + wave_scan(k);  // pieces up to this lane's
     const bool mine = want >= 0 ? s + lane == want : item >= upto - k && item < upto;
     const uint64_t hit = __ballot(mine);
     if (hit) {
       const int at = __builtin_ctzll(hit);
       p.seq = s + at;
+      p.len = __builtin_amdgcn_readlane(len, at);
       p.n = __builtin_amdgcn_readlane(n, at);
       p.size = __builtin_amdgcn_readlane(each, at);
       p.pieces = __builtin_amdgcn_readlane(k, at);
@@ -158,9 +175,9 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   __shared__ float lds_acc[4][GM][V];
   __shared__ float2 lds_ml[4][GM];
   __shared__ int slots[PAGED ? 1 : 4][KB];
-  const int group = a.H / a.G, per = (group + GM - 1) / GM;  // workgroups per kv head
-  const int part = blockIdx.x % per;
-  const int kvh = blockIdx.x / per % a.G, item = blockIdx.x / (per * a.G);
+  const int group = a.group, per = (group + GM - 1) / GM;  // workgroups per kv head
+  const int item = blockIdx.x / (per * a.G), at_g = blockIdx.x - item * per * a.G;
+  const int kvh = per > 1 ? at_g / per : at_g, part = at_g - kvh * per;
   const int h0 = kvh * group + part * GM, heads = min(GM, group - part * GM);
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, j = lane >> 4;           // product: column (head), rows 4 j ..
@@ -168,7 +185,7 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
 
   const Pieces p = find_pieces(a, -1, item);
   if (p.pieces == 0) return;  // more workgroups than pieces
-  const int seq = p.seq, pos = a.seq_lens[seq] - 1, nth = item - p.first;
+  const int seq = p.seq, pos = p.len - 1, nth = item - p.first;
   const Blocks blocks = visible_blocks(a, pos);
   const int end = min(p.n, (nth + 1) * p.size);
   const int lo = first_key(a, pos);
@@ -374,34 +391,46 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   }
 }
 
-// Merge the pieces of one row: a workgroup of V threads per (head, sequence).
-template <bool SIG>
-__global__ __launch_bounds__(256) void merge_pieces_kernel(const GroupedArgs a, const int v) {
-  const int h = blockIdx.x, seq = blockIdx.y, e = threadIdx.x;
+// Merge the pieces of the rows: a lane has 4 dims of a head.  Workgroups are few, so that those
+// with nothing to merge cost little: one wave each up to MERGE_ROWS rows, else 4.
+#define MERGE_ROWS 1024
+template <int VN, bool SIG>
+__global__ __launch_bounds__(256) void merge_pieces_kernel(const GroupedArgs a) {
+  constexpr int V = 64 * VN, LANES = V / 4;  // lanes a head
+  const int at = blockIdx.x * blockDim.x + threadIdx.x;
+  const int h = min(at / LANES, a.H - 1), e = at % LANES * 4, seq = blockIdx.y;
   const Pieces p = find_pieces(a, seq, -1);
   if (p.pieces == 1) return;  // written by the piece's workgroup
-  float m = NEG, l = 0.f, o = 0.f;
+  float m = NEG, l = 0.f, o[4] = {};
   if (!SIG) {
     // maxima and sums, a lane each
-    float sum = 0.f;
-    const int lane = threadIdx.x & 63;
-    for (int i = lane; i < p.pieces; i += 64) m = fmaxf(m, a.part_ml[(int64_t)(p.first + i) * a.H + h].x);
-    m = wave_max(m);
-    for (int i = lane; i < p.pieces; i += 64) {
+    for (int i = e / 4; i < p.pieces; i += LANES)
+      m = fmaxf(m, a.part_ml[(int64_t)(p.first + i) * a.H + h].x);
+#pragma unroll
+    for (int off = LANES / 2; off; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    for (int i = e / 4; i < p.pieces; i += LANES) {
       const float2 ml = a.part_ml[(int64_t)(p.first + i) * a.H + h];
-      sum += ml.y * __builtin_amdgcn_exp2f(ml.x - m);
+      l += ml.y * __builtin_amdgcn_exp2f(ml.x - m);
     }
-    l = wave_sum(sum);
+#pragma unroll
+    for (int off = LANES / 2; off; off >>= 1) l += __shfl_xor(l, off, 64);
   }
 #pragma unroll 8
   for (int i = 0; i < p.pieces; ++i) {
-    const int64_t at = (int64_t)(p.first + i) * a.H + h;
-    const float w = SIG ? 1.f : __builtin_amdgcn_exp2f(a.part_ml[at].x - m);
-    o += w * a.part[at * v + e];
+    const int64_t row = (int64_t)(p.first + i) * a.H + h;
+    const float w = SIG ? 1.f : __builtin_amdgcn_exp2f(a.part_ml[row].x - m);
+    const float4 v = *(const float4*)(a.part + row * V + e);
+    o[0] += w * v.x;
+    o[1] += w * v.y;
+    o[2] += w * v.z;
+    o[3] += w * v.w;
   }
-  if (!SIG) o = l > 0.f ? o / l : 0.f;
-  if (a.gate) o *= sigmoid_f(bf2f(((const bf16_t*)a.gate)[seq * a.gate_stride + h]));
-  ((bf16_t*)a.out)[seq * a.out_stride + (int64_t)h * v + e] = from_f<bf16_t>(o);
+  if (at / LANES >= a.H) return;
+  float by = SIG ? 1.f : l > 0.f ? 1.f / l : 0.f;
+  if (a.gate) by *= sigmoid_f(bf2f(((const bf16_t*)a.gate)[seq * a.gate_stride + h]));
+#pragma unroll
+  for (int n = 0; n < 4; ++n) o[n] *= by;
+  store_f<4>((bf16_t*)a.out + seq * a.out_stride + (int64_t)h * V + e, o);
 }
 
 // Any dtype and size: a workgroup per (token, head), its 4 waves stride over the keys,
@@ -513,8 +542,7 @@ __global__ __launch_bounds__(256) void cache_keys_values_kernel(
 
 template <int DN, int VN, int GM, bool SIG>
 static void launch_decode(const GroupedArgs& a, hipStream_t stream) {
-  const int group = a.H / a.G;
-  const int grid = (a.pieces + a.seqs) * a.G * ((group + GM - 1) / GM);
+  const int grid = (a.pieces + a.seqs) * a.G * ((a.group + GM - 1) / GM);
   const bool paged = a.kv_block >= 16 && (a.kv_block & (a.kv_block - 1)) == 0;
   auto kernel = paged ? grouped_decode_kernel<DN, VN, GM, SIG, true>
                       : grouped_decode_kernel<DN, VN, GM, SIG, false>;
@@ -525,6 +553,8 @@ template <int DN, int VN>
 static bool launch_decode(const GroupedArgs& a, int gm, hipStream_t stream) {
   if (gm == 1)
     (a.sigmoid ? launch_decode<DN, VN, 1, true> : launch_decode<DN, VN, 1, false>)(a, stream);
+  else if (gm == 2)
+    (a.sigmoid ? launch_decode<DN, VN, 2, true> : launch_decode<DN, VN, 2, false>)(a, stream);
   else if (gm == 4)
     (a.sigmoid ? launch_decode<DN, VN, 4, true> : launch_decode<DN, VN, 4, false>)(a, stream);
   else if (gm == 8)
@@ -532,8 +562,9 @@ static bool launch_decode(const GroupedArgs& a, int gm, hipStream_t stream) {
   else
     return false;
   if (a.pieces == 0) return true;
-  auto merge = a.sigmoid ? merge_pieces_kernel<true> : merge_pieces_kernel<false>;
-  merge<<<dim3(a.H, a.seqs), 64 * VN, 0, stream>>>(a, 64 * VN);
+  auto merge = a.sigmoid ? merge_pieces_kernel<VN, true> : merge_pieces_kernel<VN, false>;
+  const int threads = a.H * a.seqs <= MERGE_ROWS ? 64 : 256, lanes = a.H * 16 * VN;
+  merge<<<dim3((lanes + threads - 1) / threads, a.seqs), threads, 0, stream>>>(a);
   return true;
 }
 
@@ -564,7 +595,7 @@ static bool launch_plain(const GroupedArgs& a, int d, int v, int tokens, hipStre
 
 extern "C" {
 
-// gm: query heads of one key/value head per workgroup, 1, 4 or 8
+// gm: query heads of one key/value head per workgroup, 1, 2, 4 or 8
 bool launch_grouped_decode(const GroupedArgs* a, int d, int v, int gm, hipStream_t stream) {
   switch (d) {
     case 64: return launch_decode_v<1>(*a, v, gm, stream);

@@ -4,6 +4,7 @@
 All tests are @gpu — run via gpurun on an MI355X.
 """
 import math
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -158,6 +159,73 @@ def test_decode_pieces(block, H, G, lens):
         w = torch.softmax((k * q[b].float()).sum(-1) * 0.09, 0)
         # fp32 but for the result: 2^-9 of values up to 5
         assert maxerr(out[b], (w.unsqueeze(-1) * v).sum(0)) < 0.012, (b, lens[b])
+
+
+STEADY = {  # lengths, heads, key heads, head size, options
+    "ragged": ([300 + 97 * i * 53 % 3701 for i in range(44)], 32, 8, 128, {}),
+    "over_64": ([150 + 97 * i * 61 % 1501 for i in range(90)], 16, 8, 128, {}),
+    "one": ([4003], 28, 4, 128, {}),
+    "whole": ([301 + 97 * i * 37 % 403 for i in range(130)], 16, 8, 128, {}),
+    "window": ([200 + 97 * i * 71 % 2801 for i in range(41)], 16, 8, 128,
+               dict(window=1000, keep_first=5, cap=20.0, sink=True)),
+    "sigmoid": ([900 + 97 * i * 71 % 1801 for i in range(24)], 12, 4, 128, dict(sigmoid=True)),
+    "wide": ([700 + 97 * i * 31 % 2301 for i in range(20)], 12, 2, 256,
+             dict(window=1500, keep_first=70, sink=True)),
+    "narrow": ([500 + 97 * i * 31 % 2301 for i in range(33)], 12, 4, 64, dict(window=1 << 20)),
+}
+
+
+@requires_gpu
+@pytest.mark.parametrize("block", [16, 24, 64])
+@pytest.mark.parametrize("case", STEADY)
+def test_decode_over_many_blocks(case, block):
+    """Several blocks of 32 keys a wave, in pieces of one size, of sizes that are evened out and
+    in whole sequences; what no token has written is NaN."""
+    lens, H, G, d, options = STEADY[case]
+    options = dict(options)
+    gen = torch.Generator().manual_seed(len(lens))
+    need = [-(-n // block) for n in lens]
+    order = torch.randperm(sum(need) + 1, generator=gen)
+    tables = torch.zeros(len(lens), max(need) + 3, dtype=torch.int32)
+    kc, vc = torch.full((2, len(order), block, G, d), float("nan"), device="cuda").bfloat16()
+    rows, at = [], 0
+    for b, (n, k) in enumerate(zip(lens, need)):
+        tables[b, :k] = order[at : at + k]
+        p = torch.arange(n)
+        rows.append((order[at : at + k][p // block] * block + p % block).cuda())
+        at += k
+        for c in (kc, vc):
+            c.view(-1, G, d)[rows[b]] = torch.randn(n, G, d, device="cuda").bfloat16()
+    q = (2 * torch.randn(len(lens), H, d, generator=gen)).bfloat16().cuda()
+    seq_lens, scale = torch.tensor(lens, dtype=torch.int32).cuda(), d ** -0.5
+    sink = torch.randn(H, generator=gen).cuda() if options.pop("sink", None) else None
+    if options:
+        batch = SimpleNamespace(
+            num_prefill_tokens=0, prefills=[], num_decode=len(lens),
+            decode_tables_i32=lambda t=tables.cuda(): t, decode_lens_i32=lambda: seq_lens,
+        )
+        form = {"cap": None, "window": None, "keep_first": 0, **options}
+        out = torch.empty_like(q)
+        hip().grouped_attention(q, kc, vc, batch, scale, sink=sink, out=out, **form)
+    else:
+        form = {"cap": None, "window": None, "keep_first": 0}
+        out = hip().attention_decode_raw(q, kc, vc, tables.cuda(), seq_lens, scale)
+    for b, n in enumerate(lens):
+        k, v = (c.view(-1, G, d)[rows[b]].float().repeat_interleave(H // G, 1) for c in (kc, vc))
+        s = (k * q[b].float()).sum(-1) * scale
+        if form["cap"]:
+            s = form["cap"] * torch.tanh(s / form["cap"])
+        if form["window"]:
+            p = torch.arange(n, device="cuda")[:, None]
+            s = s.masked_fill((p <= n - 1 - form["window"]) & (p >= form["keep_first"]), -math.inf)
+        if form.get("sigmoid"):
+            w = torch.sigmoid(s)
+        else:
+            w = torch.softmax(s if sink is None else torch.cat([s, sink[None]]), 0)[:n]
+        want = (w.unsqueeze(-1) * v).sum(0)
+        # fp32 but for the result: 2^-9 of it, and 2^-20 of sums of up to 4003 terms
+        slack = 2.0 ** -8 * want.abs() + 2.0 ** -20 * (w.unsqueeze(-1) * v.abs()).sum(0) + 1e-4
+        assert ((out[b].float() - want).abs() <= slack).all(), (b, n)
 
 
 @requires_gpu
