@@ -44,7 +44,8 @@ void launch_embed_positions(bool, float*, float*, const int64_t*, const int64_t*
 void launch_attn_inputs(bool, const AttnInputsArgs*, hipStream_t);
 void launch_moe_route(bool, int*, float*, const void*, const void*, const float*, int, int, int,
                       int, int64_t, bool, float, hipStream_t);
-void launch_moe_group(int*, int*, int*, int*, const int*, int, int, int, hipStream_t);
+void launch_moe_group(int*, int*, int*, int*, const int*, int, int, const TiledProducts*,
+                      hipStream_t);
 void launch_experts_small(bool, const ExpertsArgs*, int, hipStream_t);
 void launch_experts_f32(bool, const ExpertsArgs*, hipStream_t);
 void launch_experts_gemm(bool, const ExpertsArgs*, hipStream_t);
@@ -926,19 +927,23 @@ static void moe_route(torch::Tensor ids, torch::Tensor weights, torch::Tensor h,
                    h.stride(0), sigmoid, (float)scale, cur_stream());
 }
 
-// perm [n], offsets [E + 2]; tiles of at least EXPERT_TILE rows: at most ceil(n / tile) + E, each
-// multiplied in this many columns of workgroups
+// perm [n], offsets [E + 2]; tiles of at least EXPERT_TILE rows: at most ceil(n / tile) + E, for
+// products with these many inner elements and outputs
 static void moe_group(torch::Tensor perm, torch::Tensor offsets, OptTensor tile_expert,
-                      OptTensor tile_row, torch::Tensor ids, int64_t E, int64_t columns) {
+                      OptTensor tile_row, torch::Tensor ids, int64_t E, int64_t width,
+                      int64_t inner, int64_t outputs) {
   const int64_t n = ids.numel();
   CHECK_CUDA(ids); CHECK_CONT(ids);
   TORCH_CHECK(ids.scalar_type() == at::kInt && E > 0 && E <= 512 && n < (1 << 30));
-  const int64_t tiles = tile_expert ? n / EXPERT_TILE + E : 0;
+  const int64_t most = n / EXPERT_TILE + E, tiles = tile_expert ? most : 0;
   int* te = (int*)opt_int(tile_expert, tiles);
   int* tr = (int*)opt_int(tile_row, tiles);
-  TORCH_CHECK(!te == !tr && columns > 0 && columns * (n / EXPERT_TILE + E) < (1 << 30), "tiles");
+  const int64_t columns1 = (inner + 127) / 128, columns2 = (outputs + 255) / 256;
+  TORCH_CHECK(!te == !tr && width > 0 && width < (1 << 30) && inner > 0 && outputs > 0 &&
+              std::max(columns1, columns2) * most < (1 << 30), "tiles");
+  const TiledProducts sizes = {(int)width, (int)columns1, (int)inner, (int)columns2};
   launch_moe_group((int*)opt_int(perm, n), (int*)opt_int(offsets, E + 2), te, tr,
-                   ids.data_ptr<int>(), (int)n, (int)E, (int)columns, cur_stream());
+                   ids.data_ptr<int>(), (int)n, (int)E, &sizes, cur_stream());
 }
 
 // One product of the routed experts (experts.h).  kind: 0 fp32, 1 few rows, 2 tiles

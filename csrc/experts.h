@@ -18,6 +18,12 @@ struct ExpertsArgs {
   float limit, alpha, offset, cubic;  // gate_up: the gated unit
 };
 
+// Sizes of the two tiled products: inner elements and columns of workgroups of a tile
+struct TiledProducts {
+  int width, columns1;  // gate and up
+  int inner, columns2;  // down
+};
+
 // rows of one tile of the large-batch product, at most TALL_TILE
 #define EXPERT_TILE 256
 #define TALL_TILE 320

@@ -146,7 +146,7 @@ static DEV uint64_t same_id(int id, int bits) {
 __global__ __launch_bounds__(1024) void group_kernel(
     int* __restrict__ perm, int* __restrict__ offsets, int* __restrict__ tile_expert,
     int* __restrict__ tile_row, const int* __restrict__ ids, const int n, const int E,
-    const int columns) {
+    const TiledProducts sizes) {
   extern __shared__ int counts[];
   int* total = counts + 16 * E;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -185,27 +185,49 @@ __global__ __launch_bounds__(1024) void group_kernel(
   }
   __syncthreads();
   if (wid == 0) {  // first rows and tiles of the experts
-    // Tall tiles take up to an eighth longer each, which pays where they save a round of
-    // workgroups (one a CU, columns a tile): 16 experts of 256 rows and few more, 10 columns, 120
-    // us in tiles of 256, 135 in tall ones; 32 of 512 and few more, 20 columns, both products
-    // 1364 and 1094.
-    int plain_tiles = 0, tall_tiles = 0;
-    for (int e = lane; tile_expert && e < E; e += 64) {
-      const int c = total[e], high = tall_tile(c);
-      plain_tiles += (c + EXPERT_TILE - 1) / EXPERT_TILE;
-      tall_tiles += (c + high - 1) / high;
-    }
-    auto rounds = [&](int tiles) {
+    // Tall tiles take up to an eighth longer each, which pays where they save rounds of
+    // workgroups (one a CU, columns a tile) in one of the two products; a tile of up to 192 rows
+    // takes about 0.6 of a round.  Both products, us, in tiles of 256 and tall ones: 32 experts,
+    // 4 of them a token at random, 2560 inner, 4096 outputs: 2048 tokens 853 and 665, 4093 1342
+    // and 1091, 6500 1910 and 1707, but 2600 880 and 1007, 7500 1822 and 1987; 16, 2 a token,
+    // 1280 inner, 2048 outputs: 1800 tokens 138 and 140, 4093 241 and 212. Taken where it is not
+    // faster: 2500 and 7000 tokens of the first (870 and 884, 1753 and 1819).
+    bool tall = false;
+    if (tile_expert) {
+      int tiles[2] = {}, small[2] = {};  // of 256 rows, tall
+      for (int e = lane; e < E; e += 64) {
+        const int c = total[e], t = (c + EXPERT_TILE - 1) / EXPERT_TILE;
+        const int high = (c + TALL_TILE - 1) / TALL_TILE;
+        const bool whole = c > EXPERT_TILE * high, last = c > 0 && c - EXPERT_TILE * (t - 1) <= 192;
+        tiles[0] += t;
+        small[0] += last;
+        tiles[1] += whole ? high : t;
+        small[1] += whole ? 0 : last;
+      }
+      float cost[2];
 #pragma unroll
-      for (int off = 32; off; off >>= 1) tiles += __shfl_xor(tiles, off, 64);
-      return (tiles * columns + 255) / 256;
-    };
-    const bool tall = tile_expert && rounds(tall_tiles) * 9 < rounds(plain_tiles) * 8;
+      for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int off = 32; off; off >>= 1) {
+          tiles[i] += __shfl_xor(tiles[i], off, 64);
+          small[i] += __shfl_xor(small[i], off, 64);
+        }
+        auto rounds = [&](int columns) {
+          return (float)((tiles[i] * columns + 255) / 256) - 0.4f / 256 * (small[i] * columns);
+        };
+        cost[i] = sizes.width * rounds(sizes.columns1) + sizes.inner * rounds(sizes.columns2);
+      }
+      tall = cost[1] < 0.92f * cost[0];
+    }
     int row = 0, tile = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + lane;
-      const int c = e < E ? total[e] : 0, high = tall ? tall_tile(c) : EXPERT_TILE;
-      const int t = (c + high - 1) / high;
+      const int c = e < E ? total[e] : 0;
+      int high = EXPERT_TILE, t = (c + EXPERT_TILE - 1) / EXPERT_TILE;
+      if (tall) {
+        high = tall_tile(c);
+        t = (c + high - 1) / high;
+      }
       int cs = c, ts = t;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
@@ -367,9 +389,9 @@ void launch_moe_route(bool bf16, int* ids, float* weights, const void* h, const 
 }
 
 void launch_moe_group(int* perm, int* offsets, int* tile_expert, int* tile_row, const int* ids,
-                      int n, int E, int columns, hipStream_t stream) {
+                      int n, int E, const TiledProducts* sizes, hipStream_t stream) {
   group_kernel<<<1, 1024, 17 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E,
-                                                columns);
+                                                *sizes);
 }
 
 // tt: token fragments at a time, 1 or 2

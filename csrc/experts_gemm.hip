@@ -19,8 +19,9 @@
 //
 // 32 experts of 4096 x 2560, both products: 512 rows each 1212 us; 520 rows 1568 with a third tile
 // for 8 of them, which reads 2 GB of weights once more at 5.5 TB/s, 1295 in two tall tiles. At
-// random to 4 of 32, 2048 tokens 887, now 652; 4093 1364, now 1094; 8192 2260, now 2119. Tiles of
-// up to 128 rows with 3 or 4 chunks in flight gained nothing.
+// random to 4 of 32 (group_kernel chooses), before and with tall tiles: 2048 tokens 799 and 678,
+// 4093 1300 and 1091, 8192 2271 and 2011. Tiles of up to 128 rows with 3 or 4 chunks in flight
+// gained nothing.
 #include <type_traits>
 
 #include "experts.h"

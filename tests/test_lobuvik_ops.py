@@ -533,6 +533,34 @@ def test_experts_tile_heights(I):
             close(got[t, 0], oracle.clamped_glu(h.double().cpu()[t], x, "", 1.25), torch.bfloat16)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,tiles", [(128, 33), (1024, 26)], ids=["plain", "tall"])
+def test_experts_choose_tile_heights(K, tiles):
+    """Tall tiles where they save a round of the larger product (660 workgroups, 520), not where
+    that product is the smaller part; the results are the same to a rounding."""
+    from agentcontrolplane_amd import _C
+
+    rows = [0, 1, 64, 65, 255, 256, 257, 288, 289, 320, 321, 512, 513, 577, 640, 641, 961]
+    E, I, W = len(rows), 2432, 520
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).int()
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(2))].view(-1, 1)
+    h = rand(len(ids), K, dtype=torch.bfloat16, device="cuda")
+    gate_up = rand(E, 2 * I, K, dtype=torch.bfloat16, device="cuda", seed=1, scale=2 * K ** -0.5)
+    down = rand(E, W, I, dtype=torch.bfloat16, device="cuda", seed=2, scale=I ** -0.5)
+    ids, spec = ids.cuda(), ClampedGluSpec(I, 1.25)
+    made = torch.empty(3, len(ids) // _C.EXPERT_TILE + E, dtype=torch.int32, device="cuda")
+    perm, offsets = torch.empty_like(ids[:, 0]), made.new_empty(E + 2)
+    _C.moe_group(perm, offsets, made[0], made[1], ids, E, K, I, W)
+    assert offsets[E + 1].item() == tiles
+    got = ops.moe_experts(h, gate_up, down, ids, spec)
+    for e, n in enumerate(rows):
+        if n:
+            x = {"gate": gate_up[e, :I].double(), "up": gate_up[e, I:].double(),
+                 "down": down[e].double()}
+            t = (ids[:, 0] == e).nonzero()[:, 0]
+            close(got[t, 0], oracle.clamped_glu(h[t].double(), x, "", 1.25), torch.bfloat16)
+
+
 @pytest.mark.parametrize("skew", [False, True])
 @pytest.mark.parametrize("n,E,top,K,I,W", EXPERTS)
 def test_experts(device, dtype, n, E, top, K, I, W, skew):
