@@ -63,26 +63,43 @@ def _aligned(t):
     return t.clone(memory_format=torch.contiguous_format)
 
 
-def attention_prefill_batch(q, k_cache, v_cache, batch, scale, out=None):
+def _attend_into(out, q, attend):
+    """attend(a tensor of q's shape) into ``out``: any contiguous memory for it, or None."""
     if out is None:
         out = _attn_out(q)
+    if not out.is_contiguous():
+        raise RuntimeError("out must be contiguous")
+    to = out if out.shape == q.shape else out.view(-1)[: q.numel()].view(q.shape)
+    if to.data_ptr() % 16 == 0:
+        attend(to)
+    else:  # the kernels write whole units of 16 bytes
+        there = _attn_out(q)
+        attend(there)
+        to.copy_(there)
+    return out
+
+
+def attention_prefill_batch(q, k_cache, v_cache, batch, scale, out=None):
     if _PREFILL_IMPL == "mfma":
         if q.shape[2] != 128:
             raise RuntimeError("prefill kernel requires head_dim 128")
-        q = _aligned(q)
         meta = batch.prefill_meta(tile_q=128)
-        _C.grouped_attn(
-            out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens, meta.ctx_lens,
-            meta.row_starts, meta.tile_seq, meta.tile_q0, *(None,) * 6,
-            scale, 0.0, _NO_WINDOW, _NO_WINDOW, 0, False, _PREFILL, 1, 1,
-        )
+
+        def attend(to):
+            _C.grouped_attn(
+                to, _aligned(q), k_cache, v_cache, meta.block_tables, meta.seq_lens,
+                meta.ctx_lens, meta.row_starts, meta.tile_seq, meta.tile_q0, *(None,) * 6,
+                scale, 0.0, _NO_WINDOW, _NO_WINDOW, 0, False, _PREFILL, 1, 1,
+            )
     else:
         meta = batch.prefill_meta(tile_q=64)
-        _C.prefill_attn(
-            out, q, k_cache, v_cache, meta.block_tables, meta.seq_lens, meta.ctx_lens,
-            meta.row_starts, meta.tile_seq, meta.tile_q0, scale,
-        )
-    return out
+
+        def attend(to):
+            _C.prefill_attn(
+                to, q, k_cache, v_cache, meta.block_tables, meta.seq_lens, meta.ctx_lens,
+                meta.row_starts, meta.tile_seq, meta.tile_q0, scale,
+            )
+    return _attend_into(out, q, attend)
 
 
 def attention_decode_batch(q, k_cache, v_cache, batch, scale, out=None):
@@ -98,17 +115,14 @@ def attention_decode_raw(q, k_cache, v_cache, block_tables, seq_lens, scale):
 
 
 def _attention_decode(q, k_cache, v_cache, tables, seq_lens, scale, out=None):
-    if out is None:
-        out = _attn_out(q)
     if q.shape[2] != 128:
         raise RuntimeError("decode kernel requires head_dim 128")
     if q.shape[1] > 8 * k_cache.shape[2]:
         raise RuntimeError("GQA group must be <= 8")
-    _grouped_decode(
-        out, _aligned(q), k_cache, v_cache, tables, seq_lens, None, None, None, scale, 0.0,
+    return _attend_into(out, q, lambda to: _grouped_decode(
+        to, _aligned(q), k_cache, v_cache, tables, seq_lens, None, None, None, scale, 0.0,
         _NO_WINDOW, _NO_WINDOW, 0, False,
-    )
-    return out
+    ))
 
 
 def gemm_bf16(x, w):

@@ -161,6 +161,33 @@ def test_decode_pieces(block, H, G, lens):
         assert maxerr(out[b], (w.unsqueeze(-1) * v).sum(0)) < 0.012, (b, lens[b])
 
 
+@requires_gpu
+@pytest.mark.parametrize("step", ["prompt", "decode"])
+def test_attention_writes_into_any_contiguous_memory(step):
+    """``out`` off a 16-byte boundary, flat, or larger than the result; strided ones are refused."""
+    from op_helpers import make_batch
+
+    H, G, n = 8, 2, 37
+    torch.manual_seed(1)
+    batch, _, tables, pages = make_batch([(0, n)] if step == "prompt" else [(n, 1)] * 3, 16, "cuda")
+    kc, vc = torch.randn(2, pages, 16, G, 128, device="cuda").bfloat16()
+    rows = n if step == "prompt" else 3
+    q = torch.randn(rows, H, 128, device="cuda").bfloat16()
+    attend = hip().attention_prefill_batch if step == "prompt" else hip().attention_decode_batch
+    want = attend(q, kc, vc, batch, 0.1).flatten()
+    size = rows * H * 128
+    for shift, more in [(0, 0), (3, 0), (3, 5), (8, 17)]:
+        space = torch.full((size + 64,), 7.0, device="cuda").bfloat16()
+        out = space[shift : shift + size + more]
+        if more == 0:
+            out = out.view(rows, H * 128)
+        assert attend(q, kc, vc, batch, 0.1, out=out) is out
+        assert torch.equal(space[shift : shift + size], want)
+        assert (space[:shift] == 7).all() and (space[shift + size :] == 7).all()
+    with pytest.raises(RuntimeError, match="contiguous"):
+        attend(q, kc, vc, batch, 0.1, out=q.new_empty(rows, H, 256)[..., :128])
+
+
 STEADY = {  # lengths, heads, key heads, head size, options
     "ragged": ([300 + 97 * i * 53 % 3701 for i in range(44)], 32, 8, 128, {}),
     "over_64": ([150 + 97 * i * 61 % 1501 for i in range(90)], 16, 8, 128, {}),
