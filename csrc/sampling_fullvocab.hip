@@ -1,6 +1,6 @@
 // Full-vocabulary token sampling (gfx950): temperature → optional grammar
 // mask → exact top-k → top-p (nucleus) → inverse-CDF draw in token-id
-// order; one workgroup per row, any vocabulary size (Llama-3: 128256).
+// order; one workgroup per row, vocabularies up to 2^18 (Llama-3: 128256).
 //
 // The ≤512-entry LDS bitonic sampler (sampling.hip) covers the byte
 // tokenizer; a real BPE vocabulary needs per-row selection over 128k
@@ -32,10 +32,8 @@
 //                  cumulative <= p            (boundary-key ties all kept)
 #include "common.h"
 
-#define WG 1024
-#define WAVES (WG / 64)
 #define STRIPES 256
-#define TILE 64         // tokens of a stripe that are summed at a time
+#define MOST_VOCAB (1 << 18)
 #define OCTAVE 64       // first buckets: of m - x, per octave, from 2^-8 to 2^16
 #define FIRST (24 * OCTAVE)
 #define HEAD 12.f       // logits of at least exp(-HEAD) of the largest's weight come first
@@ -56,17 +54,30 @@ __device__ __forceinline__ float ldf(const bf16_t* p) { return bf2f(*p); }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-struct Shared {
+// Threads of a workgroup, and tokens of a stripe that are summed at a time.  With 1024 threads and
+// 160 KB a CU has one row, and each step of a row ends in a wait for 16 waves: small vocabularies
+// take 256 threads and 61 KB.  1024 and 256 threads, us: 512 rows of 600 greedy 10.7 and 5.7, plain
+// 24.9 and 10.9, 16 rows of 4096 plain 14.2 and 9.8, top-p 29 and 24.  From there on only where
+// the rows are more than the CUs: 512 rows of 8192 plain 30.8 and 15.6, but 16 rows top-p with a
+// mask 32 and 39.
+template <int THREADS, int TOKENS>
+struct Form {
+  static constexpr int WG = THREADS, WAVES = WG / 64, TILE = TOKENS;
+  static constexpr int BUCKETS = (FIRST + WG - 1) / WG;  // of a thread
+};
+
+template <typename F>
+struct Shared : F {
   uint32_t count[FIRST];
   unsigned long long mass[FIRST];  // in units of 2^-44: integer atomics are the fast ones
   union {
-    uint32_t list[LIST][WG];
-    float tile[2][STRIPES][TILE + 4];
+    uint32_t list[LIST][F::WG];
+    float tile[2][STRIPES][F::TILE + 4];
   };
   float stripe[STRIPES], cdf[STRIPES + 1];
-  double wave[WAVES];
-  float red[WAVES];
-  int red_i[WAVES];
+  double wave[F::WAVES];
+  float red[F::WAVES];
+  int red_i[F::WAVES];
   int n, pick;
   uint32_t lo, hi;
   double above;
@@ -80,7 +91,7 @@ __device__ __forceinline__ unsigned long long units(float w) {
   return ((unsigned long long)(uint32_t)hi << 20) + (uint32_t)lo;
 }
 
-template <typename T>
+template <typename T, int WG>
 struct Row {
   const T* x;
   const uint8_t* mask;  // or null
@@ -126,34 +137,48 @@ struct Row {
     return min(max(b, 0), FIRST - 1);
   }
 };
-static_assert(TILE == 64, "a wave takes 64 tokens of a stripe");
 static_assert(OCTAVE == 64, "bucket() takes 6 bits of the mantissa");
 
-// The first of ``n`` (at most 2 WG) buckets whose sum with those before and ``above`` reaches
+// The first of ``n`` (at most FIRST) buckets whose sum with those before and ``above`` reaches
 // target, and the sum before it; -1: none does.
-template <bool BY_MASS>
-__device__ int find_bucket(Shared& s, int n, double target, double* above) {
+template <bool BY_MASS, typename S>
+__device__ int find_bucket(S& s, int n, double target, double* above) {
+  constexpr int PER = S::BUCKETS;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  auto at = [&](int i) { return i >= n ? 0.0 : BY_MASS ? s.mass[i] * UNIT : (double)s.count[i]; };
-  const double w0 = at(2 * threadIdx.x), w1 = at(2 * threadIdx.x + 1);
-  double sum = w0 + w1;
+  double w[PER], sum = 0.0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = PER * threadIdx.x + j;
+    w[j] = i >= n ? 0.0 : BY_MASS ? s.mass[i] * UNIT : (double)s.count[i];
+    sum += w[j];
+  }
+  double upto = sum;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
-    const double v = __shfl_up(sum, off, 64);
-    if (lane >= off) sum += v;
+    const double v = __shfl_up(upto, off, 64);
+    if (lane >= off) upto += v;
   }
-  if (lane == 63) s.wave[wid] = sum;
+  if (lane == 63) s.wave[wid] = upto;
   if (threadIdx.x == 0) s.n = 1 << 30;
   __syncthreads();
   double before = *above;
-  for (int w = 0; w < wid; ++w) before += s.wave[w];
-  sum += before;  // up to and with this thread's two
-  const double b1 = sum - w1, b0 = b1 - w0;
-  const int mine = b1 >= target ? 2 * threadIdx.x : sum >= target ? 2 * threadIdx.x + 1 : n;
+  for (int i = 0; i < wid; ++i) before += s.wave[i];
+  before += upto - sum;
+  int mine = n;
+  double mine_before = 0.0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const double after = before + w[j];
+    if (mine == n && after >= target) {
+      mine = min(n, (int)(PER * threadIdx.x) + j);
+      mine_before = before;
+    }
+    before = after;
+  }
   if (mine < n) atomicMin(&s.n, mine);
   __syncthreads();
   const int got = s.n;
-  if (got < n && got / 2 == (int)threadIdx.x) s.above = got % 2 ? b1 : b0;
+  if (mine == got) s.above = mine_before;
   __syncthreads();
   if (got < n) *above = s.above;
   return got < n ? got : -1;
@@ -161,14 +186,14 @@ __device__ int find_bucket(Shared& s, int n, double target, double* above) {
 
 // Splits the keys [lo, hi] among those that each_key(f) hands out until one is left: the one at
 // which the sum from the top reaches target.
-template <bool BY_MASS, typename T, typename E>
-__device__ uint32_t split_keys(Shared& s, const Row<T>& row, uint32_t lo, uint32_t hi,
+template <bool BY_MASS, typename S, typename R, typename E>
+__device__ uint32_t split_keys(S& s, const R& row, uint32_t lo, uint32_t hi,
                                double above, double target, E each_key) {
   for (;;) {
     const uint32_t range = hi - lo;
     const int shift = range < SPLIT ? 0 : 32 - __builtin_clz(range) - 10;
     const int n = (int)(range >> shift) + 1;
-    for (int i = threadIdx.x; i < n; i += WG) {
+    for (int i = threadIdx.x; i < n; i += S::WG) {
       s.count[i] = 0;
       s.mass[i] = 0;
     }
@@ -191,22 +216,23 @@ __device__ uint32_t split_keys(Shared& s, const Row<T>& row, uint32_t lo, uint32
   }
 }
 
-__device__ double block_total(Shared& s, double v) {
+template <typename S>
+__device__ double block_total(S& s, double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   if ((threadIdx.x & 63) == 0) s.wave[threadIdx.x >> 6] = v;
   __syncthreads();
   double t = 0.0;
-  for (int w = 0; w < WAVES; ++w) t += s.wave[w];
+  for (int w = 0; w < S::WAVES; ++w) t += s.wave[w];
   __syncthreads();
   return t;
 }
 
 // Histograms over m - x up to ``far``; the mass of the others: a boundary is seldom among
 // them, and their atomics take most of the time.
-template <bool BY_MASS, typename T>
-__device__ float fill(Shared& s, const Row<T>& row, float far) {
-  for (int i = threadIdx.x; i < FIRST; i += WG) {
+template <bool BY_MASS, typename S, typename R>
+__device__ float fill(S& s, const R& row, float far) {
+  for (int i = threadIdx.x; i < FIRST; i += S::WG) {
     s.count[i] = 0;
     s.mass[i] = 0;
   }
@@ -230,8 +256,8 @@ __device__ float fill(Shared& s, const Row<T>& row, float far) {
 
 // The key at which the sum from the largest logit down reaches target, which is ``part`` of all
 // weights if it is given; 0: nowhere.  ``plain``: all logits are numbers.
-template <bool BY_MASS, typename T>
-__device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double part, bool plain) {
+template <bool BY_MASS, typename S, typename R>
+__device__ uint32_t boundary(S& s, const R& row, double target, double part, bool plain) {
   if (target <= 0.0) return f2key(row.m);  // reached before the first, which is kept all the same
   auto stream = [&](auto f) { row.each([&](int, float v) { f(f2key(v)); }); };
   if (!plain) return split_keys<BY_MASS>(s, row, 0u, 0xffffffffu, 0.0, target, stream);
@@ -239,7 +265,7 @@ __device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double
   const float rest = fill<BY_MASS>(s, row, HEAD / row.invT);
   if (part > 0.0) {
     double all = 0.0;
-    for (int i = threadIdx.x; i < FIRST; i += WG) all += s.mass[i] * UNIT;
+    for (int i = threadIdx.x; i < FIRST; i += S::WG) all += s.mass[i] * UNIT;
     target = part * block_total(s, all + rest);
     if (target <= 0.0) return f2key(row.m);
   }
@@ -283,8 +309,8 @@ __device__ uint32_t boundary(Shared& s, const Row<T>& row, double target, double
   });
 }
 
-template <typename T>
-__global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
+template <typename T, typename F>
+__global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(
     int64_t* __restrict__ out,           // [B]
     const T* __restrict__ logits,        // [B, V]
     const float* __restrict__ temps,     // [B]
@@ -294,14 +320,15 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
     const uint8_t* __restrict__ mask,    // [M, V] bool, may be null
     const int32_t* __restrict__ mask_map,// [B] row -> mask row (-1 = none)
     const int V) {
-  __shared__ Shared s;
+  constexpr int WG = F::WG, WAVES = F::WAVES, TILE = F::TILE;
+  __shared__ Shared<F> s;
   const int n_row = blockIdx.x, t = threadIdx.x, lane = t & 63, wid = t >> 6;
   // compact masks: only constrained rows carry one (a dense [B,V] mask at
   // B=1k, V=128k would be 128 MB of pinned staging per step)
   const bool masked = mask && mask_map && mask_map[n_row] >= 0;
   const float Tmp = temps[n_row];
   const bool greedy = Tmp <= 0.f;
-  Row<T> row = {logits + (int64_t)n_row * V,
+  Row<T, WG> row = {logits + (int64_t)n_row * V,
                 masked ? mask + (int64_t)mask_map[n_row] * V : nullptr, V, 0.f,
                 greedy ? 1.f : 1.f / Tmp};
 
@@ -370,7 +397,7 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
   const int stride = (V + STRIPES - 1) / STRIPES;
   constexpr int PER = STRIPES * TILE / WG, ROWS = WG / TILE;  // a thread's tokens of a tile
   // token of the thread's k-th of a tile: k * ROWS stripes on
-  const int i_first = wid * stride + lane;
+  const int r = t / TILE, c = t % TILE, i_first = r * stride + c;
   float ahead[PER];
   auto fetch = [&](int j0) {
 #pragma unroll
@@ -389,14 +416,14 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
     if (even && by_value && plain && !row.mask && j0 + TILE <= stride) {
 #pragma unroll
       for (int k = 0; k < PER; ++k)
-        tile[k * ROWS + wid][lane] = ahead[k] >= from ? row.weight(ahead[k]) : 0.f;
+        tile[k * ROWS + r][c] = ahead[k] >= from ? row.weight(ahead[k]) : 0.f;
     } else {
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
         const int i = k * ROWS * stride + j0 + i_first;
-        const bool in = j0 + lane < stride && i < V && f2key(ahead[k]) >= kmin &&
+        const bool in = j0 + c < stride && i < V && f2key(ahead[k]) >= kmin &&
                         !(row.mask && !row.mask[i]);
-        tile[k * ROWS + wid][lane] = in ? row.weight(ahead[k]) : 0.f;
+        tile[k * ROWS + r][c] = in ? row.weight(ahead[k]) : 0.f;
       }
     }
     if (j0 + TILE < stride) fetch(j0 + TILE);
@@ -437,46 +464,36 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
     // the stripe's weights, added up in order by one thread until they exceed the target;
     // its last kept token if rounding lets none do so
     float* const buf = &s.tile[0][0][0];
-    constexpr int ROOM = 4096;
-    float cum = s.cdf[n];
-    const int end = min(stride, V - n * stride);
-    for (int j0 = 0; j0 < end; j0 += ROOM) {
-      const int here = min(end - j0, ROOM), i0 = n * stride + j0;
-      int last = -1;
-      for (int j = t; j < (here + STEP - 1) / STEP * STEP; j += WG) {
-        float w = 0.f;
-        if (j < here && !(row.mask && !row.mask[i0 + j])) {
-          const float v = ldf(row.x + i0 + j);
-          if (f2key(v) >= kmin) {
-            w = row.weight(v);
-            last = i0 + j;
-          }
+    static_assert(sizeof(s.tile) >= 4 * (MOST_VOCAB / STRIPES + STEP), "a stripe fits");
+    const int i0 = n * stride, here = min(stride, V - i0);
+    int last = -1;
+    for (int j = t; j < (here + STEP - 1) / STEP * STEP; j += WG) {
+      float w = 0.f;
+      if (j < here && !(row.mask && !row.mask[i0 + j])) {
+        const float v = ldf(row.x + i0 + j);
+        if (f2key(v) >= kmin) {
+          w = row.weight(v);
+          last = i0 + j;
         }
-        buf[j] = w;
       }
-      if (last >= 0) atomicMax(&s.pick, last);
-      if (t == 0) s.n = -1;
-      __syncthreads();
-      if (t == 0) {
-        for (int j = 0; j < here && s.n < 0; j += STEP) {
-          float w[STEP];
+      buf[j] = w;
+    }
+    if (last >= 0) atomicMax(&s.pick, last);
+    __syncthreads();
+    if (t == 0) {
+      float cum = s.cdf[n];
+      int first = STEP;
+      for (int j = 0; j < here && first == STEP; j += STEP) {
+        float w[STEP];
 #pragma unroll
-          for (int e = 0; e < STEP; e += 4) *(float4*)(w + e) = *(const float4*)(buf + j + e);
-          int first = STEP;
+        for (int e = 0; e < STEP; e += 4) *(float4*)(w + e) = *(const float4*)(buf + j + e);
 #pragma unroll
-          for (int e = 0; e < STEP; ++e) {
-            cum += w[e];
-            if (first == STEP && cum > target) first = e;
-          }
-          if (first < STEP) {
-            s.n = i0 + j + first;
-            break;
-          }
+        for (int e = 0; e < STEP; ++e) {
+          cum += w[e];
+          if (first == STEP && cum > target) first = e;
         }
-        if (s.n >= 0) s.pick = s.n;
+        if (first < STEP) s.pick = i0 + j + first;
       }
-      __syncthreads();
-      if (s.n >= 0) break;
     }
   }
   __syncthreads();
@@ -497,19 +514,25 @@ __global__ __launch_bounds__(WG) void sample_fullvocab_kernel(
   if (t == 0) out[n_row] = s.pick;
 }
 
+template <typename T>
+static void launch(int64_t* out, const T* logits, const float* temps, const int64_t* top_ks,
+                   const float* top_ps, const float* uniforms, const uint8_t* mask,
+                   const int32_t* mask_map, int B, int V, hipStream_t stream) {
+  using Small = Form<256, 16>;
+  using Large = Form<1024, 64>;
+  const bool small = V <= 4096 || (V <= 8192 && B > 256);
+  auto kernel = small ? sample_fullvocab_kernel<T, Small> : sample_fullvocab_kernel<T, Large>;
+  kernel<<<B, small ? Small::WG : Large::WG, 0, stream>>>(out, logits, temps, top_ks, top_ps,
+                                                          uniforms, mask, mask_map, V);
+}
+
 extern "C" void launch_sample_fullvocab(int64_t* out, const void* logits, bool bf16,
                              const float* temps, const int64_t* top_ks,
                              const float* top_ps, const float* uniforms,
                              const uint8_t* mask, const int32_t* mask_map,
                              int B, int V, hipStream_t stream) {
-  dim3 grid(B), block(WG);
-  if (bf16) {
-    hipLaunchKernelGGL((sample_fullvocab_kernel<bf16_t>), grid, block, 0,
-                       stream, out, (const bf16_t*)logits, temps,
-                       top_ks, top_ps, uniforms, mask, mask_map, V);
-  } else {
-    hipLaunchKernelGGL((sample_fullvocab_kernel<float>), grid, block, 0,
-                       stream, out, (const float*)logits, temps, top_ks,
-                       top_ps, uniforms, mask, mask_map, V);
-  }
+  if (bf16)
+    launch(out, (const bf16_t*)logits, temps, top_ks, top_ps, uniforms, mask, mask_map, B, V, stream);
+  else
+    launch(out, (const float*)logits, temps, top_ks, top_ps, uniforms, mask, mask_map, B, V, stream);
 }

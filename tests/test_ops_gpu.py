@@ -373,6 +373,26 @@ def test_fullvocab_draws_lie_in_the_kept_cdf(V, dtype):
 
 
 @requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [4093, 4096, 4097, 8191, 8192, 8193])
+def test_fullvocab_draws_with_few_and_many_threads(V, dtype):
+    """Around the sizes up to which a row has 256 threads, with few rows and with many: the
+    same tokens, and stripes of 16, 17 and 32 tokens."""
+    test_fullvocab_draws_lie_in_the_kept_cdf(V, dtype)
+    n = 300
+    x = (2.5 * torch.randn(n, V)).to(dtype).cuda()
+    args = [torch.full((n,), 0.8).cuda(), torch.tensor([0, 40, 0] * 100).cuda(),
+            torch.tensor([1.0, 1.0, 0.9] * 100).cuda()]
+    u = torch.rand(n).cuda()
+    many = hip().softmax_sample(x, *args, None, None, u)
+    few = torch.cat([
+        hip().softmax_sample(x[i : i + 100], *(a[i : i + 100] for a in args), None, None,
+                             u[i : i + 100]) for i in range(0, n, 100)
+    ])
+    assert torch.equal(many, few)
+
+
+@requires_gpu
 @pytest.mark.parametrize("k", [0, 3])
 @pytest.mark.parametrize("p", [0.0, -1.0])
 @pytest.mark.parametrize("V", [600, 128256])
