@@ -43,10 +43,8 @@ struct LatentPrefillArgs {
 // Where merged rows go: row r is head r % H of token r / H.
 struct SplitOut {
   void* out;              // bf16, tokens out_stride apart
-  const void* gate;       // [tokens, H] bf16 before its sigmoid, or null
-  int64_t out_stride, gate_stride;
+  int64_t out_stride;
   int H;
-  bool sum;               // partial results are summed as they are, no softmax
 };
 
 // bf16 rows of ``width`` from n_split (at most 64) partial sums [n_split, rows, width]

@@ -296,9 +296,7 @@ __global__ __launch_bounds__(128) void split_combine_kernel(
   const float w = ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - m) : 0.f;
   const float l = wave_sum(w * fmaxf(ml.y, 0.f));
   const int token = row / dst.H, head = row % dst.H;
-  const float gate =
-      dst.gate ? sigmoid_f(bf2f(((const bf16_t*)dst.gate)[token * dst.gate_stride + head])) : 1.f;
-  if (threadIdx.x < 64) weight[lane] = dst.sum ? gate : l > 0.f ? gate * w / l : 0.f;
+  if (threadIdx.x < 64) weight[lane] = l > 0.f ? w / l : 0.f;
   bf16_t* out = (bf16_t*)dst.out + token * dst.out_stride + (int64_t)head * rank;
   __syncthreads();
   for (int i = threadIdx.x * 4; i < rank; i += 512) {
@@ -443,7 +441,7 @@ bool launch_latent_attn(bool bf16, bool mfma, const LatentArgs* a, int rank, int
     default: return false;
   }
   if (a->n_split > 1) {
-    const SplitOut out = {a->out, nullptr, (int64_t)a->H * rank, 0, a->H, false};
+    const SplitOut out = {a->out, (int64_t)a->H * rank, a->H};
     launch_split_combine(&out, a->part, a->part_ml, a->rows, rank, a->n_split, stream);
   }
   return true;

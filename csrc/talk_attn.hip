@@ -768,7 +768,7 @@ bool launch_talk_decode(const GroupedArgs* a, int d, int v, int seqs, hipStream_
    : a->H <= 32 ? launch_decode_group<2>
                 : launch_decode_group<4>)(*a, d, v, gm, seqs, stream);
   if (a->n_split > 1) {
-    const SplitOut out = {a->out, a->gate, a->out_stride, a->gate_stride, a->H, a->sigmoid};
+    const SplitOut out = {a->out, a->out_stride, a->H};
     launch_split_combine(&out, a->part, a->part_ml, a->rows, v, a->n_split, stream);
   }
   return true;
