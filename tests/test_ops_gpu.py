@@ -393,6 +393,49 @@ def test_fullvocab_draws_with_few_and_many_threads(V, dtype):
 
 
 @requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [700, 50257])
+@pytest.mark.parametrize("T,k,p", [(0.0, 0, 1.0), (0.8, 0, 1.0), (0.8, 1, 1.0), (0.8, 5, 1.0),
+                                   (0.8, 0, 0.9), (0.8, 40, 0.5)])
+def test_fullvocab_rows_with_infinities_and_nan(V, dtype, T, k, p):
+    """Tokens are allowed ones, an infinite logit wins where the largest must, a masked one and
+    other rows' change nothing."""
+    torch.manual_seed(V)
+    x = torch.randn(8, V)
+    x[1, 3] = math.inf
+    x[2, [5, V // 2, V - 2]] = math.inf
+    x[3, [0, 9, V - 1]] = math.nan
+    x[4, 11] = math.nan  # masked
+    x[5, 12] = math.inf  # masked
+    x[6, 13] = math.inf
+    x[6, 14] = -math.nan
+    mask = torch.rand(2, V) < 0.3
+    mask[:, [11, 12]] = False
+    mask[1, 20] = True
+    rows = [-1, -1, -1, -1, 0, 1, -1, 1]
+    u = torch.rand(8)
+
+    def draw(x):
+        n = len(x)
+        return hip().softmax_sample(
+            x.to(dtype).cuda(), torch.full((n,), T).cuda(), torch.full((n,), k).cuda(),
+            torch.full((n,), p).cuda(), None, mask.cuda(), u.cuda(),
+            torch.tensor(rows, dtype=torch.int32).cuda(),
+        ).tolist()
+
+    got = draw(x)
+    for r, m in enumerate(rows):
+        assert 0 <= got[r] < V and (m < 0 or mask[m, got[r]]), r
+    if T == 0:
+        assert got[1] == 3 and got[2] == 5 and got[6] == 13
+    if k == 1:
+        assert got[1] == 3 and got[2] in (5, V // 2, V - 2)
+    finite = torch.where(x.isfinite(), x, torch.zeros(()))
+    plain = draw(finite)
+    assert [got[r] for r in (0, 4, 5, 7)] == [plain[r] for r in (0, 4, 5, 7)]
+
+
+@requires_gpu
 @pytest.mark.parametrize("k", [0, 3])
 @pytest.mark.parametrize("p", [0.0, -1.0])
 @pytest.mark.parametrize("V", [600, 128256])
@@ -450,6 +493,55 @@ def test_prompt_tiles_over_pages(block, H, G, scale):
         # weights and results are rounded to 8 bits: 2 * 2^-9 of values up to 5
         assert maxerr(out[mine].cpu(), want) < 0.02, m
         row += m.query_len
+
+
+@requires_gpu
+@pytest.mark.parametrize("block", [16, 24, 64])
+@pytest.mark.parametrize("d,v", [(64, 256), (256, 64), (256, 128), (256, 256)])
+@pytest.mark.parametrize("form", [dict(window=90, keep_first=3, sink=True), dict(sigmoid=True)])
+def test_prompt_head_sizes_over_pages(block, d, v, form):
+    """Every count of keys that one load brings, on pages of every kind; what no token has
+    written is NaN."""
+    from op_helpers import make_batch
+
+    H, G, scale = 6, 2, d ** -0.5
+    form = {"cap": None, "window": None, "keep_first": 0, **form}
+    gen = torch.Generator().manual_seed(d + v)
+    batch, _, _, pages = make_batch([(0, 131), (70, 65), (250, 7)], block, "cuda")
+    kc = torch.full((pages, block, G, d), float("nan"), device="cuda").bfloat16()
+    vc = torch.full((pages, block, G, v), float("nan"), device="cuda").bfloat16()
+    q = torch.randn(batch.num_prefill_tokens, H, d, generator=gen).bfloat16().cuda()
+    sink = torch.randn(H, generator=gen).cuda() if form.pop("sink", None) else None
+    slots = []
+    for m in batch.prefills:
+        p = torch.arange(m.seq_len)
+        slots.append((torch.tensor(m.block_table)[p // block] * block + p % block).cuda())
+        for c in (kc, vc):
+            c.view(-1, G, c.shape[3])[slots[-1]] = torch.randn(
+                m.seq_len, G, c.shape[3], generator=gen).bfloat16().cuda()
+    out = torch.empty(len(q), H, v, dtype=torch.bfloat16, device="cuda")
+    hip().grouped_attention(q, kc, vc, batch, scale, sink=sink, out=out, **form)
+    row = 0
+    for m, at in zip(batch.prefills, slots):
+        mine = slice(row, row + m.query_len)
+        row += m.query_len
+        k, x = (c.view(-1, G, c.shape[3])[at].float().repeat_interleave(H // G, 1)
+                for c in (kc, vc))
+        s = (q[mine].float()[:, None] * k).sum(-1) * scale  # [queries, keys, H]
+        pos = m.ctx_len + torch.arange(m.query_len, device="cuda")[:, None, None]
+        key = torch.arange(m.seq_len, device="cuda")[None, :, None]
+        hidden = key > pos
+        if form["window"]:
+            hidden |= (key <= pos - form["window"]) & (key >= form["keep_first"])
+        s = s.masked_fill(hidden, -math.inf)
+        if form.get("sigmoid"):
+            w = torch.sigmoid(s)
+        else:
+            w = torch.softmax(torch.cat([s, sink.expand(len(s), 1, H)], 1), 1)[:, :-1]
+        want = torch.einsum("nkh,khv->nhv", w, x)
+        # each weight is rounded to 8 bits, and the result
+        slack = 2.0 ** -8 * (torch.einsum("nkh,khv->nhv", w, x.abs()) + want.abs()) + 1e-3
+        assert ((out[mine].float() - want).abs() <= slack).all(), m
 
 
 @requires_gpu
