@@ -143,6 +143,7 @@ static DEV uint64_t same_id(int id, int bits) {
 
 // Group the entries by expert, in their order: a counting sort by one workgroup, each
 // wave counting and placing its own run of entries.  Dynamic LDS: [17][E] ints.
+template <bool TILED>
 __global__ __launch_bounds__(1024) void group_kernel(
     int* __restrict__ perm, int* __restrict__ offsets, int* __restrict__ tile_expert,
     int* __restrict__ tile_row, const int* __restrict__ ids, const int n, const int E,
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(1024) void group_kernel(
     // 1280 inner, 2048 outputs: 1800 tokens 138 and 140, 4093 241 and 212. Taken where it is not
     // faster: 2500 and 7000 tokens of the first (870 and 884, 1753 and 1819).
     bool tall = false;
-    if (tile_expert) {
+    if (TILED) {
       int tiles[2] = {}, small[2] = {};  // of 256 rows, tall
       for (int e = lane; e < E; e += 64) {
         const int c = total[e], t = (c + EXPERT_TILE - 1) / EXPERT_TILE;
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(1024) void group_kernel(
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + lane;
       const int c = e < E ? total[e] : 0;
-      int high = EXPERT_TILE, t = (c + EXPERT_TILE - 1) / EXPERT_TILE;
+      int high = EXPERT_TILE, t = TILED ? (c + EXPERT_TILE - 1) / EXPERT_TILE : 0;
       if (tall) {
         high = tall_tile(c);
         t = (c + high - 1) / high;
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(1024) void group_kernel(
         const int first = row + cs - c;
         total[e] = first;
         offsets[e] = first;
-        for (int j = 0; j < t && tile_expert; ++j) {
+        for (int j = 0; j < t; ++j) {
           tile_expert[tile + ts - t + j] = e;
           tile_row[tile + ts - t + j] = first + j * high;
         }
@@ -390,8 +391,8 @@ void launch_moe_route(bool bf16, int* ids, float* weights, const void* h, const 
 
 void launch_moe_group(int* perm, int* offsets, int* tile_expert, int* tile_row, const int* ids,
                       int n, int E, const TiledProducts* sizes, hipStream_t stream) {
-  group_kernel<<<1, 1024, 17 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E,
-                                                *sizes);
+  auto kernel = tile_expert ? group_kernel<true> : group_kernel<false>;
+  kernel<<<1, 1024, 17 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E, *sizes);
 }
 
 // tt: token fragments at a time, 1 or 2
