@@ -80,7 +80,9 @@ def build(verbose: bool = False) -> str:
     if not os.path.exists(so_path):
         raise RuntimeError(f"build produced no _C.so in {BUILD}")
     dest = os.path.join(PKG, "_C.so")
-    shutil.copy2(so_path, dest)
+    # into a file of its own: a running program keeps the one that it has mapped
+    shutil.copy2(so_path, dest + ".new")
+    os.replace(dest + ".new", dest)
     print(f"built {dest}")
     return dest
 
