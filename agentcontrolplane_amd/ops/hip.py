@@ -392,7 +392,7 @@ def _grouped_decode(out, q, k_cache, v_cache, tables, seq_lens, sink, bias, gate
     keys = min(tables.shape[1] * k_cache.shape[1], window + keep_first, chunk)
     groups = G * -(-(H // G) // gm)
     pieces, part, ml = 0, None, None
-    if B * groups < _WHOLE_GROUPS and keys > 128 and B * keys <= _C.DECODE_KEYS:
+    if B * groups < _WHOLE_GROUPS and keys > 128:
         pieces = max(1, _DECODE_GROUPS // groups)
         part = torch.empty((pieces + B) * H * v, dtype=torch.float32, device=q.device)
         ml = torch.empty(2 * (pieces + B) * H, dtype=torch.float32, device=q.device)

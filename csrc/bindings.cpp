@@ -760,8 +760,6 @@ static void grouped_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
     CHECK_CUDA((*part)); CHECK_CUDA((*part_ml));
     TORCH_CHECK(part->numel() >= rows * v && part_ml->numel() >= 2 * rows, "split workspace");
     TORCH_CHECK((uintptr_t)part->data_ptr() % 16 == 0, "split workspace alignment");
-    const int64_t seen = std::min({tables.size(1) * k_cache.size(1), window + keep, chunk});
-    TORCH_CHECK(kind != 1 || seqs * seen <= DECODE_KEYS, "too many keys for pieces");
     a.part = part->data_ptr<float>();
     a.part_ml = (float2*)part_ml->data_ptr<float>();
   }
@@ -1117,7 +1115,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma_probe", &mfma_probe);
   m.def("gemm_bf16", &gemm_bf16);
   m.attr("DEPTH_AHEAD") = DEPTH_AHEAD;
-  m.attr("DECODE_KEYS") = DECODE_KEYS;
   m.def("residual_norm", &residual_norm);
   m.def("side_gate", &side_gate);
   m.def("add_to_residual", &add_to_residual);

@@ -27,9 +27,6 @@ struct GroupedArgs {
   bool sigmoid;           // weights sigmoid(score), not a softmax
 };
 
-// keys of a step that is cut into pieces: the kernel counts their blocks of 32 in 22 bits
-#define DECODE_KEYS (1ll << 26)
-
 #ifdef __HIPCC__
 // first key that position pos sees beyond the kept ones
 static inline __device__ int first_key(const GroupedArgs& a, int pos) {

@@ -8,20 +8,24 @@ def quotient(n, d):
     """As the kernel divides, with a reciprocal that may be off by one unit in either direction."""
     n, d = np.asarray(n, np.int64), np.asarray(d, np.int64)
     for step in (-1, 0, 1):
-        r = (np.float32(1) / d.astype(np.float32)).view(np.int32) + np.int32(step)
-        q = (n.astype(np.float32) * r.view(np.float32)).astype(np.int64)
+        by = (np.float32(1) / d.astype(np.float32)).view(np.int32) + np.int32(step)
+        by = by.view(np.float32)
+        q = (n.astype(np.float32) * by).astype(np.int64)
+        more = ((n - q * d).astype(np.float32) * by).astype(np.int64)
+        q = q + more
         rest = n - q * d
-        q = q + (rest >= d) - (rest < 0)
-        yield q
+        assert (np.abs(q * d) < 1 << 31).all()  # no overflow on the way
+        yield q + (rest >= d) - (rest < 0)
 
 
 def test_quotient_is_exact():
     gen = np.random.default_rng(1)
-    d = np.concatenate([np.arange(1, 3000), gen.integers(1, 1 << 21, 20000)])
+    d = np.concatenate([np.arange(1, 3000), gen.integers(1, 1 << 29, 20000),
+                        gen.integers(1, 1 << 12, 20000)])
+    top = (1 << 30) - 1
     for shift in (0, 3, 8, 15, 22):
-        top = (1 << 22) - 1
-        n = np.minimum(top, gen.integers(0, top + 1, d.shape) >> shift)
-        near = np.minimum(top, n // d * d)  # multiples and one less
+        n = gen.integers(0, top + 1, d.shape) >> shift
+        near = n // d * d  # multiples and one less
         for x in (n, near, np.maximum(near - 1, 0), np.full_like(d, top)):
             for q in quotient(x, d):
                 assert (q == x // d).all()

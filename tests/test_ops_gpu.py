@@ -256,6 +256,20 @@ def test_decode_over_many_blocks(case, block):
 
 
 @requires_gpu
+def test_decode_pieces_of_wide_tables():
+    """Room for 2^22 blocks of 32 keys, whose count is divided in another way: the same pieces."""
+    torch.manual_seed(2)
+    lens = torch.tensor([700, 33, 2100, 0, 1, 4000, 950], dtype=torch.int32).cuda()
+    tables = torch.randint(0, 90, (7, 260), dtype=torch.int32).cuda()
+    kc, vc = torch.randn(2, 90, 16, 4, 128, device="cuda").bfloat16()
+    q = torch.randn(7, 16, 128, device="cuda").bfloat16()
+    wide = torch.zeros(7, 1 << 21, dtype=torch.int32, device="cuda")
+    wide[:, :260] = tables
+    got, want = (hip().attention_decode_raw(q, kc, vc, t, lens, 0.1) for t in (wide, tables))
+    assert torch.equal(got, want)
+
+
+@requires_gpu
 def test_mfma_fragment_layout_probe():
     """The assumed A/B/D lane maps for v_mfma_f32_32x32x16_bf16 must
     reproduce a plain matmul (asymmetric operands per guide G9/rule 16)."""
