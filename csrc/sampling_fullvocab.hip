@@ -19,11 +19,11 @@
 //
 // Bound by the passes over the row: 20 us for the largest logit, 15 for the histogram of a top-k
 // and 62 for that of a top-p (30 of it weights, 32 atomics), 16 to gather the bucket, 15 for the
-// draw's sums, where 190 rows of 128256 in fp32 come from the memory-side cache.  Whole calls:
-// 23 us greedy, 60 plain, 93 top-k, 146 top-p or a mix; before 305, 421, 1129, 1302 and 1229
-// (thresholds by three histograms of key bits, whose few buckets met nearly all atomics, walked by
-// one thread; draws by strides of a thread).  Floating masses instead of whole ones in the
-// histogram took as long, a shared list of the bucket 25 us more.
+// draw's sums, where 190 rows of 128256 in fp32 come from the memory-side cache.  Whole calls
+// with other logits each time: 34 us greedy, 67 plain, 100 top-k, 153 top-p, 193 both; before 315,
+// 428, 1135, 1305 and 1978 (thresholds by three histograms of key bits, whose few buckets met
+// nearly all atomics, walked by one thread; draws by strides of a thread).  Floating masses
+// instead of whole ones in the histogram took as long, a shared list of the bucket 25 us more.
 //
 // Semantics match the oracle:
 //   greedy (T<=0): argmax, lowest index on ties
