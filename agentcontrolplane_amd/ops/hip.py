@@ -405,7 +405,9 @@ def _grouped_decode(out, q, k_cache, v_cache, tables, seq_lens, sink, bias, gate
 #: workgroups that a decode step's keys are cut for: 2 rounds of the 2 a CU that fit
 _DECODE_GROUPS = 1024
 #: from so many sequences and key heads on a sequence is one piece (190 x 8, 700 to 1300 keys:
-#: 159 us, cut as fewer ones 169; 250 x 8, 200 to 2000 keys: 235 and 250 us)
+#: 159 us, cut as fewer ones 169; 250 x 8, 200 to 2000 keys: 235 and 250 us; 130 x 8, 100 to 8000
+#: keys: 454 and 476).  The host does not see the lengths: where one sequence is by far the longest
+#: that is the slower choice (129 x 300 keys and one of 8000: 156 and 59 us)
 _WHOLE_GROUPS = 1024
 
 
