@@ -134,10 +134,8 @@ class LobuvikLayer:
         mixed = torch.empty(N, m.out_dim + self.ff_pad, dtype=h1.dtype, device=h1.device)
         routed = self.experts.forward(h2) if self.experts else None
         if self.glu:
-            g = self.glu
-            ops.clamped_glu(
-                ops.step_linear(h2[:, : self.width], self.gate_up), g.limit, g.alpha, g.offset,
-                mixed[:, m.out_dim :], g.cubic,
+            ops.step_linear_glu(
+                h2[:, : self.width], self.gate_up, self.glu, mixed[:, m.out_dim :]
             )
         heads, bias = mixed[:, : m.out_dim], None
         if self.latent:

@@ -100,9 +100,8 @@ class TezinexLayer:
         return out
 
     def feed_forward(self, h: torch.Tensor) -> torch.Tensor:
-        gate_up = ops.step_linear(h, self.gate_up)
         act = torch.empty(h.shape[0], self.ff_pad, dtype=h.dtype, device=h.device)
-        ops.clamped_glu(gate_up, self.mlp.limit, self.mlp.alpha, self.mlp.offset, act)
+        ops.step_linear_glu(h, self.gate_up, self.mlp, act)
         return ops.step_linear(act, self.down)
 
 

@@ -46,18 +46,13 @@ def _impl(t: torch.Tensor):
 
 import os
 
-# Measured A/B (tools/gemm_bench.py, profiles/r01_gemm_ab.md): the TunableOp-
-# tuned hipBLASLt stream-K kernels hold 1.3-1.6 PF on every engine projection
-# shape; the hand-written 8-phase kernel (csrc/gemm_bf16.hip) reaches 1.1 PF
-# (zero LDS conflicts, barrier/issue-stall bound).  The library stays the
-# default; set ACP_GEMM_MIN_M to route M >= threshold to the custom kernel.
+# Rows from which linear() takes csrc/linear.hip whatever the sizes; step_linear() has a rule
 _GEMM_MIN_M = int(os.environ.get("ACP_GEMM_MIN_M", str(1 << 30)))
 
 
 def linear(x, w, bias=None):
-    """x[*, K] @ w[N, K]^T (+ bias[N]) → [*, N].  Large-M bf16 shapes go to the
-    hand-written 8-phase MFMA GEMM (csrc/gemm_bf16.hip); everything else
-    (decode-sized M, ragged shards, CPU) to torch.nn.functional.linear."""
+    """x[*, K] @ w[N, K]^T (+ bias[N]) → [*, N] by the library, unless ACP_GEMM_MIN_M says
+    otherwise for that many bf16 rows."""
     if (
         x.is_cuda
         and bias is None
@@ -97,27 +92,29 @@ def _few_rows_pay(m: int, outs: int, k: int, glu: bool) -> bool:
     return 7680 < k < 8192 and (outs <= 64 or 512 <= outs <= 4096)
 
 
+def _rows(t) -> bool:
+    """Rows of 16-byte units."""
+    return (
+        t.dim() == 2
+        and t.is_cuda
+        and t.dtype == torch.bfloat16
+        and t.stride(1) == 1
+        and (t.shape[0] == 1 or t.stride(0) % 8 == 0)
+        and t.data_ptr() % 16 == 0
+    )
+
+
+def _recorded(*ts) -> bool:
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts)
+
+
 def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
     """Whether csrc/step_linear.hip takes x w^T: what it can, at the sizes at which it pays.
     It has no derivative: what autograd records is left to the library."""
-
-    def recorded(t):
-        return t is not None and t.requires_grad
-
-    def rows(t):  # of 16-byte units
-        return (
-            t.dim() == 2
-            and t.is_cuda
-            and t.dtype == torch.bfloat16
-            and t.stride(1) == 1
-            and (t.shape[0] == 1 or t.stride(0) % 8 == 0)
-            and t.data_ptr() % 16 == 0
-        )
-
     return (
         0 < x.shape[0] <= 4
-        and rows(x)
-        and rows(w)
+        and _rows(x)
+        and _rows(w)
         and x.device == w.device
         and x.shape[1] == w.shape[1]
         and w.shape[0] > 0
@@ -129,23 +126,100 @@ def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
             or bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
             and bias.shape == w.shape[:1]
         )
-        and not (torch.is_grad_enabled() and (recorded(x) or recorded(w) or recorded(bias)))
+        and not _recorded(x, w, bias)
+    )
+
+
+def _many_rows_pay(m: int, n: int, k: int, glu: bool) -> bool:
+    """Whether csrc/linear.hip is the faster one for m rows, n outputs (of a GLU: gates and ups)
+    and k inner elements; the GEMM library (with a pass of its own for the GLU) is in brackets,
+    us.  Up to about 2000 rows at nearly all sizes: 8 x 22016 x 4096 GLU 40 (53), 64 x 4096 x
+    14336 30 (53), 192 x 4096 x 4096 20 (33), 512 x 6288 x 2048 19 (22), 1739 x 4096 x 11008 140
+    (166), and by a few percent not: 16 x 3072 x 768 5.6 (5.3), 96 x 12288 x 4096 36 (31).  Small
+    weights are the launch, whoever's it is.  Beyond that the library is 2 to 7% ahead where
+    256 x 256 tiles fill their last round, 5000 x 6144 x 4096 194 (188), 7664 x 2048 x 8192 185
+    (172), 8131 x 4096 x 4096 185 (176), but not for the GLU, 7664 x 28672 x 4096 1296 (1458),
+    for outputs that are no whole tiles, 7664 x 17744 x 2048 437 (494), and for rows that
+    together are beyond the memory-side cache, 7664 x 4096 x 14336 630 (995); with a last
+    round that is not full it is slower, 5000 x 4096 x 4096 132 (142), 10000 x 4096 x 4096 251 (361)."""
+    if m <= 4 or n * k < 1 << 21:
+        return False
+    if m < 2048 or glu or n % 256 or m * k >= 100 << 20:
+        return True
+    tiles = -(-m // 256) * (n // 256)
+    return tiles < 0.93 * 256 * -(-tiles // 256)
+
+
+def _many_rows(x, w, bias=None, glu: bool = False, out=None) -> bool:
+    """Whether csrc/linear.hip takes x w^T: what it can, at the sizes at which it pays.  It has
+    no derivative and is not seen by what follows the library's calls: that is left to it."""
+
+    def below_2gib(t):
+        return (t.shape[0] - 1) * t.stride(0) + t.shape[1] < 1 << 30
+
+    def whole(t):
+        return type(t) in (torch.Tensor, torch.nn.Parameter)
+
+    def seen():  # by transforms, forward-mode derivatives, dispatch modes or a trace
+        return (
+            torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._get_tracing_state() is not None
+        )
+
+    return (
+        x.dim() == 2
+        and w.dim() == 2
+        and x.shape[1] == w.shape[1]
+        and w.shape[1] % 64 == 0
+        and w.shape[0] % (16 if glu else 8) == 0
+        and _many_rows_pay(x.shape[0], w.shape[0], w.shape[1], glu)
+        and whole(x)
+        and whole(w)
+        and not seen()
+        and _rows(x)
+        and _rows(w)
+        and x.device == w.device
+        and below_2gib(x)
+        and below_2gib(w)
+        and (out is None or _rows(out))
+        and (
+            bias is None
+            or whole(bias) and bias.device == x.device and bias.dtype == torch.bfloat16
+            and bias.is_contiguous() and bias.shape == w.shape[:1] and bias.data_ptr() % 16 == 0
+        )
+        and not _recorded(x, w, bias)
     )
 
 
 def step_linear(x, w, bias=None):
-    """linear() of a step's activations in a model's forward pass: the few rows of a small decode
-    step go to a kernel of their own, unless autograd records them."""
+    """linear() of a step's activations in a model's forward pass: rows of 16 bits go to kernels of
+    their own where those are the faster ones, unless autograd records them."""
     if _few_rows(x, w, bias):
         return _hip().step_linear(x, w, bias)
+    if _many_rows(x, w, bias):
+        return _hip().linear(x, w, bias)
     return linear(x, w, bias)
 
 
 def step_linear_swiglu(x, w):
-    """swiglu(step_linear(x, w)), in one pass for a few rows."""
+    """swiglu(step_linear(x, w)), in one pass where step_linear() has a kernel of its own."""
     if w.shape[0] % 16 == 0 and _few_rows(x, w, None, True):
         return _hip().step_linear(x, w, None, True)
+    if _many_rows(x, w, None, True):
+        return _hip().linear(x, w, unit="swiglu")
     return swiglu(linear(x, w))
+
+
+def step_linear_glu(x, w, glu, out):
+    """clamped_glu(step_linear(x, w)) -> out [N, I] (row-strided), likewise.  ``glu`` has limit,
+    alpha, offset and maybe cubic."""
+    cubic = getattr(glu, "cubic", 0.0)
+    if _many_rows(x, w, None, True, out):
+        _hip().linear(x, w, None, "glu", (glu.limit, glu.alpha, glu.offset, cubic), out)
+    else:
+        clamped_glu(step_linear(x, w), glu.limit, glu.alpha, glu.offset, out, cubic)
 
 
 def linear_add_(y, x, w):

@@ -131,6 +131,15 @@ def gemm_bf16(x, w):
     return out
 
 
+def linear(x, w, bias=None, unit="plain", form=(0.0, 0.0, 0.0, 0.0), out=None, tile=-1, splits=1):
+    """csrc/linear.hip; ``tile`` and ``splits`` as it chooses them unless given."""
+    if out is None:
+        outs = w.shape[0] // (1 if unit == "plain" else 2)
+        out = torch.empty((x.shape[0], outs), dtype=x.dtype, device=x.device)
+    _C.linear(out, x, w, bias, unit, *form, tile, splits)
+    return out
+
+
 def step_linear(x, w, bias=None, glu=False):
     out = torch.empty((x.shape[0], w.shape[0] >> glu), dtype=x.dtype, device=x.device)
     _C.step_linear(out, x, w, bias, glu)

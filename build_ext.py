@@ -41,7 +41,7 @@ def build(verbose: bool = False) -> str:
         os.path.join(CSRC, "rope_cache.hip"),
         os.path.join(CSRC, "prefill_attn.hip"),
         os.path.join(CSRC, "mfma_probe.hip"),
-        os.path.join(CSRC, "gemm_bf16.hip"),
+        os.path.join(CSRC, "linear.hip"),
         os.path.join(CSRC, "step_linear.hip"),
         os.path.join(CSRC, "residual_norm.hip"),
         os.path.join(CSRC, "gated_act.hip"),

@@ -15,6 +15,7 @@
 #include "grouped_attn.h"
 #include "latent_attn.h"
 #include "residual_norm.h"
+#include "linear.h"
 #include "step_linear.h"
 
 namespace py = pybind11;
@@ -79,7 +80,6 @@ void launch_latent_gather(void*, const void*, const int*, const int*, const int*
                           int, int, int, int, int, hipStream_t);
 bool launch_latent_attn(bool, bool, const LatentArgs*, int, int, int, int, hipStream_t);
 void launch_mfma_probe(float*, const void*, const void*, hipStream_t);
-void launch_gemm_bf16(void*, const void*, const void*, int, int, int, hipStream_t);
 }
 
 #define CHECK_CUDA(x) TORCH_CHECK(x.is_cuda(), #x " must be a GPU tensor")
@@ -199,18 +199,68 @@ static void prefill_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
                       max_blocks, kv_block, q_stride, cur_stream());
 }
 
-// C[M,N] = A[M,K] @ B[N,K]^T — the hand-written 256²-tile 8-phase MFMA
-// GEMM (csrc/gemm_bf16.hip) for large-M bf16 projections
+// The launch of x w^T by csrc/linear.hip: tile and splits from the sizes, or the given ones
+static void run_linear(const LinearArgs& a, int unit, int tile, int splits,
+                       const torch::Tensor& x) {
+  if (tile < 0) linear_choice(a.M, a.N, a.K, unit, &tile, &splits);
+  torch::Tensor parts;
+  if (splits > 1)
+    parts = torch::empty({(int64_t)splits * a.M * a.N}, x.options().dtype(torch::kFloat32));
+  launch_linear(&a, unit, tile, splits, splits > 1 ? parts.data_ptr() : nullptr, cur_stream());
+}
+
+// out = x w^T + bias, or the gated unit of its halves: "swiglu", "glu" with the form's numbers
+static void linear(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                   const c10::optional<torch::Tensor>& bias, const std::string& unit,
+                   double limit, double alpha, double offset, double cubic, int64_t tile,
+                   int64_t splits) {
+  CHECK_CUDA(x); CHECK_CUDA(w); CHECK_CUDA(out);
+  CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(out);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  const bool glu = unit == "swiglu" || unit == "glu";
+  TORCH_CHECK(glu || unit == "plain", "unknown unit");
+  const int64_t outs = glu ? N / 2 : N;
+  TORCH_CHECK(M > 0 && K > 0 && N > 0 && w.size(1) == K && K % 64 == 0 && outs % 8 == 0 &&
+              (!glu || N % 2 == 0) && out.size(0) == M && out.size(1) == outs, "linear: sizes");
+  TORCH_CHECK(x.device() == w.device() && x.device() == out.device());
+  TORCH_CHECK(x.stride(1) == 1 && w.stride(1) == 1 && out.stride(1) == 1);
+  LinearArgs a = {};
+  a.x_stride = M > 1 ? x.stride(0) : K;
+  a.w_stride = N > 1 ? w.stride(0) : K;
+  a.out_stride = M > 1 ? out.stride(0) : outs;
+  for (int64_t stride : {a.x_stride, a.w_stride, a.out_stride})
+    TORCH_CHECK(stride >= 0 && stride % 8 == 0, "linear: strides");
+  for (const void* p : {x.data_ptr(), w.data_ptr(), out.data_ptr()})
+    TORCH_CHECK((uintptr_t)p % 16 == 0, "linear: alignment");
+  // byte offsets of 32 bits; tiles past the end have up to 256 rows more
+  TORCH_CHECK(((M - 1) * a.x_stride + K) * 2 < (1ll << 31) &&
+              ((N - 1) * a.w_stride + K) * 2 < (1ll << 31) && M < (1 << 30) && N < (1 << 30),
+              "linear: operands of 2 GiB and more");
+  if (bias) {
+    CHECK_CUDA((*bias)); CHECK_BF16((*bias)); CHECK_CONT((*bias));
+    TORCH_CHECK(!glu && bias->numel() == N && (uintptr_t)bias->data_ptr() % 16 == 0);
+    a.bias = bias->data_ptr();
+  }
+  TORCH_CHECK(tile < 0 || (linear_fits((int)tile, glu && splits == 1) && splits >= 1 &&
+                           splits <= K / 64), "linear: tile");
+  a.out = out.data_ptr();
+  a.x = x.data_ptr();
+  a.w = w.data_ptr();
+  a.M = (int)M; a.N = (int)N; a.K = (int)K;
+  a.limit = (float)limit; a.alpha = (float)alpha; a.offset = (float)offset;
+  a.cubic = (float)cubic;
+  const at::DeviceGuard guard(x.device());
+  run_linear(a, unit == "swiglu" ? LINEAR_SWIGLU : glu ? LINEAR_GLU
+             : bias ? LINEAR_BIAS : LINEAR_PLAIN, (int)tile, (int)splits, x);
+}
+
+// C[M,N] = A[M,K] @ B[N,K]^T on the largest tiles
 static void gemm_bf16(torch::Tensor C, torch::Tensor A, torch::Tensor B) {
-  CHECK_CUDA(A); CHECK_CONT(A); CHECK_BF16(A);
-  CHECK_CONT(B); CHECK_BF16(B); CHECK_CONT(C); CHECK_BF16(C);
-  const int M = A.size(0), K = A.size(1), N = B.size(0);
-  TORCH_CHECK(B.size(1) == K && C.size(0) == M && C.size(1) == N,
-              "gemm_bf16 shape mismatch");
-  TORCH_CHECK(K % 128 == 0, "gemm_bf16 requires K % 128 == 0");
-  TORCH_CHECK(N % 256 == 0, "gemm_bf16 requires N % 256 == 0");
-  launch_gemm_bf16(C.data_ptr(), A.data_ptr(), B.data_ptr(), M, N, K,
-                   cur_stream());
+  CHECK_CONT(A); CHECK_CONT(B); CHECK_CONT(C);
+  TORCH_CHECK(A.size(1) % 128 == 0, "gemm_bf16 requires K % 128 == 0");
+  TORCH_CHECK(B.size(0) % 256 == 0, "gemm_bf16 requires N % 256 == 0");
+  linear(C, A, B, c10::nullopt, "plain", 0, 0, 0, 0, 0, 1);
 }
 
 static torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b) {
@@ -1113,6 +1163,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_cache", &rope_cache);
   m.def("prefill_attn", &prefill_attn);
   m.def("mfma_probe", &mfma_probe);
+  m.def("linear", &linear, py::arg("out"), py::arg("x"), py::arg("w"),
+        py::arg("bias") = py::none(), py::arg("unit") = "plain", py::arg("limit") = 0.0,
+        py::arg("alpha") = 0.0, py::arg("offset") = 0.0, py::arg("cubic") = 0.0,
+        py::arg("tile") = -1, py::arg("splits") = 1);
+  m.def("linear_fits", [](int tile, bool glu) { return linear_fits(tile, glu); });
   m.def("gemm_bf16", &gemm_bf16);
   m.attr("DEPTH_AHEAD") = DEPTH_AHEAD;
   m.def("residual_norm", &residual_norm);
