@@ -491,6 +491,9 @@ _TILED_ROWS = 12
 
 def moe_experts(h, gate_up, down, ids, glu):
     (N, k), E, inner = ids.shape, gate_up.shape[0], down.shape[2]
+    if N * h.stride(0) >= 1 << 30 and N > 1:  # the tiled product's offsets have 32 bits
+        halves = [slice(0, N // 2), slice(N // 2, N)]
+        return torch.cat([moe_experts(h[r], gate_up, down, ids[r], glu) for r in halves])
     n, device = N * k, h.device
     act = torch.empty(n, inner, dtype=h.dtype, device=device)
     rows = torch.empty(N, k, down.shape[1], dtype=h.dtype, device=device)
@@ -498,7 +501,10 @@ def moe_experts(h, gate_up, down, ids, glu):
     perm = offsets = tile_expert = tile_row = None
     kind, tt = 0, 1
     if h.dtype == torch.bfloat16:
-        tiled = n >= _TILED_ROWS * E and gate_up.shape[2] % 128 == 0 and inner % 128 == 0
+        tiled = (
+            n >= _TILED_ROWS * E and gate_up.shape[2] % 128 == 0 and inner % 128 == 0
+            and max(gate_up[0].numel(), down[0].numel()) < 1 << 30
+        )
         kind, tt = (2, 1) if tiled else (1, 1 if n <= 8 * E else 2)
         perm = torch.empty(n, dtype=torch.int32, device=device)
         offsets = torch.empty(E + 2, dtype=torch.int32, device=device)
@@ -506,7 +512,8 @@ def moe_experts(h, gate_up, down, ids, glu):
             tiles = torch.empty(2, n // _C.EXPERT_TILE + E, dtype=torch.int32, device=device)
             tile_expert, tile_row = tiles
         _C.moe_group(
-            perm, offsets, tile_expert, tile_row, ids, E, gate_up.shape[2], inner, down.shape[1]
+            perm, offsets, tile_expert, tile_row, ids, E, gate_up.shape[2], inner, down.shape[1],
+            True,
         )
     grouped = (ids, perm, offsets, tile_expert, tile_row)
     _C.experts_linear(act, h, gate_up, *grouped, True, *form, kind, tt)

@@ -979,7 +979,7 @@ static void moe_route(torch::Tensor ids, torch::Tensor weights, torch::Tensor h,
 // products with these many inner elements and outputs
 static void moe_group(torch::Tensor perm, torch::Tensor offsets, OptTensor tile_expert,
                       OptTensor tile_row, torch::Tensor ids, int64_t E, int64_t width,
-                      int64_t inner, int64_t outputs) {
+                      int64_t inner, int64_t outputs, bool even) {
   const int64_t n = ids.numel();
   CHECK_CUDA(ids); CHECK_CONT(ids);
   TORCH_CHECK(ids.scalar_type() == at::kInt && E > 0 && E <= 512 && n < (1 << 30));
@@ -989,7 +989,7 @@ static void moe_group(torch::Tensor perm, torch::Tensor offsets, OptTensor tile_
   const int64_t columns1 = (inner + 127) / 128, columns2 = (outputs + 255) / 256;
   TORCH_CHECK(!te == !tr && width > 0 && width < (1 << 30) && inner > 0 && outputs > 0 &&
               std::max(columns1, columns2) * most < (1 << 30), "tiles");
-  const TiledProducts sizes = {(int)width, (int)columns1, (int)inner, (int)columns2};
+  const TiledProducts sizes = {(int)width, (int)columns1, (int)inner, (int)columns2, even};
   launch_moe_group((int*)opt_int(perm, n), (int*)opt_int(offsets, E + 2), te, tr,
                    ids.data_ptr<int>(), (int)n, (int)E, &sizes, cur_stream());
 }
@@ -1039,6 +1039,9 @@ static void experts_linear(torch::Tensor out, torch::Tensor x, torch::Tensor w, 
     return;
   }
   TORCH_CHECK(tile_expert && a.K % 128 == 0, "tiles");
+  // byte offsets of 32 bits in the rows that a workgroup reads
+  TORCH_CHECK(w.size(1) * (int64_t)a.K < (1 << 30) &&
+              (glu ? x.size(0) : TALL_TILE) * a.x_stride < (1 << 30), "rows of 2 GiB and more");
   a.tiles = a.entries / EXPERT_TILE + a.E;
   a.tile_expert = opt_int(tile_expert, a.tiles);
   a.tile_row = opt_int(tile_row, a.tiles);
@@ -1189,7 +1192,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attention_inputs", &attention_inputs);
   m.attr("EXPERT_TILE") = EXPERT_TILE;
   m.def("moe_route", &moe_route);
-  m.def("moe_group", &moe_group);
+  m.def("moe_group", &moe_group, py::arg("perm"), py::arg("offsets"), py::arg("tile_expert"),
+        py::arg("tile_row"), py::arg("ids"), py::arg("E"), py::arg("width"), py::arg("inner"),
+        py::arg("outputs"), py::arg("even") = false);
   m.def("experts_linear", &experts_linear);
   m.def("delta_prompts", &delta_prompts);
   m.def("delta_step", &delta_step);

@@ -22,6 +22,7 @@ struct ExpertsArgs {
 struct TiledProducts {
   int width, columns1;  // gate and up
   int inner, columns2;  // down
+  bool even;            // an expert's tiles have the same height
 };
 
 // rows of one tile of the large-batch product, at most TALL_TILE

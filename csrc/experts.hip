@@ -194,7 +194,7 @@ __global__ __launch_bounds__(1024) void group_kernel(
     // 1280 inner, 2048 outputs: 1800 tokens 138 and 140, 4093 241 and 212. Taken where it is not
     // faster: 2500 and 7000 tokens of the first (870 and 884, 1753 and 1819).
     bool tall = false;
-    if (TILED) {
+    if (TILED && !sizes.even) {
       int tiles[2] = {}, small[2] = {};  // of 256 rows, tall
       for (int e = lane; e < E; e += 64) {
         const int c = total[e], t = (c + EXPERT_TILE - 1) / EXPERT_TILE;
@@ -220,35 +220,56 @@ __global__ __launch_bounds__(1024) void group_kernel(
       }
       tall = cost[1] < 0.92f * cost[0];
     }
-    int row = 0, tile = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + lane;
-      const int c = e < E ? total[e] : 0;
-      int high = EXPERT_TILE, t = TILED ? (c + EXPERT_TILE - 1) / EXPERT_TILE : 0;
+    auto tiles_of = [&](int c, int& high) {
+      high = EXPERT_TILE;
+      int t = TILED ? (c + EXPERT_TILE - 1) / EXPERT_TILE : 0;
       if (tall) {
         high = tall_tile(c);
         t = (c + high - 1) / high;
+      } else if (TILED && sizes.even && t > 0) {
+        high = (c + t - 1) / t;
       }
-      int cs = c, ts = t;
+      return t;
+    };
+    auto before = [&](int v, int& sum) {  // the lanes before this one's; the wave's sum
+      int s = v;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
-        const int a = __shfl_up(cs, off, 64), b = __shfl_up(ts, off, 64);
-        if (lane >= off) {
-          cs += a;
-          ts += b;
+        const int w = __shfl_up(s, off, 64);
+        if (lane >= off) s += w;
+      }
+      sum = __shfl(s, 63, 64);
+      return s - v;
+    };
+    int row = 0, tile = 0, sum;
+    // the highest tiles first, by steps of 32 rows: workgroups that end early then fill up with
+    // the lower ones
+    for (int step = TILED && sizes.even ? EXPERT_TILE / 32 : 1; TILED && step > 0; --step) {
+      row = 0;
+      for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane, c = e < E ? total[e] : 0;
+        int high;
+        int t = tiles_of(c, high);
+        if (sizes.even && (high + 31) / 32 != step) t = 0;
+        const int first = row + before(c, sum);
+        row += sum;
+        const int at = tile + before(t, sum);
+        tile += sum;
+        for (int j = 0; j < t; ++j) {
+          tile_expert[at + j] = e;
+          tile_row[at + j] = first + j * high;
         }
       }
+    }
+    row = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, c = e < E ? total[e] : 0;
+      const int first = row + before(c, sum);
+      row += sum;
       if (e < E) {
-        const int first = row + cs - c;
         total[e] = first;
         offsets[e] = first;
-        for (int j = 0; j < t; ++j) {
-          tile_expert[tile + ts - t + j] = e;
-          tile_row[tile + ts - t + j] = first + j * high;
-        }
       }
-      row += __shfl(cs, 63, 64);
-      tile += __shfl(ts, 63, 64);
     }
     if (lane == 0) {
       offsets[E] = row;

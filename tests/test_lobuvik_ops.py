@@ -583,3 +583,52 @@ def test_experts(device, dtype, n, E, top, K, I, W, skew):
         t, c = (ids == e).nonzero(as_tuple=True)
         if len(t):
             close(got[t, c], oracle.clamped_glu(hd[t], x, "", 1.25), dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("even", [True, False], ids=["even", "tall"])
+@pytest.mark.parametrize("I,W", [(128, 264), (2432, 130)])
+def test_experts_tile_lists(I, W, even):
+    """The tiles cover every expert's rows once, even ones the highest first; the products follow
+    either list, tiles of more than 256 rows among them, also for outputs that are no whole
+    16-byte units."""
+    from agentcontrolplane_amd import _C
+
+    rows = [0, 1, 33, 64, 65, 128, 129, 161, 193, 225, 256, 257, 289, 320, 321, 513, 640, 1100]
+    E, K = len(rows), 1024
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).int()
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(3))]
+    n, cuda = len(ids), ids.cuda().view(-1, 1)
+    lists = torch.full((2, n // _C.EXPERT_TILE + E), -1, dtype=torch.int32, device="cuda")
+    perm, offsets = torch.empty_like(cuda[:, 0]), lists.new_empty(E + 2)
+    _C.moe_group(perm, offsets, lists[0], lists[1], cuda, E, K, I, W, even)
+    used, first = offsets[E + 1].item(), offsets.tolist()
+    expert, row = lists[:, :used].tolist()
+    heights = []
+    for i, (e, r) in enumerate(zip(expert, row)):
+        last = i + 1 == used or expert[i + 1] != e
+        heights.append((first[e + 1] if last else row[i + 1]) - r)
+        assert r == first[e] if i == 0 or expert[i - 1] != e else r > row[i - 1]
+    for e, count in enumerate(rows):
+        assert sum(h for h, x in zip(heights, expert) if x == e) == count
+    assert 0 < min(heights) and max(heights) <= (256 if even else 320)
+    if even:
+        steps = [-(-h // 32) for h in heights]
+        # an expert's last tile may be the lower one
+        assert all(a >= b for a, b, e, f in zip(steps, steps[1:], expert, expert[1:]) if e == f)
+        tops = [s for s, e, f in zip(steps, expert, [-1] + expert) if e != f]
+        assert tops == sorted(tops, reverse=True)
+    h = rand(n, K, dtype=torch.bfloat16, device="cuda")
+    gate_up = rand(E, 2 * I, K, dtype=torch.bfloat16, device="cuda", seed=1, scale=2 * K ** -0.5)
+    down = rand(E, W, I, dtype=torch.bfloat16, device="cuda", seed=2, scale=I ** -0.5)
+    act, got = h.new_empty(n, I), h.new_full((n + 1, W), 7.0)
+    form, grouped = (1.25, 1.702, 1.0, 0.0), (cuda, perm, offsets, lists[0], lists[1])
+    _C.experts_linear(act, h, gate_up, *grouped, True, *form, 2, 1)
+    _C.experts_linear(got[:n], act, down, *grouped, False, *form, 2, 1)
+    assert (got[n] == 7.0).all()
+    for e in range(E):
+        x = {"gate": gate_up[e, :I].double(), "up": gate_up[e, I:].double(),
+             "down": down[e].double()}
+        t = (ids == e).nonzero()[:, 0].cuda()
+        if len(t):
+            close(got[t], oracle.clamped_glu(h[t].double(), x, "", 1.25), torch.bfloat16)
