@@ -170,42 +170,33 @@ class LlamaForCausalLM:
         """Returns logits [len(batch.sample_seq_ids), vocab]."""
         cfg = self.cfg
         N = batch.num_tokens
-        x = F.embedding(batch.token_ids, self.embed)
-        residual = None
+        residual = F.embedding(batch.token_ids, self.embed)
         qd = self.n_heads * self.head_dim
-        kvd = self.n_kv_heads * self.head_dim
+        norms = [lw.input_norm for lw in self.layers] + [self.final_norm]
+        normed = ops.rmsnorm(residual, norms[0], cfg.rms_eps)
         for li, lw in enumerate(self.layers):
-            if residual is None:
-                residual = x
-                normed = ops.rmsnorm(x, lw.input_norm, cfg.rms_eps)
-            else:
-                normed, residual = ops.fused_add_rmsnorm(x, residual, lw.input_norm, cfg.rms_eps)
-            qkv = ops.step_linear(normed, lw.qkv)
-            if lw.qkv_bias is not None:
-                qkv = qkv + lw.qkv_bias
-            # strided views into the fused GEMM output: the HIP kernels take
-            # a token stride, so no .contiguous() copies on the hot path
-            row = qkv.stride(0)
-            q = qkv.as_strided((N, self.n_heads, self.head_dim), (row, self.head_dim, 1))
-            k = qkv.as_strided(
-                (N, self.n_kv_heads, self.head_dim), (row, self.head_dim, 1), qd
-            )
-            v = qkv.as_strided(
-                (N, self.n_kv_heads, self.head_dim), (row, self.head_dim, 1), qd + kvd
-            )
-            q, k = ops.rope_and_cache(
-                q, k, v, batch.positions, batch.slot_mapping,
-                self.k_caches[li], self.v_caches[li], self.cos_sin,
-            )
+            q = self._queries(li, lw, normed, batch)
             attn = self._attention(li, q, batch)
-            o = ops.step_linear(attn.reshape(N, qd), lw.o)
-            if self.all_reduce is not None:
-                o = self.all_reduce(o)
-            normed2, residual = ops.fused_add_rmsnorm(o, residual, lw.post_norm, cfg.rms_eps)
-            mlp = ops.step_linear(ops.step_linear_swiglu(normed2, lw.gate_up), lw.down)
-            if self.all_reduce is not None:
-                mlp = self.all_reduce(mlp)
-            x = mlp
-        normed, _ = ops.fused_add_rmsnorm(x, residual, self.final_norm, cfg.rms_eps)
+            normed, residual = self._add_norm(attn.reshape(N, qd), lw.o, residual, lw.post_norm)
+            act = ops.step_linear_swiglu(normed, lw.gate_up)
+            normed, residual = self._add_norm(act, lw.down, residual, norms[li + 1])
         sel = normed[batch.logit_rows]
         return ops.step_linear(sel, self.lm_head).float()
+
+    def _queries(self, layer_idx: int, lw: LlamaLayerWeights, normed, batch: FlatBatch):
+        """Rotated queries [N, Hq, D]; the keys and values go to the layer's caches."""
+        to = (batch.positions, batch.slot_mapping, self.k_caches[layer_idx],
+              self.v_caches[layer_idx], self.cos_sin)
+        if lw.qkv_bias is None:
+            return ops.step_linear_rope_and_cache(normed, lw.qkv, self.n_heads, *to)
+        qkv = ops.step_linear(normed, lw.qkv) + lw.qkv_bias
+        H, G = self.n_heads, self.n_kv_heads
+        qkv = qkv.view(-1, H + 2 * G, self.head_dim)
+        return ops.rope_and_cache(qkv[:, :H], qkv[:, H : H + G], qkv[:, H + G :], *to)[0]
+
+    def _add_norm(self, x, w, residual, norm):
+        """The residual with x w^T added (over all ranks), in place, and its norm before it."""
+        if self.all_reduce is None:
+            return ops.step_linear_add_rmsnorm(x, w, residual, norm, self.cfg.rms_eps)
+        y = self.all_reduce(ops.step_linear(x, w))
+        return ops.fused_add_rmsnorm(y, residual, norm, self.cfg.rms_eps)

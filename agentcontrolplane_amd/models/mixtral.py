@@ -133,31 +133,15 @@ class MixtralForCausalLM(LlamaForCausalLM):
         x = F.embedding(batch.token_ids, self.embed)
         residual = None
         qd = self.n_heads * self.head_dim
-        kvd = self.n_kv_heads * self.head_dim
         for li, lw in enumerate(self.layers):
             if residual is None:
                 residual = x
                 normed = ops.rmsnorm(x, lw.input_norm, cfg.rms_eps)
             else:
                 normed, residual = ops.fused_add_rmsnorm(x, residual, lw.input_norm, cfg.rms_eps)
-            qkv = ops.step_linear(normed, lw.qkv)
-            row = qkv.stride(0)
-            q = qkv.as_strided((N, self.n_heads, self.head_dim), (row, self.head_dim, 1))
-            k = qkv.as_strided(
-                (N, self.n_kv_heads, self.head_dim), (row, self.head_dim, 1), qd
-            )
-            v = qkv.as_strided(
-                (N, self.n_kv_heads, self.head_dim), (row, self.head_dim, 1), qd + kvd
-            )
-            q, k = ops.rope_and_cache(
-                q, k, v, batch.positions, batch.slot_mapping,
-                self.k_caches[li], self.v_caches[li], self.cos_sin,
-            )
+            q = self._queries(li, lw, normed, batch)
             attn = self._attention(li, q, batch)
-            o = ops.step_linear(attn.reshape(N, qd), lw.o)
-            if self.all_reduce is not None:
-                o = self.all_reduce(o)
-            normed2, residual = ops.fused_add_rmsnorm(o, residual, lw.post_norm, cfg.rms_eps)
+            normed2, residual = self._add_norm(attn.reshape(N, qd), lw.o, residual, lw.post_norm)
             x = self._moe_mlp(li, normed2)
             if self.all_reduce is not None and self.moe_dispatch is None:
                 # TP-sharded experts (intermediate split): partial sums reduce

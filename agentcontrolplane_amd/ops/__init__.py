@@ -222,6 +222,45 @@ def step_linear_glu(x, w, glu, out):
         clamped_glu(step_linear(x, w), glu.limit, glu.alpha, glu.offset, out, cubic)
 
 
+def step_linear_add_rmsnorm(x, w, residual, weight, eps: float = 1e-5):
+    """fused_add_rmsnorm(step_linear(x, w), residual, weight, eps); a product in parts leaves
+    their sum to the norm's pass."""
+    if (
+        _many_rows(x, w)
+        and w.shape[0] <= _hip()._C.ADD_RMSNORM_MOST
+        and all(
+            t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
+            and t.data_ptr() % 16 == 0 for t in (residual, weight)
+        )
+        and residual.shape == (x.shape[0], w.shape[0])
+        and weight.shape == w.shape[:1]
+    ):
+        return _hip().linear_add_rmsnorm(x, w, residual, weight, eps)
+    return fused_add_rmsnorm(step_linear(x, w), residual, weight, eps)
+
+
+def step_linear_rope_and_cache(x, w, heads: int, positions, slot_mapping, k_cache, v_cache,
+                               cos_sin):
+    """rope_and_cache() of step_linear(x, w), rows of ``heads`` queries, then keys, then values as
+    the caches [.., Hkv, D] hold them, with a product in parts added up in its pass.  Returns the
+    queries [N, heads, D]."""
+    kv, d = k_cache.shape[-2:]
+    caches = (positions, slot_mapping, k_cache, v_cache, cos_sin)
+    if (
+        _many_rows(x, w)
+        and d % 128 == 0
+        and w.shape[0] == (heads + 2 * kv) * d
+        and k_cache.shape == v_cache.shape
+        and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in caches[2:])
+        and k_cache.dtype == v_cache.dtype == x.dtype
+        and positions.numel() == slot_mapping.numel() == x.shape[0]
+    ):
+        return _hip().linear_rope_and_cache(x, w, heads, *caches)
+    y = step_linear(x, w)
+    y = y.view(-1, heads + 2 * kv, d)
+    return rope_and_cache(y[:, :heads], y[:, heads:-kv], y[:, -kv:], *caches)[0]
+
+
 def linear_add_(y, x, w):
     """y += x @ w^T in one GEMM."""
     return y.addmm_(x, w.t())

@@ -23,6 +23,29 @@ def fused_add_rmsnorm(x, residual, weight, eps: float = 1e-5):
     return out, residual
 
 
+def linear_add_rmsnorm(x, w, residual, weight, eps: float):
+    y = _C.linear_parts(x, w)
+    if y.dim() == 2:
+        return fused_add_rmsnorm(y, residual, weight, eps)
+    out = torch.empty_like(residual)
+    _C.parts_add_rmsnorm(out, residual, y, weight, eps)
+    return out, residual
+
+
+def linear_rope_and_cache(x, w, heads: int, positions, slot_mapping, k_cache, v_cache, cos_sin):
+    y = _C.linear_parts(x, w)
+    kv, d = k_cache.shape[-2:]
+    if y.dim() == 2:
+        y = y.view(-1, heads + 2 * kv, d)
+        return rope_and_cache(
+            y[:, :heads], y[:, heads:-kv], y[:, -kv:], positions, slot_mapping, k_cache, v_cache,
+            cos_sin,
+        )[0]
+    q = torch.empty(x.shape[0], heads, d, dtype=x.dtype, device=x.device)
+    _C.rope_cache(q, None, None, positions, slot_mapping, k_cache, v_cache, cos_sin, y)
+    return q
+
+
 def rope_and_cache(q, k, v, positions, slot_mapping, k_cache, v_cache, cos_sin):
     _C.rope_cache(q, k, v, positions, slot_mapping, k_cache, v_cache, cos_sin)
     return q, k

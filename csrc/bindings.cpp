@@ -26,6 +26,11 @@ extern "C" {
 void launch_rmsnorm(void*, const void*, const void*, float, int, int, hipStream_t);
 void launch_fused_add_rmsnorm(void*, void*, const void*, const void*, float, int, int,
                               hipStream_t);
+void launch_parts_add_rmsnorm(void*, void*, const void*, const void*, float, int, int, int,
+                              hipStream_t);
+void launch_rope_cache_units(void*, void*, const void*, void*, void*, const int64_t*,
+                             const int64_t*, const float*, int, int, int, int, int64_t, int64_t,
+                             int64_t, const float*, int, hipStream_t);
 void launch_swiglu(void*, const void*, int64_t, int, hipStream_t);
 void launch_rope_cache(void*, void*, const void*, void*, void*, const int64_t*,
                        const int64_t*, const float*, int, int, int, int, int64_t,
@@ -119,6 +124,22 @@ static void fused_add_rmsnorm(torch::Tensor out, torch::Tensor residual,
                            weight.data_ptr(), (float)eps, n, h, cur_stream());
 }
 
+// parts [n, rows, h] fp32 of a product (linear_parts): out = rmsnorm(residual += their sum)
+static void parts_add_rmsnorm(torch::Tensor out, torch::Tensor residual, torch::Tensor parts,
+                              torch::Tensor weight, double eps) {
+  CHECK_CUDA(parts); CHECK_CONT(parts); CHECK_CONT(out); CHECK_CONT(residual); CHECK_CONT(weight);
+  CHECK_BF16(out); CHECK_BF16(residual); CHECK_BF16(weight);
+  TORCH_CHECK(parts.dim() == 3 && parts.scalar_type() == at::kFloat && parts.size(0) > 0);
+  const int64_t n = parts.size(1), h = parts.size(2);
+  TORCH_CHECK(h % 8 == 0 && h <= ADD_RMSNORM_MOST && n > 0 && n < (1 << 30) &&
+              out.numel() == n * h && residual.numel() == n * h && weight.numel() == h);
+  for (const void* p : {out.data_ptr(), residual.data_ptr(), weight.data_ptr()})
+    TORCH_CHECK((uintptr_t)p % 16 == 0, "alignment");
+  launch_parts_add_rmsnorm(out.data_ptr(), residual.data_ptr(), parts.data_ptr(),
+                           weight.data_ptr(), (float)eps, (int)n, (int)h, (int)parts.size(0),
+                           cur_stream());
+}
+
 static void swiglu(torch::Tensor out, torch::Tensor gate_up) {
   CHECK_CUDA(gate_up); CHECK_CONT(gate_up); CHECK_BF16(gate_up); CHECK_CONT(out);
   const int inter = gate_up.size(-1) / 2;
@@ -154,24 +175,49 @@ static void step_linear(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   launch_step_linear(&a, glu, cur_stream());
 }
 
-static void rope_cache(torch::Tensor q, torch::Tensor k, torch::Tensor v,
-                       torch::Tensor positions, torch::Tensor slot_mapping,
-                       torch::Tensor k_cache, torch::Tensor v_cache,
-                       torch::Tensor cos_sin) {
+// q, k (rotated in place) and v into the caches; ``parts`` [n, N, (Hq + 2 Hkv) D] fp32 of a
+// product (linear_parts): the queries of their sum into q, which is not read, no k and v
+static void rope_cache(torch::Tensor q, c10::optional<torch::Tensor> k,
+                       c10::optional<torch::Tensor> v, torch::Tensor positions,
+                       torch::Tensor slot_mapping, torch::Tensor k_cache, torch::Tensor v_cache,
+                       torch::Tensor cos_sin, c10::optional<torch::Tensor> parts) {
   CHECK_CUDA(q);
   CHECK_CONT(k_cache); CHECK_CONT(v_cache); CHECK_CONT(cos_sin);
+  TORCH_CHECK((k && v) != parts.has_value(), "keys and values, or parts");
   const int64_t q_stride = q_token_stride(q);
-  const int64_t kv_stride = q_token_stride(k);
-  TORCH_CHECK(v.stride(0) == kv_stride, "k/v must share layout");
+  const int64_t kv_stride = k ? q_token_stride(*k) : 0;
+  if (k) TORCH_CHECK(v->stride(0) == kv_stride, "k/v must share layout");
   TORCH_CHECK(positions.scalar_type() == at::kLong && slot_mapping.scalar_type() == at::kLong);
   TORCH_CHECK(cos_sin.scalar_type() == at::kFloat);
   const int N = q.size(0);
   const int Hq = q.size(1);
-  const int Hkv = k.size(1);
+  const int Hkv = k ? k->size(1) : k_cache.size(-2);
   const int D = q.size(2);
   const int64_t P = cos_sin.size(1);
   TORCH_CHECK(D % 128 == 0 || D <= 512, "head_dim constraint");
-  launch_rope_cache(q.data_ptr(), k.data_ptr(), v.data_ptr(), k_cache.data_ptr(),
+  auto aligned = [](const torch::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+  const bool units = D % 128 == 0 && q_stride % 8 == 0 && kv_stride % 8 == 0 && aligned(q) &&
+                     (!k || (aligned(*k) && aligned(*v))) && aligned(k_cache) &&
+                     aligned(v_cache) && aligned(cos_sin);
+  if (parts) {
+    CHECK_BF16(q); CHECK_BF16(k_cache); CHECK_BF16(v_cache);
+    CHECK_CUDA((*parts)); CHECK_CONT((*parts));
+    TORCH_CHECK(units && N > 0 && parts->dim() == 3 && parts->scalar_type() == at::kFloat &&
+                parts->size(0) > 0 && parts->size(1) == N &&
+                parts->size(2) == (int64_t)(Hq + 2 * Hkv) * D && k_cache.size(-1) == D &&
+                positions.numel() == N && slot_mapping.numel() == N, "rope_cache: parts");
+  }
+  void* kp = k ? k->data_ptr() : nullptr;
+  void* vp = v ? v->data_ptr() : nullptr;
+  if (units && N > 0) {
+    launch_rope_cache_units(q.data_ptr(), kp, vp, k_cache.data_ptr(), v_cache.data_ptr(),
+                            positions.data_ptr<int64_t>(), slot_mapping.data_ptr<int64_t>(),
+                            cos_sin.data_ptr<float>(), N, Hq, Hkv, D, P, q_stride, kv_stride,
+                            parts ? parts->data_ptr<float>() : nullptr,
+                            parts ? (int)parts->size(0) : 0, cur_stream());
+    return;
+  }
+  launch_rope_cache(q.data_ptr(), kp, vp, k_cache.data_ptr(),
                     v_cache.data_ptr(), positions.data_ptr<int64_t>(),
                     slot_mapping.data_ptr<int64_t>(), cos_sin.data_ptr<float>(), N,
                     Hq, Hkv, D, P, q_stride, kv_stride, cur_stream());
@@ -209,50 +255,82 @@ static void run_linear(const LinearArgs& a, int unit, int tile, int splits,
   launch_linear(&a, unit, tile, splits, splits > 1 ? parts.data_ptr() : nullptr, cur_stream());
 }
 
-// out = x w^T + bias, or the gated unit of its halves: "swiglu", "glu" with the form's numbers
-static void linear(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-                   const c10::optional<torch::Tensor>& bias, const std::string& unit,
-                   double limit, double alpha, double offset, double cubic, int64_t tile,
-                   int64_t splits) {
-  CHECK_CUDA(x); CHECK_CUDA(w); CHECK_CUDA(out);
-  CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(out);
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2);
+// The operands of x w^T, checked
+static LinearArgs linear_operands(const torch::Tensor& x, const torch::Tensor& w) {
+  CHECK_CUDA(x); CHECK_CUDA(w); CHECK_BF16(x); CHECK_BF16(w);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.device() == w.device());
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  const bool glu = unit == "swiglu" || unit == "glu";
-  TORCH_CHECK(glu || unit == "plain", "unknown unit");
-  const int64_t outs = glu ? N / 2 : N;
-  TORCH_CHECK(M > 0 && K > 0 && N > 0 && w.size(1) == K && K % 64 == 0 && outs % 8 == 0 &&
-              (!glu || N % 2 == 0) && out.size(0) == M && out.size(1) == outs, "linear: sizes");
-  TORCH_CHECK(x.device() == w.device() && x.device() == out.device());
-  TORCH_CHECK(x.stride(1) == 1 && w.stride(1) == 1 && out.stride(1) == 1);
+  TORCH_CHECK(M > 0 && K > 0 && N > 0 && w.size(1) == K && K % 64 == 0 && N % 8 == 0,
+              "linear: sizes");
+  TORCH_CHECK(x.stride(1) == 1 && w.stride(1) == 1);
   LinearArgs a = {};
   a.x_stride = M > 1 ? x.stride(0) : K;
   a.w_stride = N > 1 ? w.stride(0) : K;
-  a.out_stride = M > 1 ? out.stride(0) : outs;
-  for (int64_t stride : {a.x_stride, a.w_stride, a.out_stride})
+  for (int64_t stride : {a.x_stride, a.w_stride})
     TORCH_CHECK(stride >= 0 && stride % 8 == 0, "linear: strides");
-  for (const void* p : {x.data_ptr(), w.data_ptr(), out.data_ptr()})
+  for (const void* p : {x.data_ptr(), w.data_ptr()})
     TORCH_CHECK((uintptr_t)p % 16 == 0, "linear: alignment");
   // byte offsets of 32 bits; tiles past the end have up to 256 rows more
   TORCH_CHECK(((M - 1) * a.x_stride + K) * 2 < (1ll << 31) &&
               ((N - 1) * a.w_stride + K) * 2 < (1ll << 31) && M < (1 << 30) && N < (1 << 30),
               "linear: operands of 2 GiB and more");
+  a.x = x.data_ptr();
+  a.w = w.data_ptr();
+  a.M = (int)M; a.N = (int)N; a.K = (int)K;
+  return a;
+}
+
+// out = x w^T + bias, or the gated unit of its halves: "swiglu", "glu" with the form's numbers
+static void linear(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                   const c10::optional<torch::Tensor>& bias, const std::string& unit,
+                   double limit, double alpha, double offset, double cubic, int64_t tile,
+                   int64_t splits) {
+  LinearArgs a = linear_operands(x, w);
+  CHECK_CUDA(out); CHECK_BF16(out);
+  const int64_t M = a.M, N = a.N;
+  const bool glu = unit == "swiglu" || unit == "glu";
+  TORCH_CHECK(glu || unit == "plain", "unknown unit");
+  const int64_t outs = glu ? N / 2 : N;
+  TORCH_CHECK(outs % 8 == 0 && (!glu || N % 2 == 0) && out.dim() == 2 && out.size(0) == M &&
+              out.size(1) == outs, "linear: sizes");
+  TORCH_CHECK(x.device() == out.device() && out.stride(1) == 1);
+  a.out_stride = M > 1 ? out.stride(0) : outs;
+  TORCH_CHECK(a.out_stride >= 0 && a.out_stride % 8 == 0, "linear: strides");
+  TORCH_CHECK((uintptr_t)out.data_ptr() % 16 == 0, "linear: alignment");
   if (bias) {
     CHECK_CUDA((*bias)); CHECK_BF16((*bias)); CHECK_CONT((*bias));
     TORCH_CHECK(!glu && bias->numel() == N && (uintptr_t)bias->data_ptr() % 16 == 0);
     a.bias = bias->data_ptr();
   }
   TORCH_CHECK(tile < 0 || (linear_fits((int)tile, glu && splits == 1) && splits >= 1 &&
-                           splits <= K / 64), "linear: tile");
+                           splits <= a.K / 64), "linear: tile");
   a.out = out.data_ptr();
-  a.x = x.data_ptr();
-  a.w = w.data_ptr();
-  a.M = (int)M; a.N = (int)N; a.K = (int)K;
   a.limit = (float)limit; a.alpha = (float)alpha; a.offset = (float)offset;
   a.cubic = (float)cubic;
   const at::DeviceGuard guard(x.device());
   run_linear(a, unit == "swiglu" ? LINEAR_SWIGLU : glu ? LINEAR_GLU
              : bias ? LINEAR_BIAS : LINEAR_PLAIN, (int)tile, (int)splits, x);
+}
+
+// x w^T [M, N], or fp32 [parts, M, N] whose sum in their order it is, as the sizes call for where
+// what reads it adds them up
+static torch::Tensor linear_parts(torch::Tensor x, torch::Tensor w, int64_t tile,
+                                  int64_t splits) {
+  LinearArgs a = linear_operands(x, w);
+  TORCH_CHECK(tile < 0 || (linear_fits((int)tile, false) && splits >= 1 && splits <= a.K / 64),
+              "linear: tile");
+  int t = (int)tile, parts = (int)splits;
+  if (t < 0) linear_choice(a.M, a.N, a.K, LINEAR_PARTS, &t, &parts);
+  const int chunks = a.K / 64, each = (chunks + parts - 1) / parts;
+  parts = (chunks + each - 1) / each;  // all that have chunks
+  const at::DeviceGuard guard(x.device());
+  torch::Tensor out = parts > 1
+      ? torch::empty({parts, a.M, a.N}, x.options().dtype(torch::kFloat32))
+      : torch::empty({a.M, a.N}, x.options());
+  a.out = out.data_ptr();
+  a.out_stride = a.N;
+  launch_linear(&a, LINEAR_PARTS, t, parts, out.data_ptr(), cur_stream());
+  return out;
 }
 
 // C[M,N] = A[M,K] @ B[N,K]^T on the largest tiles
@@ -1163,7 +1241,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("swiglu", &swiglu);
   m.def("step_linear", &step_linear);
-  m.def("rope_cache", &rope_cache);
+  m.def("parts_add_rmsnorm", &parts_add_rmsnorm);
+  m.attr("ADD_RMSNORM_MOST") = ADD_RMSNORM_MOST;
+  m.def("rope_cache", &rope_cache, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("positions"),
+        py::arg("slot_mapping"), py::arg("k_cache"), py::arg("v_cache"), py::arg("cos_sin"),
+        py::arg("parts") = py::none());
+  m.def("linear_parts", &linear_parts, py::arg("x"), py::arg("w"), py::arg("tile") = -1,
+        py::arg("splits") = 1);
   m.def("prefill_attn", &prefill_attn);
   m.def("mfma_probe", &mfma_probe);
   m.def("linear", &linear, py::arg("out"), py::arg("x"), py::arg("w"),

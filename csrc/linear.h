@@ -15,10 +15,15 @@ struct LinearArgs {
   float limit, alpha, offset, cubic;  // LINEAR_GLU
 };
 
-// The tile and the parts of the inner dimension that the sizes call for
+// The tile and the parts of the inner dimension that the sizes call for; unit LINEAR_PARTS: where
+// the parts' sums are added up by what reads them
 extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* splits);
-// tile: a number that linear_fits(); from 2 splits on with parts [splits, M, N] fp32
+// tile: a number that linear_fits(); from 2 splits on with parts [splits, M, N] fp32, which are
+// all that unit LINEAR_PARTS writes
 extern "C" void launch_linear(const LinearArgs* a, int unit, int tile, int splits, void* parts,
                               hipStream_t stream);
 // Is there such a tile, for gates and ups?
 extern "C" bool linear_fits(int tile, bool glu);
+
+// The longest rows that are added up and normed in one pass (elementwise.hip)
+#define ADD_RMSNORM_MOST 16384

@@ -181,7 +181,8 @@ extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* spl
       const double sums = s > 1 ? 8.0 * s * M * N : 2.0 * M * N;
       const double memory = (2.0 * N * K + 2.0 * M * K + sums) / 6.4e6;
       const double us =
-          sqrt(busiest * busiest + memory * memory) + (s > 1 ? 4.3 + sums / 21.7e6 : 0);
+          sqrt(busiest * busiest + memory * memory) +
+          (s > 1 ? (unit == LINEAR_PARTS ? 0.5 : 4.3) + sums / 21.7e6 : 0);
       if (*tile >= 0 && us >= best) continue;
       best = us;
       *tile = i;
@@ -198,6 +199,8 @@ extern "C" void launch_linear(const LinearArgs* args, int unit, int tile, int sp
   if (splits > 1) {
     kind = LINEAR_PARTS;
     a.out = parts;
+  } else if (unit == LINEAR_PARTS) {
+    kind = LINEAR_PLAIN;
   }
 #define LAUNCH_AS(n, m, ws_, xs_, u)                                       \
   if (kind == u && t.fn == n && t.fm == m && t.ws == ws_ && t.xs == xs_)   \
@@ -212,7 +215,7 @@ extern "C" void launch_linear(const LinearArgs* args, int unit, int tile, int sp
   LAUNCH_AS(n, m, ws, xs, LINEAR_GLU)
   TILES(LAUNCH)
   PLAIN_TILES(LAUNCH_PLAIN)
-  if (splits > 1) {
+  if (splits > 1 && unit != LINEAR_PARTS) {
     a.out = args->out;
     unit == LINEAR_PLAIN    ? sum<LINEAR_PLAIN>(a, parts, splits, stream)
     : unit == LINEAR_BIAS   ? sum<LINEAR_BIAS>(a, parts, splits, stream)

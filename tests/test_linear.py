@@ -137,3 +137,99 @@ def test_rule_of_many_rows():
     want = torch.empty_like(out)
     ops.clamped_glu(ops.linear(x + 1, w + 0.01), 7.0, 1.702, 1.0, want)
     assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,tile,splits", [
+    (1, 8, 128, 11, 2), (61, 4096, 4096, 6, 4), (190, 4096, 1024, 6, 3), (13, 9224, 448, 12, 5),
+    (1100, 16384, 128, 0, 2), (3, 520, 192, 9, 3), (7, 16392, 256, 12, 4),
+])
+def test_parts_into_the_norm(m, n, k, tile, splits):
+    """As the parts' own sum and the norm of it: the same roundings, in the same order."""
+    hip = ops._hip()
+    x, w = operands(m, n, k, m + n)
+    gen = torch.Generator().manual_seed(n)
+    residual = torch.randn(m, n, generator=gen).bfloat16().cuda()
+    weight = torch.rand(n, generator=gen).bfloat16().cuda()
+    parts = hip._C.linear_parts(x, w, tile, splits)
+    if n > hip._C.ADD_RMSNORM_MOST:
+        with pytest.raises(RuntimeError):
+            hip._C.parts_add_rmsnorm(residual.clone(), residual, parts, weight, 1e-5)
+        return
+    y = parts if parts.dim() == 2 else hip.linear(x, w, tile=tile, splits=splits)
+    sums = residual.clone()
+    got = torch.empty_like(residual)
+    if parts.dim() == 3:
+        hip._C.parts_add_rmsnorm(got, sums, parts, weight, 1e-5)
+    else:
+        hip._C.fused_add_rmsnorm(got, sums, y, weight, 1e-5)
+    new = (y.float() + residual.float()).bfloat16()
+    assert torch.equal(sums, new)
+    want = new.double() * torch.rsqrt((new.double() ** 2).mean(-1, keepdim=True) + 1e-5)
+    # one rounding of the result, and sums of n squares in 32 bits
+    assert ((got.double() - want * weight.double()).abs() <=
+            (2.0 ** -8 + n * 2.0 ** -24) * (want * weight.double()).abs()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,heads,kv,d,k,tile,splits", [
+    (1, 1, 1, 128, 128, 11, 2), (61, 32, 8, 128, 256, 5, 3), (13, 4, 4, 256, 448, 12, 5),
+    (300, 2, 1, 512, 64, 0, 1),
+])
+def test_parts_into_the_caches(m, heads, kv, d, k, tile, splits):
+    """Queries and cached rows are those of the sum's own pass and a rotation a head at a time."""
+    hip = ops._hip()
+    x, w = operands(m, (heads + 2 * kv) * d, k, m)
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    angles = torch.rand(2 * 50 * (d // 2) + 1, generator=gen, device="cuda")
+    aside = angles[1:].view(2, 50, d // 2)  # rows of no 16-byte units
+    tables = aside.clone()
+    pos = torch.randint(0, 50, (m,), generator=gen, device="cuda")
+    slots = torch.randperm(m + 9, generator=gen, device="cuda")[:m]
+
+    def caches():
+        return [torch.zeros(m + 9, kv, d, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+
+    y = hip.linear(x, w, tile=tile, splits=splits).view(m, heads + 2 * kv, d)
+    results = []
+    for cos_sin in (aside, tables):
+        q, key, v = (t.clone() for t in y.split([heads, kv, kv], 1))
+        results.append((q, *caches()))
+        hip.rope_and_cache(q, key, v, pos, slots, *results[-1][1:], cos_sin)
+    parts = hip._C.linear_parts(x, w, tile, splits)
+    if parts.dim() == 3:
+        results.append((torch.empty_like(results[0][0]), *caches()))
+        to = results[-1]
+        hip._C.rope_cache(to[0], None, None, pos, slots, *to[1:], tables, parts)
+    for other in results[1:]:
+        for a, b in zip(results[0], other):
+            # the compiler may round a product before the sum in one of two kernels
+            assert ((a.float() - b.float()).abs() <= 2.0 ** -7 * a.float().abs() + 1e-6).all()
+        assert torch.equal(results[0][2], other[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 61, 190, 2100])
+def test_step_linear_with_what_follows(m):
+    """The entries are the passes one after another, to a rounding of the product."""
+    x, w = operands(m, 2048, 1024, m)
+    residual = x.repeat(1, 2)
+    weight = torch.rand(2048, device="cuda").bfloat16()
+    got, sums = ops.step_linear_add_rmsnorm(x, w, residual.clone(), weight)
+    want, new = ops.fused_add_rmsnorm(ops.step_linear(x, w), residual.clone(), weight)
+    assert torch.allclose(sums.float(), new.float(), rtol=2.0 ** -6, atol=0.5)
+    assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -6, atol=0.03)
+    cos_sin = torch.rand(2, 9, 64, device="cuda")
+    pos, slots = torch.arange(m, device="cuda") % 9, torch.arange(m, device="cuda")
+    both = []
+    for fused in (True, False):
+        kc, vc = (torch.zeros(m, 4, 128, device="cuda").bfloat16() for _ in range(2))
+        to = (pos, slots, kc, vc, cos_sin)
+        if fused:
+            q = ops.step_linear_rope_and_cache(x, w, 8, *to)
+        else:
+            y = ops.step_linear(x, w).view(m, 16, 128)
+            q = ops.rope_and_cache(y[:, :8], y[:, 8:12], y[:, 12:], *to)[0]
+        both.append((q, kc, vc))
+    for a, b in zip(*both):
+        assert torch.allclose(a.float(), b.float(), rtol=2.0 ** -6, atol=0.5)
