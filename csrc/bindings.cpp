@@ -49,7 +49,8 @@ void launch_embed_positions(bool, float*, float*, const int64_t*, const int64_t*
                             const float*, float, int, int, int64_t, int64_t, hipStream_t);
 void launch_attn_inputs(bool, const AttnInputsArgs*, hipStream_t);
 void launch_moe_route(bool, int*, float*, const void*, const void*, const float*, int, int, int,
-                      int, int64_t, bool, float, hipStream_t);
+                      int, int64_t, bool, float, float*, int, hipStream_t);
+int moe_route_parts(bool, int, int, int);
 void launch_moe_group(int*, int*, int*, int*, const int*, int, int, const TiledProducts*,
                       hipStream_t);
 void launch_experts_small(bool, const ExpertsArgs*, int, hipStream_t);
@@ -1048,9 +1049,13 @@ static void moe_route(torch::Tensor ids, torch::Tensor weights, torch::Tensor h,
   if (bias) check_vec(*bias, at::kFloat, E);
   TORCH_CHECK(K % 64 == 0 && E <= 512 && top > 0 && top <= E && top <= 64, "router sizes");
   if (N == 0) return;
+  const int parts = moe_route_parts(is_bf16(h), N, E, K);
+  torch::Tensor sums;
+  if (parts > 1) sums = torch::empty({parts, N, (E + 15) / 16 * 16}, weights.options());
   launch_moe_route(is_bf16(h), ids.data_ptr<int>(), weights.data_ptr<float>(), h.data_ptr(),
                    w.data_ptr(), bias ? bias->data_ptr<float>() : nullptr, N, E, K, top,
-                   h.stride(0), sigmoid, (float)scale, cur_stream());
+                   h.stride(0), sigmoid, (float)scale,
+                   parts > 1 ? sums.data_ptr<float>() : nullptr, parts, cur_stream());
 }
 
 // perm [n], offsets [E + 2]; tiles of at least EXPERT_TILE rows: at most ceil(n / tile) + E, for

@@ -10,6 +10,8 @@ typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef float f32x4_v __attribute__((ext_vector_type(4)));
 
 #define ROUTE_T 16  // tokens per workgroup
+#define ROUTE_WAVES 4     // of a workgroup that has a part of K
+#define ROUTE_MOST 1024
 #define AHEAD 8      // turns whose ids are loaded together
 
 // The wave picks the ``top`` largest of logits[0 .. E) (overwritten), the lower index
@@ -56,14 +58,20 @@ static DEV void choose(float* logits, const float* scores, int E, int top, float
 // 16 tokens a workgroup: its waves split K in blocks of 64, partial logits meet in LDS.
 // NF fragments of 16 experts at a time.
 // Dynamic LDS: [waves][16][E16] floats, E16 = E rounded up to 16.
+// A CU takes about 25 GB/s from memory, so the weights of 32 experts of 4096 take one 10 us,
+// and few tokens leave the others idle.  With ``sums`` [parts of K][N][E16] the workgroups of
+// grid row y take part y of K, and route_sums_kernel chooses: 48 tokens, 32 experts of 4096
+// 18.4 to 11.1 us for both launches.
 template <int NF>
 __global__ __launch_bounds__(1024) void route_mfma_kernel(
     int* __restrict__ ids, float* __restrict__ weights, const bf16_t* __restrict__ h,
     const bf16_t* __restrict__ w, const float* __restrict__ bias, const int N, const int E,
-    const int K, const int top, const int64_t h_stride, const bool sigmoid, const float scale) {
+    const int K, const int top, const int64_t h_stride, const bool sigmoid, const float scale,
+    float* __restrict__ sums) {
   extern __shared__ float part[];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int c = lane & 15, g = lane >> 4;
+  const int blocks = gridDim.y * waves, block = blockIdx.y * waves + wid;
   const int E16 = (E + 15) & ~15, logits = ROUTE_T * E16;
   const int n0 = blockIdx.x * ROUTE_T;
   const bf16_t* hp = h + (int64_t)min(n0 + c, N - 1) * h_stride + g * 8;
@@ -75,7 +83,7 @@ __global__ __launch_bounds__(1024) void route_mfma_kernel(
       wp[i] = w + (int64_t)min(e0 + i * 16 + c, E - 1) * K + g * 8;
     f32x4_v acc[NF] = {};
 #pragma unroll 4
-    for (int k = wid * 64; k < K; k += waves * 64) {
+    for (int k = block * 64; k < K; k += blocks * 64) {
 #pragma unroll
       for (int s = 0; s < 64; s += 32) {
         const bf16x8_v b = *(const bf16x8_v*)(hp + k + s);
@@ -98,13 +106,38 @@ __global__ __launch_bounds__(1024) void route_mfma_kernel(
     const int e = i % E16;
     float z = 0.f;
     for (int p = 0; p < waves; ++p) z += part[(int64_t)p * logits + i];
+    if (sums) {
+      const int n = n0 + i / E16;
+      if (n < N) sums[((int64_t)blockIdx.y * N + n) * E16 + e] = z;
+      continue;
+    }
     if (sigmoid) part[logits + i] = z = 1.f / (1.f + expf(-z));
     part[i] = e < E ? z + (bias ? bias[e] : 0.f) : -INFINITY;
   }
+  if (sums) return;
   __syncthreads();
   for (int t = wid; t < min(ROUTE_T, N - n0); t += waves)
     choose(part + t * E16, sigmoid ? part + logits + t * E16 : nullptr, E, top, scale,
            ids + (int64_t)(n0 + t) * top, weights + (int64_t)(n0 + t) * top);
+}
+
+// The logits from their parts, in order; a wave a token, at most 128 experts.
+__global__ __launch_bounds__(64) void route_sums_kernel(
+    int* __restrict__ ids, float* __restrict__ weights, const float* __restrict__ sums,
+    const float* __restrict__ bias, const int N, const int E, const int parts, const int top,
+    const bool sigmoid, const float scale) {
+  __shared__ float logits[128], scores[128];
+  const int E16 = (E + 15) & ~15;
+  const int64_t n = blockIdx.x;
+  for (int e = threadIdx.x; e < E; e += 64) {
+    float z = 0.f;
+#pragma unroll 16
+    for (int p = 0; p < parts; ++p) z += sums[((int64_t)p * N + n) * E16 + e];
+    if (sigmoid) scores[e] = z = 1.f / (1.f + expf(-z));
+    logits[e] = z + (bias ? bias[e] : 0.f);
+  }
+  __syncthreads();
+  choose(logits, sigmoid ? scores : nullptr, E, top, scale, ids + n * top, weights + n * top);
 }
 
 // Any dtype: a workgroup per token, a wave per expert in turn.
@@ -141,51 +174,70 @@ static DEV uint64_t same_id(int id, int bits) {
   return m;
 }
 
-// Group the entries by expert, in their order: a counting sort by one workgroup, each
-// wave counting and placing its own run of entries.  Dynamic LDS: [17][E] ints.
+// Group the entries by expert, in their order: a counting sort.  Every workgroup counts all
+// entries (atomics in LDS), its waves their own runs of its share as well, which they then
+// place; the last one lists the tiles.  One workgroup for all, whose waves placed 1 / 16 each,
+// took 33.6 us for 16372 entries of 32 experts with the tiles (now 14.4), 8.9 for 192 (now 7.1).
+// Dynamic LDS: [18][E] ints.
 template <bool TILED>
 __global__ __launch_bounds__(1024) void group_kernel(
     int* __restrict__ perm, int* __restrict__ offsets, int* __restrict__ tile_expert,
     int* __restrict__ tile_row, const int* __restrict__ ids, const int n, const int E,
     const TiledProducts sizes) {
   extern __shared__ int counts[];
+  __shared__ int step_tiles[EXPERT_TILE / 32];
   int* total = counts + 16 * E;
+  int* earlier = total + E;  // in the shares before this one
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int bits = 32 - __clz(E);  // E itself marks lanes past the end
-  for (int i = threadIdx.x; i < 16 * E; i += 1024) counts[i] = 0;
+  const int shares = gridDim.x - 1, per = ((n + shares - 1) / shares + 1023) / 1024 * 64;  // a wave's
+  const bool lists = blockIdx.x == shares;
+  const int share = blockIdx.x * per * 16;
+  for (int i = threadIdx.x; i < 18 * E; i += 1024) counts[i] = 0;
   __syncthreads();
-  const int per = ((n + 15) / 16 + 63) / 64 * 64;
-  const int i0 = wid * per, i1 = min(n, i0 + per);
-  int* mine = counts + wid * E;
-  auto turns = [&](auto&& turn) {  // over this wave's entries, their ids loaded ahead
-    for (int i = i0; i < i1; i += 64 * AHEAD) {
+  auto turns = [&](int i0, int i1, int step, auto&& turn) {  // with the ids loaded ahead
+    for (int i = i0; i < i1; i += step * AHEAD) {
       int id[AHEAD];
 #pragma unroll
       for (int j = 0; j < AHEAD; ++j) {
-        const int at = i + j * 64 + lane;
+        const int at = i + j * step;
         id[j] = at < i1 ? ids[at] : E;
       }
 #pragma unroll
-      for (int j = 0; j < AHEAD; ++j) turn(i + j * 64 + lane, id[j]);
+      for (int j = 0; j < AHEAD; ++j) turn(i + j * step, id[j]);
     }
   };
-  turns([&](int, int id) {
-    const uint64_t m = same_id(id, bits);
-    if (id < E && lane == __builtin_ctzll(m)) mine[id] += __popcll(m);
-    asm volatile("" ::: "memory");  // the next turn reads what other lanes wrote
+  turns(threadIdx.x, n, 1024, [&](int at, int id) {
+    if (id >= E) return;
+    atomicAdd(&total[id], 1);
+    if (at < share) atomicAdd(&earlier[id], 1);
+  });
+  const int i0 = lists ? n : share + wid * per, i1 = min(n, i0 + per);
+  int* mine = counts + wid * E;
+  turns(i0 + lane, i1, 64, [&](int, int id) {
+    if (id < E) atomicAdd(&mine[id], 1);
   });
   __syncthreads();
-  for (int e = threadIdx.x; e < E; e += 1024) {
-    int run = 0;
-    for (int w = 0; w < 16; ++w) {
-      const int t = counts[w * E + e];
-      counts[w * E + e] = run;
-      run += t;
+  if (!lists)
+    for (int e = threadIdx.x; e < E; e += 1024) {
+      int run = earlier[e];
+      for (int w = 0; w < 16; ++w) {
+        const int t = counts[w * E + e];
+        counts[w * E + e] = run;
+        run += t;
+      }
     }
-    total[e] = run;
-  }
-  __syncthreads();
-  if (wid == 0) {  // first rows and tiles of the experts
+  auto before = [&](int v, int& sum) {  // the lanes before this one's; the wave's sum
+    int s = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int w = __shfl_up(s, off, 64);
+      if (lane >= off) s += w;
+    }
+    sum = __shfl(s, 63, 64);
+    return s - v;
+  };
+  if (lists) {  // first rows of the experts and their tiles
     // Tall tiles take up to an eighth longer each, which pays where they save rounds of
     // workgroups (one a CU, columns a tile) in one of the two products; a tile of up to 192 rows
     // takes about 0.6 of a round.  Both products, us, in tiles of 256 and tall ones: 32 experts,
@@ -231,21 +283,13 @@ __global__ __launch_bounds__(1024) void group_kernel(
       }
       return t;
     };
-    auto before = [&](int v, int& sum) {  // the lanes before this one's; the wave's sum
-      int s = v;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const int w = __shfl_up(s, off, 64);
-        if (lane >= off) s += w;
-      }
-      sum = __shfl(s, 63, 64);
-      return s - v;
-    };
-    int row = 0, tile = 0, sum;
-    // the highest tiles first, by steps of 32 rows: workgroups that end early then fill up with
-    // the lower ones
-    for (int step = TILED && sizes.even ? EXPERT_TILE / 32 : 1; TILED && step > 0; --step) {
-      row = 0;
+    // the highest tiles first, by steps of 32 rows, a wave each: workgroups that end early then
+    // fill up with the lower ones
+    const int steps = !TILED ? 0 : sizes.even ? EXPERT_TILE / 32 : 1;
+    const int step = steps - wid;  // of rows
+    int tile = 0;
+    auto list = [&](bool count) {
+      int row = 0, sum;
       for (int e0 = 0; e0 < E; e0 += 64) {
         const int e = e0 + lane, c = e < E ? total[e] : 0;
         int high;
@@ -255,29 +299,50 @@ __global__ __launch_bounds__(1024) void group_kernel(
         row += sum;
         const int at = tile + before(t, sum);
         tile += sum;
-        for (int j = 0; j < t; ++j) {
+        for (int j = 0; j < t && !count; ++j) {
           tile_expert[at + j] = e;
           tile_row[at + j] = first + j * high;
         }
       }
+    };
+    if (step > 0) {
+      list(true);
+      if (lane == 0) step_tiles[wid] = tile;
     }
-    row = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + lane, c = e < E ? total[e] : 0;
-      const int first = row + before(c, sum);
-      row += sum;
-      if (e < E) {
-        total[e] = first;
-        offsets[e] = first;
+    __syncthreads();
+    if (step > 0) {
+      tile = 0;
+      for (int w = 0; w < wid; ++w) tile += step_tiles[w];
+      list(false);
+    }
+    if (wid == 15) {
+      int row = 0, sum;
+      for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane;
+        const int first = row + before(e < E ? total[e] : 0, sum);
+        row += sum;
+        if (e < E) offsets[e] = first;
+      }
+      if (lane == 0) {
+        offsets[E] = row;
+        tile = 0;
+        for (int w = 0; w < steps; ++w) tile += step_tiles[w];
+        offsets[E + 1] = tile;
       }
     }
-    if (lane == 0) {
-      offsets[E] = row;
-      offsets[E + 1] = tile;
+    return;
+  }
+  if (wid == 0) {
+    int row = 0, sum;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane;
+      const int first = row + before(e < E ? total[e] : 0, sum);
+      row += sum;
+      if (e < E) total[e] = first;
     }
   }
   __syncthreads();
-  turns([&](int at, int id) {
+  turns(i0 + lane, i1, 64, [&](int at, int id) {
     const uint64_t m = same_id(id, bits);
     const int leader = __builtin_ctzll(m);
     int base = 0;
@@ -386,19 +451,30 @@ __global__ __launch_bounds__(256) void experts_f32_kernel(const ExpertsArgs a) {
 
 extern "C" {
 
+// Parts of K for few tokens: a block of 64 a wave, and no more workgroups than CUs; from
+// ROUTE_MOST tokens on the CUs are busy as it is
+int moe_route_parts(bool bf16, int N, int E, int K) {
+  const int tiles = (N + ROUTE_T - 1) / ROUTE_T;
+  if (!bf16 || E > 128 || N >= ROUTE_MOST) return 1;
+  return max(1, min(256 / tiles, K / (64 * ROUTE_WAVES)));
+}
+
 void launch_moe_route(bool bf16, int* ids, float* weights, const void* h, const void* w,
                       const float* bias, int N, int E, int K, int top, int64_t h_stride,
-                      bool sigmoid, float scale, hipStream_t stream) {
+                      bool sigmoid, float scale, float* sums, int parts, hipStream_t stream) {
   const int E16 = (E + 15) & ~15;
   if (bf16 && E <= 128) {  // at most 64 KiB of partial logits
     // few workgroups: more waves share the weights' latency
-    const int waves = N <= 4096 && E16 <= 64 ? 16 : 8;
+    const int waves = parts > 1 ? ROUTE_WAVES : N <= 4096 && E16 <= 64 ? 16 : 8;
     auto k = E16 <= 16   ? route_mfma_kernel<1>
              : E16 <= 32 ? route_mfma_kernel<2>
                          : route_mfma_kernel<4>;
-    k<<<(N + ROUTE_T - 1) / ROUTE_T, 64 * waves, waves * ROUTE_T * E16 * 4, stream>>>(
+    k<<<dim3((N + ROUTE_T - 1) / ROUTE_T, parts), 64 * waves, waves * ROUTE_T * E16 * 4, stream>>>(
         ids, weights, (const bf16_t*)h, (const bf16_t*)w, bias, N, E, K, top, h_stride, sigmoid,
-        scale);
+        scale, parts > 1 ? sums : nullptr);
+    if (parts > 1)
+      route_sums_kernel<<<N, 64, 0, stream>>>(ids, weights, sums, bias, N, E, parts, top, sigmoid,
+                                              scale);
   } else if (bf16) {
     route_plain_kernel<bf16_t><<<N, 256, E * 8, stream>>>(
         ids, weights, (const bf16_t*)h, (const bf16_t*)w, bias, E, K, top, h_stride, sigmoid,
@@ -413,7 +489,9 @@ void launch_moe_route(bool bf16, int* ids, float* weights, const void* h, const 
 void launch_moe_group(int* perm, int* offsets, int* tile_expert, int* tile_row, const int* ids,
                       int n, int E, const TiledProducts* sizes, hipStream_t stream) {
   auto kernel = tile_expert ? group_kernel<true> : group_kernel<false>;
-  kernel<<<1, 1024, 17 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E, *sizes);
+  // a share has at least 1024 entries, a turn of its waves; one more workgroup for the lists
+  const int shares = max(1, min(64, n / 1024));
+  kernel<<<shares + 1, 1024, 18 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E, *sizes);
 }
 
 // tt: token fragments at a time, 1 or 2

@@ -494,6 +494,45 @@ def test_route(device, dtype, n, E, K, top):
                        ops.moe_route(h, w, torch.full_like(b, 3.0), top)[0].sort(-1).values.cpu())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("sigmoid", [False, True])
+@pytest.mark.parametrize("n,E,K,top", [
+    (1, 32, 4096, 4), (17, 100, 512, 8), (1023, 128, 576, 2), (1024, 32, 512, 4), (48, 1, 8192, 1),
+])
+def test_route_in_parts(n, E, K, top, sigmoid):
+    """Few tokens take K in parts: odd numbers of tokens, of experts and of parts, and the first
+    number of tokens that does not."""
+    h = rand(n, K, dtype=torch.bfloat16, device="cuda")
+    w = rand(E, K, dtype=torch.bfloat16, device="cuda", seed=1, scale=K ** -0.5)
+    b = rand(E, dtype=F32, device="cuda", seed=2, scale=0.5)
+    ids, weights = ops.moe_route(h, w, b, top, sigmoid, 1.5)
+    z = h.double() @ w.double().T
+    z = torch.sigmoid(z) if sigmoid else z
+    chosen = (z + b.double()).gather(1, ids.long())
+    # a close call may go either way, by sums of K products in 32 bits
+    assert (chosen - torch.topk(z + b.double(), top, -1).values).abs().max() < 1e-5
+    of = z.gather(1, ids.long())
+    want = of / of.sum(-1, keepdim=True) if sigmoid else torch.softmax(chosen, -1)
+    close(weights.cpu(), 1.5 * want.cpu(), F32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("n,E", [(1, 1), (1025, 512), (16372, 32), (2048, 7), (70001, 64)])
+def test_group(n, E, tiled):
+    """One share of the entries, several, with a last one of few; skewed: as a stable sort."""
+    from agentcontrolplane_amd import _C
+
+    g = torch.Generator().manual_seed(n)
+    ids = (torch.rand(n, generator=g) ** 3 * E).int().clamp(max=E - 1).cuda()
+    lists = torch.empty(2, n // _C.EXPERT_TILE + E, dtype=torch.int32, device="cuda")
+    perm, offsets = torch.empty_like(ids), lists.new_empty(E + 2)
+    _C.moe_group(perm, offsets, *(lists if tiled else (None, None)), ids, E, 64, 64, 64, True)
+    assert torch.equal(perm.long(), torch.sort(ids, stable=True).indices)
+    first = torch.bincount(ids, minlength=E).cumsum(0)
+    assert offsets[0] == 0 and torch.equal(offsets[1 : E + 1].long(), first)
+
+
 def test_route_ties_and_order(device, dtype):
     """Equal logits: the lower expert first; the weights fall."""
     w = torch.zeros(6, 64, dtype=dtype, device=device)
@@ -509,6 +548,7 @@ EXPERTS = [
     (1, 4, 2, 64, 64, 40), (3, 6, 3, 192, 64, 160), (50, 8, 4, 128, 128, 96),
     (70, 3, 2, 64, 192, 31), (300, 4, 2, 128, 128, 130), (700, 2, 1, 256, 256, 258),
     (260, 3, 3, 128, 384, 512), (40, 40, 1, 64, 64, 64), (1030, 5, 2, 512, 128, 72),
+    (512, 100, 2, 64, 64, 40), (513, 100, 2, 64, 64, 40),
 ]
 
 
