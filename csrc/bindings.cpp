@@ -40,7 +40,9 @@ void launch_prefill_attn(void*, const void*, const void*, const void*, const int
                          float, int, int, int, int, int, int, int64_t, hipStream_t);
 void launch_sample_fullvocab(int64_t*, const void*, bool, const float*, const int64_t*,
                              const float*, const float*, const uint8_t*, const int32_t*,
-                             int, int, hipStream_t);
+                             int, int, void*, int, hipStream_t);
+int sample_fullvocab_chunks(int, int);
+int64_t sample_fullvocab_bytes(int, int);
 void launch_sample(int64_t*, const float*, const float*, const int64_t*, const float*,
                    const float*, const uint8_t*, int, int, hipStream_t);
 void launch_residual_norm(bool, float*, const void*, const void*, const void*, void*, float,
@@ -371,7 +373,7 @@ static void sample_fullvocab(torch::Tensor out, torch::Tensor logits,
                              torch::Tensor temps, torch::Tensor top_ks,
                              torch::Tensor top_ps, torch::Tensor uniforms,
                              c10::optional<torch::Tensor> mask,
-                             c10::optional<torch::Tensor> mask_map) {
+                             c10::optional<torch::Tensor> mask_map, int64_t chunks) {
   CHECK_CUDA(logits); CHECK_CONT(logits);
   const bool bf16 = logits.scalar_type() == at::kBFloat16;
   TORCH_CHECK(bf16 || logits.scalar_type() == at::kFloat,
@@ -388,10 +390,14 @@ static void sample_fullvocab(torch::Tensor out, torch::Tensor logits,
     mptr = (const uint8_t*)mask->data_ptr();
     mapptr = mask_map->data_ptr<int32_t>();
   }
+  const int n = chunks < 0 ? sample_fullvocab_chunks(B, V) : (int)chunks;
+  TORCH_CHECK(n == 0 || n == 8 || n == 16 || n == 32, "chunks");
+  torch::Tensor work;
+  if (n) work = torch::empty({sample_fullvocab_bytes(B, n)}, logits.options().dtype(at::kByte));
   launch_sample_fullvocab(out.data_ptr<int64_t>(), logits.data_ptr(), bf16,
                           temps.data_ptr<float>(), top_ks.data_ptr<int64_t>(),
                           top_ps.data_ptr<float>(), uniforms.data_ptr<float>(),
-                          mptr, mapptr, B, V, cur_stream());
+                          mptr, mapptr, B, V, n ? work.data_ptr() : nullptr, n, cur_stream());
 }
 
 // ---- fp32-residual norms, gated activations, latent attention: bf16 or fp32
@@ -1288,5 +1294,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("delta_prompts", &delta_prompts);
   m.def("delta_step", &delta_step);
   m.def("sample", &sample);
-  m.def("sample_fullvocab", &sample_fullvocab);
+  m.def("sample_fullvocab", &sample_fullvocab, py::arg("out"), py::arg("logits"),
+        py::arg("temps"), py::arg("top_ks"), py::arg("top_ps"), py::arg("uniforms"),
+        py::arg("mask"), py::arg("mask_map"), py::arg("chunks") = -1);
 }

@@ -698,6 +698,48 @@ def test_gemm_bf16(m, n, k):
     assert maxerr(got, want) < tol, maxerr(got, want)
 
 
+@requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [513, 4099, 16384, 32000, 50257, 128256, 152064])
+def test_sample_fullvocab_chunks(V, dtype):
+    """Rows in chunks draw what a workgroup a row does: every kind of row, with masks, few distinct
+    logits (more keys in a bucket than a list takes), thresholds beyond the head, infinities and
+    NaN, greedy ties, a mask that leaves one token."""
+    C = hip()._C
+    gen = torch.Generator(device="cuda").manual_seed(V)
+    B = 48
+    x = torch.randn(B, V, generator=gen, device="cuda") * 2.5
+    x[8:16] = (x[8:16]).round()
+    x[16:20, ::3] = float("-inf")
+    x[20, 5] = float("inf")
+    x[21, V - 1] = float("nan")
+    x[22:24] = 1.0
+    x[24:28] *= 40
+    i = torch.arange(B, device="cuda")
+    temps = torch.where(i % 8 == 7, 0.0, 0.8)
+    ks = torch.where((i % 4 == 1) | (i % 4 == 3), 50, 0)
+    ks[40:44] = torch.tensor([1, V - 1, V, V // 2], device="cuda")
+    ps = torch.where(i % 4 >= 2, 0.9, 1.0)
+    ps[44:48] = torch.tensor([0.0, 1e-6, 0.99999, 0.5], device="cuda")
+    u = torch.rand(B, generator=gen, device="cuda")
+    mask = torch.rand(3, V, generator=gen, device="cuda") < 0.5
+    mask[2] = False
+    mask[2, V - 2] = True
+    which = torch.where(i % 5 == 0, (i // 5) % 3, -1).int()
+    x = x.to(dtype)
+    for m, to in ((None, None), (mask, which)):
+        outs = []
+        for chunks in (0, 8, 16, 32):
+            out = torch.full((B,), -1, device="cuda")
+            C.sample_fullvocab(out, x, temps, ks, ps, u, m, to, chunks)
+            outs.append(out.tolist())
+        assert outs[0] == outs[1] == outs[2] == outs[3]
+        assert all(0 <= t < V for t in outs[0])
+        if m is not None:
+            assert all(mask[w, t] for w, t in zip(which.tolist(), outs[0]) if w >= 0)
+
+
+
 @pytest.mark.gpu
 def test_sample_fullvocab_vs_oracle():
     """csrc/sampling_fullvocab.hip vs the fp32 reference over a Llama-3
