@@ -18,7 +18,8 @@
 // Bound by memory: 5.2 to 5.3 TB/s of keys and values at 64 x 4096 and 256 x 1024 tokens, 32
 // heads over 8.  Before, with products and sums over dims on the VALU, 4.1 TB/s there and 2.0 to
 // 3.0 where lengths differ: 61 x 310 to 4000 tokens 268 -> 122 us, 190 x 700 to 1300 265 -> 159,
-// 1 x 4002 203 -> 14 (two launches and their first loads, not memory).  Without the next block in
+// 1 x 4002 203 -> 14; with the values' loads, whole lines each, past the caches 190 x 700 to 1300 148
+// -> 139, 61 x 310 to 4000 120 -> 112.5, and 13 x 300 to 3900 of 32 key heads 95 -> 88 (two launches and their first loads, not memory).  Without the next block in
 // flight the same kernel takes 350 us at 190 x 700 to 1300; at 3 waves a SIMD the registers for
 // it are not there.
 #include "common_t.h"
@@ -231,8 +232,8 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
           r.k[g][s] = *(const bf16x8_v*)(kp + (uint64_t)(uint32_t)at.slot[g] * k_row + k_off + s * 64);
 #pragma unroll
       for (int n = 0; n < NV; ++n)
-        r.v[n] = *(const bf16x8_v*)(vp + (uint64_t)(uint32_t)at.slot[n * KPL / 16] * v_row +
-                                  n * KPL % 16 * v_row + v_off);
+        r.v[n] = __builtin_nontemporal_load((const bf16x8_v*)(
+            vp + (uint64_t)(uint32_t)at.slot[n * KPL / 16] * v_row + n * KPL % 16 * v_row + v_off));
     } else {
       const int k = min(blocks.key(i) + (lane & (KB - 1)), pos);
       const int page = k / a.kv_block;
