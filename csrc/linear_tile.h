@@ -30,8 +30,9 @@ DEV float unit_of(const LinearArgs& a, float gate, float up) {
 
 #ifdef __HIP_DEVICE_COMPILE__  // the host knows no buffer resources
 // Works start, start + step .. below total of a workgroup of 4 waves.  Fragments of a wave along
-// the outputs (FN) and the rows (FM); chunks of w (WS) and x (XS) in LDS.
-template <int FN, int FM, int WS, int XS, int UNIT, class Work>
+// the outputs (FN) and the rows (FM); chunks of w (WS) and x (XS) in LDS.  ONCE: no other
+// workgroup reads the same weights, whose loads then pass by the caches (nt).
+template <int FN, int FM, int WS, int XS, int UNIT, bool ONCE = false, class Work>
 DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   constexpr bool GLU = UNIT == LINEAR_SWIGLU || UNIT == LINEAR_GLU;
   constexpr int TN = 32 * FN, TM = 32 * FM;    // rows of w and of x of a tile
@@ -85,7 +86,7 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   };
   auto load_w = [&](int i) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(bw, (lds_char*)(lds + sw + (wid * LW + i) * 1024), 16,
-                                             vw[i], cw * 128, 0, 0);
+                                             vw[i], cw * 128, 0, ONCE ? 2 : 0);
   };
   auto load_x = [&](int i) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
