@@ -1,6 +1,7 @@
 """Which sizes the kernel of a small decode step's projections takes: those at which it was
 measured to be faster than the GEMM library."""
 import pytest
+import torch
 
 from agentcontrolplane_amd import ops
 
@@ -20,3 +21,26 @@ from agentcontrolplane_amd import ops
 ])
 def test_few_rows_go_where_they_are_faster(m, outs, k, glu, pays):
     assert ops._few_rows_pay(m, outs, k, glu) == pays
+
+
+@pytest.mark.parametrize("m,outs,k,glu,pays", [
+    (1, 5120, 5120, False, False), (4, 65536, 1024, False, False), (1, 512, 14336, False, False),
+    (4, 5120, 13824, False, False), (5, 4096, 14336, False, False),
+    (4, 4096, 14336, False, True), (1, 128256, 4096, False, True), (4, 18944, 3584, True, True),
+    (1, 4096, 7168, False, True), (4, 65536, 1536, False, True), (4, 6144, 4096, False, True),
+])
+def test_whole_lines_pay(m, outs, k, glu, pays):
+    assert ops._whole_lines_pay(m, outs, k, glu) == pays
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 3, 4])
+@pytest.mark.parametrize("n,k", [(2056, 5664), (6160, 3104)])
+def test_step_linear_of_whole_lines(m, n, k):
+    """Sizes of the second rule, with outputs that are no whole tiles and half a line at the end,
+    against double precision."""
+    x, w = torch.randn(m, k).bfloat16().cuda(), torch.randn(n, k).bfloat16().cuda()
+    assert not ops._few_rows_pay(m, n, k, False) and ops._few_rows(x, w)
+    got, want = ops.step_linear(x, w).double(), x.double() @ w.double().T
+    slack = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + slack + 1e-30).all()
