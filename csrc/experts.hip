@@ -356,6 +356,24 @@ __global__ __launch_bounds__(1024) void group_kernel(
   });
 }
 
+// Four outputs of a row from its sums, with GLU of the gates y and ups u
+template <bool GLU>
+static DEV void store_outputs(const ExpertsArgs& a, int64_t row, int o, f32x4_v v, f32x4_v u) {
+  float y[4] = {v[0], v[1], v[2], v[3]};
+  if (GLU) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {  // through the model's precision, as a GEMM stores it
+      const float gate = to_f(from_f<bf16_t>(y[k])), up = to_f(from_f<bf16_t>(u[k]));
+      y[k] = clamped_glu_f(gate, up, a.limit, a.alpha, a.offset, a.cubic);
+    }
+  }
+  bf16_t* dst = (bf16_t*)a.out + row * a.O + o;
+  if (a.O % 4 == 0)
+    store_f<4>(dst, y);
+  else
+    for (int k = 0; k < 4 && o + k < a.O; ++k) dst[k] = from_f<bf16_t>(y[k]);
+}
+
 // Few rows per expert: bound by the weights.  grid (outputs / 16 or 32, E); the 4 waves
 // of a workgroup split K in blocks of 64 and meet in LDS.  Two 16-row weight fragments:
 // gate and up of the same 16 outputs, or 32 outputs.  TT token fragments of 16 at a time.
@@ -404,22 +422,88 @@ __global__ __launch_bounds__(256) void experts_small_kernel(const ExpertsArgs a)
       const int l = j & 63, t = (j >> 6) % TT, i = (j >> 6) / TT;
       const int r = r0 + t * 16 + (l & 15), o = o0 + i * 16 + (l >> 4) * 4;
       if (r >= rows || o >= a.O) continue;
-      f32x4_v v = red[0][i][t][l] + red[1][i][t][l] + red[2][i][t][l] + red[3][i][t][l];
-      float y[4] = {v[0], v[1], v[2], v[3]};
-      if (GLU) {
-        v = red[0][1][t][l] + red[1][1][t][l] + red[2][1][t][l] + red[3][1][t][l];
+      const f32x4_v v = red[0][i][t][l] + red[1][i][t][l] + red[2][i][t][l] + red[3][i][t][l];
+      f32x4_v u = {};
+      if (GLU) u = red[0][1][t][l] + red[1][1][t][l] + red[2][1][t][l] + red[3][1][t][l];
+      store_outputs<GLU>(a, GLU ? row0 + r : a.perm[row0 + r], o, v, u);
+    }
+  }
+}
+
+// The same for weights that the memory-side cache (256 MB) cannot keep: a load has 8 rows of a whole
+// line (64 of K), past the caches.  The upper 8 rows and columns of a product have the line's other
+// half, and of its results those count whose row and column have the same half; 8 TT tokens at
+// a time.  32 experts of 4096 x 2560, 4 a token, both products with routing, us, by
+// experts_small_kernel and so: 2 tokens 129 and 105, 8 252 and 225, 48 374 and 334, 95 413 and 376.
+// Where a caller has no other layers between, smaller weights come from the caches, and half the
+// waves a CU are the slower choice: 16 of 2048 x 1536 1 token 36 and 40 us, 16 73 and 76.
+template <bool GLU, int TT>
+__global__ __launch_bounds__(256) void experts_lines_kernel(const ExpertsArgs a) {
+  __shared__ f32x4_v red[4][2][2][TT][2][16];  // wave, tile, 8 rows, tokens, half, (4 rows, token)
+  const int e = blockIdx.y;
+  const int row0 = a.offsets[e], rows = a.offsets[e + 1] - row0;
+  if (rows == 0) return;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int c = lane & 7, half = lane >> 3 & 1, j = lane >> 4, in = half * 32 + j * 8;
+  const int o0 = blockIdx.x * (GLU ? 16 : 32);
+  const bf16_t* w = (const bf16_t*)a.w + (int64_t)e * (GLU ? 2 : 1) * a.O * a.K + in;
+  const bf16_t* wp[2][2];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {  // through the model's precision, as a GEMM stores it
-          const float gate = to_f(from_f<bf16_t>(y[k])), up = to_f(from_f<bf16_t>(v[k]));
-          y[k] = clamped_glu_f(gate, up, a.limit, a.alpha, a.offset, a.cubic);
-        }
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int o = GLU ? o0 + p * 8 + c + i * a.O : min(o0 + i * 16 + p * 8 + c, a.O - 1);
+      wp[i][p] = w + (int64_t)o * a.K;
+    }
+  for (int r0 = 0; r0 < rows; r0 += 8 * TT) {
+    const bf16_t* xp[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      const int r = row0 + min(r0 + t * 8 + c, rows - 1);
+      xp[t] = (const bf16_t*)a.x + (int64_t)(GLU ? a.perm[r] / a.top : r) * a.x_stride + in;
+    }
+    f32x4_v acc[2][2][TT] = {};
+#pragma unroll 2
+    for (int k = wid * 64; k < a.K; k += 256) {
+      bf16x8_v f[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          f[i][p] = __builtin_nontemporal_load((const bf16x8_v*)(wp[i][p] + k));
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const bf16x8_v b = *(const bf16x8_v*)(xp[t] + k);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+            acc[i][p][t] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i][p], b, acc[i][p][t], 0, 0, 0);
       }
-      const int64_t row = GLU ? row0 + r : a.perm[row0 + r];
-      bf16_t* dst = (bf16_t*)a.out + row * a.O + o;
-      if (a.O % 4 == 0)
-        store_f<4>(dst, y);
-      else
-        for (int k = 0; k < 4 && o + k < a.O; ++k) dst[k] = from_f<bf16_t>(y[k]);
+    }
+    if (r0) __syncthreads();
+    if (half == j >> 1) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int t = 0; t < TT; ++t) red[wid][i][p][t][half][(j & 1) * 8 + c] = acc[i][p][t];
+    }
+    __syncthreads();
+    // a thread sums 4 outputs of one row
+    for (int n = threadIdx.x; n < (GLU ? 1 : 2) * 2 * TT * 16; n += 256) {
+      const int l = n & 15, t = (n >> 4) % TT, p = (n >> 4) / TT & 1, i = (n >> 5) / TT;
+      const int r = r0 + t * 8 + (l & 7), o = o0 + i * 16 + p * 8 + (l >> 3) * 4;
+      if (r >= rows || o >= a.O) continue;
+      auto sum = [&](int i) {
+        f32x4_v v = {};
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v += red[x][i][p][t][0][l] + red[x][i][p][t][1][l];
+        return v;
+      };
+      store_outputs<GLU>(a, GLU ? row0 + r : a.perm[row0 + r], o, sum(i), sum(1));
     }
   }
 }
@@ -494,12 +578,14 @@ void launch_moe_group(int* perm, int* offsets, int* tile_expert, int* tile_row, 
   kernel<<<shares + 1, 1024, 18 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E, *sizes);
 }
 
-// tt: token fragments at a time, 1 or 2
+// tt: 16 tokens at a time, or twice as many
 void launch_experts_small(bool glu, const ExpertsArgs* a, int tt, hipStream_t stream) {
   const int per = glu ? 16 : 32;
   const dim3 grid((a->O + per - 1) / per, a->E);
-  auto k = glu ? (tt == 1 ? experts_small_kernel<true, 1> : experts_small_kernel<true, 2>)
-               : (tt == 1 ? experts_small_kernel<false, 1> : experts_small_kernel<false, 2>);
+  const bool lines = (glu ? 4ll : 2ll) * a->E * a->O * a->K > 256 << 20;
+#define SMALL(kernel, t) (glu ? kernel<true, t> : kernel<false, t>)
+  auto k = lines ? (tt == 1 ? SMALL(experts_lines_kernel, 2) : SMALL(experts_lines_kernel, 4))
+                 : (tt == 1 ? SMALL(experts_small_kernel, 1) : SMALL(experts_small_kernel, 2));
   k<<<grid, 256, 0, stream>>>(*a);
 }
 

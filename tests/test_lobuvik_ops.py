@@ -626,6 +626,29 @@ def test_experts(device, dtype, n, E, top, K, I, W, skew):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,top,E,K,I,W", [(40, 3, 96, 2048, 384, 3722),
+                                           (260, 3, 96, 2048, 384, 3749)])
+def test_experts_of_large_weights(n, top, E, K, I, W):
+    """Beyond 256 MB of weights, few rows' loads are whole lines: 16 rows at a time and twice as
+    many, experts of more rows than that; outputs that are no whole tiles."""
+    g = torch.Generator().manual_seed(n)
+    p = torch.rand(n, E, generator=g) ** 4
+    ids = torch.multinomial(p, top, generator=g).int()
+    h = rand(n, K, dtype=torch.bfloat16, device="cuda")
+    gate_up = rand(E, 2 * I, K, dtype=torch.bfloat16, device="cuda", seed=1, scale=2 * K ** -0.5)
+    down = rand(E, W, I, dtype=torch.bfloat16, device="cuda", seed=2, scale=I ** -0.5)
+    assert gate_up.numel() * 2 > 256 << 20 and down.numel() * 2 > 256 << 20
+    got = ops.moe_experts(h, gate_up, down, ids.cuda(), ClampedGluSpec(I, 1.25))
+    for e in range(0, E, 7):
+        x = {"gate": gate_up[e, :I].double(), "up": gate_up[e, I:].double(),
+             "down": down[e].double()}
+        t, c = (ids == e).nonzero(as_tuple=True)
+        if len(t):
+            t, c = t.cuda(), c.cuda()
+            close(got[t, c], oracle.clamped_glu(h[t].double(), x, "", 1.25), torch.bfloat16)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("even", [True, False], ids=["even", "tall"])
 @pytest.mark.parametrize("I,W", [(128, 264), (2432, 130)])
 def test_experts_tile_lists(I, W, even):
