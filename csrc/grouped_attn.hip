@@ -19,7 +19,9 @@
 // heads over 8.  Before, with products and sums over dims on the VALU, 4.1 TB/s there and 2.0 to
 // 3.0 where lengths differ: 61 x 310 to 4000 tokens 268 -> 122 us, 190 x 700 to 1300 265 -> 159,
 // 1 x 4002 203 -> 14; with the values' loads, whole lines each, past the caches 190 x 700 to 1300 148
-// -> 139, 61 x 310 to 4000 120 -> 112.5, and 13 x 300 to 3900 of 32 key heads 95 -> 88 (two launches and their first loads, not memory).  Without the next block in
+// -> 139, 61 x 310 to 4000 120 -> 112.5, and 13 x 300 to 3900 of 32 key heads 95 -> 88; with the
+// keys' loads likewise, instead of 16 rows of half a line, 137, 109 and 85, 200 x 100 to 1000 of 64
+// heads over 8 130 -> 116, but 64 x 128 16.0 -> 16.7 (two launches and their first loads, not memory).  Without the next block in
 // flight the same kernel takes 350 us at 190 x 700 to 1300; at 3 waves a SIMD the registers for
 // it are not there.
 #include "common_t.h"
@@ -219,17 +221,25 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
     }
     return at;
   };
+  // A load of keys has 8 rows of whole lines, 64 dims: the upper 8 rows of a product, and its upper 8
+  // columns for the queries, have a line's other half.  Of its results those count whose row and
+  // column have the same half; the halves' sums meet across lanes.
+  constexpr int LINES = STEPS / 2;
   struct Rows {
-    bf16x8_v k[2][STEPS], v[NV];
+    bf16x8_v k[2][2][LINES], v[NV];
   };
-  const uint32_t k_off = c * k_row + j * 16, v_off = kl * v_row + el * 16;
+  const int c8 = c & 7, half = c >> 3;
+  const uint32_t k_off = c8 * k_row + half * 64 + j * 16, v_off = kl * v_row + el * 16;
   auto load = [&](int i, const Place& at, Rows& r) {
     if constexpr (PAGED) {
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s)
-          r.k[g][s] = *(const bf16x8_v*)(kp + (uint64_t)(uint32_t)at.slot[g] * k_row + k_off + s * 64);
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int s = 0; s < LINES; ++s)
+            r.k[g][p][s] = __builtin_nontemporal_load((const bf16x8_v*)(
+                kp + (uint64_t)(uint32_t)at.slot[g] * k_row + p * 8 * k_row + k_off + s * 128));
 #pragma unroll
       for (int n = 0; n < NV; ++n)
         r.v[n] = __builtin_nontemporal_load((const bf16x8_v*)(
@@ -240,11 +250,14 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
       if (lane < KB) slots[wid][lane] = table[page] * a.kv_block + k - page * a.kv_block;
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        const char* kr = kp + (uint64_t)(uint32_t)slots[wid][g * 16 + c] * k_row + j * 16;
+      for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) r.k[g][s] = *(const bf16x8_v*)(kr + s * 64);
-      }
+        for (int p = 0; p < 2; ++p) {
+          const uint32_t slot = slots[wid][g * 16 + p * 8 + c8];
+          const char* kr = kp + (uint64_t)slot * k_row + half * 64 + j * 16;
+#pragma unroll
+          for (int s = 0; s < LINES; ++s) r.k[g][p][s] = *(const bf16x8_v*)(kr + s * 128);
+        }
 #pragma unroll
       for (int n = 0; n < NV; ++n)
         r.v[n] = *(const bf16x8_v*)(vp + (uint64_t)(uint32_t)slots[wid][n * KPL + kl] * v_row + el * 16);
@@ -260,11 +273,12 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   }
 
   // the heads' queries as columns, 8 dims a lane and step
-  const int head = h0 + min(c, heads - 1);
-  bf16x8_v q[STEPS];
+  const int head = h0 + min(c8, heads - 1);
+  bf16x8_v q[LINES];
 #pragma unroll
-  for (int s = 0; s < STEPS; ++s)
-    q[s] = *(const bf16x8_v*)((const bf16_t*)a.q + seq * a.q_stride + (int64_t)head * D + s * 32 + j * 8);
+  for (int s = 0; s < LINES; ++s)
+    q[s] = *(const bf16x8_v*)((const bf16_t*)a.q + seq * a.q_stride + (int64_t)head * D + s * 64 +
+                              half * 32 + j * 8);
   // scores in the exp2 domain: a factor, or c1 - 2 c1 / (exp2(c3 s) + 1)
   const float c1 = a.cap * LOG2E;
   const float mul = a.cap > 0.f ? 2.f * LOG2E * a.scale / a.cap : a.scale * LOG2E;
@@ -279,12 +293,25 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   auto work = [&](int i, Rows& r) {
     const int key0 = blocks.key(i);
     auto hidden = [&](int key) { return (key > pos) | ((key < lo) & (key >= a.keep)); };
-    f32x4_v s[2] = {};
+    f32x4_v halves[2][2] = {}, s[2];
 #pragma unroll
-    for (int st = 0; st < STEPS; ++st)
+    for (int st = 0; st < LINES; ++st)
 #pragma unroll
       for (int g = 0; g < 2; ++g)
-        s[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.k[g][st], q[st], s[g], 0, 0, 0);
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          halves[g][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.k[g][p][st], q[st],
+                                                                 halves[g][p], 0, 0, 0);
+    // lanes of columns below 8: 4 keys of their row group, as of a product of 16 keys
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto of = __builtin_amdgcn_permlane32_swap(__float_as_int(halves[g][0][e]),
+                                                         __float_as_int(halves[g][1][e]), false, false);
+        const int upper = __builtin_amdgcn_update_dpp(0, of[1], 0x128, 0xf, 0xf, false);  // row_ror:8
+        s[g][e] = __int_as_float(of[0]) + __int_as_float(upper);
+      }
     float w[8], mt = NEG;
     const bool edge = key0 + KB - 1 > pos || (key0 < lo && key0 + KB > a.keep);
     const bool near = bias && pos - (key0 + KB - 1) < far;
@@ -308,7 +335,7 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
       for (int e = 0; e < 8; ++e) w[e] = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-w[e]));
     } else {
       mt = max_with<32>(max_with<16>(mt));
-      if (__any(mt > m)) {
+      if (__any(c < 8 && mt > m)) {
         const float up = fmaxf(m, mt), alpha = __builtin_amdgcn_exp2f(m - up);
         m = up;
         l *= alpha;
