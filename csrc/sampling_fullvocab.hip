@@ -1021,7 +1021,7 @@ extern "C" int sample_fullvocab_chunks(int B, int V) {
   if (V < SPLIT_VOCAB || (B == 1 && V < 48000)) return 0;
   const double whole = (B + 255) / 256 * (28 + 0.95e-3 * V);
   const double split = 34 + 1.9e-4 * V + B * (0.09 + 2.3e-6 * V);
-  if (whole <= split) return 0;
+  if (whole <= 1.08 * split) return 0;  // the launches cost rows that are all greedy more
   if (B <= 16) return V >= 100000 ? 32 : 16;
   return B <= 64 && V >= 48000 ? 16 : 8;
 }
