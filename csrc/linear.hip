@@ -126,12 +126,11 @@ static void launch(const LinearArgs& a, int splits, hipStream_t stream) {
   const int total = g.tiles_m * g.tiles_n * g.splits, fit = CUS * (LDS_OF_A_CU / LDS);
   const int workgroups = total < fit ? total : fit;
   // One tile of rows reads the weights once: past the caches, us: 13 x 28672 x 4096 SwiGLU 48.6 to
-  // 44.3, 13 x 12288 x 4096 22.5 to 20.9, 61 x 128256 x 4096 209 to 193.  Weights of 33 MB are not
-  // worth it, 13 x 2048 x 8192 12.9 and 13.9, nor are those up to 90 MB, which a looped model finds in
-  // the memory-side cache again: 40 x 20096 x 2048 there 22.1 and 24.9, from memory 2 to 4% faster.
-  const bool once = g.tiles_m == 1 && (int64_t)a.N * a.K >= 48 << 20;
+  // 44.3, 13 x 12288 x 4096 22.5 to 20.9, 61 x 128256 x 4096 209 to 193, 13 x 17792 x 2048 19.4 to
+  // 18.6; weights of 33 MB are not worth it, 13 x 2048 x 8192 12.9 and 13.9
+  const bool once = g.tiles_m == 1 && (int64_t)a.N * a.K >= 32 << 20;
   auto kernel = once ? linear_kernel<FN, FM, WS, XS, UNIT, true>
-                     : linear_kernel<FN, FM, WS, XS, UNIT, false>;
+                               : linear_kernel<FN, FM, WS, XS, UNIT, false>;
   kernel<<<dim3(workgroups), 256, LDS, stream>>>(a, g);
 }
 
