@@ -117,11 +117,32 @@ def _recorded(*ts) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts)
 
 
+def _whole(t) -> bool:
+    """No subclass, which may have a product of its own."""
+    return type(t) in (torch.Tensor, torch.nn.Parameter)
+
+
+def _followed() -> bool:
+    """Whether something follows the library's calls, which kernels of our own are not seen by:
+    transforms, forward-mode derivatives, dispatch modes, a trace, a compiler, autocast."""
+    return (
+        torch.compiler.is_compiling()
+        or torch._C._functorch.peek_interpreter_stack() is not None
+        or torch.autograd.forward_ad._current_level >= 0
+        or torch._C._len_torch_dispatch_stack() > 0
+        or torch._C._get_tracing_state() is not None
+        or torch.is_autocast_enabled("cuda")
+    )
+
+
 def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
     """Whether csrc/step_linear.hip takes x w^T: what it can, at the sizes at which it pays.
-    It has no derivative: what autograd records is left to the library."""
+    It has no derivative: what autograd records or others follow is left to the library."""
     return (
         0 < x.shape[0] <= 4
+        and _whole(x)
+        and _whole(w)
+        and not _followed()
         and _rows(x)
         and _rows(w)
         and x.device == w.device
@@ -135,8 +156,8 @@ def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
         )
         and (
             bias is None
-            or bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
-            and bias.shape == w.shape[:1]
+            or _whole(bias) and bias.is_cuda and bias.dtype == torch.bfloat16
+            and bias.is_contiguous() and bias.shape == w.shape[:1]
         )
         and not _recorded(x, w, bias)
     )
@@ -169,17 +190,6 @@ def _many_rows(x, w, bias=None, glu: bool = False, out=None) -> bool:
     def below_2gib(t):
         return (t.shape[0] - 1) * t.stride(0) + t.shape[1] < 1 << 30
 
-    def whole(t):
-        return type(t) in (torch.Tensor, torch.nn.Parameter)
-
-    def seen():  # by transforms, forward-mode derivatives, dispatch modes or a trace
-        return (
-            torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._get_tracing_state() is not None
-        )
-
     return (
         x.dim() == 2
         and w.dim() == 2
@@ -187,9 +197,9 @@ def _many_rows(x, w, bias=None, glu: bool = False, out=None) -> bool:
         and w.shape[1] % 64 == 0
         and w.shape[0] % (16 if glu else 8) == 0
         and _many_rows_pay(x.shape[0], w.shape[0], w.shape[1], glu)
-        and whole(x)
-        and whole(w)
-        and not seen()
+        and _whole(x)
+        and _whole(w)
+        and not _followed()
         and _rows(x)
         and _rows(w)
         and x.device == w.device
@@ -198,7 +208,7 @@ def _many_rows(x, w, bias=None, glu: bool = False, out=None) -> bool:
         and (out is None or _rows(out))
         and (
             bias is None
-            or whole(bias) and bias.device == x.device and bias.dtype == torch.bfloat16
+            or _whole(bias) and bias.device == x.device and bias.dtype == torch.bfloat16
             and bias.is_contiguous() and bias.shape == w.shape[:1] and bias.data_ptr() % 16 == 0
         )
         and not _recorded(x, w, bias)

@@ -2,6 +2,7 @@
 and which calls its rule takes."""
 import pytest
 import torch
+from torch.utils.flop_counter import FlopCounterMode
 
 from agentcontrolplane_amd import ops
 from agentcontrolplane_amd.engine.config import ClampedGluSpec
@@ -120,6 +121,32 @@ def test_linear_leaves_other_forms():
     w.requires_grad_()
     ops.step_linear(x, w).float().sum().backward()
     assert w.grad is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 4096, 14336), (4, 6144, 4096), (2, 2048, 64), (64, 2048, 1024)])
+def test_what_follows_the_library_sees_products(m, n, k):
+    """Forward-mode derivatives, vmap, traces, dispatch modes and autocast, of few rows and many."""
+    x, w = operands(m, n, k, m)
+    lin = torch.nn.functional.linear
+    assert ops._few_rows(x, w) if m <= 4 else ops._many_rows(x, w)
+    ones = torch.ones_like(x)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, ones)
+        tangent = torch.autograd.forward_ad.unpack_dual(ops.step_linear(dual, w)).tangent
+        assert tangent is not None and torch.equal(tangent, lin(ones, w))
+    assert torch.equal(torch.func.jvp(lambda t: ops.step_linear(t, w), (x,), (ones,))[1],
+                       lin(ones, w))
+    each = torch.func.vmap(lambda t: ops.step_linear(t, w))(torch.stack([x, x + 1]))
+    assert each.shape == (2, m, n)
+    traced = torch.jit.trace(lambda t: ops.step_linear(t, w), (x,), check_trace=False)
+    assert torch.equal(traced(ones), lin(ones, w))
+    with FlopCounterMode(display=False) as flops:
+        ops.step_linear(x, w)
+    assert flops.get_total_flops() == 2 * m * n * k
+    with torch.autocast("cuda", torch.float16):
+        y, want = ops.step_linear(x, w), lin(x, w)
+    assert y.dtype == torch.float16 and torch.equal(y, want)
 
 
 def test_rule_of_many_rows():
