@@ -67,38 +67,35 @@ def linear(x, w, bias=None):
 
 
 def _few_rows_pay(m: int, outs: int, k: int, glu: bool) -> bool:
-    """Whether csrc/step_linear.hip was the faster one for m rows, outs outputs (of a GLU: pairs)
-    and k inner elements while it loaded half lines; _whole_lines_pay() has what came to it since.
-    The GEMM library (with a pass of its own for the GLU) is in brackets, us.  Four rows then: 4096
-    x 4096 9 (16), 20048 x 2048 21 (50), 3584 x 3584 9 (12), pairs of 14336 x 4096 56 (57) and of 11008
-    x 4096 43 (53), 1024 x 4608 10 (17); not 65536 x 1024 33 (28), 16 x 5120 9 (6), 64 x 8160 13 (13),
-    256 x 8064 14 (13).  Eight rows: 28672 x 4096 54 (53)."""
+    """Whether csrc/step_linear.hip is the faster one for m rows, outs outputs (of a GLU: pairs)
+    and k inner elements; the GEMM library (with a pass of its own for the GLU) is in brackets, us
+    of every weight from memory.  Up to 4096 elements at nearly all sizes: one row 4096 x 4096 8.1
+    (15), 20048 x 2048 16 (49), four rows 6144 x 4096 13.6 (15.1), pairs of 14336 x 4096 41 (64), but
+    short rows of many outputs not, 65536 x 1024 30 (27).  Above that not
+    where few outputs are long sums, 512 x 14336 17 (13), 16 x 5120 9 (7.5), pairs of 2048 x 7168 19.5
+    (17.1), nor between one and two workgroups a CU, four rows 4608 x 4608 13.7 (12.2), 6144 x 7168
+    20.3 (19.1), pairs of 5632 x 14336 68 (63), where the second round is not full; rows that are no
+    multiples of 512 are the library's slow ones, four rows 6144 x 8064 22 (29), pairs of 2048 x
+    11008 23 (37)."""
     if m > 4:
         return False
-    if k < 2048:
+    if k < 1536:
         return outs <= 28672
-    if k == 2048:
-        return outs <= 51200
-    if k < 4096:
-        return outs <= 4096
-    if k == 4096:
-        return outs <= 65536 and (m <= 2 or glu or not 4096 < outs <= 8192)
+    if k <= 4096:
+        return True
+    if glu and k <= 5120:
+        return outs >= 64
+    if glu:
+        return (
+            (k <= 6144 or 8192 < k <= 11008) and outs >= 2048
+            or 7680 < k < 8192 and (outs <= 64 or 512 <= outs)
+            or outs >= 4096 and not (k > 11008 and 4096 < outs < 8192)
+        )
+    if 4096 < outs < 8192:
+        return outs >= 6144 and (m == 1 or k % 512 > 0)
     if k <= 5120:
-        return 64 <= outs <= 2048
-    return 7680 < k < 8192 and (outs <= 64 or 512 <= outs <= 4096)
-
-
-def _whole_lines_pay(m: int, outs: int, k: int, glu: bool) -> bool:
-    """Sizes beyond _few_rows_pay() at which csrc/step_linear.hip is the faster one since its loads
-    are whole lines; the GEMM library (with a pass of its own for the GLU) is in brackets, us.
-    One row: 4096 x 14336 22 (27), 128256 x 4096 153 (185), pairs of 18944 x 3584 45 (58) and of
-    28672 x 8192 142 (186), 65536 x 1536 34 (40), 4096 x 7168 12.3 (14.9), 32000 x 5120 52 (64), 2048
-    x 5632 8.9 (10.3); four rows at 6144 x 4096 13.4 (14.8).  Not for short rows, 65536 x 1024 30
-    (27), long ones of few outputs, 512 x 14336 17 (13), and between one and two workgroups a
-    CU, 5120 x 5120 14.9 (13.9), 5120 x 13824 34 (29)."""
-    if m > 4 or k < 1536 or outs < 2048 or outs * k < 10 << 20:
-        return False
-    return k < 5120 or glu or not 4096 < outs < 6144
+        return outs >= 64
+    return outs >= 2048 or 7680 < k < 8192 and (outs <= 64 or 512 <= outs)
 
 
 def _rows(t) -> bool:
@@ -150,10 +147,7 @@ def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
         and w.shape[0] > 0
         and w.shape[1] > 0
         and w.shape[1] % 32 == 0
-        and any(
-            pay(x.shape[0], w.shape[0] >> glu, w.shape[1], glu)
-            for pay in (_few_rows_pay, _whole_lines_pay)
-        )
+        and _few_rows_pay(x.shape[0], w.shape[0] >> glu, w.shape[1], glu)
         and (
             bias is None
             or _whole(bias) and bias.is_cuda and bias.dtype == torch.bfloat16
