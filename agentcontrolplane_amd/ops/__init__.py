@@ -157,27 +157,40 @@ def _few_rows(x, w, bias=None, glu: bool = False) -> bool:
     )
 
 
-def _many_rows_pay(m: int, n: int, k: int, glu: bool) -> bool:
+def _many_rows_pay(m: int, n: int, k: int, glu: bool, adds: bool = False) -> bool:
     """Whether csrc/linear.hip is the faster one for m rows, n outputs (of a GLU: gates and ups)
-    and k inner elements; the GEMM library (with a pass of its own for the GLU) is in brackets,
-    us.  Up to about 2000 rows at nearly all sizes: 8 x 22016 x 4096 GLU 40 (53), 64 x 4096 x
-    14336 30 (53), 192 x 4096 x 4096 20 (33), 512 x 6288 x 2048 19 (22), 1739 x 4096 x 11008 140
-    (166), and by a few percent not: 16 x 3072 x 768 5.6 (5.3), 96 x 12288 x 4096 36 (31).  Small
-    weights are the launch, whoever's it is.  Beyond that the library is 2 to 7% ahead where
-    256 x 256 tiles fill their last round, 5000 x 6144 x 4096 194 (188), 7664 x 2048 x 8192 185
-    (172), 8131 x 4096 x 4096 185 (176), but not for the GLU, 7664 x 28672 x 4096 1296 (1458),
+    and k inner elements, where ``adds``: what reads it adds up its parts, which saves a launch of
+    4.3 us.  The GEMM library (with a pass of its own for the GLU) is in brackets, us of every
+    weight from memory.  Up to about 2000 rows at most sizes: 8 x 22016 x 4096 GLU 41 (59), 64 x
+    4096 x 14336 40 (54), 192 x 4096 x 4096 20 (30), 512 x 6288 x 2048 25 (28), 1739 x 4096 x 11008 138
+    (165).  Without ``adds`` not: up to 32 rows of medium weights, 8 x 6144 x 4096 17.8 (14.9), 16 x 4096 x
+    8192 19.9 (16.3), or very large ones, 24 x 128256 x 4096 195 (185), 8 x 2048 x 8192 14.1 (12.8); tiles that
+    leave half of the CUs idle, 61 x 4096 x 4096 17.1 (13.7), 80 x 2048 x 4096 12.8 (11.2); weights
+    that two tiles of rows read, 96 x 12288 x 4096 36 (30).  The library has other sizes of its own
+    beside slow ones, 190 x 6288 x 2048 18.2 (16.2), 160 x 6288 x 2048 17.7 (20.0): not told apart.  From 1024
+    rows on (2048 with a GLU or ``adds``) it is 2 to 9% ahead where
+    256 x 256 tiles fill their last round, 1400 x 32000 x 4096 287 (273), 5000 x 6144 x 4096 194 (188),
+    7664 x 2048 x 8192 185 (172), 8131 x 4096 x 4096 185 (176), but not for the GLU, 7664 x 28672 x 4096 1296 (1458),
     for outputs that are no whole tiles, 7664 x 17744 x 2048 437 (494), and for rows that
     together are beyond the memory-side cache, 7664 x 4096 x 14336 630 (995); with a last
     round that is not full it is slower, 5000 x 4096 x 4096 132 (142), 10000 x 4096 x 4096 251 (361)."""
     if m <= 4 or n * k < 1 << 21:
         return False
-    if m < 2048 or glu or n % 256 or m * k >= 100 << 20:
+    plain = not (glu or adds)
+    if plain and m <= 32:
+        medium = 4096 <= k <= 8192 and n <= 8192 and n * k >= 24 << 20
+        return not (medium or n * k >= 256 << 20 or (m <= 16 and k >= 4 * n))
+    if plain and 3584 <= k < 8192 and -(-m // 32) * n <= 8192:
+        return False
+    if plain and k >= 4096 and 64 < m <= 128 and 10240 < n < 16384:
+        return False
+    if m < (1024 if plain else 2048) or glu or n % 256 or m * k >= 100 << 20:
         return True
     tiles = -(-m // 256) * (n // 256)
     return tiles < 0.93 * 256 * -(-tiles // 256)
 
 
-def _many_rows(x, w, bias=None, glu: bool = False, out=None) -> bool:
+def _many_rows(x, w, bias=None, glu: bool = False, out=None, adds: bool = False) -> bool:
     """Whether csrc/linear.hip takes x w^T: what it can, at the sizes at which it pays.  It has
     no derivative and is not seen by what follows the library's calls: that is left to it."""
 
@@ -190,7 +203,7 @@ def _many_rows(x, w, bias=None, glu: bool = False, out=None) -> bool:
         and x.shape[1] == w.shape[1]
         and w.shape[1] % 64 == 0
         and w.shape[0] % (16 if glu else 8) == 0
-        and _many_rows_pay(x.shape[0], w.shape[0], w.shape[1], glu)
+        and _many_rows_pay(x.shape[0], w.shape[0], w.shape[1], glu, adds)
         and _whole(x)
         and _whole(w)
         and not _followed()
@@ -242,7 +255,7 @@ def step_linear_add_rmsnorm(x, w, residual, weight, eps: float = 1e-5):
     """fused_add_rmsnorm(step_linear(x, w), residual, weight, eps); a product in parts leaves
     their sum to the norm's pass."""
     if (
-        _many_rows(x, w)
+        _many_rows(x, w, adds=True)
         and w.shape[0] <= _hip()._C.ADD_RMSNORM_MOST
         and all(
             t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
@@ -263,7 +276,7 @@ def step_linear_rope_and_cache(x, w, heads: int, positions, slot_mapping, k_cach
     kv, d = k_cache.shape[-2:]
     caches = (positions, slot_mapping, k_cache, v_cache, cos_sin)
     if (
-        _many_rows(x, w)
+        _many_rows(x, w, adds=True)
         and d % 128 == 0
         and w.shape[0] == (heads + 2 * kv) * d
         and k_cache.shape == v_cache.shape
