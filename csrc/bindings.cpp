@@ -336,12 +336,23 @@ static torch::Tensor linear_parts(torch::Tensor x, torch::Tensor w, int64_t tile
   return out;
 }
 
-// C[M,N] = A[M,K] @ B[N,K]^T on the largest tiles
+// C[M,N] = A[M,K] @ B[N,K]^T on the largest tiles, in blocks of operands below 2 GiB
 static void gemm_bf16(torch::Tensor C, torch::Tensor A, torch::Tensor B) {
   CHECK_CONT(A); CHECK_CONT(B); CHECK_CONT(C);
-  TORCH_CHECK(A.size(1) % 128 == 0, "gemm_bf16 requires K % 128 == 0");
-  TORCH_CHECK(B.size(0) % 256 == 0, "gemm_bf16 requires N % 256 == 0");
-  linear(C, A, B, c10::nullopt, "plain", 0, 0, 0, 0, 0, 1);
+  TORCH_CHECK(A.dim() == 2 && B.dim() == 2 && C.dim() == 2);
+  const int64_t M = A.size(0), N = B.size(0), K = A.size(1);
+  TORCH_CHECK(B.size(1) == K && C.size(0) == M && C.size(1) == N, "gemm_bf16 shape mismatch");
+  TORCH_CHECK(K > 0 && K % 128 == 0, "gemm_bf16 requires K % 128 == 0");
+  TORCH_CHECK(N % 256 == 0, "gemm_bf16 requires N % 256 == 0");
+  for (torch::Tensor* t : {&A, &B})
+    if ((uintptr_t)t->data_ptr() % 16) *t = t->clone();
+  const int64_t most = std::max<int64_t>(256, ((1ll << 30) - 1) / K / 256 * 256);  // rows
+  for (int64_t m = 0; m < M; m += most)
+    for (int64_t n = 0; n < N; n += most) {
+      const int64_t rows = std::min(most, M - m), outs = std::min(most, N - n);
+      linear(C.narrow(0, m, rows).narrow(1, n, outs), A.narrow(0, m, rows), B.narrow(0, n, outs),
+             c10::nullopt, "plain", 0, 0, 0, 0, 0, 1);
+    }
 }
 
 static torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b) {

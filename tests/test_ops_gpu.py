@@ -338,6 +338,27 @@ def test_prefill_attn_multi_seq(impl, monkeypatch):
 
 
 @requires_gpu
+@pytest.mark.parametrize("m,n,k,at", [
+    (75000, 256, 14336, (0, 74751, 74752, 74999)), (3, 152064, 8192, (0, 130815, 130816, 152063)),
+    (0, 256, 128, ()), (5, 256, 128, (0, 4)),
+])
+def test_linear_of_large_operands(m, n, k, at, monkeypatch):
+    """The threshold for the own kernel's rows takes operands of 2 GiB and more, in blocks, and
+    rows of no 16-byte units: rows and outputs at the blocks' edges against double precision."""
+    monkeypatch.setattr(ops, "_GEMM_MIN_M", 0)
+    gen = torch.Generator("cuda").manual_seed(k)
+    x = torch.empty(m * k + 4, device="cuda", dtype=torch.bfloat16).normal_(generator=gen)
+    w = torch.empty(n, k, device="cuda", dtype=torch.bfloat16).normal_(generator=gen)
+    x = x[4:].view(m, k) if m == 5 else x[:-4].view(m, k)
+    got = ops.linear(x, w)
+    assert got.shape == (m, n)
+    rows, outs = (slice(None), list(at)) if n > 256 else (list(at), slice(None))
+    a, b = x[rows].double(), w[outs].double()
+    exact, slack = a @ b.T, k * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    assert ((got[rows][:, outs].double() - exact).abs() <= 2.0 ** -8 * exact.abs() + slack).all()
+
+
+@requires_gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("V", [513, 1023, 16385, 50257, 128256, 262144])
 def test_fullvocab_draws_lie_in_the_kept_cdf(V, dtype):
@@ -696,6 +717,27 @@ def test_gemm_bf16(m, n, k):
     # bf16 inputs, fp32 accumulation: error scales with sqrt(K)
     tol = 0.03 * math.sqrt(k)  # bf16 output rounding of ~4.5σ results
     assert maxerr(got, want) < tol, maxerr(got, want)
+
+
+@requires_gpu
+@pytest.mark.parametrize("m,n,k,at", [
+    (75000, 256, 14336, (0, 74751, 74752, 74999)), (3, 152064, 8192, (0, 130815, 130816, 152063)),
+    (0, 256, 128, ()), (5, 256, 128, (0, 4)),
+])
+def test_linear_of_large_operands(m, n, k, at, monkeypatch):
+    """The threshold for the own kernel's rows takes operands of 2 GiB and more, in blocks, and
+    rows of no 16-byte units: rows and outputs at the blocks' edges against double precision."""
+    monkeypatch.setattr(ops, "_GEMM_MIN_M", 0)
+    gen = torch.Generator("cuda").manual_seed(k)
+    x = torch.empty(m * k + 4, device="cuda", dtype=torch.bfloat16).normal_(generator=gen)
+    w = torch.empty(n, k, device="cuda", dtype=torch.bfloat16).normal_(generator=gen)
+    x = x[4:].view(m, k) if m == 5 else x[:-4].view(m, k)
+    got = ops.linear(x, w)
+    assert got.shape == (m, n)
+    rows, outs = (slice(None), list(at)) if n > 256 else (list(at), slice(None))
+    a, b = x[rows].double(), w[outs].double()
+    exact, slack = a @ b.T, k * 2.0 ** -24 * (a.abs() @ b.abs().T)
+    assert ((got[rows][:, outs].double() - exact).abs() <= 2.0 ** -8 * exact.abs() + slack).all()
 
 
 @requires_gpu
