@@ -24,8 +24,8 @@ template <int UNIT>
 DEV float unit_of(const LinearArgs& a, float gate, float up) {
   gate = (float)(__bf16)gate;
   up = (float)(__bf16)up;
-  if (UNIT == LINEAR_SWIGLU) return gate * __builtin_amdgcn_rcpf(1.f + __expf(-gate)) * up;
-  return clamped_glu_f<true>(gate, up, a.limit, a.alpha, a.offset, a.cubic);
+  if (UNIT == LINEAR_SWIGLU) return gate / (1.f + __expf(-gate)) * up;
+  return clamped_glu_f(gate, up, a.limit, a.alpha, a.offset, a.cubic);
 }
 
 #ifdef __HIP_DEVICE_COMPILE__  // the host knows no buffer resources

@@ -76,6 +76,26 @@ def test_linear_gated(tile, m, n, k, splits, unit):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("unit", ["swiglu", "glu"])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_gated_unit_is_that_of_two_passes(unit, splits):
+    """Bit for bit: a unit with fewer bits than the passes apart have shows in some of a million
+    outputs.  The products' sums do not depend on the tile."""
+    hip = ops._hip()
+    x, w = operands(600, 4096, 256, 5)
+    form = (3.0, 1.702, 1.0, 0.0) if unit == "glu" else (0.0,) * 4
+    for tile in range(10):
+        y = hip.linear(x, w, tile=tile, splits=splits)
+        got = hip.linear(x, w, None, unit, form, tile=tile, splits=splits)
+        want = torch.empty_like(got)
+        if unit == "glu":
+            ops.clamped_glu(y, *form[:3], want)
+        else:
+            want = ops.swiglu(y)
+        assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [(5, 4096, 512), (100, 2048, 1024), (700, 2056, 1024),
                                    (3000, 1024, 2048)])
 def test_step_linear_takes_its_rows(m, n, k):

@@ -626,6 +626,24 @@ def test_experts(device, dtype, n, E, top, K, I, W, skew):
 
 
 @pytest.mark.gpu
+def test_experts_of_prompts_have_the_unit_of_two_passes():
+    """Bit for bit, as for products outside of the experts, where a reciprocal of one ulp less shows
+    in about one of 3 million outputs."""
+    hip, I, K = ops._hip(), 2560, 1024
+    rows, ids = 3000, torch.arange(6000, device="cuda").remainder(2).int().view(-1, 1)
+    down = torch.eye(I, dtype=torch.bfloat16, device="cuda").expand(2, I, I).contiguous()
+    for seed in range(4):
+        g = torch.Generator("cuda").manual_seed(seed)
+        h = torch.randn(len(ids), K, device="cuda", generator=g).bfloat16()
+        gate_up = (torch.randn(2, 2 * I, K, device="cuda", generator=g) * 2 * K ** -0.5).bfloat16()
+        got = ops.moe_experts(h, gate_up, down, ids, ClampedGluSpec(I, 7.0, 1.702, 1.0))
+        for e in range(2):
+            want = torch.empty(rows, I, dtype=torch.bfloat16, device="cuda")
+            ops.clamped_glu(hip.linear(h[e::2], gate_up[e], tile=0), 7.0, 1.702, 1.0, want)
+            assert torch.equal(got[e::2, 0], want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,top,E,K,I,W", [(40, 3, 96, 2048, 384, 3722),
                                            (260, 3, 96, 2048, 384, 3749)])
 def test_experts_of_large_weights(n, top, E, K, I, W):
