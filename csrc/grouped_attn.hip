@@ -21,9 +21,11 @@
 // 1 x 4002 203 -> 14; with the values' loads, whole lines each, past the caches 190 x 700 to 1300 148
 // -> 139, 61 x 310 to 4000 120 -> 112.5, and 13 x 300 to 3900 of 32 key heads 95 -> 88; with the
 // keys' loads likewise, instead of 16 rows of half a line, 137, 109 and 85, 200 x 100 to 1000 of 64
-// heads over 8 130 -> 116, but 64 x 128 16.0 -> 16.7 (two launches and their first loads, not memory).  Without the next block in
+// heads over 8 130 -> 116; 64 x 128 17.1 -> 16.5, 64 x 16 7.3 -> 7.7 (launches and their first loads, not memory).  Without the next block in
 // flight the same kernel takes 350 us at 190 x 700 to 1300; at 3 waves a SIMD the registers for
 // it are not there.
+#include <type_traits>
+
 #include "common_t.h"
 #include "grouped_attn.h"
 
@@ -210,14 +212,35 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   const int* table = a.tables + (int64_t)seq * a.max_blocks;
   const const_int* pages = (const const_int*)table;
   const int shift = __builtin_ctz(a.kv_block);
-  struct Place { int slot[2]; };  // of a block's two groups of 16 keys
+  // Sequences that begin alike hold the same pages, at the same places of their tables.  Lanes look
+  // at the next 64 sequences' page where this piece begins; a block whose pages are those of one that
+  // has it too is left in the caches, others pass by them, as do not those that another workgroup of
+  // the same key head reads.  All kept, all past, and so, us: 190 x 700 to 1300 keys of 8 heads, 608
+  // in common 107, 117, 103, none 147, 133, 134; 60 of 32 heads 121, 131, 115 and 184, 168, 167; 16
+  // heads a key head 64 x 700 to 1300 114, 121, 107.
+  const const_int* others = pages;
+  bool begins_alike = false;
+  auto look = [&](int page, int there) {
+    const uint64_t alike = __ballot(page == there && lane + 1 < a.seqs);
+    begins_alike = alike != 0;
+    int other = seq + 1 + (alike ? __builtin_ctzll(alike) : 0);
+    if (other >= a.seqs) other -= a.seqs;
+    others = (const const_int*)(a.tables + (int64_t)(begins_alike ? other : seq) * a.max_blocks);
+  };
+  struct Place {
+    int slot[2];  // of a block's two groups of 16 keys
+    bool shared;
+  };
   auto find = [&](int i) {
     Place at;
+    at.shared = begins_alike;
     const int key0 = blocks.key(i);
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       const int k = min(key0 + 16 * g, pos & ~15);
-      at.slot[g] = PAGED ? (pages[k >> shift] << shift) + (k & (a.kv_block - 1)) : 0;
+      const int page = PAGED ? pages[k >> shift] : 0;
+      if (PAGED) at.shared &= page == others[k >> shift];
+      at.slot[g] = PAGED ? (page << shift) + (k & (a.kv_block - 1)) : 0;
     }
     return at;
   };
@@ -230,20 +253,35 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   };
   const int c8 = c & 7, half = c >> 3;
   const uint32_t k_off = c8 * k_row + half * 64 + j * 16, v_off = kl * v_row + el * 16;
+  auto load_paged = [&](auto shared, const Place& at, Rows& r) {
+    auto get = [&](const char* p) {
+      if constexpr (decltype(shared)::value) return *(const bf16x8_v*)p;
+      return __builtin_nontemporal_load((const bf16x8_v*)p);
+    };
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int s = 0; s < LINES; ++s)
+          r.k[g][p][s] =
+              get(kp + (uint64_t)(uint32_t)at.slot[g] * k_row + p * 8 * k_row + k_off + s * 128);
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      r.v[n] = get(vp + (uint64_t)(uint32_t)at.slot[n * KPL / 16] * v_row + n * KPL % 16 * v_row + v_off);
+  };
   auto load = [&](int i, const Place& at, Rows& r) {
     if constexpr (PAGED) {
-#pragma unroll
-      for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-          for (int s = 0; s < LINES; ++s)
-            r.k[g][p][s] = __builtin_nontemporal_load((const bf16x8_v*)(
-                kp + (uint64_t)(uint32_t)at.slot[g] * k_row + p * 8 * k_row + k_off + s * 128));
-#pragma unroll
-      for (int n = 0; n < NV; ++n)
-        r.v[n] = __builtin_nontemporal_load((const bf16x8_v*)(
-            vp + (uint64_t)(uint32_t)at.slot[n * KPL / 16] * v_row + n * KPL % 16 * v_row + v_off));
+      // the comments keep the compiler from making one load of both kinds, which loses the hint
+      if (per > 1 || at.shared) {
+        asm volatile("; kept" ::: "memory");
+        load_paged(std::true_type(), at, r);
+        asm volatile("; kept, end" ::: "memory");
+      } else {
+        asm volatile("; past" ::: "memory");
+        load_paged(std::false_type(), at, r);
+        asm volatile("; past, end" ::: "memory");
+      }
     } else {
       const int k = min(blocks.key(i) + (lane & (KB - 1)), pos);
       const int page = k / a.kv_block;
@@ -268,7 +306,17 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   int i = nth * p.size + wid;
   Place at{};
   if (i < end) {
+    // a piece of a few blocks is over before the answer pays
+    const bool ask = PAGED && per == 1 && a.seqs > 1 && p.size > 8;
+    int there = 0;
+    const int first = min(blocks.key(nth * p.size), pos & ~15) >> shift;
+    if (ask) {
+      int other = seq + 1 + lane;
+      other -= other >= a.seqs ? a.seqs : 0;
+      there = a.tables[(int64_t)min(other, a.seqs - 1) * a.max_blocks + first];
+    }
     load(i, find(i), r0);
+    if (ask) look(pages[first], there);
     if (AHEAD && PAGED) at = find(min(i + 4, p.n - 1));
   }
 

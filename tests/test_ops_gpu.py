@@ -338,27 +338,6 @@ def test_prefill_attn_multi_seq(impl, monkeypatch):
 
 
 @requires_gpu
-@pytest.mark.parametrize("m,n,k,at", [
-    (75000, 256, 14336, (0, 74751, 74752, 74999)), (3, 152064, 8192, (0, 130815, 130816, 152063)),
-    (0, 256, 128, ()), (5, 256, 128, (0, 4)),
-])
-def test_linear_of_large_operands(m, n, k, at, monkeypatch):
-    """The threshold for the own kernel's rows takes operands of 2 GiB and more, in blocks, and
-    rows of no 16-byte units: rows and outputs at the blocks' edges against double precision."""
-    monkeypatch.setattr(ops, "_GEMM_MIN_M", 0)
-    gen = torch.Generator("cuda").manual_seed(k)
-    x = torch.empty(m * k + 4, device="cuda", dtype=torch.bfloat16).normal_(generator=gen)
-    w = torch.empty(n, k, device="cuda", dtype=torch.bfloat16).normal_(generator=gen)
-    x = x[4:].view(m, k) if m == 5 else x[:-4].view(m, k)
-    got = ops.linear(x, w)
-    assert got.shape == (m, n)
-    rows, outs = (slice(None), list(at)) if n > 256 else (list(at), slice(None))
-    a, b = x[rows].double(), w[outs].double()
-    exact, slack = a @ b.T, k * 2.0 ** -24 * (a.abs() @ b.abs().T)
-    assert ((got[rows][:, outs].double() - exact).abs() <= 2.0 ** -8 * exact.abs() + slack).all()
-
-
-@requires_gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("V", [513, 1023, 16385, 50257, 128256, 262144])
 def test_fullvocab_draws_lie_in_the_kept_cdf(V, dtype):
@@ -717,6 +696,38 @@ def test_gemm_bf16(m, n, k):
     # bf16 inputs, fp32 accumulation: error scales with sqrt(K)
     tol = 0.03 * math.sqrt(k)  # bf16 output rounding of ~4.5σ results
     assert maxerr(got, want) < tol, maxerr(got, want)
+
+
+@requires_gpu
+@pytest.mark.parametrize("block", [16, 64])
+@pytest.mark.parametrize("B,lo,hi,shared,kv", [
+    (2, 900, 1000, 640, 8), (3, 2000, 4000, 1920, 2), (70, 300, 900, 320, 8), (200, 700, 1100, 640, 8),
+    (40, 300, 1100, 64, 32),
+])
+def test_decode_over_shared_pages(B, lo, hi, shared, kv, block):
+    """Sequences that begin alike read the same pages, by other loads: as from pages of their own.
+    Two beginnings take turns, one sequence has neither."""
+    gen = torch.Generator("cuda").manual_seed(B)
+    lens = torch.randint(lo, hi + 1, (B,), generator=gen, device="cuda", dtype=torch.int32)
+    pages, head = -(-hi // block), shared // block
+    own = torch.randperm(B * pages, generator=gen, device="cuda").int().view(B, pages)
+    caches = [torch.randn(B * pages, block, kv, 128, generator=gen, device="cuda").bfloat16()
+              for _ in range(2)]
+    tables = own.clone()
+    for s in range(2, B - 1):
+        tables[s, :head] = own[s % 2, :head]
+        for cache in caches:
+            cache[own[s, :head].long()] = cache[own[s % 2, :head].long()]
+    H = min(32, 8 * kv)
+    q = torch.randn(B, H, 128, generator=gen, device="cuda").bfloat16()
+    run = hip().attention_decode_raw
+    got, want = (run(q, *caches, t, lens, 128 ** -0.5) for t in (tables, own))
+    assert torch.equal(got, want)
+    s = B // 2
+    k, v = (c[own[s].long()].flatten(0, 1)[: lens[s]].double() for c in caches)
+    k, v = (t.repeat_interleave(H // kv, 1) for t in (k, v))
+    w = torch.softmax(torch.einsum("hd,khd->hk", q[s].double(), k) * 128 ** -0.5, -1)
+    assert maxerr(got[s], torch.einsum("hk,khd->hd", w, v)) < 0.01
 
 
 @requires_gpu
