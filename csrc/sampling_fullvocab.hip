@@ -55,6 +55,9 @@ __device__ __forceinline__ float key2f(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
 }
 
+// A function that is not inlined gets a row and LDS by reference and no longer knows which memory is which:
+// its loads and atomics wait for both
+#define INLINE __device__ __forceinline__
 __device__ __forceinline__ float ldf(const float* p) { return *p; }
 __device__ __forceinline__ float ldf(const bf16_t* p) { return bf2f(*p); }
 
@@ -113,12 +116,12 @@ struct Row {
 
   // f(token, logit) for every allowed token, a thread's in rising order
   template <typename F>
-  __device__ void each(F f) const {
+  INLINE void each(F f) const {
     each(0, V, f);
   }
   // likewise of tokens i0 .. i1 - 1
   template <typename F>
-  __device__ void each(int i0, int i1, F f) const {
+  INLINE void each(int i0, int i1, F f) const {
     constexpr int N = 16 / sizeof(T), AHEAD = 4;
     auto one = [&](int i, float v) {
       if (!mask || mask[i]) f(i, v);
@@ -168,7 +171,7 @@ static_assert(OCTAVE == 64, "bucket() takes 6 bits of the mantissa");
 // The first of ``n`` (at most FIRST) buckets whose sum with those before and ``above`` reaches
 // target, and the sum before it; -1: none does.
 template <bool BY_MASS, typename S>
-__device__ int find_bucket(S& s, int n, double target, double* above) {
+INLINE int find_bucket(S& s, int n, double target, double* above) {
   constexpr int PER = S::BUCKETS;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   double w[PER], sum = 0.0;
@@ -213,7 +216,7 @@ __device__ int find_bucket(S& s, int n, double target, double* above) {
 // Splits the keys [lo, hi] among those that each_key(f) hands out until one is left: the one at
 // which the sum from the top reaches target.
 template <bool BY_MASS, typename S, typename R, typename E>
-__device__ uint32_t split_keys(S& s, const R& row, uint32_t lo, uint32_t hi,
+INLINE uint32_t split_keys(S& s, const R& row, uint32_t lo, uint32_t hi,
                                double above, double target, E each_key) {
   for (;;) {
     const uint32_t range = hi - lo;
@@ -243,7 +246,7 @@ __device__ uint32_t split_keys(S& s, const R& row, uint32_t lo, uint32_t hi,
 }
 
 template <typename S>
-__device__ double block_total(S& s, double v) {
+INLINE double block_total(S& s, double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   if ((threadIdx.x & 63) == 0) s.wave[threadIdx.x >> 6] = v;
@@ -256,7 +259,7 @@ __device__ double block_total(S& s, double v) {
 
 // The largest of the threads' logits, the lowest token among equals, whether one is odd
 template <typename S>
-__device__ void block_max(S& s, float& mx, int& best, int& odd) {
+INLINE void block_max(S& s, float& mx, int& best, int& odd) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     const float v = __shfl_xor(mx, off, 64);
@@ -284,7 +287,7 @@ __device__ void block_max(S& s, float& mx, int& best, int& odd) {
 // Histograms over m - x up to ``far``; the mass of the others: a boundary is seldom among
 // them, and their atomics take most of the time.
 template <bool BY_MASS, typename S, typename R>
-__device__ float fill(S& s, const R& row, float far) {
+INLINE float fill(S& s, const R& row, float far) {
   for (int i = threadIdx.x; i < FIRST; i += S::WG) {
     s.count[i] = 0;
     s.mass[i] = 0;
@@ -310,7 +313,7 @@ __device__ float fill(S& s, const R& row, float far) {
 // The key at which the sum from the largest logit down reaches target, which is ``part`` of all
 // weights if it is given; 0: nowhere.  ``plain``: all logits are numbers.
 template <bool BY_MASS, typename S, typename R>
-__device__ uint32_t boundary(S& s, const R& row, double target, double part, bool plain) {
+INLINE uint32_t boundary(S& s, const R& row, double target, double part, bool plain) {
   if (target <= 0.0) return f2key(row.m);  // reached before the first, which is kept all the same
   auto stream = [&](auto f) { row.each([&](int, float v) { f(f2key(v)); }); };
   if (!plain) return split_keys<BY_MASS>(s, row, 0u, 0xffffffffu, 0.0, target, stream);
@@ -377,7 +380,7 @@ struct SampleArgs {
 // compact masks: only constrained rows carry one (a dense [B,V] mask at
 // B=1k, V=128k would be 128 MB of pinned staging per step)
 template <typename T, int WG>
-__device__ Row<T, WG> row_of(const SampleArgs& a, int n) {
+INLINE Row<T, WG> row_of(const SampleArgs& a, int n) {
   const bool masked = a.mask && a.mask_map && a.mask_map[n] >= 0;
   const float temp = a.temps[n];
   return {(const T*)a.logits + (int64_t)n * a.V,
@@ -387,7 +390,7 @@ __device__ Row<T, WG> row_of(const SampleArgs& a, int n) {
 
 // ---- inverse-CDF draw in token-id order from the stripes' sums, ``mine`` of the t-th thread's
 template <typename S, typename R>
-__device__ void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin,
+INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin,
                      float mine) {
   constexpr int WG = S::WG;
   const int t = threadIdx.x, V = row.V, stride = (V + STRIPES - 1) / STRIPES;
@@ -580,7 +583,7 @@ __global__ __launch_bounds__(256) void chunk_max_kernel(const SampleArgs a, RowS
 
 // the row's largest logit, the lowest token that has it, and whether all are numbers
 template <typename R>
-__device__ bool whole_max(const RowState& state, int chunks, R& row, int* best) {
+INLINE bool whole_max(const RowState& state, int chunks, R& row, int* best) {
   float mx = -3.4e38f;
   int at = row.V, odd = 0;
   for (int i = 0; i < chunks; ++i) {
@@ -794,7 +797,7 @@ __global__ __launch_bounds__(256) void draw_kernel(const SampleArgs a, const Row
 // least one if rounding lets none do so.  A thread compares its key with all others, which takes
 // 33 ns a key; the two rounds of split_keys take about 12 us whatever the list: RANKED keys.
 template <bool BY_MASS, typename S>
-__device__ uint32_t rank_keys(S& s, int n, double above, double target) {
+INLINE uint32_t rank_keys(S& s, int n, double above, double target) {
   if (threadIdx.x == 0) s.lo = 0xffffffffu;
   __syncthreads();
   uint32_t least = 0xffffffffu, at = 0;
@@ -834,7 +837,7 @@ __device__ uint32_t rank_keys(S& s, int n, double above, double target) {
 
 // The least kept key from a row's list of at most KEYS
 template <typename S, typename R>
-__device__ uint32_t least_of_list(S& s, const RowState& state, const RowPlan& plan,
+INLINE uint32_t least_of_list(S& s, const RowState& state, const RowPlan& plan,
                                   const Wants& want, const R& row) {
   const int n = plan.n;
   for (int i = threadIdx.x; i < (n + 3) / 4 * 4; i += S::WG) {
@@ -880,9 +883,8 @@ __device__ uint32_t least_of_list(S& s, const RowState& state, const RowPlan& pl
   return max(kmin, find(std::true_type(), 0.0, target));
 }
 
-// ---- a row by one workgroup; with ``states`` the thresholds of rows in chunks, and those rows that
-// are left to it
-template <typename T, typename F>
+// ---- a row by one workgroup; of rows in CHUNKS the thresholds, and those rows that are left to it
+template <typename T, typename F, bool CHUNKS>
 __global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(const SampleArgs a,
                                                                  RowState* states) {
   constexpr int WG = F::WG, TILE = F::TILE;
@@ -891,7 +893,7 @@ __global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(const SampleArg
   const Wants want = wants_of(a, n_row);
   const int V = a.V;
   Row<T, WG> row = row_of<T, WG>(a, n_row);
-  if (states) {
+  if (CHUNKS) {
     RowState& state = states[n_row];
     const RowPlan plan = state.plan;
     if (want.greedy || plan.mode == NO_LIST) return;
@@ -995,18 +997,18 @@ static void launch(const SampleArgs& a, void* work, int chunks, hipStream_t stre
   using Small = Form<256, 16>;
   using Large = Form<1024, 64>;
   RowState* const states = (RowState*)work;
-  const bool small = a.V <= 4096 || (a.V <= 8192 && a.B > 256);
-  auto whole = small ? sample_fullvocab_kernel<T, Small> : sample_fullvocab_kernel<T, Large>;
-  const int grid = a.B * chunks, threads = small ? Small::WG : Large::WG;
+  const int grid = a.B * chunks;
   if (chunks) {
     chunk_max_kernel<T><<<grid, 256, 0, stream>>>(a, states, chunks);
     chunk_histogram_kernel<T><<<grid, 256, 0, stream>>>(a, states, chunks);
     chunk_keys_kernel<T><<<grid, 256, 0, stream>>>(a, states, chunks);
-  }
-  whole<<<a.B, threads, 0, stream>>>(a, states);
-  if (chunks) {
+    sample_fullvocab_kernel<T, Large, true><<<a.B, Large::WG, 0, stream>>>(a, states);
     chunk_sums_kernel<T><<<grid, 256, 0, stream>>>(a, states, chunks);
     draw_kernel<T><<<a.B, 256, 0, stream>>>(a, states);
+  } else if (a.V <= 4096 || (a.V <= 8192 && a.B > 256)) {
+    sample_fullvocab_kernel<T, Small, false><<<a.B, Small::WG, 0, stream>>>(a, states);
+  } else {
+    sample_fullvocab_kernel<T, Large, false><<<a.B, Large::WG, 0, stream>>>(a, states);
   }
 }
 
