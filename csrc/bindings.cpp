@@ -402,7 +402,7 @@ static void sample_fullvocab(torch::Tensor out, torch::Tensor logits,
     mapptr = mask_map->data_ptr<int32_t>();
   }
   const int n = chunks < 0 ? sample_fullvocab_chunks(B, V) : (int)chunks;
-  TORCH_CHECK(n == 0 || n == 8 || n == 16 || n == 32, "chunks");
+  TORCH_CHECK(n == 0 || n == 16 || n == 32, "chunks");
   torch::Tensor work;
   if (n) work = torch::empty({sample_fullvocab_bytes(B, n)}, logits.options().dtype(at::kByte));
   launch_sample_fullvocab(out.data_ptr<int64_t>(), logits.data_ptr(), bf16,
@@ -1305,6 +1305,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("delta_prompts", &delta_prompts);
   m.def("delta_step", &delta_step);
   m.def("sample", &sample);
+  m.def("sample_fullvocab_chunks", &sample_fullvocab_chunks);
   m.def("sample_fullvocab", &sample_fullvocab, py::arg("out"), py::arg("logits"),
         py::arg("temps"), py::arg("top_ks"), py::arg("top_ps"), py::arg("uniforms"),
         py::arg("mask"), py::arg("mask_map"), py::arg("chunks") = -1);

@@ -1,6 +1,6 @@
 // Full-vocabulary token sampling (gfx950): temperature → optional grammar
 // mask → exact top-k → top-p (nucleus) → inverse-CDF draw in token-id
-// order; one workgroup per row, or several for large vocabularies ("rows in chunks" below), up to
+// order; one workgroup per row, or several for few rows of large vocabularies ("rows in chunks"), up to
 // 2^18 tokens (Llama-3: 128256).
 //
 // The ≤512-entry LDS bitonic sampler (sampling.hip) covers the byte
@@ -18,11 +18,10 @@
 // weights of 64 tokens of every stripe are made at a time by all threads and added up by one
 // thread a stripe, so that the order of the sums does not depend on the threads.
 //
-// A workgroup a row is bound by its passes over the row: 20 us for the largest logit, 15 for the histogram of a top-k
-// and 62 for that of a top-p (30 of it weights, 32 atomics), 16 to gather the bucket, 15 for the
-// draw's sums, where 190 rows of 128256 in fp32 come from the memory-side cache.  Whole calls
-// with other logits each time: 34 us greedy, 67 plain, 100 top-k, 153 top-p, 193 both (in chunks on
-// another card 36, 71, 109, 127 and 116, where these took 24, 53, 120, 167 and 236); before 315,
+// A workgroup a row is bound by its passes over the row.  190 rows of 128256 in fp32, other logits each
+// time, whole calls: 25 us greedy, 48 plain, 79 top-k, 95 top-p, 135 both (26, 58, 97, 168 and 238 with
+// calls of functions, which take a row and LDS by reference: their loads and atomics then go by
+// unknown memory and wait for both kinds); before 315,
 // 428, 1135, 1305 and 1978 (thresholds by three histograms of key bits, whose few buckets met
 // nearly all atomics, walked by one thread; draws by strides of a thread).  Floating masses
 // instead of whole ones in the histogram took as long, a shared list of the bucket 25 us more.
@@ -55,8 +54,6 @@ __device__ __forceinline__ float key2f(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
 }
 
-// A function that is not inlined gets a row and LDS by reference and no longer knows which memory is which:
-// its loads and atomics wait for both
 #define INLINE __device__ __forceinline__
 __device__ __forceinline__ float ldf(const float* p) { return *p; }
 __device__ __forceinline__ float ldf(const bf16_t* p) { return bf2f(*p); }
@@ -475,8 +472,8 @@ INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t km
 
 // ---- rows in chunks
 //
-// Large vocabularies: a row's 256 stripes go to ``chunks`` workgroups in launches of their own, so
-// that the rows whose thresholds take longest, or the few that there are, have the whole chip.
+// Few rows of large vocabularies: a row's 256 stripes go to ``chunks`` workgroups in launches of their
+// own, so that they have the whole chip.
 //   1 the largest logit of a chunk
 //   2 a chunk's histograms, added to the row's
 //   3 the boundary's bucket from those, by every workgroup; its keys into the row's list
@@ -486,9 +483,9 @@ INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t km
 // All that workgroups share are whole numbers or added up in a fixed order, so that they agree.  A
 // row that this does not fit (logits that are no numbers, a boundary beyond the head or among more
 // keys than the list has) is taken as a whole in launch 4.
-// 190 x 128256 of plain, top-k, top-p and greedy rows in turns 120 us (by a workgroup a row 162):
-// largest logits 21, histograms 20, keys 23, thresholds 18, sums 27, draws 11.
-#define SPLIT_VOCAB 20000
+// 16 x 128256 of plain, top-k, top-p and greedy rows in turns 63 us, by a workgroup a row 84.
+#define SPLIT_VOCAB 100000
+#define LEAST_CHUNKS 16
 #define MOST_CHUNKS 32
 
 enum Mode { NO_LIST, BY_LIST, WHOLE };
@@ -525,7 +522,7 @@ struct ChunkShared : ChunkForm {
       uint32_t count[FIRST];
       unsigned long long mass[FIRST];
     };
-    float tile[2][STRIPES / 8][TILE + 4];
+    float tile[2][STRIPES / LEAST_CHUNKS][TILE + 4];
   };
   uint32_t keys[KEYS];
   double wave[WAVES];
@@ -735,7 +732,7 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, Row
   const uint32_t kmin = plan.kmin;
   // stripes' weights by all threads, 64 tokens of each at a time, added up by a thread a stripe
   const int r = t / TILE, col = t % TILE;
-  constexpr int ROWS = 256 / TILE, MOST = STRIPES / 8 / ROWS;
+  constexpr int ROWS = 256 / TILE, MOST = STRIPES / LEAST_CHUNKS / ROWS;
   const float least = key2f(kmin);
   const bool by_value = kmin == 0 || (least == least && least != 0.f);
   const float from = kmin == 0 ? -INFINITY : least;
@@ -1012,20 +1009,14 @@ static void launch(const SampleArgs& a, void* work, int chunks, hipStream_t stre
   }
 }
 
-// Chunks of a row, the more of them the fewer the rows and the more tokens; 0 where a workgroup a row
-// is expected to be faster, in us by what rows of all kinds took: rounds of CUs there, six launches
-// and the chip's time here.  By a workgroup a row and in chunks, us: 24000 tokens 2 rows 38 and
-// 37, 8 49 and 41, 100 51 and 50, 190 52 and 59, 300 101 and 83, 512 108 and 112; 48000 8 69 and
-// 45, 190 79 and 71; 128256 8 137 and 59, 100 158 and 92, 190 162 and 120, 512 335 and 258.  One row
-// alone has no other to wait for: 32000 a plain one 20 and 24, top-k 39 and 36, top-p 50 and 37.
-// Rows that are all greedy wait for the launches: 190 x 128256 24 and 36, 512 60 and 79.
+// Chunks of a row, the more of them the fewer the rows; 0: a workgroup a row, which is faster from 100 rows
+// on, for smaller vocabularies, and for greedy rows that would wait for the launches.  By a workgroup a
+// row and in chunks, us, greedy, plain, top-p and all kinds in turns: 128256 tokens 1 row 19 38 81 38 and
+// 17 29 54 29, 16 20 41 85 84 and 19 34 63 63, 64 22 42 89 88 and 24 42 78 77, 100 23 44 90 89 and 27 51
+// 95 94, 190 25 48 94 91 and 38 73 129 123; 100000 16 17 42 79 78 and 19 33 61 62; 65536 8 12 25 53 52
+// and 17 27 49 50; 50257 8 13 30 60 59 and 18 28 47 48; 32000 8 8 20 39 39 and 15 24 40 41.
 extern "C" int sample_fullvocab_chunks(int B, int V) {
-  if (V < SPLIT_VOCAB || (B == 1 && V < 48000)) return 0;
-  const double whole = (B + 255) / 256 * (28 + 0.95e-3 * V);
-  const double split = 34 + 1.9e-4 * V + B * (0.09 + 2.3e-6 * V);
-  if (whole <= 1.08 * split) return 0;  // the launches cost rows that are all greedy more
-  if (B <= 16) return V >= 100000 ? 32 : 16;
-  return B <= 64 && V >= 48000 ? 16 : 8;
+  return V < SPLIT_VOCAB || B > 64 ? 0 : B <= 16 ? 32 : 16;
 }
 
 // What sample_fullvocab with that many chunks works in

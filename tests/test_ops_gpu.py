@@ -751,6 +751,16 @@ def test_linear_of_large_operands(m, n, k, at, monkeypatch):
     assert ((got[rows][:, outs].double() - exact).abs() <= 2.0 ** -8 * exact.abs() + slack).all()
 
 
+def test_sample_fullvocab_takes_chunks_where_no_kind_of_row_waits():
+    """Rows that are all greedy or plain were 20 to 50% slower in chunks at the last five sizes."""
+    from agentcontrolplane_amd import _C
+
+    chunks = _C.sample_fullvocab_chunks
+    assert chunks(1, 128256) == 32 and chunks(16, 100000) == 32 and chunks(64, 152064) == 16
+    for rows, vocab in [(65, 128256), (190, 128256), (512, 152064), (8, 65536), (16, 32000)]:
+        assert chunks(rows, vocab) == 0
+
+
 @requires_gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("V", [513, 4099, 16384, 32000, 50257, 128256, 152064])
@@ -782,11 +792,11 @@ def test_sample_fullvocab_chunks(V, dtype):
     x = x.to(dtype)
     for m, to in ((None, None), (mask, which)):
         outs = []
-        for chunks in (0, 8, 16, 32):
+        for chunks in (0, 16, 32):
             out = torch.full((B,), -1, device="cuda")
             C.sample_fullvocab(out, x, temps, ks, ps, u, m, to, chunks)
             outs.append(out.tolist())
-        assert outs[0] == outs[1] == outs[2] == outs[3]
+        assert outs[0] == outs[1] == outs[2]
         assert all(0 <= t < V for t in outs[0])
         if m is not None:
             assert all(mask[w, t] for w, t in zip(which.tolist(), outs[0]) if w >= 0)
