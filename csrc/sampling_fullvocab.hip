@@ -506,7 +506,8 @@ __device__ __forceinline__ bool left_whole(const RowPlan& plan) {
 // A row's state between the launches
 struct RowState {
   RowPlan plan;
-  float chunk_max[MOST_CHUNKS], rest[MOST_CHUNKS];
+  double rest[MOST_CHUNKS];
+  float chunk_max[MOST_CHUNKS];
   int chunk_best[MOST_CHUNKS], chunk_odd[MOST_CHUNKS];
   float stripe[STRIPES];
   uint32_t list[KEYS];
@@ -640,7 +641,7 @@ __global__ __launch_bounds__(256) void chunk_histogram_kernel(const SampleArgs a
     if (want.by_k) atomicAdd(&s.count[b], 1u);
   });
   const double all = block_total(s, (double)rest);
-  if (threadIdx.x == 0) state.rest[c.at] = (float)all;
+  if (threadIdx.x == 0) state.rest[c.at] = all;
   __syncthreads();
   for (int i = threadIdx.x; i < FIRST; i += 256) {
     if (s.count[i]) atomicAdd(&state.count[i], s.count[i]);

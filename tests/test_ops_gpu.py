@@ -751,6 +751,34 @@ def test_linear_of_large_operands(m, n, k, at, monkeypatch):
     assert ((got[rows][:, outs].double() - exact).abs() <= 2.0 ** -8 * exact.abs() + slack).all()
 
 
+@requires_gpu
+@pytest.mark.parametrize("chunks", [16, 32])
+def test_sample_fullvocab_chunks_keep_the_tail_in_64_bits(chunks):
+    """A nucleus that reaches just past the largest logit, by what chunks' tails lose in 32 bits.
+    Tail weights are 2^-18 and, too few of them in a chunk to round up, 2^-36, so that sums of a
+    thread's tokens are exact."""
+    V, each, few = 128256, 128256 // chunks, 960 // chunks
+    log2e = torch.tensor(1.44269504, dtype=torch.float32)
+    near = torch.arange(-40, 41, dtype=torch.float32)
+
+    def logit_of(power):  # exp of it is 2^power
+        x = power / log2e * (1 + near * 2.0 ** -24)
+        return x[x * log2e == power][0].item()
+
+    x = torch.full((V,), logit_of(-18.0))
+    for c in range(chunks):
+        x[c * each + 5 : c * each + 5 + few] = logit_of(-36.0)
+    tail = (V - chunks * few - 2) * 2.0 ** -18 + chunks * few * 2.0 ** -36
+    p = torch.tensor(1 / (1 + tail + 1e-3), dtype=torch.float32)
+    x[0] = 0.0
+    x[1] = math.log(1 / p.item() + 0.7e-8 - 1 - tail)
+    one = torch.ones(1, device="cuda")
+    out = torch.zeros(1, dtype=torch.long, device="cuda")
+    hip()._C.sample_fullvocab(out, x.cuda().view(1, V), one, out.clone(), one * p.cuda(), one * 0.9999,
+                              None, None, chunks)
+    assert out.item() == 1
+
+
 def test_sample_fullvocab_takes_chunks_where_no_kind_of_row_waits():
     """Rows that are all greedy or plain were 20 to 50% slower in chunks at the last five sizes."""
     from agentcontrolplane_amd import _C
