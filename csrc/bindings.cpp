@@ -248,6 +248,12 @@ static void prefill_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
                       max_blocks, kv_block, q_stride, cur_stream());
 }
 
+// An error of the launches before it
+static void launched(const char* what) {
+  const hipError_t e = hipGetLastError();
+  TORCH_CHECK(e == hipSuccess, what, ": ", hipGetErrorString(e));
+}
+
 // The launch of x w^T by csrc/linear.hip: tile and splits from the sizes, or the given ones
 static void run_linear(const LinearArgs& a, int unit, int tile, int splits,
                        const torch::Tensor& x) {
@@ -256,6 +262,7 @@ static void run_linear(const LinearArgs& a, int unit, int tile, int splits,
   if (splits > 1)
     parts = torch::empty({(int64_t)splits * a.M * a.N}, x.options().dtype(torch::kFloat32));
   launch_linear(&a, unit, tile, splits, splits > 1 ? parts.data_ptr() : nullptr, cur_stream());
+  launched("linear");
 }
 
 // The operands of x w^T, checked
@@ -333,6 +340,7 @@ static torch::Tensor linear_parts(torch::Tensor x, torch::Tensor w, int64_t tile
   a.out = out.data_ptr();
   a.out_stride = a.N;
   launch_linear(&a, LINEAR_PARTS, t, parts, out.data_ptr(), cur_stream());
+  launched("linear_parts");
   return out;
 }
 
@@ -1146,6 +1154,7 @@ static void experts_linear(torch::Tensor out, torch::Tensor x, torch::Tensor w, 
   a.tile_expert = opt_int(tile_expert, a.tiles);
   a.tile_row = opt_int(tile_row, a.tiles);
   launch_experts_gemm(glu, &a, cur_stream());
+  launched("experts_gemm");
 }
 
 static DeltaArgs delta_args(const torch::Tensor& out, const torch::Tensor& qkv,

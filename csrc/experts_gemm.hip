@@ -14,6 +14,7 @@
 // 416, 1024 538 and 428, 2048 669 and 612, 4093 1084 and 993, 8192 2009 and 1738; 16 of 2048 x
 // 1536: 512 tokens 127 and 98, 2048 220 and 212, 4093 360 and 346, 8192 755 and 612.
 #include "experts.h"
+#include "launch.h"
 #include "linear_tile.h"
 
 #define LDS_BYTES 163840
@@ -93,12 +94,7 @@ __global__ __launch_bounds__(256, 1) void experts_gemm_kernel(const ExpertsArgs 
 
 template <bool GLU>
 static void launch(const ExpertsArgs& a, hipStream_t stream) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)experts_gemm_kernel<GLU>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-    attr_set = true;
-  }
+  allow_lds<experts_gemm_kernel<GLU>>(LDS_BYTES);
   const int per = GLU ? 128 : 256;
   const int tiles_n = (a.O + per - 1) / per;
   const int groups = (tiles_n + 4) / 5, columns = (tiles_n + groups - 1) / groups;

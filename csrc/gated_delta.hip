@@ -21,6 +21,7 @@
 // comes first.
 #include "common_t.h"
 #include "gated_delta.h"
+#include "launch.h"
 
 DEV float silu_f(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
@@ -702,12 +703,7 @@ static void launch_scan(const DeltaArgs& a, hipStream_t stream) {
   constexpr int TT = DPL <= 16 ? 16 : 256 / DPL;
   constexpr int bytes = 4 * (2 * (HEAD ? 2 : 3) * TT * 16 * DPL + 2 * TT * (16 * CPL + 4));
   static_assert(bytes <= 160 * 1024, "LDS");
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)delta_scan_kernel<T, DPL, CPL, FULL, HEAD>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    attr_set = true;
-  }
+  allow_lds<delta_scan_kernel<T, DPL, CPL, FULL, HEAD>>(bytes);
   const dim3 grid((a.V + 16 * CPL - 1) / (16 * CPL), a.H, a.seqs);
   delta_scan_kernel<T, DPL, CPL, FULL, HEAD><<<grid, 256, bytes, stream>>>(a);
 }

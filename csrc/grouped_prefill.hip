@@ -30,6 +30,7 @@
 // 15 prompts of 700 to 1400 tokens, whose half-empty diagonal tiles weigh more: 264 -> 225 us.
 #include "common_t.h"
 #include "grouped_attn.h"
+#include "launch.h"
 
 typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_v __attribute__((ext_vector_type(4)));
@@ -414,12 +415,7 @@ template <int DN, int VN, int FORM, bool PAGED>
 static void launch_paged(const GroupedArgs& a, hipStream_t stream) {
   constexpr int bytes = 2 * KT * (64 * DN + 64 * VN) * 2 + 2 * KT * 4;
   static_assert(bytes <= 160 * 1024, "LDS");
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)grouped_prefill_kernel<DN, VN, FORM, PAGED>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    attr_set = true;
-  }
+  allow_lds<grouped_prefill_kernel<DN, VN, FORM, PAGED>>(bytes);
   grouped_prefill_kernel<DN, VN, FORM, PAGED><<<a.n_tiles * a.H, 256, bytes, stream>>>(a);
 }
 

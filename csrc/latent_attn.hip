@@ -24,6 +24,7 @@
 // values only (capture-safe); lengths are read on the device.
 #include "common_t.h"
 #include "latent_attn.h"
+#include "launch.h"
 
 typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_v __attribute__((ext_vector_type(4)));
@@ -389,12 +390,7 @@ static void launch_mfma(const LatentArgs& a, int tiles, hipStream_t stream) {
   constexpr int M = 16 * MG;
   constexpr int bytes = 2 * KT * (64 * NR + ROT) * 2 + M * PPAD * 2 + M * 16 + 2 * KT * 4;
   static_assert(bytes <= 160 * 1024, "LDS");
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)latent_attn_kernel<NR, MG>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    attr_set = true;
-  }
+  allow_lds<latent_attn_kernel<NR, MG>>(bytes);
   latent_attn_kernel<NR, MG><<<dim3(tiles, a.n_split), 256, bytes, stream>>>(a);
 }
 

@@ -19,6 +19,7 @@
 // workgroups stay together so that their keys share its L2.
 #include "common_t.h"
 #include "latent_attn.h"
+#include "launch.h"
 
 typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_v __attribute__((ext_vector_type(4)));
@@ -249,12 +250,7 @@ template <int DN, int VN>
 static void launch(const LatentPrefillArgs& a, hipStream_t stream) {
   constexpr int bytes = 2 * KT * (64 * DN + ROT + 64 * VN) * 2;
   static_assert(bytes <= 160 * 1024, "LDS");
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)latent_prefill_kernel<DN, VN>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    attr_set = true;
-  }
+  allow_lds<latent_prefill_kernel<DN, VN>>(bytes);
   latent_prefill_kernel<DN, VN><<<a.n_tiles * a.H, 256, bytes, stream>>>(a);
 }
 

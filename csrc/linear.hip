@@ -24,6 +24,7 @@
 // 4096 SwiGLU 329 (422), 7664 x 28672 x 4096 SwiGLU 1296 (1458), 10000 x 4096 x 4096 251 (361).
 #include <math.h>
 
+#include "launch.h"
 #include "linear_tile.h"
 
 #define CUS 256
@@ -107,14 +108,8 @@ static void launch(const LinearArgs& a, int splits, hipStream_t stream) {
   constexpr int TN = 32 * FN, TM = 32 * FM, LDS = 128 * (WS * TN + XS * TM);
   constexpr bool GLU = UNIT == LINEAR_SWIGLU || UNIT == LINEAR_GLU;
   static_assert(LDS <= LDS_OF_A_CU);
-  static bool attr_set = false;
-  if (!attr_set) {
-    for (auto kernel : {linear_kernel<FN, FM, WS, XS, UNIT, false>,
-                        linear_kernel<FN, FM, WS, XS, UNIT, true>})
-      (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                LDS);
-    attr_set = true;
-  }
+  allow_lds<linear_kernel<FN, FM, WS, XS, UNIT, false>>(LDS);
+  allow_lds<linear_kernel<FN, FM, WS, XS, UNIT, true>>(LDS);
   const int outs = GLU ? a.N / 2 : a.N, per = GLU ? TN / 2 : TN, chunks = a.K / 64;
   LinearGrid g;
   g.tiles_m = (a.M + TM - 1) / TM;

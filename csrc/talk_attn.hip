@@ -19,6 +19,7 @@
 #include "common_t.h"
 #include "grouped_attn.h"
 #include "latent_attn.h"
+#include "launch.h"
 
 typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_v __attribute__((ext_vector_type(4)));
@@ -285,12 +286,7 @@ static int decode_bytes(const GroupedArgs& a, int d, int v, int ht, int gm) {
 
 template <int HT, int GM, int UL>
 static void launch_decode(const GroupedArgs& a, int d, int v, int seqs, hipStream_t stream) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)talk_decode_kernel<HT, GM, UL>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr_set = true;
-  }
+  allow_lds<talk_decode_kernel<HT, GM, UL>>(160 * 1024);
   talk_decode_kernel<HT, GM, UL>
       <<<dim3(seqs, a.n_split), 256, decode_bytes(a, d, v, HT, GM), stream>>>(a, d, v);
 }
@@ -703,12 +699,7 @@ template <int DN, int VN, int HT, int GV>
 static bool launch_prefill(const GroupedArgs& a, hipStream_t stream) {
   const int bytes = prompt_lds(a.H, a.G, 32 / (a.H / a.G), 64 * VN).total;
   if (bytes > 160 * 1024) return false;
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)talk_prefill_kernel<DN, VN, HT, GV>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr_set = true;
-  }
+  allow_lds<talk_prefill_kernel<DN, VN, HT, GV>>(160 * 1024);
   talk_prefill_kernel<DN, VN, HT, GV><<<a.n_tiles, 64 * a.G, bytes, stream>>>(a);
   return true;
 }

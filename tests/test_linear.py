@@ -115,6 +115,28 @@ def test_step_linear_takes_its_rows(m, n, k):
 
 
 @pytest.mark.gpu
+def test_linear_from_several_threads():
+    """Every thread may be the first to launch a kernel, each on a stream of its own."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    x, w = operands(70, 264, 320, 9)
+    torch.cuda.synchronize()
+
+    def run(first):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            outs = [ops._hip().linear(x, w, tile=(first + i) % 13) for i in range(13)]
+        stream.synchronize()
+        return outs
+
+    with ThreadPoolExecutor(6) as pool:
+        results = list(pool.map(run, range(6)))
+    for outs in results:
+        for out in outs:
+            assert torch.equal(out, results[0][0])
+
+
+@pytest.mark.gpu
 def test_linear_leaves_other_forms():
     """What the kernel does not take, and what others follow, stays with the library."""
     x, w = operands(64, 2048, 1024, 0)
