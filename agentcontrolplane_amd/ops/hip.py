@@ -534,10 +534,7 @@ def moe_experts(h, gate_up, down, ids, glu):
         if tiled:
             tiles = torch.empty(2, n // _C.EXPERT_TILE + E, dtype=torch.int32, device=device)
             tile_expert, tile_row = tiles
-        _C.moe_group(
-            perm, offsets, tile_expert, tile_row, ids, E, gate_up.shape[2], inner, down.shape[1],
-            True,
-        )
+        _C.moe_group(perm, offsets, tile_expert, tile_row, ids, E)
     grouped = (ids, perm, offsets, tile_expert, tile_row)
     _C.experts_linear(act, h, gate_up, *grouped, True, *form, kind, tt)
     _C.experts_linear(rows.view(n, -1), act, down, *grouped, False, *form, kind, tt)

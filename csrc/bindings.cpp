@@ -53,8 +53,7 @@ void launch_attn_inputs(bool, const AttnInputsArgs*, hipStream_t);
 void launch_moe_route(bool, int*, float*, const void*, const void*, const float*, int, int, int,
                       int, int64_t, bool, float, float*, int, hipStream_t);
 int moe_route_parts(bool, int, int, int);
-void launch_moe_group(int*, int*, int*, int*, const int*, int, int, const TiledProducts*,
-                      hipStream_t);
+void launch_moe_group(int*, int*, int*, int*, const int*, int, int, hipStream_t);
 void launch_experts_small(bool, const ExpertsArgs*, int, hipStream_t);
 void launch_experts_f32(bool, const ExpertsArgs*, hipStream_t);
 void launch_experts_gemm(bool, const ExpertsArgs*, hipStream_t);
@@ -1083,23 +1082,18 @@ static void moe_route(torch::Tensor ids, torch::Tensor weights, torch::Tensor h,
                    parts > 1 ? sums.data_ptr<float>() : nullptr, parts, cur_stream());
 }
 
-// perm [n], offsets [E + 2]; tiles of at least EXPERT_TILE rows: at most ceil(n / tile) + E, for
-// products with these many inner elements and outputs
+// perm [n], offsets [E + 2]; tiles of at most EXPERT_TILE rows: at most n / EXPERT_TILE + E
 static void moe_group(torch::Tensor perm, torch::Tensor offsets, OptTensor tile_expert,
-                      OptTensor tile_row, torch::Tensor ids, int64_t E, int64_t width,
-                      int64_t inner, int64_t outputs, bool even) {
+                      OptTensor tile_row, torch::Tensor ids, int64_t E) {
   const int64_t n = ids.numel();
   CHECK_CUDA(ids); CHECK_CONT(ids);
   TORCH_CHECK(ids.scalar_type() == at::kInt && E > 0 && E <= 512 && n < (1 << 30));
-  const int64_t most = n / EXPERT_TILE + E, tiles = tile_expert ? most : 0;
+  const int64_t tiles = tile_expert ? n / EXPERT_TILE + E : 0;
   int* te = (int*)opt_int(tile_expert, tiles);
   int* tr = (int*)opt_int(tile_row, tiles);
-  const int64_t columns1 = (inner + 127) / 128, columns2 = (outputs + 255) / 256;
-  TORCH_CHECK(!te == !tr && width > 0 && width < (1 << 30) && inner > 0 && outputs > 0 &&
-              std::max(columns1, columns2) * most < (1 << 30), "tiles");
-  const TiledProducts sizes = {(int)width, (int)columns1, (int)inner, (int)columns2, even};
+  TORCH_CHECK(!te == !tr, "tiles");
   launch_moe_group((int*)opt_int(perm, n), (int*)opt_int(offsets, E + 2), te, tr,
-                   ids.data_ptr<int>(), (int)n, (int)E, &sizes, cur_stream());
+                   ids.data_ptr<int>(), (int)n, (int)E, cur_stream());
 }
 
 // One product of the routed experts (experts.h).  kind: 0 fp32, 1 few rows, 2 tiles
@@ -1149,8 +1143,9 @@ static void experts_linear(torch::Tensor out, torch::Tensor x, torch::Tensor w, 
   TORCH_CHECK(tile_expert && a.K % 128 == 0, "tiles");
   // byte offsets of 32 bits in the rows that a workgroup reads
   TORCH_CHECK(w.size(1) * (int64_t)a.K < (1 << 30) &&
-              (glu ? x.size(0) : TALL_TILE) * a.x_stride < (1 << 30), "rows of 2 GiB and more");
+              (glu ? x.size(0) : EXPERT_TILE) * a.x_stride < (1 << 30), "rows of 2 GiB and more");
   a.tiles = a.entries / EXPERT_TILE + a.E;
+  TORCH_CHECK((a.O / (glu ? 128 : 256) + 1) * (int64_t)a.tiles < (1 << 30), "tiles");
   a.tile_expert = opt_int(tile_expert, a.tiles);
   a.tile_row = opt_int(tile_row, a.tiles);
   launch_experts_gemm(glu, &a, cur_stream());
@@ -1307,9 +1302,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attention_inputs", &attention_inputs);
   m.attr("EXPERT_TILE") = EXPERT_TILE;
   m.def("moe_route", &moe_route);
-  m.def("moe_group", &moe_group, py::arg("perm"), py::arg("offsets"), py::arg("tile_expert"),
-        py::arg("tile_row"), py::arg("ids"), py::arg("E"), py::arg("width"), py::arg("inner"),
-        py::arg("outputs"), py::arg("even") = false);
+  m.def("moe_group", &moe_group);
   m.def("experts_linear", &experts_linear);
   m.def("delta_prompts", &delta_prompts);
   m.def("delta_step", &delta_step);

@@ -18,21 +18,5 @@ struct ExpertsArgs {
   float limit, alpha, offset, cubic;  // gate_up: the gated unit
 };
 
-// Sizes of the two tiled products: inner elements and columns of workgroups of a tile
-struct TiledProducts {
-  int width, columns1;  // gate and up
-  int inner, columns2;  // down
-  bool even;            // an expert's tiles have the same height
-};
-
-// rows of one tile of the large-batch product, at most TALL_TILE
+// rows of one tile of the large-batch product at most
 #define EXPERT_TILE 256
-#define TALL_TILE 320
-
-// Rows of an expert's tiles: even ones of 257 to 320 rows if they cover the expert in fewer tiles,
-// as a small last tile takes all of the expert's weights once more.
-__device__ static inline int tall_tile(int rows) {
-  const int tiles = (rows + TALL_TILE - 1) / TALL_TILE;
-  const int even = tiles > 0 ? (rows + tiles - 1) / tiles : 0;
-  return even > EXPERT_TILE ? even : EXPERT_TILE;
-}

@@ -182,8 +182,7 @@ static DEV uint64_t same_id(int id, int bits) {
 template <bool TILED>
 __global__ __launch_bounds__(1024) void group_kernel(
     int* __restrict__ perm, int* __restrict__ offsets, int* __restrict__ tile_expert,
-    int* __restrict__ tile_row, const int* __restrict__ ids, const int n, const int E,
-    const TiledProducts sizes) {
+    int* __restrict__ tile_row, const int* __restrict__ ids, const int n, const int E) {
   extern __shared__ int counts[];
   __shared__ int step_tiles[EXPERT_TILE / 32];
   int* total = counts + 16 * E;
@@ -238,54 +237,15 @@ __global__ __launch_bounds__(1024) void group_kernel(
     return s - v;
   };
   if (lists) {  // first rows of the experts and their tiles
-    // Tall tiles take up to an eighth longer each, which pays where they save rounds of
-    // workgroups (one a CU, columns a tile) in one of the two products; a tile of up to 192 rows
-    // takes about 0.6 of a round.  Both products, us, in tiles of 256 and tall ones: 32 experts,
-    // 4 of them a token at random, 2560 inner, 4096 outputs: 2048 tokens 853 and 665, 4093 1342
-    // and 1091, 6500 1910 and 1707, but 2600 880 and 1007, 7500 1822 and 1987; 16, 2 a token,
-    // 1280 inner, 2048 outputs: 1800 tokens 138 and 140, 4093 241 and 212. Taken where it is not
-    // faster: 2500 and 7000 tokens of the first (870 and 884, 1753 and 1819).
-    bool tall = false;
-    if (TILED && !sizes.even) {
-      int tiles[2] = {}, small[2] = {};  // of 256 rows, tall
-      for (int e = lane; e < E; e += 64) {
-        const int c = total[e], t = (c + EXPERT_TILE - 1) / EXPERT_TILE;
-        const int high = (c + TALL_TILE - 1) / TALL_TILE;
-        const bool whole = c > EXPERT_TILE * high, last = c > 0 && c - EXPERT_TILE * (t - 1) <= 192;
-        tiles[0] += t;
-        small[0] += last;
-        tiles[1] += whole ? high : t;
-        small[1] += whole ? 0 : last;
-      }
-      float cost[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int off = 32; off; off >>= 1) {
-          tiles[i] += __shfl_xor(tiles[i], off, 64);
-          small[i] += __shfl_xor(small[i], off, 64);
-        }
-        auto rounds = [&](int columns) {
-          return (float)((tiles[i] * columns + 255) / 256) - 0.4f / 256 * (small[i] * columns);
-        };
-        cost[i] = sizes.width * rounds(sizes.columns1) + sizes.inner * rounds(sizes.columns2);
-      }
-      tall = cost[1] < 0.92f * cost[0];
-    }
+    // an expert's tiles have the same height
     auto tiles_of = [&](int c, int& high) {
-      high = EXPERT_TILE;
-      int t = TILED ? (c + EXPERT_TILE - 1) / EXPERT_TILE : 0;
-      if (tall) {
-        high = tall_tile(c);
-        t = (c + high - 1) / high;
-      } else if (TILED && sizes.even && t > 0) {
-        high = (c + t - 1) / t;
-      }
+      const int t = TILED ? (c + EXPERT_TILE - 1) / EXPERT_TILE : 0;
+      high = t > 0 ? (c + t - 1) / t : 0;
       return t;
     };
     // the highest tiles first, by steps of 32 rows, a wave each: workgroups that end early then
     // fill up with the lower ones
-    const int steps = !TILED ? 0 : sizes.even ? EXPERT_TILE / 32 : 1;
+    const int steps = TILED ? EXPERT_TILE / 32 : 0;
     const int step = steps - wid;  // of rows
     int tile = 0;
     auto list = [&](bool count) {
@@ -294,7 +254,7 @@ __global__ __launch_bounds__(1024) void group_kernel(
         const int e = e0 + lane, c = e < E ? total[e] : 0;
         int high;
         int t = tiles_of(c, high);
-        if (sizes.even && (high + 31) / 32 != step) t = 0;
+        if ((high + 31) / 32 != step) t = 0;
         const int first = row + before(c, sum);
         row += sum;
         const int at = tile + before(t, sum);
@@ -571,11 +531,11 @@ void launch_moe_route(bool bf16, int* ids, float* weights, const void* h, const 
 }
 
 void launch_moe_group(int* perm, int* offsets, int* tile_expert, int* tile_row, const int* ids,
-                      int n, int E, const TiledProducts* sizes, hipStream_t stream) {
+                      int n, int E, hipStream_t stream) {
   auto kernel = tile_expert ? group_kernel<true> : group_kernel<false>;
   // a share has at least 1024 entries, a turn of its waves; one more workgroup for the lists
   const int shares = max(1, min(64, n / 1024));
-  kernel<<<shares + 1, 1024, 18 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E, *sizes);
+  kernel<<<shares + 1, 1024, 18 * E * 4, stream>>>(perm, offsets, tile_expert, tile_row, ids, n, E);
 }
 
 // tt: 16 tokens at a time, or twice as many

@@ -1,5 +1,5 @@
 // The routed experts' products for many rows per expert (gfx950): a grouped GEMM over
-// tiles of 256 rows of one expert, or up to 320.
+// tiles of up to 256 rows of one expert.
 //
 // Rows come grouped by expert.  The first product gathers its token rows and applies the gated
 // unit to its sums; the second reads the grouped rows in place and scatters its results to their
@@ -19,21 +19,19 @@
 
 #define LDS_BYTES 163840
 
-// One tile, or the two halves of more rows than the largest of the products' tiles
+// One tile
 template <bool GLU>
 struct ExpertWork {
   static constexpr bool ANY_WIDTH = !GLU;
   const ExpertsArgs& a;
   int row0, rows, o0;  // of the grouped rows
   const void* w;
-  int start, step, total;
+  static constexpr int start = 0, step = 1, total = 1;
 
-  DEV int next(int t) const { return t + 1 < total ? t + 1 : t; }
-  DEV LinearSpot spot(int t) const {
-    const int high = (rows + total - 1) / total, m0 = t * high;
+  DEV int next(int t) const { return t; }
+  DEV LinearSpot spot(int) const {
     const __bf16* x = (const __bf16*)a.x + (GLU ? 0 : row0 * a.x_stride);
-    return {m0, min(rows, m0 + high), o0, 0, a.K >> 6, 0, w, x, GLU ? a.entries / a.top : rows,
-            row0};
+    return {0, rows, o0, 0, a.K >> 6, 0, w, x, GLU ? a.entries / a.top : rows, row0};
   }
   DEV int64_t x_row(const LinearSpot& s, int m) const {
     return GLU ? a.perm[s.row0 + m] / a.top : m;
@@ -72,16 +70,14 @@ __global__ __launch_bounds__(256, 1) void experts_gemm_kernel(const ExpertsArgs 
   l.alpha = a.alpha;
   l.offset = a.offset;
   l.cubic = a.cubic;
-  const bool halves = rows > 256;
   const ExpertWork<GLU> work = {a, row0, rows, tn * (GLU ? 128 : 256),
-                                (const __bf16*)a.w + (int64_t)e * l.N * a.K,
-                                0, 1, halves ? 2 : 1};
+                                (const __bf16*)a.w + (int64_t)e * l.N * a.K};
   constexpr int UNIT = GLU ? LINEAR_GLU : LINEAR_PLAIN;
-  if (rows > 224 && !halves)
+  if (rows > 224)
     linear_tiles<8, 8, 3, 2, UNIT>(l, work, lds);
-  else if (rows > 192 && !halves)
+  else if (rows > 192)
     linear_tiles<8, 7, 3, 2, UNIT>(l, work, lds);
-  else if (rows > 160 && !halves)
+  else if (rows > 160)
     linear_tiles<8, 6, 3, 2, UNIT>(l, work, lds);
   else if (rows > 128)
     linear_tiles<8, 5, 3, 3, UNIT>(l, work, lds);

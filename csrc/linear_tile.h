@@ -39,11 +39,9 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   constexpr int LW = FN, LX = FM;              // a wave's loads of a chunk, 8 rows each
   constexpr int SW = TN * 128, SX = TM * 128;  // a chunk's bytes
   constexpr int NM = FN * FM;
-  // w is a chunk further ahead than its ring alone allows, or goes with x
-  constexpr bool AHEAD = WS > 2;
   // loads behind a chunk's last one when it is waited for
   constexpr int BEHIND = XS < WS ? LW + (XS - 2) * (LW + LX) : (WS - 2) * (LW + LX);
-  static_assert(BEHIND < 64 && XS >= 2 && WS >= 2 && (WS > 2 || XS == 2));
+  static_assert(BEHIND < 64 && XS >= 2 && WS >= 3);
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wn = wid & 1, wm = wid >> 1;
   const int c = lane & 15, g = lane >> 4;
@@ -159,7 +157,7 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   aim_x(tx);
 #pragma unroll
   for (int k = 0; k < (WS - 1 > XS ? WS - 1 : XS); ++k) {
-    if (k < (AHEAD ? WS - 1 : 2)) {
+    if (k < WS - 1) {
 #pragma unroll
       for (int i = 0; i < LW; ++i) load_w(i);
       next_w();
@@ -187,9 +185,8 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
       typedef std::integral_constant<int, NM> All;
       typedef std::integral_constant<int, FN + FM> Reads;
       look(1);
-      multiply(first, I0(), I0(), All(), Reads(), std::integral_constant<int, AHEAD ? LW : 0>(),
-               load_w);
-      if (AHEAD) next_w();
+      multiply(first, I0(), I0(), All(), Reads(), std::integral_constant<int, LW>(), load_w);
+      next_w();
       multiply(std::false_type(), I1(), I0(), Ahead(), I0(), I0(), load_x);
       // this chunk is read, the next one has landed, for every wave after the barrier; what
       // may be under way are the loads behind the next chunk's
@@ -200,11 +197,9 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
       rw = rw == (WS - 1) * SW ? 0 : rw + SW;
       rx = rx == (XS - 1) * SX ? 0 : rx + SX;
       look(0);
-      multiply(std::false_type(), I1(), Ahead(), All(), Reads(),
-               std::integral_constant<int, AHEAD ? LX : LX + LW>(),
-               [&](int i) { i < LX ? load_x(i) : load_w(i - LX); });
+      multiply(std::false_type(), I1(), Ahead(), All(), Reads(), std::integral_constant<int, LX>(),
+               load_x);
       next_x();
-      if (!AHEAD) next_w();
     };
     chunk(std::true_type());
     for (int k = spot.last - spot.first; k > 1; --k) chunk(std::false_type());

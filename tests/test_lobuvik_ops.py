@@ -527,7 +527,7 @@ def test_group(n, E, tiled):
     ids = (torch.rand(n, generator=g) ** 3 * E).int().clamp(max=E - 1).cuda()
     lists = torch.empty(2, n // _C.EXPERT_TILE + E, dtype=torch.int32, device="cuda")
     perm, offsets = torch.empty_like(ids), lists.new_empty(E + 2)
-    _C.moe_group(perm, offsets, *(lists if tiled else (None, None)), ids, E, 64, 64, 64, True)
+    _C.moe_group(perm, offsets, *(lists if tiled else (None, None)), ids, E)
     assert torch.equal(perm.long(), torch.sort(ids, stable=True).indices)
     first = torch.bincount(ids, minlength=E).cumsum(0)
     assert offsets[0] == 0 and torch.equal(offsets[1 : E + 1].long(), first)
@@ -555,8 +555,7 @@ EXPERTS = [
 @pytest.mark.gpu
 @pytest.mark.parametrize("I", [256, 3072], ids=["one round", "several"])
 def test_experts_tile_heights(I):
-    """Every height of an expert's tiles: few rows, 256, the even ones up to 320, several; the
-    tall ones where they save a round of workgroups."""
+    """Every height of an expert's tiles: few rows, 256, several of equal heights."""
     rows = [0, 1, 64, 65, 255, 256, 257, 288, 289, 320, 321, 512, 513, 577, 640, 641, 961]
     E, K, W = len(rows), 128, 264
     ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).int()
@@ -571,34 +570,6 @@ def test_experts_tile_heights(I):
         t = (ids[:, 0] == e).nonzero()[:, 0]
         if len(t):
             close(got[t, 0], oracle.clamped_glu(h.double().cpu()[t], x, "", 1.25), torch.bfloat16)
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("K,tiles", [(128, 33), (1024, 26)], ids=["plain", "tall"])
-def test_experts_choose_tile_heights(K, tiles):
-    """Tall tiles where they save a round of the larger product (660 workgroups, 520), not where
-    that product is the smaller part; the results are the same to a rounding."""
-    from agentcontrolplane_amd import _C
-
-    rows = [0, 1, 64, 65, 255, 256, 257, 288, 289, 320, 321, 512, 513, 577, 640, 641, 961]
-    E, I, W = len(rows), 2432, 520
-    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).int()
-    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(2))].view(-1, 1)
-    h = rand(len(ids), K, dtype=torch.bfloat16, device="cuda")
-    gate_up = rand(E, 2 * I, K, dtype=torch.bfloat16, device="cuda", seed=1, scale=2 * K ** -0.5)
-    down = rand(E, W, I, dtype=torch.bfloat16, device="cuda", seed=2, scale=I ** -0.5)
-    ids, spec = ids.cuda(), ClampedGluSpec(I, 1.25)
-    made = torch.empty(3, len(ids) // _C.EXPERT_TILE + E, dtype=torch.int32, device="cuda")
-    perm, offsets = torch.empty_like(ids[:, 0]), made.new_empty(E + 2)
-    _C.moe_group(perm, offsets, made[0], made[1], ids, E, K, I, W)
-    assert offsets[E + 1].item() == tiles
-    got = ops.moe_experts(h, gate_up, down, ids, spec)
-    for e, n in enumerate(rows):
-        if n:
-            x = {"gate": gate_up[e, :I].double(), "up": gate_up[e, I:].double(),
-                 "down": down[e].double()}
-            t = (ids[:, 0] == e).nonzero()[:, 0]
-            close(got[t, 0], oracle.clamped_glu(h[t].double(), x, "", 1.25), torch.bfloat16)
 
 
 @pytest.mark.parametrize("skew", [False, True])
@@ -667,12 +638,11 @@ def test_experts_of_large_weights(n, top, E, K, I, W):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("even", [True, False], ids=["even", "tall"])
 @pytest.mark.parametrize("I,W", [(128, 264), (2432, 130)])
-def test_experts_tile_lists(I, W, even):
-    """The tiles cover every expert's rows once, even ones the highest first; the products follow
-    either list, tiles of more than 256 rows among them, also for outputs that are no whole
-    16-byte units."""
+def test_experts_tile_lists(I, W):
+    """The tiles cover every expert's rows once, in as few of up to 256 rows as there can be, the
+    highest first; the products follow the list, also for outputs that are no whole 16-byte
+    units."""
     from agentcontrolplane_amd import _C
 
     rows = [0, 1, 33, 64, 65, 128, 129, 161, 193, 225, 256, 257, 289, 320, 321, 513, 640, 1100]
@@ -682,7 +652,7 @@ def test_experts_tile_lists(I, W, even):
     n, cuda = len(ids), ids.cuda().view(-1, 1)
     lists = torch.full((2, n // _C.EXPERT_TILE + E), -1, dtype=torch.int32, device="cuda")
     perm, offsets = torch.empty_like(cuda[:, 0]), lists.new_empty(E + 2)
-    _C.moe_group(perm, offsets, lists[0], lists[1], cuda, E, K, I, W, even)
+    _C.moe_group(perm, offsets, lists[0], lists[1], cuda, E)
     used, first = offsets[E + 1].item(), offsets.tolist()
     expert, row = lists[:, :used].tolist()
     heights = []
@@ -692,13 +662,12 @@ def test_experts_tile_lists(I, W, even):
         assert r == first[e] if i == 0 or expert[i - 1] != e else r > row[i - 1]
     for e, count in enumerate(rows):
         assert sum(h for h, x in zip(heights, expert) if x == e) == count
-    assert 0 < min(heights) and max(heights) <= (256 if even else 320)
-    if even:
-        steps = [-(-h // 32) for h in heights]
-        # an expert's last tile may be the lower one
-        assert all(a >= b for a, b, e, f in zip(steps, steps[1:], expert, expert[1:]) if e == f)
-        tops = [s for s, e, f in zip(steps, expert, [-1] + expert) if e != f]
-        assert tops == sorted(tops, reverse=True)
+    assert 0 < min(heights) and max(heights) <= 256 and used == sum(-(-n // 256) for n in rows)
+    steps = [-(-h // 32) for h in heights]
+    # an expert's last tile may be the lower one
+    assert all(a >= b for a, b, e, f in zip(steps, steps[1:], expert, expert[1:]) if e == f)
+    tops = [s for s, e, f in zip(steps, expert, [-1] + expert) if e != f]
+    assert tops == sorted(tops, reverse=True)
     h = rand(n, K, dtype=torch.bfloat16, device="cuda")
     gate_up = rand(E, 2 * I, K, dtype=torch.bfloat16, device="cuda", seed=1, scale=2 * K ** -0.5)
     down = rand(E, W, I, dtype=torch.bfloat16, device="cuda", seed=2, scale=I ** -0.5)
