@@ -335,70 +335,17 @@ static DEV void store_outputs(const ExpertsArgs& a, int64_t row, int o, f32x4_v 
 }
 
 // Few rows per expert: bound by the weights.  grid (outputs / 16 or 32, E); the 4 waves
-// of a workgroup split K in blocks of 64 and meet in LDS.  Two 16-row weight fragments:
-// gate and up of the same 16 outputs, or 32 outputs.  TT token fragments of 16 at a time.
+// of a workgroup split K in blocks of 64 and meet in LDS.  Two tiles of 16 rows of weights: gate
+// and up of the same 16 outputs, or 32 outputs.  A load has 8 rows of a whole line (64 of K), past
+// the caches: a model's other layers have come between.  The upper 8 rows and columns of a product
+// have the line's other half, and of its results those count whose row and column have the same
+// half; 8 TT tokens at a time.  Both products with routing, weights from memory, us, by loads of 16
+// rows of half a line through the caches, and so: 32 experts of 4096 x 2560, 4 a token, 2 tokens 129
+// and 105, 8 252 and 225, 48 374 and 334, 95 413 and 376; 16 of 2048 x 1536 1 token 42 and 42, 4 66 and
+// 59, 8 75 and 70, 16 78.5 and 74, 32 79 and 77.  Weights that are still in the caches, as in a loop
+// over one layer, are no slower so but for 1 and 2 tokens of the smaller ones (38 and 42, 47 and 53).
 template <bool GLU, int TT>
 __global__ __launch_bounds__(256) void experts_small_kernel(const ExpertsArgs a) {
-  __shared__ f32x4_v red[4][2][TT][64];
-  const int e = blockIdx.y;
-  const int row0 = a.offsets[e], rows = a.offsets[e + 1] - row0;
-  if (rows == 0) return;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int c = lane & 15, g = lane >> 4;
-  const int o0 = blockIdx.x * (GLU ? 16 : 32);
-  const bf16_t* w = (const bf16_t*)a.w + (int64_t)e * (GLU ? 2 : 1) * a.O * a.K + g * 8;
-  const bf16_t* w0 = w + (int64_t)min(o0 + c, a.O - 1) * a.K;
-  const bf16_t* w1 = w + (int64_t)(GLU ? a.O + o0 + c : min(o0 + 16 + c, a.O - 1)) * a.K;
-  for (int r0 = 0; r0 < rows; r0 += 16 * TT) {
-    const bf16_t* xp[TT];
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      const int r = row0 + min(r0 + t * 16 + c, rows - 1);
-      xp[t] = (const bf16_t*)a.x + (int64_t)(GLU ? a.perm[r] / a.top : r) * a.x_stride + g * 8;
-    }
-    f32x4_v acc[2][TT] = {};
-#pragma unroll 2
-    for (int k = wid * 64; k < a.K; k += 256) {
-#pragma unroll
-      for (int s = 0; s < 64; s += 32) {
-        const bf16x8_v f0 = *(const bf16x8_v*)(w0 + k + s);
-        const bf16x8_v f1 = *(const bf16x8_v*)(w1 + k + s);
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-          const bf16x8_v b = *(const bf16x8_v*)(xp[t] + k + s);
-          acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f0, b, acc[0][t], 0, 0, 0);
-          acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f1, b, acc[1][t], 0, 0, 0);
-        }
-      }
-    }
-    if (r0) __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int t = 0; t < TT; ++t) red[wid][i][t][lane] = acc[i][t];
-    __syncthreads();
-    // a thread sums 4 outputs of one row
-    for (int j = threadIdx.x; j < (GLU ? 1 : 2) * TT * 64; j += 256) {
-      const int l = j & 63, t = (j >> 6) % TT, i = (j >> 6) / TT;
-      const int r = r0 + t * 16 + (l & 15), o = o0 + i * 16 + (l >> 4) * 4;
-      if (r >= rows || o >= a.O) continue;
-      const f32x4_v v = red[0][i][t][l] + red[1][i][t][l] + red[2][i][t][l] + red[3][i][t][l];
-      f32x4_v u = {};
-      if (GLU) u = red[0][1][t][l] + red[1][1][t][l] + red[2][1][t][l] + red[3][1][t][l];
-      store_outputs<GLU>(a, GLU ? row0 + r : a.perm[row0 + r], o, v, u);
-    }
-  }
-}
-
-// The same for weights that the memory-side cache (256 MB) cannot keep: a load has 8 rows of a whole
-// line (64 of K), past the caches.  The upper 8 rows and columns of a product have the line's other
-// half, and of its results those count whose row and column have the same half; 8 TT tokens at
-// a time.  32 experts of 4096 x 2560, 4 a token, both products with routing, us, by
-// experts_small_kernel and so: 2 tokens 129 and 105, 8 252 and 225, 48 374 and 334, 95 413 and 376.
-// Where a caller has no other layers between, smaller weights come from the caches, and half the
-// waves a CU are the slower choice: 16 of 2048 x 1536 1 token 36 and 40 us, 16 73 and 76.
-template <bool GLU, int TT>
-__global__ __launch_bounds__(256) void experts_lines_kernel(const ExpertsArgs a) {
   __shared__ f32x4_v red[4][2][2][TT][2][16];  // wave, tile, 8 rows, tokens, half, (4 rows, token)
   const int e = blockIdx.y;
   const int row0 = a.offsets[e], rows = a.offsets[e + 1] - row0;
@@ -542,10 +489,8 @@ void launch_moe_group(int* perm, int* offsets, int* tile_expert, int* tile_row, 
 void launch_experts_small(bool glu, const ExpertsArgs* a, int tt, hipStream_t stream) {
   const int per = glu ? 16 : 32;
   const dim3 grid((a->O + per - 1) / per, a->E);
-  const bool lines = (glu ? 4ll : 2ll) * a->E * a->O * a->K > 256 << 20;
-#define SMALL(kernel, t) (glu ? kernel<true, t> : kernel<false, t>)
-  auto k = lines ? (tt == 1 ? SMALL(experts_lines_kernel, 2) : SMALL(experts_lines_kernel, 4))
-                 : (tt == 1 ? SMALL(experts_small_kernel, 1) : SMALL(experts_small_kernel, 2));
+  auto k = glu ? (tt == 1 ? experts_small_kernel<true, 2> : experts_small_kernel<true, 4>)
+               : (tt == 1 ? experts_small_kernel<false, 2> : experts_small_kernel<false, 4>);
   k<<<grid, 256, 0, stream>>>(*a);
 }
 
