@@ -34,7 +34,7 @@ def sums(x, w, bias=None):
 ])
 def test_linear(tile, m, n, k, splits, kind):
     """One rounding of the sum to 16 bits, and sums of k terms in 32 bits; nothing is written
-    beside the outputs.  The last case has several tiles a workgroup."""
+    beside the outputs.  The last case has several of the smaller tiles a workgroup."""
     hip = ops._hip()
     x, w = operands(m, n, k, m + n + k, kind == "strided")
     bias = torch.randn(n, device="cuda").bfloat16() if kind == "bias" else None
@@ -45,6 +45,23 @@ def test_linear(tile, m, n, k, splits, kind):
     assert ((out.double() - exact).abs() <= 2.0 ** -8 * exact.abs() + slack + 1e-30).all()
     pad[1:-1, 8:-8] = 7.0
     assert (pad == 7.0).all()
+
+
+FORMS = {"swiglu": (0.0,) * 4, "glu": (7.0, 1.702, 1.0, 0.0)}  # limit, alpha, offset, cubic
+
+
+def check_gated(got, x, w, unit):
+    exact, slack = sums(x, w)
+    g, u = exact.chunk(2, 1)
+    # both halves are off by a rounding and the sums' slack
+    dg, du = (2.0 ** -8 * t.abs() + s for t, s in zip((g, u), slack.chunk(2, 1)))
+    alpha, plus = (1.702, 1.0) if unit == "glu" else (1.0, 0.0)
+    if unit == "glu":
+        g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
+    act = g * torch.sigmoid(alpha * g)  # slope at most 1.1 for any alpha
+    want = act * (u + plus)
+    bound = 1.1 * dg * (u.abs() + du + plus) + act.abs() * du
+    assert ((got.double() - want).abs() <= bound + 2.0 ** -7 * want.abs() + 1e-30).all()
 
 
 @pytest.mark.gpu
@@ -60,19 +77,55 @@ def test_linear_gated(tile, m, n, k, splits, unit):
             hip.linear(*operands(m, n, k, 1), unit=unit, tile=tile)
         return
     x, w = operands(m, n, k, m + n + k)
-    form = (7.0, 1.702, 1.0, 0.0) if unit == "glu" else (0.0,) * 4
-    got = hip.linear(x, w, None, unit, form, tile=tile, splits=splits).double()
+    check_gated(hip.linear(x, w, None, unit, FORMS[unit], tile=tile, splits=splits), x, w, unit)
+
+
+#: outputs and rows of the tiles
+SIZES = [(256, 256), (256, 224), (256, 192), (256, 160), (256, 128), (128, 192), (128, 128),
+         (128, 96), (128, 64), (128, 32), (192, 128), (64, 64), (64, 32)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(5))
+@pytest.mark.parametrize("k", [64, 128, 192, 320])
+def test_linear_of_several_tiles_a_workgroup(tile, k):
+    """The large tiles, one workgroup a CU: the loads run ahead over the end of a tile of 1, 2, 3
+    and 5 chunks, into ragged rows and outputs, behind every kind of store."""
+    hip, m, n = ops._hip(), 4200, 8208
+    assert -(-m // SIZES[tile][1]) * -(-n // SIZES[tile][0]) > 2 * 256
+    x, w = operands(m, n, k, k)
     exact, slack = sums(x, w)
-    g, u = exact.chunk(2, 1)
-    # both halves are off by a rounding and the sums' slack
-    dg, du = (2.0 ** -8 * t.abs() + s for t, s in zip((g, u), slack.chunk(2, 1)))
-    alpha, plus = (1.702, 1.0) if unit == "glu" else (1.0, 0.0)
-    if unit == "glu":
-        g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
-    act = g * torch.sigmoid(alpha * g)  # slope at most 1.1 for any alpha
-    want = act * (u + plus)
-    bound = 1.1 * dg * (u.abs() + du + plus) + act.abs() * du
-    assert ((got - want).abs() <= bound + 2.0 ** -7 * want.abs() + 1e-30).all()
+    got = hip.linear(x, w, tile=tile).double()
+    assert ((got - exact).abs() <= 2.0 ** -8 * exact.abs() + slack + 1e-30).all()
+    bias = torch.randn(n, device="cuda").bfloat16()
+    exact += bias.double()
+    got = hip.linear(x, w, bias, tile=tile).double()
+    assert ((got - exact).abs() <= 2.0 ** -8 * exact.abs() + slack + 1e-30).all()
+    for unit in FORMS:
+        check_gated(hip.linear(x, w, None, unit, FORMS[unit], tile=tile), x, w, unit)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+def test_linear_of_large_weights_and_one_tile_of_rows(tile):
+    """Those that no other workgroup reads pass by the caches, in kernels of their own: plain,
+    bias, both units and parts, at the smallest weights that take them."""
+    hip, m, n, k = ops._hip(), SIZES[tile][1] - 6, 8208, 4096
+    assert n * k >= 32 << 20 > (n - 32) * k
+    x, w = operands(m, n, k, m)
+    exact, slack = sums(x, w)
+    bias = torch.randn(n, device="cuda").bfloat16()
+    for splits in (1, 3):
+        got = hip.linear(x, w, tile=tile, splits=splits).double()
+        assert ((got - exact).abs() <= 2.0 ** -8 * exact.abs() + slack).all()
+        got, want = hip.linear(x, w, bias, tile=tile, splits=splits).double(), exact + bias.double()
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + slack).all()
+        for unit in FORMS:
+            if splits > 1 or hip._C.linear_fits(tile, True):
+                check_gated(hip.linear(x, w, None, unit, FORMS[unit], tile=tile, splits=splits),
+                            x, w, unit)
+    parts = hip._C.linear_parts(x, w, tile, 3)
+    assert parts.shape == (3, m, n) and ((parts.double().sum(0) - exact).abs() <= slack).all()
 
 
 @pytest.mark.gpu
@@ -290,14 +343,24 @@ def test_parts_into_the_caches(m, heads, kv, d, k, tile, splits):
 @pytest.mark.gpu
 @pytest.mark.parametrize("m", [3, 61, 190, 2100])
 def test_step_linear_with_what_follows(m):
-    """The entries are the passes one after another, to a rounding of the product."""
+    """The entries are the passes one after another, but for the product's sums of 32 bits, which
+    may round to the next 16-bit value: an ulp, up to 2^-7 of it, and so may what follows."""
     x, w = operands(m, 2048, 1024, m)
+    y, slack = sums(x, w)
     residual = x.repeat(1, 2)
     weight = torch.rand(2048, device="cuda").bfloat16()
-    got, sums = ops.step_linear_add_rmsnorm(x, w, residual.clone(), weight)
+    ulp = 2.0 ** -7
+    dy = ulp * y.abs() + 2 * slack
+    got, total = ops.step_linear_add_rmsnorm(x, w, residual.clone(), weight)
     want, new = ops.fused_add_rmsnorm(ops.step_linear(x, w), residual.clone(), weight)
-    assert torch.allclose(sums.float(), new.float(), rtol=2.0 ** -6, atol=0.5)
-    assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -6, atol=0.03)
+    new = new.double()
+    dt = dy + ulp * new.abs()
+    assert ((total.double() - new).abs() <= dt).all()
+    inv = torch.rsqrt((new ** 2).mean(-1, keepdim=True) + 1e-5)
+    # the norm moves by its share of what its squares do
+    turn = inv ** 2 * (2 * new.abs() * dt).mean(-1, keepdim=True) / 2
+    bound = inv * weight.double() * (dt + new.abs() * turn) + ulp * want.double().abs()
+    assert ((got.double() - want.double()).abs() <= bound).all()
     cos_sin = torch.rand(2, 9, 64, device="cuda")
     pos, slots = torch.arange(m, device="cuda") % 9, torch.arange(m, device="cuda")
     both = []
@@ -307,8 +370,11 @@ def test_step_linear_with_what_follows(m):
         if fused:
             q = ops.step_linear_rope_and_cache(x, w, 8, *to)
         else:
-            y = ops.step_linear(x, w).view(m, 16, 128)
-            q = ops.rope_and_cache(y[:, :8], y[:, 8:12], y[:, 12:], *to)[0]
-        both.append((q, kc, vc))
-    for a, b in zip(*both):
-        assert torch.allclose(a.float(), b.float(), rtol=2.0 ** -6, atol=0.5)
+            y16 = ops.step_linear(x, w).view(m, 16, 128)
+            q = ops.rope_and_cache(y16[:, :8], y16[:, 8:12], y16[:, 12:], *to)[0]
+        both.append([t.double() for t in (q, kc, vc)])
+    dy = dy.view(m, 16, 128)
+    # a rotated value has both of its pair, each times at most 1
+    pair = dy + dy.roll(64, -1)
+    for a, b, d in zip(*both, (pair[:, :8], pair[:, 8:12], dy[:, 12:])):
+        assert ((a - b).abs() <= d + ulp * b.abs()).all()
