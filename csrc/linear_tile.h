@@ -19,13 +19,30 @@ struct LinearSpot {
   int x_rows, row0;
 };
 
+// n / (1 + exp(-z)), the same bits as the division's for all n of 16 bits, in fewer instructions: a
+// quarter of the divisor has a reciprocal at all its sizes and needs no scaling.  The reciprocal is
+// one ulp off before a Newton step, the quotient takes in its remainder (Markstein's way), and the
+// hardware puts infinities and what is no number right.  The unit ends a tile of products and nothing
+// else runs beside it: 15675 x 28672 x 4096 SwiGLU takes 1.8% longer than with the reciprocal
+// alone, by the division 2.7%.
+DEV float by_sigmoid(float n, float z) {
+  const float d = __builtin_fmaf(__expf(-z), 0.25f, 0.25f), n4 = 0.25f * n;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+  const float q = n4 * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, n4), r, q), d, n4);
+}
+
 // The gated unit of two sums, both rounded first, as they are between two passes
 template <int UNIT>
 DEV float unit_of(const LinearArgs& a, float gate, float up) {
   gate = (float)(__bf16)gate;
   up = (float)(__bf16)up;
-  if (UNIT == LINEAR_SWIGLU) return gate / (1.f + __expf(-gate)) * up;
-  return clamped_glu_f(gate, up, a.limit, a.alpha, a.offset, a.cubic);
+  if (UNIT == LINEAR_SWIGLU) return by_sigmoid(gate, gate) * up;
+  gate = fminf(gate, a.limit);
+  float z = a.alpha * gate;
+  if (a.cubic != 0.f) z *= 1.f + a.cubic * gate * gate;
+  return gate * by_sigmoid(1.f, z) * (fminf(fmaxf(up, -a.limit), a.limit) + a.offset);
 }
 
 #ifdef __HIP_DEVICE_COMPILE__  // the host knows no buffer resources

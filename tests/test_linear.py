@@ -86,6 +86,30 @@ SIZES = [(256, 256), (256, 224), (256, 192), (256, 160), (256, 128), (128, 192),
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", [None, (7.0, 1.702, 1.0, 0.0), (1e30, 1.0, 0.0, 0.0),
+                                  (3e38, 1.5957691, 0.0, 0.044715)])
+def test_gated_unit_of_every_gate(form):
+    """All 65536 gates of 16 bits, zeros, denormals, infinities and what is no number among them, come out
+    as from the unit's own pass, beside their like and beside ordinary ones."""
+    hip, n = ops._hip(), 1 << 16
+    gates = torch.arange(n, device="cuda").short().view(torch.bfloat16)
+    for order in (gates, gates[torch.randperm(n, device="cuda")]):
+        w = torch.zeros(2 * n, 64, device="cuda", dtype=torch.bfloat16)
+        w[:n, 0], w[n:, 0] = order, torch.linspace(-3, 3, n, device="cuda").bfloat16()
+        x = torch.zeros(33, 64, device="cuda", dtype=torch.bfloat16)
+        x[:, 0] = 1.0
+        y = hip.linear(x, w, tile=6)
+        if form is None:
+            got, want = hip.linear(x, w, unit="swiglu", tile=6), ops.swiglu(y)
+        else:
+            got = hip.linear(x, w, None, "glu", form, tile=6)
+            want = torch.empty_like(got)
+            ops.clamped_glu(y, *form[:3], want, form[3])
+        nan = want.isnan()
+        assert torch.equal(got.isnan(), nan) and torch.equal(got[~nan], want[~nan])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tile", range(5))
 @pytest.mark.parametrize("k", [64, 128, 192, 320])
 def test_linear_of_several_tiles_a_workgroup(tile, k):
