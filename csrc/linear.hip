@@ -19,9 +19,9 @@
 // among them 663, the reads done at three quarters of a step 652.  Stores of whole lines past
 // the caches: 8131 x 28672 x 4096 1335 to 1299.
 //
-// Against the GEMM library (and the unit's own pass), us: 64 x 4096 x 14336 30 (53), 192 x 28672
-// x 4096 SwiGLU 69 (72), 192 x 4096 x 14336 42 (111), 512 x 4096 x 14336 70 (98), 1739 x 28672 x
-// 4096 SwiGLU 329 (422), 7664 x 28672 x 4096 SwiGLU 1296 (1458), 10000 x 4096 x 4096 251 (361).
+// Against the GEMM library (and the unit's own pass), us: 64 x 4096 x 14336 31 (41), 192 x 28672
+// x 4096 SwiGLU 58 (67), 192 x 4096 x 14336 46 (103), 512 x 4096 x 14336 67 (91), 1739 x 28672 x
+// 4096 SwiGLU 328 (417), 7664 x 28672 x 4096 SwiGLU 1259 (1376), 10000 x 4096 x 4096 244 (370).
 #include <math.h>
 
 #include "launch.h"
