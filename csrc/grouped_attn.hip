@@ -21,7 +21,7 @@
 // 1 x 4002 203 -> 14; with the values' loads, whole lines each, past the caches 190 x 700 to 1300 148
 // -> 139, 61 x 310 to 4000 120 -> 112.5, and 13 x 300 to 3900 of 32 key heads 95 -> 88; with the
 // keys' loads likewise, instead of 16 rows of half a line, 137, 109 and 85, 200 x 100 to 1000 of 64
-// heads over 8 130 -> 116; 64 x 128 17.1 -> 16.5, 64 x 16 7.3 -> 7.7 (launches and their first loads, not memory).  Without the next block in
+// heads over 8 130 -> 116; 64 x 128 17.1 -> 16.7, 64 x 16 7.3 -> 7.7 (launches and their first loads, not memory).  Without the next block in
 // flight the same kernel takes 350 us at 190 x 700 to 1300; at 3 waves a SIMD the registers for
 // it are not there.
 #include <type_traits>
@@ -233,15 +233,15 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   };
   auto find = [&](int i) {
     Place at;
-    at.shared = begins_alike;
     const int key0 = blocks.key(i);
+    auto key = [&](int g) { return min(key0 + 16 * g, pos & ~15); };
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
-      const int k = min(key0 + 16 * g, pos & ~15);
-      const int page = PAGED ? pages[k >> shift] : 0;
-      if (PAGED) at.shared &= page == others[k >> shift];
-      at.slot[g] = PAGED ? (page << shift) + (k & (a.kv_block - 1)) : 0;
+      const int k = key(g);
+      at.slot[g] = PAGED ? (pages[k >> shift] << shift) + (k & (a.kv_block - 1)) : 0;
     }
+    at.shared = PAGED && begins_alike && pages[key(0) >> shift] == others[key(0) >> shift] &&
+                pages[key(1) >> shift] == others[key(1) >> shift];
     return at;
   };
   // A load of keys has 8 rows of whole lines, 64 dims: the upper 8 rows of a product, and its upper 8
