@@ -680,14 +680,14 @@ def test_model_forward_gpu_vs_cpu_reference():
 @pytest.mark.parametrize(
     "m,n,k",
     [
-        (256, 256, 128),      # single tile, one 8-phase iteration
+        (256, 256, 128),      # a single tile, two chunks
         (300, 512, 256),      # ragged M (row-clamp + store guard)
         (1024, 1536, 4096),   # multi-tile, deep K
         (2048, 768, 1664),    # K % 128 == 0 but K % 256 != 0; odd tile grid
     ],
 )
 def test_gemm_bf16(m, n, k):
-    """Hand-written 256²-tile 8-phase MFMA GEMM vs fp32 matmul oracle."""
+    """The own products by threshold, on the largest tiles, vs fp32 matmul oracle."""
     torch.manual_seed(11)
     x = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
     w = torch.randn(n, k, device="cuda", dtype=torch.bfloat16)

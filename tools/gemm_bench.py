@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""A/B the hand-written 256²-tile 8-phase MFMA GEMM against the library
+"""A/B the own products on the largest tiles (csrc/linear.hip) against the library
 (hipBLASLt via torch.nn.functional.linear) on the engine's projection
 shapes.  Run on the GPU box:
 
