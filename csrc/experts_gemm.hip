@@ -31,7 +31,7 @@ struct ExpertWork {
   DEV int next(int t) const { return t; }
   DEV LinearSpot spot(int) const {
     const __bf16* x = (const __bf16*)a.x + (GLU ? 0 : row0 * a.x_stride);
-    return {0, rows, o0, 0, a.K >> 6, 0, w, x, GLU ? a.entries / a.top : rows, row0};
+    return {0, rows, o0, 0, a.K >> 6, 0, w, x, GLU ? a.entries / a.top : rows, row0, 0};
   }
   DEV int64_t x_row(const LinearSpot& s, int m) const {
     return GLU ? a.perm[s.row0 + m] / a.top : m;

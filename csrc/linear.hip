@@ -33,6 +33,7 @@
 struct LinearGrid {
   int tiles_m, tiles_n, band;
   int splits, each;  // parts of the inner dimension, chunks of one
+  uint64_t apart;    // chunks from where a tile begins to where its neighbour does, times 2^32
 };
 
 struct LinearWork {
@@ -54,9 +55,11 @@ struct LinearWork {
     const int part = grid.splits > 1 ? id / tiles : 0;
     id -= part * tiles;
     const int per = grid.band * grid.tiles_n, b = id / per, rest = id - b * per;
-    const int high = min(grid.band, grid.tiles_m - b * grid.band);
-    return {(b * grid.band + rest % high) * tm, a.M, rest / high * tn, part * grid.each,
-            min(chunks, (part + 1) * grid.each), part, a.w, a.x, a.M, 0};
+    const int high = min(grid.band, grid.tiles_m - b * grid.band), column = rest / high;
+    const int first = part * grid.each, last = min(chunks, first + grid.each);
+    const int at = first + (int)(column * grid.apart >> 32);
+    return {(b * grid.band + rest % high) * tm, a.M, column * tn, first, last, part, a.w, a.x, a.M,
+            0, at};
   }
 };
 
@@ -124,8 +127,16 @@ static void launch(const LinearArgs& a, int splits, hipStream_t stream) {
   // 44.3, 13 x 12288 x 4096 22.5 to 20.9, 61 x 128256 x 4096 209 to 193, 13 x 17792 x 2048 19.4 to
   // 18.6; weights of 33 MB are not worth it, 13 x 2048 x 8192 12.9 and 13.9
   const bool once = g.tiles_m == 1 && (int64_t)a.N * a.K >= 32 << 20;
+  // Rows of a power of two lie 4 KB and more apart, so that their columns are in a few of the memory's
+  // channels, all of which are busy only if tiles are at different columns.  us, before and now: 61 x
+  // 28672 x 4096 SwiGLU 50.9 and 42.5, 13 x 28672 x 4096 47.0 and 39.5, 13 x 12288 x 4096 20.6 and
+  // 18.3, 61 x 20480 x 4096 44.5 and 42.1, 190 x 128256 x 4096 231 and 192; at K = 5120 or 3584 the
+  // same as before.  Weights in rows of 64 elements more give no less, for more memory; an eighth
+  // of K apart by XCD 1 to 5% less, by twos or fours of tiles nothing.  Parts are apart by themselves: 61 x
+  // 6144 x 4096 in 4 parts 14.0, in turns 14.9.
+  g.apart = once && g.splits == 1 ? ((uint64_t)chunks << 32) / g.tiles_n : 0;
   auto kernel = once ? linear_kernel<FN, FM, WS, XS, UNIT, true>
-                               : linear_kernel<FN, FM, WS, XS, UNIT, false>;
+                     : linear_kernel<FN, FM, WS, XS, UNIT, false>;
   kernel<<<dim3(workgroups), 256, LDS, stream>>>(a, g);
 }
 

@@ -11,12 +11,13 @@ typedef float f32x4_v __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4_v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) char lds_char;
 
-// Where a piece of work is: rows m0 .. m1 - 1, first output, chunks of the inner dimension,
-// its number among the parts of that, w, x with as many rows, what its Work adds to rows
+// Where a piece of work is: rows m0 .. m1 - 1, first output, chunks of the inner dimension, its number
+// among the parts of that, w, x with as many rows, what its Work adds to rows, the chunk that it
+// begins with where linear_tiles() takes them in turn
 struct LinearSpot {
   int m0, m1, o0, first, last, part;
   const void *w, *x;
-  int x_rows, row0;
+  int x_rows, row0, at;
 };
 
 // n / (1 + exp(-z)), the same bits as the division's for all n of 16 bits, in fewer instructions: a
@@ -48,10 +49,12 @@ DEV float unit_of(const LinearArgs& a, float gate, float up) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host knows no buffer resources
 // Works start, start + step .. below total of a workgroup of 4 waves.  Fragments of a wave along
 // the outputs (FN) and the rows (FM); chunks of w (WS) and x (XS) in LDS.  ONCE: no other
-// workgroup reads the same weights, whose loads then pass by the caches (nt).
+// workgroup reads the same weights, whose loads then pass by the caches (nt), and the chunks of a work
+// that is no part are taken in turn from its spot's ``at`` on.
 template <int FN, int FM, int WS, int XS, int UNIT, bool ONCE = false, class Work>
 DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   constexpr bool GLU = UNIT == LINEAR_SWIGLU || UNIT == LINEAR_GLU;
+  constexpr bool TURNS = ONCE && UNIT != LINEAR_PARTS;
   constexpr int TN = 32 * FN, TM = 32 * FM;    // rows of w and of x of a tile
   constexpr int LW = FN, LX = FM;              // a wave's loads of a chunk, 8 rows each
   constexpr int SW = TN * 128, SX = TM * 128;  // a chunk's bytes
@@ -71,12 +74,17 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   const int slot = ((lane & 7) ^ (lane >> 3)) * 16;
   int vw[LW], vx[LX];  // this lane's rows
   // cursors of the loads: work, chunk, its last one, place in LDS; past the last work its
-  // chunks again
-  int tw = work.start, cw, ew, sw = 0, tx = work.start, cx, ex, sx = 0;
+  // chunks again.  In turn: its first chunk and the ones left
+  int tw = work.start, cw, ew, fw0 = 0, nw = 0, sw = 0;
+  int tx = work.start, cx, ex, fx0 = 0, nx = 0, sx = 0;
   auto aim_w = [&](int t) {
     const LinearSpot spot = work.spot(t);
-    cw = spot.first;
+    cw = TURNS ? spot.at : spot.first;
     ew = spot.last;
+    if (TURNS) {
+      fw0 = spot.first;
+      nw = spot.last - spot.first;
+    }
     bw = buffer(spot.w, a.N, a.w_stride, a.K);
 #pragma unroll
     for (int i = 0; i < LW; ++i) {
@@ -90,8 +98,12 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   };
   auto aim_x = [&](int t) {
     const LinearSpot spot = work.spot(t);
-    cx = spot.first;
+    cx = TURNS ? spot.at : spot.first;
     ex = spot.last;
+    if (TURNS) {
+      fx0 = spot.first;
+      nx = spot.last - spot.first;
+    }
     bx = buffer(spot.x, spot.x_rows, a.x_stride, a.K);
 #pragma unroll
     for (int i = 0; i < LX; ++i) {
@@ -109,14 +121,18 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   };
   auto next_w = [&]() {
     sw = sw == (WS - 1) * SW ? 0 : sw + SW;
-    if (++cw == ew) {
+    ++cw;
+    if (TURNS && cw == ew) cw = fw0;
+    if (TURNS ? --nw == 0 : cw == ew) {
       tw = work.next(tw);
       aim_w(tw);
     }
   };
   auto next_x = [&]() {
     sx = sx == (XS - 1) * SX ? 0 : sx + SX;
-    if (++cx == ex) {
+    ++cx;
+    if (TURNS && cx == ex) cx = fx0;
+    if (TURNS ? --nx == 0 : cx == ex) {
       tx = work.next(tx);
       aim_x(tx);
     }

@@ -131,10 +131,12 @@ def test_linear_of_several_tiles_a_workgroup(tile, k):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("tile", TILES)
-def test_linear_of_large_weights_and_one_tile_of_rows(tile):
-    """Those that no other workgroup reads pass by the caches, in kernels of their own: plain,
-    bias, both units and parts, at the smallest weights that take them."""
-    hip, m, n, k = ops._hip(), SIZES[tile][1] - 6, 8208, 4096
+@pytest.mark.parametrize("n,k", [(8208, 4096), (65552, 512), (1040, 32320)])
+def test_linear_of_large_weights_and_one_tile_of_rows(tile, n, k):
+    """Those that no other workgroup reads pass by the caches, in kernels of their own, and tiles
+    begin apart in the inner dimension: plain, bias, both units and parts, at the smallest weights
+    that take them, several tiles a workgroup, fewer tiles than chunks."""
+    hip, m = ops._hip(), SIZES[tile][1] - 6
     assert n * k >= 32 << 20 > (n - 32) * k
     x, w = operands(m, n, k, m)
     exact, slack = sums(x, w)
