@@ -161,13 +161,14 @@ def _many_rows_pay(m: int, n: int, k: int, glu: bool, adds: bool = False) -> boo
     """Whether csrc/linear.hip is the faster one for m rows, n outputs (of a GLU: gates and ups)
     and k inner elements, where ``adds``: what reads it adds up its parts, which saves a launch of
     4.3 us.  The GEMM library (with a pass of its own for the GLU) is in brackets, us of every
-    weight from memory.  Up to about 2000 rows at most sizes: 8 x 22016 x 4096 GLU 38 (55), 64 x
-    4096 x 14336 31 (41), 192 x 4096 x 4096 22 (32), 512 x 6288 x 2048 25 (28), 1739 x 4096 x 11008 138
-    (165).  Without ``adds`` not: up to 32 rows of medium weights, 8 x 6144 x 4096 17.8 (14.9), 16 x 4096 x
-    8192 19.9 (16.3), or very large ones, 24 x 128256 x 4096 195 (185), 8 x 2048 x 8192 14.1 (12.8); tiles that
-    leave half of the CUs idle, 61 x 4096 x 4096 17.1 (13.7), 80 x 2048 x 4096 12.8 (11.2); weights
-    that two tiles of rows read, 96 x 12288 x 4096 36 (30).  The library has other sizes of its own
-    beside slow ones, 190 x 6288 x 2048 18.2 (16.2), 160 x 6288 x 2048 17.7 (20.0): not told apart.  From 1024
+    weight from memory.  Up to about 2000 rows at most sizes: 8 x 22016 x 4096 GLU 33 (55), 64 x
+    4096 x 14336 29 (39), 192 x 4096 x 4096 21 (32), 512 x 6288 x 2048 22 (24), 1739 x 4096 x 11008 130
+    (148).  Without ``adds`` not: up to 32 rows of medium weights, 8 x 6144 x 4096 16.8 (15.4), 16 x 4096 x
+    8192 19.1 (16.5), or very large ones, 24 x 128256 x 4096 195 (185) when all tiles began at the same
+    column, or few outputs, 8 x 2048 x 8192 13.6 (12.7); where unsplit tiles leave half of the CUs idle, 61
+    x 4096 x 4096 17.1, in parts as fast as the library, 13.7 (14.3); weights that two tiles of rows
+    read, 96 x 12288 x 4096 34 (30).  The library has other sizes of its own beside slow ones, 190 x
+    6288 x 2048 16.7 (15.9), 160 x 6288 x 2048 15.0 (16.5): not told apart.  From 1024
     rows on (2048 with a GLU or ``adds``) it is 2 to 9% ahead where
     256 x 256 tiles fill their last round, 1400 x 32000 x 4096 287 (273), 5000 x 6144 x 4096 194 (188),
     7664 x 2048 x 8192 185 (172), 8131 x 4096 x 4096 185 (176), but not for the GLU, 7664 x 28672 x 4096 1259 (1376),

@@ -19,9 +19,9 @@
 // among them 663, the reads done at three quarters of a step 652.  Stores of whole lines past
 // the caches: 8131 x 28672 x 4096 1335 to 1299.
 //
-// Against the GEMM library (and the unit's own pass), us: 64 x 4096 x 14336 31 (41), 192 x 28672
-// x 4096 SwiGLU 58 (67), 192 x 4096 x 14336 46 (103), 512 x 4096 x 14336 67 (91), 1739 x 28672 x
-// 4096 SwiGLU 328 (417), 7664 x 28672 x 4096 SwiGLU 1259 (1376), 10000 x 4096 x 4096 244 (370).
+// Against the GEMM library (and the unit's own pass), us: 64 x 4096 x 14336 29 (39), 192 x 28672
+// x 4096 SwiGLU 54 (67), 192 x 4096 x 14336 40 (103), 512 x 4096 x 14336 67 (91), 1739 x 28672 x
+// 4096 SwiGLU 310 (417), 7664 x 28672 x 4096 SwiGLU 1259 (1376), 10000 x 4096 x 4096 244 (370).
 #include <math.h>
 
 #include "launch.h"
@@ -30,9 +30,26 @@
 #define CUS 256
 #define LDS_OF_A_CU 163840
 
+// n / by for n below 2^31 as a product (Granlund and Montgomery, 1994).  A division is about 30
+// instructions one after another, and a launch waited for four times five of them ahead of its
+// first and its last loads: 2048 x 2048 of 40 rows 8.8 us and now 8.3, 13 x 4096 x 4096 9.4 and 9.0, 61 x
+// 6144 x 4096 15.6 and 15.4; by divisions of 64 bits one more each took 2 to 3 us.
+struct Over {
+  unsigned by, mul, shift;
+};
+static Over over(unsigned by) {
+  unsigned shift = 0;
+  while ((1ull << shift) < by) ++shift;
+  return {by, (unsigned)(((1ull << 32) * ((1ull << shift) - by)) / by + 1), shift};
+}
+DEV int operator/(int n, const Over& d) {
+  return (int)((__umulhi((unsigned)n, d.mul) + (unsigned)n) >> d.shift);
+}
+
 struct LinearGrid {
   int tiles_m, tiles_n, band;
   int splits, each;  // parts of the inner dimension, chunks of one
+  Over step, tiles, per, high, low;  // workgroups, tiles, those of a band, rows of one, of the last
   uint64_t apart;    // chunks from where a tile begins to where its neighbour does, times 2^32
 };
 
@@ -48,17 +65,17 @@ struct LinearWork {
   DEV int64_t out_row(const LinearSpot&, int m) const { return m; }
   // XCDs have runs of a round's works, in bands of up to 8 tiles of rows beside each other
   DEV LinearSpot spot(int t) const {
-    const int tiles = grid.tiles_m * grid.tiles_n, chunks = a.K >> 6;
-    const int base = t / step * step, i = t - base;
+    const int chunks = a.K >> 6, base = t / grid.step * step, i = t - base;
     const int here = min(step, total - base), q = here >> 3, r = here & 7, xcd = i & 7;
     int id = base + (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (i >> 3);
-    const int part = grid.splits > 1 ? id / tiles : 0;
-    id -= part * tiles;
-    const int per = grid.band * grid.tiles_n, b = id / per, rest = id - b * per;
-    const int high = min(grid.band, grid.tiles_m - b * grid.band), column = rest / high;
+    const int part = grid.splits > 1 ? id / grid.tiles : 0;
+    id -= part * (int)grid.tiles.by;
+    const int b = id / grid.per, rest = id - b * (int)grid.per.by;
+    const Over& high = (b + 1) * grid.band <= grid.tiles_m ? grid.high : grid.low;
+    const int column = rest / high;
     const int first = part * grid.each, last = min(chunks, first + grid.each);
     const int at = first + (int)(column * grid.apart >> 32);
-    return {(b * grid.band + rest % high) * tm, a.M, column * tn, first, last, part, a.w, a.x, a.M,
+    return {(b * grid.band + rest - column * (int)high.by) * tm, a.M, column * tn, first, last, part, a.w, a.x, a.M,
             0, at};
   }
 };
@@ -111,33 +128,40 @@ static void launch(const LinearArgs& a, int splits, hipStream_t stream) {
   constexpr int TN = 32 * FN, TM = 32 * FM, LDS = 128 * (WS * TN + XS * TM);
   constexpr bool GLU = UNIT == LINEAR_SWIGLU || UNIT == LINEAR_GLU;
   static_assert(LDS <= LDS_OF_A_CU);
-  allow_lds<linear_kernel<FN, FM, WS, XS, UNIT, false>>(LDS);
-  allow_lds<linear_kernel<FN, FM, WS, XS, UNIT, true>>(LDS);
-  const int outs = GLU ? a.N / 2 : a.N, per = GLU ? TN / 2 : TN, chunks = a.K / 64;
-  LinearGrid g;
-  g.tiles_m = (a.M + TM - 1) / TM;
-  g.tiles_n = (outs + per - 1) / per;
-  const int bands = (g.tiles_m + 7) / 8;
-  g.band = (g.tiles_m + bands - 1) / bands;
-  g.each = (chunks + splits - 1) / splits;
-  g.splits = (chunks + g.each - 1) / g.each;
-  const int total = g.tiles_m * g.tiles_n * g.splits, fit = CUS * (LDS_OF_A_CU / LDS);
-  const int workgroups = total < fit ? total : fit;
-  // One tile of rows reads the weights once: past the caches, us: 13 x 28672 x 4096 SwiGLU 48.6 to
-  // 44.3, 13 x 12288 x 4096 22.5 to 20.9, 61 x 128256 x 4096 209 to 193, 13 x 17792 x 2048 19.4 to
-  // 18.6; weights of 33 MB are not worth it, 13 x 2048 x 8192 12.9 and 13.9
-  const bool once = g.tiles_m == 1 && (int64_t)a.N * a.K >= 32 << 20;
-  // Rows of a power of two lie 4 KB and more apart, so that their columns are in a few of the memory's
-  // channels, all of which are busy only if tiles are at different columns.  us, before and now: 61 x
-  // 28672 x 4096 SwiGLU 50.9 and 42.5, 13 x 28672 x 4096 47.0 and 39.5, 13 x 12288 x 4096 20.6 and
-  // 18.3, 61 x 20480 x 4096 44.5 and 42.1, 190 x 128256 x 4096 231 and 192; at K = 5120 or 3584 the
-  // same as before.  Weights in rows of 64 elements more give no less, for more memory; an eighth
-  // of K apart by XCD 1 to 5% less, by twos or fours of tiles nothing.  Parts are apart by themselves: 61 x
-  // 6144 x 4096 in 4 parts 14.0, in turns 14.9.
-  g.apart = once && g.splits == 1 ? ((uint64_t)chunks << 32) / g.tiles_n : 0;
-  auto kernel = once ? linear_kernel<FN, FM, WS, XS, UNIT, true>
-                     : linear_kernel<FN, FM, WS, XS, UNIT, false>;
-  kernel<<<dim3(workgroups), 256, LDS, stream>>>(a, g);
+  if constexpr (!(GLU && FN % 4)) {  // linear_fits()
+    allow_lds<linear_kernel<FN, FM, WS, XS, UNIT, false>>(LDS);
+    allow_lds<linear_kernel<FN, FM, WS, XS, UNIT, true>>(LDS);
+    const int outs = GLU ? a.N / 2 : a.N, per = GLU ? TN / 2 : TN, chunks = a.K / 64;
+    LinearGrid g;
+    g.tiles_m = (a.M + TM - 1) / TM;
+    g.tiles_n = (outs + per - 1) / per;
+    const int bands = (g.tiles_m + 7) / 8;
+    g.band = (g.tiles_m + bands - 1) / bands;
+    g.each = (chunks + splits - 1) / splits;
+    g.splits = (chunks + g.each - 1) / g.each;
+    const int total = g.tiles_m * g.tiles_n * g.splits, fit = CUS * (LDS_OF_A_CU / LDS);
+    const int workgroups = total < fit ? total : fit;
+    g.step = over(workgroups);
+    g.tiles = over(g.tiles_m * g.tiles_n);
+    g.per = over(g.band * g.tiles_n);
+    g.high = over(g.band);
+    g.low = over(g.tiles_m % g.band ? g.tiles_m % g.band : g.band);
+    // One tile of rows reads the weights once: past the caches, us: 13 x 28672 x 4096 SwiGLU 48.6 to
+    // 44.3, 13 x 12288 x 4096 22.5 to 20.9, 61 x 128256 x 4096 209 to 193, 13 x 17792 x 2048 19.4 to
+    // 18.6; weights of 33 MB are not worth it, 13 x 2048 x 8192 12.9 and 13.9
+    const bool once = g.tiles_m == 1 && (int64_t)a.N * a.K >= 32 << 20;
+    // Rows of a power of two lie 4 KB and more apart, so that their columns are in a few of the memory's
+    // channels, all of which are busy only if tiles are at different columns.  us, before and now: 61 x
+    // 28672 x 4096 SwiGLU 50.9 and 42.5, 13 x 28672 x 4096 47.0 and 39.5, 13 x 12288 x 4096 20.6 and
+    // 18.3, 61 x 20480 x 4096 44.5 and 42.1, 190 x 128256 x 4096 231 and 192; at K = 5120 or 3584 the
+    // same as before.  Weights in rows of 64 elements more give no less, for more memory; an eighth
+    // of K apart by XCD 1 to 5% less, by twos or fours of tiles nothing.  Parts are apart by themselves: 61 x
+    // 6144 x 4096 in 4 parts 14.0, in turns 14.9.
+    g.apart = once && g.splits == 1 ? ((uint64_t)chunks << 32) / g.tiles_n : 0;
+    auto kernel = once ? linear_kernel<FN, FM, WS, XS, UNIT, true>
+                       : linear_kernel<FN, FM, WS, XS, UNIT, false>;
+    kernel<<<dim3(workgroups), 256, LDS, stream>>>(a, g);
+  }
 }
 
 template <int UNIT>
@@ -149,53 +173,60 @@ static void sum(const LinearArgs& a, const void* parts, int splits, hipStream_t 
   kernel<<<dim3((a.M * outs / 8 + 255) / 256), 256, 0, stream>>>(a, (const float*)parts, count);
 }
 
+// step: us of a chunk
 struct Tile {
   int fn, fm, ws, xs;
+  double step;
 };
-// an odd number of pairs of fragments cannot hold gates and ups
-#define TILES(T) \
-  T(8, 8, 3, 2) T(8, 7, 3, 2) T(8, 6, 3, 2) T(8, 5, 3, 3) T(8, 4, 3, 4) \
-  T(4, 6, 4, 4) T(4, 4, 5, 5) T(4, 3, 5, 5) T(4, 2, 3, 3) T(4, 1, 4, 4)
-#define PLAIN_TILES(T) T(6, 4, 4, 4) T(2, 2, 5, 5) T(2, 1, 6, 6)
-#define SIZES(fn, fm, ws, xs) {fn, fm, ws, xs},
-static const Tile tiles[] = {TILES(SIZES) PLAIN_TILES(SIZES)};
-static constexpr int GLU_TILES = 10;
-
+// The rings' depths: 61 x 28672 x 4096 SwiGLU by 128 x 64 with 3 chunks of both 42.5, with 4 40.0;
+// 190 rows of it by 128 x 192 with 4 59.7, with 3 57.2
+#define TILES(T)                                                                          \
+  T(8, 8, 3, 2, 1.04) T(8, 7, 3, 2, 0.98) T(8, 6, 3, 2, 0.85) T(8, 5, 3, 3, 0.77)         \
+  T(8, 4, 3, 4, 0.71) T(4, 6, 3, 3, 0.56) T(4, 4, 5, 5, 0.48) T(4, 3, 5, 5, 0.41)         \
+  T(4, 2, 4, 4, 0.34) T(4, 1, 4, 4, 0.32) T(6, 4, 4, 4, 0.67) T(2, 2, 5, 5, 0.18)         \
+  T(2, 1, 6, 6, 0.16) T(4, 5, 4, 3, 0.52)
+#define SIZES(fn, fm, ws, xs, step) {fn, fm, ws, xs, step},
+static const Tile tiles[] = {TILES(SIZES)};
 static constexpr int TILE_COUNT = sizeof(tiles) / sizeof(Tile);
 
+// an odd number of pairs of fragments cannot hold gates and ups
 extern "C" bool linear_fits(int tile, bool glu) {
-  return tile >= 0 && tile < (glu ? GLU_TILES : TILE_COUNT);
+  return tile >= 0 && tile < TILE_COUNT && !(glu && tiles[tile].fn % 4);
 }
 
 // The tile and the parts that are expected to be the fastest, in us: the chunks of the busiest
-// CU, by its matrix cores or its LDS, beside the memory's time.  Fitted to 286 sizes of 8 to
-// 10000 rows, 2048 to 128256 outputs and 768 to 14336 inner elements; what it chooses is on
-// average 1% slower than the best of all tiles and parts, 12 to 19% where it is worst (64 x 4096 x
-// 4096: 16.4, best 13.8).
+// CU beside the memory's time, for the operands once and for what tiles read again, and a launch.  Fitted
+// to 754 sizes of 5 to 2100 rows, 2048 to 32000 outputs and 1280 to 14336 inner elements; what it chooses is
+// on average 1.1% slower than the best of all tiles and parts, 1.5% where the parts are added up
+// elsewhere, and 24% where it is worst.  With steps by the fragments alone, max(0.015 fn fm, 0.053
+// (fn + fm)), 1.7 and 3.2%: 190 x 4096 x 14336 into the norm 39.8 and now 35.3, 190 x 6144 x 4096 into
+// the rotation 22.9 and 21.2, 61 x 4096 x 4096 17.0 and 13.7.
 extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* splits) {
-  static const int parts[] = {1, 2, 3, 4, 6, 8, 12, 16};
+  static const int parts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
   const bool glu = unit == LINEAR_SWIGLU || unit == LINEAR_GLU;
   const int chunks = K / 64;
+  const double rows = 2.0 * M * K, weights = 2.0 * N * K;
   double best = 0;
   *tile = -1;
   for (int i = 0; i < TILE_COUNT; ++i) {
     const Tile& t = tiles[i];
     if (t.fm > 1 && (t.fm - 1) * 32 >= M) continue;  // rows of nothing
-    const int64_t grid = ((int64_t)M + 32 * t.fm - 1) / (32 * t.fm) *
-                         (((int64_t)N + 32 * t.fn - 1) / (32 * t.fn));
-    const double step = fmax(0.015 * t.fn * t.fm, 0.053 * (t.fn + t.fm));
+    const int64_t high = ((int64_t)M + 32 * t.fm - 1) / (32 * t.fm);
+    const int64_t wide = ((int64_t)N + 32 * t.fn - 1) / (32 * t.fn);
     for (int s : parts) {
-      if (s == 1 && glu && i >= GLU_TILES) continue;
-      if (s > 1 && (chunks < 4 * s || M > 2600 || grid * s > 4 * CUS)) break;
-      const int each = (chunks + s - 1) / s;
-      const int64_t works = grid * ((chunks + each - 1) / each);
+      if (s == 1 && !linear_fits(i, glu)) continue;
+      if (s > 1 && (chunks < 4 * s || M > 2600 || high * wide * s > 4 * CUS)) break;
+      const int each = (chunks + s - 1) / s, count = (chunks + each - 1) / each;
+      const int64_t works = high * wide * count;
       const double busiest =
-          (double)((works + CUS - 1) / CUS) * (each * step + 0.08 * t.fn * t.fm + 0.57);
-      const double sums = s > 1 ? 8.0 * s * M * N : 2.0 * M * N;
-      const double memory = (2.0 * N * K + 2.0 * M * K + sums) / 6.4e6;
-      const double us =
-          sqrt(busiest * busiest + memory * memory) +
-          (s > 1 ? (unit == LINEAR_PARTS ? 0.5 : 4.3) + sums / 21.7e6 : 0);
+          (double)((works + CUS - 1) / CUS) * (each * t.step + 0.09 * t.fn * t.fm + 0.09);
+      const double sums = (s > 1 ? 8.0 * count : glu ? 1.0 : 2.0) * M * N;
+      const double memory =
+          (weights + rows + sums) / 8.8e6 + (wide * rows + high * weights) / 160e6;
+      const double rest =
+          1.6 + (s > 1 ? (unit == LINEAR_PARTS ? 1.15 : 4.8) + sums / 72e6 : 0);
+      if (*tile >= 0 && fmax(busiest, memory) + rest >= best) continue;  // nor is the sum less
+      const double us = pow(pow(busiest, 1.36) + pow(memory, 1.36), 1 / 1.36) + rest;
       if (*tile >= 0 && us >= best) continue;
       best = us;
       *tile = i;
@@ -218,16 +249,13 @@ extern "C" void launch_linear(const LinearArgs* args, int unit, int tile, int sp
 #define LAUNCH_AS(n, m, ws_, xs_, u)                                       \
   if (kind == u && t.fn == n && t.fm == m && t.ws == ws_ && t.xs == xs_)   \
     launch<n, m, ws_, xs_, u>(a, splits, stream);
-#define LAUNCH_PLAIN(n, m, ws, xs)        \
+#define LAUNCH(n, m, ws, xs, step)        \
   LAUNCH_AS(n, m, ws, xs, LINEAR_PLAIN)   \
   LAUNCH_AS(n, m, ws, xs, LINEAR_BIAS)    \
-  LAUNCH_AS(n, m, ws, xs, LINEAR_PARTS)
-#define LAUNCH(n, m, ws, xs)              \
-  LAUNCH_PLAIN(n, m, ws, xs)              \
+  LAUNCH_AS(n, m, ws, xs, LINEAR_PARTS)   \
   LAUNCH_AS(n, m, ws, xs, LINEAR_SWIGLU)  \
   LAUNCH_AS(n, m, ws, xs, LINEAR_GLU)
   TILES(LAUNCH)
-  PLAIN_TILES(LAUNCH_PLAIN)
   if (splits > 1 && unit != LINEAR_PARTS) {
     a.out = args->out;
     unit == LINEAR_PLAIN    ? sum<LINEAR_PLAIN>(a, parts, splits, stream)

@@ -74,17 +74,15 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   const int slot = ((lane & 7) ^ (lane >> 3)) * 16;
   int vw[LW], vx[LX];  // this lane's rows
   // cursors of the loads: work, chunk, its last one, place in LDS; past the last work its
-  // chunks again.  In turn: its first chunk and the ones left
-  int tw = work.start, cw, ew, fw0 = 0, nw = 0, sw = 0;
-  int tx = work.start, cx, ex, fx0 = 0, nx = 0, sx = 0;
+  // chunks again.  In turn: the chunks left
+  int tw = work.start, cw, ew, w0, nw = 0, sw = 0;
+  int tx = work.start, cx, ex, x0, nx = 0, sx = 0;
   auto aim_w = [&](int t) {
     const LinearSpot spot = work.spot(t);
     cw = TURNS ? spot.at : spot.first;
     ew = spot.last;
-    if (TURNS) {
-      fw0 = spot.first;
-      nw = spot.last - spot.first;
-    }
+    w0 = spot.first;
+    if (TURNS) nw = ew - w0;
     bw = buffer(spot.w, a.N, a.w_stride, a.K);
 #pragma unroll
     for (int i = 0; i < LW; ++i) {
@@ -100,10 +98,8 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
     const LinearSpot spot = work.spot(t);
     cx = TURNS ? spot.at : spot.first;
     ex = spot.last;
-    if (TURNS) {
-      fx0 = spot.first;
-      nx = spot.last - spot.first;
-    }
+    x0 = spot.first;
+    if (TURNS) nx = ex - x0;
     bx = buffer(spot.x, spot.x_rows, a.x_stride, a.K);
 #pragma unroll
     for (int i = 0; i < LX; ++i) {
@@ -122,19 +118,27 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
   auto next_w = [&]() {
     sw = sw == (WS - 1) * SW ? 0 : sw + SW;
     ++cw;
-    if (TURNS && cw == ew) cw = fw0;
-    if (TURNS ? --nw == 0 : cw == ew) {
-      tw = work.next(tw);
-      aim_w(tw);
+    const bool end = TURNS ? --nw == 0 : cw == ew;
+    if (cw == ew) cw = w0;
+    if (end) {
+      const int t = work.next(tw);
+      if (t != tw)
+        aim_w(tw = t);
+      else if (TURNS)
+        nw = ew - w0;
     }
   };
   auto next_x = [&]() {
     sx = sx == (XS - 1) * SX ? 0 : sx + SX;
     ++cx;
-    if (TURNS && cx == ex) cx = fx0;
-    if (TURNS ? --nx == 0 : cx == ex) {
-      tx = work.next(tx);
-      aim_x(tx);
+    const bool end = TURNS ? --nx == 0 : cx == ex;
+    if (cx == ex) cx = x0;
+    if (end) {
+      const int t = work.next(tx);
+      if (t != tx)
+        aim_x(tx = t);
+      else if (TURNS)
+        nx = ex - x0;
     }
   };
 

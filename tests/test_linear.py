@@ -7,7 +7,7 @@ from torch.utils.flop_counter import FlopCounterMode
 from agentcontrolplane_amd import ops
 from agentcontrolplane_amd.engine.config import ClampedGluSpec
 
-TILES = range(13)
+TILES = range(14)
 
 
 def operands(m, n, k, seed, strided=False):
@@ -82,7 +82,7 @@ def test_linear_gated(tile, m, n, k, splits, unit):
 
 #: outputs and rows of the tiles
 SIZES = [(256, 256), (256, 224), (256, 192), (256, 160), (256, 128), (128, 192), (128, 128),
-         (128, 96), (128, 64), (128, 32), (192, 128), (64, 64), (64, 32)]
+         (128, 96), (128, 64), (128, 32), (192, 128), (64, 64), (64, 32), (128, 160)]
 
 
 @pytest.mark.gpu
