@@ -16,14 +16,12 @@
 // token-id order, and walks the stripe with the target: the inverse CDF runs in token-id order
 // and draws match the fp32 oracle (ops/reference.py softmax_sample) for a given uniform.  The
 // weights of 64 tokens of every stripe are made at a time by all threads and added up by one
-// thread a stripe, so that the order of the sums does not depend on the threads.
+// thread a stripe, by fours in fp32 and those in 64 bits, so that all the ways a row can take agree.
 //
-// A workgroup a row is bound by its passes over the row.  190 rows of 128256 in fp32, other logits each
-// time, whole calls: 25 us greedy, 48 plain, 79 top-k, 95 top-p, 135 both (26, 58, 97, 168 and 238 with
-// calls of functions, which take a row and LDS by reference: their loads and atomics then go by
-// unknown memory and wait for both kinds); before 315,
-// 428, 1135, 1305 and 1978 (thresholds by three histograms of key bits, whose few buckets met
-// nearly all atomics, walked by one thread; draws by strides of a thread).  Floating masses
+// Rows of whole units by one workgroup take another way, by units (below), and this one where that does
+// not fit: 190 rows of 128256 in fp32, other logits each time, whole calls: 25 us greedy, 48 plain, 79
+// top-k, 95 top-p, 135 both (26, 58, 97, 168 and 238 with calls of functions, which take a row and LDS by
+// reference: their loads and atomics then go by unknown memory and wait for both kinds).  Floating masses
 // instead of whole ones in the histogram took as long, a shared list of the bucket 25 us more.
 //
 // Semantics match the oracle:
@@ -45,6 +43,17 @@
 #define KEYS 2048       // of the list of a row in chunks
 #define RANKED 320      // of them at most are compared with one another
 
+#define HELD 16      // units of a thread in registers
+#define STREAM 2     // others asked for ahead
+#define UNIT_KEYS 4096
+#define UNIT_BUCKETS 512
+#define PARTS 128    // of a bucket
+#define PER_OCTAVE 16
+#define PER_LOGIT 8  // likewise, of a top-k
+// beyond it more keys are within the masses' error than the list takes: normal logits 3000 at 0.99 of
+// 128256 and 4400 of 152064
+#define MOST_P(V) (1.f - (V) * 7.6e-8f)
+
 // order-preserving float -> uint32 key
 __device__ __forceinline__ uint32_t f2key(float x) {
   uint32_t u = __float_as_uint(x);
@@ -59,6 +68,24 @@ __device__ __forceinline__ float ldf(const float* p) { return *p; }
 __device__ __forceinline__ float ldf(const bf16_t* p) { return bf2f(*p); }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Tokens of a stripe, in whole fours of the row
+__device__ __forceinline__ int stripe_tokens(int V) {
+  return ((V + STRIPES - 1) / STRIPES + 3) & ~3;
+}
+// Weights are added up by fours, those in 64 bits
+__device__ __forceinline__ float sum_of_four(float a, float b, float c, float d) {
+  return (a + c) + (b + d);
+}
+// The token of a four whose weight takes ``before`` beyond target, or the last one of any weight
+__device__ __forceinline__ int token_of_four(const float* w, double before, double target) {
+  int last = 0;
+  for (int e = 0; e < 4; ++e) {
+    if (w[e] > 0.f) last = e;
+    if ((before += w[e]) > target) return e;
+  }
+  return last;
+}
 
 // Threads of a workgroup, and tokens of a stripe that are summed at a time.  With 1024 threads and
 // 160 KB a CU has one row, and each step of a row ends in a wait for 16 waves: small vocabularies
@@ -80,13 +107,21 @@ struct Shared : F {
     uint32_t list[LIST][F::WG];
     float tile[2][STRIPES][F::TILE + 4];
     float buffer[2 * STRIPES * (F::TILE + 4)];  // of the drawn stripe
+    // a row's by units, by lanes, so that no two lanes of a wave meet: count, and parts of a bucket
+    alignas(16) uint32_t column[F::WG < 1024 ? 1 : UNIT_BUCKETS][64];
     struct {
-      alignas(16) uint32_t key[KEYS];  // of a row in chunks
-      unsigned long long key_mass[KEYS];
+      alignas(16) uint32_t key[UNIT_KEYS];  // of a row in chunks, or by units
+      unsigned long long key_mass[UNIT_KEYS];
+      int key_wave[F::WG < 1024 ? 1 : UNIT_KEYS];
+      alignas(16) uint32_t sub_key[RANKED + 4];
+      unsigned long long sub_mass[RANKED + 4];
+      unsigned long long wave_units[F::WAVES];
+      // of the drawn wave
+      double unit_sum[F::WG < 1024 ? 1 : MOST_VOCAB / 4 / F::WAVES + 64];
+      double turn_sum[F::WG < 1024 ? 1 : MOST_VOCAB / 256 / F::WAVES + 1];
     };
   };
-  float stripe[STRIPES], cdf[STRIPES + 1];
-  double wave[F::WAVES];
+  double stripe[STRIPES], cdf[STRIPES + 1], wave[F::WAVES];
   float red[F::WAVES];
   int red_i[F::WAVES], red_odd[F::WAVES];
   int n, pick;
@@ -107,9 +142,9 @@ struct Row {
   const T* x;
   const uint8_t* mask;  // or null
   int V;
-  float m, invT;
+  float m, invT, scale;  // the largest logit, 1 / temperature, that in octaves
 
-  __device__ float weight(float v) const { return __expf((v - m) * invT); }
+  __device__ float weight(float v) const { return __builtin_amdgcn_exp2f((v - m) * scale); }
 
   // f(token, logit) for every allowed token, a thread's in rising order
   template <typename F>
@@ -254,6 +289,29 @@ INLINE double block_total(S& s, double v) {
   return t;
 }
 
+// Sum over the threads before, and of all
+template <typename S>
+INLINE double scan_block(S& s, double v, double* all) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  double upto = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double w = __shfl_up(upto, off, 64);
+    if (lane >= off) upto += w;
+  }
+  if (lane == 63) s.wave[wid] = upto;
+  __syncthreads();
+  double before = 0.0, total = 0.0;
+#pragma unroll 2
+  for (int i = 0; i < S::WAVES; ++i) {
+    if (i == wid) before = total;
+    total += s.wave[i];
+  }
+  __syncthreads();
+  *all = total;
+  return before + upto - v;
+}
+
 // The largest of the threads' logits, the lowest token among equals, whether one is odd
 template <typename S>
 INLINE void block_max(S& s, float& mx, int& best, int& odd) {
@@ -379,39 +437,39 @@ struct SampleArgs {
 template <typename T, int WG>
 INLINE Row<T, WG> row_of(const SampleArgs& a, int n) {
   const bool masked = a.mask && a.mask_map && a.mask_map[n] >= 0;
-  const float temp = a.temps[n];
+  const float temp = a.temps[n], invT = temp <= 0.f ? 1.f : 1.f / temp;
   return {(const T*)a.logits + (int64_t)n * a.V,
-          masked ? a.mask + (int64_t)a.mask_map[n] * a.V : nullptr, a.V, 0.f,
-          temp <= 0.f ? 1.f : 1.f / temp};
+          masked ? a.mask + (int64_t)a.mask_map[n] * a.V : nullptr, a.V, 0.f, invT,
+          invT * 1.44269504f};
 }
 
 // ---- inverse-CDF draw in token-id order from the stripes' sums, ``mine`` of the t-th thread's
 template <typename S, typename R>
 INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin,
-                     float mine) {
+                     double mine) {
   constexpr int WG = S::WG;
-  const int t = threadIdx.x, V = row.V, stride = (V + STRIPES - 1) / STRIPES;
+  const int t = threadIdx.x, V = row.V, stride = stripe_tokens(V);
   if (t < STRIPES) s.stripe[t] = mine;
   if (t == 0) s.pick = s.n = -1;
   __syncthreads();
   constexpr int STEP = 32;  // one thread's LDS reads in flight
   if (t == 0) {
-    float sum = 0.f;
-    s.cdf[0] = 0.f;
-    for (int i = 0; i < STRIPES; i += STEP) {
-      float w[STEP];
+    double sum = 0.0;
+    s.cdf[0] = 0.0;
+    for (int i = 0; i < STRIPES; i += STEP / 2) {
+      double w[STEP / 2];
 #pragma unroll
-      for (int e = 0; e < STEP; ++e) w[e] = s.stripe[i + e];
+      for (int e = 0; e < STEP / 2; ++e) w[e] = s.stripe[i + e];
 #pragma unroll
-      for (int e = 0; e < STEP; ++e) s.cdf[i + e + 1] = sum += w[e];
+      for (int e = 0; e < STEP / 2; ++e) s.cdf[i + e + 1] = sum += w[e];
     }
   }
   __syncthreads();
-  const float target = a.uniforms[n_row] * s.cdf[STRIPES];
+  const double target = (double)a.uniforms[n_row] * s.cdf[STRIPES];
   // exactly one stripe satisfies prefix <= target < prefix + mine
   // (mine > 0 guaranteed for the owner since the CDF strictly increases
   // across it); fp edge cases fall through to the fallback below
-  if (t < STRIPES && mine > 0.f && s.cdf[t] <= target && target < s.cdf[t + 1]) s.n = t;
+  if (t < STRIPES && mine > 0.0 && s.cdf[t] <= target && target < s.cdf[t + 1]) s.n = t;
   __syncthreads();
   const int n = s.n;
   __syncthreads();
@@ -436,19 +494,26 @@ INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t km
     if (last >= 0) atomicMax(&s.pick, last);
     __syncthreads();
     if (t == 0) {
-      float cum = s.cdf[n];
-      int first = STEP;
-      for (int j = 0; j < here && first == STEP; j += STEP) {
-        float w[STEP], upto = cum;
+      double cum = s.cdf[n];
+      int first = -1;
+      for (int j = 0; j < here && first < 0; j += STEP) {
+        float w[STEP], fours[STEP / 4];
+        double upto = cum;
 #pragma unroll
-        for (int e = 0; e < STEP; e += 4) *(float4*)(w + e) = *(const float4*)(buf + j + e);
-#pragma unroll
-        for (int e = 0; e < STEP; ++e) upto += w[e];
+        for (int e = 0; e < STEP; e += 4) {
+          *(float4*)(w + e) = *(const float4*)(buf + j + e);
+          fours[e / 4] = sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
+          upto += fours[e / 4];
+        }
         if (!(upto <= target))  // the same sums again: weights are not negative
-          for (int e = 0; e < STEP && first == STEP; ++e)
-            if ((cum += buf[j + e]) > target) first = e;
+#pragma unroll
+          for (int g = 0; g < STEP / 4; ++g) {
+            if (first < 0 && cum + fours[g] > target)
+              first = 4 * g + token_of_four(w + 4 * g, cum, target);
+            cum += fours[g];
+          }
         cum = upto;
-        if (first < STEP) s.pick = i0 + j + first;
+        if (first >= 0) s.pick = i0 + j + first;
       }
     }
   }
@@ -507,9 +572,9 @@ __device__ __forceinline__ bool left_whole(const RowPlan& plan) {
 struct RowState {
   RowPlan plan;
   double rest[MOST_CHUNKS];
+  double stripe[STRIPES];
   float chunk_max[MOST_CHUNKS];
   int chunk_best[MOST_CHUNKS], chunk_odd[MOST_CHUNKS];
-  float stripe[STRIPES];
   uint32_t list[KEYS];
   uint32_t count[FIRST];
   unsigned long long mass[FIRST];
@@ -541,7 +606,7 @@ __device__ __forceinline__ Chunk chunk_of(const SampleArgs& a, int chunks) {
   Chunk c;
   c.row = blockIdx.x / chunks;
   c.at = blockIdx.x - c.row * chunks;
-  c.stride = (a.V + STRIPES - 1) / STRIPES;
+  c.stride = stripe_tokens(a.V);
   c.stripes = STRIPES / chunks;
   c.i0 = min(a.V, c.at * c.stripes * c.stride);
   c.i1 = min(a.V, c.i0 + c.stripes * c.stride);
@@ -737,7 +802,8 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, Row
   const float least = key2f(kmin);
   const bool by_value = kmin == 0 || (least == least && least != 0.f);
   const float from = kmin == 0 ? -INFINITY : least;
-  float ahead[MOST], mine = 0.f;
+  float ahead[MOST];
+  double mine = 0.0;
   auto fetch = [&](int j0) {
 #pragma unroll
     for (int k = 0; k < MOST; ++k)
@@ -759,11 +825,15 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, Row
     if (j0 + TILE < c.stride) fetch(j0 + TILE);
     __syncthreads();  // the other tile is added up before it is written again
     if (t < c.stripes) {
-      float4 w[TILE / 4];
+      constexpr int FOURS = TILE < 32 ? TILE / 4 : 8;
+#pragma unroll 1
+      for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
+        float4 w[FOURS];
 #pragma unroll
-      for (int j = 0; j < TILE / 4; ++j) w[j] = *(const float4*)&tile[t][4 * j];
+        for (int j = 0; j < FOURS; ++j) w[j] = *(const float4*)&tile[t][4 * (j0 + j)];
 #pragma unroll
-      for (int j = 0; j < TILE / 4; ++j) mine = mine + w[j].x + w[j].y + w[j].z + w[j].w;
+        for (int j = 0; j < FOURS; ++j) mine += sum_of_four(w[j].x, w[j].y, w[j].z, w[j].w);
+      }
     }
   }
   if (t < c.stripes) state.stripe[c.at * c.stripes + t] = mine;
@@ -771,7 +841,7 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, Row
 
 struct DrawShared : ChunkForm {
   alignas(16) float buffer[MOST_VOCAB / STRIPES + 64];
-  float stripe[STRIPES], cdf[STRIPES + 1];
+  double stripe[STRIPES], cdf[STRIPES + 1];
   int n, pick;
 };
 
@@ -795,19 +865,20 @@ __global__ __launch_bounds__(256) void draw_kernel(const SampleArgs a, const Row
 // least one if rounding lets none do so.  A thread compares its key with all others, which takes
 // 33 ns a key; the two rounds of split_keys take about 12 us whatever the list: RANKED keys.
 template <bool BY_MASS, typename S>
-INLINE uint32_t rank_keys(S& s, int n, double above, double target) {
+INLINE uint32_t rank_keys(S& s, const uint32_t* keys, const unsigned long long* masses, int n,
+                          double above, double target) {
   if (threadIdx.x == 0) s.lo = 0xffffffffu;
   __syncthreads();
   uint32_t least = 0xffffffffu, at = 0;
   bool found = false;
   for (int i = threadIdx.x; i < n; i += S::WG) {
-    const uint32_t key = s.key[i];
+    const uint32_t key = keys[i];
     unsigned long long higher = 0, same = 0;
     for (int j = 0; j < n; j += 4) {
-      const u32x4 k = *(const u32x4*)&s.key[j];
+      const u32x4 k = *(const u32x4*)&keys[j];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {  // the units behind the last key are 0
-        const unsigned long long w = BY_MASS ? s.key_mass[j + e] : j + e < n;
+        const unsigned long long w = BY_MASS ? masses[j + e] : j + e < n;
         higher += k[e] > key ? w : 0;
         same += k[e] == key ? w : 0;
       }
@@ -835,11 +906,10 @@ INLINE uint32_t rank_keys(S& s, int n, double above, double target) {
 
 // The least kept key from a row's list of at most KEYS
 template <typename S, typename R>
-INLINE uint32_t least_of_list(S& s, const RowState& state, const RowPlan& plan,
-                                  const Wants& want, const R& row) {
-  const int n = plan.n;
+INLINE uint32_t least_of_list(S& s, const uint32_t* list, int n, double above, double target,
+                              const Wants& want, const R& row) {
   for (int i = threadIdx.x; i < (n + 3) / 4 * 4; i += S::WG) {
-    const uint32_t key = i < n ? state.list[i] : 0;
+    const uint32_t key = i < n ? list[i] : 0;
     s.key[i] = key;
     s.key_mass[i] = i < n && want.by_p ? units(row.weight(key2f(key))) : 0;
   }
@@ -867,42 +937,70 @@ INLINE uint32_t least_of_list(S& s, const RowState& state, const RowPlan& plan,
   };
   auto find = [&](auto by_mass, double above, double target) {
     constexpr bool BY_MASS = decltype(by_mass)::value;
-    return n <= RANKED ? rank_keys<BY_MASS>(s, n, above, target)
-                       : split_keys<BY_MASS>(s, row, lo, hi, above, target, each_key);
+    if (n <= RANKED) return rank_keys<BY_MASS>(s, s.key, s.key_mass, n, above, target);
+    if constexpr (S::WG == 1024) {
+      // a round of split_keys(), after which its bucket has few: 500 keys 6 us, its two rounds 12
+      const int shift = hi - lo < SPLIT ? 0 : 32 - __builtin_clz(hi - lo) - 10;
+      for (int i = threadIdx.x; i < SPLIT; i += S::WG) s.mass[i] = 0;
+      if (threadIdx.x == 0) s.n = 0;
+      __syncthreads();
+      for (int i = threadIdx.x; i < n; i += S::WG)
+        atomicAdd(&s.mass[(hi - s.key[i]) >> shift], BY_MASS ? s.key_mass[i] : 1ull);
+      __syncthreads();
+      const double unit = BY_MASS ? UNIT : 1.0;
+      double all, mine = s.mass[threadIdx.x] * unit;
+      const double before = above + scan_block(s, mine, &all);
+      if (before < target && before + mine >= target) {
+        s.above = before;
+        s.n = 1 + (int)threadIdx.x;
+      }
+      __syncthreads();
+      const int bucket = s.n - 1;
+      const double sub_above = s.above;
+      __syncthreads();
+      if (threadIdx.x == 0) s.n = 0;
+      __syncthreads();
+      if (bucket >= 0) {
+        for (int i = threadIdx.x; i < n; i += S::WG)
+          if ((int)((hi - s.key[i]) >> shift) == bucket) {
+            const int at = atomicAdd(&s.n, 1);
+            if (at < RANKED) {
+              s.sub_key[at] = s.key[i];
+              s.sub_mass[at] = s.key_mass[i];
+            }
+          }
+        __syncthreads();
+        const int few = s.n;
+        if (few <= RANKED) {
+          if (threadIdx.x < 4) {
+            s.sub_key[few + threadIdx.x] = 0;
+            s.sub_mass[few + threadIdx.x] = 0;
+          }
+          __syncthreads();
+          return rank_keys<BY_MASS>(s, s.sub_key, s.sub_mass, few, sub_above, target);
+        }
+        __syncthreads();
+      }
+    }
+    return split_keys<BY_MASS>(s, row, lo, hi, above, target, each_key);
   };
-  if (!want.by_k) return find(std::true_type(), plan.above, plan.target);
-  const uint32_t kmin = find(std::false_type(), plan.above, plan.target);
+  if (!want.by_k) return find(std::true_type(), above, target);
+  const uint32_t kmin = find(std::false_type(), above, target);
   if (!want.by_p) return kmin;
   double kept = 0.0;  // the list has all that the first threshold keeps
   for (int i = threadIdx.x; i < n; i += S::WG)
     if (s.key[i] >= kmin) kept += s.key_mass[i] * UNIT;
-  const double target = (double)want.p * (float)block_total(s, kept);
-  if (target <= 0.0) return max(kmin, f2key(row.m));
-  return max(kmin, find(std::true_type(), 0.0, target));
+  const double of_kept = (double)want.p * (float)block_total(s, kept);
+  if (of_kept <= 0.0) return max(kmin, f2key(row.m));
+  return max(kmin, find(std::true_type(), 0.0, of_kept));
 }
 
-// ---- a row by one workgroup; of rows in CHUNKS the thresholds, and those rows that are left to it
-template <typename T, typename F, bool CHUNKS>
-__global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(const SampleArgs a,
-                                                                 RowState* states) {
-  constexpr int WG = F::WG, TILE = F::TILE;
-  __shared__ Shared<F> s;
-  const int n_row = blockIdx.x, t = threadIdx.x;
-  const Wants want = wants_of(a, n_row);
-  const int V = a.V;
-  Row<T, WG> row = row_of<T, WG>(a, n_row);
-  if (CHUNKS) {
-    RowState& state = states[n_row];
-    const RowPlan plan = state.plan;
-    if (want.greedy || plan.mode == NO_LIST) return;
-    if (!left_whole(plan)) {
-      row.m = plan.m;
-      const uint32_t least = least_of_list(s, state, plan, want, row);
-      if (t == 0) state.plan.kmin = least;
-      return;
-    }
-  }
-  const int stride = (V + STRIPES - 1) / STRIPES;
+// ---- a row by one workgroup, in as many passes over it as its thresholds call for
+template <typename T, typename S>
+INLINE void whole_row(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG>& row, int n_row) {
+  constexpr int WG = S::WG, TILE = S::TILE;
+  const int t = threadIdx.x, V = a.V;
+  const int stride = stripe_tokens(V);
 
   // ---- the largest allowed logit, the lowest token that has it, and whether all are numbers
   float mx = -3.4e38f;
@@ -959,15 +1057,16 @@ __global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(const SampleArg
   const float least = key2f(kmin);
   const bool by_value = kmin == 0 || (least == least && least != 0.f);
   const float from = kmin == 0 ? -INFINITY : least;
-  const bool even = V == STRIPES * stride;  // no stripe is shorter
-  float mine = 0.f;
+  double mine = 0.0;
   fetch(0);
   for (int j0 = 0; j0 < stride; j0 += TILE) {
     float(*tile)[TILE + 4] = s.tile[j0 / TILE % 2];
-    if (even && by_value && plain && !row.mask && j0 + TILE <= stride) {
+    if (by_value && plain && !row.mask && j0 + TILE <= stride) {
 #pragma unroll
-      for (int k = 0; k < PER; ++k)
-        tile[k * ROWS + r][c] = ahead[k] >= from ? row.weight(ahead[k]) : 0.f;
+      for (int k = 0; k < PER; ++k) {
+        const bool in = ahead[k] >= from && k * ROWS * stride + j0 + i_first < V;
+        tile[k * ROWS + r][c] = in ? row.weight(ahead[k]) : 0.f;
+      }
     } else {
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
@@ -980,14 +1079,436 @@ __global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(const SampleArg
     if (j0 + TILE < stride) fetch(j0 + TILE);
     __syncthreads();  // the other tile is added up before it is written again
     if (t < STRIPES) {
-      float4 w[TILE / 4];
+      constexpr int FOURS = TILE < 32 ? TILE / 4 : 8;
+#pragma unroll 1
+      for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
+        float4 w[FOURS];
 #pragma unroll
-      for (int j = 0; j < TILE / 4; ++j) w[j] = *(const float4*)&tile[t][4 * j];
+        for (int j = 0; j < FOURS; ++j) w[j] = *(const float4*)&tile[t][4 * (j0 + j)];
 #pragma unroll
-      for (int j = 0; j < TILE / 4; ++j) mine = mine + w[j].x + w[j].y + w[j].z + w[j].w;
+        for (int j = 0; j < FOURS; ++j) mine += sum_of_four(w[j].x, w[j].y, w[j].z, w[j].w);
+      }
     }
   }
   draw(s, a, row, n_row, kmin, mine);
+}
+
+// ---- a row by one workgroup, by units of 16 bytes
+//
+// A wave owns consecutive units, 64 a turn, and keeps the first HELD turns in registers (half of a row
+// of 128256 in fp32); the rest comes from memory in every pass.  An instruction an element is about 1 us a
+// pass for 16 waves, and reading a row 16 to 19, so both count:
+//   1 the largest logit, by three-way maxima; a greedy row's is found again in its unit
+//   2 for a threshold, a histogram over the distance to it, 16 buckets an octave of the weight or finer:
+//     per bucket and lane the count and the sum of the distances within it, in one word, so that no
+//     two lanes of a wave meet (64-bit atomics on one table took 75 us instead of 10).  A bucket's
+//     mass is known to 4e-4 from both, so which buckets the boundary can be in, and no weight is made
+//   3 the weights above those buckets in a thread's own sum, the keys in them into a list, from which the
+//     least kept key follows exactly
+// The draw goes to the wave that has the target, then to its turn, a unit, a token, in token-id order.
+// 190 rows of 128256 in fp32, whole_row() and this, us: greedy 24.6 and 22.5, plain 48 and 33, top-k 80 and
+// 55, top-p 95 and 72, both 135 and 60, top-p 0.9 at a temperature of 6.4 100 and 74; bf16 22 and 14, 46 and
+// 24, 70 and 45, 92 and 67, 118 and 50; 32000 in fp32 10 and 8.8, 21 and 13, 35 and 25, 42 and 33, 58 and 31.
+// Without HELD plain rows take 41, with more registers spill; 4 units ahead instead of 2 as long.
+// A row that this does not fit is whole_row()'s: one of no whole units, logits that are no numbers, a
+// boundary among more keys than the list has or beyond the last bucket, a top-p beyond MOST_P.
+template <typename T, bool MASKED>
+struct Units {
+  static constexpr int N = 16 / sizeof(T);
+  const char* x;
+  const uint8_t* mask;      // or null, MASKED
+  int count, first, turns;  // units of the row, the wave's first one and its turns of 64
+
+  DEV static float at(const u32x4& v, int e) {
+    const uint32_t bits = N == 4 ? v[e & 3] : (e & 1) ? v[e >> 1] & 0xffff0000u : v[e >> 1] << 16;
+    return __uint_as_float(bits);
+  }
+  // the last one in place of units beyond it
+  DEV u32x4 load(int u) const { return *(const u32x4*)(x + (uint32_t)min(u, count - 1) * 16u); }
+  // units beyond the last one, and tokens that are not allowed, are logits of no weight; ``some``:
+  // there may be units beyond
+  DEV void clear(u32x4& v, int u, bool some) const {
+    if (some && u >= count) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) v[d] = N == 4 ? 0xff800000u : 0xff80ff80u;
+    }
+    if (MASKED && mask) {
+      const uint8_t* const allowed = mask + min(u, count - 1) * N;
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        if (allowed[e]) continue;
+        if (N == 4)
+          v[e & 3] = 0xff800000u;
+        else
+          v[e >> 1] = (e & 1) ? (v[e >> 1] & 0xffffu) | 0xff800000u : (v[e >> 1] & 0xffff0000u) | 0xff80u;
+      }
+    }
+  }
+  // without a branch, behind which a load would have to be waited for
+  DEV u32x4 turn(int a) const { return load(first + a * 64 + (int)(threadIdx.x & 63)); }
+  DEV void clear_turn(u32x4& v, int a) const {
+    const int u = first + a * 64;
+    clear(v, u + (int)(threadIdx.x & 63), u + 64 > count);
+  }
+  // f(unit, turn) of all turns, the held ones from registers.  The first time units beyond the last one
+  // are that one again
+  template <bool FIRST_TIME, typename F>
+  DEV void each(u32x4 (&held)[HELD], F f) const {
+    u32x4 next[STREAM];
+#pragma unroll
+    for (int g = 0; g < STREAM; ++g) next[g] = turn(HELD + g);
+#pragma unroll
+    for (int a = 0; a < HELD; ++a)
+      if (a < turns) {
+        if (FIRST_TIME && MASKED) clear_turn(held[a], a);
+        f(held[a], a);
+        if (FIRST_TIME && !MASKED) clear_turn(held[a], a);
+      }
+    for (int a = HELD; a < turns; a += STREAM) {
+#pragma unroll
+      for (int g = 0; g < STREAM; ++g) {
+        u32x4 v = next[g];
+        next[g] = turn(a + STREAM + g);
+        if (a + g < turns) {
+          if (!FIRST_TIME || MASKED) clear_turn(v, a + g);
+          f(v, a + g);
+        }
+      }
+    }
+  }
+};
+
+DEV float max3(float a, float b, float c) {
+  asm("v_max3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+  return a;
+}
+DEV float min3(float a, float b, float c) {
+  asm("v_min3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+  return a;
+}
+
+// The least of the threads' logits
+template <typename S>
+INLINE float block_least(S& s, float v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off, 64));
+  if ((threadIdx.x & 63) == 0) s.red[threadIdx.x >> 6] = v;
+  __syncthreads();
+#pragma unroll 4
+  for (int w = 0; w < S::WAVES; ++w) v = fminf(v, s.red[w]);
+  __syncthreads();
+  return v;
+}
+
+// The first lane whose sum with those before it exceeds target, and the sum before it; 64: none
+INLINE int first_above(double v, double target, double* before) {
+  const int lane = threadIdx.x & 63;
+  double upto = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double w = __shfl_up(upto, off, 64);
+    if (lane >= off) upto += w;
+  }
+  const unsigned long long above = __ballot(v > 0.0 && upto > target);
+  if (!above) return 64;
+  const int at = __builtin_ctzll(above);
+  *before = __shfl(upto - v, at, 64);
+  return at;
+}
+
+template <typename T, bool MASKED, typename S>
+INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG>& row, int n_row) {
+  using U = Units<T, MASKED>;
+  constexpr int N = U::N, WAVES = S::WAVES;
+  const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6), V = a.V;
+  if (V % N || (uintptr_t)row.x % 16) return false;
+  if (!want.greedy && want.by_p && !(want.p > 0.f && (want.by_k || want.p <= MOST_P(V)))) return false;
+  U units_of;
+  units_of.x = (const char*)row.x;
+  units_of.mask = row.mask;
+  units_of.count = V / N;
+  units_of.turns = (units_of.count + 64 * WAVES - 1) / (64 * WAVES);
+  units_of.first = wid * units_of.turns * 64;
+  const bool cuts = want.by_k || want.by_p;
+  if (!want.greedy && cuts)
+    for (int i = t; i < UNIT_BUCKETS * 16; i += S::WG) ((u32x4*)s.column)[i] = u32x4{};
+  if (t == 0) s.n = 0;
+
+  // ---- 1
+  u32x4 held[HELD];
+#pragma unroll
+  for (int k = 0; k < HELD; ++k) held[k] = units_of.turn(k);
+  float mx = -3.4e38f, least = INFINITY;
+  int best = 1 << 30, odd = 0;
+  if (want.greedy) {
+    units_of.template each<true>(held, [&](const u32x4& v, int k) {
+      float y = -3.4e38f;
+#pragma unroll
+      for (int e = 0; e < N; e += 2) y = max3(y, U::at(v, e), U::at(v, e + 1));
+      if (y > mx) {
+        mx = y;
+        best = units_of.first + k * 64 + lane;
+      }
+    });
+    block_max(s, mx, best, odd);
+    if (t == 0) {
+      int at = 0;
+      if (best < units_of.count) {
+        u32x4 v = units_of.load(best);
+        units_of.clear(v, best, false);
+#pragma unroll
+        for (int e = N - 1; e >= 0; --e)
+          if (U::at(v, e) == mx) at = best * N + e;
+      }
+      a.out[n_row] = at;
+    }
+    return true;
+  }
+  unsigned long long odd_lanes = 0;
+  units_of.template each<true>(held, [&](const u32x4& v, int) {
+#pragma unroll
+    for (int e = 0; e < N; e += 2) {
+      const float x = U::at(v, e), y = U::at(v, e + 1);
+      mx = max3(mx, x, y);
+      least = min3(least, x, y);
+      odd_lanes |= __ballot(__builtin_isunordered(x, y));
+    }
+  });
+  odd = odd_lanes != 0;
+  block_max(s, mx, best, odd);
+  // top-k's buckets are of logits, so that no temperature takes the k-th beyond the last one
+  const float per_octave = row.scale;
+  float scale = want.by_k ? (float)PER_LOGIT / PER_OCTAVE : per_octave;
+  if (cuts) {
+    // finer ones where the row does not reach the last one
+    least = block_least(s, least);
+    const float span = (mx - least) * scale, most = UNIT_BUCKETS / PER_OCTAVE - 2;
+    if (!(span > 1e-20f)) return false;
+    if (span < most) scale *= most / span;
+    if (!(scale < 1e25f)) return false;
+  }
+  const float fine = scale * (PER_OCTAVE * PARTS), bucket_octaves = per_octave / scale / PER_OCTAVE;
+  if (odd || !(mx > -1e37f && mx < INFINITY) || !(per_octave < 1e20f && per_octave > 1e-20f)) return false;
+  row.m = mx;
+
+  // ---- 2: the buckets lo .. hi - 1 that the boundary can be in
+  int lo = 0, hi = 0;
+  double k_above = 0.0;
+  if (cuts) {
+    uint32_t* const mine = &s.column[0][lane];
+    units_of.template each<false>(held, [&](const u32x4& v, int) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        const float d = (mx - U::at(v, e)) * fine;
+        if (d < (float)(UNIT_BUCKETS * PARTS)) {  // beyond 32 octaves all weigh less than the slack
+          const uint32_t q = (uint32_t)d;
+          atomicAdd(mine + q / PARTS * 64, (uint32_t)(1 << 19) | (q % PARTS));
+        }
+      }
+    });
+    if (t == 0) s.lo = s.hi = UNIT_BUCKETS;
+    __syncthreads();
+    // two threads a bucket
+    static_assert(S::WG == 2 * UNIT_BUCKETS && MOST_VOCAB / 64 <= 1 << 13 && PARTS <= 128);
+    const int b = t >> 1;
+    uint32_t numbers = 0, parts = 0;
+#pragma unroll 4
+    for (int i = 0; i < 32; ++i) {
+      const uint32_t h = s.column[b][(i + lane) % 32 + (t & 1) * 32];
+      numbers += h >> 19;
+      parts += h & ((1 << 19) - 1);
+    }
+    numbers += __shfl_xor(numbers, 1);
+    parts += __shfl_xor(parts, 1);
+    const double n = t & 1 ? 0.0 : (double)numbers;
+    double after = 0.0, before = 0.0, all = 0.0;
+    if (want.by_k) {
+      // the bucket of the k-th; with both, all down to it are listed
+      before = scan_block(s, n, &all);
+      if (before < want.k && before + n >= want.k) {
+        s.hi = b + 1;
+        s.above = before;
+      }
+    } else {
+      // the mean of a bucket's weights, in units of that at its edge, by the mean of the distances
+      const double off =
+          n > 0.0 ? ((double)parts / n + 0.5) * (0.6931471806 / PARTS) * bucket_octaves : 0.0;
+      const double mass =
+          n * (1.0 - off + 0.5 * off * off) * (double)__builtin_amdgcn_exp2f(b * -bucket_octaves);
+      before = scan_block(s, mass, &all);
+      after = before + mass;
+      constexpr double SLACK = 5e-4;
+      const double low = (double)want.p * all * (1 - SLACK), high = (double)want.p * all * (1 + SLACK);
+      if (before * (1 + SLACK) < low && after * (1 + SLACK) >= low) s.lo = b;
+      if (before * (1 - SLACK) < high && after * (1 - SLACK) >= high) s.hi = b + 1;
+    }
+    __syncthreads();
+    hi = (int)s.hi;
+    lo = want.by_p ? (want.by_k ? 0 : (int)s.lo) : hi - 1;
+    k_above = want.by_k && !want.by_p ? s.above : 0.0;
+    // what is beyond the last bucket is not told apart
+    if (hi >= UNIT_BUCKETS || lo >= hi) return false;
+  }
+
+  // ---- 3
+  // as the buckets are, whose scale differs by a power of two
+  const float edge_lo = lo * (-1.f / PER_OCTAVE), edge_hi = hi * (-1.f / PER_OCTAVE);
+  double kept = 0.0, all = 0.0;
+  // not the differences of pass 2, which would be kept for it beside the logits
+  float top = mx;
+  asm volatile("" : "+v"(top));
+  auto weigh = [&](float x) { return __builtin_amdgcn_exp2f((x - top) * per_octave); };
+  auto add_fours = [](const float (&w)[N], double& to) {
+#pragma unroll
+    for (int e = 0; e < N; e += 4) to += (double)sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
+  };
+  if (!cuts) {
+    units_of.template each<false>(held, [&](const u32x4& v, int) {
+      float w[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) w[e] = weigh(U::at(v, e));
+      add_fours(w, kept);
+    });
+  } else {
+    units_of.template each<false>(held, [&](const u32x4& v, int) {
+      float w[N], in[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        const float x = U::at(v, e), z = (x - top) * scale;
+        w[e] = weigh(x);
+        in[e] = z > edge_lo ? w[e] : 0.f;
+        if (z > edge_hi && !(z > edge_lo)) {
+          const int at = atomicAdd(&s.n, 1);
+          if (at < UNIT_KEYS) {
+            s.key[at] = f2key(x);
+            s.key_wave[at] = wid;
+          }
+        }
+      }
+      add_fours(in, kept);
+      if (want.by_p) add_fours(w, all);
+    });
+  }
+  uint32_t kmin = 0;
+  if (t < WAVES) s.wave_units[t] = 0;
+  if (cuts) {
+    const double above = want.by_k ? k_above : block_total(s, kept);
+    const double target = want.by_k ? want.k : (double)want.p * block_total(s, all);
+    __syncthreads();
+    const int n = s.n;
+    if (n > UNIT_KEYS || n == 0 || !(above < target)) return false;
+    kmin = least_of_list(s, s.key, n, above, target, want, row);
+    // the least key of the list may be so because the list ends there
+    double sum = 0.0;
+    if (!want.by_k)
+      for (int i = t; i < n; i += S::WG) sum += s.key_mass[i] * UNIT;
+    if (!want.by_k && above + block_total(s, sum) < target) return false;
+    for (int i = t; i < n; i += S::WG)
+      if (s.key[i] >= kmin) atomicAdd(&s.wave_units[s.key_wave[i]], units(row.weight(key2f(s.key[i]))));
+  }
+  __syncthreads();
+
+  // ---- the draw: the wave, then 64 units, a unit, a token
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) kept += __shfl_xor(kept, off, 64);
+  if (lane == 0) s.wave[wid] = kept + s.wave_units[wid] * UNIT;
+  __syncthreads();
+  double total = 0.0;
+#pragma unroll 2
+  for (int i = 0; i < WAVES; ++i) total += s.wave[i];
+  if (!(total > 0.0 && total < 1e30)) return false;
+  const double target = (double)a.uniforms[n_row] * total;
+  double before = 0.0;
+  int drawn = -1, last = 0;
+#pragma unroll 1
+  for (int i = 0; i < WAVES && drawn < 0; ++i) {
+    const double w = s.wave[i];
+    if (w > 0.0) {
+      last = i;
+      if (before + w > target) drawn = i;
+    }
+    if (drawn < 0) before += w;
+  }
+  if (drawn < 0) {
+    drawn = last;  // its last token
+    before = -1e300;
+  }
+  const double rest = before > -1e299 ? target - before : 1e300;
+  auto weights_of = [&](int u, float (&w)[N]) {
+    u32x4 v = units_of.load(u);
+    units_of.clear(v, u, true);
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const float x = U::at(v, e);
+      w[e] = f2key(x) >= kmin ? weigh(x) : 0.f;
+    }
+  };
+  const int first = drawn * units_of.turns * 64;
+  for (int k = wid; k < units_of.turns; k += WAVES) {
+    float w[N];
+    weights_of(first + k * 64 + lane, w);
+    double sum = 0.0;
+    add_fours(w, sum);
+    s.unit_sum[k * 64 + lane] = sum;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    if (lane == 0) s.turn_sum[k] = sum;
+  }
+  __syncthreads();
+  if (wid) return true;
+  double ahead = 0.0, at_turn = 0.0;
+  const double mine = lane < units_of.turns ? s.turn_sum[lane] : 0.0;
+  int k = first_above(mine, rest, &at_turn), u;
+  const unsigned long long some = __ballot(mine > 0.0);
+  bool end = k == 64;
+  if (end) k = some ? 63 - __builtin_clzll(some) : 0;
+  const double in_turn = s.unit_sum[k * 64 + lane];
+  u = end ? 64 : first_above(in_turn, rest - at_turn, &ahead);
+  const unsigned long long these = __ballot(in_turn > 0.0);
+  if (u == 64) {
+    end = true;
+    u = these ? 63 - __builtin_clzll(these) : 0;
+  }
+  if (lane == 0) {
+    float w[N];
+    const int unit = first + k * 64 + u;
+    weights_of(unit, w);
+    double upto = at_turn + ahead;
+    int pick = -1, last = 0;
+#pragma unroll
+    for (int e = 0; e < N; e += 4) {
+      const float four = sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
+      if (four > 0.f) last = e + token_of_four(w + e, 0.0, INFINITY);
+      if (pick < 0 && !end && upto + four > rest) pick = e + token_of_four(w + e, upto, rest);
+      upto += four;
+    }
+    a.out[n_row] = min(unit * N + (pick < 0 ? last : pick), V - 1);
+  }
+  return true;
+}
+
+// ---- a workgroup a row; of rows in CHUNKS the thresholds, and those rows that are left to it
+template <typename T, typename F, bool CHUNKS, bool MASKED = true>
+__global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(const SampleArgs a,
+                                                                 RowState* states) {
+  __shared__ Shared<F> s;
+  const int n_row = blockIdx.x;
+  const Wants want = wants_of(a, n_row);
+  Row<T, F::WG> row = row_of<T, F::WG>(a, n_row);
+  if constexpr (CHUNKS) {
+    RowState& state = states[n_row];
+    const RowPlan plan = state.plan;
+    if (want.greedy || plan.mode == NO_LIST) return;
+    if (!left_whole(plan)) {
+      row.m = plan.m;
+      const uint32_t least = least_of_list(s, state.list, plan.n, plan.above, plan.target, want, row);
+      if (threadIdx.x == 0) state.plan.kmin = least;
+      return;
+    }
+  } else if constexpr (F::WG == 1024) {
+    if (row_by_units<T, MASKED>(s, a, want, row, n_row)) return;
+  }
+  whole_row<T>(s, a, want, row, n_row);
 }
 
 template <typename T>
@@ -1005,17 +1526,20 @@ static void launch(const SampleArgs& a, void* work, int chunks, hipStream_t stre
     draw_kernel<T><<<a.B, 256, 0, stream>>>(a, states);
   } else if (a.V <= 4096 || (a.V <= 8192 && a.B > 256)) {
     sample_fullvocab_kernel<T, Small, false><<<a.B, Small::WG, 0, stream>>>(a, states);
-  } else {
+  } else if (a.mask && a.mask_map) {
     sample_fullvocab_kernel<T, Large, false><<<a.B, Large::WG, 0, stream>>>(a, states);
+  } else {
+    sample_fullvocab_kernel<T, Large, false, false><<<a.B, Large::WG, 0, stream>>>(a, states);
   }
 }
 
 // Chunks of a row, the more of them the fewer the rows; 0: a workgroup a row, which is faster from 100 rows
-// on, for smaller vocabularies, and for greedy rows that would wait for the launches.  By a workgroup a
-// row and in chunks, us, greedy, plain, top-p and all kinds in turns: 128256 tokens 1 row 19 38 81 38 and
-// 17 29 54 29, 16 20 41 85 84 and 19 34 63 63, 64 22 42 89 88 and 24 42 78 77, 100 23 44 90 89 and 27 51
-// 95 94, 190 25 48 94 91 and 38 73 129 123; 100000 16 17 42 79 78 and 19 33 61 62; 65536 8 12 25 53 52
-// and 17 27 49 50; 50257 8 13 30 60 59 and 18 28 47 48; 32000 8 8 20 39 39 and 15 24 40 41.
+// on and for smaller vocabularies.  By a workgroup a row, by units and by whole_row(), and in chunks, us,
+// greedy, plain, top-p and all kinds in turns: 128256 tokens 1 row 10 19 57 19, 19 38 81 38 and 17 30 55 30,
+// 16 11 21 59 58, 20 41 85 84 and 19 34 62 62, 64 17 26 63 63, 22 42 89 88 and 24 43 77 76, 100 19 28 66 65,
+// 23 44 90 89 and 27 51 95 94; 65536 8 8 15 44 43, 12 25 53 52 and 17 27 49 50.  Up to 64 rows in chunks all the
+// same: what rows want is known on the device, and what only whole_row() can, a top-p of 0.999 for one, takes 125 us
+// by it and 55 in chunks.
 extern "C" int sample_fullvocab_chunks(int B, int V) {
   return V < SPLIT_VOCAB || B > 64 ? 0 : B <= 16 ? 32 : 16;
 }

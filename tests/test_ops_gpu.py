@@ -831,6 +831,52 @@ def test_sample_fullvocab_chunks(V, dtype):
 
 
 
+@requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [8200, 32000, 128256, 262144])
+@pytest.mark.parametrize("std", [0.05, 2.5, 8.0])
+def test_sample_fullvocab_rows_by_units(V, std, dtype):
+    """A row by units of 16 bytes, from a few of them a wave to more than its registers hold, against 64
+    bits: logits over a part of an octave and over more than the buckets have, a few far above the rest,
+    ones without weight, temperatures that take the boundary to either end.  Weights are rounded to 32
+    bits, so one draw of 32 may fall between the two sums."""
+    C, B = hip()._C, 32
+    gen = torch.Generator(device="cuda").manual_seed(V)
+    x = torch.randn(B, V, generator=gen, device="cuda") * std
+    x[:4] *= 3
+    x[4:6, :100] += 12
+    x[6:8, ::7] = float("-inf")
+    x[8] = x[8].abs()
+    x = x.to(dtype)
+    u, one = torch.rand(B, generator=gen, device="cuda"), torch.ones(B, device="cuda")
+    mask = torch.rand(2, V, generator=gen, device="cuda") < 0.7
+    which = (torch.arange(B, device="cuda") % 3 - 1).int()
+    for t, k, p in [(0.8, 0, 1.0), (0.8, 1, 1.0), (0.8, 50, 1.0), (0.8, 7000, 1.0), (0.05, 40, 1.0),
+                    (0.8, 0, 0.1), (0.8, 0, 0.95), (0.8, 0, 0.99), (0.8, 0, 0.999), (6.4, 0, 0.9),
+                    (0.1, 0, 0.9), (0.8, 50, 0.95), (1.5, 3000, 0.6)]:
+        for m, to in ((None, None), (mask, which)):
+            out = torch.full((B,), -1, device="cuda")
+            C.sample_fullvocab(out, x, one * t, (one * k).long(), one * p, u, m, to, 0)
+            v = x.double()
+            if m is not None:
+                v = torch.where((which >= 0).view(-1, 1) & ~mask[which.clamp(min=0)], -torch.inf, v)
+            keep = v >= v.topk(k, 1).values[:, -1:] if k else torch.ones_like(v, dtype=torch.bool)
+            w = torch.where(keep, ((v - v.max(1, keepdim=True).values) / t).exp(), 0.0)
+            if p < 1:
+                top, order = w.sort(1, descending=True)
+                ahead = top.cumsum(1) - top
+                n = (ahead < (one * p).double().view(-1, 1) * w.sum(1, keepdim=True)).sum(1)
+                least = v.gather(1, order).gather(1, n.view(-1, 1) - 1)
+                w = torch.where(v >= least, w, 0.0)
+            cdf = w.cumsum(1)
+            want = (cdf > u.double().view(-1, 1) * cdf[:, -1:]).int().argmax(1)
+            assert int((out != want).sum()) <= 1, (t, k, p, m is not None)
+    out = torch.full((B,), -1, device="cuda")
+    C.sample_fullvocab(out, x, one * 0, (one * 0).long(), one, u, None, None, 0)
+    first = torch.where(x == x.max(1, keepdim=True).values, torch.arange(V, device="cuda"), V).min(1)
+    assert torch.equal(out, first.values)
+
+
 @pytest.mark.gpu
 def test_sample_fullvocab_vs_oracle():
     """csrc/sampling_fullvocab.hip vs the fp32 reference over a Llama-3
