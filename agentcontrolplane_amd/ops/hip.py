@@ -262,8 +262,10 @@ def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefi
     n_split = 1
     if mfma:
         keys = min(max_keys, window)
-        # workgroups that fill the chip: the tiles of a wide latent take a CU's LDS
-        fill = 256 if q.shape[2] >= 256 else 512
+        # workgroups that fill the chip: the tiles of a wide latent take a CU's LDS, but for up to 16 rows
+        # half of it.  40 x 200 to 6000 keys of rank 512, a step's 20 layers: 512 2400 us, 256 and 1024
+        # 2600 and 2455
+        fill = 256 if q.shape[2] >= 256 and mg > 1 else 512
         n_split = max(1, min(_MAX_SPLIT, fill // tiles, -(-keys // 128)))
     part = ml = None
     if n_split > 1:

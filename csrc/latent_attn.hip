@@ -5,7 +5,7 @@
 // twice.  Queries are flattened (token, head) rows; a workgroup owns 16*MG of
 // them, which for decode are the heads of one sequence.
 //
-//   tile = 64 keys staged once in LDS by direct global->LDS loads (row-major,
+//   tile = 64 keys (32) staged once in LDS by direct global->LDS loads (row-major,
 //     16-byte units XOR-swizzled on the source address), double buffered
 //   QK^T: wave w takes keys 16w..16w+15, all query rows (A = keys, B = queries,
 //     so a lane owns one query row and 4 of its keys)
@@ -33,10 +33,8 @@ typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) bf16x4_v lds_bf16x4;
 typedef __attribute__((address_space(1))) const char glob_char;
 
-#define KT 64          // keys per tile
 #define ROT 64         // padded rotated dims
 #define NEG -1e30f
-#define PPAD 72        // probability row in LDS, bf16 elements
 
 // one query tile's place
 struct Tile {
@@ -63,9 +61,11 @@ static DEV Tile find_tile(const LatentArgs& a, int rows_per_tile) {
   return t;
 }
 
-template <int NR, int MG>
-__global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
+// KT: keys of a tile, 16 a wave for the scores
+template <int NR, int MG, int KT>
+__global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(const LatentArgs a) {
   constexpr int RANK = 64 * NR;
+  constexpr int PPAD = KT + 8;             // probability row in LDS, bf16 elements
   constexpr int ROW = RANK + ROT;
   constexpr int UPR = ROW / 8;             // 16-byte units per row
   constexpr int STEPS = ROW / 32;          // MFMA k-steps of QK^T
@@ -75,6 +75,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
   bf16_t* const prob = (bf16_t*)(lds + 2 * TILE_BYTES);          // [M][PPAD]
   float* const red = (float*)(prob + M * PPAD);                   // [M][4]
   int* const slots = (int*)(red + M * 4);                         // [2][KT]
+  int* const pages = slots + 2 * KT;                              // [2][KT]
 
   const Tile tl = find_tile(a, M);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -131,11 +132,17 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
     }
   }
 
-  auto find_slots = [&](int t) {
-    if (threadIdx.x < KT) {
-      const int k = min(k_begin + t * KT + (int)threadIdx.x, k_end - 1);
-      slots[(t & 1) * KT + threadIdx.x] = table[k / a.kv_block] * a.kv_block + k % a.kv_block;
-    }
+  // Pages go from the tables to LDS, three tiles ahead, and become slots two tiles ahead: in registers
+  // they would be waited for, and with them, as loads come back in order, all of the tile behind them
+  auto key_of = [&](int t) { return min(k_begin + t * KT + (int)threadIdx.x, k_end - 1); };
+  auto ask_pages = [&](int t) {
+    if (threadIdx.x < KT)
+      __builtin_amdgcn_global_load_lds((glob_char*)(table + key_of(t) / a.kv_block),
+                                       (lds_char*)(pages + (t & 1) * KT), 4, 0, 0);
+  };
+  auto put_slots = [&](int t, const int* from) {
+    if (threadIdx.x < KT)
+      slots[(t & 1) * KT + threadIdx.x] = *from * a.kv_block + key_of(t) % a.kv_block;
   };
   // piece = 1 KiB of the tile image; lane-linear in LDS, swizzled at the source
   auto stage = [&](int t) {
@@ -153,9 +160,10 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
     }
   };
 
-  find_slots(t_begin);
-  if (t_begin + 1 < t_end) find_slots(t_begin + 1);
+  put_slots(t_begin, table + key_of(t_begin) / a.kv_block);
+  put_slots(t_begin + 1, table + key_of(t_begin + 1) / a.kv_block);
   __syncthreads();
+  ask_pages(t_begin + 2);
   stage(t_begin);
 
   f32x4_v o[MG][NR] = {};
@@ -170,15 +178,24 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
   const float scale2 = a.scale * 1.44269504088896f;  // exp2 domain
   const int sw_c = ((c & 3) << 1) | ((c >> 2) & 1);
 
+  // LDS writes of all waves are done, but not the loads of the next tile, which __syncthreads() waits for
+  auto meet = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
   for (int t = t_begin; t < t_end; ++t) {
+    // tile t landed for every wave; tile t-1 is fully read
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();  // tile t landed for every wave; tile t-1 is fully read
+    meet();
+    if (t + 3 < t_end) ask_pages(t + 3);
     if (t + 1 < t_end) stage(t + 1);
     const char* tile = lds + (t & 1) * TILE_BYTES;
 
     // scores: lane holds query row c, keys wid*16 + 4g + {0..3}
     f32x4_v s[MG] = {};
-    {
+    const bool scores = wid * 16 < KT;
+    if (scores) {
       const char* krow = tile + (wid * 16 + c) * (ROW * 2);
 #pragma unroll
       for (int st = 0; st < STEPS; ++st) {
@@ -195,7 +212,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int key = key0 + r;
-        const bool see = key <= qpos[m] && qpos[m] - key < a.window;
+        const bool see = scores && key <= qpos[m] && qpos[m] - key < a.window;
         s[m][r] = see ? s[m][r] * scale2 : -INFINITY;
         mt = fmaxf(mt, s[m][r]);
       }
@@ -203,7 +220,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
       mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
       if (g == 0) red[(m * 16 + c) * 4 + wid] = mt;
     }
-    __syncthreads();
+    meet();
 #pragma unroll
     for (int m = 0; m < MG; ++m) {
       const float4 w4 = *(const float4*)(red + (m * 16 + c) * 4);
@@ -217,16 +234,16 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(const LatentArgs a) {
         sum += p[r];
       }
       l_run[m] = l_run[m] * alpha + sum;
-      store_f<4>(prob + (m * 16 + c) * PPAD + wid * 16 + 4 * g, p);
+      if (scores) store_f<4>(prob + (m * 16 + c) * PPAD + wid * 16 + 4 * g, p);
 #pragma unroll
       for (int n = 0; n < NR; ++n) o[m][n] *= alpha;
     }
-    if (t + 2 < t_end) find_slots(t + 2);  // tile t's slots were consumed by its stage
-    __syncthreads();
+    if (t + 2 < t_end) put_slots(t + 2, pages + (t & 1) * KT + threadIdx.x);  // tile t's slots were consumed by its stage
+    meet();
 
     // values: A = latent columns (transposed read), B = probabilities
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+    for (int ks = 0; ks < KT / 32; ++ks) {
       bf16x8_v pf[MG];
 #pragma unroll
       for (int m = 0; m < MG; ++m)
@@ -385,13 +402,25 @@ __global__ __launch_bounds__(256) void latent_attn_plain_kernel(
   }
 }
 
+template <int NR, int MG, int KT>
+static void launch_tiles(const LatentArgs& a, int tiles, hipStream_t stream) {
+  constexpr int M = 16 * MG;
+  constexpr int bytes = 2 * KT * (64 * NR + ROT) * 2 + M * (KT + 8) * 2 + M * 16 + 4 * KT * 4;
+  static_assert(bytes <= 160 * 1024, "LDS");
+  allow_lds<latent_attn_kernel<NR, MG, KT>>(bytes);
+  latent_attn_kernel<NR, MG, KT><<<dim3(tiles, a.n_split), 256, bytes, stream>>>(a);
+}
+
+// A tile is a chain of reads, products and three barriers, during which a CU with one workgroup waits:
+// with tiles of 32 keys of a wide latent it has two, where there are as many.  40 x 200 to 6000 keys of
+// 16 heads 72 us by 64 keys, 57 by 32; four tiles in LDS, three of them under way, of one workgroup a
+// CU 91.  By 32 keys alone a step over 1 x 5000 1671 us, else 1651, over 8 x 200 to 800 1928 and 1893.
+#define CUS 256
 template <int NR, int MG>
 static void launch_mfma(const LatentArgs& a, int tiles, hipStream_t stream) {
-  constexpr int M = 16 * MG;
-  constexpr int bytes = 2 * KT * (64 * NR + ROT) * 2 + M * PPAD * 2 + M * 16 + 2 * KT * 4;
-  static_assert(bytes <= 160 * 1024, "LDS");
-  allow_lds<latent_attn_kernel<NR, MG>>(bytes);
-  latent_attn_kernel<NR, MG><<<dim3(tiles, a.n_split), 256, bytes, stream>>>(a);
+  if constexpr (MG == 1 && NR >= 4)
+    if (tiles * (int64_t)a.n_split > CUS) return launch_tiles<NR, MG, 32>(a, tiles, stream);
+  launch_tiles<NR, MG, 64>(a, tiles, stream);
 }
 
 template <int NR>

@@ -170,6 +170,10 @@ SHAPES = [
     (32, 512, None, 16, [(0, 150), (90, 1), (2000, 1), (777, 2)]),
     (128, 512, 300, 16, [(0, 3), (900, 1), (1200, 1)]),
     (2, 600, 50, 16, [(0, 60), (70, 1), (70, 2)]),
+    # more workgroups of decode than CUs: smaller tiles, of every number of keys modulo theirs
+    (16, 512, None, 16, [(0, 20)] + [(7 * i, 1) for i in range(48)] + [(1000, 1)]),
+    (9, 250, None, 4, [(0, 3)] + [(9 * i + 1, 1) for i in range(40)] + [(930, 1), (1023, 1)]),
+    (5, 384, 900, 16, [(0, 2)] + [(23 * i, 1) for i in range(45)] + [(1100, 1)]),
 ]
 
 
