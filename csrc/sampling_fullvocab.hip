@@ -16,10 +16,11 @@
 // token-id order, and walks the stripe with the target: the inverse CDF runs in token-id order
 // and draws match the fp32 oracle (ops/reference.py softmax_sample) for a given uniform.  The
 // weights of 64 tokens of every stripe are made at a time by all threads and added up by one
-// thread a stripe, by fours in fp32 and those in 64 bits, so that all the ways a row can take agree.
+// thread a stripe: one after another in fp32 without a threshold (all CUTS are false), by fours in fp32
+// and those in 64 bits with one, so that all the ways such a row can take agree.
 //
-// Rows of whole units by one workgroup take another way, by units (below), and this one where that does
-// not fit: 190 rows of 128256 in fp32, other logits each time, whole calls: 25 us greedy, 48 plain, 79
+// Greedy rows of whole units by one workgroup, and those with a threshold, take another way, by units
+// (below), and this one where that does not fit: 190 rows of 128256 in fp32, other logits each time, whole calls: 25 us greedy, 48 plain, 79
 // top-k, 95 top-p, 135 both (26, 58, 97, 168 and 238 with calls of functions, which take a row and LDS by
 // reference: their loads and atomics then go by unknown memory and wait for both kinds).  Floating masses
 // instead of whole ones in the histogram took as long, a shared list of the bucket 25 us more.
@@ -69,11 +70,13 @@ __device__ __forceinline__ float ldf(const bf16_t* p) { return bf2f(*p); }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Tokens of a stripe, in whole fours of the row
+// Tokens of a stripe; with a threshold in whole fours of the row
+template <bool CUTS = true>
 __device__ __forceinline__ int stripe_tokens(int V) {
-  return ((V + STRIPES - 1) / STRIPES + 3) & ~3;
+  const int n = (V + STRIPES - 1) / STRIPES;
+  return CUTS ? (n + 3) & ~3 : n;
 }
-// Weights are added up by fours, those in 64 bits
+// Weights of a row with a threshold are added up by fours, those in 64 bits
 __device__ __forceinline__ float sum_of_four(float a, float b, float c, float d) {
   return (a + c) + (b + d);
 }
@@ -144,7 +147,10 @@ struct Row {
   int V;
   float m, invT, scale;  // the largest logit, 1 / temperature, that in octaves
 
-  __device__ float weight(float v) const { return __builtin_amdgcn_exp2f((v - m) * scale); }
+  template <bool CUTS = true>
+  __device__ float weight(float v) const {
+    return CUTS ? __builtin_amdgcn_exp2f((v - m) * scale) : __expf((v - m) * invT);
+  }
 
   // f(token, logit) for every allowed token, a thread's in rising order
   template <typename F>
@@ -443,29 +449,49 @@ INLINE Row<T, WG> row_of(const SampleArgs& a, int n) {
           invT * 1.44269504f};
 }
 
+// A stripe's weights of a tile
+template <bool CUTS, int TILE, typename Sum>
+INLINE void add_tile(const float* tile, Sum& sum) {
+  constexpr int FOURS = TILE < 32 ? TILE / 4 : 8;
+#pragma unroll 1
+  for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
+    float4 w[FOURS];
+#pragma unroll
+    for (int j = 0; j < FOURS; ++j) w[j] = *(const float4*)(tile + 4 * (j0 + j));
+#pragma unroll
+    for (int j = 0; j < FOURS; ++j) {
+      if constexpr (CUTS)
+        sum += sum_of_four(w[j].x, w[j].y, w[j].z, w[j].w);
+      else
+        sum = sum + w[j].x + w[j].y + w[j].z + w[j].w;
+    }
+  }
+}
+
 // ---- inverse-CDF draw in token-id order from the stripes' sums, ``mine`` of the t-th thread's
-template <typename S, typename R>
+template <bool CUTS, typename S, typename R>
 INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin,
                      double mine) {
+  using Sum = std::conditional_t<CUTS, double, float>;
   constexpr int WG = S::WG;
-  const int t = threadIdx.x, V = row.V, stride = stripe_tokens(V);
+  const int t = threadIdx.x, V = row.V, stride = stripe_tokens<CUTS>(V);
   if (t < STRIPES) s.stripe[t] = mine;
   if (t == 0) s.pick = s.n = -1;
   __syncthreads();
   constexpr int STEP = 32;  // one thread's LDS reads in flight
   if (t == 0) {
-    double sum = 0.0;
+    Sum sum = 0;
     s.cdf[0] = 0.0;
     for (int i = 0; i < STRIPES; i += STEP / 2) {
-      double w[STEP / 2];
+      Sum w[STEP / 2];
 #pragma unroll
-      for (int e = 0; e < STEP / 2; ++e) w[e] = s.stripe[i + e];
+      for (int e = 0; e < STEP / 2; ++e) w[e] = (Sum)s.stripe[i + e];
 #pragma unroll
       for (int e = 0; e < STEP / 2; ++e) s.cdf[i + e + 1] = sum += w[e];
     }
   }
   __syncthreads();
-  const double target = (double)a.uniforms[n_row] * s.cdf[STRIPES];
+  const Sum target = (Sum)a.uniforms[n_row] * (Sum)s.cdf[STRIPES];
   // exactly one stripe satisfies prefix <= target < prefix + mine
   // (mine > 0 guaranteed for the owner since the CDF strictly increases
   // across it); fp edge cases fall through to the fallback below
@@ -485,7 +511,7 @@ INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t km
       if (j < here && !(row.mask && !row.mask[i0 + j])) {
         const float v = ldf(row.x + i0 + j);
         if (f2key(v) >= kmin) {
-          w = row.weight(v);
+          w = row.template weight<CUTS>(v);
           last = i0 + j;
         }
       }
@@ -494,24 +520,34 @@ INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t km
     if (last >= 0) atomicMax(&s.pick, last);
     __syncthreads();
     if (t == 0) {
-      double cum = s.cdf[n];
+      Sum cum = (Sum)s.cdf[n];
       int first = -1;
       for (int j = 0; j < here && first < 0; j += STEP) {
         float w[STEP], fours[STEP / 4];
-        double upto = cum;
+        Sum upto = cum;
 #pragma unroll
         for (int e = 0; e < STEP; e += 4) {
           *(float4*)(w + e) = *(const float4*)(buf + j + e);
-          fours[e / 4] = sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
-          upto += fours[e / 4];
-        }
-        if (!(upto <= target))  // the same sums again: weights are not negative
-#pragma unroll
-          for (int g = 0; g < STEP / 4; ++g) {
-            if (first < 0 && cum + fours[g] > target)
-              first = 4 * g + token_of_four(w + 4 * g, cum, target);
-            cum += fours[g];
+          if constexpr (CUTS) {
+            fours[e / 4] = sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
+            upto += fours[e / 4];
+          } else {
+            upto = upto + w[e] + w[e + 1] + w[e + 2] + w[e + 3];
           }
+        }
+        if (!(upto <= target)) {  // the same sums again: weights are not negative
+          if constexpr (CUTS) {
+#pragma unroll
+            for (int g = 0; g < STEP / 4; ++g) {
+              if (first < 0 && cum + fours[g] > target)
+                first = 4 * g + token_of_four(w + 4 * g, cum, target);
+              cum += fours[g];
+            }
+          } else {
+            for (int e = 0; e < STEP && first < 0; ++e)
+              if ((cum += buf[j + e]) > target) first = e;
+          }
+        }
         cum = upto;
         if (first >= 0) s.pick = i0 + j + first;
       }
@@ -602,11 +638,12 @@ struct ChunkShared : ChunkForm {
 struct Chunk {
   int row, at, stride, stripes, i0, i1;
 };
+template <bool CUTS = true>
 __device__ __forceinline__ Chunk chunk_of(const SampleArgs& a, int chunks) {
   Chunk c;
   c.row = blockIdx.x / chunks;
   c.at = blockIdx.x - c.row * chunks;
-  c.stride = stripe_tokens(a.V);
+  c.stride = stripe_tokens<CUTS>(a.V);
   c.stripes = STRIPES / chunks;
   c.i0 = min(a.V, c.at * c.stripes * c.stride);
   c.i1 = min(a.V, c.i0 + c.stripes * c.stride);
@@ -781,20 +818,11 @@ __global__ __launch_bounds__(256) void chunk_keys_kernel(const SampleArgs a, Row
   for (int i = threadIdx.x; i < n && s.base + i < KEYS; i += 256) state.list[s.base + i] = s.keys[i];
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, RowState* states,
-                                                         const int chunks) {
+template <bool CUTS, typename T>
+INLINE void chunk_sums(ChunkShared& s, const SampleArgs& a, const Chunk& c, const Row<T, 256>& row,
+                       const RowPlan& plan, RowState& state) {
   constexpr int TILE = ChunkForm::TILE;
-  __shared__ ChunkShared s;
-  const Chunk c = chunk_of(a, chunks);
-  const Wants want = wants_of(a, c.row);
-  if (want.greedy) return;
-  Row<T, 256> row = row_of<T, 256>(a, c.row);
-  RowState& state = states[c.row];
-  const RowPlan plan = state.plan;
   const int t = threadIdx.x;
-  row.m = plan.m;
-  if (left_whole(plan)) return;
   const uint32_t kmin = plan.kmin;
   // stripes' weights by all threads, 64 tokens of each at a time, added up by a thread a stripe
   const int r = t / TILE, col = t % TILE;
@@ -803,7 +831,7 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, Row
   const bool by_value = kmin == 0 || (least == least && least != 0.f);
   const float from = kmin == 0 ? -INFINITY : least;
   float ahead[MOST];
-  double mine = 0.0;
+  std::conditional_t<CUTS, double, float> mine = 0;
   auto fetch = [&](int j0) {
 #pragma unroll
     for (int k = 0; k < MOST; ++k)
@@ -820,23 +848,31 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, Row
       // comparing logits is comparing keys, but for zeros and what is no number
       const bool keep = by_value && plan.plain ? ahead[k] >= from : f2key(ahead[k]) >= kmin;
       const bool in = j0 + col < c.stride && i < a.V && keep && !(row.mask && !row.mask[i]);
-      tile[k * ROWS + r][col] = in ? row.weight(ahead[k]) : 0.f;
+      tile[k * ROWS + r][col] = in ? row.template weight<CUTS>(ahead[k]) : 0.f;
     }
     if (j0 + TILE < c.stride) fetch(j0 + TILE);
     __syncthreads();  // the other tile is added up before it is written again
-    if (t < c.stripes) {
-      constexpr int FOURS = TILE < 32 ? TILE / 4 : 8;
-#pragma unroll 1
-      for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
-        float4 w[FOURS];
-#pragma unroll
-        for (int j = 0; j < FOURS; ++j) w[j] = *(const float4*)&tile[t][4 * (j0 + j)];
-#pragma unroll
-        for (int j = 0; j < FOURS; ++j) mine += sum_of_four(w[j].x, w[j].y, w[j].z, w[j].w);
-      }
-    }
+    if (t < c.stripes) add_tile<CUTS, TILE>(tile[t], mine);
   }
   if (t < c.stripes) state.stripe[c.at * c.stripes + t] = mine;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, RowState* states,
+                                                         const int chunks) {
+  __shared__ ChunkShared s;
+  const int n_row = blockIdx.x / chunks;
+  const Wants want = wants_of(a, n_row);
+  if (want.greedy) return;
+  Row<T, 256> row = row_of<T, 256>(a, n_row);
+  RowState& state = states[n_row];
+  const RowPlan plan = state.plan;
+  row.m = plan.m;
+  if (left_whole(plan)) return;
+  if (want.by_k || want.by_p)
+    chunk_sums<true>(s, a, chunk_of<true>(a, chunks), row, plan, state);
+  else
+    chunk_sums<false>(s, a, chunk_of<false>(a, chunks), row, plan, state);
 }
 
 struct DrawShared : ChunkForm {
@@ -858,7 +894,11 @@ __global__ __launch_bounds__(256) void draw_kernel(const SampleArgs a, const Row
   if (left_whole(plan)) return;
   Row<T, 256> row = row_of<T, 256>(a, n_row);
   row.m = plan.m;
-  draw(s, a, row, n_row, plan.kmin, state.stripe[threadIdx.x]);
+  const Wants want = wants_of(a, n_row);
+  if (want.by_k || want.by_p)
+    draw<true>(s, a, row, n_row, plan.kmin, state.stripe[threadIdx.x]);
+  else
+    draw<false>(s, a, row, n_row, plan.kmin, state.stripe[threadIdx.x]);
 }
 
 // The key of a list at which the sum from the top, with what is ``above``, reaches target, the
@@ -995,12 +1035,67 @@ INLINE uint32_t least_of_list(S& s, const uint32_t* list, int n, double above, d
   return max(kmin, find(std::true_type(), 0.0, of_kept));
 }
 
+// inverse-CDF draw in token-id order over the kept set, {key >= kmin}
+template <typename S, typename R>
+INLINE void sum_and_draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin, bool plain,
+                         bool cuts) {
+  constexpr int WG = S::WG, TILE = S::TILE;
+  const int t = threadIdx.x, V = row.V;
+  const int stride = cuts ? stripe_tokens<true>(V) : stripe_tokens<false>(V);
+  // Stripe n is tokens [n * stride, (n + 1) * stride).
+  constexpr int PER = STRIPES * TILE / WG, ROWS = WG / TILE;  // a thread's tokens of a tile
+  // token of the thread's k-th of a tile: k * ROWS stripes on
+  const int r = t / TILE, c = t % TILE, i_first = r * stride + c;
+  auto weight = [&](float v) { return cuts ? row.template weight<true>(v) : row.template weight<false>(v); };
+  float ahead[PER];
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      ahead[k] = ldf(row.x + min(k * ROWS * stride + j0 + i_first, V - 1));
+  };
+  // comparing logits is comparing keys, but for zeros and what is no number
+  const float least = key2f(kmin);
+  const bool by_value = kmin == 0 || (least == least && least != 0.f);
+  const float from = kmin == 0 ? -INFINITY : least;
+  double mine = 0.0;  // or a sum in fp32, which it holds as it is
+  fetch(0);
+  for (int j0 = 0; j0 < stride; j0 += TILE) {
+    float(*tile)[TILE + 4] = s.tile[j0 / TILE % 2];
+    if (by_value && plain && !row.mask && j0 + TILE <= stride) {
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const bool in = ahead[k] >= from && k * ROWS * stride + j0 + i_first < V;
+        tile[k * ROWS + r][c] = in ? weight(ahead[k]) : 0.f;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int i = k * ROWS * stride + j0 + i_first;
+        const bool in = j0 + c < stride && i < V && f2key(ahead[k]) >= kmin &&
+                        !(row.mask && !row.mask[i]);
+        tile[k * ROWS + r][c] = in ? weight(ahead[k]) : 0.f;
+      }
+    }
+    if (j0 + TILE < stride) fetch(j0 + TILE);
+    __syncthreads();  // the other tile is added up before it is written again
+    if (t < STRIPES && cuts) {
+      add_tile<true, TILE>(tile[t], mine);
+    } else if (t < STRIPES) {
+      float sum = (float)mine;
+      add_tile<false, TILE>(tile[t], sum);
+      mine = sum;
+    }
+  }
+  if (cuts)
+    draw<true>(s, a, row, n_row, kmin, mine);
+  else
+    draw<false>(s, a, row, n_row, kmin, mine);
+}
+
 // ---- a row by one workgroup, in as many passes over it as its thresholds call for
 template <typename T, typename S>
 INLINE void whole_row(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG>& row, int n_row) {
-  constexpr int WG = S::WG, TILE = S::TILE;
   const int t = threadIdx.x, V = a.V;
-  const int stride = stripe_tokens(V);
 
   // ---- the largest allowed logit, the lowest token that has it, and whether all are numbers
   float mx = -3.4e38f;
@@ -1042,55 +1137,7 @@ INLINE void whole_row(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG
     if (pmin > kmin) kmin = pmin;
   }
 
-  // ---- inverse-CDF draw in token-id order over the kept set.
-  // Stripe n is tokens [n * stride, (n + 1) * stride).
-  constexpr int PER = STRIPES * TILE / WG, ROWS = WG / TILE;  // a thread's tokens of a tile
-  // token of the thread's k-th of a tile: k * ROWS stripes on
-  const int r = t / TILE, c = t % TILE, i_first = r * stride + c;
-  float ahead[PER];
-  auto fetch = [&](int j0) {
-#pragma unroll
-    for (int k = 0; k < PER; ++k)
-      ahead[k] = ldf(row.x + min(k * ROWS * stride + j0 + i_first, V - 1));
-  };
-  // comparing logits is comparing keys, but for zeros and what is no number
-  const float least = key2f(kmin);
-  const bool by_value = kmin == 0 || (least == least && least != 0.f);
-  const float from = kmin == 0 ? -INFINITY : least;
-  double mine = 0.0;
-  fetch(0);
-  for (int j0 = 0; j0 < stride; j0 += TILE) {
-    float(*tile)[TILE + 4] = s.tile[j0 / TILE % 2];
-    if (by_value && plain && !row.mask && j0 + TILE <= stride) {
-#pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const bool in = ahead[k] >= from && k * ROWS * stride + j0 + i_first < V;
-        tile[k * ROWS + r][c] = in ? row.weight(ahead[k]) : 0.f;
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int i = k * ROWS * stride + j0 + i_first;
-        const bool in = j0 + c < stride && i < V && f2key(ahead[k]) >= kmin &&
-                        !(row.mask && !row.mask[i]);
-        tile[k * ROWS + r][c] = in ? row.weight(ahead[k]) : 0.f;
-      }
-    }
-    if (j0 + TILE < stride) fetch(j0 + TILE);
-    __syncthreads();  // the other tile is added up before it is written again
-    if (t < STRIPES) {
-      constexpr int FOURS = TILE < 32 ? TILE / 4 : 8;
-#pragma unroll 1
-      for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
-        float4 w[FOURS];
-#pragma unroll
-        for (int j = 0; j < FOURS; ++j) w[j] = *(const float4*)&tile[t][4 * (j0 + j)];
-#pragma unroll
-        for (int j = 0; j < FOURS; ++j) mine += sum_of_four(w[j].x, w[j].y, w[j].z, w[j].w);
-      }
-    }
-  }
-  draw(s, a, row, n_row, kmin, mine);
+  sum_and_draw(s, a, row, n_row, kmin, plain, by_k || by_p);
 }
 
 // ---- a row by one workgroup, by units of 16 bytes
@@ -1106,11 +1153,12 @@ INLINE void whole_row(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG
 //   3 the weights above those buckets in a thread's own sum, the keys in them into a list, from which the
 //     least kept key follows exactly
 // The draw goes to the wave that has the target, then to its turn, a unit, a token, in token-id order.
-// 190 rows of 128256 in fp32, whole_row() and this, us: greedy 24.6 and 22.5, plain 48 and 33, top-k 80 and
-// 55, top-p 95 and 72, both 135 and 60, top-p 0.9 at a temperature of 6.4 100 and 74; bf16 22 and 14, 46 and
-// 24, 70 and 45, 92 and 67, 118 and 50; 32000 in fp32 10 and 8.8, 21 and 13, 35 and 25, 42 and 33, 58 and 31.
-// Without HELD plain rows take 41, with more registers spill; 4 units ahead instead of 2 as long.
-// A row that this does not fit is whole_row()'s: one of no whole units, logits that are no numbers, a
+// 190 rows of 128256 in fp32, whole_row() and this, us: greedy 24.6 and 22.5, top-k 80 and 55, top-p 95 and
+// 72, both 135 and 60, top-p 0.9 at a temperature of 6.4 100 and 74; bf16 22 and 14, 70 and 45, 92 and 67,
+// 118 and 50; 32000 in fp32 10 and 8.8, 35 and 25, 42 and 33, 58 and 31.  Plain rows took 33 instead of 48, but
+// their draws are by sums in fp32, in order, and one in 50 was another one by these sums: they stay
+// whole_row()'s.  With more registers HELD they spill; 4 units ahead instead of 2 as long.
+// A row that this does not fit is whole_row()'s: one of no threshold that is not greedy, of no whole units, logits that are no numbers, a
 // boundary among more keys than the list has or beyond the last bucket, a top-p beyond MOST_P.
 template <typename T, bool MASKED>
 struct Units {
@@ -1264,6 +1312,7 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
     }
     return true;
   }
+  if (!cuts) return false;  // here: ahead of the greedy rows the compiler spills registers
   unsigned long long odd_lanes = 0;
   units_of.template each<true>(held, [&](const u32x4& v, int) {
 #pragma unroll
@@ -1279,14 +1328,12 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   // top-k's buckets are of logits, so that no temperature takes the k-th beyond the last one
   const float per_octave = row.scale;
   float scale = want.by_k ? (float)PER_LOGIT / PER_OCTAVE : per_octave;
-  if (cuts) {
-    // finer ones where the row does not reach the last one
-    least = block_least(s, least);
-    const float span = (mx - least) * scale, most = UNIT_BUCKETS / PER_OCTAVE - 2;
-    if (!(span > 1e-20f)) return false;
-    if (span < most) scale *= most / span;
-    if (!(scale < 1e25f)) return false;
-  }
+  // finer ones where the row does not reach the last one
+  least = block_least(s, least);
+  const float span = (mx - least) * scale, most = UNIT_BUCKETS / PER_OCTAVE - 2;
+  if (!(span > 1e-20f)) return false;
+  if (span < most) scale *= most / span;
+  if (!(scale < 1e25f)) return false;
   const float fine = scale * (PER_OCTAVE * PARTS), bucket_octaves = per_octave / scale / PER_OCTAVE;
   if (odd || !(mx > -1e37f && mx < INFINITY) || !(per_octave < 1e20f && per_octave > 1e-20f)) return false;
   row.m = mx;
@@ -1294,7 +1341,7 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   // ---- 2: the buckets lo .. hi - 1 that the boundary can be in
   int lo = 0, hi = 0;
   double k_above = 0.0;
-  if (cuts) {
+  {
     uint32_t* const mine = &s.column[0][lane];
     units_of.template each<false>(held, [&](const u32x4& v, int) {
 #pragma unroll
@@ -1362,36 +1409,27 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
 #pragma unroll
     for (int e = 0; e < N; e += 4) to += (double)sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
   };
-  if (!cuts) {
-    units_of.template each<false>(held, [&](const u32x4& v, int) {
-      float w[N];
+  units_of.template each<false>(held, [&](const u32x4& v, int) {
+    float w[N], in[N];
 #pragma unroll
-      for (int e = 0; e < N; ++e) w[e] = weigh(U::at(v, e));
-      add_fours(w, kept);
-    });
-  } else {
-    units_of.template each<false>(held, [&](const u32x4& v, int) {
-      float w[N], in[N];
-#pragma unroll
-      for (int e = 0; e < N; ++e) {
-        const float x = U::at(v, e), z = (x - top) * scale;
-        w[e] = weigh(x);
-        in[e] = z > edge_lo ? w[e] : 0.f;
-        if (z > edge_hi && !(z > edge_lo)) {
-          const int at = atomicAdd(&s.n, 1);
-          if (at < UNIT_KEYS) {
-            s.key[at] = f2key(x);
-            s.key_wave[at] = wid;
-          }
+    for (int e = 0; e < N; ++e) {
+      const float x = U::at(v, e), z = (x - top) * scale;
+      w[e] = weigh(x);
+      in[e] = z > edge_lo ? w[e] : 0.f;
+      if (z > edge_hi && !(z > edge_lo)) {
+        const int at = atomicAdd(&s.n, 1);
+        if (at < UNIT_KEYS) {
+          s.key[at] = f2key(x);
+          s.key_wave[at] = wid;
         }
       }
-      add_fours(in, kept);
-      if (want.by_p) add_fours(w, all);
-    });
-  }
+    }
+    add_fours(in, kept);
+    if (want.by_p) add_fours(w, all);
+  });
   uint32_t kmin = 0;
   if (t < WAVES) s.wave_units[t] = 0;
-  if (cuts) {
+  {
     const double above = want.by_k ? k_above : block_total(s, kept);
     const double target = want.by_k ? want.k : (double)want.p * block_total(s, all);
     __syncthreads();

@@ -869,6 +869,14 @@ def test_sample_fullvocab_rows_by_units(V, std, dtype):
                 least = v.gather(1, order).gather(1, n.view(-1, 1) - 1)
                 w = torch.where(v >= least, w, 0.0)
             cdf = w.cumsum(1)
+            if not k and p == 1:
+                # the general path, whose sums are of 32 bits: V / 256 weights and then 256 stripes in
+                # order, each rounded to 2^-24 of them, and the weights to less than 2^-18
+                off = (V / 256 + 256) * 2.0**-24 + 2.0**-18
+                to_here = (cdf / cdf[:, -1:]).gather(1, out.view(-1, 1)).view(-1)
+                share = (w / cdf[:, -1:]).gather(1, out.view(-1, 1)).view(-1)
+                assert bool(((to_here >= u - off) & (to_here - share <= u + off) & (share > 0)).all())
+                continue
             want = (cdf > u.double().view(-1, 1) * cdf[:, -1:]).int().argmax(1)
             assert int((out != want).sum()) <= 1, (t, k, p, m is not None)
     out = torch.full((B,), -1, device="cuda")
