@@ -1575,7 +1575,7 @@ static void launch(const SampleArgs& a, void* work, int chunks, hipStream_t stre
 // on and for smaller vocabularies.  By a workgroup a row, by units and by whole_row(), and in chunks, us,
 // greedy, plain, top-p and all kinds in turns: 128256 tokens 1 row 10 19 57 19, 19 38 81 38 and 17 30 55 30,
 // 16 11 21 59 58, 20 41 85 84 and 19 34 62 62, 64 17 26 63 63, 22 42 89 88 and 24 43 77 76, 100 19 28 66 65,
-// 23 44 90 89 and 27 51 95 94; 65536 8 8 15 44 43, 12 25 53 52 and 17 27 49 50.  Up to 64 rows in chunks all the
+// 23 44 90 89 and 27 51 95 94 (plain rows are whole_row()'s in either way); 65536 8 8 15 44 43, 12 25 53 52 and 17 27 49 50.  Up to 64 rows in chunks all the
 // same: what rows want is known on the device, and what only whole_row() can, a top-p of 0.999 for one, takes 125 us
 // by it and 55 in chunks.
 extern "C" int sample_fullvocab_chunks(int B, int V) {
