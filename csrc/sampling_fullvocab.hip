@@ -77,6 +77,8 @@ __device__ __forceinline__ int stripe_tokens(int V) {
   return CUTS ? (n + 3) & ~3 : n;
 }
 // Weights of a row with a threshold are added up by fours, those in 64 bits
+template <bool CUTS>
+using SumOf = std::conditional_t<CUTS, double, float>;
 __device__ __forceinline__ float sum_of_four(float a, float b, float c, float d) {
   return (a + c) + (b + d);
 }
@@ -124,7 +126,8 @@ struct Shared : F {
       double turn_sum[F::WG < 1024 ? 1 : MOST_VOCAB / 256 / F::WAVES + 1];
     };
   };
-  double stripe[STRIPES], cdf[STRIPES + 1], wave[F::WAVES];
+  float stripe[STRIPES], cdf[STRIPES + 1];  // of a row without a threshold
+  double wave[F::WAVES];
   float red[F::WAVES];
   int red_i[F::WAVES], red_odd[F::WAVES];
   int n, pick;
@@ -450,8 +453,8 @@ INLINE Row<T, WG> row_of(const SampleArgs& a, int n) {
 }
 
 // A stripe's weights of a tile
-template <bool CUTS, int TILE, typename Sum>
-INLINE void add_tile(const float* tile, Sum& sum) {
+template <bool CUTS, int TILE>
+INLINE void add_tile(const float* tile, SumOf<CUTS>& sum) {
   constexpr int FOURS = TILE < 32 ? TILE / 4 : 8;
 #pragma unroll 1
   for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
@@ -468,37 +471,62 @@ INLINE void add_tile(const float* tile, Sum& sum) {
   }
 }
 
-// ---- inverse-CDF draw in token-id order from the stripes' sums, ``mine`` of the t-th thread's
+// ---- inverse-CDF draw in token-id order from the stripes' sums, ``mine`` of the t-th thread's.
+// Without a threshold sums are in fp32, in order, by one thread; with one in 64 bits, where a scan
+// is the faster one: 1 x 128256 top-k in chunks 43.5 us in order, 41.2 by the scan.  Compiled apart,
+// since what asks for the kind at each weight, or has both kinds' sums in 64 bits, is slower: plain
+// rows by a workgroup a row 60 us for 190 x 128256, 49 so; 64 x 4104 18.2 and 13.9.
 template <bool CUTS, typename S, typename R>
 INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin,
-                     double mine) {
-  using Sum = std::conditional_t<CUTS, double, float>;
+                     SumOf<CUTS> mine) {
+  using Sum = SumOf<CUTS>;
   constexpr int WG = S::WG;
   const int t = threadIdx.x, V = row.V, stride = stripe_tokens<CUTS>(V);
-  if (t < STRIPES) s.stripe[t] = mine;
-  if (t == 0) s.pick = s.n = -1;
-  __syncthreads();
   constexpr int STEP = 32;  // one thread's LDS reads in flight
-  if (t == 0) {
-    Sum sum = 0;
-    s.cdf[0] = 0.0;
-    for (int i = 0; i < STRIPES; i += STEP / 2) {
-      Sum w[STEP / 2];
-#pragma unroll
-      for (int e = 0; e < STEP / 2; ++e) w[e] = (Sum)s.stripe[i + e];
-#pragma unroll
-      for (int e = 0; e < STEP / 2; ++e) s.cdf[i + e + 1] = sum += w[e];
+  Sum ahead = 0, target = 0;
+  int n = -1;
+  if constexpr (CUTS) {
+    if (t == 0) {
+      s.pick = -1;
+      s.n = STRIPES;
     }
+    const double own = t < STRIPES ? mine : 0.0;
+    double all;
+    const double before = scan_block(s, own, &all);
+    target = (double)a.uniforms[n_row] * all;
+    if (own > 0.0 && before + own > target) atomicMin(&s.n, t);
+    __syncthreads();
+    n = s.n;
+    if (t == n) s.above = before;
+    __syncthreads();
+    ahead = s.above;
+    if (n == STRIPES) n = -1;
+  } else {
+    if (t < STRIPES) s.stripe[t] = mine;
+    if (t == 0) s.pick = s.n = -1;
+    __syncthreads();
+    if (t == 0) {
+      float sum = 0.f;
+      s.cdf[0] = 0.f;
+      for (int i = 0; i < STRIPES; i += STEP) {
+        float w[STEP];
+#pragma unroll
+        for (int e = 0; e < STEP; ++e) w[e] = s.stripe[i + e];
+#pragma unroll
+        for (int e = 0; e < STEP; ++e) s.cdf[i + e + 1] = sum += w[e];
+      }
+    }
+    __syncthreads();
+    target = a.uniforms[n_row] * s.cdf[STRIPES];
+    // exactly one stripe satisfies prefix <= target < prefix + mine
+    // (mine > 0 guaranteed for the owner since the CDF strictly increases
+    // across it); fp edge cases fall through to the fallback below
+    if (t < STRIPES && mine > 0.f && s.cdf[t] <= target && target < s.cdf[t + 1]) s.n = t;
+    __syncthreads();
+    n = s.n;
+    __syncthreads();
+    if (n >= 0) ahead = s.cdf[n];
   }
-  __syncthreads();
-  const Sum target = (Sum)a.uniforms[n_row] * (Sum)s.cdf[STRIPES];
-  // exactly one stripe satisfies prefix <= target < prefix + mine
-  // (mine > 0 guaranteed for the owner since the CDF strictly increases
-  // across it); fp edge cases fall through to the fallback below
-  if (t < STRIPES && mine > 0.0 && s.cdf[t] <= target && target < s.cdf[t + 1]) s.n = t;
-  __syncthreads();
-  const int n = s.n;
-  __syncthreads();
   if (n >= 0) {
     // the stripe's weights, added up in order by one thread until they exceed the target;
     // its last kept token if rounding lets none do so
@@ -520,7 +548,7 @@ INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t km
     if (last >= 0) atomicMax(&s.pick, last);
     __syncthreads();
     if (t == 0) {
-      Sum cum = (Sum)s.cdf[n];
+      Sum cum = ahead;
       int first = -1;
       for (int j = 0; j < here && first < 0; j += STEP) {
         float w[STEP], fours[STEP / 4];
@@ -531,9 +559,11 @@ INLINE void draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t km
           if constexpr (CUTS) {
             fours[e / 4] = sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
             upto += fours[e / 4];
-          } else {
-            upto = upto + w[e] + w[e + 1] + w[e + 2] + w[e + 3];
           }
+        }
+        if constexpr (!CUTS) {
+#pragma unroll
+          for (int e = 0; e < STEP; ++e) upto += w[e];
         }
         if (!(upto <= target)) {  // the same sums again: weights are not negative
           if constexpr (CUTS) {
@@ -831,7 +861,7 @@ INLINE void chunk_sums(ChunkShared& s, const SampleArgs& a, const Chunk& c, cons
   const bool by_value = kmin == 0 || (least == least && least != 0.f);
   const float from = kmin == 0 ? -INFINITY : least;
   float ahead[MOST];
-  std::conditional_t<CUTS, double, float> mine = 0;
+  SumOf<CUTS> mine = 0;
   auto fetch = [&](int j0) {
 #pragma unroll
     for (int k = 0; k < MOST; ++k)
@@ -877,7 +907,8 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(const SampleArgs a, Row
 
 struct DrawShared : ChunkForm {
   alignas(16) float buffer[MOST_VOCAB / STRIPES + 64];
-  double stripe[STRIPES], cdf[STRIPES + 1];
+  float stripe[STRIPES], cdf[STRIPES + 1];
+  double wave[WAVES], above;
   int n, pick;
 };
 
@@ -898,7 +929,7 @@ __global__ __launch_bounds__(256) void draw_kernel(const SampleArgs a, const Row
   if (want.by_k || want.by_p)
     draw<true>(s, a, row, n_row, plan.kmin, state.stripe[threadIdx.x]);
   else
-    draw<false>(s, a, row, n_row, plan.kmin, state.stripe[threadIdx.x]);
+    draw<false>(s, a, row, n_row, plan.kmin, (float)state.stripe[threadIdx.x]);
 }
 
 // The key of a list at which the sum from the top, with what is ``above``, reaches target, the
@@ -1036,17 +1067,15 @@ INLINE uint32_t least_of_list(S& s, const uint32_t* list, int n, double above, d
 }
 
 // inverse-CDF draw in token-id order over the kept set, {key >= kmin}
-template <typename S, typename R>
-INLINE void sum_and_draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin, bool plain,
-                         bool cuts) {
+template <bool CUTS, typename S, typename R>
+INLINE void sum_and_draw(S& s, const SampleArgs& a, const R& row, int n_row, uint32_t kmin,
+                         bool plain) {
   constexpr int WG = S::WG, TILE = S::TILE;
-  const int t = threadIdx.x, V = row.V;
-  const int stride = cuts ? stripe_tokens<true>(V) : stripe_tokens<false>(V);
+  const int t = threadIdx.x, V = row.V, stride = stripe_tokens<CUTS>(V);
   // Stripe n is tokens [n * stride, (n + 1) * stride).
   constexpr int PER = STRIPES * TILE / WG, ROWS = WG / TILE;  // a thread's tokens of a tile
   // token of the thread's k-th of a tile: k * ROWS stripes on
   const int r = t / TILE, c = t % TILE, i_first = r * stride + c;
-  auto weight = [&](float v) { return cuts ? row.template weight<true>(v) : row.template weight<false>(v); };
   float ahead[PER];
   auto fetch = [&](int j0) {
 #pragma unroll
@@ -1057,15 +1086,21 @@ INLINE void sum_and_draw(S& s, const SampleArgs& a, const R& row, int n_row, uin
   const float least = key2f(kmin);
   const bool by_value = kmin == 0 || (least == least && least != 0.f);
   const float from = kmin == 0 ? -INFINITY : least;
-  double mine = 0.0;  // or a sum in fp32, which it holds as it is
+  const bool even = V == STRIPES * stride;  // no stripe is shorter
+  SumOf<CUTS> mine = 0;
   fetch(0);
   for (int j0 = 0; j0 < stride; j0 += TILE) {
     float(*tile)[TILE + 4] = s.tile[j0 / TILE % 2];
-    if (by_value && plain && !row.mask && j0 + TILE <= stride) {
+    const bool by_values = by_value && plain && !row.mask && j0 + TILE <= stride;
+    if (by_values && even) {
+#pragma unroll
+      for (int k = 0; k < PER; ++k)
+        tile[k * ROWS + r][c] = ahead[k] >= from ? row.template weight<CUTS>(ahead[k]) : 0.f;
+    } else if (by_values) {
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
         const bool in = ahead[k] >= from && k * ROWS * stride + j0 + i_first < V;
-        tile[k * ROWS + r][c] = in ? weight(ahead[k]) : 0.f;
+        tile[k * ROWS + r][c] = in ? row.template weight<CUTS>(ahead[k]) : 0.f;
       }
     } else {
 #pragma unroll
@@ -1073,23 +1108,14 @@ INLINE void sum_and_draw(S& s, const SampleArgs& a, const R& row, int n_row, uin
         const int i = k * ROWS * stride + j0 + i_first;
         const bool in = j0 + c < stride && i < V && f2key(ahead[k]) >= kmin &&
                         !(row.mask && !row.mask[i]);
-        tile[k * ROWS + r][c] = in ? weight(ahead[k]) : 0.f;
+        tile[k * ROWS + r][c] = in ? row.template weight<CUTS>(ahead[k]) : 0.f;
       }
     }
     if (j0 + TILE < stride) fetch(j0 + TILE);
     __syncthreads();  // the other tile is added up before it is written again
-    if (t < STRIPES && cuts) {
-      add_tile<true, TILE>(tile[t], mine);
-    } else if (t < STRIPES) {
-      float sum = (float)mine;
-      add_tile<false, TILE>(tile[t], sum);
-      mine = sum;
-    }
+    if (t < STRIPES) add_tile<CUTS, TILE>(tile[t], mine);
   }
-  if (cuts)
-    draw<true>(s, a, row, n_row, kmin, mine);
-  else
-    draw<false>(s, a, row, n_row, kmin, mine);
+  draw<CUTS>(s, a, row, n_row, kmin, mine);
 }
 
 // ---- a row by one workgroup, in as many passes over it as its thresholds call for
@@ -1137,7 +1163,10 @@ INLINE void whole_row(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG
     if (pmin > kmin) kmin = pmin;
   }
 
-  sum_and_draw(s, a, row, n_row, kmin, plain, by_k || by_p);
+  if (by_k || by_p)
+    sum_and_draw<true>(s, a, row, n_row, kmin, plain);
+  else
+    sum_and_draw<false>(s, a, row, n_row, kmin, plain);
 }
 
 // ---- a row by one workgroup, by units of 16 bytes
@@ -1270,6 +1299,7 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   constexpr int N = U::N, WAVES = S::WAVES;
   const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6), V = a.V;
   if (V % N || (uintptr_t)row.x % 16) return false;
+  const bool cuts = want.by_k || want.by_p;
   if (!want.greedy && want.by_p && !(want.p > 0.f && (want.by_k || want.p <= MOST_P(V)))) return false;
   U units_of;
   units_of.x = (const char*)row.x;
@@ -1277,18 +1307,16 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   units_of.count = V / N;
   units_of.turns = (units_of.count + 64 * WAVES - 1) / (64 * WAVES);
   units_of.first = wid * units_of.turns * 64;
-  const bool cuts = want.by_k || want.by_p;
-  if (!want.greedy && cuts)
-    for (int i = t; i < UNIT_BUCKETS * 16; i += S::WG) ((u32x4*)s.column)[i] = u32x4{};
-  if (t == 0) s.n = 0;
-
   // ---- 1
-  u32x4 held[HELD];
-#pragma unroll
-  for (int k = 0; k < HELD; ++k) held[k] = units_of.turn(k);
   float mx = -3.4e38f, least = INFINITY;
   int best = 1 << 30, odd = 0;
   if (want.greedy) {
+    // loads beyond a short row's end take longer than the passes save: 64 x 8192 7.6 us, 7.0 by
+    // whole_row(); 64 x 16384 7.5 and 7.7
+    if (units_of.turns < 4) return false;
+    u32x4 held[HELD];
+#pragma unroll
+    for (int k = 0; k < HELD; ++k) held[k] = units_of.turn(k);
     units_of.template each<true>(held, [&](const u32x4& v, int k) {
       float y = -3.4e38f;
 #pragma unroll
@@ -1312,7 +1340,14 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
     }
     return true;
   }
-  if (!cuts) return false;  // here: ahead of the greedy rows the compiler spills registers
+  // plain rows turn back ahead of the loads (61 us and 49: 190 x 128256), which greedy rows have
+  // their own of: with one set of them for all rows, and a return ahead of it, registers spill
+  if (!cuts) return false;
+  u32x4 held[HELD];
+#pragma unroll
+  for (int k = 0; k < HELD; ++k) held[k] = units_of.turn(k);
+  if (t == 0) s.n = 0;
+  for (int i = t; i < UNIT_BUCKETS * 16; i += S::WG) ((u32x4*)s.column)[i] = u32x4{};
   unsigned long long odd_lanes = 0;
   units_of.template each<true>(held, [&](const u32x4& v, int) {
 #pragma unroll
