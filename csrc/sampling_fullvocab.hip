@@ -1179,8 +1179,8 @@ INLINE void whole_row(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG
 //     per bucket and lane the count and the sum of the distances within it, in one word, so that no
 //     two lanes of a wave meet (64-bit atomics on one table took 75 us instead of 10).  A bucket's
 //     mass is known to 4e-4 from both, so which buckets the boundary can be in, and no weight is made
-//   3 the weights above those buckets in a thread's own sum, the keys in them into a list, from which the
-//     least kept key follows exactly
+//   3 the weights above those buckets in a thread's own sum in 64 bits, the keys in them into a list, from
+//     which the least kept key follows exactly
 // The draw goes to the wave that has the target, then to its turn, a unit, a token, in token-id order.
 // 190 rows of 128256 in fp32, whole_row() and this, us: greedy 24.6 and 22.5, top-k 80 and 55, top-p 95 and
 // 72, both 135 and 60, top-p 0.9 at a temperature of 6.4 100 and 74; bf16 22 and 14, 70 and 45, 92 and 67,
@@ -1435,15 +1435,15 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   // ---- 3
   // as the buckets are, whose scale differs by a power of two
   const float edge_lo = lo * (-1.f / PER_OCTAVE), edge_hi = hi * (-1.f / PER_OCTAVE);
+  // The masses that a top-p compares are added up weight by weight, so that the small ones count beside
+  // a large one: by fours in fp32 a row's is off by up to 2^-25 of it.  190 x 128256 top-p 77 us, by
+  // fours 73.  A top-k compares counts, and its sums are those of the draw alone
+  const bool by_mass = !want.by_k;
   double kept = 0.0, all = 0.0;
   // not the differences of pass 2, which would be kept for it beside the logits
   float top = mx;
   asm volatile("" : "+v"(top));
   auto weigh = [&](float x) { return __builtin_amdgcn_exp2f((x - top) * per_octave); };
-  auto add_fours = [](const float (&w)[N], double& to) {
-#pragma unroll
-    for (int e = 0; e < N; e += 4) to += (double)sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
-  };
   units_of.template each<false>(held, [&](const u32x4& v, int) {
     float w[N], in[N];
 #pragma unroll
@@ -1459,8 +1459,17 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
         }
       }
     }
-    add_fours(in, kept);
-    if (want.by_p) add_fours(w, all);
+    if (by_mass) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        kept += (double)in[e];
+        all += (double)w[e];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < N; e += 4)
+        kept += (double)sum_of_four(in[e], in[e + 1], in[e + 2], in[e + 3]);
+    }
   });
   uint32_t kmin = 0;
   if (t < WAVES) s.wave_units[t] = 0;
@@ -1521,7 +1530,8 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
     float w[N];
     weights_of(first + k * 64 + lane, w);
     double sum = 0.0;
-    add_fours(w, sum);
+#pragma unroll
+    for (int e = 0; e < N; ++e) sum += (double)w[e];
     s.unit_sum[k * 64 + lane] = sum;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
@@ -1549,11 +1559,10 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
     double upto = at_turn + ahead;
     int pick = -1, last = 0;
 #pragma unroll
-    for (int e = 0; e < N; e += 4) {
-      const float four = sum_of_four(w[e], w[e + 1], w[e + 2], w[e + 3]);
-      if (four > 0.f) last = e + token_of_four(w + e, 0.0, INFINITY);
-      if (pick < 0 && !end && upto + four > rest) pick = e + token_of_four(w + e, upto, rest);
-      upto += four;
+    for (int e = 0; e < N; ++e) {
+      upto += (double)w[e];
+      if (w[e] > 0.f) last = e;
+      if (pick < 0 && !end && w[e] > 0.f && upto > rest) pick = e;
     }
     a.out[n_row] = min(unit * N + (pick < 0 ? last : pick), V - 1);
   }

@@ -833,6 +833,45 @@ def test_sample_fullvocab_chunks(V, dtype):
 
 @requires_gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("chunks", [0, 32])
+def test_sample_fullvocab_mass_of_small_weights(dtype, chunks):
+    """All weights are powers of two: 16384 of 1, next to each three of 2^-26, then groups of 1/2 and
+    1/4, the last of which a top-p just reaches.  Their sum is exact in 64 bits, and the small ones,
+    which are 7e-4 together, count: by fours in fp32 they are lost beside the 1, and so is the group."""
+    C, n, V = hip()._C, 16384, 1 << 17
+    T = torch.tensor(1.44269504)  # logits are octaves: 1 / T times log2 e rounds to 1
+    assert T.reciprocal() * 1.44269504 == 1
+    rows, ps, firsts = [], [], []
+    for half in range(200, 1000, 40):
+        for quarter in range(1000, 3000, 100):
+            above = n + half / 2
+            total = above + quarter / 4 + 3 * n * 2.0**-26
+            p = torch.tensor(above / total)
+            while float(p) * total <= above:
+                p = torch.nextafter(p, torch.tensor(1.0))
+            if 2e-5 < float(p) * total - above < 4e-4:
+                rows.append([(half, -1.0), (quarter, -2.0)])
+                ps.append(p)
+                firsts.append((4 * n + half, above, above + quarter / 4))
+    assert len(rows) >= 20
+    x = torch.full((len(rows), V), float("-inf"))
+    x[:, : 4 * n] = -26.0
+    x[:, : 4 * n : 4] = 0.0
+    for row, groups in zip(x, rows):
+        at = 4 * n
+        for count, value in groups:
+            row[at : at + count] = value
+            at += count
+    out, u = torch.full((len(rows),), -1, device="cuda"), torch.full((len(rows),), 0.9995)
+    C.sample_fullvocab(out, x.to("cuda", dtype), T.expand(len(rows)).contiguous().cuda(),
+                       torch.zeros(len(rows), dtype=torch.long, device="cuda"),
+                       torch.stack(ps).cuda(), u.cuda(), None, None, chunks)
+    want = [at + int((float(u[0]) * total - above) * 4) for at, above, total in firsts]
+    assert out.tolist() == want
+
+
+@requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("V", [8200, 32000, 128256, 262144])
 @pytest.mark.parametrize("std", [0.05, 2.5, 8.0])
 def test_sample_fullvocab_rows_by_units(V, std, dtype):
