@@ -53,7 +53,8 @@
 #define PER_LOGIT 8  // likewise, of a top-k
 // beyond it more keys are within the masses' error than the list takes: normal logits 3000 at 0.99 of
 // 128256 and 4400 of 152064
-#define MOST_P(V) (1.f - (V) * 7.6e-8f)
+// (from 0.999 on the masses' error reaches all of the row)
+#define MOST_P(V) fminf(1.f - (V) * 7.6e-8f, 0.9985f)
 
 // order-preserving float -> uint32 key
 __device__ __forceinline__ uint32_t f2key(float x) {
@@ -130,7 +131,7 @@ struct Shared : F {
   double wave[F::WAVES];
   float red[F::WAVES];
   int red_i[F::WAVES], red_odd[F::WAVES];
-  int n, pick;
+  int n, pick, finite, listed;
   uint32_t lo, hi;
   double above;
 };
@@ -1300,7 +1301,11 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6), V = a.V;
   if (V % N || (uintptr_t)row.x % 16) return false;
   const bool cuts = want.by_k || want.by_p;
-  if (!want.greedy && want.by_p && !(want.p > 0.f && (want.by_k || want.p <= MOST_P(V)))) return false;
+  // with both the list has all that the top-k keeps: 190 x 128256 top-k 7000 and top-p 152 us, in 3
+  // passes ahead of whole_row() 200
+  if (!want.greedy && want.by_p &&
+      !(want.p > 0.f && (want.by_k ? want.k <= UNIT_KEYS : want.p <= MOST_P(V))))
+    return false;
   U units_of;
   units_of.x = (const char*)row.x;
   units_of.mask = row.mask;
@@ -1346,10 +1351,23 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   u32x4 held[HELD];
 #pragma unroll
   for (int k = 0; k < HELD; ++k) held[k] = units_of.turn(k);
-  if (t == 0) s.n = 0;
+  if (t == 0) s.n = s.finite = s.listed = 0;
   for (int i = t; i < UNIT_BUCKETS * 16; i += S::WG) ((u32x4*)s.column)[i] = u32x4{};
   unsigned long long odd_lanes = 0;
+  int finite = 0;  // of a masked row: the wave's logits above -inf
   units_of.template each<true>(held, [&](const u32x4& v, int) {
+    if (MASKED && row.mask) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        const float x = U::at(v, e);
+        const bool some = !(x == -INFINITY);
+        mx = fmaxf(mx, x);
+        least = fminf(least, some ? x : INFINITY);
+        finite += __popcll(__ballot(some));
+        odd_lanes |= __ballot(x != x);
+      }
+      return;
+    }
 #pragma unroll
     for (int e = 0; e < N; e += 2) {
       const float x = U::at(v, e), y = U::at(v, e + 1);
@@ -1364,11 +1382,18 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   const float per_octave = row.scale;
   float scale = want.by_k ? (float)PER_LOGIT / PER_OCTAVE : per_octave;
   // finer ones where the row does not reach the last one
+  if (lane == 0) atomicAdd(&s.finite, finite);
   least = block_least(s, least);
-  const float span = (mx - least) * scale, most = UNIT_BUCKETS / PER_OCTAVE - 2;
-  if (!(span > 1e-20f)) return false;
-  if (span < most) scale *= most / span;
-  if (!(scale < 1e25f)) return false;
+  // a masked row of no more logits than its top-k keeps them all: no buckets.  190 x 128256 of 256 tokens,
+  // top-k 2000: 57 us, 222 where the buckets were looked through for it before whole_row(), which takes
+  // 187.  Likewise buckets span the allowed logits alone: normal ones times 0.05, top-k 78, 232 and 171
+  const bool whole = MASKED && row.mask && want.by_k && s.finite <= want.k;
+  if (!whole) {
+    const float span = (mx - least) * scale, most = UNIT_BUCKETS / PER_OCTAVE - 2;
+    if (!(span > 1e-20f)) return false;
+    if (span < most) scale *= most / span;
+    if (!(scale < 1e25f)) return false;
+  }
   const float fine = scale * (PER_OCTAVE * PARTS), bucket_octaves = per_octave / scale / PER_OCTAVE;
   if (odd || !(mx > -1e37f && mx < INFINITY) || !(per_octave < 1e20f && per_octave > 1e-20f)) return false;
   row.m = mx;
@@ -1376,7 +1401,7 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   // ---- 2: the buckets lo .. hi - 1 that the boundary can be in
   int lo = 0, hi = 0;
   double k_above = 0.0;
-  {
+  if (!whole) {
     uint32_t* const mine = &s.column[0][lane];
     units_of.template each<false>(held, [&](const u32x4& v, int) {
 #pragma unroll
@@ -1430,11 +1455,15 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
     k_above = want.by_k && !want.by_p ? s.above : 0.0;
     // what is beyond the last bucket is not told apart
     if (hi >= UNIT_BUCKETS || lo >= hi) return false;
+    if (n > 0.0 && b >= lo && b < hi) atomicAdd(&s.listed, (int)numbers);
+    __syncthreads();
+    if (s.listed > UNIT_KEYS) return false;  // not after a pass that lists them, 30 us
   }
 
   // ---- 3
   // as the buckets are, whose scale differs by a power of two
-  const float edge_lo = lo * (-1.f / PER_OCTAVE), edge_hi = hi * (-1.f / PER_OCTAVE);
+  const float edge_lo = whole && !want.by_p ? -INFINITY : lo * (-1.f / PER_OCTAVE);
+  const float edge_hi = whole ? -INFINITY : hi * (-1.f / PER_OCTAVE);
   // The masses that a top-p compares are added up weight by weight, so that the small ones count beside
   // a large one: by fours in fp32 a row's is off by up to 2^-25 of it.  190 x 128256 top-p 77 us, by
   // fours 73.  A top-k compares counts, and its sums are those of the draw alone
@@ -1473,7 +1502,7 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   });
   uint32_t kmin = 0;
   if (t < WAVES) s.wave_units[t] = 0;
-  {
+  if (!whole || want.by_p) {
     const double above = want.by_k ? k_above : block_total(s, kept);
     const double target = want.by_k ? want.k : (double)want.p * block_total(s, all);
     __syncthreads();

@@ -924,6 +924,45 @@ def test_sample_fullvocab_rows_by_units(V, std, dtype):
     assert torch.equal(out, first.values)
 
 
+@requires_gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [8200, 128256])
+@pytest.mark.parametrize("std", [0.0, 0.02, 2.5])
+def test_sample_fullvocab_few_allowed(V, std, dtype):
+    """Masks that leave fewer tokens than a top-k, as many, and more, some of them of no weight, in a
+    narrow range and all alike: against 64 bits, where one draw of a row's five may fall between sums."""
+    C, gen = hip()._C, torch.Generator(device="cuda").manual_seed(V)
+    counts = [1, 2, 49, 50, 51, 320, 321, 3000, 4097, 6000]
+    B = len(counts)
+    x = (torch.randn(B, V, generator=gen, device="cuda") * std + 0.0).to(dtype)  # and no -0
+    mask = torch.zeros(B, V, dtype=torch.bool, device="cuda")
+    for i, n in enumerate(counts):
+        at = torch.randperm(V, generator=gen, device="cuda")[:n]
+        mask[i, at] = True
+        x[i, at[: n // 8]] = float("-inf")
+    v = torch.where(mask, x.double(), -torch.inf)
+    to, one = torch.arange(B, device="cuda").int(), torch.ones(B, device="cuda")
+    finite = torch.where(v > -torch.inf, v, 0.0)
+    for k in (1, 50, 4096, 4097, V - 1):
+        keep = (v >= v.topk(k, 1).values[:, -1:]) & (v > -torch.inf)
+        for p in (1.0, 0.9):
+            w = torch.where(keep, ((finite - v.max(1, keepdim=True).values) / 0.8).exp(), 0.0)
+            if p < 1:
+                top, order = w.sort(1, descending=True)
+                ahead = top.cumsum(1) - top
+                n = (ahead < (one * p).double().view(-1, 1) * w.sum(1, keepdim=True)).sum(1)
+                w = torch.where(v >= v.gather(1, order).gather(1, n.view(-1, 1) - 1), w, 0.0)
+            cdf, off = w.cumsum(1), 0
+            for _ in range(5):
+                u = torch.rand(B, generator=gen, device="cuda")
+                out = torch.full((B,), -1, device="cuda")
+                C.sample_fullvocab(out, x, one * 0.8, (one * k).long(), one * p, u, mask, to, 0)
+                assert bool(mask.gather(1, out.view(-1, 1)).all())
+                want = (cdf > u.double().view(-1, 1) * cdf[:, -1:]).int().argmax(1)
+                off += int((out != want).sum())
+            assert off <= 1, (k, p)
+
+
 @pytest.mark.gpu
 def test_sample_fullvocab_vs_oracle():
     """csrc/sampling_fullvocab.hip vs the fp32 reference over a Llama-3
