@@ -456,7 +456,7 @@ INLINE Row<T, WG> row_of(const SampleArgs& a, int n) {
 // A stripe's weights of a tile
 template <bool CUTS, int TILE>
 INLINE void add_tile(const float* tile, SumOf<CUTS>& sum) {
-  constexpr int FOURS = TILE < 32 ? TILE / 4 : 8;
+  constexpr int FOURS = !CUTS || TILE < 32 ? TILE / 4 : 8;
 #pragma unroll 1
   for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
     float4 w[FOURS];
@@ -1007,7 +1007,8 @@ INLINE uint32_t least_of_list(S& s, const uint32_t* list, int n, double above, d
   auto each_key = [&](auto f) {
     for (int i = threadIdx.x; i < n; i += S::WG) f(s.key[i]);
   };
-  auto find = [&](auto by_mass, double above, double target) {
+  auto find = [&, first = lo, last = hi](auto by_mass, double above, double target) {
+    uint32_t lo = first, hi = last;
     constexpr bool BY_MASS = decltype(by_mass)::value;
     if (n <= RANKED) return rank_keys<BY_MASS>(s, s.key, s.key_mass, n, above, target);
     if constexpr (S::WG == 1024) {
@@ -1043,6 +1044,15 @@ INLINE uint32_t least_of_list(S& s, const uint32_t* list, int n, double above, d
           }
         __syncthreads();
         const int few = s.n;
+        // many of one key, as logits of 16 bits have them, need neither ranks nor a split: 16 x 128256 in
+        // chunks, logits of a twentieth and a top-p of 0.9, 75 us by ranks, 62 so
+        hi -= (uint32_t)bucket << shift;
+        lo = max(lo, hi - ((1u << shift) - 1));
+        const uint32_t one = s.sub_key[0];
+        int others = 0;
+        for (int i = threadIdx.x; i < n; i += S::WG)
+          others |= s.key[i] >= lo && s.key[i] <= hi && s.key[i] != one;
+        if (!__syncthreads_or(others)) return one;
         if (few <= RANKED) {
           if (threadIdx.x < 4) {
             s.sub_key[few + threadIdx.x] = 0;
@@ -1051,7 +1061,7 @@ INLINE uint32_t least_of_list(S& s, const uint32_t* list, int n, double above, d
           __syncthreads();
           return rank_keys<BY_MASS>(s, s.sub_key, s.sub_mass, few, sub_above, target);
         }
-        __syncthreads();
+        above = sub_above;
       }
     }
     return split_keys<BY_MASS>(s, row, lo, hi, above, target, each_key);
@@ -1301,10 +1311,10 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6), V = a.V;
   if (V % N || (uintptr_t)row.x % 16) return false;
   const bool cuts = want.by_k || want.by_p;
-  // with both the list has all that the top-k keeps: 190 x 128256 top-k 7000 and top-p 152 us, in 3
-  // passes ahead of whole_row() 200
+  // with both the list has all that the top-k keeps, and what else its last bucket has: 190 x 128256
+  // top-k 7000 and top-p 152 us, in 3 passes ahead of whole_row() 200
   if (!want.greedy && want.by_p &&
-      !(want.p > 0.f && (want.by_k ? want.k <= UNIT_KEYS : want.p <= MOST_P(V))))
+      !(want.p > 0.f && (want.by_k ? want.k <= UNIT_KEYS / 8 * 7 : want.p <= MOST_P(V))))
     return false;
   U units_of;
   units_of.x = (const char*)row.x;
