@@ -56,6 +56,9 @@
 // (from 0.999 on the masses' error reaches all of the row)
 #define MOST_P(V) fminf(1.f - (V) * 7.6e-8f, 0.9985f)
 
+// the number before the -3.4e38 that a row's largest logit is at least: what is equal to that is found
+#define BELOW -0x1.ff933ep127f
+
 // order-preserving float -> uint32 key
 __device__ __forceinline__ uint32_t f2key(float x) {
   uint32_t u = __float_as_uint(x);
@@ -1323,7 +1326,7 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
   units_of.turns = (units_of.count + 64 * WAVES - 1) / (64 * WAVES);
   units_of.first = wid * units_of.turns * 64;
   // ---- 1
-  float mx = -3.4e38f, least = INFINITY;
+  float mx = BELOW, least = INFINITY;
   int best = 1 << 30, odd = 0;
   if (want.greedy) {
     // loads beyond a short row's end take longer than the passes save: 64 x 8192 7.6 us, 7.0 by
@@ -1333,7 +1336,7 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
 #pragma unroll
     for (int k = 0; k < HELD; ++k) held[k] = units_of.turn(k);
     units_of.template each<true>(held, [&](const u32x4& v, int k) {
-      float y = -3.4e38f;
+      float y = BELOW;
 #pragma unroll
       for (int e = 0; e < N; e += 2) y = max3(y, U::at(v, e), U::at(v, e + 1));
       if (y > mx) {

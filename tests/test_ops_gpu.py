@@ -925,6 +925,28 @@ def test_sample_fullvocab_rows_by_units(V, std, dtype):
 
 
 @requires_gpu
+@pytest.mark.parametrize("V,chunks", [(600, 0), (32000, 0), (32001, 0), (128256, 0), (128256, 16)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_sample_fullvocab_greedy_of_lowest_logits(V, chunks, masked):
+    """The first of the largest logits, however low: -3.4e38, with which masks are written, is one."""
+    C, B = hip()._C, 4
+    x = torch.full((B, V), float("-inf"), device="cuda")
+    first = [0, 77, V // 2, V - 1]
+    for i, at in enumerate(first):
+        x[i, at:] = -3.4e38
+    x[1, 78:] = torch.finfo(torch.float32).min
+    mask = torch.ones(B, V, dtype=torch.bool, device="cuda") if masked else None
+    if masked:
+        for i, at in enumerate(first):
+            x[i, :at] = 1.0
+            mask[i, :at] = False
+    to = torch.arange(B, device="cuda").int() if masked else None
+    out, zero = torch.full((B,), -1, device="cuda"), torch.zeros(B, device="cuda")
+    C.sample_fullvocab(out, x, zero, zero.long(), zero + 1, zero, mask, to, chunks)
+    assert out.tolist() == first
+
+
+@requires_gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("V", [8200, 128256])
 @pytest.mark.parametrize("std", [0.0, 0.02, 2.5])
