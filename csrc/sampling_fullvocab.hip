@@ -49,6 +49,7 @@
 #define UNIT_KEYS 4096
 #define UNIT_BUCKETS 512
 #define PARTS 128    // of a bucket
+#define PARTS_OF_BUCKET (1 << 19)  // of a column: from there on its count
 #define PER_OCTAVE 16
 #define PER_LOGIT 8  // likewise, of a top-k
 // beyond it more keys are within the masses' error than the list takes: normal logits 3000 at 0.99 of
@@ -1422,21 +1423,23 @@ INLINE bool row_by_units(S& s, const SampleArgs& a, const Wants& want, Row<T, S:
         const float d = (mx - U::at(v, e)) * fine;
         if (d < (float)(UNIT_BUCKETS * PARTS)) {  // beyond 32 octaves all weigh less than the slack
           const uint32_t q = (uint32_t)d;
-          atomicAdd(mine + q / PARTS * 64, (uint32_t)(1 << 19) | (q % PARTS));
+          atomicAdd(mine + q / PARTS * 64, (uint32_t)PARTS_OF_BUCKET | (q % PARTS));
         }
       }
     });
     if (t == 0) s.lo = s.hi = UNIT_BUCKETS;
     __syncthreads();
     // two threads a bucket
-    static_assert(S::WG == 2 * UNIT_BUCKETS && MOST_VOCAB / 64 <= 1 << 13 && PARTS <= 128);
+    static_assert(S::WG == 2 * UNIT_BUCKETS);
+    static_assert(MOST_VOCAB / 64 * (PARTS - 1) < PARTS_OF_BUCKET, "a lane's parts stay below its count");
+    static_assert((int64_t)MOST_VOCAB / 64 * PARTS_OF_BUCKET < 1ll << 32, "and its count in the word");
     const int b = t >> 1;
     uint32_t numbers = 0, parts = 0;
 #pragma unroll 4
     for (int i = 0; i < 32; ++i) {
       const uint32_t h = s.column[b][(i + lane) % 32 + (t & 1) * 32];
-      numbers += h >> 19;
-      parts += h & ((1 << 19) - 1);
+      numbers += h / PARTS_OF_BUCKET;
+      parts += h % PARTS_OF_BUCKET;
     }
     numbers += __shfl_xor(numbers, 1);
     parts += __shfl_xor(parts, 1);
