@@ -106,6 +106,7 @@ __device__ __forceinline__ int token_of_four(const float* w, double before, doub
 template <int THREADS, int TOKENS>
 struct Form {
   static constexpr int WG = THREADS, WAVES = WG / 64, TILE = TOKENS;
+  static constexpr bool LISTS = WG == 1024;  // rows by units, and lists of rows in chunks
   static constexpr int BUCKETS = (FIRST + WG - 1) / WG;  // of a thread
 };
 
@@ -118,17 +119,17 @@ struct Shared : F {
     float tile[2][STRIPES][F::TILE + 4];
     float buffer[2 * STRIPES * (F::TILE + 4)];  // of the drawn stripe
     // a row's by units, by lanes, so that no two lanes of a wave meet: count, and parts of a bucket
-    alignas(16) uint32_t column[F::WG < 1024 ? 1 : UNIT_BUCKETS][64];
+    alignas(16) uint32_t column[F::LISTS ? UNIT_BUCKETS : 1][64];
     struct {
-      alignas(16) uint32_t key[UNIT_KEYS];  // of a row in chunks, or by units
-      unsigned long long key_mass[UNIT_KEYS];
-      int key_wave[F::WG < 1024 ? 1 : UNIT_KEYS];
-      alignas(16) uint32_t sub_key[RANKED + 4];
-      unsigned long long sub_mass[RANKED + 4];
+      alignas(16) uint32_t key[F::LISTS ? UNIT_KEYS : 1];  // of a row in chunks, or by units
+      unsigned long long key_mass[F::LISTS ? UNIT_KEYS : 1];
+      int key_wave[F::LISTS ? UNIT_KEYS : 1];
+      alignas(16) uint32_t sub_key[F::LISTS ? RANKED + 4 : 1];
+      unsigned long long sub_mass[F::LISTS ? RANKED + 4 : 1];
       unsigned long long wave_units[F::WAVES];
       // of the drawn wave
-      double unit_sum[F::WG < 1024 ? 1 : MOST_VOCAB / 4 / F::WAVES + 64];
-      double turn_sum[F::WG < 1024 ? 1 : MOST_VOCAB / 256 / F::WAVES + 1];
+      double unit_sum[F::LISTS ? MOST_VOCAB / 4 / F::WAVES + 64 : 1];
+      double turn_sum[F::LISTS ? MOST_VOCAB / 256 / F::WAVES + 1 : 1];
     };
   };
   float stripe[STRIPES], cdf[STRIPES + 1];  // of a row without a threshold
@@ -1015,7 +1016,7 @@ INLINE uint32_t least_of_list(S& s, const uint32_t* list, int n, double above, d
     uint32_t lo = first, hi = last;
     constexpr bool BY_MASS = decltype(by_mass)::value;
     if (n <= RANKED) return rank_keys<BY_MASS>(s, s.key, s.key_mass, n, above, target);
-    if constexpr (S::WG == 1024) {
+    if constexpr (S::LISTS) {
       // a round of split_keys(), after which its bucket has few: 500 keys 6 us, its two rounds 12
       const int shift = hi - lo < SPLIT ? 0 : 32 - __builtin_clz(hi - lo) - 10;
       for (int i = threadIdx.x; i < SPLIT; i += S::WG) s.mass[i] = 0;
@@ -1632,7 +1633,7 @@ __global__ __launch_bounds__(F::WG) void sample_fullvocab_kernel(const SampleArg
       if (threadIdx.x == 0) state.plan.kmin = least;
       return;
     }
-  } else if constexpr (F::WG == 1024) {
+  } else if constexpr (F::LISTS) {
     if (row_by_units<T, MASKED>(s, a, want, row, n_row)) return;
   }
   whole_row<T>(s, a, want, row, n_row);
