@@ -262,11 +262,18 @@ def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefi
     n_split = 1
     if mfma:
         keys = min(max_keys, window)
-        # workgroups that fill the chip: the tiles of a wide latent take a CU's LDS, but for up to 16 rows
-        # half of it.  40 x 200 to 6000 keys of rank 512, a step's 20 layers: 512 2400 us, 256 and 1024
-        # 2600 and 2455
-        fill = 256 if q.shape[2] >= 256 and mg > 1 else 512
-        n_split = max(1, min(_MAX_SPLIT, fill // tiles, -(-keys // 128)))
+        most = min(_MAX_SPLIT, -(-keys // 128))
+        # workgroups that fill the chip: the tiles of a wide latent take a CU's LDS
+        wide = q.shape[2] >= 256
+        n_split = max(1, min(most, (256 if wide else 512) // tiles))
+        # Or half of it for up to 16 rows, by smaller tiles, which pays for parts of 320 keys, or 768
+        # undivided, from 16 sequences on.  16 heads of rank 512, us by up to 256 workgroups and 512: 12 x
+        # 7500 31.1 and 32.8, 16 x 8000 38.8 and 35.5, 32 x 2000 of 250 keys a part 26.1 and 28.7, 40 x
+        # 2000 of 333 35.5 and 34.0, 64 x 4200 71 and 65; undivided 190 x 500 32.5 and 36.0, x 1000 56.4 and
+        # 53.4, 129 x 2000 98 and 64.  More workgroups than 512 gain nothing: 40 x 200 to 6000, a step's 20
+        # layers, 2400 by 512 and 2455 by 1024
+        if wide and mg == 1 and 16 <= tiles <= 256 and keys >= (320 * n_split if n_split > 1 else 768):
+            n_split = max(1, min(most, 512 // tiles))
     part = ml = None
     if n_split > 1:
         rows = q.shape[0] * q.shape[1]

@@ -132,8 +132,11 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
     }
   }
 
-  // Pages go from the tables to LDS, three tiles ahead, and become slots two tiles ahead: in registers
-  // they would be waited for, and with them, as loads come back in order, all of the tile behind them
+  // Where a CU has two workgroups pages go from the tables to LDS, three tiles ahead, and become slots two
+  // tiles ahead: in registers they would be waited for, and with them, as loads come back in order, all of
+  // the tile behind them.  A workgroup alone does not gain by it: 129 x 4096 keys of 32 heads 244 us so,
+  // 233 by registers and barriers that wait for the tile
+  constexpr bool APART = KT == 32;
   auto key_of = [&](int t) { return min(k_begin + t * KT + (int)threadIdx.x, k_end - 1); };
   auto ask_pages = [&](int t) {
     if (threadIdx.x < KT)
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
   put_slots(t_begin, table + key_of(t_begin) / a.kv_block);
   put_slots(t_begin + 1, table + key_of(t_begin + 1) / a.kv_block);
   __syncthreads();
-  ask_pages(t_begin + 2);
+  if constexpr (APART) ask_pages(t_begin + 2);
   stage(t_begin);
 
   f32x4_v o[MG][NR] = {};
@@ -180,21 +183,26 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
 
   // LDS writes of all waves are done, but not the loads of the next tile, which __syncthreads() waits for
   auto meet = [] {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    if constexpr (APART) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    } else {
+      __syncthreads();
+    }
   };
   for (int t = t_begin; t < t_end; ++t) {
     // tile t landed for every wave; tile t-1 is fully read
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     meet();
-    if (t + 3 < t_end) ask_pages(t + 3);
+    if constexpr (APART)
+      if (t + 3 < t_end) ask_pages(t + 3);
     if (t + 1 < t_end) stage(t + 1);
     const char* tile = lds + (t & 1) * TILE_BYTES;
 
     // scores: lane holds query row c, keys wid*16 + 4g + {0..3}
     f32x4_v s[MG] = {};
-    const bool scores = wid * 16 < KT;
+    const bool scores = KT == 64 || wid * 16 < KT;
     if (scores) {
       const char* krow = tile + (wid * 16 + c) * (ROW * 2);
 #pragma unroll
@@ -238,7 +246,8 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
 #pragma unroll
       for (int n = 0; n < NR; ++n) o[m][n] *= alpha;
     }
-    if (t + 2 < t_end) put_slots(t + 2, pages + (t & 1) * KT + threadIdx.x);  // tile t's slots were consumed by its stage
+    if (t + 2 < t_end)  // tile t's slots were consumed by its stage
+      put_slots(t + 2, APART ? pages + (t & 1) * KT + threadIdx.x : table + key_of(t + 2) / a.kv_block);
     meet();
 
     // values: A = latent columns (transposed read), B = probabilities
@@ -412,14 +421,16 @@ static void launch_tiles(const LatentArgs& a, int tiles, hipStream_t stream) {
 }
 
 // A tile is a chain of reads, products and three barriers, during which a CU with one workgroup waits:
-// with tiles of 32 keys of a wide latent it has two, where there are as many.  40 x 200 to 6000 keys of
-// 16 heads 72 us by 64 keys, 57 by 32; four tiles in LDS, three of them under way, of one workgroup a
+// with tiles of 32 keys of a wide latent it has two, where there are more than CUs.  40 x 200 to 6000 keys
+// of 16 heads 72 us by 64 keys, 57 by 32; four tiles in LDS, three of them under way, of one workgroup a
 // CU 91.  By 32 keys alone a step over 1 x 5000 1671 us, else 1651, over 8 x 200 to 800 1928 and 1893.
+// A few more than CUs wait for the longest of them, which is slower by 32 keys: 257 x 200 to 2000 99 us by
+// 64 keys, 114 by 32, 270 of them 122 and 120; of 100 to 500 34.8 and 36.2, 45.3 and 37.1.
 #define CUS 256
 template <int NR, int MG>
 static void launch_mfma(const LatentArgs& a, int tiles, hipStream_t stream) {
   if constexpr (MG == 1 && NR >= 4)
-    if (tiles * (int64_t)a.n_split > CUS) return launch_tiles<NR, MG, 32>(a, tiles, stream);
+    if (tiles * (int64_t)a.n_split > CUS + CUS / 32) return launch_tiles<NR, MG, 32>(a, tiles, stream);
   launch_tiles<NR, MG, 64>(a, tiles, stream);
 }
 

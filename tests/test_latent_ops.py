@@ -174,6 +174,9 @@ SHAPES = [
     (16, 512, None, 16, [(0, 20)] + [(7 * i, 1) for i in range(48)] + [(1000, 1)]),
     (9, 250, None, 4, [(0, 3)] + [(9 * i + 1, 1) for i in range(40)] + [(930, 1), (1023, 1)]),
     (5, 384, 900, 16, [(0, 2)] + [(23 * i, 1) for i in range(45)] + [(1100, 1)]),
+    # as many without a split: written by the smaller tiles themselves, few and many of them
+    (16, 512, None, 16, [(0, 3)] + [(i % 100, 1) for i in range(270)]),
+    (3, 250, 70, 4, [(0, 1)] + [(2 * i % 131, 1) for i in range(300)]),
 ]
 
 
