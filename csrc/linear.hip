@@ -194,6 +194,21 @@ extern "C" bool linear_fits(int tile, bool glu) {
   return tile >= 0 && tile < TILE_COUNT && !(glu && tiles[tile].fn % 4);
 }
 
+// (a^1.36 + b^1.36)^(1 / 1.36), by the ratio of a to b: a table's 256 steps of it, which are at most 1e-4
+// off, take a tenth of three powers
+struct Together {
+  double of[258];
+  Together() {
+    for (int i = 0; i < 258; ++i) of[i] = pow(1 + pow(i / 256.0, 1.36), 1 / 1.36);
+  }
+  double operator()(double a, double b) const {
+    const double high = a > b ? a : b, at = (a > b ? b : a) / high * 256;
+    const int i = (int)at;
+    return high * (of[i] + (at - i) * (of[i + 1] - of[i]));
+  }
+};
+static const Together together;
+
 // The tile and the parts that are expected to be the fastest, in us: the chunks of the busiest
 // CU beside the memory's time, for the operands once and for what tiles read again, and a launch.  Fitted
 // to 754 sizes of 5 to 2100 rows, 2048 to 32000 outputs and 1280 to 14336 inner elements; what it chooses is
@@ -201,32 +216,42 @@ extern "C" bool linear_fits(int tile, bool glu) {
 // elsewhere, and 24% where it is worst.  With steps by the fragments alone, max(0.015 fn fm, 0.053
 // (fn + fm)), 1.7 and 3.2%: 190 x 4096 x 14336 into the norm 39.8 and now 35.3, 190 x 6144 x 4096 into
 // the rotation 22.9 and 21.2, 61 x 4096 x 4096 17.0 and 13.7.
+// It is asked for every launch and takes 0.1 to 0.6 us, 0.3 to 3.8 with powers for each of up to 154 pairs.
 extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* splits) {
   static const int parts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
+  constexpr int PARTS = sizeof(parts) / sizeof(int);
   const bool glu = unit == LINEAR_SWIGLU || unit == LINEAR_GLU;
-  const int chunks = K / 64;
-  const double rows = 2.0 * M * K, weights = 2.0 * N * K;
+  const int chunks = K / 64, most = M > 2600 ? 1 : chunks / 4;
+  const double rows = 2.0 * M * K, weights = 2.0 * N * K, outs = (double)M * N;
+  int each[PARTS], count[PARTS], n = 1;
+  each[0] = chunks, count[0] = 1;
+  for (; n < PARTS && parts[n] <= most; ++n) {
+    each[n] = (chunks + parts[n] - 1) / parts[n];
+    count[n] = (chunks + each[n] - 1) / each[n];
+  }
   double best = 0;
   *tile = -1;
   for (int i = 0; i < TILE_COUNT; ++i) {
     const Tile& t = tiles[i];
     if (t.fm > 1 && (t.fm - 1) * 32 >= M) continue;  // rows of nothing
-    const int64_t high = ((int64_t)M + 32 * t.fm - 1) / (32 * t.fm);
-    const int64_t wide = ((int64_t)N + 32 * t.fn - 1) / (32 * t.fn);
-    for (int s : parts) {
+    const unsigned high = (M - 1u) / (32 * t.fm) + 1, wide = (N - 1u) / (32 * t.fn) + 1;
+    const int64_t grid = (int64_t)high * wide;
+    const double fragments = t.fn * t.fm;
+    const double ends = 0.09 * fragments + 0.09, again = (wide * rows + high * weights) / 160e6;
+    for (int j = 0; j < n; ++j) {
+      const int s = parts[j];
       if (s == 1 && !linear_fits(i, glu)) continue;
-      if (s > 1 && (chunks < 4 * s || M > 2600 || high * wide * s > 4 * CUS)) break;
-      const int each = (chunks + s - 1) / s, count = (chunks + each - 1) / each;
-      const int64_t works = high * wide * count;
-      const double busiest =
-          (double)((works + CUS - 1) / CUS) * (each * t.step + 0.09 * t.fn * t.fm + 0.09);
-      const double sums = (s > 1 ? 8.0 * count : glu ? 1.0 : 2.0) * M * N;
-      const double memory =
-          (weights + rows + sums) / 8.8e6 + (wide * rows + high * weights) / 160e6;
+      if (s > 1 && grid * s > 4 * CUS) break;
+      const int64_t works = grid * count[j];
+      const double busiest = (double)((works + CUS - 1) / CUS) * (each[j] * t.step + ends);
+      const double sums = (s > 1 ? 8.0 * count[j] : glu ? 1.0 : 2.0) * outs;
+      const double memory = (weights + rows + sums) / 8.8e6 + again;
       const double rest =
           1.6 + (s > 1 ? (unit == LINEAR_PARTS ? 1.15 : 4.8) + sums / 72e6 : 0);
-      if (*tile >= 0 && fmax(busiest, memory) + rest >= best) continue;  // nor is the sum less
-      const double us = pow(pow(busiest, 1.36) + pow(memory, 1.36), 1 / 1.36) + rest;
+      // both together take less than their sum, and no less than by squares
+      const double squares = busiest * busiest + memory * memory, room = best - rest;
+      if (*tile >= 0 && (room <= 0 || squares >= room * room)) continue;
+      const double us = rest + together(busiest, memory);
       if (*tile >= 0 && us >= best) continue;
       best = us;
       *tile = i;
