@@ -1281,6 +1281,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("alpha") = 0.0, py::arg("offset") = 0.0, py::arg("cubic") = 0.0,
         py::arg("tile") = -1, py::arg("splits") = 1);
   m.def("linear_fits", [](int tile, bool glu) { return linear_fits(tile, glu); });
+  m.def("linear_choice", [](int m, int n, int k, bool glu, bool parts) {
+    int tile, splits;
+    linear_choice(m, n, k, parts ? LINEAR_PARTS : glu ? LINEAR_GLU : LINEAR_PLAIN, &tile, &splits);
+    return std::make_pair(tile, splits);
+  });
   m.def("gemm_bf16", &gemm_bf16);
   m.attr("DEPTH_AHEAD") = DEPTH_AHEAD;
   m.def("residual_norm", &residual_norm);

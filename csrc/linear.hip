@@ -211,16 +211,22 @@ static const Together together;
 
 // The tile and the parts that are expected to be the fastest, in us: the chunks of the busiest
 // CU beside the memory's time, for the operands once and for what tiles read again, and a launch.  Fitted
-// to 754 sizes of 5 to 2100 rows, 2048 to 32000 outputs and 1280 to 14336 inner elements; what it chooses is
-// on average 1.1% slower than the best of all tiles and parts, 1.5% where the parts are added up
-// elsewhere, and 24% where it is worst.  With steps by the fragments alone, max(0.015 fn fm, 0.053
-// (fn + fm)), 1.7 and 3.2%: 190 x 4096 x 14336 into the norm 39.8 and now 35.3, 190 x 6144 x 4096 into
-// the rotation 22.9 and 21.2, 61 x 4096 x 4096 17.0 and 13.7.
+// to 754 sizes of 5 to 2100 rows, 2048 to 32000 outputs and 1280 to 14336 inner elements, on which what it
+// chooses is on average 1.1% slower than the best of all tiles and parts, 1.5% where the parts are added up
+// elsewhere, and 24% where it is worst.  On 11 sizes of weights that it was not fitted to, of 6 to 1900
+// rows, it chooses otherwise than steps by the fragments alone, max(0.015 fn fm, 0.053 (fn + fm)), for
+// 119 products, which are 3.9% faster on average, 23% at best, and 15% slower at worst (150 x 3072 x 3072
+// in parts 10.1 us and 11.6).
+// Above 2100 rows, where the matrix cores and the card's power bound a tile, steps are by the fragments,
+// as fitted to 8 to 10000 rows.  The table's choice there, where it is another one, is 0.6% slower on average
+// of 110 products of 2101 to 16384 rows, 5.7% at worst and 5.2% faster at best: 2500 x 28672 x 4096 SwiGLU
+// 444 us by fragments and 469, 7664 x 16384 x 2048 399 and 414, 10000 x 6144 x 4096 371 and 387, but 13000 x
+// 28672 x 4096 2178 and 2129; 15675 rows of it 2562 and 2548, 2584 and 2580.
 // It is asked for every launch and takes 0.1 to 0.6 us, 0.3 to 3.8 with powers for each of up to 154 pairs.
 extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* splits) {
   static const int parts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
   constexpr int PARTS = sizeof(parts) / sizeof(int);
-  const bool glu = unit == LINEAR_SWIGLU || unit == LINEAR_GLU;
+  const bool glu = unit == LINEAR_SWIGLU || unit == LINEAR_GLU, few = M <= 2100;
   const int chunks = K / 64, most = M > 2600 ? 1 : chunks / 4;
   const double rows = 2.0 * M * K, weights = 2.0 * N * K, outs = (double)M * N;
   int each[PARTS], count[PARTS], n = 1;
@@ -237,21 +243,24 @@ extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* spl
     const unsigned high = (M - 1u) / (32 * t.fm) + 1, wide = (N - 1u) / (32 * t.fn) + 1;
     const int64_t grid = (int64_t)high * wide;
     const double fragments = t.fn * t.fm;
-    const double ends = 0.09 * fragments + 0.09, again = (wide * rows + high * weights) / 160e6;
+    const double step = few ? t.step : fmax(0.015 * fragments, 0.053 * (t.fn + t.fm));
+    const double ends = few ? 0.09 * fragments + 0.09 : 0.08 * fragments + 0.57;
+    const double again = few ? (wide * rows + high * weights) / 160e6 : 0;
     for (int j = 0; j < n; ++j) {
       const int s = parts[j];
       if (s == 1 && !linear_fits(i, glu)) continue;
       if (s > 1 && grid * s > 4 * CUS) break;
       const int64_t works = grid * count[j];
-      const double busiest = (double)((works + CUS - 1) / CUS) * (each[j] * t.step + ends);
-      const double sums = (s > 1 ? 8.0 * count[j] : glu ? 1.0 : 2.0) * outs;
-      const double memory = (weights + rows + sums) / 8.8e6 + again;
+      const double busiest = (double)((works + CUS - 1) / CUS) * (each[j] * step + ends);
+      const double sums = (s > 1 ? 8.0 * count[j] : glu && few ? 1.0 : 2.0) * outs;
+      const double memory = (weights + rows + sums) / (few ? 8.8e6 : 6.4e6) + again;
       const double rest =
-          1.6 + (s > 1 ? (unit == LINEAR_PARTS ? 1.15 : 4.8) + sums / 72e6 : 0);
+          few ? 1.6 + (s > 1 ? (unit == LINEAR_PARTS ? 1.15 : 4.8) + sums / 72e6 : 0)
+              : (s > 1 ? (unit == LINEAR_PARTS ? 0.5 : 4.3) + sums / 21.7e6 : 0);
       // both together take less than their sum, and no less than by squares
       const double squares = busiest * busiest + memory * memory, room = best - rest;
       if (*tile >= 0 && (room <= 0 || squares >= room * room)) continue;
-      const double us = rest + together(busiest, memory);
+      const double us = rest + (few ? together(busiest, memory) : sqrt(squares));
       if (*tile >= 0 && us >= best) continue;
       best = us;
       *tile = i;

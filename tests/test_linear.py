@@ -85,6 +85,32 @@ SIZES = [(256, 256), (256, 224), (256, 192), (256, 160), (256, 128), (128, 192),
          (128, 96), (128, 64), (128, 32), (192, 128), (64, 64), (64, 32), (128, 160)]
 
 
+@pytest.mark.parametrize("m,n,k,glu,parts,want", [
+    (2500, 28672, 4096, True, False, ((256, 160), 1)),
+    (6000, 28672, 4096, True, False, ((256, 224), 1)),
+    (7664, 16384, 2048, True, False, ((256, 192), 1)),
+    (10000, 6144, 4096, False, False, ((256, 192), 1)),
+    (10000, 12288, 4096, False, True, ((256, 192), 1)),
+    (160, 28672, 4096, True, False, ((128, 160), 1)),
+    (190, 6144, 4096, False, True, ((128, 192), 5)),
+])
+def test_choice_of_tiles(m, n, k, glu, parts, want):
+    """Measured to be the faster one of the two models' choices; above 2100 rows it is by the fragments
+    alone, which the step times of few rows do not speak for."""
+    tile, splits = ops._hip()._C.linear_choice(m, n, k, glu, parts)
+    assert (SIZES[tile], splits) == want
+
+
+@pytest.mark.parametrize("m", [1, 33, 2100, 2101, 2600, 2601, 1 << 20, (1 << 30) - 1])
+@pytest.mark.parametrize("n,k", [(8, 64), (16, 320), (4104, 4096), (1 << 20, 64), (64, 1 << 20)])
+@pytest.mark.parametrize("glu,parts", [(False, False), (True, False), (False, True)])
+def test_choice_is_of_what_there_is(m, n, k, glu, parts):
+    C = ops._hip()._C
+    tile, splits = C.linear_choice(m, n, k, glu, parts)
+    assert 0 <= tile < len(SIZES) and 1 <= splits <= k // 64
+    assert C.linear_fits(tile, glu and splits == 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [None, (7.0, 1.702, 1.0, 0.0), (1e30, 1.0, 0.0, 0.0),
                                   (3e38, 1.5957691, 0.0, 0.044715)])
