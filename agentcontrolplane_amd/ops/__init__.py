@@ -162,25 +162,26 @@ def _many_rows_pay(m: int, n: int, k: int, glu: bool, adds: bool = False) -> boo
     and k inner elements, where ``adds``: what reads it adds up its parts, which saves a launch of
     4.3 us.  The GEMM library (with a pass of its own for the GLU) is in brackets, us of every
     weight from memory.  Up to about 2000 rows at most sizes: 8 x 22016 x 4096 GLU 33 (55), 64 x
-    4096 x 14336 29 (39), 192 x 4096 x 4096 21 (32), 512 x 6288 x 2048 22 (24), 1739 x 4096 x 11008 130
-    (148).  Without ``adds`` not: up to 32 rows of medium weights, 8 x 6144 x 4096 16.8 (15.4), 16 x 4096 x
-    8192 19.1 (16.5), or very large ones, 24 x 128256 x 4096 195 (185) when all tiles began at the same
-    column, or few outputs, 8 x 2048 x 8192 13.6 (12.7); where unsplit tiles leave half of the CUs idle, 61
-    x 4096 x 4096 17.1, in parts as fast as the library, 13.7 (14.3); weights that two tiles of rows
-    read, 96 x 12288 x 4096 34 (30).  The library has other sizes of its own beside slow ones, 190 x
-    6288 x 2048 16.7 (15.9), 160 x 6288 x 2048 15.0 (16.5): not told apart.  From 1024
+    4096 x 14336 31 (41), 192 x 4096 x 4096 21 (33), 512 x 6288 x 2048 19 (24), 1739 x 4096 x 11008 139
+    (169), 24 x 128256 x 4096 165 (196).  Without ``adds`` not: up to 32 rows of medium weights, 8 x
+    6144 x 4096 17.2 (16.5), 32 x 7168 x 4096 22.4 (17.6), 16 x 4096 x 8192 19.6 (17.9), or few outputs, 8 x
+    2048 x 8192 13.7 (12.4); where unsplit tiles leave half of the CUs idle and parts gain little, 80 x
+    2048 x 4096 12.0 (11.3), 61 x 3584 x 3584 12.5 (11.0), 33 to 64 x 4096 x 4096 within 5% either way; weights
+    that two tiles of rows read, 128 x 12288 x 4096 38 (35), 96 of them 34 (34).  The library has other
+    sizes of its own beside slow ones, 61 x 6144 x 4096 20.6 (19.5), 160 x 12288 x 4096 40.2 (39.5): not told
+    apart.  From 1024
     rows on (2048 with a GLU or ``adds``) it is 2 to 9% ahead where
-    256 x 256 tiles fill their last round, 1400 x 32000 x 4096 287 (273), 5000 x 6144 x 4096 194 (188),
-    7664 x 2048 x 8192 185 (172), 8131 x 4096 x 4096 185 (176), but not for the GLU, 7664 x 28672 x 4096 1259 (1376),
-    for outputs that are no whole tiles, 7664 x 17744 x 2048 437 (494), and for rows that
-    together are beyond the memory-side cache, 7664 x 4096 x 14336 630 (995); with a last
-    round that is not full it is slower, 5000 x 4096 x 4096 132 (142), 10000 x 4096 x 4096 251 (361)."""
+    256 x 256 tiles fill their last round, 1400 x 32000 x 4096 301 (287), 5000 x 6144 x 4096 188 (179),
+    7664 x 2048 x 8192 190 (174), 8131 x 4096 x 4096 195 (183), but not for the GLU, 7664 x 28672 x 4096 1287 (1380),
+    for outputs that are no whole tiles, 7664 x 17744 x 2048 424 (506), and for rows that
+    together are beyond the memory-side cache, 7664 x 4096 x 14336 619 (1001); with a last
+    round that is not full it is slower, 5000 x 4096 x 4096 134 (141), 10000 x 4096 x 4096 243 (373)."""
     if m <= 4 or n * k < 1 << 21:
         return False
     plain = not (glu or adds)
     if plain and m <= 32:
         medium = 4096 <= k <= 8192 and n <= 8192 and n * k >= 24 << 20
-        return not (medium or n * k >= 256 << 20 or (m <= 16 and k >= 4 * n))
+        return not (medium or (m <= 16 and k >= 4 * n))
     if plain and 3584 <= k < 8192 and -(-m // 32) * n <= 8192:
         return False
     if plain and k >= 4096 and 64 < m <= 128 and 10240 < n < 16384:
