@@ -16,14 +16,15 @@
 // token-id order, and walks the stripe with the target: the inverse CDF runs in token-id order
 // and draws match the fp32 oracle (ops/reference.py softmax_sample) for a given uniform.  The
 // weights of 64 tokens of every stripe are made at a time by all threads and added up by one
-// thread a stripe: one after another in fp32 without a threshold (all CUTS are false), by fours in fp32
-// and those in 64 bits with one, so that all the ways such a row can take agree.
+// thread a stripe: one after another in fp32 without a threshold (all CUTS are false), by fours in
+// fp32 and those in 64 bits with one.
 //
-// Greedy rows of whole units by one workgroup, and those with a threshold, take another way, by units
-// (below), and this one where that does not fit: 190 rows of 128256 in fp32, other logits each time, whole calls: 25 us greedy, 48 plain, 79
-// top-k, 95 top-p, 135 both (26, 58, 97, 168 and 238 with calls of functions, which take a row and LDS by
-// reference: their loads and atomics then go by unknown memory and wait for both kinds).  Floating masses
-// instead of whole ones in the histogram took as long, a shared list of the bucket 25 us more.
+// Greedy rows of whole units by one workgroup, and those with a threshold, take another way, by
+// units (below), and this one where that does not fit.  190 rows of 128256 in fp32 by this one,
+// other logits each time, whole calls: 25 us greedy, 49 plain, 79 top-k, 95 top-p, 135 both (26,
+// 58, 97, 168 and 238 with calls of functions, which take a row and LDS by reference: their loads
+// and atomics then go by unknown memory and wait for both kinds).  Floating masses instead of whole
+// ones in the histogram took as long, a shared list of the bucket 25 us more.
 //
 // Semantics match the oracle:
 //   greedy (T<=0): argmax, lowest index on ties
@@ -1198,13 +1199,17 @@ INLINE void whole_row(S& s, const SampleArgs& a, const Wants& want, Row<T, S::WG
 //   3 the weights above those buckets in a thread's own sum in 64 bits, the keys in them into a list, from
 //     which the least kept key follows exactly
 // The draw goes to the wave that has the target, then to its turn, a unit, a token, in token-id order.
-// 190 rows of 128256 in fp32, whole_row() and this, us: greedy 24.6 and 22.5, top-k 80 and 55, top-p 95 and
-// 72, both 135 and 60, top-p 0.9 at a temperature of 6.4 100 and 74; bf16 22 and 14, 70 and 45, 92 and 67,
-// 118 and 50; 32000 in fp32 10 and 8.8, 35 and 25, 42 and 33, 58 and 31.  Plain rows took 33 instead of 48, but
-// their draws are by sums in fp32, in order, and one in 50 was another one by these sums: they stay
-// whole_row()'s.  With more registers HELD they spill; 4 units ahead instead of 2 as long.
-// A row that this does not fit is whole_row()'s: one of no threshold that is not greedy, of no whole units, logits that are no numbers, a
-// boundary among more keys than the list has or beyond the last bucket, a top-p beyond MOST_P.
+// 190 rows of 128256 in fp32, whole_row() and this, us: greedy 25 and 23, top-k 81 and 56, top-p 96 and
+// 77, both 136 and 62, top-p 0.9 at a temperature of 6.4 100 and 79; bf16 22 and 14, 71 and 47, 93 and
+// 64, 119 and 52; 32000 in fp32 11 and 10, 37 and 27, 43 and 36, 59 and 33; 70% allowed by a mask 59
+// and 33, 173 and 79, 221 and 96, 310 and 85.  Plain rows took 33 instead of 49, but their draws are by
+// sums in fp32, in order, and one in 50 was another one by these sums: they stay whole_row()'s.  With
+// more registers HELD they spill, and a build with spills drew wrong tokens; 4 units ahead instead of 2
+// as long.
+// A row that this does not fit is whole_row()'s: one of no threshold that is not greedy, of no whole
+// units, logits that are no numbers or all alike, a boundary among more keys than the list has (from
+// -inf among logits that no mask has out, buckets do not narrow) or beyond the last bucket, a top-p
+// beyond MOST_P.
 template <typename T, bool MASKED>
 struct Units {
   static constexpr int N = 16 / sizeof(T);
@@ -1661,13 +1666,18 @@ static void launch(const SampleArgs& a, void* work, int chunks, hipStream_t stre
   }
 }
 
-// Chunks of a row, the more of them the fewer the rows; 0: a workgroup a row, which is faster from 100 rows
-// on and for smaller vocabularies.  By a workgroup a row, by units and by whole_row(), and in chunks, us,
-// greedy, plain, top-p and all kinds in turns: 128256 tokens 1 row 10 19 57 19, 19 38 81 38 and 17 30 55 30,
-// 16 11 21 59 58, 20 41 85 84 and 19 34 62 62, 64 17 26 63 63, 22 42 89 88 and 24 43 77 76, 100 19 28 66 65,
-// 23 44 90 89 and 27 51 95 94 (plain rows are whole_row()'s in either way); 65536 8 8 15 44 43, 12 25 53 52 and 17 27 49 50.  Up to 64 rows in chunks all the
-// same: what rows want is known on the device, and what only whole_row() can, a top-p of 0.999 for one, takes 125 us
-// by it and 55 in chunks.
+// Chunks of a row, the more of them the fewer the rows; 0: a workgroup a row, which is faster from 65
+// rows on and for smaller vocabularies.  By a workgroup a row and in chunks, us of fp32:
+//                  greedy     plain      top-k      top-p      both       all kinds in turns
+//   1 x 128256     10 17      39 28      42 42      60 53      48 48
+//   16             11 19      41 33      43 48      62 62      49 56      62 62
+//   32             11 19      42 36      43 52      64 68      50 59      63 67
+//   64             17 24      44 41      47 61      67 78      54 69      66 77
+//   100            19 32      44 57      49 90      68 108     55 98      68 94
+//   16 x 65536     8 18       27 29      29 42      45 54      36 49      42 53
+// So up to 64 rows it is plain rows, which go by whole_row(), that chunks are for; what rows want is known
+// on the device alone.  A top-p of 0.999 takes 117 us in one workgroup and 139 in chunks, whose lists it
+// does not fit either.
 extern "C" int sample_fullvocab_chunks(int B, int V) {
   return V < SPLIT_VOCAB || B > 64 ? 0 : B <= 16 ? 32 : 16;
 }
