@@ -170,10 +170,13 @@ SHAPES = [
     (32, 512, None, 16, [(0, 150), (90, 1), (2000, 1), (777, 2)]),
     (128, 512, 300, 16, [(0, 3), (900, 1), (1200, 1)]),
     (2, 600, 50, 16, [(0, 60), (70, 1), (70, 2)]),
-    # more workgroups of decode than CUs: smaller tiles, of every number of keys modulo theirs
+    # as many workgroups of decode as CUs, of every number of keys modulo a tile's
     (16, 512, None, 16, [(0, 20)] + [(7 * i, 1) for i in range(48)] + [(1000, 1)]),
     (9, 250, None, 4, [(0, 3)] + [(9 * i + 1, 1) for i in range(40)] + [(930, 1), (1023, 1)]),
     (5, 384, 900, 16, [(0, 2)] + [(23 * i, 1) for i in range(45)] + [(1100, 1)]),
+    # long parts, of which there are more than CUs: smaller tiles
+    (16, 512, None, 16, [(0, 20)] + [(23 * i, 1) for i in range(40)] + [(2050, 1)]),
+    (9, 250, None, 4, [(0, 3)] + [(31 * i + 1, 1) for i in range(40)] + [(2001, 1), (2051, 1)]),
     # as many without a split: written by the smaller tiles themselves, few and many of them
     (16, 512, None, 16, [(0, 3)] + [(i % 100, 1) for i in range(270)]),
     (3, 250, 70, 4, [(0, 1)] + [(2 * i % 131, 1) for i in range(300)]),
