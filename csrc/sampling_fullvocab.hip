@@ -459,10 +459,11 @@ INLINE Row<T, WG> row_of(const SampleArgs& a, int n) {
           invT * 1.44269504f};
 }
 
-// A stripe's weights of a tile
-template <bool CUTS, int TILE>
+// A stripe's weights of a tile; WIDE: all of them on their way from LDS at once also for sums in 64
+// bits, where a thread has the registers (rows in chunks: 16 x 128256 top-k 7.6 us by halves, 7.0)
+template <bool CUTS, int TILE, bool WIDE = false>
 INLINE void add_tile(const float* tile, SumOf<CUTS>& sum) {
-  constexpr int FOURS = !CUTS || TILE < 32 ? TILE / 4 : 8;
+  constexpr int FOURS = !CUTS || WIDE || TILE < 32 ? TILE / 4 : 8;
 #pragma unroll 1
   for (int j0 = 0; j0 < TILE / 4; j0 += FOURS) {
     float4 w[FOURS];
@@ -641,16 +642,17 @@ __device__ __forceinline__ bool left_whole(const RowPlan& plan) {
   return plan.mode == WHOLE || (plan.mode == BY_LIST && plan.n > KEYS);
 }
 
-// A row's state between the launches
+// A row's state between the launches.  What many workgroups add to or read begins at a cache line, 16 x
+// 128256 top-k: histogram 8.2 us otherwise and 7.7, keys 13.7 and 12.9
 struct RowState {
   RowPlan plan;
   double rest[MOST_CHUNKS];
-  double stripe[STRIPES];
   float chunk_max[MOST_CHUNKS];
   int chunk_best[MOST_CHUNKS], chunk_odd[MOST_CHUNKS];
-  uint32_t list[KEYS];
-  uint32_t count[FIRST];
-  unsigned long long mass[FIRST];
+  double stripe[STRIPES];
+  alignas(128) uint32_t list[KEYS];
+  alignas(128) uint32_t count[FIRST];
+  alignas(128) unsigned long long mass[FIRST];
 };
 
 typedef Form<256, 64> ChunkForm;
@@ -889,7 +891,7 @@ INLINE void chunk_sums(ChunkShared& s, const SampleArgs& a, const Chunk& c, cons
     }
     if (j0 + TILE < c.stride) fetch(j0 + TILE);
     __syncthreads();  // the other tile is added up before it is written again
-    if (t < c.stripes) add_tile<CUTS, TILE>(tile[t], mine);
+    if (t < c.stripes) add_tile<CUTS, TILE, true>(tile[t], mine);
   }
   if (t < c.stripes) state.stripe[c.at * c.stripes + t] = mine;
 }
@@ -1669,12 +1671,12 @@ static void launch(const SampleArgs& a, void* work, int chunks, hipStream_t stre
 // Chunks of a row, the more of them the fewer the rows; 0: a workgroup a row, which is faster from 65
 // rows on and for smaller vocabularies.  By a workgroup a row and in chunks, us of fp32:
 //                  greedy     plain      top-k      top-p      both       all kinds in turns
-//   1 x 128256     10 17      39 28      42 42      60 53      48 48
-//   16             11 19      41 33      43 48      62 62      49 56      62 62
-//   32             11 19      42 36      43 52      64 68      50 59      63 67
-//   64             17 24      44 41      47 61      67 78      54 69      66 77
-//   100            19 32      44 57      49 90      68 108     55 98      68 94
-//   16 x 65536     8 18       27 29      29 42      45 54      36 49      42 53
+//   1 x 128256      8 17      37 27      40 40      52 51      46 47
+//   16             10 19      40 32      42 45      59 59      48 52      58 58
+//   32             10 19      41 34      43 50      60 65      49 57      60 63
+//   64             11 22      41 39      43 59      61 73      50 66      60 70
+//   100            13 28      42 53      45 86      62 103     51 93      61 81
+//   16 x 65536      7 20      26 28      28 39      37 45      34 46      36 49
 // So up to 64 rows it is plain rows, which go by whole_row(), that chunks are for; what rows want is known
 // on the device alone.  A top-p of 0.999 takes 117 us in one workgroup and 139 in chunks, whose lists it
 // does not fit either.
