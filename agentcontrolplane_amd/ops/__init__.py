@@ -162,8 +162,8 @@ def _many_rows_pay(m: int, n: int, k: int, glu: bool, adds: bool = False) -> boo
     and k inner elements, where ``adds``: what reads it adds up its parts, which saves a launch of
     4.3 us.  The GEMM library (with a pass of its own for the GLU) is in brackets, us of every
     weight from memory.  Up to about 2000 rows at most sizes: 8 x 22016 x 4096 GLU 33 (55), 64 x
-    4096 x 14336 31 (41), 192 x 4096 x 4096 21 (33), 512 x 6288 x 2048 19 (24), 1739 x 4096 x 11008 139
-    (169), 24 x 128256 x 4096 165 (196).  Without ``adds`` not: up to 32 rows of medium weights, 8 x
+    4096 x 14336 29 (43), 192 x 4096 x 4096 22 (34), 512 x 6288 x 2048 22 (26), 1739 x 4096 x 11008 130
+    (159), 24 x 128256 x 4096 167 (195).  Without ``adds`` not: up to 32 rows of medium weights, 8 x
     6144 x 4096 17.2 (16.5), 32 x 7168 x 4096 22.4 (17.6), 16 x 4096 x 8192 19.6 (17.9), or few outputs, 8 x
     2048 x 8192 13.7 (12.4); where unsplit tiles leave half of the CUs idle and parts gain little, 80 x
     2048 x 4096 12.0 (11.3), 61 x 3584 x 3584 12.5 (11.0), 33 to 64 x 4096 x 4096 within 5% either way; weights

@@ -19,9 +19,10 @@
 // among them 663, the reads done at three quarters of a step 652.  Stores of whole lines past
 // the caches: 8131 x 28672 x 4096 1335 to 1299.
 //
-// Against the GEMM library (and the unit's own pass), us: 64 x 4096 x 14336 29 (39), 192 x 28672
-// x 4096 SwiGLU 54 (67), 192 x 4096 x 14336 40 (103), 512 x 4096 x 14336 67 (91), 1739 x 28672 x
-// 4096 SwiGLU 310 (417), 7664 x 28672 x 4096 SwiGLU 1259 (1376), 10000 x 4096 x 4096 244 (370).
+// Against the GEMM library (and the unit's own pass), us: 64 x 4096 x 14336 29 (43), 192 x 28672
+// x 4096 SwiGLU 56 (67), 192 x 4096 x 14336 41 (104), 512 x 4096 x 14336 68 (91), 1739 x 28672 x
+// 4096 SwiGLU 315 (422), 7664 x 28672 x 4096 SwiGLU 1278 (1397), 10000 x 4096 x 4096 242 (361),
+// 15675 x 28672 x 4096 SwiGLU 2538 (2765), 1.45 PFLOP/s.
 #include <math.h>
 
 #include "launch.h"
