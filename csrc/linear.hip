@@ -181,11 +181,11 @@ struct Tile {
 };
 // The rings' depths: 61 x 28672 x 4096 SwiGLU by 128 x 64 with 3 chunks of both 42.5, with 4 40.0;
 // 190 rows of it by 128 x 192 with 4 59.7, with 3 57.2
-#define TILES(T)                                                                          \
-  T(8, 8, 3, 2, 1.04) T(8, 7, 3, 2, 0.98) T(8, 6, 3, 2, 0.85) T(8, 5, 3, 3, 0.77)         \
-  T(8, 4, 3, 4, 0.71) T(4, 6, 3, 3, 0.56) T(4, 4, 5, 5, 0.48) T(4, 3, 5, 5, 0.41)         \
-  T(4, 2, 4, 4, 0.34) T(4, 1, 4, 4, 0.32) T(6, 4, 4, 4, 0.67) T(2, 2, 5, 5, 0.18)         \
-  T(2, 1, 6, 6, 0.16) T(4, 5, 4, 3, 0.52)
+#define TILES(T)                                                                             \
+  T(8, 8, 3, 2, 1.142) T(8, 7, 3, 2, 1.0)   T(8, 6, 3, 2, 0.891) T(8, 5, 3, 3, 0.802)        \
+  T(8, 4, 3, 4, 0.753) T(4, 6, 3, 3, 0.614) T(4, 4, 5, 5, 0.55) T(4, 3, 5, 5, 0.446)         \
+  T(4, 2, 4, 4, 0.393) T(4, 1, 4, 4, 0.34) T(6, 4, 4, 4, 0.674) T(2, 2, 5, 5, 0.234)         \
+  T(2, 1, 6, 6, 0.185) T(4, 5, 4, 3, 0.561)
 #define SIZES(fn, fm, ws, xs, step) {fn, fm, ws, xs, step},
 static const Tile tiles[] = {TILES(SIZES)};
 static constexpr int TILE_COUNT = sizeof(tiles) / sizeof(Tile);
@@ -211,15 +211,17 @@ struct Together {
 static const Together together;
 
 // The tile and the parts that are expected to be the fastest, in us: the chunks of the busiest
-// CU beside the memory's time, for the operands once and for what tiles read again, and a launch.  Fitted
-// to 754 sizes of 5 to 2100 rows, 2048 to 32000 outputs and 1280 to 14336 inner elements, on which what it
-// chooses is on average 1.1% slower than the best of all tiles and parts, 1.5% where the parts are added up
-// elsewhere, and 24% where it is worst.  On 11 sizes of weights that it was not fitted to, of 6 to 1900
-// rows, it chooses otherwise than steps by the fragments alone, max(0.015 fn fm, 0.053 (fn + fm)), for
-// 119 products, which are 3.9% faster on average, 23% at best, and 15% slower at worst (150 x 3072 x 3072
-// in parts 10.1 us and 11.6).
+// CU beside the memory's time.  A chunk takes as long as its rows take to be loaded, so that a tile of
+// rows which is not full takes less.  Fitted to 2200 products of 5 to 2100 rows by 32 sizes of weights,
+// 1024 to 37888 outputs and 1280 to 13824 inner elements, some with the norm that adds up their parts.
+// What it chooses is on average 1.1% slower than the best of all tiles and parts, 7% and more in one of
+// 20, 20% where it is worst; fitted to one half of the weights 1.4 and 1.7% on the other half, and 1.0% on
+// 396 products into the rotation that it was not fitted to.  A model with one time for a tile's chunks, full
+// or not, and a term for what tiles read again: 1.7%, 28% where it is worst, as it took tiles of 64 x 64 that
+// are whole in the inner dimension, and few large ones in parts.  us by it and now: 190 x 5120 x 5120 into
+// the norm 28.9 and 22.6, 777 x 4096 x 4096 40.3 and 32.2, 512 x 2048 x 8192 36.4 and 30.2.
 // Above 2100 rows, where the matrix cores and the card's power bound a tile, steps are by the fragments,
-// as fitted to 8 to 10000 rows.  The table's choice there, where it is another one, is 0.6% slower on average
+// as fitted to 8 to 10000 rows.  A choice by a table there, where it was another one, was 0.6% slower on average
 // of 110 products of 2101 to 16384 rows, 5.7% at worst and 5.2% faster at best: 2500 x 28672 x 4096 SwiGLU
 // 444 us by fragments and 469, 7664 x 16384 x 2048 399 and 414, 10000 x 6144 x 4096 371 and 387, but 13000 x
 // 28672 x 4096 2178 and 2129; 15675 rows of it 2562 and 2548, 2584 and 2580.
@@ -244,9 +246,9 @@ extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* spl
     const unsigned high = (M - 1u) / (32 * t.fm) + 1, wide = (N - 1u) / (32 * t.fn) + 1;
     const int64_t grid = (int64_t)high * wide;
     const double fragments = t.fn * t.fm;
-    const double step = few ? t.step : fmax(0.015 * fragments, 0.053 * (t.fn + t.fm));
-    const double ends = few ? 0.09 * fragments + 0.09 : 0.08 * fragments + 0.57;
-    const double again = few ? (wide * rows + high * weights) / 160e6 : 0;
+    const double loaded = (32.0 * t.fn + (double)M / high) / (32 * (t.fn + t.fm));
+    const double step = few ? t.step * loaded : fmax(0.015 * fragments, 0.053 * (t.fn + t.fm));
+    const double ends = few ? 0.125 * fragments + 0.887 : 0.08 * fragments + 0.57;
     for (int j = 0; j < n; ++j) {
       const int s = parts[j];
       if (s == 1 && !linear_fits(i, glu)) continue;
@@ -254,10 +256,11 @@ extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* spl
       const int64_t works = grid * count[j];
       const double busiest = (double)((works + CUS - 1) / CUS) * (each[j] * step + ends);
       const double sums = (s > 1 ? 8.0 * count[j] : glu && few ? 1.0 : 2.0) * outs;
-      const double memory = (weights + rows + sums) / (few ? 8.8e6 : 6.4e6) + again;
+      const double memory = (weights + rows + sums) / (few ? 6.1e6 : 6.4e6);
       const double rest =
-          few ? 1.6 + (s > 1 ? (unit == LINEAR_PARTS ? 1.15 : 4.8) + sums / 72e6 : 0)
-              : (s > 1 ? (unit == LINEAR_PARTS ? 0.5 : 4.3) + sums / 21.7e6 : 0);
+          s == 1 ? 0
+          : few  ? (unit == LINEAR_PARTS ? 0 : 4.0) + sums / 27e6  // 3.5 in a graph, 4.3 outside
+                 : (unit == LINEAR_PARTS ? 0.5 : 4.3) + sums / 21.7e6;
       // both together take less than their sum, and no less than by squares
       const double squares = busiest * busiest + memory * memory, room = best - rest;
       if (*tile >= 0 && (room <= 0 || squares >= room * room)) continue;

@@ -92,10 +92,15 @@ SIZES = [(256, 256), (256, 224), (256, 192), (256, 160), (256, 128), (128, 192),
     (10000, 6144, 4096, False, False, ((256, 192), 1)),
     (10000, 12288, 4096, False, True, ((256, 192), 1)),
     (160, 28672, 4096, True, False, ((128, 160), 1)),
-    (190, 6144, 4096, False, True, ((128, 192), 5)),
+    (190, 4096, 14336, False, True, ((128, 192), 8)),
+    # tiles that are whole in the inner dimension, or large ones in parts, were 15 to 26% slower
+    (190, 5120, 5120, False, True, ((128, 96), 3)),
+    (777, 4096, 4096, False, False, ((128, 128), 1)),
+    (128, 5120, 5120, False, False, ((128, 64), 3)),
+    (256, 3072, 3072, False, True, ((128, 96), 3)),
 ])
 def test_choice_of_tiles(m, n, k, glu, parts, want):
-    """Measured to be the faster one of the two models' choices; above 2100 rows it is by the fragments
+    """Measured to be the faster one of two models' choices; above 2100 rows it is by the fragments
     alone, which the step times of few rows do not speak for."""
     tile, splits = ops._hip()._C.linear_choice(m, n, k, glu, parts)
     assert (SIZES[tile], splits) == want
