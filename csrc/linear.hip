@@ -182,7 +182,7 @@ struct Tile {
 // The rings' depths: 61 x 28672 x 4096 SwiGLU by 128 x 64 with 3 chunks of both 42.5, with 4 40.0;
 // 190 rows of it by 128 x 192 with 4 59.7, with 3 57.2
 #define TILES(T)                                                                             \
-  T(8, 8, 3, 2, 1.142) T(8, 7, 3, 2, 1.0)   T(8, 6, 3, 2, 0.891) T(8, 5, 3, 3, 0.802)        \
+  T(8, 8, 3, 2, 1.142) T(8, 7, 3, 2, 1.034) T(8, 6, 3, 2, 0.891) T(8, 5, 3, 3, 0.802)        \
   T(8, 4, 3, 4, 0.753) T(4, 6, 3, 3, 0.614) T(4, 4, 5, 5, 0.55) T(4, 3, 5, 5, 0.446)         \
   T(4, 2, 4, 4, 0.393) T(4, 1, 4, 4, 0.34) T(6, 4, 4, 4, 0.674) T(2, 2, 5, 5, 0.234)         \
   T(2, 1, 6, 6, 0.185) T(4, 5, 4, 3, 0.561)
