@@ -225,7 +225,7 @@ static const Together together;
 // of 110 products of 2101 to 16384 rows, 5.7% at worst and 5.2% faster at best: 2500 x 28672 x 4096 SwiGLU
 // 444 us by fragments and 469, 7664 x 16384 x 2048 399 and 414, 10000 x 6144 x 4096 371 and 387, but 13000 x
 // 28672 x 4096 2178 and 2129; 15675 rows of it 2562 and 2548, 2584 and 2580.
-// It is asked for every launch and takes 0.1 to 0.6 us, 0.3 to 3.8 with powers for each of up to 154 pairs.
+// It is asked for every launch and takes 0.1 to 0.7 us, 0.3 to 3.8 with powers for each of up to 154 pairs.
 extern "C" void linear_choice(int M, int N, int K, int unit, int* tile, int* splits) {
   static const int parts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
   constexpr int PARTS = sizeof(parts) / sizeof(int);
