@@ -205,7 +205,12 @@ DEV void linear_tiles(const LinearArgs& a, const Work& work, char* const lds) {
       next_x();
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // The first chunk has landed.  To wait for the whole rings, as was done, has the memory run idle once
+  // while no loads follow them, us of products alone: 40 x 2048 x 2048 9.4 and now 8.7, 61 x 4096 x
+  // 4096 14.0 and 13.4, 61 x 28672 x 4096 SwiGLU 38.6 and 38.1; experts of 4093 tokens 1010 and 1000
+  constexpr int STARTED = (WS - 2) * LW + (XS - 1) * LX;
+  static_assert(STARTED < 64);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STARTED) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   look(0);
