@@ -573,6 +573,20 @@ def _scan_columns(prefills, columns: int) -> int:
     return 2 if sum(lens) * columns > 3 * 4096 * max(lens) else 1
 
 
+def _scan_in_chunks(prefills, H: int, D: int, V: int, dtype) -> int:
+    """16s of columns a workgroup of the recurrence by chunks of 16 tokens, 0: token by token.  By
+    chunks, heads of 128 key channels from 49 tokens on: a launch more, a shorter chain.  All launches of a layer
+    with 16 heads of 128 x 128, us, token by token and by chunks: 17 tokens 33, 36; 33 36, 38; 64 42, 39; 256
+    78, 54; 8000 1444, 631; 9 x 17 45, 51; 12 x 64 70, 66; 24 x 300 381, 320.  In fp32, where it would be
+    1.05 to 1.2 times as far from 64 bits (1.8e-7), token by token.  16 columns a workgroup are the shorter chain,
+    32 less work beside the longest sequence's: 760 to 2140 330, 380 (3.2 times the longest one's
+    tokens); 4 x 400 103, 99; 8 x 1000 419, 340; with 32 heads 3 x 600 184, 180; 8000 795, 948."""
+    lens = [m.query_len for m in prefills]
+    if dtype != torch.bfloat16 or D != 128 or V % 16 or max(lens) <= 48:
+        return 0
+    return 2 if V % 32 == 0 and sum(lens) * H * V > 4 * 2048 * max(lens) else 1
+
+
 def gated_delta(qkv, conv, b, z, A_log, dt_bias, gate, norm, eps, unit_eps, kv_heads,
                 state, conv_state, batch, gate_silu=False):
     H, D, V = state.shape[1:]
@@ -589,12 +603,21 @@ def gated_delta(qkv, conv, b, z, A_log, dt_bias, gate, norm, eps, unit_eps, kv_h
         def space(n, dtype=torch.float32):
             return torch.empty(P * n, dtype=dtype, device=qkv.device)
 
-        cpl = batch.memo(("scan_columns", H * V), lambda: _scan_columns(batch.prefills, H * V))
+        chunks = None
+        cpl = batch.memo(
+            ("scan_chunks", H, D, V, qkv.dtype),
+            lambda: _scan_in_chunks(batch.prefills, H, D, V, qkv.dtype),
+        )
+        if cpl:
+            n = (P // 16 + len(batch.prefills)) * H * _C.DELTA_CHUNK_FLOATS
+            chunks = torch.empty(n, device=qkv.device)
+        else:
+            cpl = batch.memo(("scan_columns", H * V), lambda: _scan_columns(batch.prefills, H * V))
         _C.delta_prompts(
             *rows(slice(0, P)), meta.seq_lens, meta.state_slots, kv_heads, eps, unit_eps,
             gate_silu, meta.ctx_lens, meta.row_starts, meta.tile_seq, meta.tile_q0,
             space(qkv.shape[1], qkv.dtype), space(3 * kv_heads),
-            None if z.shape[1] == H else space(H * D), space(H * V), cpl,
+            None if z.shape[1] == H else space(H * D), space(H * V), cpl, chunks,
         )
     if batch.num_decode:
         _C.delta_step(

@@ -1220,7 +1220,8 @@ static void delta_prompts(torch::Tensor out, torch::Tensor qkv, torch::Tensor co
                           torch::Tensor slots, int64_t kv_heads, double eps, double unit_eps,
                           bool gate_silu, torch::Tensor ctx_lens, torch::Tensor row_starts,
                           torch::Tensor tile_seq, torch::Tensor tile_q0, torch::Tensor y,
-                          torch::Tensor unit, OptTensor g, torch::Tensor o, int64_t cpl) {
+                          torch::Tensor unit, OptTensor g, torch::Tensor o, int64_t cpl,
+                          OptTensor chunks) {
   DeltaArgs a = delta_args(out, qkv, conv, b, z, A_log, dt_bias, gate, norm, state, ring,
                            seq_lens, slots, kv_heads, eps, unit_eps, gate_silu);
   check_vec(y, qkv.scalar_type(), (int64_t)a.N * a.C);
@@ -1234,6 +1235,12 @@ static void delta_prompts(torch::Tensor out, torch::Tensor qkv, torch::Tensor co
   a.y = y.data_ptr();
   a.unit = unit.data_ptr<float>();
   a.o = o.data_ptr<float>();
+  if (chunks) {
+    TORCH_CHECK(is_bf16(qkv) && a.D == 128 && a.V % 16 == 0 && (cpl == 1 || (cpl == 2 && a.V % 32 == 0)),
+                "delta rule: chunks");
+    check_vec(*chunks, at::kFloat, (int64_t)(a.N / 16 + a.seqs) * a.H * DELTA_CHUNK_FLOATS);
+    a.chunks = chunks->data_ptr<float>();
+  }
   a.n_tiles = tile_seq.numel();
   a.ctx_lens = opt_int(ctx_lens, a.seqs);
   a.row_starts = opt_int(row_starts, a.seqs);
@@ -1310,6 +1317,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_group", &moe_group);
   m.def("experts_linear", &experts_linear);
   m.def("delta_prompts", &delta_prompts);
+  m.attr("DELTA_CHUNK_FLOATS") = DELTA_CHUNK_FLOATS;
   m.def("delta_step", &delta_step);
   m.def("sample", &sample);
   m.def("sample_fullvocab_chunks", &sample_fullvocab_chunks);

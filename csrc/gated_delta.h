@@ -2,6 +2,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+// Workspace of 16 tokens and a head (delta_chunks.hip), floats
+#define DELTA_CHUNK_FLOATS 6784
+
 struct DeltaArgs {
   // inputs by token row, in the model's dtype; q | k | v channels, C = 2 G D + H V
   const void* qkv;        // [N, C] before the convolution
@@ -20,6 +23,7 @@ struct DeltaArgs {
   float* unit;            // [N, G, 3] factors that make q and k unit vectors, then q . k
   float* g;               // [N, H * D] decays; null with head_decay
   float* o;               // [N, H, V] before the norm
+  float* chunks;          // [H, N / 16 + seqs, DELTA_CHUNK_FLOATS], or null: token by token
   const int* seq_lens;    // [seqs] tokens including this step's
   const int* ctx_lens;    // [seqs] before this step; null: decode
   const int* row_starts;  // [seqs]
@@ -32,3 +36,6 @@ struct DeltaArgs {
   bool head_decay;        // one decay per head
   bool gate_silu;         // gate silu(x), else sigmoid(x)
 };
+
+// In place of the recurrence token by token, with chunks given: bf16, D = 128, V a multiple of 16 columns
+extern "C" void launch_delta_chunks(const DeltaArgs* a, int columns, hipStream_t stream);

@@ -14,28 +14,18 @@
 //                 lanes a column; q, k, g of the head's next tokens wait in LDS, shared
 //                 by the workgroup's columns
 //   delta_output: norm over the head and gate
+// Long prompts of bf16 with heads of 128 channels take delta_chunks.hip's two launches instead of delta_scan.
 // One token per sequence: delta_step does all of it, S once through registers.
 //
 // The convolution's inputs are kept in a ring by position, so that a token's write
 // never hits an entry that the token's own convolution reads, whichever workgroup
 // comes first.
-#include "common_t.h"
-#include "gated_delta.h"
+#include "delta_device.h"
 #include "launch.h"
 
 DEV float silu_f(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
-// log(1 + e^x) with a small relative error everywhere: log(u) e / (u - 1), u = 1 + e
-DEV float softplus_f(float x) {
-  if (x > 20.f) return x;
-  const float e = __expf(x), u = 1.f + e;
-  return u == 1.f ? e : __logf(u) * e * __builtin_amdgcn_rcpf(u - 1.f);
-}
-
 DEV float gate_f(float x, bool silu) { return (silu ? x : 1.f) * sigmoid_f(x); }
-
-// rate = exp(A_log)
-DEV float decay_f(float z, float rate) { return __expf(-rate * softplus_f(z)); }
 
 // Where a token's convolution finds its inputs: ``back`` rows before ``row`` belong to
 // this step, older ones are in the ring.  p: the token's position.
@@ -286,28 +276,6 @@ struct Words {
   }
 };
 
-// The sequence of workgroups z.  The longest ones come first, as workgroups start in order of
-// z and a sequence's tokens are a serial chain, and they go first on a SIMD, too: 16 heads of 128,
-// 5 sequences of 571 to 2536 tokens 687 us as they came, 556 longest first; 12 of 443 to 2536 979,
-// 920 in order, 884 with priorities.  More than a wave's lanes: as they come.
-static DEV int longest_first(const DeltaArgs& a, int z) {
-  if (a.seqs == 1 || a.seqs > 64) return z;
-  const int lane = threadIdx.x & 63, at = min(lane, a.seqs - 1);
-  const int len = a.seq_lens[at] - a.ctx_lens[at];
-  int rank = 0, most = 0;
-  for (int i = 0; i < a.seqs; ++i) {
-    const int other = __builtin_amdgcn_readlane(len, i);
-    rank += other > len || (other == len && i < lane);
-    most = max(most, other);
-  }
-  const int seq = __builtin_ctzll(__ballot(lane < a.seqs && rank == z));
-  const int mine = __builtin_amdgcn_readlane(len, seq);
-  if (mine > most / 4 * 3) __builtin_amdgcn_s_setprio(3);
-  else if (mine > most / 2) __builtin_amdgcn_s_setprio(2);
-  else if (mine > most / 4) __builtin_amdgcn_s_setprio(1);
-  return seq;
-}
-
 // grid (column blocks, H, seqs).  Lane j of a column's 16 holds the dims
 // (e / VW) * 16 VW + j VW + e % VW: its LDS reads are VW wide and 16 lanes contiguous.
 // FULL: D = 16 DPL and rows are aligned to VW channels.  HEAD: one decay per head.
@@ -489,19 +457,8 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const DeltaArgs a) {
       if (dim(e) < a.D && col < a.V) S[(int64_t)dim(e) * a.V + col] = s[c][e];
     }
 
-  // the head's last convolution inputs; delta_inputs has read the old ones
-  if (blockIdx.x == 0) {
-    const int group = a.H / a.G;
-    const int total = (h % group == 0 ? 2 * a.D : 0) + a.V;
-    T* ring = (T*)a.ring + slot * a.taps * a.C;
-    for (int i = tid; i < total; i += 256) {
-      const int c = i < a.V ? 2 * a.G * a.D + h * a.V + i
-                  : i < a.V + a.D ? kvh * a.D + i - a.V : (a.G + kvh) * a.D + i - a.V - a.D;
-      for (int t = max(0, len - a.taps); t < len; ++t)
-        ring[(int64_t)((ctx + t) % a.taps) * a.C + c] =
-            ((const T*)a.qkv)[(row0 + t) * a.qkv_stride + c];
-    }
-  }
+  // delta_inputs has read the old ones
+  if (blockIdx.x == 0) keep_inputs<T>(a, h, ctx, len, row0, slot);
 }
 
 // LANES lanes per token and head, 16 or a wave.
@@ -743,7 +700,8 @@ static void prompts(const DeltaArgs& a, int cpl, hipStream_t stream) {
     auto inputs = even ? delta_inputs_kernel<T, 2> : delta_inputs_kernel<T, 1>;
     inputs<<<grid, 256, 0, stream>>>(a);
   }
-  if (a.D <= 16) launch_scan_cols<T, 1>(a, cpl, stream);
+  if (a.chunks) launch_delta_chunks(&a, cpl, stream);
+  else if (a.D <= 16) launch_scan_cols<T, 1>(a, cpl, stream);
   else if (a.D <= 32) launch_scan_cols<T, 2>(a, cpl, stream);
   else if (a.D <= 64) launch_scan_cols<T, 4>(a, cpl, stream);
   else if (a.D <= 128) launch_scan_cols<T, 8>(a, cpl, stream);

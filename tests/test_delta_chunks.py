@@ -1,0 +1,76 @@
+"""The gated delta rule of a prompt by chunks of 16 tokens (csrc/delta_chunks.hip) against double
+precision and against the recurrence token by token, and which prompts take it."""
+import pytest
+import torch
+
+from agentcontrolplane_amd.engine.batch import SeqMeta
+from agentcontrolplane_amd.ops import hip
+from op_helpers import BF16, close
+from test_noganex_ops import HeadDeltaCase
+from test_tezinex_ops import DeltaCase
+
+
+@pytest.mark.parametrize("lens,H,D,V,dtype,want", [
+    ([48] * 9, 16, 128, 128, BF16, 0), ([49], 16, 128, 128, BF16, 1), ([1, 8000], 32, 128, 128, BF16, 1),
+    ([500] * 4, 16, 128, 128, BF16, 1), ([500] * 5, 16, 128, 128, BF16, 2),
+    ([500] * 5, 16, 128, 144, BF16, 1), ([500], 16, 64, 128, BF16, 0), ([500], 16, 128, 130, BF16, 0),
+    ([500], 16, 128, 128, torch.float32, 0),
+])
+def test_which_prompts_go_by_chunks(lens, H, D, V, dtype, want):
+    metas = [SeqMeta(i, n, n, 0, [0], True, i) for i, n in enumerate(lens)]
+    assert hip._scan_in_chunks(metas, H, D, V, dtype) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [DeltaCase, HeadDeltaCase])
+@pytest.mark.parametrize("H,G,V,lens,columns", [
+    (4, 2, 128, [49, 5, 64, 16, 1, 17, 130], 1), (4, 2, 128, [49, 5, 64, 16, 1, 17, 130], 2),
+    (3, 3, 48, [81], 1), (2, 1, 32, [97, 33, 32], 2), (1, 1, 16, [50, 2], 1),
+])
+def test_delta_by_chunks(kind, H, G, V, lens, columns, monkeypatch):
+    """Whole chunks, an odd and an even number of them, ragged and single tokens, first from nothing and then
+    from the kept state.  States differ from those token by token by sums of 128 terms in
+    32 bits, results by a rounding to 16 bits besides."""
+    ends = {}
+    for mode in (0, columns):
+        monkeypatch.setattr(hip, "_scan_in_chunks", lambda *a, mode=mode: mode)
+        case = kind(H, G, 128, V, 4, [2 * n for n in lens], BF16, "cuda")
+        plan = [(s, n) for s, n in enumerate(lens)]
+        got = [torch.cat(rows) for rows in zip(case.step(plan), case.step(plan))]
+        for s, rows in enumerate(got):
+            close(rows, case.want(s), BF16)
+        ends[mode] = torch.cat(got).double(), case.state[case.slots].double()
+    (rows, state), (rows0, state0) = ends[columns], ends[0]
+    slack = 128 * 2.0 ** -24
+    assert ((state - state0).abs() <= slack * state0.abs().amax()).all()
+    assert ((rows - rows0).abs() <= 2.0 ** -7 * rows0.abs() + 64 * slack * rows0.abs().amax()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("columns", [1, 2])
+def test_chunks_of_extreme_decays(columns, monkeypatch):
+    """Decays of exactly one and zero, keys that are all the same: no overflow, no loss."""
+    monkeypatch.setattr(hip, "_scan_in_chunks", lambda *a: columns)
+    case = DeltaCase(2, 2, 128, 32, 4, [75], BF16, "cuda")
+    case.z[:, ::3], case.z[:, 1::3] = 300.0, -300.0
+    close(case.step([(0, 75)])[0], case.want(0), BF16)
+    case = DeltaCase(2, 2, 128, 32, 4, [75], BF16, "cuda")
+    case.qkv[:, 256:512], case.b[:], case.A_log[:] = case.qkv[:1, 256:512], 8.0, -8.0
+    close(case.step([(0, 75)])[0], case.want(0), BF16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("columns", [1, 2])
+@pytest.mark.parametrize("at,what", [("v", "nan"), ("v", "inf"), ("k", "nan"), ("z", "nan")])
+def test_chunks_are_causal(columns, at, what, monkeypatch):
+    """What is no number reaches no token ahead of it, and no other sequence."""
+    monkeypatch.setattr(hip, "_scan_in_chunks", lambda *a: columns)
+    case = DeltaCase(2, 2, 128, 32, 1, [60, 20], BF16, "cuda")
+    want = [case.want(0), case.want(1)]
+    t = 41
+    rows = {"v": case.qkv[t, 512:], "k": case.qkv[t, 256:512], "z": case.z[t]}[at]
+    rows[:] = float(what)
+    first, second = case.step([(0, 60), (1, 20)])
+    close(first[:t], want[0][:t], BF16)
+    close(second, want[1], BF16)
+    assert first[t + 1 :].isnan().all()
