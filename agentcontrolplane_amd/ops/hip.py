@@ -429,26 +429,26 @@ def _grouped_decode(out, q, k_cache, v_cache, tables, seq_lens, sink, bias, gate
     depend on sizes alone, not on the lengths, so that a step can be captured."""
     (B, H, d), v, G = q.shape, out.shape[2], k_cache.shape[2]
     gm = next((n for n in (1, 2, 4) if n >= H // G), 8)  # query heads a workgroup holds
-    # pieces of the step's keys: workgroups that fill the chip
+    # workgroups that fill the chip at once
     keys = min(tables.shape[1] * k_cache.shape[1], window + keep_first, chunk)
     groups = G * -(-(H // G) // gm)
     pieces, part, ml = 0, None, None
     if B * groups < _WHOLE_GROUPS and keys > 128:
         pieces = max(1, _DECODE_GROUPS // groups)
-        part = torch.empty((pieces + B) * H * v, dtype=torch.float32, device=q.device)
-        ml = torch.empty(2 * (pieces + B) * H, dtype=torch.float32, device=q.device)
+        part = torch.empty(2 * (2 * pieces + B) * H * v, dtype=torch.float32, device=q.device)
+        ml = torch.empty(4 * (2 * pieces + B) * H, dtype=torch.float32, device=q.device)
     _C.grouped_attn(
         out, q, k_cache, v_cache, tables, seq_lens, None, None, None, None, sink, bias, gate,
         None, part, ml, scale, cap, window, chunk, keep_first, sigmoid, _DECODE, gm, pieces,
     )
 
 
-#: workgroups that a decode step's keys are cut for: 2 rounds of the 2 a CU that fit
-_DECODE_GROUPS = 1024
-#: from so many sequences and key heads on a sequence is one piece (190 x 8, 700 to 1300 keys:
-#: 159 us, cut as fewer ones 169; 250 x 8, 200 to 2000 keys: 235 and 250 us; 130 x 8, 100 to 8000
-#: keys: 454 and 476).  The host does not see the lengths: where one sequence is by far the longest
-#: that is the slower choice (129 x 300 keys and one of 8000: 156 and 59 us)
+#: workgroups that share a decode step's keys: the 2 a CU that fit
+_DECODE_GROUPS = 512
+#: from so many sequences and key heads on a sequence is one workgroup's (of 8 heads 190 x 700 to 1300 keys: 141
+#: us, in even shares 144 with the merge; 256 x 1024 174 and 194; 230 x 500 to 3500 331 and 326).  The host
+#: does not see the lengths: where one sequence is by far the longest that is the slower choice (129 x 300
+#: keys and one of 8000: 155 and 58 us)
 _WHOLE_GROUPS = 1024
 
 

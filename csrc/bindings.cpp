@@ -894,7 +894,7 @@ static void grouped_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
   CHECK_CUDA(tables); CHECK_CONT(tables);
   TORCH_CHECK(tables.scalar_type() == at::kInt && tables.dim() == 2);
   const int seqs = tables.size(0);
-  // kind 1: n_split is the pieces that a step's keys are cut into, 0: one a sequence
+  // kind 1: n_split is the workgroups of a key head that share a step's keys, 0: one a sequence
   TORCH_CHECK(window > 0 && keep >= 0 && cap >= 0 && n_split >= (kind != 1) &&
               n_split <= (kind == 1 ? 1 << 16 : 64));
   TORCH_CHECK(chunk > 0 && chunk <= (1 << 30) && (keep == 0 || chunk == (1 << 30)),
@@ -907,7 +907,7 @@ static void grouped_attn(torch::Tensor out, torch::Tensor q, torch::Tensor k_cac
   GroupedArgs a{};
   a.out = out.data_ptr();
   if (kind == 1 ? n_split > 0 : n_split > 1) {
-    const int64_t rows = kind == 1 ? (n_split + seqs) * H : n_split * tokens * H;
+    const int64_t rows = kind == 1 ? 2 * (2 * n_split + seqs) * H : n_split * tokens * H;
     TORCH_CHECK(part && part_ml && part->is_contiguous() && part_ml->is_contiguous());
     TORCH_CHECK(part->scalar_type() == at::kFloat && part_ml->scalar_type() == at::kFloat);
     CHECK_CUDA((*part)); CHECK_CUDA((*part_ml));

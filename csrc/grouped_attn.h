@@ -4,8 +4,8 @@
 
 struct GroupedArgs {
   void* out;              // [tokens, H, v], tokens out_stride apart
-  float* part;            // [n_split, rows, v], decode [pieces + seqs, H, v]
-  float2* part_ml;        // [n_split, rows], decode [pieces + seqs, H]
+  float* part;            // [n_split, rows, v], decode [2 (2 pieces + seqs), H, v]
+  float2* part_ml;        // [n_split, rows], decode [2 (2 pieces + seqs), H]
   const void* q;          // [tokens, H, d], tokens q_stride apart
   const void* k_cache;    // [slots, G, d]
   const void* v_cache;    // [slots, G, v]
@@ -21,7 +21,9 @@ struct GroupedArgs {
   const int* tile_q0;     // [tiles] first token of the tile within the chunk
   int64_t q_stride, out_stride, gate_stride;
   int H, G, group, n_tiles, max_blocks, kv_block, window, keep, n_split, rows, n_bias;
-  int seqs, pieces;       // decode: about how many pieces the step's keys are cut into
+  int seqs, pieces;       // decode: workgroups of a key head that share the step's keys; 0: one a sequence
+  int gm;                 // decode: query heads of a workgroup
+  bool ranges;            // decode: they may take parts of several sequences each
   int chunk;              // only keys of the query's own chunk; 2^30: all
   float scale, cap;       // cap 0: none
   bool sigmoid;           // weights sigmoid(score), not a softmax

@@ -12,12 +12,13 @@
 // the next 32 in flight meanwhile: keys as the matrix cores want them (16 keys by 8 dims a lane),
 // the heads that share them are the columns of one product; values as 8 dims a lane, weighted in
 // fp32 by the VALU.  Between the two the weights pass through a few LDS rows of the wave.
-// The blocks of 32 that a sequence's query sees are cut into pieces of one size, so that the
-// pieces of a step, whatever its lengths, fill the chip evenly; a workgroup finds its piece from
-// the lengths by itself, and a second launch merges sequences of several pieces.
-// Bound by memory: 5.2 to 5.3 TB/s of keys and values at 64 x 4096 and 256 x 1024 tokens, 32
-// heads over 8.  Before, with products and sums over dims on the VALU, 4.1 TB/s there and 2.0 to
-// 3.0 where lengths differ: 61 x 310 to 4000 tokens 268 -> 122 us, 190 x 700 to 1300 265 -> 159,
+// The blocks of 32 that the sequences' queries see are cut into even shares of the workgroups that are resident at
+// once, whatever the lengths (Cut, below); a workgroup finds its share from the lengths by itself, and a
+// second launch merges sequences of several workgroups.
+// Bound by memory: 6.0 to 6.2 TB/s of keys and values at 64 x 4096 and 256 x 1024 tokens, 32
+// heads over 8; 61 x 310 to 4000 118 -> 111 us by even shares of all keys, 61 x 670 to 7900 210 -> 188.
+// Before, with products and sums over dims on the VALU, 4.1 TB/s there and 2.0 to 3.0 where
+// lengths differ: 61 x 310 to 4000 tokens 268 -> 122 us, 190 x 700 to 1300 265 -> 159,
 // 1 x 4002 203 -> 14; with the values' loads, whole lines each, past the caches 190 x 700 to 1300 148
 // -> 139, 61 x 310 to 4000 120 -> 112.5, and 13 x 300 to 3900 of 32 key heads 95 -> 88; with the
 // keys' loads likewise, instead of 16 rows of half a line, 137, 109 and 85, 200 x 100 to 1000 of 64
@@ -66,9 +67,9 @@ static DEV Blocks visible_blocks(const GroupedArgs& a, int pos) {
   return b;
 }
 
-// A sequence's pieces: ``n`` blocks, ``size`` of them a piece, numbered from ``first`` on.
-struct Pieces {
-  int seq, len, n, size, pieces, first;
+// A sequence's blocks, one if it has none, or pieces (``n``), and those of the sequences ahead of it
+struct Stretch {
+  int seq, len, n, before;
 };
 
 // sum of the lanes up to this one (row shifts and broadcasts of rows' last lanes)
@@ -111,70 +112,94 @@ static DEV float max_with(float v) {
   return fmaxf(r.x, r.y);
 }
 
-// Pieces have about equally many blocks, a multiple of 4, so many that they are at most
-// a.pieces and one for every sequence.  Half as many pieces, one round of workgroups, are better
-// while they have up to 12 blocks (20 x 300 to 1024 keys: 24 us, else 29; with up to 16, 50 x 400 to
-// 1500 in windows of 1024: 49.9, else 46.3) or are whole sequences (64 x 1024: 60, else 69); long
-// parts are too uneven (61 x 310 to 4000: 141, else 122).  a.pieces == 0: every sequence is one
-// piece.  Finds those of sequence ``want``, or those with piece ``item`` (pieces == 0: there is
-// none).  A wave's lanes read the lengths, 64 at a time.
-// Every workgroup begins with this and then waits for its first keys, so that its length counts: with
-// general divisions and a length read twice 64 x 128 keys took 16.6 us, now 15.5, 16 x 1024 with two
-// heads a key head 22.1 and 21.2.  Fewer workgroups with several pieces each: 1 us more.
-static DEV Pieces find_pieces(const GroupedArgs& a, int want, int item) {
+// How a step's blocks are cut for the a.pieces workgroups of a key head.
+//
+// Into ranges of all sequences' blocks, one after the other, whatever the sequences: a workgroup's
+// parts of sequences follow each other, and all workgroups, which are resident at once, end at about the
+// same time.  Of many blocks a workgroup has two ranges half as long, of two key heads, as rows
+// of some heads come more slowly than others (XCDs and channels share unevenly: one head each, 64 x 2048
+// keys end after 68 to 93 us, two 64 to 87).  61 x 310 to 4000 keys of 8 heads, the kernel alone: pieces of
+// sequences, up to 1112 workgroups in turn, 105 us, ranges 98, of two heads 93.
+//
+// Or few blocks into pieces of one sequence each, where that leaves no workgroup with much more than its share:
+// parts have starts and ends, 4 x 300 keys 16.0 us by ranges and 11.8 by pieces, 64 x 512 35.4 and 32.
+//
+// Without a.ranges always pieces, in two rounds of half of the size where one round is uneven: the kernel with
+// several parts is 0.5 to 1 us slower for one, so that few sequences go without (RANGES_FROM), and for 8 query
+// heads a workgroup it has not the registers.
+struct Cut {
+  bool aligned;  // pieces of sequences
+  int count;     // ranges of a workgroup
+  int each;      // blocks of a range, at most of a piece
+};
+
+// Finds the cut and the sequence ``want``, or the one with the first block of workgroup ``item`` of a
+// key head (seq < 0: it has none).  A wave's lanes read the lengths, 64 at a time.  Every workgroup begins
+// with this and then waits for its first keys, so that its length counts: with general divisions and a
+// length read twice 64 x 128 keys took 16.6 us instead of 15.5.
+static DEV Stretch find_range(const GroupedArgs& a, int want, int item, Cut& cut) {
   const int lane = threadIdx.x & 63;
   auto len_of = [&](int seq) { return seq < a.seqs ? a.seq_lens[seq] : 0; };
-  auto blocks_of = [&](int len) { return visible_blocks(a, len - 1).n; };
-  Pieces p = {0, 0, 0, 0, 0, 0};
-  if (a.pieces == 0) {
-    p.seq = p.first = item;
-    p.len = a.seq_lens[item];
-    p.n = p.size = blocks_of(p.len);
-    p.pieces = 1;
-    return p;
-  }
-  const int len0 = len_of(lane), mine0 = blocks_of(len0);
+  auto blocks_of = [&](int seq, int len) {  // an empty sequence has a turn, too
+    return seq < a.seqs ? max(1, visible_blocks(a, len - 1).n) : 0;
+  };
+  const int len0 = len_of(lane), mine0 = blocks_of(lane, len0);
   int total = mine0, longest = mine0;
   for (int s = 64; s < a.seqs; s += 64) {
-    const int n = blocks_of(len_of(s + lane));
+    const int n = blocks_of(s + lane, len_of(s + lane));
     total += n;
     longest = max(longest, n);
   }
   total = __builtin_amdgcn_readlane(wave_scan(total), 63);
-  const int half = max(1, quotient(total + 2 * a.pieces - 1, 2 * a.pieces));
-  const int all = max(min(half, 3), (half + 1) / 2);
-  const int size = 4 * (__any(longest > 4 * half) ? all : half);
-  const int spare = size - (size < 12 ? 0 : size / 4) - 1;
+  const int share = quotient(total + a.pieces - 1, a.pieces), spare = a.pieces - a.seqs;
+  int few = 0;
+  cut.aligned = false;
+  cut.count = 1;
+  cut.each = max(4, share);
+  if (!a.ranges || (share <= 32 && spare >= 0)) {
+    const int even = share + 3 & ~3, most = share + share / 4 + 4;
+    few = quotient(mine0 + even - 1, even);
+    cut.aligned = true;
+    if (a.seqs <= 64 && __builtin_amdgcn_readlane(wave_scan(few), 63) <= a.pieces) {
+      cut.each = even;
+    } else if (spare >= 0 && !__any(longest > most)) {  // whole sequences
+      cut.each = most;
+    } else if (!a.ranges) {  // at most 2 a.pieces and one for every sequence
+      cut.each = max(4, (share + 7) / 8 * 4);
+    } else {
+      const int each = spare > 0 ? quotient(total + spare - 1, spare) : most + 1;
+      cut.aligned = each <= most;
+      if (cut.aligned) cut.each = max(4, each);
+    }
+  } else if (share > 32 && !(a.G * ((a.group + a.gm - 1) / a.gm) & 1)) {
+    cut.count = 2;
+    cut.each = (share + 1) / 2;
+  }
+  const int first = cut.aligned ? item : item * cut.count * cut.each;
+  const bool known = cut.aligned && a.seqs <= 64 && cut.each == (share + 3 & ~3);
+  Stretch x = {-1, 0, 0, 0};
   int before = 0;
   for (int s = 0; s < a.seqs; s += 64) {
-    const int len = s ? len_of(s + lane) : len0, n = s ? blocks_of(len) : mine0;
-    // a last piece of under a quarter is shared by the others
-    int k = max(1, quotient(n + spare, size)), each = size;
-    if (k * size < n) {
-      each = 4 * quotient(n + 4 * k - 1, 4 * k);
-      k = quotient(n + each - 1, each);
-    }
-    if (s + lane >= a.seqs) k = 0;
-    const int upto = before + wave_scan(k);  // pieces up to this lane's
-    const bool mine = want >= 0 ? s + lane == want : item >= upto - k && item < upto;
-    const uint64_t hit = __ballot(mine);
+    const int len = s ? len_of(s + lane) : len0, n = s ? blocks_of(s + lane, len) : mine0;
+    const int mine = known ? few : cut.aligned ? quotient(n + cut.each - 1, cut.each) : n;
+    const int upto = before + wave_scan(mine);  // blocks or pieces up to this lane's
+    const uint64_t hit = __ballot(want >= 0 ? s + lane == want : first < upto);
     if (hit) {
       const int at = __builtin_ctzll(hit);
-      p.seq = s + at;
-      p.len = __builtin_amdgcn_readlane(len, at);
-      p.n = __builtin_amdgcn_readlane(n, at);
-      p.size = __builtin_amdgcn_readlane(each, at);
-      p.pieces = __builtin_amdgcn_readlane(k, at);
-      p.first = __builtin_amdgcn_readlane(upto - k, at);
+      x.seq = s + at;
+      x.len = __builtin_amdgcn_readlane(len, at);
+      x.n = __builtin_amdgcn_readlane(mine, at);
+      x.before = __builtin_amdgcn_readlane(upto, at) - x.n;
       break;
     }
     before = __builtin_amdgcn_readlane(upto, 63);
   }
-  return p;
+  return x;
 }
 
-// PAGED: pages of 16 2^n keys, so that a group of 16 keys has one, scalar, place
-template <int DN, int VN, int GM, bool SIG, bool PAGED>
+// PAGED: pages of 16 2^n keys, so that a group of 16 keys has one, scalar, place.  CUT: the blocks are
+// cut (a.pieces > 0), else a workgroup has a sequence.  RANGES: as a.ranges
+template <int DN, int VN, int GM, bool SIG, bool PAGED, bool CUT, bool RANGES>
 __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kernel(const GroupedArgs a) {
   constexpr int D = 64 * DN, V = 64 * VN, STEPS = D / 32;
   constexpr int LPK = V / 8, KPL = 64 / LPK, NV = KB / KPL;  // lanes a key, keys a load, loads
@@ -186,31 +211,81 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   const int group = a.group, per = (group + GM - 1) / GM;  // workgroups per kv head
   // Whole sequences of up to 8 workgroups stay on one XCD, whose L2 then sees whole rows of the
   // cache: 190 x 700 to 1300 keys of 8 heads 152 to 148 us, 230 x 500 to 3500 367 to 352, but of 32
-  // heads 60 x 100 to 800 89 to 102, and pieces 2% slower
-  const int each = per * a.G;
-  const int even = a.pieces == 0 && each <= 8 ? gridDim.x / each & ~7 : 0;
-  const bool near_by = (int)blockIdx.x < even * each;
-  const int nth_wg = near_by ? blockIdx.x >> 3 : blockIdx.x - even * each, nth_item = nth_wg / each;
-  const int at_g = nth_wg - nth_item * each;
+  // heads 60 x 100 to 800 89 to 102, and ranges 3% slower
+  const int workgroups = per * a.G;  // of the same keys
+  const int even = !CUT && workgroups <= 8 ? a.seqs & ~7 : 0;
+  const bool near_by = (int)blockIdx.x < even * workgroups;
+  const int nth_wg = near_by ? blockIdx.x >> 3 : blockIdx.x - even * workgroups;
+  const int nth_item = nth_wg / workgroups, first_at = nth_wg - nth_item * workgroups;
   const int item = near_by ? nth_item * 8 + (blockIdx.x & 7) : even + nth_item;
-  const int kvh = per > 1 ? at_g / per : at_g, part = at_g - kvh * per;
-  const int h0 = kvh * group + part * GM, heads = min(GM, group - part * GM);
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, j = lane >> 4;           // product: column (head), rows 4 j ..
   const int kl = lane / LPK, el = lane % LPK;       // values: key of a load, 8 dims
 
-  const Pieces p = find_pieces(a, -1, item);
-  if (p.pieces == 0) return;  // more workgroups than pieces
-  const int seq = p.seq, pos = p.len - 1, nth = item - p.first;
-  const Blocks blocks = visible_blocks(a, pos);
-  const int end = min(p.n, (nth + 1) * p.size);
-  const int lo = first_key(a, pos);
+  // The part of a sequence that is worked on: blocks ``from`` .. ``to`` - 1 of n
+  struct Part {
+    int seq, pos, n, from, to, lo;
+    int range, left;      // of the step's ranges; blocks up to its end
+    int at, kvh, h0, heads;  // of the workgroups of the same keys: its key head, its query heads
+    bool goes_on;         // it is not its range's first one
+    Blocks blocks;
+    const const_int* pages;
+  };
+  auto part_of = [&](Part p, int seq, int len, int from, int left) {
+    p.seq = seq;
+    p.pos = len - 1;
+    p.blocks = visible_blocks(a, p.pos);
+    p.n = p.blocks.n;
+    p.from = from;
+    p.to = min(p.n, from + left);
+    p.left = left;
+    p.lo = first_key(a, p.pos);
+    p.pages = (const const_int*)(a.tables + (int64_t)seq * a.max_blocks);
+    return p;
+  };
+  auto aim = [&](Part& p, int at) {
+    p.at = at;
+    p.kvh = per > 1 ? at / per : at;
+    p.h0 = p.kvh * group + (at - p.kvh * per) * GM;
+    p.heads = min(GM, group - (at - p.kvh * per) * GM);
+  };
+  Part p = {};  // that the loads are in
+  aim(p, first_at);
+  Cut cut = {};
+  int done = 0;  // blocks of the workgroup's ranges ahead of this part
+  if (CUT) {
+    const Stretch x = find_range(a, -1, item, cut);
+    if (x.seq < 0) return;  // more workgroups than there is work for
+    p.range = item * cut.count;
+    p = part_of(p, x.seq, x.len,
+                cut.aligned ? (item - x.before) * cut.each : p.range * cut.each - x.before, cut.each);
+  } else {
+    p = part_of(p, item, a.seq_lens[item], 0, 1 << 30);
+  }
+  // The next part: of the next sequence, or of the next range, whose keys are of the workgroup's other head.
+  // false: there is none
+  auto go_on = [&]() {
+    if (!RANGES || cut.aligned) return false;
+    const int blocks = max(1, p.to - p.from);
+    done += blocks;
+    const int left = p.left - blocks;
+    const bool same = left > 0, stays = !same && p.to < p.n;
+    if (!same) {
+      ++p.range;
+      aim(p, p.at ^ 1);
+      if (cut.count == 1 || !(p.range & 1)) return false;
+    }
+    const int seq = p.seq + !stays;
+    if (seq >= a.seqs) return false;
+    p.goes_on = same;
+    p = part_of(p, seq, stays ? p.pos + 1 : ((const const_int*)a.seq_lens)[seq], stays ? p.to : 0,
+                same ? left : cut.each);
+    return true;
+  };
 
   const uint32_t k_row = (uint32_t)a.G * D * 2, v_row = (uint32_t)a.G * V * 2;  // bytes
-  const char* kp = (const char*)a.k_cache + (int64_t)kvh * D * 2;
-  const char* vp = (const char*)a.v_cache + (int64_t)kvh * V * 2;
-  const int* table = a.tables + (int64_t)seq * a.max_blocks;
-  const const_int* pages = (const const_int*)table;
+  const char* const k0 = (const char*)a.k_cache;
+  const char* const v0 = (const char*)a.v_cache;
   const int shift = __builtin_ctz(a.kv_block);
   // Sequences that begin alike hold the same pages, at the same places of their tables.  Lanes look
   // at the next 64 sequences' page where this piece begins; a block whose pages are those of one that
@@ -218,30 +293,32 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   // the same key head reads.  All kept, all past, and so, us: 190 x 700 to 1300 keys of 8 heads, 608
   // in common 107, 117, 103, none 147, 133, 134; 60 of 32 heads 121, 131, 115 and 184, 168, 167; 16
   // heads a key head 64 x 700 to 1300 114, 121, 107.
-  const const_int* others = pages;
+  const const_int* others = p.pages;
   bool begins_alike = false;
   auto look = [&](int page, int there) {
     const uint64_t alike = __ballot(page == there && lane + 1 < a.seqs);
     begins_alike = alike != 0;
-    int other = seq + 1 + (alike ? __builtin_ctzll(alike) : 0);
+    int other = p.seq + 1 + (alike ? __builtin_ctzll(alike) : 0);
     if (other >= a.seqs) other -= a.seqs;
-    others = (const const_int*)(a.tables + (int64_t)(begins_alike ? other : seq) * a.max_blocks);
+    others = (const const_int*)(a.tables + (int64_t)(begins_alike ? other : p.seq) * a.max_blocks);
   };
   struct Place {
     int slot[2];  // of a block's two groups of 16 keys
+    int kvh;
     bool shared;
   };
   auto find = [&](int i) {
     Place at;
-    const int key0 = blocks.key(i);
-    auto key = [&](int g) { return min(key0 + 16 * g, pos & ~15); };
+    at.kvh = p.kvh;
+    const int key0 = p.blocks.key(i);
+    auto key = [&](int g) { return min(key0 + 16 * g, p.pos & ~15); };
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       const int k = key(g);
-      at.slot[g] = PAGED ? (pages[k >> shift] << shift) + (k & (a.kv_block - 1)) : 0;
+      at.slot[g] = PAGED ? (p.pages[k >> shift] << shift) + (k & (a.kv_block - 1)) : 0;
     }
-    at.shared = PAGED && begins_alike && pages[key(0) >> shift] == others[key(0) >> shift] &&
-                pages[key(1) >> shift] == others[key(1) >> shift];
+    at.shared = PAGED && begins_alike && p.pages[key(0) >> shift] == others[key(0) >> shift] &&
+                p.pages[key(1) >> shift] == others[key(1) >> shift];
     return at;
   };
   // A load of keys has 8 rows of whole lines, 64 dims: the upper 8 rows of a product, and its upper 8
@@ -254,6 +331,8 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
   const int c8 = c & 7, half = c >> 3;
   const uint32_t k_off = c8 * k_row + half * 64 + j * 16, v_off = kl * v_row + el * 16;
   auto load_paged = [&](auto shared, const Place& at, Rows& r) {
+    const char* const kp = k0 + at.kvh * D * 2;
+    const char* const vp = v0 + at.kvh * V * 2;
     auto get = [&](const char* p) {
       if constexpr (decltype(shared)::value) return *(const bf16x8_v*)p;
       return __builtin_nontemporal_load((const bf16x8_v*)p);
@@ -283,63 +362,76 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
         asm volatile("; past, end" ::: "memory");
       }
     } else {
-      const int k = min(blocks.key(i) + (lane & (KB - 1)), pos);
+      const int k = min(p.blocks.key(i) + (lane & (KB - 1)), p.pos), kvh = p.kvh;
       const int page = k / a.kv_block;
-      if (lane < KB) slots[wid][lane] = table[page] * a.kv_block + k - page * a.kv_block;
+      if (lane < KB)
+        slots[wid][lane] = a.tables[(int64_t)p.seq * a.max_blocks + page] * a.kv_block + k -
+                           page * a.kv_block;
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           const uint32_t slot = slots[wid][g * 16 + p * 8 + c8];
-          const char* kr = kp + (uint64_t)slot * k_row + half * 64 + j * 16;
+          const char* kr = k0 + kvh * D * 2 + (uint64_t)slot * k_row + half * 64 + j * 16;
 #pragma unroll
           for (int s = 0; s < LINES; ++s) r.k[g][p][s] = *(const bf16x8_v*)(kr + s * 128);
         }
 #pragma unroll
       for (int n = 0; n < NV; ++n)
-        r.v[n] = *(const bf16x8_v*)(vp + (uint64_t)(uint32_t)slots[wid][n * KPL + kl] * v_row + el * 16);
+        r.v[n] = *(const bf16x8_v*)(v0 + kvh * V * 2 + (uint64_t)(uint32_t)slots[wid][n * KPL + kl] * v_row +
+                                    el * 16);
       __builtin_amdgcn_wave_barrier();
     }
   };
+  // A part's first loads: the workgroup's blocks go to the waves in turn, whichever sequences they are of.
+  // The heads' queries are columns, 8 dims a lane and step
   Rows r0, r1;
-  int i = nth * p.size + wid;
   Place at{};
-  if (i < end) {
-    // a piece of a few blocks is over before the answer pays
-    const bool ask = PAGED && per == 1 && a.seqs > 1 && p.size > 8;
-    int there = 0;
-    const int first = min(blocks.key(nth * p.size), pos & ~15) >> shift;
-    if (ask) {
-      int other = seq + 1 + lane;
-      other -= other >= a.seqs ? a.seqs : 0;
-      there = a.tables[(int64_t)min(other, a.seqs - 1) * a.max_blocks + first];
-    }
-    load(i, find(i), r0);
-    if (ask) look(pages[first], there);
-    if (AHEAD && PAGED) at = find(min(i + 4, p.n - 1));
-  }
-
-  // the heads' queries as columns, 8 dims a lane and step
-  const int head = h0 + min(c8, heads - 1);
+  int i;
   bf16x8_v q[LINES];
+  auto begin = [&]() {
+    i = p.from + ((wid - done) & 3);
+    if (i < p.to) {
+      // a part of a few blocks is over before the answer pays
+      const bool ask = PAGED && per == 1 && a.seqs > 1 && p.to - p.from > 8;
+      int there = 0;
+      const int first = min(p.blocks.key(p.from), p.pos & ~15) >> shift;
+      if (ask) {
+        int other = p.seq + 1 + lane;
+        other -= other >= a.seqs ? a.seqs : 0;
+        there = a.tables[(int64_t)min(other, a.seqs - 1) * a.max_blocks + first];
+      }
+      begins_alike = false;
+      load(i, find(i), r0);
+      if (ask) look(p.pages[first], there);
+      if (AHEAD && PAGED) at = find(min(i + 4, p.n - 1));
+    }
+    const int head = p.h0 + min(c8, p.heads - 1);
 #pragma unroll
-  for (int s = 0; s < LINES; ++s)
-    q[s] = *(const bf16x8_v*)((const bf16_t*)a.q + seq * a.q_stride + (int64_t)head * D + s * 64 +
-                              half * 32 + j * 8);
+    for (int s = 0; s < LINES; ++s)
+      q[s] = *(const bf16x8_v*)((const bf16_t*)a.q + p.seq * a.q_stride + (int64_t)head * D +
+                                s * 64 + half * 32 + j * 8);
+  };
+  begin();
+
   // scores in the exp2 domain: a factor, or c1 - 2 c1 / (exp2(c3 s) + 1)
   const float c1 = a.cap * LOG2E;
   const float mul = a.cap > 0.f ? 2.f * LOG2E * a.scale / a.cap : a.scale * LOG2E;
-  const bool sink = a.sink && nth == 0 && wid == 0;
-  float m = sink ? a.sink[head] * LOG2E : NEG, l = sink && j == 0 ? 1.f : 0.f;
+  float m, l;
   // biases: distances of n_bias - 1 and more share one
   const int far = a.n_bias - 1;
-  const float* bias = a.bias ? a.bias + (int64_t)head * a.n_bias : nullptr;
-  const float b_far = bias ? bias[far] * LOG2E : 0.f;
-  float acc[GM][8] = {};
+  const float* bias = nullptr;
+  float b_far = 0.f;
+  float acc[GM][8];
+  auto barrier = [&]() {  // of LDS alone: loads stay under way
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
 
   auto work = [&](int i, Rows& r) {
-    const int key0 = blocks.key(i);
+    const int key0 = p.blocks.key(i), pos = p.pos, lo = p.lo;
     auto hidden = [&](int key) { return (key > pos) | ((key < lo) & (key >= a.keep)); };
     f32x4_v halves[2][2] = {}, s[2];
 #pragma unroll
@@ -420,63 +512,90 @@ __global__ __launch_bounds__(256, DN + VN <= 4 ? 2 : 1) void grouped_decode_kern
     }
     __builtin_amdgcn_wave_barrier();
   };
-  if constexpr (AHEAD) {
-    for (; i < end; i += 8) {
-      if (i + 4 < end) {
-        load(i + 4, at, r1);
-        if (PAGED) at = find(min(i + 8, p.n - 1));
+  for (;;) {
+    const int head = p.h0 + min(c8, p.heads - 1);
+    if (a.bias) {
+      bias = a.bias + (int64_t)head * a.n_bias;
+      b_far = bias[far] * LOG2E;
+    }
+    const bool sink = a.sink && p.from == 0 && wid == 0;
+    m = sink ? a.sink[head] * LOG2E : NEG;
+    l = sink && j == 0 ? 1.f : 0.f;
+#pragma unroll
+    for (int g = 0; g < GM; ++g)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
+    if constexpr (AHEAD) {
+      for (; i < p.to; i += 8) {
+        if (i + 4 < p.to) {
+          load(i + 4, at, r1);
+          if (PAGED) at = find(min(i + 8, p.n - 1));
+        }
+        work(i, r0);
+        if (i + 4 >= p.to) break;
+        if (i + 8 < p.to) {
+          load(i + 8, at, r0);
+          if (PAGED) at = find(min(i + 12, p.n - 1));
+        }
+        work(i + 4, r1);
       }
-      work(i, r0);
-      if (i + 4 >= end) break;
-      if (i + 8 < end) {
-        load(i + 8, at, r0);
-        if (PAGED) at = find(min(i + 12, p.n - 1));
-      }
-      work(i + 4, r1);
-    }
-  } else {
-    for (; i < end; i += 4) {
-      work(i, r0);
-      if (i + 4 < end) load(i + 4, find(i + 4), r0);
-    }
-  }
-
-  // the lanes with the same dims, then the waves
-  l = sum_with<32>(sum_with<16>(l));
-  if (lane < GM) lds_ml[wid][lane] = float2{m, l};
-#pragma unroll
-  for (int g = 0; g < GM; ++g)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float o = acc[g][e];
-      if (LPK <= 8) o = sum_with<8>(o);
-      if (LPK <= 16) o = sum_with<16>(o);
-      o = sum_with<32>(o);
-      if (lane < LPK) lds_acc[wid][g][el * 8 + e] = o;
-    }
-  __syncthreads();
-  for (int n = threadIdx.x; n < heads * V; n += 256) {
-    const int g = n / V, e = n % V;
-    float mx = NEG, sum = 0.f, o = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) mx = fmaxf(mx, lds_ml[w][g].x);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float f = SIG ? 1.f : __builtin_amdgcn_exp2f(lds_ml[w][g].x - mx);
-      sum += f * lds_ml[w][g].y;
-      o += f * lds_acc[w][g][e];
-    }
-    if (p.pieces == 1) {
-      if (!SIG) o = sum > 0.f ? o / sum : 0.f;
-      if (a.gate) o *= sigmoid_f(bf2f(((const bf16_t*)a.gate)[seq * a.gate_stride + h0 + g]));
-      ((bf16_t*)a.out)[seq * a.out_stride + (int64_t)(h0 + g) * V + e] = from_f<bf16_t>(o);
     } else {
-      const int64_t row = (int64_t)item * a.H + h0 + g;
-      a.part[row * V + e] = o;
-      if (e == 0) a.part_ml[row] = float2{mx, sum};
+      for (; i < p.to; i += 4) {
+        work(i, r0);
+        if (i + 4 < p.to) load(i + 4, find(i + 4), r0);
+      }
     }
+
+    // where the results go, and the next part, whose first loads run meanwhile
+    const int seq = p.seq, slot = 2 * p.range + (p.to < p.n && p.goes_on);
+    const int h0 = p.h0, heads = p.heads;
+    const bool whole = p.from == 0 && p.to == p.n, more = go_on();
+    if (RANGES && more) begin();
+    // the lanes with the same dims, then the waves
+    l = sum_with<32>(sum_with<16>(l));
+    if (lane < GM) lds_ml[wid][lane] = float2{m, l};
+#pragma unroll
+    for (int g = 0; g < GM; ++g)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float o = acc[g][e];
+        if (LPK <= 8) o = sum_with<8>(o);
+        if (LPK <= 16) o = sum_with<16>(o);
+        o = sum_with<32>(o);
+        if (lane < LPK) lds_acc[wid][g][el * 8 + e] = o;
+      }
+    barrier();
+    for (int n = threadIdx.x; n < heads * V; n += 256) {
+      const int g = n / V, e = n % V;
+      float mx = NEG, sum = 0.f, o = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) mx = fmaxf(mx, lds_ml[w][g].x);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float f = SIG ? 1.f : __builtin_amdgcn_exp2f(lds_ml[w][g].x - mx);
+        sum += f * lds_ml[w][g].y;
+        o += f * lds_acc[w][g][e];
+      }
+      if (whole) {
+        if (!SIG) o = sum > 0.f ? o / sum : 0.f;
+        if (a.gate) o *= sigmoid_f(bf2f(((const bf16_t*)a.gate)[seq * a.gate_stride + h0 + g]));
+        ((bf16_t*)a.out)[seq * a.out_stride + (int64_t)(h0 + g) * V + e] = from_f<bf16_t>(o);
+      } else {
+        const int64_t row = (int64_t)slot * a.H + h0 + g;
+        a.part[row * V + e] = o;
+        if (e == 0) a.part_ml[row] = float2{mx, sum};
+      }
+    }
+    if (!RANGES || !more) break;
+    barrier();
   }
 }
+
+// Sequences and workgroups of the same keys from which ranges are the faster cut, us with the merge: of 8 key heads
+// 1 x 4001 keys 13.9 by pieces and 14.4, 12 x 150 to 980 16.5 and 17.5, 16 x 350 to 1000 21.0 and 21.9, 20 x 130 to
+// 3900 45.5 and 45.0, 24 x 510 to 2400 43.5 and 41.0; of 32, 3 x 850 to 2700 28.6 and 29.0, 6 x 720 to 3800 49.7
+// and 49.1
+#define RANGES_FROM 160
 
 // Merge the pieces of the rows: a lane has 4 dims of a head.  Workgroups are few, so that those
 // with nothing to merge cost little: one wave each up to MERGE_ROWS rows, else 4.
@@ -486,25 +605,35 @@ __global__ __launch_bounds__(256) void merge_pieces_kernel(const GroupedArgs a) 
   constexpr int V = 64 * VN, LANES = V / 4;  // lanes a head
   const int at = blockIdx.x * blockDim.x + threadIdx.x;
   const int h = min(at / LANES, a.H - 1), e = at % LANES * 4, seq = blockIdx.y;
-  const Pieces p = find_pieces(a, seq, -1);
-  if (p.pieces == 1) return;  // written by the piece's workgroup
+  Cut cut;
+  const Stretch x = find_range(a, seq, 0, cut);
+  int first = x.before, pieces, ahead = 0;
+  if (cut.aligned) {
+    pieces = x.n;
+  } else {
+    first = quotient(x.before, cut.each);
+    pieces = quotient(x.before + x.n - 1, cut.each) - first + 1;
+    // a range's part of a sequence that goes on is its second one if another sequence is ahead of it
+    ahead = first * cut.each < x.before;
+  }
+  if (pieces == 1) return;  // written by the workgroup
+  auto row_of = [&](int i) { return (int64_t)(2 * (first + i) + (i == 0 && ahead)) * a.H + h; };
   float m = NEG, l = 0.f, o[4] = {};
   if (!SIG) {
     // maxima and sums, a lane each
-    for (int i = e / 4; i < p.pieces; i += LANES)
-      m = fmaxf(m, a.part_ml[(int64_t)(p.first + i) * a.H + h].x);
+    for (int i = e / 4; i < pieces; i += LANES) m = fmaxf(m, a.part_ml[row_of(i)].x);
 #pragma unroll
     for (int off = LANES / 2; off; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    for (int i = e / 4; i < p.pieces; i += LANES) {
-      const float2 ml = a.part_ml[(int64_t)(p.first + i) * a.H + h];
+    for (int i = e / 4; i < pieces; i += LANES) {
+      const float2 ml = a.part_ml[row_of(i)];
       l += ml.y * __builtin_amdgcn_exp2f(ml.x - m);
     }
 #pragma unroll
     for (int off = LANES / 2; off; off >>= 1) l += __shfl_xor(l, off, 64);
   }
 #pragma unroll 8
-  for (int i = 0; i < p.pieces; ++i) {
-    const int64_t row = (int64_t)(p.first + i) * a.H + h;
+  for (int i = 0; i < pieces; ++i) {
+    const int64_t row = row_of(i);
     const float w = SIG ? 1.f : __builtin_amdgcn_exp2f(a.part_ml[row].x - m);
     const float4 v = *(const float4*)(a.part + row * V + e);
     o[0] += w * v.x;
@@ -629,15 +758,25 @@ __global__ __launch_bounds__(256) void cache_keys_values_kernel(
 
 template <int DN, int VN, int GM, bool SIG>
 static void launch_decode(const GroupedArgs& a, hipStream_t stream) {
-  const int grid = (a.pieces + a.seqs) * a.G * ((a.group + GM - 1) / GM);
+  const int per = a.G * ((a.group + GM - 1) / GM);
+  const int items = a.ranges ? a.pieces : a.pieces ? 2 * a.pieces + a.seqs : a.seqs, grid = items * per;
   const bool paged = a.kv_block >= 16 && (a.kv_block & (a.kv_block - 1)) == 0;
-  auto kernel = paged ? grouped_decode_kernel<DN, VN, GM, SIG, true>
-                      : grouped_decode_kernel<DN, VN, GM, SIG, false>;
+  auto kernel = paged ? a.pieces ? grouped_decode_kernel<DN, VN, GM, SIG, true, true, false>
+                                 : grouped_decode_kernel<DN, VN, GM, SIG, true, false, false>
+                : a.pieces ? grouped_decode_kernel<DN, VN, GM, SIG, false, true, false>
+                           : grouped_decode_kernel<DN, VN, GM, SIG, false, false, false>;
+  if constexpr (GM < 8)
+    if (a.ranges)
+      kernel = paged ? grouped_decode_kernel<DN, VN, GM, SIG, true, true, true>
+                     : grouped_decode_kernel<DN, VN, GM, SIG, false, true, true>;
   kernel<<<grid, 256, 0, stream>>>(a);
 }
 
 template <int DN, int VN>
-static bool launch_decode(const GroupedArgs& a, int gm, hipStream_t stream) {
+static bool launch_decode(const GroupedArgs& args, int gm, hipStream_t stream) {
+  GroupedArgs a = args;
+  a.gm = gm;
+  a.ranges = a.pieces && gm < 8 && a.seqs * a.G * ((a.group + gm - 1) / gm) >= RANGES_FROM;
   if (gm == 1)
     (a.sigmoid ? launch_decode<DN, VN, 1, true> : launch_decode<DN, VN, 1, false>)(a, stream);
   else if (gm == 2)
