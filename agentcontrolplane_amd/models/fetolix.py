@@ -114,8 +114,9 @@ class FetolixLayer:
             out[p + "side.norm"] = self.side_norm
         return out
 
-    def sublayers(self, h: torch.Tensor, batch: FlatBatch, cache: torch.Tensor) -> torch.Tensor:
-        """attention(h) + glu(h), [N, width]."""
+    def sublayers(self, h: torch.Tensor, batch: FlatBatch, cache: torch.Tensor,
+                  parts: bool = False) -> torch.Tensor:
+        """attention(h) + glu(h), [N, width]; ``parts``: or parts of it, as of step_linear_parts()."""
         m = self.mixer
         proj = ops.step_linear(h, self.w_in)
         mixed = torch.empty(
@@ -135,6 +136,8 @@ class FetolixLayer:
             section("q"), section("kv"), section("gate"), batch, cache,
             mixed[:, : m.out_dim],
         )
+        if parts and len(self.w_out) == 1:
+            return ops.step_linear_parts(mixed, self.w_out[0])
         return summed_linear(mixed, self.w_out)
 
 
@@ -279,18 +282,29 @@ class FetolixForCausalLM:
             if enters:
                 x = ops.step_linear(entry, self.loop_in).float()
                 h = ops.layernorm(x, layer.norm, eps, self.dtype)
-            y = layer.sublayers(h, batch, self.caches[r])
+            nxt = runs[r + 1] if r + 1 < len(runs) else None
+            norm = self.layers[nxt[0]].norm if nxt and not nxt[1] else None
+            whole = (
+                cfg.token_side_dim > 0 and self.all_reduce is None
+                and ops.side_layer_fits(
+                    x, layer.side_gate, layer.side_proj, layer.side_norm,
+                    *(() if norm is None else (norm,)),
+                )
+            )
+            y = layer.sublayers(h, batch, self.caches[r], whole)
             if self.all_reduce is not None:
                 y = self.all_reduce(y)
-            nxt = runs[r + 1] if r + 1 < len(runs) else None
             if nxt is None:
-                norm, out = None, None
-            elif nxt[1]:
-                norm, out = None, entry[:, :w]
+                out = None
             else:
-                norm, out = self.layers[nxt[0]].norm, torch.empty_like(h)
-            if cfg.token_side_dim:
-                d = cfg.token_side_dim
+                out = entry[:, :w] if nxt[1] else torch.empty_like(h)
+            d = cfg.token_side_dim
+            if whole:
+                ops.side_layer(
+                    x, y, layer.side_gate, batch.token_ids, self.side_embed, i * d,
+                    layer.side_proj, eps, layer.side_norm, norm, out,
+                )
+            elif d:
                 x, s = ops.side_gate(
                     x, y, layer.side_gate, batch.token_ids, self.side_embed, i * d
                 )

@@ -396,6 +396,25 @@ def clamped_glu(gate_up, limit: float, alpha: float, offset: float, out, cubic: 
     return _impl(gate_up).clamped_glu(gate_up, limit, alpha, offset, out, cubic)
 
 
+def step_linear_parts(x, w):
+    """step_linear(x, w), or the parts of it [parts, N, O] in fp32, which what reads them adds up in their
+    order."""
+    if _many_rows(x, w, adds=True):
+        return _hip()._C.linear_parts(x, w)
+    return step_linear(x, w)
+
+
+def side_layer_fits(x, gate, *weights) -> bool:
+    """Whether side_layer() takes this residual, this side gate and these other weights."""
+    return x.is_cuda and _hip().side_layer_fits(x, gate, *weights)
+
+
+def side_layer(x, y, gate, token_ids, table, offset: int, proj, eps: float, y_norm, x_norm, out):
+    """side_gate(x, y, ...), its product with proj, and residual_norm() of that, in one launch: x is updated
+    in place, out as of residual_norm().  y may be a product's parts (step_linear_parts())."""
+    _hip().side_layer(x, y, gate, token_ids, table, offset, proj, eps, y_norm, x_norm, out)
+
+
 def side_gate(x, y, gate, token_ids, table, offset: int):
     """The fp32 residual x + y (x itself may be reused for it) and
     gelu_tanh(gate (x + y)) * table[token, offset : offset + D]: [N, D]."""

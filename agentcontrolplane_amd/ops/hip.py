@@ -234,6 +234,26 @@ def side_gate(x, y, gate, token_ids, table, offset: int):
     return x, s
 
 
+def side_layer_fits(x, gate, *weights) -> bool:
+    """What the one launch takes, and where it is the faster: a token's workgroup reads both weights by
+    itself, which is its time once they are over 256 KB each (2048 x 64 against the three launches, without
+    the sum of the parts: 10.7 and 10.6 us with one token, 11.7 and 14.0 with 40, 22.1 and 28.9 with 512;
+    4096 x 128: 28.3 and 14.6 with one, 64 and 43 with 512)."""
+    (n, w), dim = x.shape, gate.shape[0]
+    return (
+        0 < n <= 512 and w % 8 == 0 and w <= 8192 and dim % 8 == 0 and dim <= 128
+        and 0 < w * dim <= 1 << 17
+        and all(
+            t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0
+            for t in (gate, *weights)
+        )
+    )
+
+
+def side_layer(x, y, gate, token_ids, table, offset: int, proj, eps: float, y_norm, x_norm, out):
+    _C.side_layer(x, y, gate, token_ids, table, offset, proj, eps, y_norm, x_norm, out)
+
+
 # ------------------------------------------------------------ latent attention
 
 _NO_WINDOW = 1 << 30

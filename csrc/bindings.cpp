@@ -16,6 +16,7 @@
 #include "latent_attn.h"
 #include "residual_norm.h"
 #include "linear.h"
+#include "side_layer.h"
 #include "step_linear.h"
 
 namespace py = pybind11;
@@ -69,6 +70,7 @@ void launch_cache_keys_values(void*, void*, const void*, const void*, const int6
                               int64_t, int, hipStream_t);
 void launch_delta_prompts(bool, const DeltaArgs*, int, hipStream_t);
 void launch_delta_step(bool, const DeltaArgs*, int, hipStream_t);
+void launch_side_layer(const SideLayerArgs*, hipStream_t);
 void launch_side_gate(bool, float*, const float*, const void*, const void*, const int64_t*, const void*,
                       void*, int, int, int, int64_t, hipStream_t);
 void launch_add_to_residual(bool, float*, const void*, void*, int64_t, hipStream_t);
@@ -576,6 +578,57 @@ static void side_gate(torch::Tensor s, torch::Tensor x_out, torch::Tensor x, tor
                    token_ids.data_ptr<int64_t>(),
                    (const char*)table.data_ptr() + offset * table.element_size(),
                    s.data_ptr(), n, w, dim, table.stride(0), cur_stream());
+}
+
+// x += y and the side layer; y [n, w], or [parts, n, w] fp32 of a product (linear_parts)
+static void side_layer(torch::Tensor x, torch::Tensor y, torch::Tensor gate, torch::Tensor token_ids,
+                       torch::Tensor table, int64_t offset, torch::Tensor proj, double eps,
+                       torch::Tensor y_norm, OptTensor x_norm, OptTensor out) {
+  SideLayerArgs a{};
+  const auto dt = at::kBFloat16;
+  CHECK_CUDA(x); CHECK_CONT(x);
+  TORCH_CHECK(x.dim() == 2 && x.scalar_type() == at::kFloat, "side layer: residual");
+  a.n = x.size(0);
+  a.w = x.size(1);
+  a.dim = gate.size(0);
+  TORCH_CHECK(a.w > 0 && a.w % 8 == 0 && a.w <= 8192 && a.dim > 0 && a.dim % 8 == 0 && a.dim <= 128,
+              "side layer: sizes");
+  CHECK_CUDA(y); CHECK_CONT(y);
+  if (y.dim() == 3) {
+    TORCH_CHECK(y.scalar_type() == at::kFloat && y.size(1) == a.n && y.size(2) == a.w, "side layer: parts");
+    a.parts = y.size(0);
+    TORCH_CHECK(a.parts > 0, "side layer: parts");
+  } else {
+    check_rows(y, dt, a.n, a.w);
+  }
+  check_rows(gate, dt, a.dim, a.w); CHECK_CONT(gate);
+  check_rows(proj, dt, a.w, a.dim); CHECK_CONT(proj);
+  check_rows(table, dt, table.size(0), table.size(1));
+  check_vec(y_norm, dt, a.w);
+  CHECK_CUDA(token_ids); CHECK_CONT(token_ids);
+  TORCH_CHECK(token_ids.scalar_type() == at::kLong && token_ids.numel() == a.n, "side layer: tokens");
+  TORCH_CHECK(offset >= 0 && offset + a.dim <= table.size(1), "table columns");
+  if (x_norm) check_vec(*x_norm, dt, a.w);
+  if (out) {
+    check_rows(*out, dt, a.n, a.w);
+    a.out = out->data_ptr();
+    a.out_stride = out->stride(0);
+    TORCH_CHECK(a.out_stride % 4 == 0, "side layer: strides");
+  }
+  a.x = x.data_ptr<float>();
+  a.y = y.data_ptr();
+  a.gate = gate.data_ptr();
+  a.proj = proj.data_ptr();
+  a.table = (const char*)table.data_ptr() + offset * table.element_size();
+  a.table_stride = table.stride(0);
+  a.y_norm = y_norm.data_ptr();
+  a.x_norm = x_norm ? x_norm->data_ptr() : nullptr;
+  a.token_ids = token_ids.data_ptr<int64_t>();
+  a.eps = (float)eps;
+  for (const void* p : {(const void*)a.x, a.y, a.gate, a.proj, a.y_norm, a.x_norm, (const void*)a.out})
+    TORCH_CHECK((uintptr_t)p % 16 == 0, "side layer: alignment");
+  if (a.n == 0) return;
+  launch_side_layer(&a, cur_stream());
 }
 
 static void add_to_residual(torch::Tensor x, torch::Tensor y, OptTensor out) {
@@ -1296,6 +1349,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_bf16", &gemm_bf16);
   m.attr("DEPTH_AHEAD") = DEPTH_AHEAD;
   m.def("residual_norm", &residual_norm);
+  m.def("side_layer", &side_layer);
   m.def("side_gate", &side_gate);
   m.def("add_to_residual", &add_to_residual);
   m.def("clamped_glu", &clamped_glu);

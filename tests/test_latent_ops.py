@@ -91,6 +91,41 @@ def test_side_gate(device, dtype, n, w, dim):
     close(got, want * table[tok][:, dim : 2 * dim].double().cpu(), dtype)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,w,dim,parts", [
+    (1, 8, 8, 0), (3, 40, 16, 1), (5, 4104, 24, 3), (2, 8192, 16, 16), (512, 2048, 64, 5), (40, 2048, 40, 0),
+    (7, 1000, 128, 2),
+])
+@pytest.mark.parametrize("end", ["norm", "plain", "none"])
+def test_side_layer(n, w, dim, parts, end):
+    """In one launch: the residual and what the next layer reads of it, from a product or its parts, into rows
+    of a wider tensor."""
+    device, eps = "cuda", 1e-2
+    bf = lambda *s, k, scale=1.0: rand(*s, dtype=BF16, device=device, seed=k, scale=scale)  # noqa: E731
+    x = rand(n, w, dtype=F32, device=device)
+    y = rand(parts, n, w, dtype=F32, device=device, seed=1) if parts else bf(n, w, k=1)
+    gate, proj = bf(dim, w, k=2, scale=w ** -0.5), bf(w, dim, k=3, scale=dim ** -0.5)
+    table, tok = bf(30, 3 * dim, k=4), torch.arange(n, device=device) * 7 % 30
+    y_norm, x_norm = bf(w, k=5), bf(w, k=6) if end == "norm" else None
+    wide = torch.full((n, 2 * w + 8), 7.0, device=device, dtype=BF16)
+    out = wide[:, :w] if end != "none" else None
+    assert ops.side_layer_fits(x, gate, proj, y_norm)
+    d = lambda t: t.double().cpu()  # noqa: E731
+    want = d(x) + (d(y.sum(0).bfloat16()) if parts else d(y))
+    s = oracle.gelu_tanh((want.bfloat16().double() @ d(gate).T).bfloat16().double())
+    s = (s * d(table)[tok.cpu()][:, dim : 2 * dim]).bfloat16().double()
+    z = (s @ d(proj).T).bfloat16().double()
+    want = want + z * (z.square().mean(-1, keepdim=True) + eps).rsqrt() * d(y_norm)
+    ops.side_layer(x, y, gate, tok, table, dim, proj, eps, y_norm, x_norm, out)
+    close(x, want, BF16)  # a rounding to 16 bits on its way may fall to the other side
+    assert (wide[:, w:] == 7.0).all() and (out is not None or (wide == 7.0).all())
+    if end == "norm":
+        h = torch.nn.functional.layer_norm(d(x), (w,), d(x_norm), None, eps)
+        close(out, h, BF16)
+    elif end == "plain":
+        close(out, d(x), BF16)
+
+
 # -------------------------------------------------------------- per token
 
 
