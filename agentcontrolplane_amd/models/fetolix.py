@@ -127,14 +127,14 @@ class FetolixLayer:
             at, rows = self.sections[name]
             return proj[:, at : at + rows] if rows else None
 
+        glu = None
         if self.mlp:
-            ops.clamped_glu(
-                section("glu"), self.mlp.limit, self.mlp.alpha, self.mlp.offset,
-                mixed[:, m.out_dim :],
+            glu = (
+                mixed[:, m.out_dim :], section("glu"), self.mlp.limit, self.mlp.alpha, self.mlp.offset,
             )
         m.forward(
             section("q"), section("kv"), section("gate"), batch, cache,
-            mixed[:, : m.out_dim],
+            mixed[:, : m.out_dim], glu,
         )
         if parts and len(self.w_out) == 1:
             return ops.step_linear_parts(mixed, self.w_out[0])

@@ -179,14 +179,15 @@ class LatentAttention:
     # ------------------------------------------------------------- forward
 
     def forward(self, q: torch.Tensor, kv: torch.Tensor, gate, batch: FlatBatch,
-                cache: torch.Tensor, out: torch.Tensor) -> None:
+                cache: torch.Tensor, out: torch.Tensor, glu=None) -> None:
         """q, kv, gate: the sections of the fused projection (row-strided
-        views); writes out [N, out_dim] (row-strided view)."""
+        views); writes out [N, out_dim] (row-strided view).  glu: a gated unit to do as well, as of
+        ops.latent_inputs()."""
         s, H, N = self.spec, self.heads, q.shape[0]
-        low_rank = (q, self.q_norm, s.q_rank) if s.q_rank else ()
+        low_rank = (q, self.q_norm, s.q_rank) if s.q_rank else (None, None, 0)
         cq = ops.latent_inputs(
             kv, self.kv_norm, self.eps, s.kv_rank, s.rot_dim, self.rank,
-            batch.positions, batch.slot_mapping, self.cos_sin, cache, *low_rank,
+            batch.positions, batch.slot_mapping, self.cos_sin, cache, *low_rank, glu,
         )
         if s.q_rank:
             q = ops.step_linear(cq, self.uq)

@@ -448,14 +448,15 @@ def latent_head(dim: int) -> int:
 
 
 def latent_inputs(kv, norm_w, eps: float, kv_rank: int, rot_dim: int, rank: int,
-                  positions, slot_mapping, cos_sin, cache, q=None, q_norm=None, q_rank=0):
+                  positions, slot_mapping, cos_sin, cache, q=None, q_norm=None, q_rank=0, glu=None):
     """kv [N, kv_rank + rot_dim] (row-strided): RMS-norm the latent, rotate the
     key part (interleaved pairs), scatter [latent -> rank | rotated] rows into
     cache [blocks, block, row].  With q [N, K] (low-rank query, row-strided; its
-    columns past q_rank are zero padding) returns rmsnorm(q) * q_norm."""
+    columns past q_rank are zero padding) returns rmsnorm(q) * q_norm.  With glu (out, gate_up, limit,
+    alpha, offset) does that clamped_glu() of as many rows as well."""
     return _impl(kv).latent_inputs(
         kv, norm_w, eps, kv_rank, rot_dim, rank, positions, slot_mapping, cos_sin, cache,
-        q, q_norm, q_rank,
+        q, q_norm, q_rank, glu,
     )
 
 

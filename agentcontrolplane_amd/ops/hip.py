@@ -261,11 +261,11 @@ _MAX_SPLIT = 32
 
 
 def latent_inputs(kv, norm_w, eps: float, kv_rank: int, rot_dim: int, rank: int,
-                  positions, slot_mapping, cos_sin, cache, q=None, q_norm=None, q_rank=0):
+                  positions, slot_mapping, cos_sin, cache, q=None, q_norm=None, q_rank=0, glu=None):
     cq = None if q is None else torch.empty(q.shape, dtype=q.dtype, device=q.device)
     _C.latent_inputs(
         cache, kv, norm_w, positions, slot_mapping, cos_sin, eps, kv_rank, rot_dim, rank,
-        cq, q, q_norm, q_rank,
+        cq, q, q_norm, q_rank, *(glu or (None, None, 0.0, 0.0, 0.0)),
     )
     return cq
 

@@ -237,7 +237,10 @@ def _rotate_interleaved(x, cos, sin):
 
 
 def latent_inputs(kv, norm_w, eps: float, kv_rank: int, rot_dim: int, rank: int,
-                  positions, slot_mapping, cos_sin, cache, q=None, q_norm=None, q_rank=0):
+                  positions, slot_mapping, cos_sin, cache, q=None, q_norm=None, q_rank=0, glu=None):
+    if glu is not None:
+        out, gate_up, *constants = glu
+        clamped_glu(gate_up, *constants, out)
     c = rmsnorm_rows(kv[:, :kv_rank], norm_w, eps, kv_rank)
     k_rot = _rotate_interleaved(
         kv[:, kv_rank : kv_rank + rot_dim], cos_sin[0][positions], cos_sin[1][positions]

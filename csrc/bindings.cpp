@@ -13,6 +13,7 @@
 #include "gated_delta.h"
 #include "experts.h"
 #include "grouped_attn.h"
+#include "glu_rows.h"
 #include "latent_attn.h"
 #include "residual_norm.h"
 #include "linear.h"
@@ -74,14 +75,13 @@ void launch_side_layer(const SideLayerArgs*, hipStream_t);
 void launch_side_gate(bool, float*, const float*, const void*, const void*, const int64_t*, const void*,
                       void*, int, int, int, int64_t, hipStream_t);
 void launch_add_to_residual(bool, float*, const void*, void*, int64_t, hipStream_t);
-void launch_clamped_glu(bool, void*, const void*, float, float, float, float, int, int, int64_t,
-                        int64_t, hipStream_t);
+void launch_clamped_glu(bool, const GluRows*, hipStream_t);
 void launch_gelu_gate(bool, void*, const int64_t*, const void*, int, int, int64_t,
                       hipStream_t);
 void launch_latent_inputs(bool, void*, const void*, const void*, const int64_t*,
                           const int64_t*, const float*, float, int, int, int, int, int,
                           int64_t, int64_t, void*, const void*, const void*, int, int,
-                          int64_t, hipStream_t);
+                          int64_t, const GluRows*, hipStream_t);
 void launch_head_linear(bool, void*, const void*, const void*, const void*, int, int, int,
                         int, int64_t, int, int64_t, int, int64_t, hipStream_t);
 bool launch_latent_prefill(const LatentPrefillArgs*, int, int, hipStream_t);
@@ -643,17 +643,22 @@ static void add_to_residual(torch::Tensor x, torch::Tensor y, OptTensor out) {
                          out ? out->data_ptr() : nullptr, x.numel(), cur_stream());
 }
 
-static void clamped_glu(torch::Tensor out, torch::Tensor gate_up, double limit,
-                        double alpha, double offset, double cubic) {
+static GluRows glu_rows(const torch::Tensor& out, const torch::Tensor& gate_up, double limit, double alpha,
+                        double offset, double cubic) {
   const int rows = out.size(0), inter = out.size(1);
   check_rows(out, gate_up.scalar_type(), rows, inter);
   check_rows(gate_up, gate_up.scalar_type(), rows, 2 * (int64_t)inter);
   check_aligned(out); check_aligned(gate_up);
   TORCH_CHECK(inter % 8 == 0, "padded width must be a multiple of 8");
-  if (rows == 0) return;
-  launch_clamped_glu(is_bf16(out), out.data_ptr(), gate_up.data_ptr(), (float)limit,
-                     (float)alpha, (float)offset, (float)cubic, rows, inter, gate_up.stride(0),
-                     out.stride(0), cur_stream());
+  return {out.data_ptr(), gate_up.data_ptr(), gate_up.stride(0), out.stride(0), rows, inter,
+          (float)limit, (float)alpha, (float)offset, (float)cubic};
+}
+
+static void clamped_glu(torch::Tensor out, torch::Tensor gate_up, double limit,
+                        double alpha, double offset, double cubic) {
+  const GluRows a = glu_rows(out, gate_up, limit, alpha, offset, cubic);
+  if (a.rows == 0) return;
+  launch_clamped_glu(is_bf16(out), &a, cur_stream());
 }
 
 static void gelu_gate(torch::Tensor s, torch::Tensor token_ids, torch::Tensor table,
@@ -684,7 +689,8 @@ static void latent_inputs(torch::Tensor cache, torch::Tensor kv, torch::Tensor n
                           torch::Tensor positions, torch::Tensor slots,
                           torch::Tensor cos_sin, double eps, int64_t kv_rank,
                           int64_t rot_dim, int64_t rank, OptTensor cq, OptTensor q,
-                          OptTensor q_norm, int64_t q_rank) {
+                          OptTensor q_norm, int64_t q_rank, OptTensor glu_out, OptTensor gate_up,
+                          double limit, double alpha, double offset) {
   const int n = kv.size(0);
   check_rows(kv, kv.scalar_type(), n, kv_rank + rot_dim);
   check_vec(norm_w, kv.scalar_type(), kv_rank);
@@ -703,13 +709,19 @@ static void latent_inputs(torch::Tensor cache, torch::Tensor kv, torch::Tensor n
     check_vec(*q_norm, kv.scalar_type(), k);
     TORCH_CHECK(k % 8 == 0 && q_rank > 0 && q_rank <= k);
   }
+  GluRows glu{};
+  if (glu_out) {
+    TORCH_CHECK(gate_up && gate_up->scalar_type() == kv.scalar_type(), "gated unit");
+    glu = glu_rows(*glu_out, *gate_up, limit, alpha, offset, 0.);
+    TORCH_CHECK(glu.rows == n, "gated unit");
+  }
   if (n == 0) return;
   launch_latent_inputs(is_bf16(kv), cache.data_ptr(), kv.data_ptr(), norm_w.data_ptr(),
                        positions.data_ptr<int64_t>(), slots.data_ptr<int64_t>(),
                        cos_sin.data_ptr<float>(), (float)eps, n, kv_rank, rot_dim, rank, row,
                        kv.stride(0), cos_sin.size(1), q ? cq->data_ptr() : nullptr,
                        q ? q->data_ptr() : nullptr, q ? q_norm->data_ptr() : nullptr, k,
-                       (int)q_rank, q ? q->stride(0) : 0, cur_stream());
+                       (int)q_rank, q ? q->stride(0) : 0, glu_out ? &glu : nullptr, cur_stream());
 }
 
 // [N, H, K] with dense vectors, any token and head stride

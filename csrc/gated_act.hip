@@ -15,23 +15,8 @@
 #include "side_layer.h"
 
 template <typename T, int V>
-__global__ __launch_bounds__(256) void clamped_glu_kernel(
-    T* __restrict__ out, const T* __restrict__ gate_up, const float limit,
-    const float alpha, const float offset, const float cubic, const int rows, const int inter,
-    const int64_t in_stride, const int64_t out_stride) {
-  const int per_row = inter / V;
-  const int64_t total = (int64_t)rows * per_row;
-  const int64_t step = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += step) {
-    const int64_t r = i / per_row;
-    const int c = (int)(i - r * per_row) * V;
-    float g[V], u[V];
-    load_f<V>(g, gate_up + r * in_stride + c);
-    load_f<V>(u, gate_up + r * in_stride + inter + c);
-#pragma unroll
-    for (int k = 0; k < V; ++k) g[k] = clamped_glu_f(g[k], u[k], limit, alpha, offset, cubic);
-    store_f<V>(out + r * out_stride + c, g);
-  }
+__global__ __launch_bounds__(256) void clamped_glu_kernel(const GluRows a) {
+  clamped_glu_rows<T, V>(a, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
 }
 
 DEV float gelu_tanh_f(float z) {
@@ -285,20 +270,11 @@ __global__ __launch_bounds__(256) void gelu_gate_kernel(
 
 extern "C" {
 
-void launch_clamped_glu(bool bf16, void* out, const void* gate_up, float limit,
-                        float alpha, float offset, float cubic, int rows, int inter,
-                        int64_t in_stride, int64_t out_stride, hipStream_t stream) {
-  const int v = bf16 ? 8 : 4;
-  const int64_t want = ((int64_t)rows * (inter / v) + 255) / 256;
-  const int grid = (int)(want < 4096 ? want : 4096);
+void launch_clamped_glu(bool bf16, const GluRows* a, hipStream_t stream) {
   if (bf16)
-    clamped_glu_kernel<bf16_t, 8><<<grid, 256, 0, stream>>>(
-        (bf16_t*)out, (const bf16_t*)gate_up, limit, alpha, offset, cubic, rows, inter,
-        in_stride, out_stride);
+    clamped_glu_kernel<bf16_t, 8><<<a->blocks(8, 4096), 256, 0, stream>>>(*a);
   else
-    clamped_glu_kernel<float, 4><<<grid, 256, 0, stream>>>(
-        (float*)out, (const float*)gate_up, limit, alpha, offset, cubic, rows, inter,
-        in_stride, out_stride);
+    clamped_glu_kernel<float, 4><<<a->blocks(4, 4096), 256, 0, stream>>>(*a);
 }
 
 void launch_side_gate(bool bf16, float* x_out, const float* x, const void* y, const void* gate,

@@ -3,6 +3,7 @@
 //
 // Rotations here pair dimension 2i with 2i+1; cos_sin is [2, P, rot_dim/2] fp32.
 #include "common_t.h"
+#include "gated_act.h"
 
 typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef float f32x4_v __attribute__((ext_vector_type(4)));
@@ -10,6 +11,8 @@ typedef float f32x4_v __attribute__((ext_vector_type(4)));
 // A wave per token and job.  Job 0: RMS-norm kv[:kv_rank], rotate kv[kv_rank:],
 // write the padded cache row [kv_rank -> rank | rot_dim -> row - rank] at its slot.
 // Job 1 (low-rank queries): cq = rmsnorm(q) over the first q_rank of its k columns.
+// The workgroups past these do the gated unit that reads other columns of the same product, if there is
+// one: by itself that is another launch at the cost of one (40 tokens: 4.8 us each, together 4.9).
 template <typename T, int V>
 __global__ __launch_bounds__(256) void latent_inputs_kernel(
     T* __restrict__ cache, const T* __restrict__ kv, const T* __restrict__ norm_w,
@@ -18,11 +21,18 @@ __global__ __launch_bounds__(256) void latent_inputs_kernel(
     const int kv_rank, const int rot_dim, const int rank, const int row,
     const int64_t kv_stride, const int64_t P, T* __restrict__ cq,
     const T* __restrict__ q, const T* __restrict__ q_norm, const int k,
-    const int q_rank, const int64_t q_stride) {
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int q_rank, const int64_t q_stride, const GluRows glu) {
+  const int per_job = (N + 3) / 4, jobs = q ? 2 : 1;
+  if ((int)blockIdx.x >= per_job * jobs) {
+    const int at = blockIdx.x - per_job * jobs;
+    clamped_glu_rows<T, V>(glu, (int64_t)at * 256 + threadIdx.x, (int64_t)(gridDim.x - per_job * jobs) * 256);
+    return;
+  }
+  const bool second = (int)blockIdx.x >= per_job;
+  const int n = (blockIdx.x - (second ? per_job : 0)) * 4 + (threadIdx.x >> 6);
   if (n >= N) return;
   const int lane = threadIdx.x & 63;
-  if (blockIdx.y == 1) {
+  if (second) {
     const T* src = q + n * q_stride;
     float ss = 0.f;
     for (int i = lane * V; i < k; i += 64 * V) {
@@ -175,18 +185,19 @@ void launch_latent_inputs(bool bf16, void* cache, const void* kv, const void* no
                           const float* cos_sin, float eps, int N, int kv_rank, int rot_dim,
                           int rank, int row, int64_t kv_stride, int64_t P, void* cq,
                           const void* q, const void* q_norm, int k, int q_rank,
-                          int64_t q_stride, hipStream_t stream) {
-  const dim3 grid((N + 3) / 4, q ? 2 : 1);
+                          int64_t q_stride, const GluRows* glu, hipStream_t stream) {
+  const int grid = (N + 3) / 4 * (q ? 2 : 1) + (glu ? glu->blocks(bf16 ? 8 : 4, 4096) : 0);
+  const GluRows rows = glu ? *glu : GluRows{};
   if (bf16)
     latent_inputs_kernel<bf16_t, 8><<<grid, 256, 0, stream>>>(
         (bf16_t*)cache, (const bf16_t*)kv, (const bf16_t*)norm_w, positions, slots,
         cos_sin, eps, N, kv_rank, rot_dim, rank, row, kv_stride, P, (bf16_t*)cq,
-        (const bf16_t*)q, (const bf16_t*)q_norm, k, q_rank, q_stride);
+        (const bf16_t*)q, (const bf16_t*)q_norm, k, q_rank, q_stride, rows);
   else
     latent_inputs_kernel<float, 4><<<grid, 256, 0, stream>>>(
         (float*)cache, (const float*)kv, (const float*)norm_w, positions, slots, cos_sin,
         eps, N, kv_rank, rot_dim, rank, row, kv_stride, P, (float*)cq, (const float*)q,
-        (const float*)q_norm, k, q_rank, q_stride);
+        (const float*)q_norm, k, q_rank, q_stride, rows);
 }
 
 void launch_head_linear(bool bf16, void* out, const void* x, const void* w,

@@ -162,6 +162,31 @@ def test_latent_inputs(device, dtype, kv_rank, rot_dim):
     assert (cache.view(32, row).cpu()[rest] == 7.0).all()
 
 
+@pytest.mark.parametrize("low_rank", [False, True])
+@pytest.mark.parametrize("n,inter", [(1, 8), (4, 2048), (5, 40), (2100, 5120)])
+def test_latent_inputs_with_gated_unit(device, dtype, n, inter, low_rank):
+    """The gated unit beside it: all that either does by itself, to the bit."""
+    if device == "cpu" and n > 2000:
+        pytest.skip("a range of the launch")
+    f = lambda *s, k: rand(*s, dtype=dtype, device=device, seed=k)  # noqa: E731
+    kv, w, wide = f(n, 40, k=1), f(32, k=2), f(n, 32 + 2 * inter, k=3)
+    cos_sin = build_cos_sin(9, 8, 1e4, device, exact=True)
+    pos = torch.arange(n, device=device) % 9
+    q = (wide[:, :32], f(32, k=4), 24) if low_rank else (None, None, 0)
+    got = []
+    for joint in (False, True):
+        cache = torch.zeros(n, 1, 128, dtype=dtype, device=device)
+        out = torch.zeros(n, inter + 8, dtype=dtype, device=device)
+        glu = (out[:, 8:], wide[:, 32:], 1.25, 1.702, 1.0)
+        args = (kv, w, 1e-5, 32, 8, 32, pos, torch.arange(n, device=device), cos_sin, cache, *q)
+        cq = ops.latent_inputs(*args, glu) if joint else ops.latent_inputs(*args)
+        if not joint:
+            ops.clamped_glu(glu[1], *glu[2:], glu[0])
+        got.append([t for t in (cache, out, cq) if t is not None])
+    assert got[0][0].any() and got[0][1][:, 8:].any() and not got[0][1][:, :8].any()
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("n", [1, 17, 70, 2100])
 @pytest.mark.parametrize("O,K", [(32, 32), (96, 64), (512, 128), (128, 512)])
 def test_head_linear(device, dtype, n, O, K):
