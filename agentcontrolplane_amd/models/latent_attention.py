@@ -199,11 +199,11 @@ class LatentAttention:
         if row0 < N:
             qa = torch.empty(N - row0, H, self.rank, dtype=q.dtype, device=q.device)
             ops.head_linear(q[row0:, :, : self.d], self.w_uk, qa)
-            latent = ops.latent_attention(
+            ops.latent_values(
                 qa, q[row0:, :, self.d :], self.cos_sin, s.rot_dim, cache, batch, s.scale,
                 s.window, row0, expanded, self.sink,
+                self.w_uv, out[row0:], None if gate is None else gate[row0:],
             )
-            ops.head_linear(latent, self.w_uv, out[row0:], None if gate is None else gate[row0:])
         if expanded:  # after: the rows above may include expanded chunks'
             ops.latent_expanded_prefill(
                 q, self.w_ukv, gate, self.cos_sin, s.rot_dim, cache, batch, expanded,

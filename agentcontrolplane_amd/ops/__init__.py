@@ -478,6 +478,19 @@ def latent_attention(q, q_rot, cos_sin, rot_dim: int, cache, batch, scale: float
     )
 
 
+def latent_values(q, q_rot, cos_sin, rot_dim: int, cache, batch, scale: float, window,
+                  row0: int, skip, sink, w, out, gate=None):
+    """head_linear(latent_attention(...), w, out, gate)."""
+    if q.is_cuda:
+        return _hip().latent_values(
+            q, q_rot, cos_sin, rot_dim, cache, batch, scale, window, row0, skip, sink, w, out, gate
+        )
+    latent = latent_attention(
+        q, q_rot, cos_sin, rot_dim, cache, batch, scale, window, row0, skip, sink
+    )
+    return head_linear(latent, w, out, gate)
+
+
 def can_expand(t, d: int, v: int, rot: int) -> bool:
     """Is there a kernel for expanded keys and values of these padded sizes?"""
     return t.is_cuda and _hip().can_expand(t.dtype, d, v, rot)

@@ -276,9 +276,10 @@ def head_linear(x, w, out, gate=None):
 
 
 def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefill, tiles,
-                 mg, max_keys, scale, window, mfma, sink):
+                 mg, max_keys, scale, window, mfma, sink, merge=True):
     """One launch over prefill tiles (prefill = their metadata) or decode
-    rows.  Few tiles split their keys over several workgroups."""
+    rows.  Few tiles split their keys over several workgroups; without ``merge`` their parts stay so and are
+    returned, with their sums and their number."""
     n_split = 1
     if mfma:
         keys = min(max_keys, window)
@@ -301,18 +302,45 @@ def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefi
         # rows no tile covers (skipped chunks) must merge to nothing
         new = torch.empty if prefill is None else torch.zeros
         ml = new(2 * n_split * rows, dtype=torch.float32, device=q.device)
+    # The product takes so many parts of a narrow latent one after another, longer than a launch: one sequence
+    # in 32 of them, us merged by itself and in the product: 8 heads of rank 64 12.8 and 13.3, 32 of 128 16.7
+    # and 17.6, 16 of 256 16.2 and 16.3, but of 512 22.6 and 21.3; four in 16: 11.3 and 10.7, 15.0 and 14.6
+    merge = merge or n_split > 16 and q.shape[2] <= 256
     m = prefill
     _C.latent_attn(
         out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens,
         *((m.ctx_lens, m.row_starts, m.tile_seq, m.tile_q0) if m else (None,) * 4),
-        part, ml, sink, scale, window, mg, n_split, mfma,
+        part, ml, sink, scale, window, mg, n_split, mfma, merge,
     )
+    return None if merge or n_split == 1 else (part, ml, n_split)
 
 
 def latent_attention(q, q_rot, cos_sin, rot_dim: int, cache, batch, scale: float, window,
                      row0: int = 0, skip=(), sink=None):
+    return _latent_rows(
+        q, q_rot, cos_sin, rot_dim, cache, batch, scale, window, row0, skip, sink, True
+    )[0]
+
+
+def latent_values(q, q_rot, cos_sin, rot_dim: int, cache, batch, scale: float, window,
+                  row0: int, skip, sink, w, out, gate):
+    latent, parts = _latent_rows(
+        q, q_rot, cos_sin, rot_dim, cache, batch, scale, window, row0, skip, sink, False
+    )
+    if parts is None:
+        return head_linear(latent, w, out, gate)
+    P = q.shape[0] - batch.num_decode
+    if P:
+        head_linear(latent[:P], w, out[:P], None if gate is None else gate[:P])
+    _C.merge_head_linear(out[P:], *parts, w, None if gate is None else gate[P:])
+    return out
+
+
+def _latent_rows(q, q_rot, cos_sin, rot_dim, cache, batch, scale, window, row0, skip, sink, merge):
+    """latent_attention(), and the decode rows' parts if these are not merged."""
     from . import LATENT_RANKS
 
+    parts = None
     N, H, rank = q.shape
     out = torch.empty(N, H, rank, dtype=q.dtype, device=q.device)
     window = window or _NO_WINDOW
@@ -333,12 +361,12 @@ def latent_attention(q, q_rot, cos_sin, rot_dim: int, cache, batch, scale: float
     if batch.num_decode:
         mg = 1 if H <= 16 else 2 if H <= 32 else most
         tables = batch.decode_tables_i32()
-        _latent_attn(
+        parts = _latent_attn(
             out[P:], q[P:], q_rot[P:], *common, tables, batch.decode_lens_i32(), None,
             batch.num_decode * -(-H // (16 * mg)), mg,
-            tables.shape[1] * cache.shape[1], scale, window, mfma, sink,
+            tables.shape[1] * cache.shape[1], scale, window, mfma, sink, merge,
         )
-    return out
+    return out, parts
 
 
 #: expanded keys and values built at a time

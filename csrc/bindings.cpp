@@ -87,7 +87,8 @@ void launch_head_linear(bool, void*, const void*, const void*, const void*, int,
 bool launch_latent_prefill(const LatentPrefillArgs*, int, int, hipStream_t);
 void launch_latent_gather(void*, const void*, const int*, const int*, const int*, const int*,
                           int, int, int, int, int, hipStream_t);
-bool launch_latent_attn(bool, bool, const LatentArgs*, int, int, int, int, hipStream_t);
+bool launch_latent_attn(bool, bool, const LatentArgs*, int, int, int, int, bool, hipStream_t);
+void launch_merge_head_linear(const MergedHeads*, int, hipStream_t);
 void launch_mfma_probe(float*, const void*, const void*, hipStream_t);
 }
 
@@ -758,12 +759,47 @@ static const int* opt_int(const OptTensor& t, int64_t n) {
 
 // q [tokens, H, rank] absorbed, q_rot [tokens, H, rot] -> out [tokens, H, rank].  Prefill chunks bring ctx_lens,
 // row_starts and tiles; decode (one token per table row) brings none of them.
+// out of rows that latent_attn() left in n_split parts
+static void merge_head_linear(torch::Tensor out, torch::Tensor part, torch::Tensor part_ml, int64_t n_split,
+                              torch::Tensor w, OptTensor gate) {
+  MergedHeads a{};
+  CHECK_CUDA(w); CHECK_CONT(w);
+  TORCH_CHECK(w.dim() == 3 && w.scalar_type() == at::kBFloat16, "merged heads: weights");
+  const int64_t n = out.size(0), h = w.size(0), o = w.size(1), k = w.size(2);
+  check_heads(out, at::kBFloat16, n, h);
+  TORCH_CHECK(out.size(2) == o && o % 32 == 0, "merged heads: outputs");
+  TORCH_CHECK(k == 64 || k == 128 || k == 256 || k == 384 || k == 512, "merged heads: width");
+  TORCH_CHECK(n_split >= 1 && n_split <= 64, "merged heads: parts");
+  CHECK_CUDA(part); CHECK_CONT(part); CHECK_CUDA(part_ml); CHECK_CONT(part_ml);
+  TORCH_CHECK((uintptr_t)w.data_ptr() % 16 == 0 && (uintptr_t)part.data_ptr() % 16 == 0, "merged heads: alignment");
+  TORCH_CHECK(part.scalar_type() == at::kFloat && part_ml.scalar_type() == at::kFloat &&
+              part.numel() >= n_split * n * h * k && part_ml.numel() >= 2 * n_split * n * h, "split workspace");
+  if (gate) {
+    check_rows(*gate, at::kBFloat16, n, h);
+    a.gate = gate->data_ptr();
+    a.gate_row = gate->stride(0);
+  }
+  if (n == 0) return;
+  a.out = out.data_ptr();
+  a.part = part.data_ptr<float>();
+  a.part_ml = (const float2*)part_ml.data_ptr<float>();
+  a.w = w.data_ptr();
+  a.out_row = out.stride(0);
+  a.out_head = out.stride(1);
+  a.N = n;
+  a.H = h;
+  a.O = o;
+  a.n_split = n_split;
+  launch_merge_head_linear(&a, k, cur_stream());
+}
+
+// out is left as it is where n_split > 1 and the parts are not to be merged
 static void latent_attn(torch::Tensor out, torch::Tensor q, torch::Tensor q_rot,
                         torch::Tensor cos_sin, int64_t rot_dim, torch::Tensor cache,
                         torch::Tensor tables, torch::Tensor seq_lens, OptTensor ctx_lens,
                         OptTensor row_starts, OptTensor tile_seq, OptTensor tile_r0,
                         OptTensor part, OptTensor part_ml, OptTensor sink, double scale,
-                        int64_t window, int64_t mg, int64_t n_split, bool mfma) {
+                        int64_t window, int64_t mg, int64_t n_split, bool mfma, bool merge) {
   CHECK_CUDA(q); CHECK_CONT(q); CHECK_CONT(out); CHECK_CUDA(cache); CHECK_CONT(cache);
   CHECK_CUDA(tables); CHECK_CONT(tables); CHECK_CUDA(seq_lens); CHECK_CONT(seq_lens);
   const bool bf16 = is_bf16(q);
@@ -825,7 +861,7 @@ static void latent_attn(torch::Tensor out, torch::Tensor q, torch::Tensor q_rot,
   a.n_split = (int)n_split;
   a.rows = tokens * H;
   a.scale = (float)scale;
-  TORCH_CHECK(launch_latent_attn(bf16, mfma, &a, rank, row, (int)mg, tiles, cur_stream()),
+  TORCH_CHECK(launch_latent_attn(bf16, mfma, &a, rank, row, (int)mg, tiles, merge, cur_stream()),
               "latent attention: unsupported sizes rank ", rank, " row ", row);
 }
 
@@ -1368,6 +1404,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gelu_gate", &gelu_gate);
   m.def("latent_inputs", &latent_inputs);
   m.def("head_linear", &head_linear);
+  m.def("merge_head_linear", &merge_head_linear);
   m.def("latent_attn", &latent_attn);
   m.def("latent_gather", &latent_gather);
   m.def("latent_prefill", &latent_prefill);

@@ -40,6 +40,17 @@ struct LatentPrefillArgs {
   float scale;
 };
 
+// The heads' product of rows that are still in parts (latent_proj.hip): K of w [H, O, K] is their width.
+struct MergedHeads {
+  void* out;             // [N, H, O], strides below
+  const float* part;     // [n_split, N * H, K]
+  const float2* part_ml; // [n_split, N * H]
+  const void* w;
+  const void* gate;      // [N, H], rows gate_row apart, or null
+  int64_t out_row, out_head, gate_row;
+  int N, H, O, n_split, T;
+};
+
 // Where merged rows go: row r is head r % H of token r / H.
 struct SplitOut {
   void* out;              // bf16, tokens out_stride apart

@@ -466,7 +466,7 @@ void launch_split_combine(const SplitOut* out, const float* part, const float2* 
 }
 
 bool launch_latent_attn(bool bf16, bool mfma, const LatentArgs* a, int rank, int row,
-                        int mg, int tiles, hipStream_t stream) {
+                        int mg, int tiles, bool merge, hipStream_t stream) {
   if (!mfma)
     return (bf16 ? launch_plain<bf16_t> : launch_plain<float>)(*a, rank, row, tiles, stream);
   switch (rank) {
@@ -477,7 +477,7 @@ bool launch_latent_attn(bool bf16, bool mfma, const LatentArgs* a, int rank, int
     case 512: launch_mg<8>(*a, mg, tiles, stream); break;
     default: return false;
   }
-  if (a->n_split > 1) {
+  if (a->n_split > 1 && merge) {
     const SplitOut out = {a->out, (int64_t)a->H * rank, a->H};
     launch_split_combine(&out, a->part, a->part_ml, a->rows, rank, a->n_split, stream);
   }

@@ -4,9 +4,12 @@
 // Rotations here pair dimension 2i with 2i+1; cos_sin is [2, P, rot_dim/2] fp32.
 #include "common_t.h"
 #include "gated_act.h"
+#include "latent_attn.h"
 
 typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
 typedef float f32x4_v __attribute__((ext_vector_type(4)));
+
+#define NEG -1e30f
 
 // A wave per token and job.  Job 0: RMS-norm kv[:kv_rank], rotate kv[kv_rank:],
 // write the padded cache row [kv_rank -> rank | rot_dim -> row - rank] at its slot.
@@ -154,6 +157,85 @@ __global__ __launch_bounds__(256) void head_linear_mfma_kernel(
   }
 }
 
+// out[n, h, :O] = W[h] x[n, h, :K] (* sigmoid(gate[n, h])) of rows x that are still in n_split parts (SplitOut):
+// a workgroup merges its T <= 16 tokens of one head into LDS, rounded as a merge by itself rounds them, and its 8
+// waves take 16 outputs each.  Everything is on its way from the start (a wave's first weights, the parts,
+// their sums): what is left is one latency and the reads, 128 KB of weights and T n_split 2 KB at a rank of 512.
+// Heads are neighbours in the grid, so that an XCD reads its heads' weights alone.
+// 40 tokens of 16 heads of rank 512 in 6 parts, 128 outputs: 8.0 us, before, merged (4.9) and multiplied (9.2), 14.1
+// and a gap between launches; attention and this together 40 x 3000 47.4 -> 42.9, 250 x 2000 in 2 parts
+// 116.3 -> 112.4, one of 300 keys 19.3 -> 16.5.
+template <int KS>  // K / 32
+__global__ __launch_bounds__(512) void merge_head_linear_kernel(const MergedHeads a) {
+  constexpr int K = KS * 32, BATCH = 8;
+  __shared__ bf16_t rows[16][K + 8];
+  __shared__ float weight[16][64];
+  __shared__ int live[16];
+  const int h = blockIdx.x, n0 = blockIdx.y * a.T, tokens = min(a.T, a.N - n0);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+  const int64_t n_rows = (int64_t)a.N * a.H;
+  const float* const part = a.part + ((int64_t)n0 * a.H + h) * K;
+
+  float4 v[BATCH];
+  auto load_parts = [&](int t, int k, int from) {
+#pragma unroll
+    for (int s = 0; s < BATCH; ++s)
+      v[s] = *(const float4*)(part + (min(from + s, a.n_split - 1) * n_rows + (int64_t)t * a.H) * K + k);
+  };
+  bf16x8_v w[KS];
+  auto load_weights = [&](int o) {
+    const bf16_t* src = (const bf16_t*)a.w + ((int64_t)h * a.O + min(o + c, a.O - 1)) * K + g * 8;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) w[k] = *(const bf16x8_v*)(src + k * 32);
+  };
+  const int at0 = threadIdx.x * 4;
+  load_parts(min(at0 / K, tokens - 1), at0 % K, 0);
+  load_weights(wid * 16);
+
+  for (int t = wid; t < tokens; t += 8) {
+    const float2 ml = lane < a.n_split ? a.part_ml[lane * n_rows + (int64_t)(n0 + t) * a.H + h] : float2{NEG, -1.f};
+    const int some = __popcll(__ballot(ml.y >= 0.f));
+    const float m = wave_max(ml.x);
+    const float e = ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - m) : 0.f;
+    const float l = wave_sum(e * fmaxf(ml.y, 0.f));
+    weight[t][lane] = l > 0.f ? e / l : 0.f;
+    if (lane == 0) live[t] = some;
+  }
+  __syncthreads();
+  for (int at = at0; at < 16 * K; at += 2048) {
+    const int t = at / K, k = at % K;
+    float acc[4] = {};
+    if (t < tokens) {
+      for (int from = 0; from < live[t]; from += BATCH) {
+        if (at != at0 || from) load_parts(t, k, from);
+#pragma unroll
+        for (int s = 0; s < BATCH; ++s)
+          if (from + s < live[t]) {
+            const float p = weight[t][from + s];
+            acc[0] += p * v[s].x;
+            acc[1] += p * v[s].y;
+            acc[2] += p * v[s].z;
+            acc[3] += p * v[s].w;
+          }
+      }
+    }
+    store_f<4>(&rows[t][k], acc);
+  }
+  __syncthreads();
+  const bool mine = c < tokens;
+  const int64_t n = n0 + min(c, tokens - 1);
+  const float s = a.gate ? sigmoid_f(bf2f(((const bf16_t*)a.gate)[n * a.gate_row + h])) : 1.f;
+  for (int o = wid * 16; o < a.O; o += 128) {
+    if (o != wid * 16) load_weights(o);
+    f32x4_v acc = {};
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k], *(const bf16x8_v*)&rows[c][k * 32 + g * 8], acc, 0, 0, 0);
+    const float y[4] = {acc[0] * s, acc[1] * s, acc[2] * s, acc[3] * s};
+    if (mine) store_f<4>((bf16_t*)a.out + n * a.out_row + (int64_t)h * a.out_head + o + g * 4, y);
+  }
+}
+
 // fp32 twin: a thread per output, 4 tokens per block in flight.
 __global__ __launch_bounds__(256) void head_linear_f32_kernel(
     float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w,
@@ -198,6 +280,20 @@ void launch_latent_inputs(bool bf16, void* cache, const void* kv, const void* no
         (float*)cache, (const float*)kv, (const float*)norm_w, positions, slots, cos_sin,
         eps, N, kv_rank, rot_dim, rank, row, kv_stride, P, (float*)cq, (const float*)q,
         (const float*)q_norm, k, q_rank, q_stride, rows);
+}
+
+// K one of 64 128 256 384 512, O a multiple of 32, n_split at most 64
+void launch_merge_head_linear(const MergedHeads* a, int K, hipStream_t stream) {
+  MergedHeads m = *a;
+  // tokens of a workgroup: as few as leave one to a CU, since each of them reads the head's weights
+  m.T = (int64_t)m.N * m.H <= 1024 ? 4 : (int64_t)m.N * m.H <= 2048 ? 8 : 16;
+  const dim3 grid(m.H, (m.N + m.T - 1) / m.T);
+  auto k = K == 64    ? merge_head_linear_kernel<2>
+           : K == 128 ? merge_head_linear_kernel<4>
+           : K == 256 ? merge_head_linear_kernel<8>
+           : K == 384 ? merge_head_linear_kernel<12>
+                      : merge_head_linear_kernel<16>;
+  k<<<grid, 512, 0, stream>>>(m);
 }
 
 void launch_head_linear(bool bf16, void* out, const void* x, const void* w,

@@ -282,6 +282,36 @@ def test_latent_attention(device, dtype, H, kv_rank, window, block, chunks):
         at += new
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("H,rank,O,lens,prompt", [
+    (1, 64, 32, [700], 0), (3, 128, 160, [1, 2000, 129, 900, 333], 7), (16, 512, 128, [3000, 40] * 20 + [900], 0),
+    (20, 384, 64, [4000] * 50 + [1] * 3, 30), (16, 256, 128, [1000] * 129 + [7], 0), (5, 512, 256, [6000, 2], 0),
+])
+def test_latent_values(H, rank, O, lens, prompt, gated):
+    """The heads' product of rows in parts is that of the merged rows, to the bit; beside a prompt too."""
+    device, dtype = "cuda", BF16
+    batch, _, _, pages = make_batch([(0, prompt)] * bool(prompt) + [(n - 1, 1) for n in lens], 16, device)
+    n, row = batch.num_tokens, rank + 64
+    f = lambda *s, k: rand(*s, dtype=dtype, device=device, seed=k)  # noqa: E731
+    cache, q, q_rot = f(pages, 16, row, k=1), f(n, H, rank, k=2), f(n, H, 64, k=3)
+    w, gate = f(H, O, rank, k=4), f(n, H + 8, k=5)[:, :H] if gated else None
+    args = (q, q_rot, build_cos_sin(6001, ROT, BASE, device, exact=True), ROT, cache, batch, rank ** -0.5, None, 0)
+    wide = torch.full((2, n, H * O + 8), 7.0, dtype=dtype, device=device)
+    want, got = (t[:, : H * O].view(n, H, O) for t in wide)
+    ops.head_linear(ops.latent_attention(*args), w, want, gate)
+    parts = []
+    from agentcontrolplane_amd.ops import hip
+    merge = hip._C.merge_head_linear
+    hip._C.merge_head_linear = lambda *a: (parts.append(a[3]), merge(*a))
+    try:
+        ops.latent_values(*args, (), None, w, got, gate)
+    finally:
+        hip._C.merge_head_linear = merge
+    assert len(parts) == 1 and parts[0] > 1
+    assert torch.equal(want, got) and got.isfinite().all() and (wide[:, :, H * O :] == 7.0).all()
+
+
 @pytest.mark.parametrize("where", ["first", "far", "oldest_visible", "just_hidden", "self"])
 @pytest.mark.parametrize("decode", [True, False])
 def test_standout_key(device, dtype, where, decode):
