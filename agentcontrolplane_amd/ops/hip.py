@@ -279,7 +279,7 @@ def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefi
                  mg, max_keys, scale, window, mfma, sink, merge=True):
     """One launch over prefill tiles (prefill = their metadata) or decode
     rows.  Few tiles split their keys over several workgroups; without ``merge`` their parts stay so and are
-    returned, with their sums and their number."""
+    returned, with their sums, the most that a row can have and the number that most have."""
     n_split = 1
     if mfma:
         keys = min(max_keys, window)
@@ -296,12 +296,20 @@ def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefi
         if wide and mg == 1 and 16 <= tiles <= 256 and keys >= (320 * n_split if n_split > 1 else 768):
             n_split = max(1, min(most, 512 // tiles))
     part = ml = None
+    cap = n_split
     if n_split > 1:
+        # Decode rows' parts by length, a long row's up to three times as many: us of 16 heads of rank 512 with
+        # the product behind, by as many parts a row, and so: 40 x 200 to 6000 53.1 and 44.3, 8000 beside 39 x
+        # 500 54.7 and 31.4, 100 x 500 to 3000 61.5 and 54.9, alike 40 x 2000 36.0 and 36.0, 250 x 1000 68.4
+        # and 69.2 (four times as many 36.6 and 71.1).  Not where a window makes most of them alike, 24 x 300 to
+        # 1500 by 1024 21.3 and 23.1
+        if prefill is None and tables.shape[0] <= 256 and window >= max_keys:
+            cap = max(n_split, min(most, 3 * n_split))
         rows = q.shape[0] * q.shape[1]
-        part = torch.empty(n_split * rows * q.shape[2], dtype=torch.float32, device=q.device)
+        part = torch.empty(cap * rows * q.shape[2], dtype=torch.float32, device=q.device)
         # rows no tile covers (skipped chunks) must merge to nothing
         new = torch.empty if prefill is None else torch.zeros
-        ml = new(2 * n_split * rows, dtype=torch.float32, device=q.device)
+        ml = new(2 * cap * rows, dtype=torch.float32, device=q.device)
     # The product takes so many parts of a narrow latent one after another, longer than a launch: one sequence
     # in 32 of them, us merged by itself and in the product: 8 heads of rank 64 12.8 and 13.3, 32 of 128 16.7
     # and 17.6, 16 of 256 16.2 and 16.3, but of 512 22.6 and 21.3; four in 16: 11.3 and 10.7, 15.0 and 14.6
@@ -310,9 +318,9 @@ def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefi
     _C.latent_attn(
         out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens,
         *((m.ctx_lens, m.row_starts, m.tile_seq, m.tile_q0) if m else (None,) * 4),
-        part, ml, sink, scale, window, mg, n_split, mfma, merge,
+        part, ml, sink, scale, window, mg, n_split, cap, mfma, merge,
     )
-    return None if merge or n_split == 1 else (part, ml, n_split)
+    return None if merge or n_split == 1 else (part, ml, cap, n_split)
 
 
 def latent_attention(q, q_rot, cos_sin, rot_dim: int, cache, batch, scale: float, window,

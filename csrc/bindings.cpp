@@ -761,7 +761,7 @@ static const int* opt_int(const OptTensor& t, int64_t n) {
 // row_starts and tiles; decode (one token per table row) brings none of them.
 // out of rows that latent_attn() left in n_split parts
 static void merge_head_linear(torch::Tensor out, torch::Tensor part, torch::Tensor part_ml, int64_t n_split,
-                              torch::Tensor w, OptTensor gate) {
+                              int64_t usual, torch::Tensor w, OptTensor gate) {
   MergedHeads a{};
   CHECK_CUDA(w); CHECK_CONT(w);
   TORCH_CHECK(w.dim() == 3 && w.scalar_type() == at::kBFloat16, "merged heads: weights");
@@ -769,7 +769,7 @@ static void merge_head_linear(torch::Tensor out, torch::Tensor part, torch::Tens
   check_heads(out, at::kBFloat16, n, h);
   TORCH_CHECK(out.size(2) == o && o % 32 == 0, "merged heads: outputs");
   TORCH_CHECK(k == 64 || k == 128 || k == 256 || k == 384 || k == 512, "merged heads: width");
-  TORCH_CHECK(n_split >= 1 && n_split <= 64, "merged heads: parts");
+  TORCH_CHECK(usual >= 1 && usual <= n_split && n_split <= 64, "merged heads: parts");
   CHECK_CUDA(part); CHECK_CONT(part); CHECK_CUDA(part_ml); CHECK_CONT(part_ml);
   TORCH_CHECK((uintptr_t)w.data_ptr() % 16 == 0 && (uintptr_t)part.data_ptr() % 16 == 0, "merged heads: alignment");
   TORCH_CHECK(part.scalar_type() == at::kFloat && part_ml.scalar_type() == at::kFloat &&
@@ -790,6 +790,7 @@ static void merge_head_linear(torch::Tensor out, torch::Tensor part, torch::Tens
   a.H = h;
   a.O = o;
   a.n_split = n_split;
+  a.usual = usual;
   launch_merge_head_linear(&a, k, cur_stream());
 }
 
@@ -799,7 +800,7 @@ static void latent_attn(torch::Tensor out, torch::Tensor q, torch::Tensor q_rot,
                         torch::Tensor tables, torch::Tensor seq_lens, OptTensor ctx_lens,
                         OptTensor row_starts, OptTensor tile_seq, OptTensor tile_r0,
                         OptTensor part, OptTensor part_ml, OptTensor sink, double scale,
-                        int64_t window, int64_t mg, int64_t n_split, bool mfma, bool merge) {
+                        int64_t window, int64_t mg, int64_t n_split, int64_t cap, bool mfma, bool merge) {
   CHECK_CUDA(q); CHECK_CONT(q); CHECK_CONT(out); CHECK_CUDA(cache); CHECK_CONT(cache);
   CHECK_CUDA(tables); CHECK_CONT(tables); CHECK_CUDA(seq_lens); CHECK_CONT(seq_lens);
   const bool bf16 = is_bf16(q);
@@ -834,8 +835,10 @@ static void latent_attn(torch::Tensor out, torch::Tensor q, torch::Tensor q_rot,
   if (n_split > 1) {
     TORCH_CHECK(part && part_ml && part->is_contiguous() && part_ml->is_contiguous());
     TORCH_CHECK(part->scalar_type() == at::kFloat && part_ml->scalar_type() == at::kFloat);
-    TORCH_CHECK(part->numel() >= n_split * tokens * H * rank &&
-                part_ml->numel() >= 2 * n_split * tokens * H, "split workspace");
+    TORCH_CHECK(cap >= n_split && cap <= 64 && (cap == n_split || (!tile_seq && mfma && seqs <= 256)), "parts");
+    TORCH_CHECK(part->numel() >= cap * tokens * H * rank &&
+                part_ml->numel() >= 2 * cap * tokens * H, "split workspace");
+    a.cap = (int)cap;
     a.part = part->data_ptr<float>();
     a.part_ml = (float2*)part_ml->data_ptr<float>();
   }
@@ -859,6 +862,7 @@ static void latent_attn(torch::Tensor out, torch::Tensor q, torch::Tensor q_rot,
   a.kv_block = cache.size(1);
   a.window = (int)window;
   a.n_split = (int)n_split;
+  a.seqs = seqs;
   a.rows = tokens * H;
   a.scale = (float)scale;
   TORCH_CHECK(launch_latent_attn(bf16, mfma, &a, rank, row, (int)mg, tiles, merge, cur_stream()),

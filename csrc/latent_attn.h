@@ -21,6 +21,8 @@ struct LatentArgs {
   int64_t rot_token, rot_head, positions;
   int rot_dim;
   int H, max_blocks, kv_block, window, n_split, rows;
+  int cap;                // parts of a row that part and part_ml hold; above n_split: by length (latent_attn.hip)
+  int seqs;
   float scale;
 };
 
@@ -49,6 +51,7 @@ struct MergedHeads {
   const void* gate;      // [N, H], rows gate_row apart, or null
   int64_t out_row, out_head, gate_row;
   int N, H, O, n_split, T;
+  int usual;             // parts that most rows have, from 1 up to n_split
 };
 
 // Where merged rows go: row r is head r % H of token r / H.

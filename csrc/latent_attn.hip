@@ -61,6 +61,70 @@ static DEV Tile find_tile(const LatentArgs& a, int rows_per_tile) {
   return t;
 }
 
+// Sum (or maximum) over the lanes up to this one
+template <bool MAX>
+static DEV int scan_lanes(int v) {
+  auto join = [&](int other) { v = MAX ? max(v, other) : v + other; };
+  join(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));  // row_shr
+  join(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  join(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  join(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  join(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+  join(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+  return v;
+}
+
+// A decode step's part of a sequence: tiles [index each, (index + 1) each) of its ``parts``
+struct Part {
+  int seq, index, each, parts;
+};
+
+// Parts of one size for all sequences, so that long ones have more of them and none is the launch's end alone:
+// the size with which the workgroups, n_split a sequence, are enough (each sequence has at most one part
+// that is not whole), but none smaller than 128 keys if n_split parts of the longest are not.
+// 40 x 200 to 6000 keys: the longest's 12 parts are 16 tiles of 32, these are 9: 54 us before, 44.
+template <int KT>
+static DEV Part find_part(const LatentArgs& a, int unit) {
+  const int lane = threadIdx.x & 63, per = (a.seqs + 63) / 64;  // sequences of a lane, at most 4
+  int tiles[4], sum = 0, most = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int s = lane * per + i;
+    tiles[i] = i < per && s < a.seqs ? (min(a.seq_lens[s], a.window) + KT - 1) / KT : 0;
+    sum += tiles[i];
+    most = max(most, tiles[i]);
+  }
+  const int total = __builtin_amdgcn_readlane(scan_lanes<false>(sum), 63);
+  const int longest = __builtin_amdgcn_readlane(scan_lanes<true>(most), 63);
+  auto parts_of = [](int n, int by) { return (n + by - 1) / by; };
+  const int even = parts_of(longest, a.n_split);
+  const int enough = parts_of(total, (a.n_split - 1) * a.seqs);
+  const int each = max(max(min(enough, even), parts_of(longest, a.cap)), max(min(128 / KT, even), 1));
+  int parts[4], mine = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int s = lane * per + i;
+    parts[i] = i < per && s < a.seqs ? max(1, parts_of(tiles[i], each)) : 0;
+    mine += parts[i];
+  }
+  int before = scan_lanes<false>(mine) - mine;
+  const unsigned long long here = __ballot(unit >= before && unit < before + mine);
+  if (!here) return {-1, 0, 0, 0};
+  int found = 0, index = 0, count = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (unit >= before && unit < before + parts[i]) {
+      found = lane * per + i;
+      index = unit - before;
+      count = parts[i];
+    }
+    before += parts[i];
+  }
+  const int from = __builtin_ctzll(here);
+  return {__builtin_amdgcn_readlane(found, from), __builtin_amdgcn_readlane(index, from), each,
+          __builtin_amdgcn_readlane(count, from)};
+}
+
 // KT: keys of a tile, 16 a wave for the scores
 template <int NR, int MG, int KT>
 __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(const LatentArgs a) {
@@ -77,7 +141,20 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
   int* const slots = (int*)(red + M * 4);                         // [2][KT]
   int* const pages = slots + 2 * KT;                              // [2][KT]
 
-  const Tile tl = find_tile(a, M);
+  Tile tl;
+  int split = blockIdx.y, parts = 0, each = 0;
+  if (a.cap > a.n_split) {
+    const int per_seq = (a.H + M - 1) / M, at = blockIdx.x / per_seq;
+    const Part p = find_part<KT>(a, split * a.seqs + at);
+    if (p.seq < 0) return;
+    split = p.index;
+    parts = p.parts;
+    each = p.each;
+    const int S = a.seq_lens[p.seq], r0 = (blockIdx.x - at * per_seq) * M;
+    tl = {p.seq, r0, min(M, a.H - r0), S - 1, S, p.seq};
+  } else {
+    tl = find_tile(a, M);
+  }
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
   const bf16_t* cache = (const bf16_t*)a.cache;
@@ -89,15 +166,18 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
   const int k_begin = max(0, pos_lo - a.window + 1);
   const int k_end = pos_hi + 1;
   const int n_tiles = (k_end - k_begin + KT - 1) / KT;
-  const int per_split = (n_tiles + a.n_split - 1) / a.n_split;
-  const int t_begin = min(n_tiles, (int)blockIdx.y * per_split);
+  const int per_split = parts ? each : (n_tiles + a.n_split - 1) / a.n_split;
+  const int t_begin = min(n_tiles, split * per_split);
   const int t_end = min(n_tiles, t_begin + per_split);
 
   const int64_t row0 = (int64_t)tl.token0 * a.H + tl.r0;
-  if (t_begin >= t_end) {  // an empty split; those are a row's last ones
-    for (int i = threadIdx.x; i < tl.count; i += 256)
-      a.part_ml[(int64_t)blockIdx.y * a.rows + row0 + i] = float2{NEG, -1.f};
-    return;
+  // empty splits; those are a row's last ones
+  const bool empty = t_begin >= t_end;
+  if (empty || (parts && split == 0)) {
+    const int from = empty ? split : parts, to = parts ? a.cap : split + 1;
+    for (int i = threadIdx.x; i < (to - from) * 16 * MG; i += 256)
+      if (i % M < tl.count) a.part_ml[(int64_t)(from + i / M) * a.rows + row0 + i % M] = float2{NEG, -1.f};
+    if (empty) return;
   }
 
   // B fragments of the queries: lane's row c, 8 consecutive dims per step
@@ -171,7 +251,7 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
 
   f32x4_v o[MG][NR] = {};
   // a sink is the softmax's starting state: its maximum, one term of the sum, no value
-  const bool sink = a.sink && blockIdx.y == 0;
+  const bool sink = a.sink && split == 0;
   float m_run[MG], l_run[MG];
 #pragma unroll
   for (int m = 0; m < MG; ++m) {
@@ -303,7 +383,7 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
         store_f<4>(dst + n * 16, v);
       }
     } else {
-      const int64_t at = (int64_t)blockIdx.y * a.rows + row;
+      const int64_t at = (int64_t)split * a.rows + row;
       if (wid == 0 && g == 0) a.part_ml[at] = float2{m_run[m], l};
       float* dst = a.part + at * RANK + col0;
 #pragma unroll
@@ -479,7 +559,7 @@ bool launch_latent_attn(bool bf16, bool mfma, const LatentArgs* a, int rank, int
   }
   if (a->n_split > 1 && merge) {
     const SplitOut out = {a->out, (int64_t)a->H * rank, a->H};
-    launch_split_combine(&out, a->part, a->part_ml, a->rows, rank, a->n_split, stream);
+    launch_split_combine(&out, a->part, a->part_ml, a->rows, rank, a->cap, stream);
   }
   return true;
 }

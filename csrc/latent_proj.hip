@@ -177,10 +177,10 @@ __global__ __launch_bounds__(512) void merge_head_linear_kernel(const MergedHead
   const float* const part = a.part + ((int64_t)n0 * a.H + h) * K;
 
   float4 v[BATCH];
-  auto load_parts = [&](int t, int k, int from) {
+  auto load_parts = [&](int t, int k, int from, int some) {
 #pragma unroll
     for (int s = 0; s < BATCH; ++s)
-      v[s] = *(const float4*)(part + (min(from + s, a.n_split - 1) * n_rows + (int64_t)t * a.H) * K + k);
+      v[s] = *(const float4*)(part + (min(from + s, some - 1) * n_rows + (int64_t)t * a.H) * K + k);
   };
   bf16x8_v w[KS];
   auto load_weights = [&](int o) {
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(512) void merge_head_linear_kernel(const MergedHead
     for (int k = 0; k < KS; ++k) w[k] = *(const bf16x8_v*)(src + k * 32);
   };
   const int at0 = threadIdx.x * 4;
-  load_parts(min(at0 / K, tokens - 1), at0 % K, 0);
+  load_parts(min(at0 / K, tokens - 1), at0 % K, 0, a.usual);
   load_weights(wid * 16);
 
   for (int t = wid; t < tokens; t += 8) {
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(512) void merge_head_linear_kernel(const MergedHead
     float acc[4] = {};
     if (t < tokens) {
       for (int from = 0; from < live[t]; from += BATCH) {
-        if (at != at0 || from) load_parts(t, k, from);
+        if (at != at0 || from || live[t] > a.usual) load_parts(t, k, from, live[t]);
 #pragma unroll
         for (int s = 0; s < BATCH; ++s)
           if (from + s < live[t]) {

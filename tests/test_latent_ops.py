@@ -264,7 +264,7 @@ def test_latent_attention(device, dtype, H, kv_rank, window, block, chunks):
     wide = rand(batch.num_tokens, H, 128, dtype=dtype, device=device, seed=6)
     wide[:, :, 64 + ROT :] = 0
     scale = 0.3 * kv_rank ** -0.5
-    cos_sin = build_cos_sin(2100, ROT, BASE, device, exact=True)
+    cos_sin = build_cos_sin(max(2100, max(map(sum, chunks))), ROT, BASE, device, exact=True)
     args = (cos_sin, ROT, cache, batch, scale, window)
     got = ops.latent_attention(q, wide[:, :, 64:], *args).cpu()
     part = batch.prefills[0].query_len  # rows from the second chunk on
@@ -280,6 +280,24 @@ def test_latent_attention(device, dtype, H, kv_rank, window, block, chunks):
         if at:
             close(tail[at - part : at - part + new], want, dtype)
         at += new
+
+
+# a decode step's parts by length: one long sequence, few and many of them, none whole, windows, heads of
+# several tiles, more sequences than lanes
+RAGGED = [
+    (16, 512, None, [6000] + [1, 127, 128, 129, 33, 32, 31]),
+    (16, 500, None, [150 * i + 1 for i in range(40)]),
+    (40, 128, None, [1, 2000, 3, 1999]),
+    (16, 512, 1024, [1, 700, 1024, 1025, 6000, 40]),
+    (3, 250, 300, [(37 * i) % 3000 + 1 for i in range(200)]),
+    (128, 64, None, [9, 2040]),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,kv_rank,window,lens", RAGGED)
+def test_parts_by_length(H, kv_rank, window, lens):
+    test_latent_attention("cuda", BF16, H, kv_rank, window, 16, [(0, 2)] + [(n - 1, 1) for n in lens])
 
 
 @pytest.mark.gpu
