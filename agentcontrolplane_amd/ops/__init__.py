@@ -405,8 +405,15 @@ def step_linear_parts(x, w):
 
 
 def side_layer_fits(x, gate, *weights) -> bool:
-    """Whether side_layer() takes this residual, this side gate and these other weights."""
-    return x.is_cuda and _hip().side_layer_fits(x, gate, *weights)
+    """Whether side_layer() takes this residual, this side gate and these other weights.  Its product is
+    the library's, as of linear(), where autograd records it or others follow it."""
+    return (
+        x.is_cuda
+        and all(map(_whole, (x, gate, *weights)))
+        and not _followed()
+        and not _recorded(x, gate, *weights)
+        and _hip().side_layer_fits(x, gate, *weights)
+    )
 
 
 def side_layer(x, y, gate, token_ids, table, offset: int, proj, eps: float, y_norm, x_norm, out):

@@ -126,6 +126,31 @@ def test_side_layer(n, w, dim, parts, end):
         close(out, d(x), BF16)
 
 
+@pytest.mark.gpu
+def test_side_layer_leaves_products_that_are_followed():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Follow(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    f = lambda *s: torch.zeros(*s, dtype=BF16, device="cuda")  # noqa: E731
+    x, gate, proj = f(4, 64).float(), f(16, 64), f(64, 16)
+    assert ops.side_layer_fits(x, gate, proj, f(64))
+    with Follow():
+        assert not ops.side_layer_fits(x, gate, proj)
+    with torch.autocast("cuda"):
+        assert not ops.side_layer_fits(x, gate, proj)
+    assert not ops.side_layer_fits(x, gate, torch.nn.Parameter(proj))
+    with torch.no_grad():
+        assert ops.side_layer_fits(x, gate, torch.nn.Parameter(proj))
+    for other in (x[:0], f(513, 64).float(), f(4, 8200).float()):
+        assert not ops.side_layer_fits(other, f(16, other.shape[1]), proj)
+    assert not ops.side_layer_fits(x, gate.float(), proj)
+    assert not ops.side_layer_fits(x, f(136, 64), proj) and not ops.side_layer_fits(x, f(12, 64), proj)
+    assert not ops.side_layer_fits(f(4, 4096).float(), f(64, 4096))  # too much for one workgroup
+
+
 # -------------------------------------------------------------- per token
 
 
