@@ -631,16 +631,28 @@ def _scan_columns(prefills, columns: int) -> int:
 
 def _scan_in_chunks(prefills, H: int, D: int, V: int, dtype) -> int:
     """16s of columns a workgroup of the recurrence by chunks of 16 tokens, 0: token by token.  By
-    chunks, heads of 128 key channels from 49 tokens on: a launch more, a shorter chain.  All launches of a layer
-    with 16 heads of 128 x 128, us, token by token and by chunks: 17 tokens 33, 36; 33 36, 38; 64 42, 39; 256
-    78, 54; 8000 1444, 631; 9 x 17 45, 51; 12 x 64 70, 66; 24 x 300 381, 320.  In fp32, where it would be
-    1.05 to 1.2 times as far from 64 bits (1.8e-7), token by token.  16 columns a workgroup are the shorter chain,
-    32 less work beside the longest sequence's: 760 to 2140 330, 380 (3.2 times the longest one's
-    tokens); 4 x 400 103, 99; 8 x 1000 419, 340; with 32 heads 3 x 600 184, 180; 8000 795, 948."""
+    chunks, heads of 128 key channels: a launch more, a shorter chain, but whole chunks of work for tokens past
+    the end of a portion.  So from 49 tokens on, and where all portions' chunks are at most a third more
+    work than their tokens or that is little beside the longest one's chain; and portions have 16 tokens on
+    average, which bounds the workspace.  All launches of a layer with 16 heads of 128 x 128, us, token by
+    token and by chunks: 17 tokens 28, 32; 33 31, 33; 64 36, 34; 12 x 64 69, 62; 20 x 49 84, 80; 24 x 300 387, 311;
+    8000 1444, 631; a portion of 49 beside 8 of 17 47, 48, beside 40 of 17 91, 99, beside 40 of 1 74, 78; 600 beside
+    200 x 20 354, 372; 300 beside 40 x 17 127, 113; 1000 beside 100 x 17 240, 197.  Of 320 steps of 1 to 260
+    portions and 8 to 32 heads 4 take more than 2% longer than token by token, at most 3 us; where the longest portion
+    alone decided 25 did, up to 42%.  In fp32 token by token: results of keys that are alike are further from 64 bits
+    by chunks.
+    16 columns a workgroup are the shorter chain, 32 less work beside the longest sequence's, of which a short
+    portion has more than its tokens: 760 to 2140 330, 380 (3.2 times the longest one's chunks); 4 x 400 103,
+    99; 8 x 1000 419, 340; 1000 beside 100 x 17 231, 197; with 32 heads 3 x 600 184, 180; 8000 795, 948."""
     lens = [m.query_len for m in prefills]
-    if dtype != torch.bfloat16 or D != 128 or V % 16 or max(lens) <= 48:
+    tokens, longest = sum(lens), max(lens)
+    if dtype != torch.bfloat16 or D != 128 or V % 16 or longest <= 48 or 16 * len(lens) > tokens:
         return 0
-    return 2 if V % 32 == 0 and sum(lens) * H * V > 4 * 2048 * max(lens) else 1
+    chunks = sum(-(-n // 16) for n in lens)
+    if 48 * chunks > 4 * tokens + 3 * longest:
+        return 0
+    beside = (chunks + len(lens)) * H * V > 4 * 2048 * (-(-longest // 16) + 1)
+    return 2 if V % 32 == 0 and beside else 1
 
 
 def gated_delta(qkv, conv, b, z, A_log, dt_bias, gate, norm, eps, unit_eps, kv_heads,
