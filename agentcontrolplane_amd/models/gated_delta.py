@@ -148,6 +148,10 @@ class GatedDelta:
         s = self.spec
         return 4 * self.heads * s.dim * s.vdim + s.conv * self.channels * itemsize
 
+    def step_bytes(self, tokens: int, dtype) -> int:
+        """Workspace of a step of so many prompt tokens."""
+        return ops.gated_delta_bytes(tokens, self.heads, self.spec.dim, self.spec.vdim, dtype)
+
     # ------------------------------------------------------------- forward
 
     def mix(self, h: torch.Tensor, batch: FlatBatch, state: Tuple[torch.Tensor, torch.Tensor]):

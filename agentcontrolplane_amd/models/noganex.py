@@ -287,8 +287,11 @@ class NoganexForCausalLM:
                 for t in store]
 
     def step_bytes(self, tokens: int) -> int:
-        """What a step of so many tokens holds beyond a dense layer's activations."""
-        return max((x.experts.step_bytes(tokens) for x in self.layers if x.experts), default=0)
+        """What a step of so many tokens holds beyond a dense layer's activations, in the layer that holds the
+        most: experts' rows or a recurrence's workspace, of which a layer has one after the other."""
+        held = [x.experts.step_bytes(tokens) for x in self.layers if x.experts]
+        held += [x.mixer.step_bytes(tokens, self.dtype) for x in self.layers if x.recurrent]
+        return max(held, default=0)
 
     # -------------------------------------------------------------- forward
 

@@ -232,9 +232,10 @@ class TezinexForCausalLM:
 
     def step_bytes(self, tokens: int) -> int:
         """What a step of so many tokens holds beyond a layer's activations: the
-        depth states."""
+        depth states and a recurrent layer's workspace."""
         planes = len(self.layers) + 1 + ops.DEPTH_AHEAD if self.cfg.depth_average else 0
-        return 4 * planes * tokens * self.cfg.hidden_size
+        recurrent = [x.mixer.step_bytes(tokens, self.dtype) for x in self.layers if x.recurrent]
+        return 4 * planes * tokens * self.cfg.hidden_size + max(recurrent, default=0)
 
     # -------------------------------------------------------------- forward
 

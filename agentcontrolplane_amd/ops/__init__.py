@@ -582,6 +582,12 @@ def moe_experts(h, gate_up, down, ids, glu):
 # ----------------------------------------------------------------- delta rule
 
 
+def gated_delta_bytes(tokens: int, H: int, D: int, V: int, dtype) -> int:
+    """What gated_delta() holds on the GPU for a step of so many prompt tokens, beyond what grows with a layer's
+    activations."""
+    return _hip().gated_delta_bytes(tokens, H, D, V, dtype)
+
+
 def gated_delta(qkv, conv, b, z, A_log, dt_bias, gate, norm, eps: float, unit_eps: float,
                 kv_heads: int, state, conv_state, batch, gate_silu: bool = False):
     """Gated delta rule over a FlatBatch's rows, each sequence from the state in its

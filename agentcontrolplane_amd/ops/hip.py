@@ -655,6 +655,14 @@ def _scan_in_chunks(prefills, H: int, D: int, V: int, dtype) -> int:
     return 2 if V % 32 == 0 and beside else 1
 
 
+def gated_delta_bytes(tokens: int, H: int, D: int, V: int, dtype) -> int:
+    """The most that the chunks of a step of so many prompt tokens take: _scan_in_chunks() lets through no more
+    portions than 16s of tokens."""
+    if dtype != torch.bfloat16 or D != 128 or V % 16:
+        return 0
+    return 4 * 2 * (tokens // 16) * H * _C.DELTA_CHUNK_FLOATS
+
+
 def gated_delta(qkv, conv, b, z, A_log, dt_bias, gate, norm, eps, unit_eps, kv_heads,
                 state, conv_state, batch, gate_silu=False):
     H, D, V = state.shape[1:]

@@ -1,9 +1,14 @@
 """The gated delta rule of a prompt by chunks of 16 tokens (csrc/delta_chunks.hip) against double
 precision and against the recurrence token by token, and which prompts take it."""
+import random
+
 import pytest
 import torch
 
+from agentcontrolplane_amd import ops
 from agentcontrolplane_amd.engine.batch import SeqMeta
+from agentcontrolplane_amd.engine.config import PRESETS, EngineConfig
+from agentcontrolplane_amd.models import create_model
 from agentcontrolplane_amd.ops import hip
 from op_helpers import BF16, close
 from test_noganex_ops import HeadDeltaCase
@@ -32,6 +37,29 @@ def test_which_prompts_go_by_chunks(lens, H, D, V, dtype, want):
 def test_chunks_go_by_all_portions(lens, H, want):
     metas = [SeqMeta(i, n, n, 0, [0], True, i) for i, n in enumerate(lens)]
     assert hip._scan_in_chunks(metas, H, 128, 128, BF16) == want
+
+
+@pytest.mark.parametrize("tokens", [512, 16384])
+def test_budget_holds_the_chunks(tokens):
+    """What a step's chunks take is in what the models tell the engine to leave of the GPU's memory."""
+    rng, most = random.Random(tokens), 0
+    for _ in range(400):
+        lens, top, left = [], rng.randint(1, 3000), tokens
+        while left:
+            lens.append(min(left, rng.randint(1, top)))
+            left -= lens[-1]
+        metas = [SeqMeta(i, n, n, 0, [0], True, i) for i, n in enumerate(lens)]
+        if hip._scan_in_chunks(metas, 32, 128, 128, BF16):
+            most = max(most, 4 * (tokens // 16 + len(lens)) * 32 * hip._C.DELTA_CHUNK_FLOATS)
+    held = ops.gated_delta_bytes(tokens, 32, 128, 128, BF16)
+    assert 0 < most <= held and not ops.gated_delta_bytes(tokens, 32, 128, 128, torch.float32)
+    for name in ("tezinex-8b", "noganex-8b"):
+        config = EngineConfig(model=name, device="cpu")
+        model = create_model(PRESETS[name], config, torch.device("cpu"))
+        mixers = [x.mixer for x in model.layers if x.recurrent]
+        assert mixers and model.dtype == BF16
+        want = ops.gated_delta_bytes(tokens, mixers[0].heads, mixers[0].spec.dim, mixers[0].spec.vdim, BF16)
+        assert model.step_bytes(tokens) >= want > 0
 
 
 @pytest.mark.gpu
