@@ -56,6 +56,8 @@ def test_budget_holds_the_chunks(tokens):
     for name in ("tezinex-8b", "noganex-8b"):
         config = EngineConfig(model=name, device="cpu")
         model = create_model(PRESETS[name], config, torch.device("cpu"))
+        for layer in model.layers:
+            layer.experts = None  # whose part depends on loaded weights
         mixers = [x.mixer for x in model.layers if x.recurrent]
         assert mixers and model.dtype == BF16
         want = ops.gated_delta_bytes(tokens, mixers[0].heads, mixers[0].spec.dim, mixers[0].spec.vdim, BF16)
