@@ -124,13 +124,16 @@ static DEV float max_with(float v) {
 // Or few blocks into pieces of one sequence each, where that leaves no workgroup with much more than its share:
 // parts have starts and ends, 4 x 300 keys 16.0 us by ranges and 11.8 by pieces, 64 x 512 35.4 and 32.
 //
-// Without a.ranges always pieces, in two rounds of half of the size where one round is uneven: the kernel with
-// several parts is 0.5 to 1 us slower for one, so that few sequences go without (RANGES_FROM), and for 8 query
-// heads a workgroup it has not the registers.
+// Without a.ranges always pieces: of one size where they are all resident at once, or sequences are no longer than
+// that, else in about two rounds, with a last piece of under a quarter shared by the sequence's others unless they
+// are short (of 12 blocks 20 x 130 to 3900 keys 53.7 us shared and 52.0 not).  Without that sharing 64 query heads of
+// 8 key heads, 30 x 300 to 4000 keys, 76.6 us instead of 73.2, 100 x 700 to 1300 107.2 and 104.5; 128 query
+// heads, 20 x 130 to 3900 80.0 and 75.2.  The kernel with several parts is 0.5 to 1 us slower for one, so that few
+// sequences go without (RANGES_FROM), and for 8 query heads a workgroup it has not the registers.
 struct Cut {
   bool aligned;  // pieces of sequences
   int count;     // ranges of a workgroup
-  int each;      // blocks of a range, at most of a piece
+  int each;      // blocks of a range, at most of a piece of the sequence
 };
 
 // Finds the cut and the sequence ``want``, or the one with the first block of workgroup ``item`` of a
@@ -151,21 +154,30 @@ static DEV Stretch find_range(const GroupedArgs& a, int want, int item, Cut& cut
     longest = max(longest, n);
   }
   total = __builtin_amdgcn_readlane(wave_scan(total), 63);
-  const int share = quotient(total + a.pieces - 1, a.pieces), spare = a.pieces - a.seqs;
-  int few = 0;
+  const int spare = a.pieces - a.seqs;
+  const bool one_round = a.seqs <= 64 || spare >= 0;  // that they may fit in it
+  const int share = a.ranges || one_round ? quotient(total + a.pieces - 1, a.pieces) : 0;
+  int few = 0, few_upto = 0;
+  int two_rounds = 0;  // blocks of a piece of two rounds
+  bool known = false;
   cut.aligned = false;
   cut.count = 1;
   cut.each = max(4, share);
   if (!a.ranges || (share <= 32 && spare >= 0)) {
     const int even = share + 3 & ~3, most = share + share / 4 + 4;
-    few = quotient(mine0 + even - 1, even);
     cut.aligned = true;
-    if (a.seqs <= 64 && __builtin_amdgcn_readlane(wave_scan(few), 63) <= a.pieces) {
+    if (a.seqs <= 64) {
+      few = quotient(mine0 + even - 1, even);
+      few_upto = wave_scan(few);
+      known = __builtin_amdgcn_readlane(few_upto, 63) <= a.pieces;
+    }
+    if (known) {
       cut.each = even;
     } else if (spare >= 0 && !__any(longest > most)) {  // whole sequences
       cut.each = most;
-    } else if (!a.ranges) {  // at most 2 a.pieces and one for every sequence
-      cut.each = max(4, (share + 7) / 8 * 4);
+    } else if (!a.ranges) {  // at most 2 a.pieces and one for every sequence; long parts are too uneven
+      const int half = max(1, quotient(total + 4 * a.pieces - 1, 4 * a.pieces));
+      two_rounds = 4 * (__any(longest > 4 * half) ? max(min(half, 3), (half + 1) / 2) : half);
     } else {
       const int each = spare > 0 ? quotient(total + spare - 1, spare) : most + 1;
       cut.aligned = each <= most;
@@ -176,19 +188,32 @@ static DEV Stretch find_range(const GroupedArgs& a, int want, int item, Cut& cut
     cut.each = (share + 1) / 2;
   }
   const int first = cut.aligned ? item : item * cut.count * cut.each;
-  const bool known = cut.aligned && a.seqs <= 64 && cut.each == (share + 3 & ~3);
+  const int spared = two_rounds - (two_rounds < 16 ? 0 : two_rounds / 4) - 1;
   Stretch x = {-1, 0, 0, 0};
   int before = 0;
   for (int s = 0; s < a.seqs; s += 64) {
     const int len = s ? len_of(s + lane) : len0, n = s ? blocks_of(s + lane, len) : mine0;
-    const int mine = known ? few : cut.aligned ? quotient(n + cut.each - 1, cut.each) : n;
-    const int upto = before + wave_scan(mine);  // blocks or pieces up to this lane's
+    int mine = n, each = cut.each;
+    if (known) {
+      mine = few;
+    } else if (two_rounds) {
+      mine = max(1, quotient(n + spared, each = two_rounds));
+      if (mine * each < n) {
+        each = 4 * quotient(n + 4 * mine - 1, 4 * mine);
+        mine = quotient(n + each - 1, each);
+      }
+      if (s + lane >= a.seqs) mine = 0;
+    } else if (cut.aligned) {
+      mine = quotient(n + each - 1, each);
+    }
+    const int upto = known ? few_upto : before + wave_scan(mine);  // blocks or pieces up to this lane's
     const uint64_t hit = __ballot(want >= 0 ? s + lane == want : first < upto);
     if (hit) {
       const int at = __builtin_ctzll(hit);
       x.seq = s + at;
       x.len = __builtin_amdgcn_readlane(len, at);
       x.n = __builtin_amdgcn_readlane(mine, at);
+      cut.each = __builtin_amdgcn_readlane(each, at);
       x.before = __builtin_amdgcn_readlane(upto, at) - x.n;
       break;
     }

@@ -1,5 +1,5 @@
-"""The arithmetic by which a decode step's keys are cut into pieces (csrc/grouped_attn.hip,
-find_pieces): its workspace has pieces + sequences rows."""
+"""The arithmetic by which a decode step's keys are cut into pieces of about two rounds of workgroups
+(csrc/grouped_attn.hip, find_range without ranges): at most pieces + sequences of them."""
 import numpy as np
 import pytest
 
@@ -37,7 +37,7 @@ def cut(blocks, pieces):
     size = 4 * (max(min(half, 3), (half + 1) // 2) if max(blocks) > 4 * half else half)
     out = []
     for n in blocks:
-        k, each = max(1, (n + size - (0 if size < 12 else size // 4) - 1) // size), size
+        k, each = max(1, (n + size - (0 if size < 16 else size // 4) - 1) // size), size
         if k * size < n:
             each = 4 * -(-n // (4 * k))
             k = -(-n // each)
