@@ -299,10 +299,10 @@ def _latent_attn(out, q, q_rot, cos_sin, rot_dim, cache, tables, seq_lens, prefi
     cap = n_split
     if n_split > 1:
         # Decode rows' parts by length, a long row's up to three times as many: us of 16 heads of rank 512 with
-        # the product behind, by as many parts a row, and so: 40 x 200 to 6000 53.1 and 44.3, 8000 beside 39 x
-        # 500 54.7 and 31.4, 100 x 500 to 3000 61.5 and 54.9, alike 40 x 2000 36.0 and 36.0, 250 x 1000 68.4
-        # and 69.2 (four times as many 36.6 and 71.1).  Not where a window makes most of them alike, 24 x 300 to
-        # 1500 by 1024 21.3 and 23.1
+        # the product behind, by as many parts a row, and so: 40 x 200 to 6000 51.0 and 44.0, 8000 beside 39 x
+        # 500 53.6 and 30.8, 100 x 500 to 3000 60.4 and 52.4, 4000 beside 249 x 800 131 and 68; alike 40 x 2000
+        # 35.9 and 34.3, 250 x 1000 66.6 and 66.9, 130 x 1000 46.6 and 48.4, as every workgroup reads all lengths.
+        # Not where a window makes most of them alike, 24 x 300 to 1500 by 1024 21.3 and 23.1
         if prefill is None and tables.shape[0] <= 256 and window >= max_keys:
             cap = max(n_split, min(most, 3 * n_split))
         rows = q.shape[0] * q.shape[1]

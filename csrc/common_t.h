@@ -34,3 +34,14 @@ DEV void store_f(T* p, const float* src) {
 }
 
 DEV float sigmoid_f(float x) { return 1.f / (1.f + __expf(-x)); }
+
+// n / d of whole numbers, n >= 0, d > 0: as good as the general division at a third of its length
+DEV int quotient(int n, int d) {
+  const float by = __builtin_amdgcn_rcpf((float)d);
+  int q = (int)((float)n * by), rest = n - q * d;
+  const int more = (int)((float)rest * by);  // what 24 bits were short of
+  q += more;
+  rest -= more * d;
+  q += rest >= d;
+  return q - (rest < 0);
+}

@@ -81,17 +81,6 @@ static DEV int wave_scan(int v) {
   return v;
 }
 
-// n / d of whole numbers, n >= 0, d > 0: as good as the general division at a third of its length
-static DEV int quotient(int n, int d) {
-  const float by = __builtin_amdgcn_rcpf((float)d);
-  int q = (int)((float)n * by), rest = n - q * d;
-  const int more = (int)((float)rest * by);  // what 24 bits were short of
-  q += more;
-  rest -= more * d;
-  q += rest >= d;
-  return q - (rest < 0);
-}
-
 // a value and the one of lane ^ 16 or lane ^ 32
 template <int LANES>
 static DEV float2 with_lane(float v) {

@@ -22,6 +22,8 @@
 // Keys past a sequence's end are clamped to its last key and masked; split-K
 // partials are merged by split_combine_kernel.  The grid depends on host
 // values only (capture-safe); lengths are read on the device.
+#include <type_traits>
+
 #include "common_t.h"
 #include "latent_attn.h"
 #include "launch.h"
@@ -76,57 +78,68 @@ static DEV int scan_lanes(int v) {
 
 // A decode step's part of a sequence: tiles [index each, (index + 1) each) of its ``parts``
 struct Part {
-  int seq, index, each, parts;
+  int seq, len, index, each, parts;
 };
 
 // Parts of one size for all sequences, so that long ones have more of them and none is the launch's end alone:
 // the size with which the workgroups, n_split a sequence, are enough (each sequence has at most one part
 // that is not whole), but none smaller than 128 keys if n_split parts of the longest are not.
-// 40 x 200 to 6000 keys: the longest's 12 parts are 16 tiles of 32, these are 9: 54 us before, 44.
+// Every workgroup begins with this, so that its length counts (quotient()).
 template <int KT>
 static DEV Part find_part(const LatentArgs& a, int unit) {
   const int lane = threadIdx.x & 63, per = (a.seqs + 63) / 64;  // sequences of a lane, at most 4
-  int tiles[4], sum = 0, most = 0;
+  int len[4] = {}, tiles[4] = {}, sum = 0, most = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
+    if (i >= per) break;
     const int s = lane * per + i;
-    tiles[i] = i < per && s < a.seqs ? (min(a.seq_lens[s], a.window) + KT - 1) / KT : 0;
+    len[i] = s < a.seqs ? a.seq_lens[s] : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i >= per) break;
+    tiles[i] = (min(len[i], a.window) + KT - 1) / KT;
     sum += tiles[i];
     most = max(most, tiles[i]);
   }
   const int total = __builtin_amdgcn_readlane(scan_lanes<false>(sum), 63);
   const int longest = __builtin_amdgcn_readlane(scan_lanes<true>(most), 63);
-  auto parts_of = [](int n, int by) { return (n + by - 1) / by; };
+  auto parts_of = [](int n, int by) { return quotient(n + by - 1, by); };
   const int even = parts_of(longest, a.n_split);
   const int enough = parts_of(total, (a.n_split - 1) * a.seqs);
   const int each = max(max(min(enough, even), parts_of(longest, a.cap)), max(min(128 / KT, even), 1));
-  int parts[4], mine = 0;
+  int parts[4] = {}, mine = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int s = lane * per + i;
-    parts[i] = i < per && s < a.seqs ? max(1, parts_of(tiles[i], each)) : 0;
+    if (i >= per) break;
+    parts[i] = lane * per + i < a.seqs ? max(1, parts_of(tiles[i], each)) : 0;
     mine += parts[i];
   }
   int before = scan_lanes<false>(mine) - mine;
   const unsigned long long here = __ballot(unit >= before && unit < before + mine);
-  if (!here) return {-1, 0, 0, 0};
-  int found = 0, index = 0, count = 0;
+  if (!here) return {-1, 0, 0, 0, 0};
+  int found = 0, index = 0, count = 0, length = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
+    if (i >= per) break;
     if (unit >= before && unit < before + parts[i]) {
       found = lane * per + i;
+      length = len[i];
       index = unit - before;
       count = parts[i];
     }
     before += parts[i];
   }
   const int from = __builtin_ctzll(here);
-  return {__builtin_amdgcn_readlane(found, from), __builtin_amdgcn_readlane(index, from), each,
-          __builtin_amdgcn_readlane(count, from)};
+  return {__builtin_amdgcn_readlane(found, from), __builtin_amdgcn_readlane(length, from),
+          __builtin_amdgcn_readlane(index, from), each, __builtin_amdgcn_readlane(count, from)};
 }
 
-// KT: keys of a tile, 16 a wave for the scores
-template <int NR, int MG, int KT>
+// KT: keys of a tile, 16 a wave for the scores.  LENGTHS: a decode step's parts by the sequences' lengths (a.cap >
+// a.n_split).  16 heads of rank 512, this kernel alone, us by n_split parts a sequence and by lengths: 40 x 200 to 6000
+// keys 43.9 and 33.7, alike 130 x 1000 35.5 and 36.9, 250 x 1000 55.0 and 56.4, of which find_part() is the
+// difference; with general divisions in it and for the rows, and with empty parts written first, 34.5, 37.4 and 56.8.
+template <int NR, int MG, int KT, bool LENGTHS>
 __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(const LatentArgs a) {
   constexpr int RANK = 64 * NR;
   constexpr int PPAD = KT + 8;             // probability row in LDS, bf16 elements
@@ -142,42 +155,42 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
   int* const pages = slots + 2 * KT;                              // [2][KT]
 
   Tile tl;
-  int split = blockIdx.y, parts = 0, each = 0;
-  if (a.cap > a.n_split) {
+  Part part = {0, 0, (int)blockIdx.y, 0, 0};
+  if constexpr (LENGTHS) {
     const int per_seq = (a.H + M - 1) / M, at = blockIdx.x / per_seq;
-    const Part p = find_part<KT>(a, split * a.seqs + at);
-    if (p.seq < 0) return;
-    split = p.index;
-    parts = p.parts;
-    each = p.each;
-    const int S = a.seq_lens[p.seq], r0 = (blockIdx.x - at * per_seq) * M;
-    tl = {p.seq, r0, min(M, a.H - r0), S - 1, S, p.seq};
+    part = find_part<KT>(a, part.index * a.seqs + at);
+    if (part.seq < 0) return;
+    const int r0 = (blockIdx.x - at * per_seq) * M;
+    tl = {part.seq, r0, min(M, a.H - r0), part.len - 1, part.len, part.seq};
   } else {
     tl = find_tile(a, M);
   }
+  const int split = part.index;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
   const bf16_t* cache = (const bf16_t*)a.cache;
   const int* table = a.tables + (int64_t)tl.seq * a.max_blocks;
 
   // keys any row of the tile sees
-  const int pos_lo = tl.ctx + tl.r0 / a.H;
-  const int pos_hi = tl.ctx + (tl.r0 + tl.count - 1) / a.H;
+  auto token_of = [&](int r) { return LENGTHS ? 0 : r / a.H; };  // of the tile's sequence
+  const int pos_lo = tl.ctx + token_of(tl.r0);
+  const int pos_hi = tl.ctx + token_of(tl.r0 + tl.count - 1);
   const int k_begin = max(0, pos_lo - a.window + 1);
   const int k_end = pos_hi + 1;
   const int n_tiles = (k_end - k_begin + KT - 1) / KT;
-  const int per_split = parts ? each : (n_tiles + a.n_split - 1) / a.n_split;
+  const int per_split = LENGTHS ? part.each : (n_tiles + a.n_split - 1) / a.n_split;
   const int t_begin = min(n_tiles, split * per_split);
   const int t_end = min(n_tiles, t_begin + per_split);
 
   const int64_t row0 = (int64_t)tl.token0 * a.H + tl.r0;
   // empty splits; those are a row's last ones
-  const bool empty = t_begin >= t_end;
-  if (empty || (parts && split == 0)) {
-    const int from = empty ? split : parts, to = parts ? a.cap : split + 1;
-    for (int i = threadIdx.x; i < (to - from) * 16 * MG; i += 256)
+  auto no_parts = [&](int from, int to) {
+    for (int i = threadIdx.x; i < (to - from) * M; i += 256)
       if (i % M < tl.count) a.part_ml[(int64_t)(from + i / M) * a.rows + row0 + i % M] = float2{NEG, -1.f};
-    if (empty) return;
+  };
+  if (t_begin >= t_end) {
+    no_parts(split, LENGTHS ? a.cap : split + 1);
+    return;
   }
 
   // B fragments of the queries: lane's row c, 8 consecutive dims per step
@@ -187,14 +200,14 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
   for (int m = 0; m < MG; ++m) {
     const int r = m * 16 + c;
     const bool live = r < tl.count;
-    qpos[m] = live ? tl.ctx + (tl.r0 + r) / a.H : -1;  // -1 sees no key
+    qpos[m] = live ? tl.ctx + token_of(tl.r0 + r) : -1;  // -1 sees no key
     const int64_t row = row0 + (live ? r : 0);
+    const int64_t token = LENGTHS ? tl.token0 : row / a.H;
     const bf16_t* qr = (const bf16_t*)a.q + row * RANK + g * 8;
 #pragma unroll
     for (int s = 0; s < RANK / 32; ++s) qf[m][s] = *(const bf16x8_v*)(qr + s * 32);
     // the rest is rotated on the way in: 4 pairs a lane and step
-    const bf16_t* rr = (const bf16_t*)a.q_rot + row / a.H * a.rot_token +
-                       row % a.H * a.rot_head + g * 8;
+    const bf16_t* rr = (const bf16_t*)a.q_rot + token * a.rot_token + (row - token * a.H) * a.rot_head + g * 8;
     const int pairs = a.rot_dim >> 1;
     const float* ct = a.cos_sin + (int64_t)max(qpos[m], 0) * pairs;
     const float* st = ct + a.positions * pairs;
@@ -390,6 +403,7 @@ __global__ __launch_bounds__(256, KT == 32 ? 2 : 1) void latent_attn_kernel(cons
       for (int n = 0; n < NR; ++n) *(f32x4_v*)(dst + n * 16) = o[m][n];
     }
   }
+  if (LENGTHS && split == 0) no_parts(part.parts, a.cap);  // no load waits for it here
 }
 
 // Merge the splits (at most 64) of one row.
@@ -496,8 +510,15 @@ static void launch_tiles(const LatentArgs& a, int tiles, hipStream_t stream) {
   constexpr int M = 16 * MG;
   constexpr int bytes = 2 * KT * (64 * NR + ROT) * 2 + M * (KT + 8) * 2 + M * 16 + 4 * KT * 4;
   static_assert(bytes <= 160 * 1024, "LDS");
-  allow_lds<latent_attn_kernel<NR, MG, KT>>(bytes);
-  latent_attn_kernel<NR, MG, KT><<<dim3(tiles, a.n_split), 256, bytes, stream>>>(a);
+  auto launch = [&](auto lengths) {
+    constexpr bool LENGTHS = decltype(lengths)::value;
+    allow_lds<latent_attn_kernel<NR, MG, KT, LENGTHS>>(bytes);
+    latent_attn_kernel<NR, MG, KT, LENGTHS><<<dim3(tiles, a.n_split), 256, bytes, stream>>>(a);
+  };
+  if (a.cap > a.n_split)
+    launch(std::true_type());
+  else
+    launch(std::false_type());
 }
 
 // A tile is a chain of reads, products and three barriers, during which a CU with one workgroup waits:

@@ -48,3 +48,17 @@ def make_batch(chunks, block, device, seed=0, spare=3):
         logit_rows=t([0]), sample_seq_ids=[],
     )
     return batch, chunks, [m.block_table for m in prefills] + tables, sum(need) + spare
+
+
+def record_latent_parts(monkeypatch):
+    """A list that gets every latent attention launch's (parts that most rows have, the most that one has)."""
+    from agentcontrolplane_amd.ops import hip
+
+    seen, launch = [], hip._C.latent_attn
+
+    def record(*args):
+        seen.append(args[-4:-2])
+        launch(*args)
+
+    monkeypatch.setattr(hip._C, "latent_attn", record)
+    return seen

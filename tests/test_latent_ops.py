@@ -7,7 +7,7 @@ import torch
 import fetolix_oracle as oracle
 from agentcontrolplane_amd import ops
 from agentcontrolplane_amd.ops.reference import build_cos_sin
-from op_helpers import BF16, F32, close, make_batch, rand
+from op_helpers import BF16, F32, close, make_batch, rand, record_latent_parts
 
 GPU = pytest.param("cuda", marks=pytest.mark.gpu)
 
@@ -307,22 +307,35 @@ def test_latent_attention(device, dtype, H, kv_rank, window, block, chunks):
         at += new
 
 
-# a decode step's parts by length: one long sequence, few and many of them, none whole, windows, heads of
-# several tiles, more sequences than lanes
+# a decode step's parts by length or by as many a sequence: one long sequence, few and many of them, one and
+# several sequences a lane and row tiles a sequence, windows
 RAGGED = [
-    (16, 512, None, [6000] + [1, 127, 128, 129, 33, 32, 31]),
-    (16, 500, None, [150 * i + 1 for i in range(40)]),
-    (40, 128, None, [1, 2000, 3, 1999]),
-    (16, 512, 1024, [1, 700, 1024, 1025, 6000, 40]),
-    (3, 250, 300, [(37 * i) % 3000 + 1 for i in range(200)]),
-    (128, 64, None, [9, 2040]),
+    # heads, latent, window, lengths, by length
+    (16, 512, None, [6000] + [127, 128, 129, 33, 32, 31] * 5, True),
+    (16, 500, None, [150 * i + 2 for i in range(40)], True),
+    (16, 250, None, [37 * i % 2500 + 2 for i in range(70)], True),
+    (3, 250, None, [37 * i % 3000 + 2 for i in range(130)], True),
+    (16, 500, None, [53 * i % 1500 + 2 for i in range(200)] + [4100], True),
+    (16, 100, None, [91 * i % 1100 + 2 for i in range(256)], True),
+    (7, 60, None, [40] * 255 + [5000], True),
+    (128, 64, None, [9, 2040] * 20, True),
+    (40, 128, None, [2, 2000, 3, 1999] * 16, True),
+    (128, 512, None, [300 * i + 2 for i in range(20)], True),
+    (20, 500, None, [200 * i + 40 for i in range(30)], True),
+    (16, 512, None, [6000] + [1, 127, 128, 129, 33, 32, 31], False),
+    (16, 512, 1024, [2, 700, 1024, 1025, 6000, 40] * 5, False),
+    (3, 250, 300, [37 * i % 3000 + 2 for i in range(100)], False),
+    (40, 128, None, [1, 2000, 3, 1999], False),
+    (16, 512, None, [99 * i % 700 + 2 for i in range(256)] + [2000], False),
 ]
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,kv_rank,window,lens", RAGGED)
-def test_parts_by_length(H, kv_rank, window, lens):
+@pytest.mark.parametrize("H,kv_rank,window,lens,by_length", RAGGED)
+def test_parts_by_length(H, kv_rank, window, lens, by_length, monkeypatch):
+    seen = record_latent_parts(monkeypatch)
     test_latent_attention("cuda", BF16, H, kv_rank, window, 16, [(0, 2)] + [(n - 1, 1) for n in lens])
+    assert any(cap > n > 1 for n, cap in seen) == by_length
 
 
 @pytest.mark.gpu

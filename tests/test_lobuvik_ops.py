@@ -16,7 +16,7 @@ from agentcontrolplane_amd.engine.config import (
 from agentcontrolplane_amd.models.grouped_attention import distance_buckets
 from agentcontrolplane_amd.models.layout import pair_halves, unpair_halves
 from agentcontrolplane_amd.models.rotary import frequencies, rotation_table
-from op_helpers import BF16, F32, close, make_batch, rand
+from op_helpers import BF16, F32, close, make_batch, rand, record_latent_parts
 
 GPU = pytest.param("cuda", marks=pytest.mark.gpu)
 
@@ -388,6 +388,15 @@ def test_latent_sink(device, dtype, H, kv_rank, window, chunks):
             want = oracle.sink_softmax(s[h], sink[h].double().cpu()) @ rows[:, :rank]
             close(got[at : at + new, h], want, dtype)
         at += new
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,kv_rank,sequences", [(6, 500, 40), (3, 250, 130)])
+def test_latent_sink_of_parts_by_length(H, kv_rank, sequences, monkeypatch):
+    seen = record_latent_parts(monkeypatch)
+    chunks = [(0, 5)] + [(990 * i // sequences + 1, 1) for i in range(sequences)]
+    test_latent_sink("cuda", BF16, H, kv_rank, None, chunks)
+    assert any(cap > n > 1 for n, cap in seen)
 
 
 @pytest.mark.gpu
