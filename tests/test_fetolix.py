@@ -22,6 +22,7 @@ from agentcontrolplane_amd.models import create_model
 from agentcontrolplane_amd.models.configs import read_architecture, read_model_config
 from agentcontrolplane_amd.models.weights import save_checkpoint
 from model_helpers import CUTS, assert_close, feed, make_engine, tokens
+from op_helpers import record_latent_parts
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 GPU = pytest.param("cuda", marks=pytest.mark.gpu)
@@ -364,6 +365,70 @@ def test_graph_replay_matches_eager(checkpoints, dtype):
             torch.cuda.synchronize()
         assert bool(eng._m.get("graph_steps")) != eager
         runs.append(torch.cat(rows))
+    assert (runs[0] - runs[1]).abs().max() <= 1e-3 * runs[1].abs().max()
+
+
+def write_checkpoint(path, cfg):
+    W = make_weights(cfg, seed=9)
+    save_file(W, str(path / "model.safetensors"))
+    (path / "config.json").write_text(json.dumps(cfg))
+    return {k: v.double() for k, v in W.items()}
+
+
+@pytest.mark.gpu
+def test_side_layers_of_products_in_parts(tmp_path, monkeypatch):
+    """An output product large enough to be left in parts, which the side layer adds up: in a loop, ahead of
+    it and behind it, in steps of many rows and of few."""
+    from agentcontrolplane_amd.ops import hip
+
+    cfg = {
+        "architecture": "Fetolix", "vocab": 300, "width": 512, "norm": {"eps": 1e-5},
+        "layers": [
+            full(heads=8, dim=64, rot=32, vdim=64, rank=128, base=1e4, scale=0.2, ff=3648),
+            win(heads=16, dim=32, rot=64, vdim=64, rank=64, base=2e5, q_rank=64, window=30, scale=0.2, ff=3072),
+            full(heads=8, dim=64, rot=32, vdim=64, rank=128, base=1e4, scale=0.2, ff=3648),
+        ],
+        "loop": {"start": 1, "stop": 2, "times": 2}, "token_side": {"dim": 32},
+    }
+    W, seen, launch = write_checkpoint(tmp_path, cfg), [], hip._C.side_layer
+    monkeypatch.setattr(hip._C, "side_layer", lambda x, y, *a: (seen.append((len(x), y.dim())), launch(x, y, *a)))
+    ids = tokens(150, cfg, seed=3)
+    cuts = [5, 16, 33, 1, 60, 2] + [1] * 33
+    got = feed(TraceReplay(make_engine(str(tmp_path), "cuda", "bfloat16", enforce_eager=True)), "a", ids, cuts)
+    assert_close(got, oracle.forward(cfg, W, ids), "bfloat16")
+    assert {(5, 3), (16, 3), (33, 3), (60, 3), (1, 2), (2, 2)} <= set(seen)
+
+
+@pytest.mark.gpu
+def test_graph_replay_of_parts_by_length(tmp_path, monkeypatch):
+    """The parts of a captured decode step follow the lengths that each replay meets.  One sequence is as long
+    as the model allows, so that an eager step's tables are as wide as the captured one's and both cut alike."""
+    cfg = {
+        "architecture": "Fetolix", "vocab": 300, "width": 64, "norm": {"eps": 1e-5},
+        "layers": [full(heads=4, dim=32, rot=64, vdim=32, rank=256, base=1e4, scale=0.2, ff=64)],
+        "loop": {"start": 0, "stop": 1, "times": 2}, "token_side": {"dim": 8},
+    }
+    write_checkpoint(tmp_path, cfg)
+    names = [f"r{i}" for i in range(40)]
+    runs = []
+    for eager in (False, True):
+        seen = record_latent_parts(monkeypatch)
+        eng = make_engine(str(tmp_path), "cuda", "bfloat16", enforce_eager=eager, num_kv_blocks=3000,
+                          max_batch_size=40, max_prefill_tokens=40000)
+        replay, rows = TraceReplay(eng), []
+        for turn, grow in enumerate([
+                lambda i: 3 + 11 * i if i else 1012, lambda i: 500 * (i % 7 == 3), lambda i: 400 * (i == 1)]):
+            more = [{"id": r, "tokens": tokens(grow(i), cfg, seed=i + turn), "want": []}
+                    for i, r in enumerate(names) if grow(i)]
+            replay.step(more, [])
+            for s in range(3):
+                rows.append(replay.step(
+                    [{"id": r, "tokens": tokens(1, cfg, seed=s + 5 * i), "want": [0]}
+                     for i, r in enumerate(names)], []))
+        assert any(cap > n > 1 for n, cap in seen)
+        assert eng._m.get("graph_steps", 0) == (0 if eager else 9)
+        runs.append(torch.cat(rows))
+        monkeypatch.undo()
     assert (runs[0] - runs[1]).abs().max() <= 1e-3 * runs[1].abs().max()
 
 
