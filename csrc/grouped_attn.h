@@ -23,6 +23,7 @@ struct GroupedArgs {
   int H, G, group, n_tiles, max_blocks, kv_block, window, keep, n_split, rows, n_bias;
   int seqs, pieces;       // decode: workgroups of a key head that share the step's keys; 0: one a sequence
   int gm;                 // decode: query heads of a workgroup
+  int shared_from;        // decode: blocks of a piece from which a sequence's short last one is shared
   bool ranges;            // decode: they may take parts of several sequences each
   int chunk;              // only keys of the query's own chunk; 2^30: all
   float scale, cap;       // cap 0: none

@@ -114,11 +114,13 @@ static DEV float max_with(float v) {
 // parts have starts and ends, 4 x 300 keys 16.0 us by ranges and 11.8 by pieces, 64 x 512 35.4 and 32.
 //
 // Without a.ranges always pieces: of one size where they are all resident at once, or sequences are no longer than
-// that, else in about two rounds, with a last piece of under a quarter shared by the sequence's others unless they
-// are short (of 12 blocks 20 x 130 to 3900 keys 53.7 us shared and 52.0 not).  Without that sharing 64 query heads of
-// 8 key heads, 30 x 300 to 4000 keys, 76.6 us instead of 73.2, 100 x 700 to 1300 107.2 and 104.5; 128 query
-// heads, 20 x 130 to 3900 80.0 and 75.2.  The kernel with several parts is 0.5 to 1 us slower for one, so that few
-// sequences go without (RANGES_FROM), and for 8 query heads a workgroup it has not the registers.
+// that (16 query heads of 2 key heads, 61 x 310 to 4000 keys, 40.3 us, else 48.4).  Else for about two rounds, with a
+// last piece of under a quarter shared by the sequence's others from a.shared_from blocks on (of 12 blocks 20 x 130
+// to 3900 keys shared 53.7 us and 52.0 not, of 256 dims, where a CU has one workgroup, 24 x 510 to 2400 104 and 114).
+// Without that sharing 64 query heads of 8 key heads, 30 x 300 to 4000 keys, 76.6 us instead of 73.2, 100 x 700 to
+// 1300 107.2 and 104.5; 128 query heads, 20 x 130 to 3900 80.0 and 75.2.  The kernel with several parts is 0.5 to
+// 1 us slower for one, so that few sequences go without (RANGES_FROM), and for 8 query heads a workgroup it has not
+// the registers.
 struct Cut {
   bool aligned;  // pieces of sequences
   int count;     // ranges of a workgroup
@@ -177,7 +179,7 @@ static DEV Stretch find_range(const GroupedArgs& a, int want, int item, Cut& cut
     cut.each = (share + 1) / 2;
   }
   const int first = cut.aligned ? item : item * cut.count * cut.each;
-  const int spared = two_rounds - (two_rounds < 16 ? 0 : two_rounds / 4) - 1;
+  const int spared = two_rounds - (two_rounds < a.shared_from ? 0 : two_rounds / 4) - 1;
   Stretch x = {-1, 0, 0, 0};
   int before = 0;
   for (int s = 0; s < a.seqs; s += 64) {
@@ -790,6 +792,7 @@ template <int DN, int VN>
 static bool launch_decode(const GroupedArgs& args, int gm, hipStream_t stream) {
   GroupedArgs a = args;
   a.gm = gm;
+  a.shared_from = DN + VN <= 4 ? 16 : 12;
   a.ranges = a.pieces && gm < 8 && a.seqs * a.G * ((a.group + gm - 1) / gm) >= RANGES_FROM;
   if (gm == 1)
     (a.sigmoid ? launch_decode<DN, VN, 1, true> : launch_decode<DN, VN, 1, false>)(a, stream);

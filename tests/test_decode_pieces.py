@@ -31,13 +31,13 @@ def test_quotient_is_exact():
                 assert (q == x // d).all()
 
 
-def cut(blocks, pieces):
+def cut(blocks, pieces, shared_from=12):
     """[(pieces, blocks of one)] of the sequences."""
     half = max(1, (sum(blocks) + 2 * pieces - 1) // (2 * pieces))
     size = 4 * (max(min(half, 3), (half + 1) // 2) if max(blocks) > 4 * half else half)
     out = []
     for n in blocks:
-        k, each = max(1, (n + size - (0 if size < 16 else size // 4) - 1) // size), size
+        k, each = max(1, (n + size - (0 if size < shared_from else size // 4) - 1) // size), size
         if k * size < n:
             each = 4 * -(-n // (4 * k))
             k = -(-n // each)
@@ -45,13 +45,14 @@ def cut(blocks, pieces):
     return out
 
 
+@pytest.mark.parametrize("shared_from", [12, 16])
 @pytest.mark.parametrize("pieces", [1, 7, 25, 128, 1024])
-def test_pieces_fit_their_workspace(pieces):
+def test_pieces_fit_their_workspace(pieces, shared_from):
     gen = np.random.default_rng(pieces)
     for _ in range(400):
         top = int(np.exp(gen.uniform(0, np.log(40000))))
         blocks = gen.integers(0, top + 1, int(np.exp(gen.uniform(0, np.log(1000))))).tolist()
-        parts = cut(blocks, pieces)
+        parts = cut(blocks, pieces, shared_from)
         assert sum(k for k, _ in parts) <= pieces + len(blocks)
         for n, (k, each) in zip(blocks, parts):
             assert k * each >= n and (k == 1 or (k - 1) * each < n)

@@ -21,7 +21,7 @@ def cut(blocks, P, paired, ranges):
         if spare >= 0 and max(blocks) <= most:
             return True, 1, [most] * seqs
         if not ranges:
-            return True, 1, [each for _, each in two_rounds(blocks, 2 * P)]
+            return True, 1, [each for _, each in two_rounds(blocks, 2 * P, 16)]
         each = -(-total // spare) if spare else most + 1
         return (True, 1, [max(4, each)] * seqs) if each <= most else (False, 1, max(4, share))
     return (False, 2, (share + 1) // 2) if share > 32 and paired else (False, 1, max(4, share))
