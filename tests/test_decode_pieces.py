@@ -1,5 +1,5 @@
-"""The arithmetic by which a decode step's keys are cut into pieces of about two rounds of workgroups
-(csrc/grouped_attn.hip, find_range without ranges): at most pieces + sequences of them."""
+"""The arithmetic by which a decode step's keys are cut into pieces (csrc/grouped_attn.hip,
+find_range, for pieces of about two rounds of workgroups): at most pieces + sequences."""
 import numpy as np
 import pytest
 
@@ -31,13 +31,13 @@ def test_quotient_is_exact():
                 assert (q == x // d).all()
 
 
-def cut(blocks, pieces, shared_from=12):
+def cut(blocks, pieces):
     """[(pieces, blocks of one)] of the sequences."""
     half = max(1, (sum(blocks) + 2 * pieces - 1) // (2 * pieces))
     size = 4 * (max(min(half, 3), (half + 1) // 2) if max(blocks) > 4 * half else half)
     out = []
     for n in blocks:
-        k, each = max(1, (n + size - (0 if size < shared_from else size // 4) - 1) // size), size
+        k, each = max(1, (n + size - (0 if size < 12 else size // 4) - 1) // size), size
         if k * size < n:
             each = 4 * -(-n // (4 * k))
             k = -(-n // each)
@@ -45,14 +45,13 @@ def cut(blocks, pieces, shared_from=12):
     return out
 
 
-@pytest.mark.parametrize("shared_from", [12, 16])
 @pytest.mark.parametrize("pieces", [1, 7, 25, 128, 1024])
-def test_pieces_fit_their_workspace(pieces, shared_from):
+def test_pieces_fit_their_workspace(pieces):
     gen = np.random.default_rng(pieces)
     for _ in range(400):
         top = int(np.exp(gen.uniform(0, np.log(40000))))
         blocks = gen.integers(0, top + 1, int(np.exp(gen.uniform(0, np.log(1000))))).tolist()
-        parts = cut(blocks, pieces, shared_from)
+        parts = cut(blocks, pieces)
         assert sum(k for k, _ in parts) <= pieces + len(blocks)
         for n, (k, each) in zip(blocks, parts):
             assert k * each >= n and (k == 1 or (k - 1) * each < n)

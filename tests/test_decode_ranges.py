@@ -7,59 +7,47 @@ import pytest
 import torch
 
 from agentcontrolplane_amd import ops
-from test_decode_pieces import cut as two_rounds
 
 
 def cut(blocks, P, paired, ranges):
-    """(aligned, ranges of a workgroup, blocks of one or of each sequence's pieces) as the kernel finds them."""
+    """(aligned, ranges of a workgroup, blocks of one) as the kernel finds them."""
     total, seqs = sum(blocks), len(blocks)
     share, spare = -(-total // P), P - seqs
     if not ranges or (share <= 32 and spare >= 0):
         even, most = (share + 3) // 4 * 4, share + share // 4 + 4
         if seqs <= 64 and sum(-(-n // even) for n in blocks) <= P:
-            return True, 1, [even] * seqs
+            return True, 1, even
         if spare >= 0 and max(blocks) <= most:
-            return True, 1, [most] * seqs
+            return True, 1, most
         if not ranges:
-            return True, 1, [each for _, each in two_rounds(blocks, 2 * P, 16)]
+            return True, 1, max(4, (share + 7) // 8 * 4)
         each = -(-total // spare) if spare else most + 1
-        return (True, 1, [max(4, each)] * seqs) if each <= most else (False, 1, max(4, share))
+        return (True, 1, max(4, each)) if each <= most else (False, 1, max(4, share))
     return (False, 2, (share + 1) // 2) if share > 32 and paired else (False, 1, max(4, share))
 
 
-def parts(lens, P, paired, ranges):
-    """{(workgroup, one of two heads): [(head, range, sequence, from, to, goes on)]} of sequences of so many
-    blocks, as the workgroups go on; a sequence without a block has a turn of one"""
-    turns = [max(1, n) for n in lens]
-    aligned, count, each = cut(turns, P, paired, ranges)
-    before = np.concatenate([[0], np.cumsum([-(-n // e) for n, e in zip(turns, each)] if aligned else turns)])
+def parts(blocks, P, paired, ranges):
+    """{workgroup of a key head: [(other head's, range, sequence, from, to, goes on)]}"""
+    aligned, count, each = cut(blocks, P, paired, ranges)
+    before = np.concatenate([[0], np.cumsum([-(-n // each) if aligned else n for n in blocks])])
     out = {}
-    items = P if ranges else 2 * P + len(lens)
-    assert not aligned or before[-1] <= items
-    for item in range(items):
+    for item in range(P if ranges else 2 * P + len(blocks)):
         first = item if aligned else item * count * each
         if first >= before[-1]:
             continue
-        for at in (0, 1):
-            seq = int(np.searchsorted(before, first, "right")) - 1
-            left = size = each[seq] if aligned else each
-            head, r, on, start = at, item * count, False, (first - int(before[seq])) * (size if aligned else 1)
-            mine = out[item, at] = []
-            while True:
-                to = min(lens[seq], start + left)
-                mine.append((head, r, seq, start, to, on))
-                left -= max(1, to - start)
-                if aligned:
-                    break
-                on = left > 0
-                if not on:  # the next range, of the other head
-                    r, head, left = r + 1, head ^ 1, size
-                    if count == 1 or r % 2 == 0:
-                        break
-                stays = not on and to < lens[seq]
-                seq, start = (seq, to) if stays else (seq + 1, 0)
-                if seq == len(lens):
-                    break
+        seq = int(np.searchsorted(before, first, "right")) - 1
+        at, mine = (first - int(before[seq])) * (each if aligned else 1), []
+        if aligned:
+            mine.append((0, item, seq, at, min(blocks[seq], at + each), False))
+        for j in range(0 if aligned else count):
+            left, goes_on = each, False
+            while left > 0 and seq < len(blocks):
+                to = min(blocks[seq], at + left)
+                mine.append((j, item * count + j, seq, at, to, goes_on))
+                left -= to - at
+                seq, at = (seq, to) if to < blocks[seq] else (seq + 1, 0)
+                goes_on = True
+        out[item] = mine
     return out, (aligned, each, before)
 
 
@@ -67,55 +55,52 @@ def parts(lens, P, paired, ranges):
 @pytest.mark.parametrize("P,paired", [(64, True), (16, True), (7, False), (1, True), (256, True)])
 def test_every_block_has_one_workgroup(P, paired, ranges):
     """Of either head, whose partial results have places of their own in the workspace, which are those that
-    the merge reads.  Sequences of no block are written once for either head."""
+    the merge reads."""
     gen = np.random.default_rng(P)
-    for _ in range(120):
+    for _ in range(150):
         top = int(np.exp(gen.uniform(0, np.log(3000))))
-        lens = gen.integers(0, top + 1, int(np.exp(gen.uniform(0, np.log(400))))).tolist()
-        shares, (aligned, each, before) = parts(lens, P, paired, ranges)
-        seen, slots = {}, {}
-        for mine in shares.values():
-            # a second range is of the other head
-            assert len({head for head, *_ in mine}) == len({r for _, r, *_ in mine})
-            for head, r, s, start, to, on in mine:
-                assert 0 <= start <= to <= lens[s] and (start < to or lens[s] == 0)
-                seen.setdefault((head, s), []).append((start, to))
-                if (start, to) != (0, lens[s]):
-                    slot = 2 * r + (to < lens[s] and on)
-                    assert (head, slot) not in slots and slot < 2 * (2 * P + len(lens))
-                    slots[head, slot] = s
+        blocks = gen.integers(1, top + 1, int(np.exp(gen.uniform(0, np.log(400))))).tolist()
+        shares, (aligned, each, before) = parts(blocks, P, paired, ranges)
         for head in (0, 1):
-            places = {}
-            for (h, slot), s in slots.items():
-                if h == head:
-                    places.setdefault(s, set()).add(slot)
-            for s, n in enumerate(lens):
-                own = sorted(seen[head, s])
-                assert [a for a, _ in own] == [0] + [b for _, b in own[:-1]] and own[-1][1] == n
-                turn = max(1, n)
+            seen, slots = {s: [] for s in range(len(blocks))}, {}
+            for mine in shares.values():
+                for j, r, s, at, to, goes_on in mine:
+                    # the two workgroups of a pair of heads change heads for their second range
+                    if cut(blocks, P, paired, ranges)[1] == 2 or head == 0:
+                        assert 0 <= at < to <= blocks[s]
+                        seen[s].append((at, to))
+                        if (at, to) != (0, blocks[s]):
+                            slot = 2 * r + (to < blocks[s] and goes_on)
+                            assert slot not in slots and slot < 2 * (2 * P + len(blocks))
+                            slots[slot] = s
+            if head and not slots and not any(seen.values()):
+                continue
+            for s, n in enumerate(blocks):
+                assert [a for a, _ in seen[s]] == [0] + [b for _, b in seen[s][:-1]]
+                assert seen[s][-1][1] == n
                 if aligned:
-                    first, k, ahead = int(before[s]), -(-turn // each[s]), 0
+                    first, k, ahead = int(before[s]), -(-n // each), 0
                 else:
                     first = int(before[s]) // each
-                    k = (int(before[s]) + turn - 1) // each - first + 1
+                    k = (int(before[s]) + n - 1) // each - first + 1
                     ahead = first * each < before[s]
-                # one part is written by its workgroup, several are what the merge reads
-                assert (k > 1) == (s in places)
                 if k > 1:
-                    assert places[s] == {2 * (first + i) + (i == 0 and ahead) for i in range(k)}
+                    assert {2 * (first + i) + (i == 0 and ahead) for i in range(k)} == {
+                        t for t, q in slots.items() if q == s}
 
 
-LENS = {
-    "long": [1, 0, 33, 32, 31] + [4100] + [64] * 60,     # one long sequence among short ones
-    "even": [2048] * 65,                                 # ranges that end where sequences do
-    "ragged": [37 + 211 * i % 1900 for i in range(70)],  # in the middle of them
-    "many": [5] * 200 + [9000],
-}
-
-
-def check_decode(H, G, d, lens, block=16, window=None, keep=0, cap=0.0, form=""):
-    """A step whose keys are cut, however many sequences, against fp32.  form: what else a layer has."""
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,d", [(8, 8, 128), (32, 8, 128), (6, 3, 128), (4, 2, 256)])
+@pytest.mark.parametrize("lens", [
+    [1, 0, 33, 32, 31] + [4100] + [64] * 60,            # one long sequence among short ones
+    [2048] * 65,                                        # ranges that end where sequences do
+    [37 + 211 * i % 1900 for i in range(70)],           # in the middle of them
+    [5] * 200 + [9000],
+], ids=["long", "even", "ragged", "many"])
+@pytest.mark.parametrize("form", ["plain", "window"])
+def test_decode_by_ranges(H, G, d, lens, form):
     gen = torch.Generator("cuda").manual_seed(len(lens) + H)
+    block, window = 16, (500, 40) if form == "window" else (None, 0)
     n_blocks = [-(-max(n, 1) // block) for n in lens]
     table = torch.zeros(len(lens), max(n_blocks), dtype=torch.int32, device="cuda")
     order = torch.randperm(sum(n_blocks), generator=gen, device="cuda").int()
@@ -124,21 +109,16 @@ def check_decode(H, G, d, lens, block=16, window=None, keep=0, cap=0.0, form="")
     k, v = (torch.randn(len(order), block, G, d, generator=gen, device="cuda").bfloat16()
             for _ in range(2))
     q = torch.randn(len(lens), H, d, generator=gen, device="cuda").bfloat16()
-    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
-    sink = rand(H) if "sink" in form else None
-    bias = rand(H, 100) if "bias" in form else None
-    gate = rand(len(lens), H).bfloat16() if "gate" in form else None
-    sigmoid = "sigmoid" in form
     out = torch.full_like(q, 7.0)
-    hip = ops._hip()
+    hip, rest = ops._hip(), (1 << 30, False)
     seq_lens = torch.tensor(lens, dtype=torch.int32, device="cuda")
-    whole = hip._WHOLE_GROUPS
+    keep = hip._WHOLE_GROUPS
     try:
-        hip._WHOLE_GROUPS = 1 << 30
-        hip._grouped_decode(out, q, k, v, table, seq_lens, sink, bias, gate, d ** -0.5, cap, window or 1 << 30,
-                            1 << 30, keep, sigmoid)
+        hip._WHOLE_GROUPS = 1 << 30  # cut, however many sequences
+        hip._grouped_decode(out, q, k, v, table, seq_lens, None, None, None, d ** -0.5, 0.0,
+                            window[0] or 1 << 30, rest[0], window[1], rest[1])
     finally:
-        hip._WHOLE_GROUPS = whole
+        hip._WHOLE_GROUPS = keep
     for b, n in enumerate(lens):
         if n == 0:
             assert (out[b] == 0).all()
@@ -146,53 +126,11 @@ def check_decode(H, G, d, lens, block=16, window=None, keep=0, cap=0.0, form="")
         pages = table[b, : n_blocks[b]].long()
         keys, values = (c[pages].view(-1, G, d)[:n].float().repeat_interleave(H // G, 1) for c in (k, v))
         s = torch.einsum("nhd,hd->nh", keys, q[b].float()) * d ** -0.5
-        if cap:
-            s = cap * torch.tanh(s / cap)
-        p = torch.arange(n, device="cuda")[:, None]
-        if bias is not None:
-            s = s + bias[:, (n - 1 - p[:, 0]).clamp(max=99)].T
-        if window:
-            s = s.masked_fill((p <= n - 1 - window) & (p >= keep), -math.inf)
-        if sigmoid:
-            w = torch.sigmoid(s)
-        elif sink is not None:
-            w = torch.softmax(torch.cat([s, sink[None]]), 0)[:-1]
-        else:
-            w = torch.softmax(s, 0)
-        g = 1.0 if gate is None else torch.sigmoid(gate[b].float())[:, None]
-        want = g * (w.unsqueeze(-1) * values).sum(0)
+        if window[0]:
+            p = torch.arange(n, device="cuda")[:, None]
+            s = s.masked_fill((p <= n - 1 - window[0]) & (p >= window[1]), -math.inf)
+        w = torch.softmax(s, 0)
+        want = (w.unsqueeze(-1) * values).sum(0)
         # fp32 but for the result, and sums of up to 9000 terms in it
-        slack = 2.0 ** -8 * want.abs() + 2.0 ** -20 * g * (w.unsqueeze(-1) * values.abs()).sum(0) + 1e-4
+        slack = 2.0 ** -8 * want.abs() + 2.0 ** -20 * (w.unsqueeze(-1) * values.abs()).sum(0) + 1e-4
         assert ((out[b].float() - want).abs() <= slack).all(), (b, n)
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("H,G,d", [(8, 8, 128), (32, 8, 128), (6, 3, 128), (4, 2, 256)])
-@pytest.mark.parametrize("lens", list(LENS))
-@pytest.mark.parametrize("form", ["plain", "window"])
-def test_decode_by_ranges(H, G, d, lens, form):
-    window, keep = (500, 40) if form == "window" else (None, 0)
-    check_decode(H, G, d, LENS[lens], window=window, keep=keep)
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("H,G", [(8, 8), (16, 8), (32, 8)])
-@pytest.mark.parametrize("lens", ["long", "ragged"])
-@pytest.mark.parametrize("form,block,cap,window", [
-    ("sink", 32, 5.0, None), ("sink gate", 6, 0.0, 500), ("sigmoid bias", 16, 0.0, None), ("bias", 8, 5.0, None),
-    ("sigmoid", 64, 5.0, 300),
-])
-def test_decode_by_ranges_of_other_forms(H, G, lens, form, block, cap, window):
-    """What only a sequence's first part or a whole sequence has, pages of other sizes."""
-    check_decode(H, G, 128, LENS[lens], block, window, 0, cap, form)
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("H,G,lens", [
-    (64, 8, "long"), (64, 8, "even"), (64, 8, "ragged"), (64, 8, "many"), (40, 4, "ragged"), (16, 1, "long"),
-    (32, 8, [130 + 199 * i for i in range(19)]), (8, 8, [8000, 1, 0, 300]), (4, 2, [900] * 70), (2, 1, [40] * 90 + [5000]),
-], ids=str)
-@pytest.mark.parametrize("form", ["", "sink", "sigmoid"])
-def test_decode_by_pieces(H, G, lens, form):
-    """Without ranges: many query heads a key head, and few sequences."""
-    check_decode(H, G, 128, LENS.get(lens, lens) if isinstance(lens, str) else lens, form=form)

@@ -307,9 +307,27 @@ def test_latent_attention(device, dtype, H, kv_rank, window, block, chunks):
         at += new
 
 
+# a decode step's parts by length: one long sequence, few and many of them, none whole, windows, heads of
+# several tiles, more sequences than lanes
+RAGGED = [
+    (16, 512, None, [6000] + [1, 127, 128, 129, 33, 32, 31]),
+    (16, 500, None, [150 * i + 1 for i in range(40)]),
+    (40, 128, None, [1, 2000, 3, 1999]),
+    (16, 512, 1024, [1, 700, 1024, 1025, 6000, 40]),
+    (3, 250, 300, [(37 * i) % 3000 + 1 for i in range(200)]),
+    (128, 64, None, [9, 2040]),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,kv_rank,window,lens", RAGGED)
+def test_parts_by_length(H, kv_rank, window, lens):
+    test_latent_attention("cuda", BF16, H, kv_rank, window, 16, [(0, 2)] + [(n - 1, 1) for n in lens])
+
+
 # a decode step's parts by length or by as many a sequence: one long sequence, few and many of them, one and
 # several sequences a lane and row tiles a sequence, windows
-RAGGED = [
+BY_LENGTH = [
     # heads, latent, window, lengths, by length
     (16, 512, None, [6000] + [127, 128, 129, 33, 32, 31] * 5, True),
     (16, 500, None, [150 * i + 2 for i in range(40)], True),
@@ -331,8 +349,8 @@ RAGGED = [
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,kv_rank,window,lens,by_length", RAGGED)
-def test_parts_by_length(H, kv_rank, window, lens, by_length, monkeypatch):
+@pytest.mark.parametrize("H,kv_rank,window,lens,by_length", BY_LENGTH)
+def test_which_parts_go_by_length(H, kv_rank, window, lens, by_length, monkeypatch):
     seen = record_latent_parts(monkeypatch)
     test_latent_attention("cuda", BF16, H, kv_rank, window, 16, [(0, 2)] + [(n - 1, 1) for n in lens])
     assert any(cap > n > 1 for n, cap in seen) == by_length
