@@ -236,9 +236,12 @@ def side_gate(x, y, gate, token_ids, table, offset: int):
 
 def side_layer_fits(x, gate, *weights) -> bool:
     """What the one launch takes, and where it is the faster: a token's workgroup reads both weights by
-    itself, which is its time once they are over 256 KB each (2048 x 64 against the three launches, without
-    the sum of the parts: 10.7 and 10.6 us with one token, 11.7 and 14.0 with 40, 22.1 and 28.9 with 512;
-    4096 x 128: 28.3 and 14.6 with one, 64 and 43 with 512)."""
+    itself, which is its time once they are over 256 KB each.  Us in one launch and in three, without the sum of the
+    parts, of 1, 40, 128 and 512 tokens: 2048 x 64 9.8 and 10.0, 10.2 and 11.9, 10.4 and 13.9, 20.6 and 27.8.
+    Twice that is faster or slower by width and tokens: 4096 x 64 15.5 and 12.9, 16.0 and 14.8, 16.5 and
+    17.5, 33.9 and 43.0; 2048 x 128 14.8 and 10.1, 15.4 and 13.0, 15.9 and 16.5, 34.5 and 28.2; 8192 x 32 16.3 and
+    17.3, 17.1 and 18.9, 17.9 and 20.7, 37.6 and 48.2.  4096 x 128 25.5 and 13.1, 26.2 and 16.0, 26.7 and 21.1, 58.7
+    and 43.9."""
     (n, w), dim = x.shape, gate.shape[0]
     return (
         0 < n <= 512 and w % 8 == 0 and w <= 8192 and dim % 8 == 0 and dim <= 128

@@ -757,9 +757,8 @@ static const int* opt_int(const OptTensor& t, int64_t n) {
   return t->data_ptr<int>();
 }
 
-// q [tokens, H, rank] absorbed, q_rot [tokens, H, rot] -> out [tokens, H, rank].  Prefill chunks bring ctx_lens,
-// row_starts and tiles; decode (one token per table row) brings none of them.
-// out of rows that latent_attn() left in n_split parts
+// The heads' product, gated, of decode rows that latent_attn() left in parts: most in ``usual``, none in more
+// than n_split
 static void merge_head_linear(torch::Tensor out, torch::Tensor part, torch::Tensor part_ml, int64_t n_split,
                               int64_t usual, torch::Tensor w, OptTensor gate) {
   MergedHeads a{};
@@ -794,7 +793,10 @@ static void merge_head_linear(torch::Tensor out, torch::Tensor part, torch::Tens
   launch_merge_head_linear(&a, k, cur_stream());
 }
 
-// out is left as it is where n_split > 1 and the parts are not to be merged
+// q [tokens, H, rank] absorbed, q_rot [tokens, H, rot] -> out [tokens, H, rank].  Prefill chunks bring ctx_lens,
+// row_starts and tiles; decode (one token per table row) brings none of them.  Keys go in n_split parts a row or,
+// with cap > n_split, by the rows' lengths in up to cap parts, n_split on average (decode of up to 256
+// sequences alone).  out is left as it is where n_split > 1 and the parts are not to be merged.
 static void latent_attn(torch::Tensor out, torch::Tensor q, torch::Tensor q_rot,
                         torch::Tensor cos_sin, int64_t rot_dim, torch::Tensor cache,
                         torch::Tensor tables, torch::Tensor seq_lens, OptTensor ctx_lens,

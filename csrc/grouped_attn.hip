@@ -15,8 +15,10 @@
 // The blocks of 32 that the sequences' queries see are cut into even shares of the workgroups that are resident at
 // once, whatever the lengths (Cut, below); a workgroup finds its share from the lengths by itself, and a
 // second launch merges sequences of several workgroups.
-// Bound by memory: 6.0 to 6.2 TB/s of keys and values at 64 x 4096 and 256 x 1024 tokens, 32
-// heads over 8; 61 x 310 to 4000 118 -> 111 us by even shares of all keys, 61 x 670 to 7900 210 -> 188.
+// Bound by memory: with the merge 5.9 TB/s of keys and values at 64 x 4096, 6.2 at 256 x 1024 tokens, 32
+// heads over 8; 61 x 310 to 4000 106.5 -> 101 us by even shares of all keys, 61 x 670 to 7900 201 -> 184, 13 x
+// 300 to 3900 of 32 key heads 86 -> 80.6, but one of 4001 13.1 -> 13.4 and 4 x 200 to 4000 18.8 -> 19.1, whose
+// workgroups find the same pieces by a longer way.
 // Before, with products and sums over dims on the VALU, 4.1 TB/s there and 2.0 to 3.0 where
 // lengths differ: 61 x 310 to 4000 tokens 268 -> 122 us, 190 x 700 to 1300 265 -> 159,
 // 1 x 4002 203 -> 14; with the values' loads, whole lines each, past the caches 190 x 700 to 1300 148
@@ -108,7 +110,7 @@ static DEV float max_with(float v) {
 // same time.  Of many blocks a workgroup has two ranges half as long, of two key heads, as rows
 // of some heads come more slowly than others (XCDs and channels share unevenly: one head each, 64 x 2048
 // keys end after 68 to 93 us, two 64 to 87).  61 x 310 to 4000 keys of 8 heads, the kernel alone: pieces of
-// sequences, up to 1112 workgroups in turn, 105 us, ranges 98, of two heads 93.
+// sequences, up to 1112 workgroups in turn, 105 us, ranges 98, of two heads 93 (on a faster card 92 and 85).
 //
 // Or few blocks into pieces of one sequence each, where that leaves no workgroup with much more than its share:
 // parts have starts and ends, 4 x 300 keys 16.0 us by ranges and 11.8 by pieces, 64 x 512 35.4 and 32.
